@@ -98,6 +98,9 @@ int32_t mi355_rmsnorm_f32(const float* x, const float* w, uint32_t n, float eps,
  */
 int32_t mi355_quantize_a8(const void* x, uint32_t input_kind, uint32_t rows, uint32_t width, uint64_t x_stride_bytes,
                           int8_t* codes, float* deltas, int32_t* sums, uint32_t* status, mi355_stream stream);
+/* The same with status[r] stored (0 or the flag) instead of ORed into: the caller need not clear it first. */
+int32_t mi355_quantize_a8_fresh(const void* x, uint32_t input_kind, uint32_t rows, uint32_t width, uint64_t x_stride_bytes,
+                                int8_t* codes, float* deltas, int32_t* sums, uint32_t* status, mi355_stream stream);
 
 /* ------------------------------------------------------------------------------------------------------
  * Dense Q8_0 x A8 product. Field for field strix::cpu::Q8a8View (src/cpu/core/backend.hpp:52-59); replaces

@@ -1,0 +1,186 @@
+// The Q8_0 linear operators: the A8 image of activation rows and the Q8_0 x A8 products. See include/mi355_strix.h for the contract of
+// every entry point; reference file:line citations are relative to the reference tree.
+#include "a8_rows.hpp"
+#include "gemm_q8_0.hpp"
+
+#include <type_traits>
+
+namespace strix950 {
+
+// ======================================================================================================== Q8_0 x A8 GEMV
+// One aligned group of 32 lanes per output row: lane l owns the reference's accumulator lane l (groups g = l, l + 32,
+// ... ascending), then the tree32 butterfly. Up to RB activation rows share one sweep of the weight row.
+// Reference: src/cpu/core/reference.cpp:57-84, src/core/integer_math.hpp:11-13,43-47.
+// DW: the weight rows are 4-byte aligned. A block (34 bytes: fp16 scale, 32 codes) is then fetched as nine aligned dwords
+// (two 128-bit loads and one 32-bit load) around its codes and shifted into place, instead of seventeen 16-bit loads.
+// CHAIN (RB = 1): the row contract of the reference's dense A8 profile (src/hip_q8_rows_gemv.hpp:1155-1170; host statement
+// tests/dense_a8_small_reference_tests.cpp:93-104): acc = +0, then for the blocks in ascending order acc = fma(float(d_w) * delta,
+// float(dot), acc), and a NaN result is stored as 0x7fc00000. The lanes evaluate their blocks as before and leave every block's
+// (scale, dot) pair in LDS; lane 0 of the output's 32 lanes then walks them in order.
+constexpr uint32_t kGemvChainMaxGroups = 256;          // in <= 8192 (kDenseA8MaxWidth, src/hip_q8_rows_gemv.hpp:1176)
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int RB, bool DW, bool CHAIN = false>
+__global__ __launch_bounds__(256) void gemv_q8_0_a8_kernel(mi355_q8a8_view v) {
+    __shared__ float2 chain_pairs[CHAIN ? 8 : 1][CHAIN ? kGemvChainMaxGroups : 1];
+    const uint32_t o = blockIdx.x * 8U + (threadIdx.x >> 5), l = threadIdx.x & 31U, row0 = blockIdx.y * RB;
+    if (o >= v.count) return;
+    const uint32_t groups = v.in / 32U;
+    const uint32_t nr = v.rows - row0 < static_cast<uint32_t>(RB) ? v.rows - row0 : static_cast<uint32_t>(RB);
+    const uint8_t* wrow = v.weight + static_cast<size_t>(o) * v.row_bytes;
+    float lane[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) lane[r] = 0.0F;
+    // (unrolled: the loads of four of the lane's groups are in flight together; the accumulation order does not change)
+#pragma unroll 4
+    for (uint32_t g = l; g < groups; g += 32U) {
+        const unsigned short* b = reinterpret_cast<const unsigned short*>(wrow + static_cast<size_t>(g) * kQ80Block);
+        const float scale = half_bits_to_float(b[0]);
+        int w[8];
+        if constexpr (DW) {
+            const uint32_t c0 = g * kQ80Block + 2U, shift = c0 & 3U;          // first code byte: 0 or 2 past a dword boundary
+            const uint32_t* dw = reinterpret_cast<const uint32_t*>(wrow) + (c0 >> 2);
+            const u32x4_a4 lo4 = *reinterpret_cast<const u32x4_a4*>(dw), hi4 = *reinterpret_cast<const u32x4_a4*>(dw + 4);
+            const uint32_t last = dw[shift ? 8 : 7];                          // (an aligned block ends with its eighth dword)
+            const uint32_t d[9] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w, last};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(__builtin_amdgcn_alignbyte(d[i + 1], d[i], shift));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(static_cast<uint32_t>(b[1 + 2 * i]) | (static_cast<uint32_t>(b[2 + 2 * i]) << 16));
+        }
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+            if (static_cast<uint32_t>(r) < nr) {
+                const int4* xc = reinterpret_cast<const int4*>(v.codes + static_cast<size_t>(row0 + r) * v.x_stride + g * 32U);
+                const int4 a = xc[0], c = xc[1];
+                int dot = 0;
+                dot = __builtin_amdgcn_sdot4(w[0], a.x, dot, false); dot = __builtin_amdgcn_sdot4(w[1], a.y, dot, false);
+                dot = __builtin_amdgcn_sdot4(w[2], a.z, dot, false); dot = __builtin_amdgcn_sdot4(w[3], a.w, dot, false);
+                dot = __builtin_amdgcn_sdot4(w[4], c.x, dot, false); dot = __builtin_amdgcn_sdot4(w[5], c.y, dot, false);
+                dot = __builtin_amdgcn_sdot4(w[6], c.z, dot, false); dot = __builtin_amdgcn_sdot4(w[7], c.w, dot, false);
+                const float xd = v.deltas[static_cast<size_t>(row0 + r) * (v.x_stride / 32U) + g];
+                if constexpr (CHAIN) chain_pairs[threadIdx.x >> 5][g] = make_float2(scale * xd, static_cast<float>(dot));
+                else lane[r] = lane[r] + static_cast<float>(dot) * (scale * xd);
+            }
+        }
+    }
+    if constexpr (CHAIN) {
+        // the pairs were written by lanes of this wave: program order of one wave's LDS accesses
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (l == 0) {
+            float acc = 0.0F;
+            for (uint32_t g = 0; g < groups; ++g) {
+                const float2 c = chain_pairs[threadIdx.x >> 5][g];
+                acc = __builtin_fmaf(c.x, c.y, acc);
+            }
+            v.out[static_cast<size_t>(row0) * v.out_stride + o] = acc != acc ? __builtin_bit_cast(float, 0x7fc00000U) : acc;
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+        float p = lane[r];
+        p = p + xor16_f(p); p = p + xor8_f(p); p = p + xor4_f(p); p = p + xor2_f(p); p = p + xor1_f(p);
+        if (l == 0 && static_cast<uint32_t>(r) < nr) {
+            float* y = &v.out[static_cast<size_t>(row0 + r) * v.out_stride + o];
+            *y = v.accumulate ? *y + p : p;
+        }
+    }
+}
+
+}  // namespace strix950
+
+using namespace strix950;
+
+namespace {
+int32_t a8_image(const A8RowArgs& a, uint32_t kind, uint32_t rows, hipStream_t st) {
+    const uint32_t threads = a8_row_threads(a.width);
+    if (kind == MI355_INPUT_F32) a8_rows_kernel<0><<<rows, threads, 0, st>>>(a);
+    else if (kind == MI355_INPUT_F16) a8_rows_kernel<1><<<rows, threads, 0, st>>>(a);
+    else a8_rows_kernel<2><<<rows, threads, 0, st>>>(a);
+    STRIX_LAUNCHED("quantize_a8");
+    return MI355_OK;
+}
+int32_t quantize_a8(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
+                    int32_t* sums, uint32_t* status, uint32_t status_mode, uint32_t nan_delta, mi355_stream stream) {
+    STRIX_REQUIRE(width % 32U == 0, "A8 activation width must be a multiple of 32");
+    STRIX_REQUIRE(kind <= MI355_INPUT_BF16, "A8: unknown input kind");
+    if (rows == 0 || width == 0) return MI355_OK;
+    STRIX_REQUIRE(x && codes && deltas, "A8: null pointer");
+    STRIX_REQUIRE(rows <= 65535U, "A8: at most 65535 rows per call");
+    const bool vec = aligned(x, 16) && x_stride % 16U == 0 && aligned(codes, 8);
+    return a8_image(A8RowArgs{static_cast<const uint8_t*>(x), x_stride, width, codes, deltas, sums, status, status ? status_mode : kA8StatusNone, vec, nan_delta},
+                    kind, rows, hs(stream));
+}
+}  // namespace
+
+extern "C" {
+
+int32_t mi355_quantize_a8(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
+                          int32_t* sums, uint32_t* status, mi355_stream stream) {
+    return quantize_a8(x, kind, rows, width, x_stride, codes, deltas, sums, status, kA8StatusOr, 0U, stream);
+}
+
+int32_t mi355_quantize_a8_fresh(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
+                                int32_t* sums, uint32_t* status, mi355_stream stream) {
+    return quantize_a8(x, kind, rows, width, x_stride, codes, deltas, sums, status, kA8StatusStore, 0U, stream);
+}
+
+int32_t mi355_dense_a8_quantize(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
+                                mi355_stream stream) {
+    return quantize_a8(x, kind, rows, width, x_stride, codes, deltas, nullptr, nullptr, kA8StatusNone, 1U, stream);
+}
+
+int32_t mi355_gemv_q8_0_a8_chain(const mi355_q8a8_view* v, mi355_stream stream) {
+    STRIX_REQUIRE(v, "Q8_0 chain product: null view");
+    STRIX_REQUIRE(v->in % 64U == 0 && v->in <= 32U * kGemvChainMaxGroups, "Q8_0 chain product: width must be a multiple of 64, at most 8192");   // dense_a8_width, src/hip_q8_rows_gemv.hpp:1184
+    STRIX_REQUIRE(!v->accumulate, "Q8_0 chain product: the chain starts at +0 (no accumulate)");
+    if (v->rows == 0 || v->count == 0) return MI355_OK;
+    STRIX_REQUIRE(v->weight && v->codes && v->deltas && v->out, "Q8_0 chain product: null pointer");
+    STRIX_REQUIRE(aligned(v->weight, 4) && v->row_bytes % 4U == 0, "Q8_0 chain product: weight rows must be 4-byte aligned");
+    STRIX_REQUIRE(aligned(v->codes, 16) && v->x_stride % 32U == 0 && v->x_stride >= v->in, "Q8_0 chain product: codes must be 16-byte aligned with x_stride a multiple of 32");
+    STRIX_REQUIRE(v->row_bytes >= v->in / 32U * kQ80Block && v->out_stride >= v->count && v->rows <= 65535U, "Q8_0 chain product: stride shorter than the row, or too many rows");
+    gemv_q8_0_a8_kernel<1, true, true><<<dim3((v->count + 7U) / 8U, v->rows), 256, 0, hs(stream)>>>(*v);
+    STRIX_LAUNCHED("gemv_q8_0_a8 chain");
+    return MI355_OK;
+}
+
+int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
+    STRIX_REQUIRE(v, "Q8_0 product: null view");
+    STRIX_REQUIRE(v->in % 32U == 0, "Q8_0 product width must be a multiple of 32");
+    if (v->rows == 0 || v->count == 0) return MI355_OK;
+    STRIX_REQUIRE(v->weight && v->codes && v->deltas && v->out, "Q8_0 product: null pointer");
+    STRIX_REQUIRE(aligned(v->weight, 2) && v->row_bytes % 2U == 0, "Q8_0 product: weight rows must be 2-byte aligned");
+    STRIX_REQUIRE(aligned(v->codes, 16) && v->x_stride % 32U == 0 && v->x_stride >= v->in, "Q8_0 product: codes must be 16-byte aligned with x_stride a multiple of 32");
+    STRIX_REQUIRE(v->row_bytes >= v->in / 32U * kQ80Block && v->out_stride >= v->count, "Q8_0 product: stride shorter than the row");
+    const uint32_t grid = (v->count + 7U) / 8U;
+    const bool dw = aligned(v->weight, 4) && v->row_bytes % 4U == 0;
+    hipStream_t st = hs(stream);
+    // up to RB activation rows share one sweep of a weight row; more rows are further blocks of the same launch (grid.y)
+    const auto launch = [&](auto rb_constant) {
+        constexpr int RB = decltype(rb_constant)::value;
+        const dim3 g(grid, (v->rows + RB - 1U) / RB);
+        if (dw) gemv_q8_0_a8_kernel<RB, true><<<g, 256, 0, st>>>(*v);
+        else gemv_q8_0_a8_kernel<RB, false><<<g, 256, 0, st>>>(*v);
+    };
+    STRIX_REQUIRE((v->rows + 15U) / 16U <= 65535U, "Q8_0 product: too many rows for one launch");
+    if (v->rows == 1U) launch(std::integral_constant<int, 1>{});
+    else if (v->rows == 2U) launch(std::integral_constant<int, 2>{});
+    else if (v->rows <= 4U) launch(std::integral_constant<int, 4>{});
+    else if (v->rows <= 8U) launch(std::integral_constant<int, 8>{});
+    else {
+        // Tiles of 64 weight rows x 64 activation rows where they fill the compute units, 32 weight rows (K split over twice the waves)
+        // where they do not; 32 activation rows for a batch that fits them. (4096 x 4096: 12 rows 13.1 us on the row sweep and 12.8 on the
+        // matrix cores, 16384 x 8192: 78 and 46 us; 8 rows 8.8 and 12.7 us.)
+        const uint64_t wide = static_cast<uint64_t>((v->count + 63U) / 64U) * ((v->rows + 63U) / 64U);
+        if (v->rows <= 32U) launch_gemm_q8_0<8, 1>(*v, dw, st);
+        else if (wide < compute_units()) launch_gemm_q8_0<8, 2>(*v, dw, st);
+        else launch_gemm_q8_0<4, 2>(*v, dw, st);
+    }
+    STRIX_LAUNCHED("gemv_q8_0_a8");
+    return MI355_OK;
+}
+
+}  // extern "C"

@@ -6,12 +6,11 @@
 
 #include <cmath>
 #include <cstdio>
-#include <atomic>
 #include <cstdlib>
 #include <cstring>
-#include <string>
 
 #include "device_math.hpp"
+#include "host_common.hpp"
 #include "q4k_rows.hpp"
 #include "q4k_blocks.hpp"
 #include "q4k_pairs.hpp"
@@ -26,25 +25,6 @@
 #include "route_early.hpp"
 
 namespace strix950 {
-
-// ======================================================================================================== host side
-thread_local std::string g_error;
-
-int32_t fail(int32_t code, const char* what) {
-    g_error = what;
-    return code;
-}
-int32_t hip_fail(hipError_t e, const char* what) {
-    g_error = std::string(what) + ": " + hipGetErrorString(e);
-    return MI355_E_HIP;
-}
-#define STRIX_REQUIRE(cond, what) do { if (!(cond)) return fail(MI355_E_INVALID_ARGUMENT, what); } while (0)
-#define STRIX_LAUNCHED(what) do { const hipError_t e_ = hipGetLastError(); if (e_ != hipSuccess) return hip_fail(e_, what); } while (0)
-
-inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
-inline hipStream_t hs(mi355_stream s) { return static_cast<hipStream_t>(s); }
-
-constexpr uint32_t kQ4kBlock = 144, kQ80Block = 34;
 
 // ======================================================================================================== block decode
 // One thread per output element. Q4_K: y = (d * sc) * q - (dmin * m), two products and one subtraction
@@ -158,114 +138,6 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_kernel(const float* x, const 
     __syncthreads();
     const float r = 1.0F / __builtin_sqrtf(partial[0] / static_cast<float>(n) + eps);
     for (uint32_t i = lane; i < n; i += lanes) yr[i] = w ? (xr[i] * r) * w[i] : xr[i] * r;
-}
-
-// One aligned group of 32 lanes per 32-value group; 8 groups per 256-thread block.
-// Reference: src/cpu/core/reference.cpp:35-55.
-// nan_delta: the dense A8 profile's rule for a group that holds a non-finite value (src/hip_q8_rows_gemv.hpp:1157-1161,1232-1250): its
-// delta is the canonical NaN 0x7fc00000 and its codes are 0, so that every product over the group is NaN.
-template <int KIND>
-__global__ __launch_bounds__(256) void quantize_a8_kernel(const uint8_t* x, uint64_t x_stride, uint32_t width, int8_t* codes,
-                                                          float* deltas, int32_t* sums, uint32_t* status, uint32_t nan_delta = 0) {
-    const uint32_t r = blockIdx.y, groups = width / 32U;
-    const uint32_t g = blockIdx.x * 8U + (threadIdx.x >> 5), j = threadIdx.x & 31U;
-    if (g >= groups) return;
-    const float v = load_activation<KIND>(x + r * x_stride, g * 32U + j);
-    const float amax = max32(__builtin_fabsf(v));
-    const bool tiny = amax > 0.0F && amax < 0x1p-119F;
-    const float delta = (amax == 0.0F || tiny) ? 1.0F : amax / 127.0F;
-    const int bad = or32_i(finite_f(v) ? 0 : 1);
-    const int code = (bad && nan_delta) ? 0 : a8_code(v, delta, tiny);
-    const int sum = sum32_i(code);
-    codes[static_cast<size_t>(r) * width + g * 32U + j] = static_cast<int8_t>(code);
-    if (j == 0) {
-        deltas[static_cast<size_t>(r) * groups + g] = (bad && nan_delta) ? __builtin_bit_cast(float, 0x7fc00000U) : delta;
-        if (sums) sums[static_cast<size_t>(r) * groups + g] = sum;
-        if (bad && status) atomicOr(&status[r], static_cast<uint32_t>(MI355_STATUS_NONFINITE_ACTIVATION));
-    }
-}
-
-// ======================================================================================================== Q8_0 x A8 GEMV
-// One aligned group of 32 lanes per output row: lane l owns the reference's accumulator lane l (groups g = l, l + 32,
-// ... ascending), then the tree32 butterfly. Up to RB activation rows share one sweep of the weight row.
-// Reference: src/cpu/core/reference.cpp:57-84, src/core/integer_math.hpp:11-13,43-47.
-// DW: the weight rows are 4-byte aligned. A block (34 bytes: fp16 scale, 32 codes) is then fetched as nine aligned dwords
-// (two 128-bit loads and one 32-bit load) around its codes and shifted into place, instead of seventeen 16-bit loads.
-// CHAIN (RB = 1): the row contract of the reference's dense A8 profile (src/hip_q8_rows_gemv.hpp:1155-1170; host statement
-// tests/dense_a8_small_reference_tests.cpp:93-104): acc = +0, then for the blocks in ascending order acc = fma(float(d_w) * delta,
-// float(dot), acc), and a NaN result is stored as 0x7fc00000. The lanes evaluate their blocks as before and leave every block's
-// (scale, dot) pair in LDS; lane 0 of the output's 32 lanes then walks them in order.
-constexpr uint32_t kGemvChainMaxGroups = 256;          // in <= 8192 (kDenseA8MaxWidth, src/hip_q8_rows_gemv.hpp:1176)
-typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-template <int RB, bool DW, bool CHAIN = false>
-__global__ __launch_bounds__(256) void gemv_q8_0_a8_kernel(mi355_q8a8_view v) {
-    __shared__ float2 chain_pairs[CHAIN ? 8 : 1][CHAIN ? kGemvChainMaxGroups : 1];
-    const uint32_t o = blockIdx.x * 8U + (threadIdx.x >> 5), l = threadIdx.x & 31U, row0 = blockIdx.y * RB;
-    if (o >= v.count) return;
-    const uint32_t groups = v.in / 32U;
-    const uint32_t nr = v.rows - row0 < static_cast<uint32_t>(RB) ? v.rows - row0 : static_cast<uint32_t>(RB);
-    const uint8_t* wrow = v.weight + static_cast<size_t>(o) * v.row_bytes;
-    float lane[RB];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) lane[r] = 0.0F;
-    // (unrolled: the loads of four of the lane's groups are in flight together; the accumulation order does not change)
-#pragma unroll 4
-    for (uint32_t g = l; g < groups; g += 32U) {
-        const unsigned short* b = reinterpret_cast<const unsigned short*>(wrow + static_cast<size_t>(g) * kQ80Block);
-        const float scale = half_bits_to_float(b[0]);
-        int w[8];
-        if constexpr (DW) {
-            const uint32_t c0 = g * kQ80Block + 2U, shift = c0 & 3U;          // first code byte: 0 or 2 past a dword boundary
-            const uint32_t* dw = reinterpret_cast<const uint32_t*>(wrow) + (c0 >> 2);
-            const u32x4_a4 lo4 = *reinterpret_cast<const u32x4_a4*>(dw), hi4 = *reinterpret_cast<const u32x4_a4*>(dw + 4);
-            const uint32_t last = dw[shift ? 8 : 7];                          // (an aligned block ends with its eighth dword)
-            const uint32_t d[9] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w, last};
-#pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(__builtin_amdgcn_alignbyte(d[i + 1], d[i], shift));
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(static_cast<uint32_t>(b[1 + 2 * i]) | (static_cast<uint32_t>(b[2 + 2 * i]) << 16));
-        }
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-            if (static_cast<uint32_t>(r) < nr) {
-                const int4* xc = reinterpret_cast<const int4*>(v.codes + static_cast<size_t>(row0 + r) * v.x_stride + g * 32U);
-                const int4 a = xc[0], c = xc[1];
-                int dot = 0;
-                dot = __builtin_amdgcn_sdot4(w[0], a.x, dot, false); dot = __builtin_amdgcn_sdot4(w[1], a.y, dot, false);
-                dot = __builtin_amdgcn_sdot4(w[2], a.z, dot, false); dot = __builtin_amdgcn_sdot4(w[3], a.w, dot, false);
-                dot = __builtin_amdgcn_sdot4(w[4], c.x, dot, false); dot = __builtin_amdgcn_sdot4(w[5], c.y, dot, false);
-                dot = __builtin_amdgcn_sdot4(w[6], c.z, dot, false); dot = __builtin_amdgcn_sdot4(w[7], c.w, dot, false);
-                const float xd = v.deltas[static_cast<size_t>(row0 + r) * (v.x_stride / 32U) + g];
-                if constexpr (CHAIN) chain_pairs[threadIdx.x >> 5][g] = make_float2(scale * xd, static_cast<float>(dot));
-                else lane[r] = lane[r] + static_cast<float>(dot) * (scale * xd);
-            }
-        }
-    }
-    if constexpr (CHAIN) {
-        // the pairs were written by lanes of this wave: program order of one wave's LDS accesses
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (l == 0) {
-            float acc = 0.0F;
-            for (uint32_t g = 0; g < groups; ++g) {
-                const float2 c = chain_pairs[threadIdx.x >> 5][g];
-                acc = __builtin_fmaf(c.x, c.y, acc);
-            }
-            v.out[static_cast<size_t>(row0) * v.out_stride + o] = acc != acc ? __builtin_bit_cast(float, 0x7fc00000U) : acc;
-        }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-        float p = lane[r];
-        p = p + xor16_f(p); p = p + xor8_f(p); p = p + xor4_f(p); p = p + xor2_f(p); p = p + xor1_f(p);
-        if (l == 0 && static_cast<uint32_t>(r) < nr) {
-            float* y = &v.out[static_cast<size_t>(row0 + r) * v.out_stride + o];
-            *y = v.accumulate ? *y + p : p;
-        }
-    }
 }
 
 // ======================================================================================================== router
@@ -1733,32 +1605,6 @@ __global__ __launch_bounds__(256) void swiglu_quantize_kernel(const float* gate,
     }
 }
 
-// A property of the current device, asked once per device ordinal (0 if the runtime cannot say).
-inline uint32_t device_property(hipDeviceAttribute_t what, std::atomic<uint32_t> (&known)[64]) {
-    int device = 0, value = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0) return 0;
-    if (device < 64) {
-        const uint32_t seen = known[device].load(std::memory_order_relaxed);
-        if (seen != 0) return seen;
-    }
-    if (hipDeviceGetAttribute(&value, what, device) != hipSuccess || value <= 0) return 0;
-    if (device < 64) known[device].store(static_cast<uint32_t>(value), std::memory_order_relaxed);
-    return static_cast<uint32_t>(value);
-}
-inline uint32_t compute_units() {
-    static std::atomic<uint32_t> known[64];
-    return device_property(hipDeviceAttributeMultiprocessorCount, known);
-}
-// LDS bytes of one compute unit
-inline uint32_t lds_per_unit() {
-    static std::atomic<uint32_t> known[64];
-    return device_property(hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, known);
-}
-// wavefronts of a launch that are all resident at once when each holds `lds_each` bytes of LDS
-inline uint64_t resident_waves(uint32_t lds_each) {
-    return static_cast<uint64_t>(compute_units()) * (lds_per_unit() / lds_each);
-}
-
 // ======================================================================================================== dispatch
 // Up to 4 (routed experts) or 8 (dense matrix) activation rows share one sweep of an expert's weights; an expert with
 // more assignments is swept again for the rest.
@@ -2136,86 +1982,12 @@ int32_t mi355_quantize_weight_rows(uint32_t type, const float* x, uint32_t n_row
     return MI355_OK;
 }
 
-int32_t mi355_quantize_a8(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
-                          int32_t* sums, uint32_t* status, mi355_stream stream) {
-    STRIX_REQUIRE(width % 32U == 0, "A8 activation width must be a multiple of 32");
-    STRIX_REQUIRE(kind <= MI355_INPUT_BF16, "A8: unknown input kind");
-    if (rows == 0 || width == 0) return MI355_OK;
-    STRIX_REQUIRE(x && codes && deltas, "A8: null pointer");
-    STRIX_REQUIRE(rows <= 65535U, "A8: at most 65535 rows per call");
-    const dim3 grid((width / 32U + 7U) / 8U, rows);
-    const uint8_t* xb = static_cast<const uint8_t*>(x);
-    if (kind == MI355_INPUT_F32) quantize_a8_kernel<0><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, sums, status);
-    else if (kind == MI355_INPUT_F16) quantize_a8_kernel<1><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, sums, status);
-    else quantize_a8_kernel<2><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, sums, status);
-    STRIX_LAUNCHED("quantize_a8");
-    return MI355_OK;
-}
-
-int32_t mi355_dense_a8_quantize(const void* x, uint32_t kind, uint32_t rows, uint32_t width, uint64_t x_stride, int8_t* codes, float* deltas,
-                                mi355_stream stream) {
-    STRIX_REQUIRE(width % 32U == 0, "dense A8 activation width must be a multiple of 32");
-    STRIX_REQUIRE(kind <= MI355_INPUT_BF16, "dense A8: unknown input kind");
-    if (rows == 0 || width == 0) return MI355_OK;
-    STRIX_REQUIRE(x && codes && deltas, "dense A8: null pointer");
-    STRIX_REQUIRE(rows <= 65535U, "dense A8: at most 65535 rows per call");
-    const dim3 grid((width / 32U + 7U) / 8U, rows);
-    const uint8_t* xb = static_cast<const uint8_t*>(x);
-    if (kind == MI355_INPUT_F32) quantize_a8_kernel<0><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, nullptr, nullptr, 1U);
-    else if (kind == MI355_INPUT_F16) quantize_a8_kernel<1><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, nullptr, nullptr, 1U);
-    else quantize_a8_kernel<2><<<grid, 256, 0, hs(stream)>>>(xb, x_stride, width, codes, deltas, nullptr, nullptr, 1U);
-    STRIX_LAUNCHED("dense A8 quantize");
-    return MI355_OK;
-}
-
-int32_t mi355_gemv_q8_0_a8_chain(const mi355_q8a8_view* v, mi355_stream stream) {
-    STRIX_REQUIRE(v, "Q8_0 chain product: null view");
-    STRIX_REQUIRE(v->in % 64U == 0 && v->in <= 32U * kGemvChainMaxGroups, "Q8_0 chain product: width must be a multiple of 64, at most 8192");   // dense_a8_width, src/hip_q8_rows_gemv.hpp:1184
-    STRIX_REQUIRE(!v->accumulate, "Q8_0 chain product: the chain starts at +0 (no accumulate)");
-    if (v->rows == 0 || v->count == 0) return MI355_OK;
-    STRIX_REQUIRE(v->weight && v->codes && v->deltas && v->out, "Q8_0 chain product: null pointer");
-    STRIX_REQUIRE(aligned(v->weight, 4) && v->row_bytes % 4U == 0, "Q8_0 chain product: weight rows must be 4-byte aligned");
-    STRIX_REQUIRE(aligned(v->codes, 16) && v->x_stride % 32U == 0 && v->x_stride >= v->in, "Q8_0 chain product: codes must be 16-byte aligned with x_stride a multiple of 32");
-    STRIX_REQUIRE(v->row_bytes >= v->in / 32U * kQ80Block && v->out_stride >= v->count && v->rows <= 65535U, "Q8_0 chain product: stride shorter than the row, or too many rows");
-    gemv_q8_0_a8_kernel<1, true, true><<<dim3((v->count + 7U) / 8U, v->rows), 256, 0, hs(stream)>>>(*v);
-    STRIX_LAUNCHED("gemv_q8_0_a8 chain");
-    return MI355_OK;
-}
-
 int32_t mi355_rmsnorm_f32(const float* x, const float* w, uint32_t n, float eps, float* y, uint32_t rows, mi355_stream stream) {
     if (rows == 0 || n == 0) return MI355_OK;
     STRIX_REQUIRE(x && y, "rmsnorm: null pointer");
     STRIX_REQUIRE(rows <= 0x7fffffffU, "rmsnorm: too many rows");
     rmsnorm_f32_kernel<<<rows, n >= 512U ? 256 : 128, 0, hs(stream)>>>(x, w, n, eps, y);
     STRIX_LAUNCHED("rmsnorm_f32");
-    return MI355_OK;
-}
-
-int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
-    STRIX_REQUIRE(v, "Q8_0 product: null view");
-    STRIX_REQUIRE(v->in % 32U == 0, "Q8_0 product width must be a multiple of 32");
-    if (v->rows == 0 || v->count == 0) return MI355_OK;
-    STRIX_REQUIRE(v->weight && v->codes && v->deltas && v->out, "Q8_0 product: null pointer");
-    STRIX_REQUIRE(aligned(v->weight, 2) && v->row_bytes % 2U == 0, "Q8_0 product: weight rows must be 2-byte aligned");
-    STRIX_REQUIRE(aligned(v->codes, 16) && v->x_stride % 32U == 0 && v->x_stride >= v->in, "Q8_0 product: codes must be 16-byte aligned with x_stride a multiple of 32");
-    STRIX_REQUIRE(v->row_bytes >= v->in / 32U * kQ80Block && v->out_stride >= v->count, "Q8_0 product: stride shorter than the row");
-    const uint32_t grid = (v->count + 7U) / 8U;
-    const bool dw = aligned(v->weight, 4) && v->row_bytes % 4U == 0;
-    hipStream_t st = hs(stream);
-    // up to RB activation rows share one sweep of a weight row; more rows are further blocks of the same launch (grid.y)
-    const auto launch = [&](auto rb_constant) {
-        constexpr int RB = decltype(rb_constant)::value;
-        const dim3 g(grid, (v->rows + RB - 1U) / RB);
-        if (dw) gemv_q8_0_a8_kernel<RB, true><<<g, 256, 0, st>>>(*v);
-        else gemv_q8_0_a8_kernel<RB, false><<<g, 256, 0, st>>>(*v);
-    };
-    STRIX_REQUIRE((v->rows + 15U) / 16U <= 65535U, "Q8_0 product: too many rows for one launch");
-    if (v->rows == 1U) launch(std::integral_constant<int, 1>{});
-    else if (v->rows == 2U) launch(std::integral_constant<int, 2>{});
-    else if (v->rows <= 4U) launch(std::integral_constant<int, 4>{});
-    else if (v->rows <= 8U) launch(std::integral_constant<int, 8>{});
-    else launch(std::integral_constant<int, 16>{});            // (32 rows per sweep measured slower: 5.0 vs 4.05 ms on 4096 rows)
-    STRIX_LAUNCHED("gemv_q8_0_a8");
     return MI355_OK;
 }
 

@@ -1,0 +1,81 @@
+"""The Q8_0 linear operators over their ranges: the A8 image of rows of every width and the product of many rows on the matrix cores,
+bit for bit against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+import orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("rows,width", [(1, 32), (3, 96), (2, 2048), (5, 8192), (2, 8224), (70, 1056)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_a8_image_of_rows(strix, rows, width, dtype):
+    gen = torch.Generator().manual_seed(rows * width)
+    x = torch.randn((rows, width), generator=gen)
+    x[0, :32] = 0.0
+    x[-1, -32:] *= 2.0 ** -125
+    x = x.to(dtype)
+    x[rows // 2, width // 2] = float("inf")
+    padded = torch.zeros((rows, width + 3), dtype=dtype)       # rows that are not 16-byte aligned: the unvectorised form
+    padded[:, 1:1 + width] = x
+    want = [orc.quantize_a8(r[None]) for r in x.float().numpy()]
+    for view in (x.cuda(), padded.cuda()[:, 1:1 + width]):
+        codes, deltas, sums, status = strix.quantize_a8(view)
+        assert status.cpu().tolist() == [strix.STATUS_NONFINITE_ACTIVATION if r == rows // 2 else 0 for r in range(rows)]
+        for r, (c, d, s, _) in enumerate(want):
+            if r == rows // 2:
+                continue
+            assert np.array_equal(codes[r].cpu().numpy(), c[0]) and np.array_equal(bits(deltas[r].cpu().numpy()), bits(d[0]))
+            assert np.array_equal(sums[r].cpu().numpy(), s[0])
+
+
+# rows around the matrix-core form's tiles of 32 and 64, outputs around its tiles of 32 and 64, groups around its chunks of 32 (odd
+# numbers of chunks, a last chunk of one group), one width whose rows are only 2-byte aligned
+@pytest.mark.parametrize("rows,width,count", [(16, 1024, 70), (17, 32, 1), (32, 1056, 33), (33, 2432, 31), (64, 1024, 65), (65, 2048, 96), (130, 992, 129),
+                                              (500, 64, 513), (257, 4096, 320), (40, 8192, 40), (1000, 1088, 1100)])
+def test_products_of_many_rows(strix, rows, width, count):
+    rng = np.random.default_rng(rows + width)
+    w = orc.quantize_rows(orc.Q8_0, (rng.standard_normal((count, width)) * 0.02).astype(np.float32))
+    codes, deltas, _, _ = orc.quantize_a8(rng.standard_normal((rows, width)).astype(np.float32))
+    want, _ = orc.gemv_q8_0_a8(w, codes, deltas, width, count, threads=8)
+    got = strix.gemv_q8_0_a8(dev(w), dev(codes), dev(deltas), width, count).cpu().numpy()
+    assert np.array_equal(bits(got), bits(want))
+    shifted = torch.zeros(w.size + 2, dtype=torch.uint8, device="cuda")      # weights at a pointer that is only 2-byte aligned
+    shifted[2:] = dev(w).reshape(-1)
+    out = torch.full((rows, count + 5), 3.0, device="cuda")
+    strix.gemv_q8_0_a8(shifted[2:], dev(codes), dev(deltas), width, count, out=out, accumulate=True)
+    got = out.cpu().numpy()
+    assert np.array_equal(bits(got[:, :count]), bits(want + np.float32(3.0))) and np.all(got[:, count:] == 3.0)
+
+
+def test_products_of_full_range_codes_and_wide_factors(strix):
+    """Weight bytes of the whole int8 range and scales over many binades: the largest dots (32 * 128 * 127) and subnormal factors."""
+    rng = np.random.default_rng(3)
+    rows, width, count = 70, 1536, 96
+    w = rng.integers(0, 256, (count, width // 32, 34), dtype=np.uint8)
+    w[..., 1] = rng.integers(0, 0x78, w[..., 1].shape)         # finite scales, subnormal ones among them
+    w[:4, :, 2:] = 0x80
+    codes = rng.integers(-127, 128, (rows, width)).astype(np.int8)
+    codes[:3] = -127
+    deltas = np.exp2(rng.uniform(-120, 10, (rows, width // 32))).astype(np.float32)
+    want, _ = orc.gemv_q8_0_a8(w.reshape(count, -1), codes, deltas, width, count, threads=8)
+    got = strix.gemv_q8_0_a8(dev(w.reshape(count, -1)), dev(codes), dev(deltas), width, count).cpu().numpy()
+    assert np.array_equal(bits(got), bits(want))
