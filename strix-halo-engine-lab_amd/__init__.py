@@ -206,6 +206,7 @@ def device_bytes(t):
 
 
 _lib = None
+_ops = None
 
 
 def lib():
@@ -259,7 +260,7 @@ def lib():
 
 
 EXPORTS = ["mi355_last_error", "mi355_version", "mi355_numerical_identity", "mi355_dequantize_rows",
-           "mi355_quantize_weight_rows", "mi355_quantize_a8", "mi355_gemv_q8_0_a8", "mi355_dense_a8_quantize", "mi355_gemv_q8_0_a8_chain", "mi355_moe_route",
+           "mi355_quantize_weight_rows", "mi355_quantize_a8", "mi355_quantize_a8_fresh", "mi355_gemv_q8_0_a8", "mi355_dense_a8_quantize", "mi355_gemv_q8_0_a8_chain", "mi355_moe_route",
            "mi355_moe_plan_words", "mi355_moe_enqueue_prologue", "mi355_moe_enqueue_csr", "mi355_moe_enqueue_project",
            "mi355_moe_enqueue_down", "mi355_moe_enqueue_merge", "mi355_moe_enqueue_combine", "mi355_moe_enqueue", "mi355_moe_enqueue_layer", "mi355_moe_enqueue_layer_front", "mi355_moe_enqueue_layer_back", "mi355_debug_early_route_perturb", "mi355_debug_down_merge_flat", "mi355_moe_enqueue_layer_normed", "mi355_moe_enqueue_layer_static", "mi355_static_workspace_prepare", "mi355_moe_enqueue_prefill_f16", "mi355_moe_enqueue_prefill_rows_f16", "mi355_moe_prefill_f16_workspace_bytes",
            "mi355_swiglu_quantize", "mi355_rmsnorm_f32", "mi355_shared_gate", "mi355_a8_validate", "mi355_a8_validate_down", "mi355_a8_enqueue_probe", "mi355_a8_enqueue_serial_prologue_probe", "mi355_a8_enqueue_quantize_only",
@@ -317,16 +318,30 @@ def quantize_weight_rows(qtype, x):
     return out
 
 
+def _native():
+    """The native wrappers (host/torch_ops.cpp), loaded beside the library they link."""
+    global _ops
+    if _ops is None:
+        lib()
+        from importlib import machinery, util
+        path = os.path.join(HERE, "_torch_ops.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
+        spec = util.spec_from_file_location("_torch_ops", path, loader=machinery.ExtensionFileLoader("_torch_ops", path))
+        module = util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _ops = module
+    return _ops
+
+
+def _result(r):
+    if type(r) is int:
+        check(r)
+    return r
+
+
 def quantize_a8(x, want_sums=True):
-    assert x.dim() == 2 and x.stride(1) == 1
-    rows, width = x.shape
-    codes = torch.empty((rows, width), dtype=torch.int8, device=x.device)
-    deltas = torch.empty((rows, width // 32), dtype=torch.float32, device=x.device)
-    sums = torch.empty((rows, width // 32), dtype=torch.int32, device=x.device) if want_sums else None
-    status = torch.zeros(rows, dtype=torch.int32, device=x.device)
-    check(lib().mi355_quantize_a8(_p(x), input_kind(x), rows, width, C.c_uint64(x.stride(0) * x.element_size()), _p(codes),
-                                  _p(deltas), _p(sums), _p(status), _stream()))
-    return codes, deltas, sums, status
+    return _result((_ops or _native()).quantize_a8(x, want_sums))
 
 
 def rmsnorm_f32(x, weight=None, eps=1e-6):
@@ -348,13 +363,7 @@ def shared_gate(x, scalar_weight, exp_kind=EXP_GFX1151, out=None):
 
 
 def gemv_q8_0_a8(weight, codes, deltas, n_in, count, out=None, accumulate=False, row_bytes_=None, out_stride=None):
-    rows = codes.shape[0]
-    if out is None:
-        out = torch.zeros((rows, count), dtype=torch.float32, device=codes.device)
-    v = Q8a8View(weight.data_ptr(), codes.data_ptr(), deltas.data_ptr(), out.data_ptr(),
-                 row_bytes_ or n_in // 32 * Q8_0_BLOCK, n_in, count, rows, codes.shape[1], out_stride or out.shape[1], int(accumulate))
-    check(lib().mi355_gemv_q8_0_a8(C.byref(v), _stream()))
-    return out
+    return _result((_ops or _native()).gemv_q8_0_a8(weight, codes, deltas, n_in, count, out, accumulate, row_bytes_ or 0, out_stride or 0))
 
 
 def dense_a8_quantize(x):
