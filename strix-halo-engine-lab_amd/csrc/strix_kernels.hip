@@ -11,6 +11,7 @@
 
 #include "device_math.hpp"
 #include "host_common.hpp"
+#include "launchers.hpp"
 #include "q4k_rows.hpp"
 #include "q4k_blocks.hpp"
 #include "q4k_pairs.hpp"
@@ -180,21 +181,6 @@ __host__ __device__ constexpr uint32_t plan_words_total(uint32_t experts, uint32
     return plan_items_at(experts, assignments) + 4U * plan_item_capacity(assignments);
 }
 
-// Router logits for batches above the decode bound: blocks of 8 experts x 8 rows.
-template <int KIND>
-__global__ __launch_bounds__(64) void route_logits_kernel(RouteArgs a) {
-    __shared__ RouteLds lds;
-    const uint32_t neb = (a.p.experts + 7U) / 8U;
-    route_logits_block<KIND>(lds, a, (blockIdx.x % neb) * 8U, (blockIdx.x / neb) * 8U);
-}
-
-// Router logits of large batches in the ascending fma chain order: 64 rows x 64 experts per 256-thread workgroup.
-template <int KIND>
-__global__ __launch_bounds__(256, 2) void route_batch_kernel(RouteArgs a) {
-    __shared__ __attribute__((aligned(16))) BatchTiles lds;
-    route_batch_block<KIND>(lds, a, blockIdx.y * kBatchTile, blockIdx.x * kBatchTile);
-}
-
 // A8 prologue block qb of a fused decode launch (src/cpu/core/reference.cpp:35-55): two groups of 32 at a time, 8 groups per
 // block; the last of a row's blocks publishes the row's status word. scratch: 256 floats of LDS (fused RMSNorm only).
 // Row r counts its finished blocks in ticket[r * stride] and collects its flags in flags[r * stride]. LINES: the words are reached
@@ -321,12 +307,6 @@ __global__ __launch_bounds__(64) void route_decode_kernel(RouteArgs a) {
     } else {
         a8_prologue_block<KIND, NORM>(a, bid - a.route_blocks, tickets + 16U, tickets + 128U, 1U, sel_p);
     }
-}
-
-// softmax / top-k / weights, one row per one-wave block (the plain router).
-__global__ __launch_bounds__(64) void route_select_kernel(RouteArgs a) {
-    __shared__ __attribute__((aligned(16))) float sel_p[kRouteMaxExperts];
-    route_select_row(sel_p, a, blockIdx.x);
 }
 
 // ======================================================================================================== expert plan
@@ -2006,7 +1986,7 @@ int32_t check_route(const mi355_route_policy* p, const void* x, uint32_t kind, u
     return MI355_OK;
 }
 // Logits of every (row, expert) into a.scores. Decode batches: one block per (row, 8 experts), plus a.quant_blocks blocks
-// in the fused form; larger batches: one block per (8 rows, 8 experts).
+// in the fused form; larger batches: route.hip.
 void launch_route_logits(RouteArgs& a, hipStream_t st) {
     const uint32_t neb = (a.p.experts + 7U) / 8U;
     if (a.rows <= kFusedMaxRows) {
@@ -2019,17 +1999,7 @@ void launch_route_logits(RouteArgs& a, hipStream_t st) {
         } else if (a.kind == MI355_INPUT_F32) route_decode_kernel<0><<<blocks, 64, 0, st>>>(a);
         else if (a.kind == MI355_INPUT_F16) route_decode_kernel<1><<<blocks, 64, 0, st>>>(a);
         else route_decode_kernel<2><<<blocks, 64, 0, st>>>(a);
-    } else if (a.p.logits_order == MI355_LOGITS_FMA_ASCENDING && (a.rows + kBatchTile - 1U) / kBatchTile <= 65535U) {
-        const dim3 grid((a.p.experts + kBatchTile - 1U) / kBatchTile, (a.rows + kBatchTile - 1U) / kBatchTile);
-        if (a.kind == MI355_INPUT_F32) route_batch_kernel<0><<<grid, 256, 0, st>>>(a);
-        else if (a.kind == MI355_INPUT_F16) route_batch_kernel<1><<<grid, 256, 0, st>>>(a);
-        else route_batch_kernel<2><<<grid, 256, 0, st>>>(a);
-    } else {
-        a.route_blocks = neb * ((a.rows + 7U) / 8U);
-        if (a.kind == MI355_INPUT_F32) route_logits_kernel<0><<<a.route_blocks, 64, 0, st>>>(a);
-        else if (a.kind == MI355_INPUT_F16) route_logits_kernel<1><<<a.route_blocks, 64, 0, st>>>(a);
-        else route_logits_kernel<2><<<a.route_blocks, 64, 0, st>>>(a);
-    }
+    } else launch_route_batch_logits(a, st);
 }
 }  // namespace
 
@@ -2041,7 +2011,7 @@ int32_t mi355_moe_route(const mi355_route_policy* p, const void* x, uint32_t kin
     a.p = *p; a.x = static_cast<const uint8_t*>(x); a.kind = kind; a.x_stride = x_stride; a.rows = rows; a.hidden = hidden;
     a.wr = wr; a.bias = bias; a.ids = ids; a.weights = weights; a.scores = scores;
     launch_route_logits(a, hs(stream));
-    route_select_kernel<<<rows, 64, 0, hs(stream)>>>(a);
+    launch_route_select(a, hs(stream));
     STRIX_LAUNCHED("moe_route");
     return MI355_OK;
 }

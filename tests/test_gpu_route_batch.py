@@ -1,0 +1,38 @@
+"""The router of batches past the decode sizes (its chains run on the fp32 matrix cores), bit for bit against the CPU oracle."""
+import numpy as np
+import pytest
+import torch
+
+import orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def bits(a):
+    return np.ascontiguousarray(a, np.float32).view(np.uint32)
+
+
+# rows and experts around the tiles of 16 and the workgroups of 64 experts; features around the blocks of 32 and the rings of 4 and 8
+# blocks (4112 rows x 64 experts: more workgroups than compute units, the short ring)
+@pytest.mark.parametrize("rows,experts,hidden,top_k", [(17, 5, 32, 2), (32, 16, 96, 4), (33, 130, 256, 8), (100, 63, 288, 6), (18, 300, 2080, 16), (64, 65, 4064, 8),
+                                                       (4112, 64, 160, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_logits_of_a_batch(strix, rows, experts, hidden, top_k, dtype):
+    gen = torch.Generator().manual_seed(rows + experts + hidden)
+    x = torch.randn((rows, hidden), generator=gen).to(dtype)
+    w = torch.randn((experts, hidden), generator=gen) * 0.05
+    x[0, ::3] *= 2.0 ** -20                      # subnormal halves; products over many binades
+    w[0] *= 2.0 ** -120
+    bias = torch.randn(experts, generator=gen) if experts % 2 else None
+    ids, weights, scores = strix.route(x.cuda(), w.cuda(), top_k, bias=None if bias is None else bias.cuda())
+    ids_ref, w_ref, s_ref, _ = orc.route(x.float().numpy(), w.numpy(), top_k, bias=None if bias is None else bias.numpy())
+    assert np.array_equal(bits(scores.cpu().numpy()), bits(s_ref))
+    assert np.array_equal(ids.cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(bits(weights.cpu().numpy()), bits(w_ref))
