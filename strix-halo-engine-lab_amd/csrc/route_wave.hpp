@@ -315,19 +315,24 @@ template <int N>
 __device__ __forceinline__ void chain_wait() { __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8)); }      // (and every LDS read returned: the next copy reuses a slot this wave has read)
 
 // Logits of experts [e0, e0 + 8) for one row -> scores[row][expert] (+ bias), stored for readers in other workgroups of
-// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects.
+// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects. NORM: the row's norm factor is computed here, in the fourth
+// slot, while the first three chunks are on their way.
 template <int KIND, bool NORM = false>
-__device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slots)[4], const RouteArgs& a, uint32_t row, uint32_t e0, float r = 1.0F) {
+__device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slots)[4], const RouteArgs& a, uint32_t row, uint32_t e0) {
     constexpr uint32_t NI = chain_copies<KIND, NORM>();
     const uint32_t lane = threadIdx.x & 63U, chunks = (a.hidden + kChainChunk - 1U) / kChainChunk;
     const bool butterfly = a.p.logits_order == MI355_LOGITS_LANE32_BUTTERFLY;
     const uint32_t el = lane & 7U;                      // chain form: the lane's expert
     const uint32_t bh = lane >> 5, bl = lane & 31U;     // butterfly form: experts bh, bh + 2, bh + 4, bh + 6; partial sum bl
     float acc = 0.0F, part[4] = {0.0F, 0.0F, 0.0F, 0.0F};
-    chain_publish();      // a caller may have used slot memory as scratch (the norm factor): those LDS operations are complete before any copy
 #pragma unroll
     for (uint32_t s = 0; s < 3U; ++s)
         if (s < chunks) chain_start<KIND, NORM>(*slots[s], a, row, e0, s * kChainChunk);
+    float r = 1.0F;
+    if constexpr (NORM) {
+        r = row_norm_factor<KIND>(reinterpret_cast<float*>(slots[3]), a.x + row * a.x_stride, a.hidden, a.norm_eps);
+        chain_publish();      // the scratch reads are complete before the ring reaches the fourth slot
+    }
     for (uint32_t c0 = 0; c0 < chunks; c0 += 4U) {
 #pragma unroll
         for (uint32_t s = 0; s < 4U; ++s) {
@@ -343,18 +348,15 @@ __device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slot
                 chain_widen<KIND, NORM>(slot, r, a.norm_w != nullptr);
                 const uint32_t kc = a.hidden - c * kChainChunk < kChainChunk ? a.hidden - c * kChainChunk : kChainChunk;
                 if (!butterfly) {
-                    if (kc == kChainChunk) {      // full chunk: straight-line code, operands fetched 16 features ahead
-                        ChainStep A, B;
-                        chain_load(A, slot, el, 0);
+                    if (kc == kChainChunk) {      // full chunk: straight-line code, operands fetched 48 features ahead
+                        ChainStep S[4];
 #pragma unroll
-                        for (uint32_t k = 0; k < kChainChunk; k += 32U) {     // the barriers pin "fetch next, then chain"
-                            chain_load(B, slot, el, k + 16U);
+                        for (uint32_t i = 0; i < 3U; ++i) chain_load(S[i], slot, el, 16U * i);
+#pragma unroll
+                        for (uint32_t i = 0; i < kChainChunk / 16U; ++i) {    // the barriers pin "fetch, then chain"
+                            if (i + 3U < kChainChunk / 16U) chain_load(S[(i + 3U) & 3U], slot, el, 16U * (i + 3U));
                             __builtin_amdgcn_sched_barrier(0);
-                            acc = chain_run(A, acc);
-                            __builtin_amdgcn_sched_barrier(0);
-                            if (k + 32U < kChainChunk) chain_load(A, slot, el, k + 32U);
-                            __builtin_amdgcn_sched_barrier(0);
-                            acc = chain_run(B, acc);
+                            acc = chain_run(S[i & 3U], acc);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     } else {                      // the last, partial chunk of the row

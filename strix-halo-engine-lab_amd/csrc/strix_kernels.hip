@@ -256,7 +256,7 @@ __global__ __launch_bounds__(64) void route_decode_kernel(RouteArgs a) {
     __shared__ uint32_t flag;
     ChainSlotT<NORM>* const slots[4] = {&slot0, &slot1, &slot2, &slot3};
     // the scratch of the row's norm factor and of the select lives in the fourth slot, which the ring first fills after the norm
-    // factor is known and which is free again once the chain has run: LDS per workgroup stays under half a compute unit's, so a
+    // factor is known and which is free again once the chain has run (every copy into it awaited): LDS per workgroup stays under half a compute unit's, so a
     // launch of more one-wave workgroups than compute units (16 rows x 160 experts: 320) still runs in one round (61 -> 32 us)
     static_assert(sizeof(ChainSlotT<NORM>) >= kRouteMaxExperts * sizeof(float), "select scratch");
     float* const sel_p = reinterpret_cast<float*>(&slot3);
@@ -264,9 +264,7 @@ __global__ __launch_bounds__(64) void route_decode_kernel(RouteArgs a) {
     uint32_t* tickets = a.plan ? a.plan + kPlanTicketsAt : nullptr;
     if (bid < a.route_blocks) {
         const uint32_t row = bid / neb;
-        float r = 1.0F;
-        if constexpr (NORM) r = row_norm_factor<KIND>(sel_p, a.x + row * a.x_stride, a.hidden, a.norm_eps);
-        route_chain_block<KIND, NORM>(slots, a, row, (bid % neb) * 8U, r);
+        route_chain_block<KIND, NORM>(slots, a, row, (bid % neb) * 8U);
         if (!a.plan) return;
         // hand-off between workgroups: the wave's logit stores happen before the barrier, the barrier before lane 0's
         // ticket increment, which releases them at device scope; the workgroup that takes the row's last ticket acquires with
