@@ -1,5 +1,7 @@
 // Launches whose kernels live in translation units of their own (they compile in parallel).
 #pragma once
+#include "prefill_args.hpp"
+#include "q4k_rows.hpp"
 #include "route_wave.hpp"
 
 namespace strix950 {
@@ -7,5 +9,15 @@ namespace strix950 {
 // route.hip: logits of a batch past the decode sizes into a.scores; softmax, selection and weights of every row of a.scores
 void launch_route_batch_logits(const RouteArgs& a, hipStream_t st);
 void launch_route_select(const RouteArgs& a, hipStream_t st);
+
+// prefill.hip: sub-block sums of the input rows, gate / up + SwiGLU and down rows of a planned batch. `a` holds everything but the
+// products' own fields (weights, strides, k, features, tiles, units).
+void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, uint32_t items_at, uint32_t order_at, hipStream_t st);
+
+// q4k_mma.hip: Q4_K experts on the int8 matrix cores. dense: the rows of a one-expert batch (0: planned items); width: the most rows an
+// item (or the dense batch) holds. The last leaves the raw gate and up values of a dense batch of at most 16 rows.
+void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st);
+void launch_mma_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st);
+void launch_mma_gate_up_rows(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, hipStream_t st);
 
 }  // namespace strix950

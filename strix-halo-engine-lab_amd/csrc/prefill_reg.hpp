@@ -25,12 +25,13 @@
 
 namespace strix950 {
 
-constexpr uint32_t kRgTokens = 128, kRgThreads = 512, kRgStageBytes = kRgTokens * 128U;   // one plane of one stage: 128 rows x 64 halves
-
-// Number of vector-memory operations a wave issues in stage p (= stage % 4) of every super-block: the token copies of the
+// Token copies a wave issues per stage: one 1 KB copy per plane (MODE 1: h hi and lo) and 8 WAVES rows of the live token tiles.
+template <int MODE, uint32_t WAVES> __host__ __device__ constexpr uint32_t rg_token_ops(uint32_t live) {
+    return (MODE == 1 ? 2U : 1U) * ((32U * live + 8U * WAVES - 1U) / (8U * WAVES));
+}
+// Number of vector-memory operations a wave issues in stage p (= stage % 4) of every super-block: the nt token copies of the
 // stage three ahead, one quant fetch, and the header fetch (p = 0) or the sums copy (p = 1).
-template <int MODE> __host__ __device__ constexpr uint32_t rg_token_ops() { return MODE == 1 ? 4U : 2U; }
-template <int MODE> __host__ __device__ constexpr uint32_t rg_stage_ops(uint32_t p) { return rg_token_ops<MODE>() + 1U + (p < 2U ? 1U : 0U); }
+__host__ __device__ constexpr uint32_t rg_stage_ops(uint32_t nt, uint32_t p) { return nt + 1U + (p < 2U ? 1U : 0U); }
 
 // copy16_to_lds with the LDS address (lane 0's destination) already a scalar
 __device__ __forceinline__ void copy16_to_lds_at(const uint8_t* src, uint32_t lds_at) {
@@ -39,15 +40,18 @@ __device__ __forceinline__ void copy16_to_lds_at(const uint8_t* src, uint32_t ld
 
 template <int N> __device__ __forceinline__ void rg_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-template <int MODE>
-__global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, uint32_t items_at, uint32_t order_at) {
-    constexpr uint32_t PLANES = MODE == 1 ? 2U : 1U, NT = rg_token_ops<MODE>();
-    __shared__ __attribute__((aligned(16))) uint8_t tok0[PLANES * kRgStageBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t tok1[PLANES * kRgStageBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t tok2[PLANES * kRgStageBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t tok3[PLANES * kRgStageBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t s_tile_mem[2][kRgTokens * 64U];        // [token][hi 16 | lo 16] sums of 16 sub-blocks
-    __shared__ float part_sum[8][kRgTokens];                                               // MODE 0 epilogue: a wave's 16-feature sums of h
+// WAVES, TOKENS: 8 waves over 128 tokens (one workgroup per compute unit) or 4 waves over 64 (three or two of them).
+template <int MODE, uint32_t WAVES, uint32_t TOKENS>
+__global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs a, uint32_t items_at, uint32_t order_at) {
+    static_assert(TOKENS == 16U * WAVES, "one sums copy per wave, a token copy of 8 rows per wave and part");
+    constexpr uint32_t PLANES = MODE == 1 ? 2U : 1U, TILES = TOKENS / 32U, PART_ROWS = 8U * WAVES;
+    constexpr uint32_t SUBS = kPfTile / TOKENS, STAGE = TOKENS * 128U;                     // one plane of one stage: TOKENS rows x 64 halves
+    __shared__ __attribute__((aligned(16))) uint8_t tok0[PLANES * STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t tok1[PLANES * STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t tok2[PLANES * STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t tok3[PLANES * STAGE];
+    __shared__ __attribute__((aligned(16))) uint8_t s_tile_mem[2][TOKENS * 64U];           // [token][hi 16 | lo 16] sums of 16 sub-blocks
+    __shared__ float part_sum[WAVES][TOKENS];                                              // MODE 0 epilogue: a wave's 16-feature sums of h
     pf_lds* const tok_stage[4] = {(pf_lds*)tok0, (pf_lds*)tok1, (pf_lds*)tok2, (pf_lds*)tok3};
     pf_lds* const s_tile = (pf_lds*)s_tile_mem;
 
@@ -59,30 +63,40 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
     const uint32_t last_group = (blocks + 1U) / 2U - 1U;
     const size_t sum_row = pf_sum_row_bytes(a.k);
 
-    for (uint32_t unit = blockIdx.x; unit < a.units; unit += gridDim.x) {
-    const uint32_t xcd = unit & 7U, q = unit >> 3;
-    const uint32_t item_index = (q / a.tiles) * 8U + xcd, tile = q % a.tiles;
+    // Wide: the tiles of an item run on one XCD, whose L2 then holds its token rows. Narrow: few rows per item, whose units differ in
+    // length more than their token rows cost: an item's tiles go round the XCDs (of the items that were made), and an item of more rows
+    // than TOKENS is as many units, the first of every item first.
+    const uint32_t units = SUBS == 1U ? a.units : a.plan[4] * a.tiles;
+    for (uint32_t at = blockIdx.x; at < SUBS * units; at += gridDim.x) {
+    const uint32_t sub = SUBS == 1U ? 0U : at / units, unit = at - sub * units, q = unit >> 3;
+    const uint32_t item_index = SUBS == 1U ? (q / a.tiles) * 8U + (unit & 7U) : unit / a.tiles, tile = (SUBS == 1U ? q : unit) % a.tiles;
     if (item_index >= a.items) continue;
     const uint4 item = *reinterpret_cast<const uint4*>(a.plan + items_at + 4U * item_index);
-    const uint32_t e = item.x, begin = item.y, count = item.z - item.y;
-    if (count == 0) continue;
+    const uint32_t e = item.x, begin = item.y + sub * TOKENS;
+    if (begin >= item.z) continue;
+    const uint32_t count = item.z - begin < TOKENS ? item.z - begin : TOKENS;
 
     // ---- the lane's weight row
     uint32_t feature;                                  // MODE 0: gate (n31 < 16) / up feature; MODE 1: output column
     const uint8_t* wbase = a.wa;
-    if (MODE == 0) { feature = tile * 128U + 16U * wave + (n31 & 15U); if (n31 & 16U) wbase = a.wb; }
-    else feature = tile * 256U + 32U * wave + n31;
+    if (MODE == 0) { feature = tile * (16U * WAVES) + 16U * wave + (n31 & 15U); if (n31 & 16U) wbase = a.wb; }
+    else feature = tile * (32U * WAVES) + 32U * wave + n31;
     const uint8_t* wrow = wbase + static_cast<size_t>(e) * a.expert_stride + static_cast<size_t>(feature) * a.row_stride;
 
-    // ---- token copies: copy i of a stage moves tile rows 8 (8 i + wave) .. + 8 of plane i / 2 (MODE 1); lane = (row % 8, slot)
-    const uint8_t* tsrc[NT];
+    // ---- token copies: part i of a stage moves tile rows PART_ROWS i + 8 wave .. + 8 (of both planes: MODE 1); lane = (row % 8, slot)
+    constexpr uint32_t PARTS = TOKENS / PART_ROWS;
+    const uint8_t* tsrc[PLANES][PARTS];
 #pragma unroll
-    for (uint32_t i = 0; i < NT; ++i) {
-        const uint32_t row = 8U * (8U * (i & 1U) + wave) + (lane >> 3), tok = row < count ? row : count - 1U;
+    for (uint32_t i = 0; i < PARTS; ++i) {
+        const uint32_t row = PART_ROWS * i + 8U * wave + (lane >> 3), tok = row < count ? row : count - 1U;
         const uint32_t piece = (lane & 7U) ^ ((row >> 1) & 7U);
-        if (MODE == 0) tsrc[i] = a.x + static_cast<size_t>(order[begin + tok] / a.top_k) * a.x_stride + 16U * piece;
-        // (h rows past the item's are other items' rows or the padding rows of the workspace: read, multiplied and never stored)
-        else tsrc[i] = reinterpret_cast<const uint8_t*>((i < 2U ? a.h : a.h_lo) + static_cast<size_t>(begin + row) * a.k) + 16U * piece;
+        if (MODE == 0) tsrc[0][i] = a.x + static_cast<size_t>(order[begin + tok] / a.top_k) * a.x_stride + 16U * piece;
+        else {
+            // (h rows past the item's are other items' rows or the padding rows of the workspace: read, multiplied and never stored)
+            const size_t from = static_cast<size_t>(begin + row) * a.k;
+            tsrc[0][i] = reinterpret_cast<const uint8_t*>(a.h + from) + 16U * piece;
+            tsrc[PLANES - 1U][i] = reinterpret_cast<const uint8_t*>(a.h_lo + from) + 16U * piece;
+        }
     }
     // ---- sums copy: piece = (token, part): parts 0, 1 = hi halves 0-7 / 8-15, parts 2, 3 = lo
     const uint8_t* ssrc;
@@ -92,17 +106,10 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                                         : a.h_sums + static_cast<size_t>(begin + tok) * sum_row;
         ssrc = base + 16U * (part & 1U) + (part >> 1) * (sum_row / 2U);
     }
-    const auto copy_tokens = [&](uint32_t s, pf_lds* stage) {
-        const uint32_t sc = s < last_stage ? s : last_stage;
-        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stage)) + 1024U * wave_s;
-#pragma unroll
-        for (uint32_t i = 0; i < NT; ++i)
-            copy16_to_lds_at(tsrc[i] + static_cast<size_t>(sc) * 128U, base + (i >> 1) * kRgStageBytes + 8192U * (i & 1U));
-    };
     const auto copy_sums = [&](uint32_t g) {
         const uint32_t gc = g < last_group ? g : last_group;
         copy16_to_lds_at(ssrc + static_cast<size_t>(gc) * 32U,
-                         static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_tile)) + (g & 1U) * (kRgTokens * 64U) + 1024U * wave_s);
+                         static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_tile)) + (g & 1U) * (TOKENS * 64U) + 1024U * wave_s);
     };
     const auto fetch_header = [&](uint32_t b, u32x4& hd) {
         const uint8_t* blk = wrow + static_cast<size_t>(b < last_block ? b : last_block) * 144U;
@@ -139,10 +146,17 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
     // live across a join of two instantiations (a join may copy registers, and a copy of a register whose fetch is still in
     // flight would copy stale data).
     const auto run_unit = [&](auto live_constant) __attribute__((always_inline)) {
-    constexpr uint32_t LIVE = decltype(live_constant)::value;
-    floatx16 acc[4], part[4];
+    constexpr uint32_t LIVE = decltype(live_constant)::value, NT = rg_token_ops<MODE, WAVES>(LIVE);
+    const auto copy_tokens = [&](uint32_t s, pf_lds* stage) {
+        const uint32_t sc = s < last_stage ? s : last_stage;
+        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stage)) + 1024U * wave_s;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+        for (uint32_t i = 0; i < NT; ++i)
+            copy16_to_lds_at(tsrc[i % PLANES][i / PLANES] + static_cast<size_t>(sc) * 128U, base + (i % PLANES) * STAGE + 128U * PART_ROWS * (i / PLANES));
+    };
+    floatx16 acc[LIVE], part[LIVE];
+#pragma unroll
+    for (uint32_t i = 0; i < LIVE; ++i)
 #pragma unroll
         for (int j = 0; j < 16; ++j) { acc[i][j] = 0.0F; part[i][j] = 0.0F; }
     const uint32_t trow = n31 * 128U, sw = (n31 >> 1) & 7U;
@@ -187,7 +201,7 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                 half8 frag[W];
                 const auto request = [&](uint32_t m) __attribute__((always_inline)) {
                     const uint32_t j = m / PER, pl = (m / LIVE) % PLANES, i = m % LIVE;
-                    frag[m % W] = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(tok + pl * kRgStageBytes + i * 32U * 128U + piece_at[j]);
+                    frag[m % W] = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(tok + pl * STAGE + i * 32U * 128U + piece_at[j]);
                 };
 #pragma unroll
                 for (uint32_t m = 0; m < W; ++m) request(m);
@@ -207,7 +221,7 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                             // first k-step of the next stage: its quants were fetched at the end of stage s - 3 (younger operations:
                             // the whole of stages s - 2, s - 1 and s), its header - when it opens a super-block - in stage s - 3
                             constexpr uint32_t pn = (p + 1U) & 3U;
-                            constexpr uint32_t younger = rg_stage_ops<MODE>((p + 2U) & 3U) + rg_stage_ops<MODE>((p + 3U) & 3U) + rg_stage_ops<MODE>(p);
+                            constexpr uint32_t younger = rg_stage_ops(NT, (p + 2U) & 3U) + rg_stage_ops(NT, (p + 3U) & 3U) + rg_stage_ops(NT, p);
                             if (p == 3U) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(qs[pn]), "+v"(hd_next) : "n"(younger) : "memory");
                             else asm volatile("s_waitcnt vmcnt(%1)" : "+v"(qs[pn]) : "n"(younger) : "memory");
                             uint32_t n_lo, n_hi;
@@ -261,7 +275,7 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                         for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(d, part[i][r], acc[i][r]);
                     if ((b & 1U) || b + 1U == blocks) {
                         // end of a group of 16 sub-blocks: running sum += S hi * M hi + S lo * M hi + S hi * M lo
-                        const pf_lds* st = s_tile + ((b >> 1) & 1U) * (kRgTokens * 64U) + n31 * 64U + 16U * half;
+                        const pf_lds* st = s_tile + ((b >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 16U * half;
                         const half8 mh = __builtin_bit_cast(half8, mreg_hi), ml = __builtin_bit_cast(half8, mreg_lo);
 #pragma unroll
                         for (uint32_t i = 0; i < LIVE; ++i) {
@@ -276,7 +290,7 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                 }
                 // the token copies of stage s + 1 were issued at the start of stage s - 2: younger operations = the rest of that
                 // stage and the whole of stages s - 1 and s
-                constexpr uint32_t younger_tokens = rg_stage_ops<MODE>((p + 2U) & 3U) - NT + rg_stage_ops<MODE>((p + 3U) & 3U) + rg_stage_ops<MODE>(p);
+                constexpr uint32_t younger_tokens = rg_stage_ops(NT, (p + 2U) & 3U) - NT + rg_stage_ops(NT, (p + 3U) & 3U) + rg_stage_ops(NT, p);
                 rg_wait<static_cast<int>(younger_tokens)>();
                 pf_barrier();
         };
@@ -294,7 +308,7 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
         // swap halves (the gate lane sends its tokens 8-15, the up lane its tokens 0-7), so each evaluates SwiGLU for eight
         // tokens. This class follows the exact product to a tolerance, so exp and the division are the hardware's
         // (v_exp_f32, v_rcp_f32: one ulp each).
-        const uint32_t f_out = tile * 128U + 16U * wave + (n31 & 15U);
+        const uint32_t f_out = tile * (16U * WAVES) + 16U * wave + (n31 & 15U);
         const bool gate_lane = n31 < 16U;
 #pragma unroll
         for (uint32_t i = 0; i < LIVE; ++i)
@@ -328,17 +342,17 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
                 }
             }
         __syncthreads();
-        if (threadIdx.x < 4U * kRgTokens) {
-            const uint32_t t = threadIdx.x & (kRgTokens - 1U), pair = threadIdx.x / kRgTokens;      // sub-block tile * 4 + pair of this tile
+        if (threadIdx.x < WAVES / 2U * TOKENS) {
+            const uint32_t t = threadIdx.x & (TOKENS - 1U), pair = threadIdx.x / TOKENS;            // sub-block tile * WAVES / 2 + pair
             if (t < count) {
                 const float sum = part_sum[2U * pair][t] + part_sum[2U * pair + 1U][t];
                 _Float16* sums = reinterpret_cast<_Float16*>(a.h_sums + static_cast<size_t>(begin + t) * pf_sum_row_bytes(a.features));
-                split_half(sum, sums[tile * 4U + pair], sums[pf_sum_slots(a.features) + tile * 4U + pair]);
+                split_half(sum, sums[tile * (WAVES / 2U) + pair], sums[pf_sum_slots(a.features) + tile * (WAVES / 2U) + pair]);
             }
         }
         __syncthreads();                                  // part_sum is free for the next unit
     } else {
-        const uint32_t f_out = tile * 256U + 32U * wave + n31;
+        const uint32_t f_out = tile * (32U * WAVES) + 32U * wave + n31;
 #pragma unroll
         for (uint32_t i = 0; i < LIVE; ++i)
 #pragma unroll
@@ -350,10 +364,16 @@ __global__ __launch_bounds__(kRgThreads) void prefill_reg_kernel(PrefillArgs a, 
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(hd_cur), "+v"(hd_next), "+v"(qs[0]), "+v"(qs[1]), "+v"(qs[2]), "+v"(qs[3]) : : "memory");
     };
     const uint32_t live_tiles = (count + 31U) / 32U;
-    if (live_tiles >= 4U) run_unit(std::integral_constant<uint32_t, 4>{});
-    else if (live_tiles == 3U) run_unit(std::integral_constant<uint32_t, 3>{});
-    else if (live_tiles == 2U) run_unit(std::integral_constant<uint32_t, 2>{});
-    else run_unit(std::integral_constant<uint32_t, 1>{});
+    if constexpr (TILES == 4U) {
+        if (live_tiles >= 4U) run_unit(std::integral_constant<uint32_t, 4>{});
+        else if (live_tiles == 3U) run_unit(std::integral_constant<uint32_t, 3>{});
+        else if (live_tiles == 2U) run_unit(std::integral_constant<uint32_t, 2>{});
+        else run_unit(std::integral_constant<uint32_t, 1>{});
+    } else {
+        static_assert(TILES == 2U, "live tiles of the narrow form");
+        if (live_tiles == 2U) run_unit(std::integral_constant<uint32_t, 2>{});
+        else run_unit(std::integral_constant<uint32_t, 1>{});
+    }
     }   // units
 }
 

@@ -1,5 +1,5 @@
 // Q4_K x A8 rows against 3..32 activation rows at a time: the exact group dots come from the int8 matrix cores, the
-// reference's fp32 chain stays on the vector ALU. The sweep below serves a dense matrix (q4k_mma_kernel) and the routed
+// reference's fp32 chain stays on the vector ALU. The sweep below serves dense matrices and the routed
 // experts of larger batches (q4k_mma_moe.hpp: gate + up with the SwiGLU / A8 epilogue, and the down rows).
 //
 // A workgroup (4 wavefronts) owns 32 weight rows. Wavefront p owns the reference's pair accumulator p of those rows
@@ -301,28 +301,6 @@ __device__ __forceinline__ void mma_reduce(lds_f32* red, const float (&acc)[NM][
         }
     }
     __syncthreads();
-}
-
-// ---- a dense matrix (or two that share their activation rows), rows of raw dots out
-template <int NAL, int DEPTH, int TEAMS>
-__global__ __launch_bounds__(256 * TEAMS) void q4k_mma_kernel(PairArgs args) {
-    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<NAL, 1, DEPTH, TEAMS>()];
-    __shared__ float xbuf_mem[mma_exchange_floats<NAL, TEAMS>()];
-    if (args.skip_flag && (*args.skip_flag & args.skip_mask)) return;
-    const PairMatrix& m = args.m[blockIdx.y];
-    const uint32_t lane = threadIdx.x & 63U, row0 = blockIdx.x * kMmaRows;
-    const uint8_t* const wrows[1] = {m.w + static_cast<size_t>(row0) * m.row_stride};
-    const A8Image& img = args.img;
-    const auto acts = [&](uint32_t a) {
-        return MmaActRow{reinterpret_cast<const uint8_t*>(img.codes_of(a)), reinterpret_cast<const uint8_t*>(img.deltas_of(a)),
-                         reinterpret_cast<const uint8_t*>(img.sums_of(a))};
-    };
-    float acc[1][NAL];
-    mma_sweep<NAL, DEPTH, TEAMS, 1>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, wrows, m.row_stride, args.blocks, acts, args.nacts, acc);
-    mma_reduce<NAL, 1>((lds_f32*)ring_mem, acc, args.nacts, [&](uint32_t v, const float (&value)[1]) {
-        const uint32_t a = 2U * v + (lane >> 5);
-        if (a < args.nacts) m.out[static_cast<size_t>(a) * m.out_stride + row0 + (lane & 31U)] = value[0];
-    });
 }
 
 }  // namespace strix950

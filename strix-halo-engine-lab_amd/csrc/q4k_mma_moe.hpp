@@ -5,8 +5,11 @@
 //   down:    32 hidden outputs against the A8 image of h (src/cpu/core/routed_expert.cpp:429-447, src/moe_a8_down_contract.cpp:146).
 // An item longer than 2 NAL rows is served in chunks; the second and later sweeps of the tile's weights come from the cache.
 // dense_rows > 0: no plan, expert 0, assignment i = row i; blockIdx.y picks a chunk of 2 NAL rows.
-// (Included inside namespace strix950, after the plan helpers and RowsK accessors it uses.)
 #pragma once
+#include "plan_layout.hpp"
+#include "q4k_mma.hpp"
+
+namespace strix950 {
 
 struct MmaItem { uint32_t e, begin, end; };
 __device__ __forceinline__ MmaItem mma_item(const mi355_moe_weights& w, const RowsK& r, uint32_t assignments, uint32_t dense_rows, uint32_t width) {
@@ -120,3 +123,5 @@ __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(mi355_moe_wei
         });
     }
 }
+
+}  // namespace strix950

@@ -12,16 +12,14 @@
 #include "device_math.hpp"
 #include "host_common.hpp"
 #include "launchers.hpp"
+#include "plan_layout.hpp"
 #include "q4k_rows.hpp"
 #include "q4k_blocks.hpp"
 #include "q4k_pairs.hpp"
-#include "q4k_mma.hpp"
 #include "q4k_quads.hpp"
 #include "down_groups.hpp"
 #include "q5k_quads.hpp"
 #include "q6k_quads.hpp"
-#include "prefill_f16.hpp"
-#include "prefill_reg.hpp"
 #include "route_wave.hpp"
 #include "route_early.hpp"
 
@@ -142,45 +140,6 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_kernel(const float* x, const 
 }
 
 // ======================================================================================================== router
-// Plan words (uint32): [0] assignments A = rows * top_k, [1] touched experts U, [2] largest group, [3] launch ticket,
-// [4] work items; [16, 272) ticket / scratch words; offsets[experts + 1]; touched[experts] (ids of the experts with work,
-// ascending); order[A]: assignment indices (row * top_k + slot) grouped by expert, ascending row then slot inside an
-// expert; items[A] x 4 words {expert, begin, end, 0}: the work items of the expert kernels, a touched expert's assignments
-// cut into pieces of at most `split` (zero records after the last item, up to the launch's item bound).
-// Reference: src/hip_moe_q4k_a8_probe.hip:91-147 (stable CSR of (row, slot) by expert).
-__host__ __device__ constexpr uint32_t pad4(uint32_t v) { return (v + 3U) & ~3U; }
-// ticket / scratch words right after the header, at the same place for every batch size (every launch leaves them zero, and a
-// workspace is reused with varying row counts): [0, 16) row tickets of the fused router, [16, 32) its quantiser tickets,
-// [128, 144) per-row A8 flags of the fused prologue
-constexpr uint32_t kPlanTicketsAt = 16, kPlanTicketWords = 256;
-// Behind the ticket words, also at a fixed place, the words of a decode batch planned from early routes (route_early.hpp):
-//   one word per assignment (finished projection waves in the low half, bit 31 = non-finite projection);
-//   one 64-bit tag per assignment {epoch, early expert};
-//   three 128-byte lines per row (arrival counts of the early blocks, of the A8 prologue blocks - with the row's flag word beside
-//     it - and of the exact router's side blocks) and a line with one tag per row (epoch of the call whose A8 image of that row is
-//     complete) and the epoch word.
-// Counts are zero when the plan is allocated and every launch leaves them zero. The epoch of a call is the epoch word + 1; the
-// call's down launch stores it back, so tags of earlier calls never look current and nothing has to be reset.
-constexpr uint32_t kLineWords = 32, kEarlyMaxAssignments = 128, kEarlyMinAssignments = 8, kEarlyMaxRows = 16;
-constexpr uint32_t kPlanAwordsAt = kPlanTicketsAt + kPlanTicketWords, kPlanEtagsAt = kPlanAwordsAt + kEarlyMaxAssignments;
-constexpr uint32_t kPlanLinesAt = (kPlanEtagsAt + 2U * kEarlyMaxAssignments + kLineWords - 1U) / kLineWords * kLineWords;      // (lines of a 128-byte aligned plan)
-constexpr uint32_t kLinesEarly = 0, kLinesPrologue = kEarlyMaxRows * kLineWords, kLinesSide = 2U * kEarlyMaxRows * kLineWords;
-constexpr uint32_t kLinesRowTags = 3U * kEarlyMaxRows * kLineWords, kLinesEpoch = kLinesRowTags + kEarlyMaxRows;
-constexpr uint32_t kPlanOffsetsAt = kPlanLinesAt + kLinesRowTags + kLineWords;
-static_assert(kPlanEtagsAt % 2U == 0 && kPlanOffsetsAt % 4U == 0, "tags on 8 bytes, the plan arrays on 16");
-__host__ __device__ constexpr uint32_t plan_touched_at(uint32_t experts) { return kPlanOffsetsAt + pad4(experts + 1U); }
-__host__ __device__ constexpr uint32_t plan_order_at(uint32_t experts) { return plan_touched_at(experts) + pad4(experts); }
-// most work items a plan can hold (layout) and most a launch with pieces of `split` assignments can produce (grid size)
-__host__ __device__ constexpr uint32_t plan_item_capacity(uint32_t assignments) { return assignments; }
-__host__ __device__ inline uint32_t plan_item_bound(uint32_t experts, uint32_t assignments, uint32_t split) {
-    const uint32_t most = experts + assignments / split;
-    return assignments < most ? assignments : most;
-}
-__host__ __device__ constexpr uint32_t plan_items_at(uint32_t experts, uint32_t assignments) { return plan_order_at(experts) + pad4(assignments); }
-__host__ __device__ constexpr uint32_t plan_words_total(uint32_t experts, uint32_t assignments) {
-    return plan_items_at(experts, assignments) + 4U * plan_item_capacity(assignments);
-}
-
 // A8 prologue block qb of a fused decode launch (src/cpu/core/reference.cpp:35-55): two groups of 32 at a time, 8 groups per
 // block; the last of a row's blocks publishes the row's status word. scratch: 256 floats of LDS (fused RMSNorm only).
 // Row r counts its finished blocks in ticket[r * stride] and collects its flags in flags[r * stride]. LINES: the words are reached
@@ -867,7 +826,6 @@ __global__ __launch_bounds__(64, DEPTH > 3 ? 1 : 2) void down_wave_kernel(mi355_
     }
 }
 
-#include "q4k_mma_moe.hpp"
 
 // ---- the smallest decode batches: 16 rows per wavefront, lane = (row, pair) (q4k_quads.hpp) ------------------------------
 #define STRIX_QUAD_SLOTS(DEPTH)                                                                      \
@@ -1690,44 +1648,11 @@ inline uint32_t mma_grouped_split(const mi355_moe_weights& w, uint32_t rows) {
     const uint64_t assignments = static_cast<uint64_t>(rows) * w.top_k;
     return assignments >= 16ULL * w.experts ? kMmaItemRows : assignments >= 4ULL * w.experts ? 16U : 0U;
 }
-template <int NAL>
-inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const dim3 grid(w.ffn / 32U, dense ? (dense + 2U * NAL - 1U) / (2U * NAL) : items);
-    q4k_mma_project_kernel<NAL, (NAL >= 8 ? 2 : 3)><<<grid, 256, 0, st>>>(w, r, rows * w.top_k, dense);
-}
-// A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
-// rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
-template <int NAL>
-inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const dim3 grid(w.hidden / kMmaRows, dense ? (dense + 2U * NAL - 1U) / (2U * NAL) : items);
-    if constexpr (NAL <= 8) {
-        if (static_cast<uint64_t>(grid.x) * grid.y <= compute_units()) {
-            q4k_mma_down_kernel<NAL, 2, 4><<<grid, 1024, 0, st>>>(w, r, rows * w.top_k, dense);
-            return;
-        }
-    }
-    q4k_mma_down_kernel<NAL, (NAL >= 8 ? 2 : 3), 1><<<grid, 256, 0, st>>>(w, r, rows * w.top_k, dense);
-}
-// width: the most rows an item (or the dense batch) holds
-inline void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
-    if (width <= 4U) launch_mma_project_nal<2>(w, r, rows, dense, items, st);
-    else if (width <= 8U) launch_mma_project_nal<4>(w, r, rows, dense, items, st);
-    else if (width <= 16U) launch_mma_project_nal<8>(w, r, rows, dense, items, st);
-    else launch_mma_project_nal<16>(w, r, rows, dense, items, st);
-}
 // A dense FFN's gate and up rows as raw values into the intermediates, then the SwiGLU / A8 kernel (5..16 rows, one chunk).
 inline void launch_mma_gate_up(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, hipStream_t st) {
-    const dim3 grid(w.ffn / kMmaRows, 1, 2);
-    if (rows <= 8U) q4k_mma_down_kernel<4, 3, 1, true><<<grid, 256, 0, st>>>(w, r, rows, rows);
-    else q4k_mma_down_kernel<8, 2, 1, true><<<grid, 256, 0, st>>>(w, r, rows, rows);
+    launch_mma_gate_up_rows(w, r, rows, st);
     swiglu_quantize_kernel<<<dim3((w.ffn / 32U + 7U) / 8U, rows), 256, 0, st>>>(r.gate_out, r.up_out, w.ffn, w.exp_kind, w.swiglu_limit, r.down_codes, r.down_deltas,
                                                                                 r.down_sums, r.h_out, r.status, r.job_status);
-}
-// (the down rows run best 16 rows to a sweep: 4096 rows over 256 experts, hidden 4096 / ffn 2048: 2.57 ms against 3.03 ms with 32)
-inline void launch_mma_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
-    if (width <= 4U) launch_mma_down_nal<2>(w, r, rows, dense, items, st);
-    else if (width <= 8U) launch_mma_down_nal<4>(w, r, rows, dense, items, st);
-    else launch_mma_down_nal<8>(w, r, rows, dense, items, st);
 }
 
 inline void launch_plan(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split, uint32_t bound, uint32_t* plan,
@@ -2337,41 +2262,7 @@ int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v,
     a.x_sums = x_sums;
     a.rawdots = v.rawdots; a.rawdots_rs = v.rawdots_rs; a.rawdots_bf16 = v.rawdots_bf16; a.plan = v.plan; a.experts = wv.experts; a.assignments = assignments;
     a.status = v.status; a.status_rs = v.status_rs; a.job_status = v.job_status; a.items = bound;
-    token_sums_kernel<<<rows, 256, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums);
-    if (pf_sum_slots(wv.ffn) != wv.ffn / 32U) clear_sum_padding_kernel<<<assignments, 64, 0, st>>>(a.h_sums, wv.ffn);
-    const uint32_t items_at = plan_items_at(wv.experts, assignments), order_at = plan_order_at(wv.experts), item_slots = (bound + 7U) / 8U * 8U;
-    // persistent workgroups, one per compute unit (the kernels' LDS use allows no second one)
-    const uint32_t cus = compute_units();
-    const uint32_t resident = (cus > 8U ? cus : 256U) & ~7U;
-    const auto grid_of = [&](uint32_t units) { return units < resident ? units : resident; };
-    // gate / up + SwiGLU. Q4_K tensors: every wave expands its own rows in registers (prefill_reg.hpp); Q5_K / Q8_0: the loader /
-    // multiplier kernel (prefill_f16.hpp). Both leave h as two fp16 planes and its sub-block sums.
-    a.wa = wv.gate; a.wb = wv.up; a.expert_stride = wv.gate_expert_stride; a.row_stride = wv.gate_row_stride; a.k = wv.hidden; a.features = wv.ffn;
-    a.lo_pass = 0;
-    if (wv.gate_type == MI355_TYPE_Q4_K && wv.ffn % 128U == 0) {
-        a.tiles = wv.ffn / 128U; a.units = item_slots * a.tiles;
-        prefill_reg_kernel<0><<<grid_of(a.units), kRgThreads, 0, st>>>(a, items_at, order_at);
-    } else {
-        a.tiles = wv.ffn / 64U; a.units = item_slots * a.tiles;
-        if (wv.gate_type == MI355_TYPE_Q8_0) prefill_f16_kernel<0, 1><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        else if (wv.gate_type == MI355_TYPE_Q5_K) prefill_f16_kernel<0, 2><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        else prefill_f16_kernel<0, 0><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-    }
-    // down rows: h enters as hi + lo. The register-operand kernel multiplies both planes in one sweep of the weights; the loader /
-    // multiplier kernel runs a second pass over the lo plane that adds to the first pass's outputs.
-    a.wa = wv.down; a.wb = nullptr; a.expert_stride = wv.down_expert_stride; a.row_stride = wv.down_row_stride; a.k = wv.ffn; a.features = wv.hidden;
-    if (wv.down_type == MI355_TYPE_Q4_K && wv.hidden % 256U == 0) {
-        a.tiles = wv.hidden / 256U; a.units = item_slots * a.tiles;
-        prefill_reg_kernel<1><<<grid_of(a.units), kRgThreads, 0, st>>>(a, items_at, order_at);
-    } else {
-        a.tiles = wv.hidden / 128U; a.units = item_slots * a.tiles;
-        for (uint32_t pass = 0; pass < 2U; ++pass) {
-            a.lo_pass = pass;
-            if (wv.down_type == MI355_TYPE_Q8_0) prefill_f16_kernel<1, 1><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-            else if (wv.down_type == MI355_TYPE_Q5_K) prefill_f16_kernel<1, 2><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-            else prefill_f16_kernel<1, 0><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        }
-    }
+    launch_prefill_products(wv, a, rows, x_sums, plan_items_at(wv.experts, assignments), plan_order_at(wv.experts), st);
     STRIX_LAUNCHED("moe prefill f16");
     return MI355_OK;
 }
