@@ -41,15 +41,15 @@ __device__ __forceinline__ void load_activation8(const uint8_t* row, uint32_t i,
     }
 }
 
-// The row's image by the calling workgroup (blockDim.x a multiple of 64); returns non-zero in the threads of a group with a
+// The row's image by the first `threads` (a multiple of 64) of the calling workgroup; returns non-zero in the threads of a group with a
 // non-finite value.
 template <int KIND>
-__device__ __forceinline__ int a8_row(const A8RowArgs& a, uint32_t r) {
+__device__ __forceinline__ int a8_row(const A8RowArgs& a, uint32_t r, uint32_t threads) {
     const uint8_t* row = a.x + r * a.x_stride;
     int8_t* codes = a.codes + static_cast<size_t>(r) * a.width;
     const uint32_t groups = a.width / 32U;
     int any_bad = 0;
-    for (uint32_t i = threadIdx.x * 8U; i < a.width; i += blockDim.x * 8U) {          // (a group's four threads leave the loop together)
+    for (uint32_t i = threadIdx.x * 8U; i < a.width; i += threads * 8U) {          // (a group's four threads leave the loop together)
         float v[8];
         load_activation8<KIND>(row, i, a.vec != 0, v);
         float amax = __builtin_fabsf(v[0]);
@@ -89,7 +89,7 @@ __device__ __forceinline__ int a8_row(const A8RowArgs& a, uint32_t r) {
 template <int KIND>
 __global__ __launch_bounds__(1024) void a8_rows_kernel(A8RowArgs a) {
     const uint32_t r = blockIdx.x;
-    const int bad = a8_row<KIND>(a, r);
+    const int bad = a8_row<KIND>(a, r, blockDim.x);
     if (a.status_mode == kA8StatusNone) return;
     const uint32_t bits = __syncthreads_or(bad) ? static_cast<uint32_t>(MI355_STATUS_NONFINITE_ACTIVATION) : 0U;
     if (threadIdx.x == 0) {

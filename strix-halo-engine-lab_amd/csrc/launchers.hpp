@@ -1,5 +1,6 @@
 // Launches whose kernels live in translation units of their own (they compile in parallel).
 #pragma once
+#include "a8_rows.hpp"
 #include "prefill_args.hpp"
 #include "q4k_rows.hpp"
 #include "route_wave.hpp"
@@ -9,10 +10,19 @@ namespace strix950 {
 // route.hip: logits of a batch past the decode sizes into a.scores; softmax, selection and weights of every row of a.scores
 void launch_route_batch_logits(const RouteArgs& a, hipStream_t st);
 void launch_route_select(const RouteArgs& a, hipStream_t st);
+// A8 image, routes and status words of the rows of a staged batch. select: the router whose logits are in its scores (null: the routes
+// are given); q.status is not used.
+struct RouteCheck {
+    const uint32_t* routes; const float* route_weights;      // [rows][top_k]; weights may be null
+    uint32_t experts, top_k;
+    uint32_t *status, *job_status;
+};
+void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, const RouteArgs* select, const RouteCheck& c, hipStream_t st);
 
 // prefill.hip: sub-block sums of the input rows, gate / up + SwiGLU and down rows of a planned batch. `a` holds everything but the
-// products' own fields (weights, strides, k, features, tiles, units).
-void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, uint32_t items_at, uint32_t order_at, hipStream_t st);
+// products' own fields (weights, strides, k, features, tiles, units). check: the routes' check and the status words as well.
+void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at,
+                             uint32_t order_at, hipStream_t st);
 
 // q4k_mma.hip: Q4_K experts on the int8 matrix cores. dense: the rows of a one-expert batch (0: planned items); width: the most rows an
 // item (or the dense batch) holds. The last leaves the raw gate and up values of a dense batch of at most 16 rows.

@@ -5,9 +5,49 @@
 
 namespace strix950 {
 
-void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, uint32_t items_at, uint32_t order_at, hipStream_t st) {
-    token_sums_kernel<<<rows, 256, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums);
-    if (pf_sum_slots(wv.ffn) != wv.ffn / 32U) clear_sum_padding_kernel<<<a.assignments, 64, 0, st>>>(a.h_sums, wv.ffn);
+// What a batch needs besides its plan before the products, one workgroup per row: the row's sub-block sums (a thread per sub-block of 32,
+// fp32 sum in index order), zeros in the padding slots of the sums of h of the row's assignments (ffn / 32 not a multiple of 16; every
+// assignment has a row of sums, whichever order the plan gives them), and - with a check - the routes' check and the status words.
+// Bound by latency: one launch in the place of three (333 rows: about 4.5 us each).
+__global__ __launch_bounds__(256) void prefill_prologue_kernel(const uint8_t* x, uint64_t x_stride, uint32_t k, uint8_t* x_sums, uint8_t* h_sums, uint32_t ffn,
+                                                               uint32_t top_k, RouteCheck check) {
+    const uint32_t row = blockIdx.x, slots = pf_sum_slots(k), h_slots = pf_sum_slots(ffn), h_used = ffn / 32U, pad = h_slots - h_used;
+    _Float16* hi = reinterpret_cast<_Float16*>(x_sums + static_cast<size_t>(row) * pf_sum_row_bytes(k));
+    _Float16* lo = hi + slots;
+    for (uint32_t s = threadIdx.x; s < slots; s += 256U) {
+        float sum = 0.0F;
+        if (s < k / 32U) {
+            const half8* p = reinterpret_cast<const half8*>(x + static_cast<size_t>(row) * x_stride + 64U * s);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const half8 v = p[i];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) sum += static_cast<float>(v[j]);
+            }
+        }
+        split_half(sum, hi[s], lo[s]);
+    }
+    for (uint32_t i = threadIdx.x; i < pad * top_k; i += 256U) {
+        const uint32_t slot = i / pad, s = h_used + i - slot * pad;
+        _Float16* out = reinterpret_cast<_Float16*>(h_sums + (static_cast<size_t>(row) * top_k + slot) * pf_sum_row_bytes(ffn));
+        out[s] = static_cast<_Float16>(0.0F);
+        out[h_slots + s] = static_cast<_Float16>(0.0F);
+    }
+    if (!check.status || threadIdx.x < 192U) return;
+    uint32_t bad = 0;
+    for (uint32_t i = threadIdx.x - 192U; i < top_k; i += 64U) {
+        if (check.routes[static_cast<size_t>(row) * top_k + i] >= check.experts) bad = 1;
+        if (check.route_weights && !finite_f(check.route_weights[static_cast<size_t>(row) * top_k + i])) bad = 1;
+    }
+    const bool any = __ballot(bad) != 0;
+    if (threadIdx.x == 192U) {
+        check.status[row] = any ? static_cast<uint32_t>(MI355_STATUS_INVALID_ROUTE) : 0U;
+        if (row == 0) *check.job_status = 0;
+    }
+}
+
+void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at, uint32_t order_at, hipStream_t st) {
+    prefill_prologue_kernel<<<rows, 256, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums, a.h_sums, wv.ffn, wv.top_k, check ? *check : RouteCheck{});
     const uint32_t item_slots = (a.items + 7U) / 8U * 8U;
     // persistent workgroups, as many as are resident: one per compute unit (LDS allows no second one) or `each` of the narrow form
     const uint32_t cus = compute_units();

@@ -80,33 +80,6 @@ __device__ __forceinline__ void split_half(float v, _Float16& hi, _Float16& lo) 
     lo = static_cast<_Float16>(v - static_cast<float>(hi));
 }
 
-// Sub-block sums of fp16 rows: one thread per (row, sub-block of 32), fp32 sum in index order.
-__global__ __launch_bounds__(256) void token_sums_kernel(const uint8_t* x, uint64_t x_stride, uint32_t k, uint8_t* sums) {
-    const uint32_t row = blockIdx.x, slots = pf_sum_slots(k);
-    _Float16* hi = reinterpret_cast<_Float16*>(sums + static_cast<size_t>(row) * pf_sum_row_bytes(k));
-    _Float16* lo = hi + slots;
-    for (uint32_t s = threadIdx.x; s < slots; s += 256U) {
-        float sum = 0.0F;
-        if (s < k / 32U) {
-            const half8* p = reinterpret_cast<const half8*>(x + static_cast<size_t>(row) * x_stride + 64U * s);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const half8 v = p[i];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) sum += static_cast<float>(v[j]);
-            }
-        }
-        split_half(sum, hi[s], lo[s]);
-    }
-}
-
-// Padding slots of the sums of h (ffn / 32 not a multiple of 16) must read as zero.
-__global__ __launch_bounds__(64) void clear_sum_padding_kernel(uint8_t* sums, uint32_t k) {
-    const uint32_t slots = pf_sum_slots(k), used = k / 32U;
-    _Float16* hi = reinterpret_cast<_Float16*>(sums + static_cast<size_t>(blockIdx.x) * pf_sum_row_bytes(k));
-    for (uint32_t s = used + threadIdx.x; s < slots; s += 64U) { hi[s] = static_cast<_Float16>(0.0F); hi[slots + s] = static_cast<_Float16>(0.0F); }
-}
-
 // Workgroup barrier that orders LDS traffic only. __syncthreads() also waits for every outstanding global memory operation
 // of the wave, which would drain the copies and fetches that are in flight for later steps at every barrier; their
 // arrival is awaited explicitly where it is needed.

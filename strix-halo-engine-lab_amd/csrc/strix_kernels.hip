@@ -334,24 +334,51 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* w
     return base + x - v;
 }
 
-// The expert plan in one workgroup: thread e owns expert e (counts by shared-memory atomics, three prefix sums for the
-// offsets, the item numbers and the touched list, then its own items and - for a small batch - its own stretch of the order).
+// The expert plan in one workgroup: thread e owns expert e (its count, three prefix sums for the offsets, the item numbers and the touched
+// list, then its own items). A batch of at most 1024 assignments (fill_order) is ordered here as well: wave w holds assignments
+// 64 w .. 64 w + 63, finds each one's position among its wave's assignments of the same expert by ballots (one round per expert named)
+// and leaves the wave's counts; a prefix over the waves and the expert's offset make it the position in the order. (A thread per expert
+// that walked every assignment took 12 us at 128 assignments; the order launch it saves at 257..1024 takes 4.7 us.)
+constexpr uint32_t kPlanSmall = 1024;
 __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split,
                                                     uint32_t item_bound, uint32_t fill_order, uint32_t* plan) {
-    __shared__ uint32_t count[kRouteMaxExperts];
+    __shared__ uint32_t count[kRouteMaxExperts];           // per expert: assignments, later (fill_order) its offset
+    __shared__ uint16_t wave_counts[16][kRouteMaxExperts]; // fill_order: per wave and expert, later the prefix over the waves before
     __shared__ uint32_t wave_totals[3][16];
     __shared__ uint32_t wave_largest[16];
-    __shared__ uint32_t small_routes[256];                 // fill_order: at most 256 assignments
-    const uint32_t tid = threadIdx.x, lane = tid & 63U, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63U, wave = tid >> 6, waves = (assignments + 63U) / 64U;
     count[tid] = 0;
-    __syncthreads();
-    for (uint32_t a = tid; a < assignments; a += 1024U) {
-        const uint32_t e = routes.at(a);
-        if (fill_order) small_routes[a] = e;
-        if (e < experts) atomicAdd(&count[e], 1U);
+    uint32_t mine = experts, rank = 0;                     // fill_order: this thread's assignment's expert, its position in the wave
+    if (fill_order) {
+        for (uint32_t w = 0; w < waves; ++w) wave_counts[w][tid] = 0;
+        if (tid < assignments) mine = routes.at(tid);
     }
     __syncthreads();
-    const uint32_t c = tid < experts ? count[tid] : 0U, pieces = (c + split - 1U) / split;
+    if (fill_order) {
+        uint64_t left = __ballot(mine < experts);
+        while (left) {
+            const uint32_t e = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), __builtin_ctzll(left)));
+            const uint64_t same = __ballot(mine == e);
+            if (mine == e) rank = static_cast<uint32_t>(__popcll(same & ((1ULL << lane) - 1ULL)));
+            if (lane == 0) wave_counts[wave][e] = static_cast<uint16_t>(__popcll(same));
+            left &= ~same;
+        }
+    } else {
+        for (uint32_t a = tid; a < assignments; a += 1024U) {
+            const uint32_t e = routes.at(a);
+            if (e < experts) atomicAdd(&count[e], 1U);
+        }
+    }
+    __syncthreads();
+    uint32_t c = tid < experts ? count[tid] : 0U;
+    if (fill_order && tid < experts) {
+        for (uint32_t w = 0; w < waves; ++w) {
+            const uint32_t here = wave_counts[w][tid];
+            wave_counts[w][tid] = static_cast<uint16_t>(c);
+            c += here;
+        }
+    }
+    const uint32_t pieces = (c + split - 1U) / split;
     uint32_t run, made, touched;
     const uint32_t first = block_exclusive_scan(c, wave_totals[0], run);
     const uint32_t item_from = block_exclusive_scan(pieces, wave_totals[1], made);
@@ -383,25 +410,10 @@ __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t 
         offsets[experts] = run;
         plan[0] = assignments; plan[1] = touched; plan[2] = most; plan[4] = made;
     }
-    if (!fill_order || tid >= experts || c == 0) return;   // large batches: plan_order_kernel follows
-    uint32_t at = first;
-    for (uint32_t a = 0; a < assignments; ++a)
-        if (small_routes[a] == tid) order[at++] = a;
-}
-
-__global__ __launch_bounds__(64) void clear_validate_kernel(const uint32_t* routes, const float* route_weights, uint32_t experts,
-                                                            uint32_t top_k, uint32_t* status, uint32_t* job_status) {
-    const uint32_t row = blockIdx.x;
-    uint32_t bad = 0;
-    for (uint32_t k = threadIdx.x; k < top_k; k += 64U) {
-        if (routes[row * top_k + k] >= experts) bad = MI355_STATUS_INVALID_ROUTE;
-        if (route_weights && !finite_f(route_weights[row * top_k + k])) bad = MI355_STATUS_INVALID_ROUTE;
-    }
-    for (int d = 32; d; d >>= 1) bad |= __shfl_xor(bad, d);
-    if (threadIdx.x == 0) {
-        status[row] = bad;
-        if (row == 0) *job_status = 0;
-    }
+    if (!fill_order) return;                               // large batches: plan_order_kernel follows
+    count[tid] = first;
+    __syncthreads();
+    if (mine < experts) order[count[mine] + wave_counts[wave][mine] + rank] = tid;
 }
 
 // ======================================================================================================== Q4_K x A8 rows
@@ -1657,9 +1669,8 @@ inline void launch_mma_gate_up(const mi355_moe_weights& w, const RowsK& r, uint3
 
 inline void launch_plan(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split, uint32_t bound, uint32_t* plan,
                         hipStream_t st) {
-    // plan_kernel's own order fill is one thread per expert walking every assignment: fine for a decode batch, far too slow
-    // beyond a few hundred assignments (4096 assignments of one expert: 0.55 ms), where a wave per expert does it instead
-    const bool large = assignments > 256U;
+    // past an assignment per thread of plan_kernel, a workgroup per expert orders its assignments in a launch of its own
+    const bool large = assignments > kPlanSmall;
     plan_kernel<<<1, 1024, 0, st>>>(routes, experts, assignments, split, bound, large ? 0U : 1U, plan);
     if (large) plan_order_kernel<<<experts, 1024, 0, st>>>(routes, experts, assignments, plan);
 }
@@ -1947,13 +1958,27 @@ size_t mi355_moe_plan_words(uint32_t experts, uint32_t rows, uint32_t top_k) {
     return plan_words_total(experts, rows * top_k);
 }
 
+}  // extern "C"
+namespace {
+RouteCheck route_check(const mi355_moe_weights& wv, const mi355_moe_rows& r) {
+    return RouteCheck{r.routes, r.route_weights, wv.experts, wv.top_k, r.status, r.job_status};
+}
+int32_t enqueue_prologue_rows(const mi355_moe_weights& wv, const mi355_moe_rows& r, uint32_t rows, const RouteArgs* select, hipStream_t st) {
+    STRIX_REQUIRE(r.codes && r.deltas, "A8: null pointer");
+    STRIX_REQUIRE(rows <= 65535U, "A8: at most 65535 rows per call");
+    const bool vec = aligned(r.input, 16) && r.input_stride % 16U == 0 && aligned(r.codes, 8);
+    launch_prologue_rows(A8RowArgs{static_cast<const uint8_t*>(r.input), r.input_stride, wv.hidden, r.codes, r.deltas, r.sums, nullptr, kA8StatusNone, vec, 0U},
+                         r.input_kind, rows, select, route_check(wv, r), st);
+    STRIX_LAUNCHED("moe prologue");
+    return MI355_OK;
+}
+}  // namespace
+extern "C" {
 int32_t mi355_moe_enqueue_prologue(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, mi355_stream stream) {
     mi355_moe_weights wv;
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;
     STRIX_REQUIRE(r->input && r->input_kind <= MI355_INPUT_BF16, "moe prologue: input view invalid");
-    clear_validate_kernel<<<rows, 64, 0, hs(stream)>>>(r->routes, r->route_weights, wv.experts, wv.top_k, r->status, r->job_status);
-    STRIX_LAUNCHED("moe clear/validate");
-    return mi355_quantize_a8(r->input, r->input_kind, rows, wv.hidden, r->input_stride, r->codes, r->deltas, r->sums, r->status, stream);
+    return enqueue_prologue_rows(wv, *r, rows, nullptr, hs(stream));
 }
 
 int32_t mi355_moe_enqueue_csr(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, mi355_stream stream) {
@@ -2030,13 +2055,13 @@ int32_t mi355_moe_enqueue(const mi355_moe_weights* w, const mi355_moe_rows* r, u
 namespace {
 // mi355_moe_enqueue by halves: front = prologue, plan, gate / up; back = down rows, combine.
 int32_t enqueue_staged(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, uint32_t form, mi355_stream stream, bool do_front, bool do_back,
-                       uint32_t shared_slots = 0) {
+                       uint32_t shared_slots = 0, const RouteArgs* select = nullptr) {
     mi355_moe_weights wv;
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;
     STRIX_REQUIRE(form <= MI355_COMBINE_MULADD_ASCENDING_EXPERT, "moe: unknown combine form");
     if (do_front) {
         STRIX_REQUIRE(r->input && r->input_kind <= MI355_INPUT_BF16, "moe: input view invalid");
-        if (const int32_t rc = mi355_moe_enqueue_prologue(w, r, rows, stream)) return rc;
+        if (const int32_t rc = enqueue_prologue_rows(wv, *r, rows, select, hs(stream))) return rc;
         if (!(dense_pairs_ok(wv, rows) && r->gate_out && r->up_out))
             if (const int32_t rc = mi355_moe_enqueue_csr(w, r, rows, stream)) return rc;
         if (const int32_t rc = mi355_moe_enqueue_project(w, r, rows, stream)) return rc;
@@ -2110,9 +2135,19 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
             STRIX_LAUNCHED("moe layer norm");
         }
         if (norm.on) { staged.input = norm.normed; staged.input_kind = MI355_INPUT_F32; staged.input_stride = 4ULL * wv.hidden; }
-        if (do_front)
-            if (const int32_t rc = mi355_moe_route(p, staged.input, staged.input_kind, rows, wv.hidden, staged.input_stride, router_weight, logit_bias, ids, weights, scores, stream)) return rc;
-        return enqueue_staged(w, &staged, rows, form, stream, do_front, do_back, p->shared_experts);
+        RouteArgs a{};
+        a.p = *p; a.x = static_cast<const uint8_t*>(staged.input); a.kind = staged.input_kind; a.x_stride = staged.input_stride; a.rows = rows; a.hidden = wv.hidden;
+        a.wr = router_weight; a.bias = logit_bias; a.ids = ids; a.weights = weights; a.scores = scores;
+        // the selection rides in the prologue's launch while that is one round of workgroups: its registers let a compute unit hold one
+        // (40 rows: 157.8 -> 154.4 us a layer; 1000 rows, four rounds: 631 -> 636 us, hence the line)
+        const bool fused_select = rows <= compute_units();
+        if (do_front) {
+            if (const int32_t rc = check_route(p, staged.input, staged.input_kind, wv.hidden, staged.input_stride, router_weight, ids, weights, scores)) return rc;
+            launch_route_logits(a, st);
+            if (!fused_select) launch_route_select(a, st);
+            STRIX_LAUNCHED("moe layer router");
+        }
+        return enqueue_staged(w, &staged, rows, form, stream, do_front, do_back, p->shared_experts, fused_select ? &a : nullptr);
     }
     RouteArgs a{};
     a.p = *p; a.x = static_cast<const uint8_t*>(r->input); a.kind = r->input_kind; a.x_stride = r->input_stride; a.rows = rows; a.hidden = wv.hidden;
@@ -2249,8 +2284,9 @@ struct PrefillViews {
     uint32_t* plan;
     void* h_f16;
 };
-// expert plan, sub-block sums of the input rows, gate / up + SwiGLU, down rows (the status words are already written)
-int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v, uint32_t rows, hipStream_t st) {
+// expert plan, sub-block sums of the input rows, gate / up + SwiGLU, down rows. check: the routes' check and the status words ride with the
+// sums (null: they are already written)
+int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v, uint32_t rows, hipStream_t st, const RouteCheck* check = nullptr) {
     const uint32_t assignments = rows * wv.top_k, bound = plan_item_bound(wv.experts, assignments, kPfTile);
     launch_plan(v.routes, wv.experts, assignments, kPfTile, bound, v.plan, st);
     PrefillArgs a{};
@@ -2262,7 +2298,7 @@ int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v,
     a.x_sums = x_sums;
     a.rawdots = v.rawdots; a.rawdots_rs = v.rawdots_rs; a.rawdots_bf16 = v.rawdots_bf16; a.plan = v.plan; a.experts = wv.experts; a.assignments = assignments;
     a.status = v.status; a.status_rs = v.status_rs; a.job_status = v.job_status; a.items = bound;
-    launch_prefill_products(wv, a, rows, x_sums, plan_items_at(wv.experts, assignments), plan_order_at(wv.experts), st);
+    launch_prefill_products(wv, a, rows, x_sums, check, plan_items_at(wv.experts, assignments), plan_order_at(wv.experts), st);
     STRIX_LAUNCHED("moe prefill f16");
     return MI355_OK;
 }
@@ -2279,9 +2315,9 @@ int32_t mi355_moe_enqueue_prefill_f16(const mi355_moe_weights* w, const mi355_mo
     STRIX_REQUIRE(rows <= 65535U, "moe prefill: at most 65535 rows per call");
     STRIX_REQUIRE(wv.hidden % 128U == 0 && wv.ffn % 64U == 0, "moe prefill: hidden must be a multiple of 128, ffn of 64");
     hipStream_t st = hs(stream);
-    clear_validate_kernel<<<rows, 64, 0, st>>>(r->routes, r->route_weights, wv.experts, wv.top_k, r->status, r->job_status);
     const PrefillViews v{r->input, r->input_stride, dense_routes(r->routes, wv.top_k), r->status, 4, r->job_status, r->rawdots, 0, 0U, r->plan, r->h_f16};
-    if (const int32_t rc = enqueue_prefill_core(wv, v, rows, st)) return rc;
+    const RouteCheck check = route_check(wv, *r);
+    if (const int32_t rc = enqueue_prefill_core(wv, v, rows, st, &check)) return rc;
     if (form == MI355_COMBINE_NONE) return MI355_OK;
     return mi355_moe_enqueue_merge(w, r, rows, form, stream);
 }

@@ -1,0 +1,97 @@
+"""The start of a staged batch: the plan's order around its single-launch limit, and the launch that selects, checks and quantises a row."""
+import numpy as np
+import pytest
+import torch
+
+import orc
+
+pytestmark = pytest.mark.gpu
+
+PLAN_OFFSETS_AT = 2240          # first word of the plan arrays (offsets, touched, order, items)
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def pad4(n):
+    return (n + 3) // 4 * 4
+
+
+# assignments around a wave's 64, around 1024 (an assignment per thread of the plan's workgroup) and past it; one expert that takes
+# everything, more experts than assignments
+@pytest.mark.parametrize("rows,top_k,experts,skew", [(1, 1, 2, 0), (63, 1, 5, 0), (64, 1, 1024, 0), (65, 1, 3, 2), (32, 8, 128, 0), (257, 1, 16, 1), (341, 3, 40, 0),
+                                                     (64, 16, 300, 2), (1025, 1, 64, 1), (205, 5, 7, 0)])
+def test_plan_order(strix, rows, top_k, experts, skew):
+    rng = np.random.default_rng(rows * top_k + experts)
+    ids = np.minimum(rng.integers(0, experts, (rows, top_k)), rng.integers(0, experts, (rows, top_k)) // (1 if skew == 0 else 4)) if skew < 2 else np.full((rows, top_k), experts - 1)
+    H = I = 256
+    row = H // 256 * 144
+    w = torch.zeros((experts * 256, row), dtype=torch.uint8, device="cuda")
+    layer = strix.MoeLayer(H, I, experts, top_k, w, w, w, rows)
+    x = torch.zeros((rows, H), device="cuda")
+    routes = torch.from_numpy(ids.astype(np.int32)).cuda()
+    layer.stage("csr", x, routes, torch.ones((rows, top_k), device="cuda"))
+    plan = layer.plan.cpu().numpy()
+    flat, A = ids.reshape(-1), rows * top_k
+    order_at = PLAN_OFFSETS_AT + pad4(experts + 1) + pad4(experts)
+    offsets = np.concatenate([[0], np.cumsum(np.bincount(flat, minlength=experts))])
+    assert np.array_equal(plan[PLAN_OFFSETS_AT:PLAN_OFFSETS_AT + experts + 1], offsets)
+    assert np.array_equal(plan[order_at:order_at + A], np.argsort(flat, kind="stable"))
+    items = plan[order_at + pad4(A):][:4 * plan[4]].reshape(-1, 4)
+    covered = np.concatenate([np.arange(b, e) for _, b, e, _ in items])
+    assert np.array_equal(covered, np.arange(A)) and all(offsets[e] <= b < z <= offsets[e + 1] for e, b, z, _ in items)
+
+
+# widths around the image's 448 threads of eight values; experts around the selection's register steps; a row with an infinity
+# (its weights are not finite either: both status bits), rows past and within the decode sizes (large experts: shared sweeps)
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(17, 256, 256, 5, 2), (40, 3584, 256, 130, 8), (33, 3840, 256, 16, 4), (18, 8192, 256, 20, 16), (16, 6144, 1280, 24, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_layer_equals_router_then_experts(strix, rows, hidden, ffn, experts, top_k, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    layer = strix.MoeLayer(hidden, ffn, experts, top_k, draw(experts * ffn, hidden), draw(experts * ffn, hidden), draw(experts * hidden, ffn), rows)
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(dtype)
+    x[rows // 2, hidden - 1] = float("inf")
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    out, ids, weights, scores = (t.clone() for t in layer.run_layer(x, router))
+    status = layer.status[:rows].clone()
+    ids2, weights2, scores2 = strix.route(x, router, top_k)
+    same = lambda a, b: torch.equal(a.contiguous().view(torch.int32), b.contiguous().view(torch.int32))
+    assert same(ids, ids2) and same(weights, weights2) and same(scores, scores2)
+    out2 = layer.run(x, ids2, weights2)
+    good = torch.arange(rows, device="cuda") != rows // 2
+    assert same(out[good], out2[good]) and same(status, layer.status[:rows])
+    bad = strix.STATUS_NONFINITE_ACTIVATION | strix.STATUS_INVALID_ROUTE
+    assert [s & bad for s in status.cpu().tolist()] == [bad if r == rows // 2 else 0 for r in range(rows)]
+    ids_ref, w_ref, _, _ = orc.route(x[:1].float().cpu().numpy(), router.cpu().numpy(), top_k)
+    assert np.array_equal(ids[:1].cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(weights[:1].cpu().numpy().view(np.uint32), w_ref.view(np.uint32))
+    layer.run(x, torch.full_like(ids2, experts), weights2 * 0 + 1)          # routes outside the experts
+    assert all(s & strix.STATUS_INVALID_ROUTE for s in layer.status[:rows].cpu().tolist())
+
+
+# narrow prefill (few rows per expert on average) with items of one row, around 64 and 128 rows, and the wide form for comparison
+@pytest.mark.parametrize("counts,hidden,ffn", [((1, 64, 0, 65, 31, 0, 32, 0, 0, 0, 0, 0), 256, 768), ((128, 0, 0, 0, 33, 1, 0, 0, 0, 0, 0, 0), 512, 256),
+                                               ((129, 63, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0), 1280, 768)])
+def test_narrow_prefill_equals_wide(strix, counts, hidden, ffn):
+    E = len(counts)
+    assert sum(counts) <= 24 * E                                           # the narrow form's rule
+    gen = torch.Generator(device="cuda").manual_seed(hidden)
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    gate, up, down = draw(E * ffn, hidden), draw(E * ffn, hidden), draw(E * hidden, ffn)
+    ids = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)], dtype=torch.int32)[:, None]
+    ids = ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(1))].cuda()
+    T = len(ids)
+    x = torch.randn((T, hidden), device="cuda", generator=gen).to(torch.float16)
+    ones = torch.ones((T, 1), device="cuda")
+    narrow = strix.MoeLayer(hidden, ffn, E, 1, gate, up, down, T, prefill_f16=True).run_prefill_f16(x, ids, ones)
+    for e in {int(i) for i in ids.flatten()}:                              # expert by expert as one-expert layers: the wide form past 24 rows
+        rows = (ids[:, 0] == e).nonzero()[:, 0]
+        pick = lambda t, n: t[e * n:(e + 1) * n].contiguous()
+        alone = strix.MoeLayer(hidden, ffn, 1, 1, pick(gate, ffn), pick(up, ffn), pick(down, hidden), len(rows), prefill_f16=True)
+        got = alone.run_prefill_f16(x[rows].contiguous(), torch.zeros_like(ids[rows]), ones[rows])
+        assert torch.equal(got, narrow[rows])                              # the same products and sums in the same order
