@@ -432,9 +432,10 @@ int32_t a8_probe(const mi355_a8_request* q, const mi355_a8_bindings* b, uint32_t
     r.inter_rs = 4ULL * s.top_k * r.slot_stride;
     r.union_plan = union_plan;
     const uint32_t items = R * s.top_k;
-    // the holders of an entry share the sweeps of its expert's rows, four to a sweep (a fifth holder starts a second pass, which
-    // the cache serves: 8 rows x top-16 over 64 experts take 51.2 us this way against 55.6 us with eight-row sweeps)
-    if (union_plan) launch_project_nb<4>(w, r, R, dim3(s.rows / 32U, items), st);
+    // the holders of an entry share the matrix-core sweeps of its expert's rows, four to a sweep (a fifth holder starts a second pass, which
+    // the cache serves). The three calls, Q6_K down, sweeps of four | of eight | the vector ALU's of four: 6 rows x top-16 over 64 experts of
+    // 1536 x 1536 76 | 85 | 84 us, 8 rows x top-8 over 30 experts of 4096 x 2048 138 | 141 | 167 us
+    if (union_plan) launch_mma_project(w, r, R, 0, items, 4U, st);
     else if (q->gate_type == MI355_TYPE_Q5_K) project_q5k_kernel<4><<<dim3(s.rows / 32U, items), 256, 0, st>>>(w, r, items);
     else if (items <= 16U) project_quad_kernel<4><<<dim3(s.rows / 32U, items), 256, 0, st>>>(w, r, items);
     else if (items <= kQuadMaxItems) project_quad_kernel<2><<<dim3(s.rows / 32U, items), 256, 0, st>>>(w, r, items);

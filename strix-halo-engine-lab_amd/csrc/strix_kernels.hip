@@ -1650,15 +1650,33 @@ inline void launch_down_dense(const mi355_moe_weights& w, const RowsK& r, uint32
 inline bool mma_dense(const mi355_moe_weights& w, const RowsK& r, uint32_t rows) {
     return w.gate_type == MI355_TYPE_Q4_K && w.down_type == MI355_TYPE_Q4_K && w.experts == 1U && w.top_k == 1U && rows >= 3U && !r.assignments;
 }
-// Routed experts of a batch past the decode sizes whose experts hold several rows each on average: the plan cuts an expert's
-// rows into items of this many (0: the vector-ALU sweeps serve the batch).
+// A decode batch whose expert's gate + up rows are several MB: one expert is swept once for the rows that chose it.
+inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows);
+inline bool large_expert(const mi355_moe_weights& w) { return 2ULL * w.ffn * (w.hidden / 256U) * kQ4kBlock >= (4ULL << 20); }
+// Routed experts with Q4_K gate / up rows, past the decode sizes or over large experts: the plan cuts an expert's rows into items of this
+// many for the matrix-core sweeps (0: the vector-ALU sweeps serve the batch). The sweeps are bound by latency, so the narrow instances
+// (4 or 8 rows: 128 or 151 registers, four or three waves per SIMD) win while an expert holds few rows, and even one row per expert is
+// better off here than on the vector-ALU sweep. Layer times, hidden 2048 / ffn 768 / 128 experts top-8, items of 4 rows | of 16 in sweeps of 8 |
+// in sweeps of 16 (vector-ALU sweep, which served up to 4 rows per expert): 17 rows 88 | - | 130 us (109), 28 rows 101 | 114 | 152 (126), 40
+// rows 118 | 126 | 167 (147), 60 rows 141 | 139 | 181 (171), 100 rows 177 | 163 | 189, 200 rows 266 | 220 | 218, 400 rows 445 | 340 | 337; hidden
+// 4096 / ffn 1536 / 64 experts: 24 rows 200 | 204 | 282 (260), 60 rows 300 | 267 | 288, 150 rows 550 | 439 | 414. A decode batch over large
+// experts keeps its items of two rows: one rank's half of hidden 6144 / ffn 2560 / 160 experts, 7, 10, 16 rows: 189, 231, 306 us against 199,
+// 251, 320. Down rows of another format run on their own sweeps of four rows, so items stay at four there (hidden 2048 / ffn 768 / 128
+// experts, Q6_K down, 30, 100, 300, 1000 rows: 117, 193, 394, 1101 us against 141, 234, 484, 1374; Q8_0 down 130, 217, 441, 1203 against 157, 259,
+// 532, 1474).
 // Items of up to four 32-row sweeps: the later sweeps of a tile's weights hit the cache, and an expert with thousands of rows
 // still spreads over many workgroups.
 constexpr uint32_t kMmaItemRows = 128;
 inline uint32_t mma_grouped_split(const mi355_moe_weights& w, uint32_t rows) {
-    if (w.gate_type != MI355_TYPE_Q4_K || w.down_type != MI355_TYPE_Q4_K || w.experts == 1U || rows <= kFusedMaxRows) return 0U;
+    if (w.gate_type != MI355_TYPE_Q4_K || w.experts == 1U) return 0U;
+    if (rows <= kFusedMaxRows) return w.down_type == MI355_TYPE_Q4_K && !quad_sweep(w, rows) && large_expert(w) ? 2U : 0U;
     const uint64_t assignments = static_cast<uint64_t>(rows) * w.top_k;
-    return assignments >= 16ULL * w.experts ? kMmaItemRows : assignments >= 4ULL * w.experts ? 16U : 0U;
+    if (w.down_type != MI355_TYPE_Q4_K || assignments < 4ULL * w.experts) return 4U;
+    return assignments < 16ULL * w.experts ? 16U : kMmaItemRows;
+}
+// rows of one sweep over such an item
+inline uint32_t mma_sweep_rows(const mi355_moe_weights& w, uint32_t rows, uint32_t split) {
+    return split == 16U && static_cast<uint64_t>(rows) * w.top_k < 12ULL * w.experts ? 8U : split;
 }
 // A dense FFN's gate and up rows as raw values into the intermediates, then the SwiGLU / A8 kernel (5..16 rows, one chunk).
 inline void launch_mma_gate_up(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, hipStream_t st) {
@@ -1701,7 +1719,7 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
         if (rows > 4U && rows <= 16U && r.gate_out && r.up_out && dense_rows(r, w)) return launch_mma_gate_up(w, r, rows, st);
         return launch_mma_project(w, r, rows, rows, 0, rows, st);
     }
-    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) return launch_mma_project(w, r, rows, 0, umax, split, st);
+    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) return launch_mma_project(w, r, rows, 0, umax, mma_sweep_rows(w, rows, split), st);
     if (dense_pairs_ok(w, rows) && dense_rows(r, w) && r.gate_out && r.up_out) return launch_project_dense(w, r, rows, st);
     const dim3 grid(w.ffn / 32U, umax);
     if (w.experts == 1U && rows > 4U) launch_project_nb<8>(w, r, rows, grid, st);
@@ -1731,7 +1749,7 @@ inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t row
     if (mma_dense(w, r, rows)) { launch_mma_down(w, r, rows, rows, 0, rows, st); return r.top1_form != 0; }
     RowsK plain = r;
     plain.top1_form = 0;
-    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) { launch_mma_down(w, plain, rows, 0, umax, split, st); return false; }
+    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) { launch_mma_down(w, plain, rows, 0, umax, mma_sweep_rows(w, rows, split), st); return false; }
     if (dense_pairs_ok(w, rows) && dense_rows(r, w)) { launch_down_dense(w, r, rows, st); return r.top1_form != 0; }
     const dim3 grid(w.hidden / 64U, umax);
     if (w.experts == 1U && rows > 4U) launch_down_nb<8>(w, r, rows, grid, st);
@@ -1747,10 +1765,9 @@ inline uint32_t plan_split(const mi355_moe_weights& w, uint32_t rows) {
     if (rows > kFusedMaxRows) return 4U;
     if (quad_sweep(w, rows)) return 1U;       // the 16-rows-per-wavefront sweep serves one assignment per item
     // decode batches: one item per assignment while an expert's gate + up rows are a few MB (the second sweep of an expert
-    // that two rows chose is a cache hit and the short instruction streams finish sooner); larger experts are swept once
-    // for every two rows that chose them (hidden 6144, ffn 1280, 16 rows: 384 -> 351 us)
-    const uint64_t sweep_bytes = 2ULL * w.ffn * (w.hidden / 256U) * kQ4kBlock;
-    return sweep_bytes >= (4ULL << 20) ? 2U : 1U;
+    // that two rows chose is a cache hit and the short instruction streams finish sooner); larger experts that the matrix-core sweeps
+    // do not take are swept once for every two rows that chose them (hidden 6144, ffn 1280, 16 rows: 384 -> 351 us)
+    return large_expert(w) ? 2U : 1U;
 }
 inline uint32_t item_bound(const mi355_moe_weights& w, uint32_t rows) {
     return plan_item_bound(w.experts, rows * w.top_k, plan_split(w, rows));

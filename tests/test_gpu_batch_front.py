@@ -95,3 +95,44 @@ def test_narrow_prefill_equals_wide(strix, counts, hidden, ffn):
         alone = strix.MoeLayer(hidden, ffn, 1, 1, pick(gate, ffn), pick(up, ffn), pick(down, hidden), len(rows), prefill_f16=True)
         got = alone.run_prefill_f16(x[rows].contiguous(), torch.zeros_like(ids[rows]), ones[rows])
         assert torch.equal(got, narrow[rows])                              # the same products and sums in the same order
+
+
+# rows per expert around the lines between items of 4, 8, 16 and 128 rows (3, 12 and 16 rows per expert; 8 with another down format), experts
+# with none and with all of the rows, decode batches over large experts (3 and 16 rows more than the small-batch sweeps take); against
+# batches of two rows, which the vector-ALU sweeps serve
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,down", [(17, 512, 256, 40, 2, "q4_k"), (23, 256, 512, 16, 2, "q4_k"), (24, 512, 256, 16, 2, "q4_k"), (95, 256, 256, 8, 1, "q4_k"),
+                                                                (96, 512, 256, 8, 1, "q4_k"), (65, 256, 256, 8, 2, "q4_k"), (31, 512, 256, 8, 2, "q6_k"), (33, 256, 512, 8, 2, "q8_0"),
+                                                                (33, 256, 256, 40, 8, "q5_1"), (13, 4096, 1024, 12, 4, "q4_k"), (16, 3072, 1280, 30, 8, "q4_k")])
+@pytest.mark.parametrize("skew", [False, True])
+def test_batches_equal_pairs_of_rows(strix, rows, hidden, ffn, experts, top_k, down, skew):
+    gen = torch.Generator(device="cuda").manual_seed(rows * hidden + skew)
+    kind = {"q4_k": strix.TYPE_Q4_K, "q6_k": strix.TYPE_Q6_K, "q8_0": strix.TYPE_Q8_0, "q5_1": strix.TYPE_Q5_1}[down]
+    draw = lambda t, n, m: strix.quantize_weight_rows(t, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    if down in ("q4_k", "q8_0"):
+        wd = draw(kind, experts * hidden, ffn)
+    else:                                                                  # random blocks with small finite scales
+        size, per, scales, high = {"q6_k": (210, 256, (209,), 0x08), "q5_1": (24, 32, (1, 3), 0x14)}[down]
+        wd = torch.randint(0, 256, (experts * hidden, ffn // per, size), dtype=torch.uint8, device="cuda", generator=gen)
+        for at in scales:
+            wd[..., at] = (wd[..., at] & 0x03) | high
+        wd = wd.reshape(experts * hidden, -1)
+    gate, up = draw(strix.TYPE_Q4_K, experts * ffn, hidden), draw(strix.TYPE_Q4_K, experts * ffn, hidden)
+    gate.view(-1, 144)[5, :2] = torch.tensor([0x00, 0x7C], dtype=torch.uint8, device="cuda")           # one infinite scale: a flagged projection
+    make = lambda n: strix.MoeLayer(hidden, ffn, experts, top_k, gate, up, wd, n, down_type=kind)
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+    score = torch.rand((rows, experts), device="cuda", generator=gen)
+    if skew:
+        score[:, experts - top_k:] += 2.0                                  # every row on the same experts, none of them expert 0
+    score[:, 0] = -1.0                                                     # (expert 0 holds the infinite scale)
+    ids = score.topk(top_k, dim=1).indices.to(torch.int32)
+    w = torch.rand((rows, top_k), device="cuda", generator=gen)
+    layer, pair = make(rows), make(2)
+    same = lambda a, b: torch.equal(a.contiguous().view(torch.int32), b.contiguous().view(torch.int32))
+    out = layer.run(x, ids, w)
+    assert int(layer.status[:rows].sum()) == 0
+    for r in range(0, rows - 1, max(2, rows // 8)):
+        assert same(out[r:r + 2], pair.run(x[r:r + 2], ids[r:r + 2].contiguous(), w[r:r + 2].contiguous()))
+    ids[rows // 2, 0] = 0
+    layer.run(x, ids, w)
+    nonfinite = strix.STATUS_NONFINITE_PROJECTION
+    assert [s & nonfinite for s in layer.status[:rows].cpu().tolist()] == [nonfinite if r == rows // 2 else 0 for r in range(rows)]
