@@ -348,15 +348,18 @@ __device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slot
                 chain_widen<KIND, NORM>(slot, r, a.norm_w != nullptr);
                 const uint32_t kc = a.hidden - c * kChainChunk < kChainChunk ? a.hidden - c * kChainChunk : kChainChunk;
                 if (!butterfly) {
-                    if (kc == kChainChunk) {      // full chunk: straight-line code, operands fetched 48 features ahead
-                        ChainStep S[4];
+                    // full chunk: straight-line code, operands fetched ahead: three steps of 16 features beside the norm, one without it
+                    // (6 rows, hidden 4096, no norm: three steps 74.9, one 74.7 us a layer)
+                    constexpr uint32_t AHEAD = NORM ? 3U : 1U;
+                    if (kc == kChainChunk) {
+                        ChainStep S[AHEAD + 1U];
 #pragma unroll
-                        for (uint32_t i = 0; i < 3U; ++i) chain_load(S[i], slot, el, 16U * i);
+                        for (uint32_t i = 0; i < AHEAD; ++i) chain_load(S[i], slot, el, 16U * i);
 #pragma unroll
                         for (uint32_t i = 0; i < kChainChunk / 16U; ++i) {    // the barriers pin "fetch, then chain"
-                            if (i + 3U < kChainChunk / 16U) chain_load(S[(i + 3U) & 3U], slot, el, 16U * (i + 3U));
+                            if (i + AHEAD < kChainChunk / 16U) chain_load(S[(i + AHEAD) & AHEAD], slot, el, 16U * (i + AHEAD));
                             __builtin_amdgcn_sched_barrier(0);
-                            acc = chain_run(S[i & 3U], acc);
+                            acc = chain_run(S[i & AHEAD], acc);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     } else {                      // the last, partial chunk of the row
