@@ -170,6 +170,7 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
     else if (v->rows == 2U) launch(std::integral_constant<int, 2>{});
     else if (v->rows <= 4U) launch(std::integral_constant<int, 4>{});
     else if (v->rows <= 8U) launch(std::integral_constant<int, 8>{});
+    else if (v->in == 0U) launch(std::integral_constant<int, 16>{});        // (an empty reduction: the tiles' loaders read a group before they count any)
     else {
         // Tiles of 64 weight rows x 64 activation rows where they fill the compute units, 32 weight rows (K split over twice the waves)
         // where they do not; 32 activation rows for a batch that fits them. (4096 x 4096: 12 rows 13.1 us on the row sweep and 12.8 on the

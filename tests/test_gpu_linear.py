@@ -79,3 +79,16 @@ def test_products_of_full_range_codes_and_wide_factors(strix):
     want, _ = orc.gemv_q8_0_a8(w.reshape(count, -1), codes, deltas, width, count, threads=8)
     got = strix.gemv_q8_0_a8(dev(w.reshape(count, -1)), dev(codes), dev(deltas), width, count).cpu().numpy()
     assert np.array_equal(bits(got), bits(want))
+
+
+@pytest.mark.parametrize("rows", [1, 9, 40, 300])
+def test_products_of_width_zero(strix, rows):
+    """An empty reduction is +0 stored, or the accumulated value left as it is, for any number of rows."""
+    count = 70
+    w, codes = torch.zeros((count, 34), dtype=torch.uint8, device="cuda"), torch.ones((rows, 32), dtype=torch.int8, device="cuda")
+    deltas = torch.ones((rows, 1), device="cuda")
+    out = torch.full((rows, count), 3.0, device="cuda")
+    strix.gemv_q8_0_a8(w, codes, deltas, 0, count, out=out, row_bytes_=34, accumulate=True)
+    assert torch.all(out == 3.0)
+    strix.gemv_q8_0_a8(w, codes, deltas, 0, count, out=out, row_bytes_=34)
+    assert np.all(bits(out.cpu().numpy()) == 0)
