@@ -231,12 +231,26 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
     }
 }
 
+// Workgroups of a product, and whether the tiles take it: an empty reduction has no group for the loaders to fetch, and a launch counts its
+// threads in 32 bits, which tiles of 64 x 64 outputs reach at 2^35 outputs (the row sweep's second grid dimension goes on from there).
 template <int KS, int NA>
-inline void launch_gemm_q8_0(const mi355_q8a8_view& v, bool dw, hipStream_t st) {
+constexpr uint64_t gemm_blocks(uint32_t count, uint32_t rows) {
+    return (static_cast<uint64_t>(count) + 8U * gemm_out_rows<KS>() - 1U) / (8U * gemm_out_rows<KS>()) * 8U * ((rows + 32U * NA - 1U) / (32U * NA));
+}
+template <int KS, int NA>
+constexpr bool gemm_takes(uint32_t in, uint32_t count, uint32_t rows) { return in != 0U && gemm_blocks<KS, NA>(count, rows) * kGemmThreads <= 0xffffffffULL; }
+static_assert(!gemm_takes<8, 1>(0U, 70U, 9U) && !gemm_takes<4, 2>(0U, 70U, 4096U) && gemm_takes<4, 2>(32U, 16384U, 65536U));
+static_assert(gemm_takes<4, 2>(32U, 32768U, 1048512U) && !gemm_takes<4, 2>(32U, 32768U, 1048560U) && !gemm_takes<4, 2>(32U, 1U << 27, 4096U * 64U));
+
+// false: the row sweep serves the product
+template <int KS, int NA>
+inline bool launch_gemm_q8_0(const mi355_q8a8_view& v, bool dw, hipStream_t st) {
+    if (!gemm_takes<KS, NA>(v.in, v.count, v.rows)) return false;
     const uint32_t o_tiles = (v.count + gemm_out_rows<KS>() - 1U) / gemm_out_rows<KS>(), a_tiles = (v.rows + 32U * NA - 1U) / (32U * NA);
-    const uint32_t blocks = (o_tiles + 7U) / 8U * 8U * a_tiles;
+    const uint32_t blocks = static_cast<uint32_t>(gemm_blocks<KS, NA>(v.count, v.rows));
     if (dw) gemm_q8_0_a8_kernel<KS, NA, true><<<blocks, kGemmThreads, 0, st>>>(v, o_tiles, a_tiles);
     else gemm_q8_0_a8_kernel<KS, NA, false><<<blocks, kGemmThreads, 0, st>>>(v, o_tiles, a_tiles);
+    return true;
 }
 
 }  // namespace strix950

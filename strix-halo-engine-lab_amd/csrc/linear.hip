@@ -170,15 +170,14 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
     else if (v->rows == 2U) launch(std::integral_constant<int, 2>{});
     else if (v->rows <= 4U) launch(std::integral_constant<int, 4>{});
     else if (v->rows <= 8U) launch(std::integral_constant<int, 8>{});
-    else if (v->in == 0U) launch(std::integral_constant<int, 16>{});        // (an empty reduction: the tiles' loaders read a group before they count any)
     else {
         // Tiles of 64 weight rows x 64 activation rows where they fill the compute units, 32 weight rows (K split over twice the waves)
         // where they do not; 32 activation rows for a batch that fits them. (4096 x 4096: 12 rows 13.1 us on the row sweep and 12.8 on the
-        // matrix cores, 16384 x 8192: 78 and 46 us; 8 rows 8.8 and 12.7 us.)
+        // matrix cores, 16384 x 8192: 78 and 46 us; 8 rows 8.8 and 12.7 us.) What the tiles do not take stays on the row sweep.
         const uint64_t wide = static_cast<uint64_t>((v->count + 63U) / 64U) * ((v->rows + 63U) / 64U);
-        if (v->rows <= 32U) launch_gemm_q8_0<8, 1>(*v, dw, st);
-        else if (wide < compute_units()) launch_gemm_q8_0<8, 2>(*v, dw, st);
-        else launch_gemm_q8_0<4, 2>(*v, dw, st);
+        const bool taken = v->rows <= 32U ? launch_gemm_q8_0<8, 1>(*v, dw, st)
+                           : wide < compute_units() ? launch_gemm_q8_0<8, 2>(*v, dw, st) : launch_gemm_q8_0<4, 2>(*v, dw, st);
+        if (!taken) launch(std::integral_constant<int, 16>{});
     }
     STRIX_LAUNCHED("gemv_q8_0_a8");
     return MI355_OK;
