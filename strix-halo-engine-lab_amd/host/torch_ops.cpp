@@ -2,6 +2,7 @@
 // takes a few microseconds on the GPU cost several times that when every step of them is a Python call (4096 x 4096, one row: 31.7 us a
 // pair of calls with ctypes and torch.zeros, two fill kernels among them). Each function returns its tensors, or the C ABI's error code
 // as an int, which the Python side turns into its exception; what torch throws keeps its Python type (torch.OutOfMemoryError, IndexError, ...).
+// Other Python threads run while a call allocates and enqueues.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -24,7 +25,6 @@ bool unsigned_arg(PyObject* o, uint64_t& v) {
     v = PyLong_AsUnsignedLongLongMask(o);
     return !PyErr_Occurred();
 }
-
 bool truth_arg(PyObject* o, bool& v) {
     const int truth = PyObject_IsTrue(o);
     v = truth > 0;
@@ -47,16 +47,22 @@ PyObject* quantize_a8(PyObject*, PyObject* const* args, Py_ssize_t n) {
     case at::kBFloat16: kind = MI355_INPUT_BF16; break;
     default: PyErr_SetString(PyExc_KeyError, "x must be float32, float16 or bfloat16"); return nullptr;
     }
-    const int64_t rows = x->size(0), width = x->size(1), groups = width / 32;
-    const auto like = x->options().requires_grad(false);
-    at::Tensor codes = at::empty({rows, width}, like.dtype(at::kChar)), deltas = at::empty({rows, groups}, like.dtype(at::kFloat));
-    at::Tensor sums = want_sums ? at::empty({rows, groups}, like.dtype(at::kInt)) : at::Tensor();
-    at::Tensor status = at::empty({rows}, like.dtype(at::kInt));
-    if (width == 0) status.zero_();          // (no launch for rows without values)
-    const int32_t rc = mi355_quantize_a8_fresh(x->data_ptr(), kind, static_cast<uint32_t>(rows), static_cast<uint32_t>(width),
-                                               static_cast<uint64_t>(x->stride(0)) * x->element_size(), static_cast<int8_t*>(codes.data_ptr()),
-                                               static_cast<float*>(deltas.data_ptr()), want_sums ? static_cast<int32_t*>(sums.data_ptr()) : nullptr,
-                                               static_cast<uint32_t*>(status.data_ptr()), current_stream());
+    at::Tensor codes, deltas, sums, status;
+    int32_t rc;
+    {
+        pybind11::gil_scoped_release others;
+        const int64_t rows = x->size(0), width = x->size(1), groups = width / 32;
+        const auto like = x->options().requires_grad(false);
+        codes = at::empty({rows, width}, like.dtype(at::kChar));
+        deltas = at::empty({rows, groups}, like.dtype(at::kFloat));
+        if (want_sums) sums = at::empty({rows, groups}, like.dtype(at::kInt));
+        status = at::empty({rows}, like.dtype(at::kInt));
+        if (width == 0) status.zero_();      // (no launch for rows without values)
+        rc = mi355_quantize_a8_fresh(x->data_ptr(), kind, static_cast<uint32_t>(rows), static_cast<uint32_t>(width),
+                                     static_cast<uint64_t>(x->stride(0)) * x->element_size(), static_cast<int8_t*>(codes.data_ptr()),
+                                     static_cast<float*>(deltas.data_ptr()), want_sums ? static_cast<int32_t*>(sums.data_ptr()) : nullptr,
+                                     static_cast<uint32_t*>(status.data_ptr()), current_stream());
+    }
     if (rc != 0) return PyLong_FromLong(rc);
     PyObject* out = PyTuple_New(4);
     PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(codes)));
@@ -79,19 +85,23 @@ PyObject* gemv_q8_0_a8(PyObject*, PyObject* const* args, Py_ssize_t n) {
         !unsigned_arg(args[3], n_in) || !unsigned_arg(args[4], count) || (args[5] != Py_None && !tensor_arg(args[5], "out", given)) ||
         !truth_arg(args[6], accumulate) || !unsigned_arg(args[7], row_bytes) || !unsigned_arg(args[8], out_stride))
         return nullptr;
-    const int64_t rows = codes->size(0);
     at::Tensor out;
-    if (given) out = *given;
-    else {
-        out = at::empty({rows, static_cast<int64_t>(count)}, codes->options().requires_grad(false).dtype(at::kFloat));
-        if (accumulate) out.zero_();         // (otherwise the launch writes every value)
+    int32_t rc;
+    {
+        pybind11::gil_scoped_release others;
+        const int64_t rows = codes->size(0);
+        if (given) out = *given;
+        else {
+            out = at::empty({rows, static_cast<int64_t>(count)}, codes->options().requires_grad(false).dtype(at::kFloat));
+            if (accumulate) out.zero_();     // (otherwise the launch writes every value)
+        }
+        const mi355_q8a8_view v{static_cast<const uint8_t*>(weight->data_ptr()), static_cast<const int8_t*>(codes->data_ptr()),
+                                static_cast<const float*>(deltas->data_ptr()), static_cast<float*>(out.data_ptr()),
+                                static_cast<uint32_t>(row_bytes ? row_bytes : n_in / 32U * 34U), static_cast<uint32_t>(n_in), static_cast<uint32_t>(count),
+                                static_cast<uint32_t>(rows), static_cast<uint32_t>(codes->size(1)), static_cast<uint32_t>(out_stride ? out_stride : out.size(1)),
+                                accumulate ? 1U : 0U};
+        rc = mi355_gemv_q8_0_a8(&v, current_stream());
     }
-    const mi355_q8a8_view v{static_cast<const uint8_t*>(weight->data_ptr()), static_cast<const int8_t*>(codes->data_ptr()),
-                            static_cast<const float*>(deltas->data_ptr()), static_cast<float*>(out.data_ptr()),
-                            static_cast<uint32_t>(row_bytes ? row_bytes : n_in / 32U * 34U), static_cast<uint32_t>(n_in), static_cast<uint32_t>(count),
-                            static_cast<uint32_t>(rows), static_cast<uint32_t>(codes->size(1)), static_cast<uint32_t>(out_stride ? out_stride : out.size(1)),
-                            accumulate ? 1U : 0U};
-    const int32_t rc = mi355_gemv_q8_0_a8(&v, current_stream());
     if (rc != 0) return PyLong_FromLong(rc);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS

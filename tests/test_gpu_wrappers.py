@@ -1,4 +1,9 @@
-"""The native wrappers (host/torch_ops.cpp) as Python callers see them: torch's own exception types come through."""
+"""The native wrappers (host/torch_ops.cpp) as Python callers see them: torch's own exception types come through, and other threads
+run during a call."""
+import sys
+import threading
+import time
+
 import pytest
 import torch
 
@@ -31,3 +36,35 @@ def test_shape_errors_keep_their_type(strix):
         strix.gemv_q8_0_a8(w, codes[0], deltas, width, count)
     with pytest.raises(RuntimeError, match="ambiguous"):
         strix.gemv_q8_0_a8(w, codes, deltas, width, count, accumulate=torch.ones(2))
+
+
+def test_other_threads_run_during_a_call(strix):
+    """With a switch interval longer than the test only a call that gives the interpreter up lets the other thread in."""
+    args = product(strix)
+    x = torch.randn((3, 64), device="cuda")
+    interval, turns, stop = sys.getswitchinterval(), [0], threading.Event()
+
+    def count():
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    for call in (lambda: strix.quantize_a8(x), lambda: strix.gemv_q8_0_a8(*args)):
+        stop.clear()
+        thread = threading.Thread(target=count)
+        thread.start()
+        try:
+            sys.setswitchinterval(1000.0)
+            time.sleep(0.05)                   # (a wait that the thread began before still ends after the old interval)
+            before = turns[0]
+            for _ in range(5000):
+                call()
+                if turns[0] != before:
+                    break
+            after = turns[0]
+        finally:
+            sys.setswitchinterval(interval)
+            stop.set()
+            thread.join()
+        assert after > before
+    torch.cuda.synchronize()
