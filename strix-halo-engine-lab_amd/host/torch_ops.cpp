@@ -15,11 +15,13 @@ namespace {
 
 mi355_stream current_stream() { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
-bool tensor_arg(PyObject* o, const char* what, const at::Tensor*& t) {
+// host: pinned host memory, which the GPU reaches, will do
+bool tensor_arg(PyObject* o, const char* what, const at::Tensor*& t, bool host) {
     if (!THPVariable_Check(o)) { PyErr_Format(PyExc_TypeError, "%s must be a tensor", what); return false; }
     t = &THPVariable_Unpack(o);
-    if (!t->is_cuda()) { PyErr_Format(PyExc_RuntimeError, "%s must be on the GPU", what); return false; }
-    return true;
+    if (t->is_cuda() || (host && t->is_pinned())) return true;
+    PyErr_Format(PyExc_RuntimeError, host ? "%s must be on the GPU or in pinned memory" : "%s must be on the GPU", what);
+    return false;
 }
 bool unsigned_arg(PyObject* o, uint64_t& v) {
     v = PyLong_AsUnsignedLongLongMask(o);
@@ -36,7 +38,7 @@ PyObject* quantize_a8(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     const at::Tensor* x;
     if (n != 2) { PyErr_SetString(PyExc_TypeError, "quantize_a8 takes 2 arguments"); return nullptr; }
-    if (!tensor_arg(args[0], "x", x)) return nullptr;
+    if (!tensor_arg(args[0], "x", x, false)) return nullptr;
     if (x->dim() != 2 || x->stride(1) != 1) { PyErr_SetString(PyExc_AssertionError, "x must be rows of contiguous values"); return nullptr; }
     bool want_sums;
     if (!truth_arg(args[1], want_sums)) return nullptr;
@@ -81,8 +83,9 @@ PyObject* gemv_q8_0_a8(PyObject*, PyObject* const* args, Py_ssize_t n) {
     uint64_t n_in, count, row_bytes, out_stride;
     bool accumulate;
     if (n != 9) { PyErr_SetString(PyExc_TypeError, "gemv_q8_0_a8 takes 9 arguments"); return nullptr; }
-    if (!tensor_arg(args[0], "weight", weight) || !tensor_arg(args[1], "codes", codes) || !tensor_arg(args[2], "deltas", deltas) ||
-        !unsigned_arg(args[3], n_in) || !unsigned_arg(args[4], count) || (args[5] != Py_None && !tensor_arg(args[5], "out", given)) ||
+    // (an output made here lives where the codes do)
+    if (!tensor_arg(args[0], "weight", weight, true) || !tensor_arg(args[1], "codes", codes, args[5] != Py_None) || !tensor_arg(args[2], "deltas", deltas, true) ||
+        !unsigned_arg(args[3], n_in) || !unsigned_arg(args[4], count) || (args[5] != Py_None && !tensor_arg(args[5], "out", given, true)) ||
         !truth_arg(args[6], accumulate) || !unsigned_arg(args[7], row_bytes) || !unsigned_arg(args[8], out_stride))
         return nullptr;
     at::Tensor out;

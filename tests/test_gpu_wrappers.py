@@ -68,3 +68,25 @@ def test_other_threads_run_during_a_call(strix):
             thread.join()
         assert after > before
     torch.cuda.synchronize()
+
+
+def test_operands_in_pinned_host_memory(strix):
+    """The product reads and writes host memory that the GPU can reach; memory that it cannot is refused."""
+    w, codes, deltas, width, count = product(strix)
+    want = strix.gemv_q8_0_a8(w, codes, deltas, width, count)
+
+    def pinned(t):
+        host = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)
+        host.copy_(t)
+        return host
+
+    assert torch.equal(strix.gemv_q8_0_a8(pinned(w), codes, pinned(deltas), width, count), want)
+    out = pinned(torch.zeros_like(want))
+    strix.gemv_q8_0_a8(pinned(w), pinned(codes), deltas, width, count, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want.cpu())
+    for bad in ((w.cpu(), codes, deltas), (w, codes.cpu(), deltas), (w, codes, deltas.cpu()), (w, pinned(codes), deltas)):
+        with pytest.raises(RuntimeError, match="GPU"):      # (the last has nowhere to put its output)
+            strix.gemv_q8_0_a8(*bad, width, count)
+    with pytest.raises(RuntimeError, match="GPU"):
+        strix.gemv_q8_0_a8(w, codes, deltas, width, count, out=want.cpu())
