@@ -174,7 +174,7 @@ __device__ __forceinline__ void route_logits_block(RouteLds& lds, const RouteArg
 // row stream global -> LDS by global_load_lds_dwordx4 in chunks of 512 features through a ring of 4 slots (three chunks
 // in flight during a chunk's chain, waits counted with s_waitcnt vmcnt); fp16 / bf16 activations are widened to fp32 in
 // LDS once per chunk (a widening fma, v_fma_mix_f32, more than doubles the latency of a chain step); a lane reads its
-// operands 32 features ahead of the chain with 128-bit LDS loads (the activation read is a broadcast).
+// operands up to 48 features ahead of the chain with 128-bit LDS loads (the activation read is a broadcast).
 // Lanes 8..63 repeat lanes 0..7 (a chain gains nothing from idle lanes).
 constexpr uint32_t kChainChunk = 512;                 // features per ring slot
 constexpr uint32_t kChainPitch = kChainChunk + 4;     // floats; +16 bytes keeps the 8 weight rows on different banks
@@ -275,7 +275,7 @@ __device__ __forceinline__ void chain_widen(ChainSlotT<NORM>& slot, float factor
 // Operands of 16 features: four 128-bit LDS reads of the lane's weight row and one 32-bit read that leaves feature k + t
 // in lane t of every row of 16 lanes; the fma takes its activation operand from there by a row broadcast (a DPP operand,
 // no instruction of its own). Measured on MI355X a wave pays ~5 cycles per dependent fma and ~9 per ds_read_b128, with no
-// overlap between them; the operands of the next 16 features are requested before the current 16 are chained.
+// overlap between them; operands are requested up to 48 features before they are chained.
 struct ChainStep { f32x4 w[4]; float x; };
 template <bool NORM>
 __device__ __forceinline__ void chain_load(ChainStep& s, const ChainSlotT<NORM>& slot, uint32_t el, uint32_t k) {
@@ -348,9 +348,9 @@ __device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slot
                 chain_widen<KIND, NORM>(slot, r, a.norm_w != nullptr);
                 const uint32_t kc = a.hidden - c * kChainChunk < kChainChunk ? a.hidden - c * kChainChunk : kChainChunk;
                 if (!butterfly) {
-                    // full chunk: straight-line code, operands fetched ahead: three steps of 16 features beside the norm, one without it
-                    // (6 rows, hidden 4096, no norm: three steps 74.9, one 74.7 us a layer)
-                    constexpr uint32_t AHEAD = NORM ? 3U : 1U;
+                    // full chunk: straight-line code, operands fetched three steps of 16 features ahead (against one step: layers without the
+                    // norm 0.2..0.4 us faster, e.g. hidden 3072, 8 rows 75.1 -> 74.9; with it the same, 89.7; logits alone 0.1 us slower of 30)
+                    constexpr uint32_t AHEAD = 3U;
                     if (kc == kChainChunk) {
                         ChainStep S[AHEAD + 1U];
 #pragma unroll
