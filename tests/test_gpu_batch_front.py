@@ -136,3 +136,39 @@ def test_batches_equal_pairs_of_rows(strix, rows, hidden, ffn, experts, top_k, d
     layer.run(x, ids, w)
     nonfinite = strix.STATUS_NONFINITE_PROJECTION
     assert [s & nonfinite for s in layer.status[:rows].cpu().tolist()] == [nonfinite if r == rows // 2 else 0 for r in range(rows)]
+
+
+def test_batches_inside_a_captured_graph(strix):
+    """A staged layer with its router, a narrow prefill and a projection of many rows in one graph: every replay gives the eager bits,
+    with eager calls in between."""
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    hidden, ffn, experts, top_k, rows = 512, 256, 16, 4, 40
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    tensors = draw(experts * ffn, hidden), draw(experts * ffn, hidden), draw(experts * hidden, ffn)
+    layer, prompt = strix.MoeLayer(hidden, ffn, experts, top_k, *tensors, rows), strix.MoeLayer(hidden, ffn, experts, top_k, *tensors, rows, prefill_f16=True)
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    w8 = strix.quantize_weight_rows(strix.TYPE_Q8_0, torch.randn((96, hidden), device="cuda", generator=gen))
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+
+    def program():
+        y, ids, weights, scores = layer.run_layer(x, router)
+        codes, deltas, sums, status = strix.quantize_a8(x)
+        return [y, ids, weights, scores, prompt.run_prefill_f16(x, ids, weights), strix.gemv_q8_0_a8(w8, codes, deltas, hidden, 96), codes, deltas, sums, status]
+
+    want = [t.clone() for t in program()]
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        program()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        got = program()
+    for turn in range(4):
+        for t in got:
+            t.fill_(1)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8)), turn
+        layer.run_layer(x[: rows - turn].contiguous(), router)
+        torch.cuda.synchronize()

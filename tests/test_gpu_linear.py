@@ -92,3 +92,26 @@ def test_products_of_width_zero(strix, rows):
     assert torch.all(out == 3.0)
     strix.gemv_q8_0_a8(w, codes, deltas, 0, count, out=out, row_bytes_=34)
     assert np.all(bits(out.cpu().numpy()) == 0)
+
+
+def test_products_of_any_factors(strix):
+    """Infinite, NaN, zero and negative factors, activation rows with a stride, weight rows with padding: the row sweep's values (which
+    NaN survives where two meet is open)."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rows, width, count = 40, 1056, 100
+    blocks = strix.quantize_weight_rows(strix.TYPE_Q8_0, torch.randn((count, width), device="cuda", generator=gen) * 0.02).reshape(count, -1, 34)
+    for o, half in enumerate((0x7C00, 0xFC00, 0x7E00, 0x0000, 0x8000), start=1):
+        blocks[o, o, 0], blocks[o, o, 1] = half & 255, half >> 8
+    w = torch.zeros((count, width // 32 * 34 + 6), dtype=torch.uint8, device="cuda")
+    w[:, :-6] = blocks.reshape(count, -1)
+    codes = torch.randint(-127, 128, (rows, width + 64), dtype=torch.int8, device="cuda", generator=gen)
+    deltas = torch.rand((rows, (width + 64) // 32), device="cuda", generator=gen)
+    deltas[1, 3], deltas[2, 5], deltas[3, 6], deltas[4, 7], deltas[5], deltas[6], deltas[7] = float("inf"), float("nan"), -float("inf"), 0.0, 3e38, -1.0, -0.0
+    codes[8, :32], deltas[8, 0] = 0, float("inf")
+    product = lambda r0, r1: strix.gemv_q8_0_a8(w, codes[r0:r1], deltas[r0:r1], width, count, row_bytes_=w.shape[1])
+    want = torch.cat([product(r, r + 8) for r in range(0, rows, 8)])
+    for n in (9, 32, 33, 40):
+        got = product(0, n)
+        assert torch.equal(got.isnan(), want[:n].isnan())
+        clean = ~got.isnan()
+        assert torch.equal(got[clean].view(torch.int32), want[:n][clean].view(torch.int32))

@@ -36,3 +36,26 @@ def test_logits_of_a_batch(strix, rows, experts, hidden, top_k, dtype):
     ids_ref, w_ref, s_ref, _ = orc.route(x.float().numpy(), w.numpy(), top_k, bias=None if bias is None else bias.numpy())
     assert np.array_equal(bits(scores.cpu().numpy()), bits(s_ref))
     assert np.array_equal(ids.cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(bits(weights.cpu().numpy()), bits(w_ref))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_rows_of_any_values(strix, dtype):
+    """Infinities, NaN, zeros of both signs and values that overflow, in the rows and in the router weights, rows with a stride: the
+    bits of decode batches, whose chains run on the vector ALU."""
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    rows, experts, hidden, top_k = 40, 96, 1056, 4
+    inf, nan = float("inf"), float("nan")
+    wide = torch.randn((rows, hidden + 32), device="cuda", generator=gen)
+    x = wide[:, :hidden]
+    x[1, 5], x[2, 7], x[3, 9], x[4, 3], x[4, 100], x[5], x[6], x[7], x[8] = inf, -inf, nan, inf, -inf, inf, nan, 0.0, -0.0
+    x[9] *= 3e38
+    x[10] *= 1e-42
+    x = wide.to(dtype)[:, :hidden]
+    w = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    bad = w.clone()
+    bad[3, 2], bad[4, 2], bad[5, 5] = inf, nan, -inf
+    for router, bias in ((w, None), (w, torch.randn(experts, device="cuda", generator=gen)), (bad, None)):
+        batch = strix.route(x, router, top_k, bias=bias)
+        parts = [strix.route(x[r:r + 8].contiguous(), router, top_k, bias=bias) for r in range(0, rows, 8)]
+        for got, want in zip(batch, zip(*parts)):
+            assert torch.equal(got.view(torch.int32), torch.cat(want).view(torch.int32))

@@ -71,7 +71,10 @@ def weights_of(strix, H, I, E, K, gate, up, down, gate_type, down_type):
     (orc.Q4_K, orc.Q5_1, 2560, 640, 64, 10, 16, torch.bfloat16, torch.bfloat16),      # the twin's fixed geometry but for the expert count
     (orc.Q4_K, orc.Q6_K, 512, 768, 6, 3, 5, torch.float32, torch.float32),
     (orc.Q4_K, orc.Q4_K, 1024, 1024, 1, 1, 6, torch.bfloat16, torch.bfloat16),        # a dense matrix through strided views (matrix-core sweep)
-    (orc.Q4_K, orc.Q4_K, 512, 512, 4, 2, 40, torch.bfloat16, torch.float32)])         # 20 rows per expert: items of up to 128 rows on the matrix-core sweep
+    (orc.Q4_K, orc.Q4_K, 512, 512, 4, 2, 40, torch.bfloat16, torch.float32),          # 20 rows per expert: items of up to 128 rows on the matrix-core sweep
+    (orc.Q4_K, orc.Q4_K, 512, 256, 24, 2, 17, torch.float16, torch.float32),          # one or two rows per expert: items of four there
+    (orc.Q4_K, orc.Q6_K, 256, 512, 6, 2, 20, torch.bfloat16, torch.bfloat16),         # gate / up there, down rows in their own format
+    (orc.Q4_K, orc.Q4_K, 3072, 1280, 8, 4, 13, torch.bfloat16, torch.float32)])       # a decode batch over large experts: items of two
 def test_strided_rows_every_stage(strix, gate_type, down_type, H, I, E, K, T, in_kind, out_kind):
     rng = np.random.default_rng(H + I + 3 * T + down_type)
     if I % 256 == 0:
