@@ -10,7 +10,7 @@
 // sc_j q_k is an integer <= 945: exact in fp16, so P_b is an fp16 MFMA with fp32 accumulation whose only rounding is the
 // fp32 accumulation; d_b is applied in fp32 once per super-block. The second sum is a product over K / 32 sub-blocks:
 // S and M are each carried as two fp16 numbers (hi = fp16(v), lo = fp16(v - hi)) and multiplied by three MFMAs per 16
-// sub-blocks (hi*hi + lo*hi + hi*lo). S of the input rows comes from token_sums_kernel, S of h from the epilogue of
+// sub-blocks (hi*hi + lo*hi + hi*lo). S of the input rows comes from prefill_prologue_kernel, S of h from the epilogue of
 // the gate / up launch.
 //
 // Work decomposition. The expert plan cuts every expert's assignments into items of at most 128 rows. A 512-thread
