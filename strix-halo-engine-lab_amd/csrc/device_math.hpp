@@ -139,32 +139,45 @@ __device__ __forceinline__ void store_shared_or_plain(bool device_scope, T* p, T
 }
 
 // ---- cross-lane moves inside a 64-wide wavefront ----------------------------------------------------------------
-// lane ^ 1 and lane ^ 2 are DPP quad permutes (no LDS traffic); wider distances go through the swizzle crossbar.
+// Distances inside a row of 16 lanes are DPP moves (a modifier of the instruction that reads them, no LDS traffic): lane ^ 1 and lane ^ 2
+// are quad permutes, lane ^ 4 two mirrors, lane ^ 8 a rotation of the row by half its length.
 __device__ __forceinline__ int xor1_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true); }
 __device__ __forceinline__ int xor2_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true); }
 // lane ^ 4 inside a group of 8: mirror the 8 lanes (row_half_mirror), then reverse each quad - two DPP moves.
 __device__ __forceinline__ int xor4_i(int v) { return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true); }
-__device__ __forceinline__ int xor8_i(int v) { return __builtin_amdgcn_ds_swizzle(v, 0x201F); }
+__device__ __forceinline__ int xor8_i(int v) { return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true); }
 __device__ __forceinline__ int xor16_i(int v) { return __builtin_amdgcn_ds_swizzle(v, 0x401F); }
 __device__ __forceinline__ float xor1_f(float v) { return __builtin_bit_cast(float, xor1_i(__builtin_bit_cast(int, v))); }
 __device__ __forceinline__ float xor2_f(float v) { return __builtin_bit_cast(float, xor2_i(__builtin_bit_cast(int, v))); }
 __device__ __forceinline__ float xor4_f(float v) { return __builtin_bit_cast(float, xor4_i(__builtin_bit_cast(int, v))); }
 __device__ __forceinline__ float xor8_f(float v) { return __builtin_bit_cast(float, xor8_i(__builtin_bit_cast(int, v))); }
 __device__ __forceinline__ float xor16_f(float v) { return __builtin_bit_cast(float, xor16_i(__builtin_bit_cast(int, v))); }
+// The even and the odd row of 16 of every half wavefront, each in both rows (one swap between two registers).
+__device__ __forceinline__ void rows_of_16(uint32_t v, uint32_t& even, uint32_t& odd) {
+    const auto swapped = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    even = swapped[0]; odd = swapped[1];
+}
 
-// Reductions over an aligned group of 32 lanes (a half wavefront). max and integer sums are order-free.
+// Reductions over an aligned group of 32 lanes (a half wavefront). max, integer sums and bitwise or have no order, so the steps inside a
+// row of 16 are mirrors: once the quads (groups of 8) agree, the mirror of 8 (16) lanes pairs the two.
+template <class Combine>
+__device__ __forceinline__ uint32_t reduce32(uint32_t v, Combine combine) {
+    v = combine(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0xB1, 0xF, 0xF, true)));
+    v = combine(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x4E, 0xF, 0xF, true)));
+    v = combine(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x141, 0xF, 0xF, true)));
+    v = combine(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), 0x140, 0xF, 0xF, true)));
+    uint32_t even, odd;
+    rows_of_16(v, even, odd);
+    return combine(even, odd);
+}
 __device__ __forceinline__ float max32(float v) {
-    v = __builtin_fmaxf(v, xor1_f(v)); v = __builtin_fmaxf(v, xor2_f(v)); v = __builtin_fmaxf(v, xor4_f(v));
-    v = __builtin_fmaxf(v, xor8_f(v)); v = __builtin_fmaxf(v, xor16_f(v));
-    return v;
+    return f_of(reduce32(b_of(v), [](uint32_t a, uint32_t b) { return b_of(__builtin_fmaxf(f_of(a), f_of(b))); }));
 }
 __device__ __forceinline__ int sum32_i(int v) {
-    v += xor1_i(v); v += xor2_i(v); v += xor4_i(v); v += xor8_i(v); v += xor16_i(v);
-    return v;
+    return static_cast<int>(reduce32(static_cast<uint32_t>(v), [](uint32_t a, uint32_t b) { return a + b; }));
 }
 __device__ __forceinline__ int or32_i(int v) {
-    v |= xor1_i(v); v |= xor2_i(v); v |= xor4_i(v); v |= xor8_i(v); v |= xor16_i(v);
-    return v;
+    return static_cast<int>(reduce32(static_cast<uint32_t>(v), [](uint32_t a, uint32_t b) { return a | b; }));
 }
 
 // A8 code of one value under a group delta. Reference: src/cpu/core/reference.cpp:47-48.

@@ -5,23 +5,48 @@
 
 namespace strix950 {
 
+// Tiles a workgroup runs over: as many as make about `most` stages, where a tile has few. The ring then starts once for all of them, but a
+// workgroup's end is a step of the dispatch's balance, and the gate / up sweep (two matrices, 9 KB a stage) gains nothing from a longer
+// run than eight stages. Measured (layer, run 1 | 2 | 4): hidden 2048 / ffn 768 / 128 experts top-8, 40 rows, project 117.9 | 121.3 | 127.2
+// us, down (3 stages) 131.3 | 122.5 | 121.4; one rank's half of hidden 6144 / ffn 2560 / 160 experts, 16 rows, project 310.0 | 319.7 | 326.4,
+// down (5 stages) 332.0 | 315.4 | 316.0; 1000 rows of the first (items of up to four sweeps), project 552.9 | 566.2 | 625.6, down 584.0 |
+// 566.5 | 566.2.
+inline uint32_t mma_run_tiles(uint32_t stages, uint32_t most, uint64_t tiles) {
+    const uint32_t run = stages < most ? most / stages : 1U;
+    const uint64_t full = tiles / (8ULL * compute_units());
+    return run < full ? run : full > 1U ? static_cast<uint32_t>(full) : 1U;
+}
+struct MmaGrid { dim3 grid; MmaLaunch l; };
+inline MmaGrid mma_grid(const mi355_moe_weights& w, uint32_t rows, uint32_t dense, uint32_t items, uint32_t tiles, uint32_t acts, uint32_t run) {
+    return MmaGrid{dim3((tiles + run - 1U) / run, dense ? (dense + acts - 1U) / acts : items), MmaLaunch{rows * w.top_k, dense, tiles, run}};
+}
+// the rows of a dense batch at a stride of their own (every dense buffer and strided view; not the executor's pointer tables)
+inline bool mma_direct(const A8Image& img, uint32_t dense) { return dense && img.per_row == 1U && !img.table; }
 template <int NAL>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const dim3 grid(w.ffn / 32U, dense ? (dense + 2U * NAL - 1U) / (2U * NAL) : items);
-    q4k_mma_project_kernel<NAL, (NAL >= 8 ? 2 : 3)><<<grid, 256, 0, st>>>(w, r, rows * w.top_k, dense);
+    const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items)));
+    constexpr int DEPTH = NAL >= 8 ? 2 : 3;
+    if (mma_direct(r.in, dense)) q4k_mma_project_kernel<NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    else q4k_mma_project_kernel<NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
 // rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
 template <int NAL>
 inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const dim3 grid(w.hidden / kMmaRows, dense ? (dense + 2U * NAL - 1U) / (2U * NAL) : items);
+    const uint32_t tiles = w.hidden / kMmaRows;
+    const bool direct = mma_direct(r.h, dense);
     if constexpr (NAL <= 8) {
-        if (static_cast<uint64_t>(grid.x) * grid.y <= compute_units()) {
-            q4k_mma_down_kernel<NAL, 2, 4><<<grid, 1024, 0, st>>>(w, r, rows * w.top_k, dense);
+        const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, 1U);
+        if (static_cast<uint64_t>(g.grid.x) * g.grid.y <= compute_units()) {
+            if (direct) q4k_mma_down_kernel<NAL, 2, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            else q4k_mma_down_kernel<NAL, 2, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
             return;
         }
     }
-    q4k_mma_down_kernel<NAL, (NAL >= 8 ? 2 : 3), 1><<<grid, 256, 0, st>>>(w, r, rows * w.top_k, dense);
+    const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, mma_run_tiles(w.ffn / 256U, NAL >= 8 ? 6U : 12U, static_cast<uint64_t>(tiles) * (dense ? 1U : items)));
+    constexpr int DEPTH = NAL >= 8 ? 2 : 3;
+    if (direct) q4k_mma_down_kernel<NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    else q4k_mma_down_kernel<NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // width: the most rows an item (or the dense batch) holds
 void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
@@ -37,9 +62,16 @@ void launch_mma_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, 
     else launch_mma_down_nal<8>(w, r, rows, dense, items, st);
 }
 void launch_mma_gate_up_rows(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, hipStream_t st) {
-    const dim3 grid(w.ffn / kMmaRows, 1, 2);
-    if (rows <= 8U) q4k_mma_down_kernel<4, 3, 1, true><<<grid, 256, 0, st>>>(w, r, rows, rows);
-    else q4k_mma_down_kernel<8, 2, 1, true><<<grid, 256, 0, st>>>(w, r, rows, rows);
+    const uint32_t tiles = w.ffn / kMmaRows;
+    const MmaLaunch l{rows * w.top_k, rows, tiles, 1U};
+    const dim3 grid(tiles, 1, 2);
+    const auto launch = [&](auto direct) {
+        constexpr bool D = decltype(direct)::value;
+        if (rows <= 8U) q4k_mma_down_kernel<4, 3, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
+        else q4k_mma_down_kernel<8, 2, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
+    };
+    if (mma_direct(r.in, rows)) launch(std::true_type{});
+    else launch(std::false_type{});
 }
 
 }  // namespace strix950

@@ -25,24 +25,36 @@
 // (8 deltas, 8 sums). Everything arrives by global_load_lds_dwordx4 into a ring of DEPTH slots shared by the workgroup: a
 // wavefront waits for its own copies (counted s_waitcnt vmcnt), the workgroup barrier publishes all of them, and the slot
 // consumed before the barrier is refilled after it.
+//
+// A workgroup runs over consecutive 32-row tiles against the same activation rows, and the ring does not stop between them: the
+// copies of the next tile's first stages are in flight while a tile's last stages are multiplied and its values leave. Rows of few
+// super-blocks would otherwise pay the start of a ring (the chain from the work item to the first arrival) every few stages.
 #pragma once
 #include "q4k_pairs.hpp"
+
+#include <type_traits>
 
 namespace strix950 {
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) float lds_f32;
+typedef __attribute__((address_space(3))) uint64_t lds_u64;
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 constexpr uint32_t kMmaRows = 32;
 template <int NAL> constexpr uint32_t mma_acts() { return 2U * NAL; }                         // activation slots served (multiple of 4)
 template <int NAL> constexpr uint32_t mma_code_copies() { return mma_acts<NAL>() / 4U; }      // 1 KiB = 4 rows x 256 codes
 template <int NAL> constexpr uint32_t mma_table_copies() { return (mma_acts<NAL>() + 15U) / 16U; }   // 1 KiB = 16 rows x (8 deltas, 8 sums)
-// NM matrices share the activation rows of a sweep (gate and up): 4.5 (5) KiB of weight pieces each
+// NM matrices share the activation rows of a sweep (gate and up): 4.5 KiB of weight pieces each (five copies, the last of half a wave)
 template <int NAL, int NM> constexpr uint32_t mma_copies() { return 5U * NM + mma_code_copies<NAL>() + mma_table_copies<NAL>(); }
-template <int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return 1024U * mma_copies<NAL, NM>(); }
+constexpr uint32_t kMmaWeightBytes = 144U * kMmaRows;
+template <int NAL, int NM> constexpr uint32_t mma_codes_at() { return kMmaWeightBytes * NM; }
+template <int NAL, int NM> constexpr uint32_t mma_table_at() { return mma_codes_at<NAL, NM>() + 256U * mma_acts<NAL>(); }
+template <int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<NAL, NM>() + 64U * mma_acts<NAL>(); }
 template <int NAL, int NM, int DEPTH, int TEAMS> constexpr uint32_t mma_ring_bytes() { return DEPTH * TEAMS * mma_slot_bytes<NAL, NM>(); }
 template <int NAL, int TEAMS> constexpr uint32_t mma_exchange_floats() { return TEAMS > 1 ? 2U * (TEAMS - 1U) * 4U * NAL * 64U : 1U; }
+template <int NAL, int NM> constexpr uint32_t mma_reduce_floats() { return 4U * NM * NAL * 64U; }
 
 // Workgroup barrier that orders LDS traffic only (__syncthreads() would also wait for every copy in flight, i.e. drain the
 // ring at each stage): this wavefront's LDS reads and writes complete, then the barrier; arrivals of copies are awaited by count.
@@ -53,6 +65,22 @@ __device__ __forceinline__ void mma_barrier() { asm volatile("s_waitcnt lgkmcnt(
 __device__ __forceinline__ void mma_copy16(const uint8_t* src, lds_u8* lds_at) {
     const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_at)));
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(at), "v"(src) : "memory", "m0");
+}
+__device__ __forceinline__ uint64_t mma_scalar(uint64_t v) {
+    return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32)))) << 32 |
+           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)));
+}
+// the same for the lanes of `lanes` only (every lane of the wavefront is active around it)
+__device__ __forceinline__ void mma_copy16_lanes(const uint8_t* src, lds_u8* lds_at, uint64_t lanes) {
+    const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_at)));
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1"
+                 : : "s"(at), "v"(src), "s"(mma_scalar(lanes)) : "memory", "m0");
+}
+// four bytes per lane of `lanes` (lane l lands at lds_at + 4 l)
+__device__ __forceinline__ void mma_copy4_lanes(const uint32_t* src, lds_u32* lds_at, uint64_t lanes) {
+    const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_at)));
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1"
+                 : : "s"(at), "v"(src), "s"(mma_scalar(lanes)) : "memory", "m0");
 }
 template <int N> __device__ __forceinline__ void mma_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 template <int N> __device__ __forceinline__ void mma_wait_n(uint32_t ahead) {   // at most N * ahead copies still in flight
@@ -72,10 +100,11 @@ template <int NAL> __device__ __forceinline__ uint32_t mma_slot_act(uint32_t i) 
     return (2U * v + h) % mma_acts<NAL>();
 }
 
-// Per-lane byte offsets into a ring slot (constant over the sweep); matrix m's weights sit 5120 m further on.
+// Per-lane byte offsets into a ring slot (constant over the sweep); matrix m's weights sit 4608 m further on.
 struct MmaLane {
     uint32_t head, quants, even, odd, table;
     bool sum_lane;
+    uint32_t shift, even_slot;         // halves form: of the lane's sub-block in the header words; all ones where the lane's slot is of half 0
 };
 
 // One landed super-block: for each matrix the wavefront's two group dots of its 32 rows against every activation slot, then the
@@ -89,8 +118,8 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
     u32x4 hd[NM], q[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        hd[m] = *(lds_u32x4*)(slot + 5120U * m + o.head);
-        q[m] = *(lds_u32x4*)(slot + 5120U * m + o.quants);
+        hd[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.head);
+        q[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.quants);
     }
     int32_t tab[NAL];
 #pragma unroll
@@ -128,86 +157,207 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
     }
 }
 
-// The sweep of one 32-row tile (NM matrices' tiles that share the activation rows) over `stages` super-blocks against nacts <=
-// 2 NAL activation rows: on return team 0's wavefront p holds in acc[m][v] pair accumulator p of (row j, activation row 2v + h).
-// acts(a) names activation row a < nacts: .codes / .deltas / .sums point at its A8 image (K codes, K / 32 deltas and sums).
+// The same for few activation rows (NAL == 2), where the scales, the nibbles and the layout's own moves outweigh the chain: each half of
+// the wavefront takes ONE of the pair's sub-blocks, for every activation row. Slot i serves activation row v = 4 (i / 8) + i % 4 in half
+// (i / 4) % 2, and its codes are of sub-block 2p in the slots of half 0, of 2p + 1 in those of half 1; two products - each with the other
+// half's slots zeroed - accumulate into one result, whose register v holds activation row v's dot with sub-block 2p in the lanes of half 0
+// and with sub-block 2p + 1 in those of half 1. A lane then decodes one scale and one minimum instead of two, and the terms of two
+// activation rows meet through one exchange of the halves: x[2p] + x[2p + 1] of row 2v + h lands where the wide form leaves it.
+// (4 activation rows, gate and up: 140 -> 115 vector instructions a stage; dense 27648 x 5120, 4 rows 76.1 -> 75.0 us, Q8_0 down, 120 rows in
+// items of four 237 -> 234 us. With 8 activation rows, as many conversions and two products in a row, it is the slower one: 100 rows of
+// hidden 2048 / ffn 768 / 128 experts 162.0 against 160.2 us, 90 rows of hidden 4096 / ffn 1536 / 64 experts 326 against 321.)
+template <int NAL, int NM, bool HIGH>
+__device__ __forceinline__ void mma_stage_terms_halves(const lds_u8* slot, const MmaLane& o, float (&term)[NM][NAL]) {
+    typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+    typedef const __attribute__((address_space(3))) int32_t lds_i32;
+    const u32x4 codes = *(lds_u32x4*)(slot + o.even);
+    u32x4 hd[NM], q[NM];
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        hd[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.head);
+        q[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.quants);
+    }
+    float e[2 * NAL], f[2 * NAL];
+#pragma unroll
+    for (int a = 0; a < 2 * NAL; ++a) {
+        e[a] = *(const lds_f32*)(slot + o.table + 64U * a);
+        f[a] = static_cast<float>(*(lds_i32*)(slot + o.table + 64U * a + 32U));
+    }
+    const u32x4 a_even = codes & o.even_slot, a_odd = codes & ~o.even_slot;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) {
+        const u32x4 lo = q[m] & 0x0f0f0f0fU, hi = (q[m] >> 4) & 0x0f0f0f0fU;
+        const i32x16 zero = {0};
+        i32x16 dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_even), __builtin_bit_cast(i32x4, lo), zero, 0, 0, 0);
+        dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_odd), __builtin_bit_cast(i32x4, hi), dot, 0, 0, 0);
+        uint32_t sc, mn;                                       // (q4k_factors with the shift of the lane's sub-block)
+        if (!HIGH) {
+            sc = __builtin_amdgcn_ubfe(hd[m].y, o.shift, 6U);
+            mn = __builtin_amdgcn_ubfe(hd[m].z, o.shift, 6U);
+        } else {
+            sc = __builtin_amdgcn_ubfe(hd[m].w, o.shift, 4U) | (__builtin_amdgcn_ubfe(hd[m].y, o.shift + 6U, 2U) << 4);
+            mn = __builtin_amdgcn_ubfe(hd[m].w, o.shift + 4U, 4U) | (__builtin_amdgcn_ubfe(hd[m].z, o.shift + 6U, 2U) << 4);
+        }
+        const float D = half_bits_to_float(hd[m].x & 0xffffU) * static_cast<float>(sc), M = half_bits_to_float(hd[m].x >> 16) * static_cast<float>(mn);
+#pragma unroll
+        for (int v = 0; v < NAL; ++v) {
+            const float u0 = D * static_cast<float>(dot[2 * v]), v0 = M * f[2 * v], x0 = e[2 * v] * (u0 - v0);
+            const float u1 = D * static_cast<float>(dot[2 * v + 1]), v1 = M * f[2 * v + 1], x1 = e[2 * v + 1] * (u1 - v1);
+            const auto met = __builtin_amdgcn_permlane32_swap(b_of(x0), b_of(x1), false, false);      // (half 0's rows 2v, half 1's rows 2v + 1)
+            term[m][v] = f_of(met[0]) + f_of(met[1]);
+        }
+    }
+}
+template <int NAL> constexpr bool mma_halves() { return NAL == 2; }
+
+// The activation rows of a run and where their results go, resolved once by one wavefront: addresses of the A8 image of row a (codes,
+// deltas, sums), OUT more addresses for the emitter, and the row's assignment.
+template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OUT) * mma_acts<NAL>(); }
+
+// A run of `tiles` 32-row tiles, back to back in memory (NM matrices' tiles share the activation rows), of `stages` super-blocks against
+// nacts <= 2 NAL activation rows. Wavefront p keeps pair accumulator p of (row j, activation row 2v + h) in acc[m][v]; at the end of a tile
+// value = (acc0 + acc1) + (acc2 + acc3) over the four wavefronts, through `red`: wavefront w receives the values of result registers
+// v = w, w + 4, ... and hands (tile, v, its lane, values of the NM matrices) to emit.
+//   rows.word(a): address of a word that names activation row a (its place in the plan's order); rows.put(a, nacts, word): leaves the row's
+//   addresses in rows.at. Wavefront 3 asks for the words first, then every wavefront starts the weights of the first stages, so the
+//   look-up is in flight beside them. Rows::kDirect: the addresses need no look-up (rows.codes / rows.table), every wavefront works its
+//   own out and the row table serves the emitter only.
 //
-// TEAMS > 1 (a matrix of few, long rows gives few workgroups, each with K / 256 dependent stages): TEAMS x 4 wavefronts; team
-// t takes super-blocks t, TEAMS + t, ... of the same 32 rows, so TEAMS stages are in the pipes at once. The chain order is
+// TEAMS > 1 (a matrix of few, long rows gives few workgroups, each with K / 256 dependent stages; one tile a run): TEAMS x 4 wavefronts;
+// team t takes super-blocks t, TEAMS + t, ... of the same 32 rows, so TEAMS stages are in the pipes at once. The chain order is
 // kept by team 0, which adds the terms of every super-block in ascending order: its own from registers, the other teams'
 // from an LDS exchange buffer, one stage group behind (the group's barrier publishes them).
-// Every wavefront of the workgroup calls this; the ring is free again when it returns.
-struct MmaActRow { const uint8_t *codes, *deltas, *sums; };
-template <int NAL, int DEPTH, int TEAMS, int NM, class Acts>
-__device__ __forceinline__ void mma_sweep(lds_u8* ring, lds_f32* xbuf, const uint8_t* const (&wrows)[NM], size_t row_stride, uint32_t stages,
-                                          Acts acts, uint32_t nacts, float (&acc)[NM][NAL]) {
+// Every wavefront of the workgroup calls this; ring, row table and `red` are free again when it returns.
+template <int NAL, int DEPTH, int TEAMS, int NM, class Rows, class Emit>
+__device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* red, const uint8_t* const (&wrows)[NM], size_t row_stride, uint32_t stages,
+                                        uint32_t tiles, uint32_t nacts, Rows rows, Emit emit) {
     constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<NAL, NM>(), SLOT = mma_slot_bytes<NAL, NM>();
-    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, FULL = TOTAL % 4U == 0 ? 4U : TOTAL % 4U;     // wavefronts 0 .. FULL - 1 of a team issue PERW copies
+    // Every wavefront issues PERW copies a stage, some of them for no lane (the rest of the last four; the ones that the first stage starts
+    // early or late): no branches on the wavefront's number, one count to wait for.
+    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = 5U * NM;
     constexpr uint32_t XTEAM = 4U * NAL * 64U;                                                  // floats one team exchanges per group
     static_assert(DEPTH >= 2 && DEPTH <= 4, "ring depth");
     static_assert(TEAMS == 1 || (NM == 1 && NAL <= 8), "stage teams serve one matrix, every result register");
     const uint32_t lane = threadIdx.x & 63U, j = lane & 31U, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = wave & 3U, team = wave >> 2;
-    const uint32_t groups = (stages + TEAMS - 1U) / TEAMS;
+    const uint32_t groups = (stages + TEAMS - 1U) / TEAMS;                                     // of a tile
     const uint32_t my_groups = team < stages - (groups - 1U) * TEAMS ? groups : groups - 1U;   // groups in which this team has a super-block
+    const uint32_t total = TEAMS == 1 ? groups * tiles : groups, my_total = TEAMS == 1 ? total : my_groups;
     const uint32_t nv = (nacts + 1U) / 2U;
 
-    // ---- this wavefront's copies of a stage: copy c = 4k + p lands at slot + 1024 c
+    // ---- this wavefront's copies of a stage, copy c = 4k + p: five per matrix (9 pieces of 16 bytes a row, rows back to back; the
+    // fifth moves the last half kilobyte), codes (16 pieces per row, piece t at position (t + a) % 16), table (per row [8 deltas][8 sums])
     const uint8_t* src[PERW];
-    uint32_t step[PERW];
+    uint32_t step[PERW], lands[PERW];
+    uint64_t lanes[PERW];
 #pragma unroll
     for (uint32_t k = 0; k < PERW; ++k) {
         const uint32_t c = 4U * k + p;
-        if (c < 5U * NM) {                                      // weight pieces: 9 per row, rows back to back
-            const uint32_t m = c / 5U;
-            uint32_t s = 64U * (c - 5U * m) + lane;
-            s = s < kMmaRows * 9U ? s : kMmaRows * 9U - 1U;     // the short fifth copy repeats the last piece into unused LDS
-            const uint32_t r = s / 9U, piece = s - 9U * r;
-            src[k] = wrows[m < NM ? m : 0] + static_cast<size_t>(r) * row_stride + 16U * piece;
-            step[k] = 144U;
-        } else if (c < 5U * NM + CC) {                          // codes: 16 pieces per row, piece t at position (t + a) % 16
-            const uint32_t s = 64U * (c - 5U * NM) + lane, a = s >> 4, t = ((s & 15U) - a) & 15U;
-            src[k] = acts(a < nacts ? a : 0U).codes + 16U * t;
-            step[k] = 256U;
-        } else {                                                // table: per row [8 deltas][8 sums], four pieces
-            const uint32_t a = 16U * (c - 5U * NM - CC) + (lane >> 2), q = lane & 3U;
-            const MmaActRow row = acts(a < ACTS && a < nacts ? a : 0U);
-            src[k] = q < 2U ? row.deltas + 16U * q : row.sums + 16U * (q - 2U);
-            step[k] = 32U;
+        if (c < WEIGHTS) {
+            const uint32_t m = c / 5U, i = c - 5U * m, s = 64U * i + lane < kMmaRows * 9U ? 64U * i + lane : 0U, r = s / 9U, piece = s - 9U * r;
+            src[k] = wrows[m < NM ? m : 0] + static_cast<size_t>(r) * row_stride + 16U * piece + 144U * team;
+            step[k] = 144U * TEAMS;
+            lands[k] = kMmaWeightBytes * m + 1024U * i;
+            lanes[k] = i == 4U ? 0xffffffffULL : ~0ULL;
+        } else if (c < WEIGHTS + CC) {
+            src[k] = nullptr;
+            step[k] = 256U * TEAMS;
+            lands[k] = mma_codes_at<NAL, NM>() + 1024U * (c - WEIGHTS);
+            lanes[k] = ~0ULL;
+        } else {
+            src[k] = nullptr;
+            step[k] = 32U * TEAMS;
+            lands[k] = mma_table_at<NAL, NM>() + 1024U * (c - WEIGHTS - CC);
+            lanes[k] = c >= TOTAL ? 0ULL : ACTS >= 16U ? ~0ULL : (1ULL << (4U * ACTS)) - 1ULL;
         }
-        src[k] += static_cast<size_t>(step[k]) * team;
-        step[k] *= TEAMS;
     }
-    const auto start = [&](lds_u8* slot) {
+    const size_t next_tile = kMmaRows * row_stride - 144U * static_cast<size_t>(stages);       // from a tile's end to the next one's start
+    uint32_t issued = 0, issue_stage = 0;
+    // copies of the next stage into a slot; PART 1: the weights (of the run's first stages, whose activation rows are not known yet), 2: the rest
+    const auto start = [&](auto part_constant, lds_u8* slot) __attribute__((always_inline)) {
+        constexpr int part = decltype(part_constant)::value;
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
-            const uint32_t c = 4U * k + p;
-            if (c < TOTAL) {
-                mma_copy16(src[k], slot + 1024U * c);
-                src[k] += step[k];
+            const bool mine = part == 0 || (4U * k + p < WEIGHTS) == (part == 1);
+            if (part == 0 && k == 0U) mma_copy16(src[k], slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
+            else mma_copy16_lanes(src[k], slot + lands[k], mine ? lanes[k] : 0ULL);
+            src[k] += mine ? step[k] : 0U;
+        }
+        if (TEAMS == 1 && ++issue_stage == stages) {
+            issue_stage = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < PERW; ++k) {
+                const bool weights = 4U * k + p < WEIGHTS;
+                if (part == 0 || weights == (part == 1)) src[k] += weights ? next_tile : 0U - static_cast<size_t>(step[k]) * stages;
             }
         }
     };
+    const auto slot_of = [&](uint32_t s) { return ring + SLOT * (s * TEAMS + team); };
+    const uint32_t first = my_total < DEPTH - 1U ? my_total : DEPTH - 1U;
+    const auto start_weights = [&]() {
+        for (uint32_t s = 0; s < first; ++s) start(std::integral_constant<int, 1>{}, slot_of(s));
+    };
+    const auto row_of_codes = [&](uint32_t k) { return (64U * (4U * k + p - WEIGHTS) + lane) >> 4; };                            // of the lane's 16 bytes
+    const auto row_of_table = [&](uint32_t k) { return (16U * (4U * k + p - WEIGHTS - CC) + (lane >> 2)) & (ACTS - 1U); };
+    const auto set_rows = [&](auto codes_of, auto table_of) {
+#pragma unroll
+        for (uint32_t k = 0; k < PERW; ++k) {
+            const uint32_t c = 4U * k + p;
+            if (c >= WEIGHTS && c < WEIGHTS + CC) {
+                const uint32_t a = row_of_codes(k);
+                src[k] = codes_of(a) + 16U * (((lane & 15U) - a) & 15U) + 256U * team;
+            } else if (c >= WEIGHTS + CC && c < TOTAL) {
+                const uint32_t q = lane & 3U;
+                src[k] = table_of(row_of_table(k), q < 2U) + 16U * (q & 1U) + 32U * team;
+            }
+        }
+    };
+    if constexpr (Rows::kDirect) {
+        start_weights();
+        set_rows([&](uint32_t a) { return rows.codes(a < nacts ? a : 0U); }, [&](uint32_t a, bool deltas) { return rows.table(a < nacts ? a : 0U, deltas); });
+    } else {
+        if (wave == 3U) {
+            // (the words land in LDS like everything else: a register that a load in flight writes could be copied before it does)
+            mma_copy4_lanes(rows.word(lane < nacts ? lane : 0U), rows.slot, (1ULL << ACTS) - 1ULL);
+            start_weights();
+            if (DEPTH > 2 && first == DEPTH - 1U) mma_wait<PERW * (DEPTH - 1)>();
+            else mma_wait<PERW>();
+            if (lane < ACTS) rows.put(lane, nacts, rows.slot[lane]);
+        } else start_weights();
+        mma_barrier();
+        set_rows([&](uint32_t a) { return reinterpret_cast<const uint8_t*>(rows.at[a]); },
+                 [&](uint32_t a, bool deltas) { return reinterpret_cast<const uint8_t*>(rows.at[(deltas ? ACTS : 2U * ACTS) + a]); });
+    }
 
     MmaLane o;
     {
-        const uint32_t ai = mma_slot_act<NAL>(j), c_base = 5120U * NM + 256U * ai;
+        const uint32_t ai = mma_slot_act<NAL>(j), c_base = mma_codes_at<NAL, NM>() + 256U * ai;
         o.head = 144U * j;
         o.quants = 144U * j + 16U + 32U * p + 16U * h;
         o.even = c_base + 16U * ((4U * p + h + ai) & 15U);
         o.odd = c_base + 16U * ((4U * p + 2U + h + ai) & 15U);
         // quad lane 0, 1: delta of sub-block 2p, 2p + 1; quad lane 2, 3: their code sums
-        o.table = 5120U * NM + 1024U * CC + 64U * h + 4U * (2U * p + (lane & 1U) + 4U * (lane & 2U));
+        o.table = mma_table_at<NAL, NM>() + 64U * h + 4U * (2U * p + (lane & 1U) + 4U * (lane & 2U));
         o.sum_lane = (lane & 2U) != 0;
+        if constexpr (mma_halves<NAL>()) {
+            const uint32_t odd = (j >> 2) & 1U, act = (4U * (j >> 3) + (j & 3U)) & (ACTS - 1U);
+            o.even = mma_codes_at<NAL, NM>() + 256U * act + 16U * ((4U * p + 2U * odd + h + act) & 15U);
+            o.table = mma_table_at<NAL, NM>() + 4U * (2U * p + h);
+            o.shift = 16U * (p & 1U) + 8U * h;
+            o.even_slot = odd ? 0U : ~0U;
+        }
     }
 
-    float own[NAL];
+    float acc[NM][NAL], own[NAL];
 #pragma unroll
     for (int v = 0; v < NAL; ++v) own[v] = 0.0F;
+    const auto clear = [&]() {
 #pragma unroll
-    for (int m = 0; m < NM; ++m)
+        for (int m = 0; m < NM; ++m)
 #pragma unroll
-        for (int v = 0; v < NAL; ++v) acc[m][v] = 0.0F;
+            for (int v = 0; v < NAL; ++v) acc[m][v] = 0.0F;
+    };
+    clear();
     // team 0: the terms of group g (its own, then teams 1 .. of the super-blocks that exist), in super-block order
     const auto fold = [&](uint32_t g) {
 #pragma unroll
@@ -221,27 +371,59 @@ __device__ __forceinline__ void mma_sweep(lds_u8* ring, lds_f32* xbuf, const uin
             }
         }
     };
+    const auto leave = [&]() {
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+            for (int v = 0; v < NAL; ++v) red[((m * 4U + p) * NAL + v) * 64U + lane] = acc[m][v];
+    };
+    const auto emit_tile = [&](uint32_t tile) {
+        uint32_t lane = threadIdx.x & 63U;
+        asm volatile("" : "+v"(lane));         // (what follows from it is worked out here, once a tile, not held in registers over the sweep)
+        for (uint32_t v = p; v < nv; v += 4U) {
+            float value[NM];
+#pragma unroll
+            for (uint32_t m = 0; m < NM; ++m) {
+                const lds_f32* x = red + (m * 4U * NAL + v) * 64U + lane;
+                const float left = x[0] + x[NAL * 64U], right = x[2U * NAL * 64U] + x[3U * NAL * 64U];
+                value[m] = left + right;
+            }
+            emit(tile, v, lane, value);
+        }
+    };
 
     // ---- the ring of stage groups
-    uint32_t issued = 0, issue_slot = 0, compute_slot = 0;
+    issue_stage = 0;
+    for (; issued < first; ++issued) start(std::integral_constant<int, 2>{}, slot_of(issued));
+    if (Rows::kDirect && wave == 3U && lane < ACTS) rows.put(lane, nacts, 0U);       // (first read behind the first stage's barrier)
+    uint32_t issue_slot = DEPTH - 1U, compute_slot = 0, stage = 0, tile = 0;
     const auto issue = [&]() {
-        if (issued < my_groups) { start(ring + SLOT * (issue_slot * TEAMS + team)); ++issued; }
+        if (issued < my_total) { start(std::integral_constant<int, 0>{}, slot_of(issue_slot)); ++issued; }
         issue_slot = issue_slot + 1U == DEPTH ? 0U : issue_slot + 1U;
     };
-    for (uint32_t s = 0; s + 1U < DEPTH; ++s) issue();
-    for (uint32_t g = 0; g < groups; ++g) {
-        if (g < my_groups) {
+    for (uint32_t g = 0; g < total; ++g) {
+        if (g < my_total) {
             const uint32_t ahead = issued - 1U - g;              // this wavefront's stages started after its stage of group g
-            if (p < FULL) mma_wait_n<PERW>(ahead);
-            else mma_wait_n<PERW - 1U>(ahead);
+            mma_wait_n<PERW>(ahead);
         }
         mma_barrier();         // every copy of group g is in, the slots of group g - 1 are free, its exchanged terms are written
-        issue();
+        // The values of the tile before leave in its successor's first stage. They are stores, which the counted waits count too: before
+        // the stage's copies they delay those a little, behind them the next wait would wait for copies that it does not need -
+        // except in a ring of two slots, whose every wait is for everything.
+        if (DEPTH == 2) issue();
+        if (TEAMS == 1 && stage == 0U && g != 0U) {
+            emit_tile(tile - 1U);
+            if (stages == 1U) mma_barrier();                     // (the next values are written in this stage)
+        }
+        if (DEPTH != 2) issue();
         if (TEAMS > 1 && team == 0U && g > 0U) fold(g - 1U);
-        if (g < my_groups) {
+        if (g < my_total) {
             const lds_u8* slot = ring + SLOT * (compute_slot * TEAMS + team);
             float term[NM][NAL];
-            switch (p) {
+            if constexpr (mma_halves<NAL>()) {
+                if (p < 2U) mma_stage_terms_halves<NAL, NM, false>(slot, o, term);
+                else mma_stage_terms_halves<NAL, NM, true>(slot, o, term);
+            } else switch (p) {
             case 0: mma_stage_terms<NAL, NM, 0>(slot, o, nv, term); break;
             case 1: mma_stage_terms<NAL, NM, 1>(slot, o, nv, term); break;
             case 2: mma_stage_terms<NAL, NM, 2>(slot, o, nv, term); break;
@@ -265,42 +447,20 @@ __device__ __forceinline__ void mma_sweep(lds_u8* ring, lds_f32* xbuf, const uin
             }
         }
         compute_slot = compute_slot + 1U == DEPTH ? 0U : compute_slot + 1U;
-    }
-    __syncthreads();           // no copy in flight (the last wait was for all), every LDS read of the ring is done
-    if (TEAMS > 1 && team == 0U) fold(groups - 1U);
-}
-
-// value = (acc0 + acc1) + (acc2 + acc3) over team 0's four wavefronts, through `red` (4 NM NAL 64 floats, may be the ring):
-// wavefront w of team 0 receives the values of result registers v = w, w + 4, ... and hands (v, values of the NM matrices) to
-// emit. Every wavefront of the workgroup calls this; `red` is free again when it returns.
-template <int NAL, int NM, class Emit>
-__device__ __forceinline__ void mma_reduce(lds_f32* red, const float (&acc)[NM][NAL], uint32_t nacts, Emit emit) {
-    const uint32_t lane = threadIdx.x & 63U;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = wave & 3U, team = wave >> 2;
-    const uint32_t nv = (nacts + 1U) / 2U;
-    if (team == 0U) {
-#pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int v = 0; v < NAL; ++v) red[((m * 4U + p) * NAL + v) * 64U + lane] = acc[m][v];
-    }
-    __syncthreads();
-    if (team == 0U) {
-#pragma unroll
-        for (uint32_t v = 0; v < NAL; ++v) {
-            if ((v & 3U) != p || v >= nv) continue;
-            float value[NM];
-#pragma unroll
-            for (int m = 0; m < NM; ++m) {
-                const float r0 = red[((m * 4U + 0U) * NAL + v) * 64U + lane], r1 = red[((m * 4U + 1U) * NAL + v) * 64U + lane];
-                const float r2 = red[((m * 4U + 2U) * NAL + v) * 64U + lane], r3 = red[((m * 4U + 3U) * NAL + v) * 64U + lane];
-                const float left = r0 + r1, right = r2 + r3;
-                value[m] = left + right;
-            }
-            emit(v, value);
+        if (TEAMS == 1 && ++stage == stages) {
+            stage = 0;
+            ++tile;
+            leave();
+            clear();
         }
     }
-    __syncthreads();
+    mma_barrier();             // the last values (TEAMS > 1: the last exchanged terms) are written; no copy is in flight
+    if (TEAMS > 1) {
+        if (team == 0U) { fold(groups - 1U); leave(); }
+        mma_barrier();
+        if (team == 0U) emit_tile(0U);
+    } else emit_tile(tiles - 1U);
+    mma_barrier();             // every LDS read is done
 }
 
 }  // namespace strix950
