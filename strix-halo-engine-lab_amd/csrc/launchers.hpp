@@ -19,6 +19,8 @@ struct RouteCheck {
 };
 void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, const RouteArgs* select, const RouteCheck& c, hipStream_t st);
 
+// prefill.hip: the most rows of a plan item for the products of a batch
+uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments);
 // prefill.hip: sub-block sums of the input rows, gate / up + SwiGLU and down rows of a planned batch. `a` holds everything but the
 // products' own fields (weights, strides, k, features, tiles, units). check: the routes' check and the status words as well.
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at,

@@ -46,27 +46,40 @@ __global__ __launch_bounds__(256) void prefill_prologue_kernel(const uint8_t* x,
     }
 }
 
+namespace {
+// Which Q4_K batches the four-wave form of prefill_reg.hpp serves. It sweeps an expert's weights once per 32 rows, the wide form once per
+// 128; it has three times the workgroups in flight. Measured (wide, four waves), rows per expert on average and rounds of the wide form's
+// gate / up workgroups beside them: 8.5, 5.8 256, 199 us; 12.3, 13 185, 168; 15, 8.4 776, 707; 21, 3.5 195, 178; 22, 14 965, 1028;
+// 25, 9 867, 894; 37, 7.8 879, 961; 40, 3.3 435, 419; 46, 1.8 414, 380; 50, 4.2 270, 275; 56, 4.0 194, 178; 45, 18 1847, 2312.
+bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
+    const uint64_t e = wv.experts, a = assignments;
+    return a <= 16ULL * e || (a <= 56ULL * e && (128ULL * e + a) * wv.ffn <= 4ULL * compute_units() * 128U * 128U);
+}
+bool reg_gate(const mi355_moe_weights& wv) { return wv.gate_type == MI355_TYPE_Q4_K && wv.ffn % 128U == 0; }
+bool reg_down(const mi355_moe_weights& wv) { return wv.down_type == MI355_TYPE_Q4_K && wv.hidden % 256U == 0; }
+}  // namespace
+
+uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments) {
+    return reg_gate(wv) && reg_down(wv) && few_rows(wv, assignments) ? 32U : kPfTile;
+}
+
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at, uint32_t order_at, hipStream_t st) {
     prefill_prologue_kernel<<<rows, 256, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums, a.h_sums, wv.ffn, wv.top_k, check ? *check : RouteCheck{});
     const uint32_t item_slots = (a.items + 7U) / 8U * 8U;
-    // persistent workgroups, as many as are resident: one per compute unit (LDS allows no second one) or `each` of the narrow form
+    // persistent workgroups, as many as are resident: one per compute unit (LDS allows no second one) or `each` of the four-wave form
     const uint32_t cus = compute_units();
     const uint32_t resident = (cus > 8U ? cus : 256U) & ~7U;
     const auto grid_of = [&](uint32_t units, uint32_t each = 1U) { return units < each * resident ? units : each * resident; };
-    // Up to kNarrowRows rows per expert on average the narrow form of prefill_reg.hpp: two workgroups of half the width share a compute
-    // unit, so one's start and end hide behind the other's products. Measured (wide, narrow): hidden 2048, ffn 768, 128 experts top-8, 64
-    // rows 124, 108 us; 150 rows 160, 146 us; 333 rows 198, 191 us; 1200 rows 315, 362 us; hidden 4096, ffn 1536, 64 experts, 64 rows 272,
-    // 246 us; 150 rows 312, 312 us; 333 rows 412, 438 us.
-    constexpr uint64_t kNarrowRows = 24;
-    const bool narrow = a.assignments <= kNarrowRows * wv.experts;
+    const bool few = few_rows(wv, a.assignments);
+    a.subs = prefill_split(wv, a.assignments) / 32U;
     // gate / up + SwiGLU. Q4_K tensors: every wave expands its own rows in registers (prefill_reg.hpp); Q5_K / Q8_0: the loader /
     // multiplier kernel (prefill_f16.hpp). Both leave h as two fp16 planes and its sub-block sums.
     a.wa = wv.gate; a.wb = wv.up; a.expert_stride = wv.gate_expert_stride; a.row_stride = wv.gate_row_stride; a.k = wv.hidden; a.features = wv.ffn;
     a.lo_pass = 0;
-    if (wv.gate_type == MI355_TYPE_Q4_K && wv.ffn % 128U == 0) {
-        a.tiles = wv.ffn / (narrow ? 64U : 128U); a.units = item_slots * a.tiles;
-        if (narrow) prefill_reg_kernel<0, 4, 64><<<grid_of(2U * a.units, 2U), 256, 0, st>>>(a, items_at, order_at);
-        else prefill_reg_kernel<0, 8, 128><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
+    if (reg_gate(wv)) {
+        a.tiles = wv.ffn / (few ? 64U : 128U); a.units = item_slots * a.tiles;
+        if (few) prefill_reg_kernel<0, 4><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
+        else prefill_reg_kernel<0, 8><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
     } else {
         a.tiles = wv.ffn / 64U; a.units = item_slots * a.tiles;
         if (wv.gate_type == MI355_TYPE_Q8_0) prefill_f16_kernel<0, 1><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
@@ -76,10 +89,10 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
     // down rows: h enters as hi + lo. The register-operand kernel multiplies both planes in one sweep of the weights; the loader /
     // multiplier kernel runs a second pass over the lo plane that adds to the first pass's outputs.
     a.wa = wv.down; a.wb = nullptr; a.expert_stride = wv.down_expert_stride; a.row_stride = wv.down_row_stride; a.k = wv.ffn; a.features = wv.hidden;
-    if (wv.down_type == MI355_TYPE_Q4_K && wv.hidden % 256U == 0) {
-        a.tiles = wv.hidden / (narrow ? 128U : 256U); a.units = item_slots * a.tiles;
-        if (narrow) prefill_reg_kernel<1, 4, 64><<<grid_of(2U * a.units, 2U), 256, 0, st>>>(a, items_at, order_at);
-        else prefill_reg_kernel<1, 8, 128><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
+    if (reg_down(wv)) {
+        a.tiles = wv.hidden / (few ? 128U : 256U); a.units = item_slots * a.tiles;
+        if (few) prefill_reg_kernel<1, 4><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
+        else prefill_reg_kernel<1, 8><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
     } else {
         a.tiles = wv.hidden / 128U; a.units = item_slots * a.tiles;
         for (uint32_t pass = 0; pass < 2U; ++pass) {

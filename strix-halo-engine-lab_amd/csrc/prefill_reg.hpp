@@ -16,10 +16,15 @@
 // 128 gate + 128 up rows (MODE 0) or 256 down rows (MODE 1). Wave w owns 32 of the rows x all 128 tokens: accumulators
 // 4 token tiles x 16 registers for the super-block product P and the same for the running sum. K advances in stages of 64
 // (one pair of sub-blocks = 32 quant bytes of a row): a lane (row n, half h) fetches the 16 quant bytes [16 h, 16 h + 16) of
-// the pair straight into registers four stages ahead, expands them into the B operands of the stage's four MFMA k-steps
+// the pair straight into registers, expands them into the B operands of the stage's four MFMA k-steps
 // (low nibbles: k-steps 0, 1; high nibbles: 2, 3), and the token rows of the stage (64 halves each) are copied global -> LDS
-// three stages ahead through a 4-stage ring shared by the eight waves. One barrier per stage.
+// three stages ahead through a 4-stage ring shared by the workgroup's waves. One barrier per stage, in its middle, so that the stream of
+// operand requests and MFMAs runs on over the stages' borders, and the expansions, the folds of a super-block and the requests stand
+// between the MFMAs (333 rows 194.6 -> 191.7 us, 4096 rows over 256 experts 3.66 -> 3.59 ms).
 // MODE 0 pairs gate row f with up row f in lanes n and n + 16 of one wave, so SwiGLU needs one 16-lane exchange.
+// What bounds it: with whole tiles of 128 rows a SIMD takes 38 ns a product (one such product after the other on random operands, out of
+// registers, takes it 20 ns at the clock that the chip's power leaves, with seven vector instructions beside each 26); with few rows
+// the weights' way to the registers.
 #pragma once
 #include "prefill_f16.hpp"
 
@@ -31,7 +36,10 @@ template <int MODE, uint32_t WAVES> __host__ __device__ constexpr uint32_t rg_to
 }
 // Number of vector-memory operations a wave issues in stage p (= stage % 4) of every super-block: the nt token copies of the
 // stage three ahead, one quant fetch, and the header fetch (p = 0) or the sums copy (p = 1).
-__host__ __device__ constexpr uint32_t rg_stage_ops(uint32_t nt, uint32_t p) { return nt + 1U + (p < 2U ? 1U : 0U); }
+// whole: the quants of the next super-block all at once with its header (p = 0).
+__host__ __device__ constexpr uint32_t rg_stage_ops(uint32_t nt, uint32_t p, bool whole) {
+    return whole ? nt + (p == 0U ? 5U : p == 1U ? 1U : 0U) : nt + 1U + (p < 2U ? 1U : 0U);
+}
 
 // copy16_to_lds with the LDS address (lane 0's destination) already a scalar
 __device__ __forceinline__ void copy16_to_lds_at(const uint8_t* src, uint32_t lds_at) {
@@ -40,12 +48,18 @@ __device__ __forceinline__ void copy16_to_lds_at(const uint8_t* src, uint32_t ld
 
 template <int N> __device__ __forceinline__ void rg_wait() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-// WAVES, TOKENS: 8 waves over 128 tokens (one workgroup per compute unit) or 4 waves over 64 (three or two of them).
-template <int MODE, uint32_t WAVES, uint32_t TOKENS>
-__global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs a, uint32_t items_at, uint32_t order_at) {
-    static_assert(TOKENS == 16U * WAVES, "one sums copy per wave, a token copy of 8 rows per wave and part");
+// WAVES: 8 (one workgroup per compute unit, items of up to 128 rows) or 4 (three workgroups, 32 rows at a time: batches whose experts hold
+// few rows are bound by how many weight bytes are asked for at once, and 160 registers let a third workgroup ask).
+// WHOLE: the four-wave form asks for a super-block's header and quants in one go, a super-block ahead: the 144 bytes of a row are two
+// cache lines, which the wide form's four fetches, a stage apart, bring from the L2 four times (its registers leave no room for the copy;
+// 300 rows of hidden 5120 / ffn 1536 / 160 experts 763 -> 700 us).
+template <int MODE, uint32_t WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_kernel(PrefillArgs a, uint32_t items_at, uint32_t order_at) {
+    constexpr uint32_t TOKENS = WAVES == 4U ? 32U : 128U;
+    static_assert(TOKENS <= 16U * WAVES && TOKENS % (8U * WAVES) == 0, "one sums copy per wave, a token copy of 8 rows per wave and part");
+        constexpr bool WHOLE = WAVES == 4U;
     constexpr uint32_t PLANES = MODE == 1 ? 2U : 1U, TILES = TOKENS / 32U, PART_ROWS = 8U * WAVES;
-    constexpr uint32_t SUBS = kPfTile / TOKENS, STAGE = TOKENS * 128U;                     // one plane of one stage: TOKENS rows x 64 halves
+    constexpr uint32_t STAGE = TOKENS * 128U;                     // one plane of one stage: TOKENS rows x 64 halves
     __shared__ __attribute__((aligned(16))) uint8_t tok0[PLANES * STAGE];
     __shared__ __attribute__((aligned(16))) uint8_t tok1[PLANES * STAGE];
     __shared__ __attribute__((aligned(16))) uint8_t tok2[PLANES * STAGE];
@@ -63,13 +77,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
     const uint32_t last_group = (blocks + 1U) / 2U - 1U;
     const size_t sum_row = pf_sum_row_bytes(a.k);
 
-    // Wide: the tiles of an item run on one XCD, whose L2 then holds its token rows. Narrow: few rows per item, whose units differ in
-    // length more than their token rows cost: an item's tiles go round the XCDs (of the items that were made), and an item of more rows
-    // than TOKENS is as many units, the first of every item first.
-    const uint32_t units = SUBS == 1U ? a.units : a.plan[4] * a.tiles;
-    for (uint32_t at = blockIdx.x; at < SUBS * units; at += gridDim.x) {
-    const uint32_t sub = SUBS == 1U ? 0U : at / units, unit = at - sub * units, q = unit >> 3;
-    const uint32_t item_index = SUBS == 1U ? (q / a.tiles) * 8U + (unit & 7U) : unit / a.tiles, tile = (SUBS == 1U ? q : unit) % a.tiles;
+    // Wide: the tiles of an item run on one XCD, whose L2 then holds its token rows. Four waves: few rows per item, whose units differ in
+    // length more than their token rows cost: an item's tiles go round the XCDs (of the items that were made), and where the plan's
+    // items hold more rows than TOKENS (a.subs times as many) the first rows of every item come first.
+    constexpr bool ROUND = WAVES == 4U;
+    const uint32_t units = ROUND ? a.plan[4] * a.tiles : a.units, subs = ROUND ? a.subs : 1U;
+    for (uint32_t at = blockIdx.x; at < subs * units; at += gridDim.x) {
+    const uint32_t sub = ROUND ? at / units : 0U, unit = at - sub * units, q = unit >> 3;
+    const uint32_t item_index = ROUND ? unit / a.tiles : (q / a.tiles) * 8U + (unit & 7U), tile = (ROUND ? unit : q) % a.tiles;
     if (item_index >= a.items) continue;
     const uint4 item = *reinterpret_cast<const uint4*>(a.plan + items_at + 4U * item_index);
     const uint32_t e = item.x, begin = item.y + sub * TOKENS;
@@ -101,7 +116,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
     // ---- sums copy: piece = (token, part): parts 0, 1 = hi halves 0-7 / 8-15, parts 2, 3 = lo
     const uint8_t* ssrc;
     {
-        const uint32_t row = threadIdx.x >> 2, part = threadIdx.x & 3U, tok = row < count ? row : count - 1U;
+        const uint32_t row = (threadIdx.x >> 2) & (TOKENS - 1U), part = threadIdx.x & 3U, tok = row < count ? row : count - 1U;
         const uint8_t* base = MODE == 0 ? a.x_sums + static_cast<size_t>(order[begin + tok] / a.top_k) * sum_row
                                         : a.h_sums + static_cast<size_t>(begin + tok) * sum_row;
         ssrc = base + 16U * (part & 1U) + (part >> 1) * (sum_row / 2U);
@@ -109,7 +124,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
     const auto copy_sums = [&](uint32_t g) {
         const uint32_t gc = g < last_group ? g : last_group;
         copy16_to_lds_at(ssrc + static_cast<size_t>(gc) * 32U,
-                         static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_tile)) + (g & 1U) * (TOKENS * 64U) + 1024U * wave_s);
+                         static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_tile)) + (g & 1U) * (TOKENS * 64U) + 1024U * (wave_s & (TOKENS / 16U - 1U)));
     };
     const auto fetch_header = [&](uint32_t b, u32x4& hd) {
         const uint8_t* blk = wrow + static_cast<size_t>(b < last_block ? b : last_block) * 144U;
@@ -130,6 +145,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
         const uint32_t r2 = __builtin_amdgcn_perm(0U, w1, 0x0c010c00U), r3 = __builtin_amdgcn_perm(0U, w1, 0x0c030c02U);
         const u32x4 v = {r0 * sc + magic, r1 * sc + magic, r2 * sc + magic, r3 * sc + magic};
         return __builtin_bit_cast(half8, v);
+    };
+    // one of the four: bytes 0, 1 or (odd) 2, 3 of a word
+    const auto expand_pair = [&](uint32_t w, uint32_t odd, uint32_t sc) -> uint32_t {
+        return __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U) * sc + magic;
     };
     // sc of sub-blocks 2 p and 2 p + 1 (src/cpu/core/routed_expert.cpp:65-71)
     const auto scales = [&](const u32x4& hd, uint32_t p, uint32_t& s_lo, uint32_t& s_hi) {
@@ -166,14 +185,25 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
 
     // ---- prologue: the operations of "stages -3, -2, -1" in the loop's own order, so that its counts hold from the first
     // stage on; before them the header and the quants of stage 0
-    u32x4 hd_cur, hd_next = {0U, 0U, 0U, 0U}, qs[4];
+    u32x4 hd_cur, hd_next = {0U, 0U, 0U, 0U}, qs[4], qn[4];            // (qn: the next super-block's quants, WHOLE only)
     u32x4 mreg_hi = {0U, 0U, 0U, 0U}, mreg_lo = {0U, 0U, 0U, 0U};      // B operand of the S x M product: -(1024 d + dmin m_j), j = 8 half .. + 8
-    fetch_header(0, hd_cur); fetch_quants(0, qs[0]);
-    copy_tokens(0, tok_stage[0]); copy_sums(0); fetch_quants(1, qs[1]);
-    copy_tokens(1, tok_stage[1]); fetch_quants(2, qs[2]);
-    copy_tokens(2, tok_stage[2]); fetch_quants(3, qs[3]);
-    // younger than the token copies of stage 0: sums + quants, then two stages of NT + 1
-    asm volatile("s_waitcnt vmcnt(%2)" : "+v"(hd_cur), "+v"(qs[0]) : "n"(2U * NT + 4U) : "memory");
+    if constexpr (WHOLE) {
+        fetch_header(0, hd_cur);
+#pragma unroll
+        for (uint32_t j = 0; j < 4U; ++j) fetch_quants(j, qs[j]);
+        copy_tokens(0, tok_stage[0]); copy_sums(0);
+        copy_tokens(1, tok_stage[1]);
+        copy_tokens(2, tok_stage[2]);
+        // younger than the token copies and sums of stage 0: two stages of NT
+        asm volatile("s_waitcnt vmcnt(%5)" : "+v"(hd_cur), "+v"(qs[0]), "+v"(qs[1]), "+v"(qs[2]), "+v"(qs[3]) : "n"(2U * NT) : "memory");
+    } else {
+        fetch_header(0, hd_cur); fetch_quants(0, qs[0]);
+        copy_tokens(0, tok_stage[0]); copy_sums(0); fetch_quants(1, qs[1]);
+        copy_tokens(1, tok_stage[1]); fetch_quants(2, qs[2]);
+        copy_tokens(2, tok_stage[2]); fetch_quants(3, qs[3]);
+        // younger than the token copies of stage 0: sums + quants, then two stages of NT + 1
+        asm volatile("s_waitcnt vmcnt(%2)" : "+v"(hd_cur), "+v"(qs[0]) : "n"(2U * NT + 4U) : "memory");
+    }
     pf_barrier();
 
     half8 bfrag;                                       // B operand of the next k-step
@@ -182,51 +212,72 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
         scales(hd_cur, 0, s_lo, s_hi);
         bfrag = expand(qs[0].x & 0x0f0f0f0fU, qs[0].y & 0x0f0f0f0fU, s_lo);
     }
+    // A stage's MFMAs as a flat sequence of slots m = (k-step j, plane, token tile i); the A operand of slot m + W is requested right after
+    // the MFMA of slot m into the registers that MFMA has just read (a window of W operands, which runs on over the stages' borders).
+    constexpr uint32_t PER = PLANES * LIVE, N = 4U * PER, W = N / 2U < 4U ? N / 2U : 4U;
+    half8 frag[W];
+    const auto request = [&](uint32_t m, const pf_lds* stage) __attribute__((always_inline)) {
+        const uint32_t j = m / PER, pl = (m / LIVE) % PLANES, i = m % LIVE;
+        frag[m % W] = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(stage + trow + pl * STAGE + i * 32U * 128U + piece_at[j]);
+    };
+#pragma unroll
+    for (uint32_t m = 0; m < W; ++m) request(m, tok_stage[0]);
 
     {
         const auto stage = [&](auto p_constant, uint32_t b) __attribute__((always_inline)) {
                 constexpr uint32_t p = decltype(p_constant)::value;
                 const uint32_t s = 4U * b + p;
-                // ---- issue: token copies three stages ahead, the header of the next super-block / the sums of the next group
-                copy_tokens(s + 3U, tok_stage[(p + 3U) & 3U]);
-                if (p == 0) fetch_header(b + 1U, hd_next);
-                if (p == 1) copy_sums((b >> 1) + 1U);
                 uint32_t s_lo, s_hi;
                 scales(hd_cur, p, s_lo, s_hi);
                 const u32x4 qw = qs[p];
-                const pf_lds* tok = tok_stage[p] + trow;
-                // The stage's MFMAs as a flat sequence of slots m = (k-step j, plane, token tile i); the A operand of slot m + W is
-                // requested right after the MFMA of slot m into the registers that MFMA has just read (a window of W operands).
-                constexpr uint32_t PER = PLANES * LIVE, N = 4U * PER, W = N < 4U ? N : 4U;
-                half8 frag[W];
-                const auto request = [&](uint32_t m) __attribute__((always_inline)) {
-                    const uint32_t j = m / PER, pl = (m / LIVE) % PLANES, i = m % LIVE;
-                    frag[m % W] = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(tok + pl * STAGE + i * 32U * 128U + piece_at[j]);
-                };
+                const float d_now = half_bits_to_float(hd_cur.x & 0xffffU);
+                const auto fold = [&](uint32_t i) __attribute__((always_inline)) {       // end of a super-block: running sum += d * P
 #pragma unroll
-                for (uint32_t m = 0; m < W; ++m) request(m);
+                    for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(d_now, part[i][r], acc[i][r]);
+                };
                 half8 bcur = bfrag;
+                u32x4 bnext = __builtin_bit_cast(u32x4, bfrag);
+                uint32_t nw0 = 0, nw1 = 0, nsc = 0;            // the next k-step's quant words and scale
 #pragma unroll
                 for (uint32_t m = 0; m < N; ++m) {
                     const uint32_t j = m / PER, i = m % LIVE;
                     if (m % PER == 0) {
-                        // a new k-step: take its B operand and expand the next one while this k-step multiplies
-                        bcur = bfrag;
-                        if (j == 0) bfrag = expand(qw.z & 0x0f0f0f0fU, qw.w & 0x0f0f0f0fU, s_lo);
-                        else if (j == 1) bfrag = expand((qw.x >> 4) & 0x0f0f0f0fU, (qw.y >> 4) & 0x0f0f0f0fU, s_hi);
+                        // a new k-step: take its B operand; the next one's is expanded between this one's MFMAs
+                        bcur = __builtin_bit_cast(half8, bnext);
+                        if (j == 0) { nw0 = qw.z & 0x0f0f0f0fU; nw1 = qw.w & 0x0f0f0f0fU; nsc = s_lo; }
+                        else if (j == 1) { nw0 = (qw.x >> 4) & 0x0f0f0f0fU; nw1 = (qw.y >> 4) & 0x0f0f0f0fU; nsc = s_hi; }
                         else if (j == 2) {
-                            bfrag = expand((qw.z >> 4) & 0x0f0f0f0fU, (qw.w >> 4) & 0x0f0f0f0fU, s_hi);
-                            fetch_quants(s + 4U, qs[p]);             // the stage's quant registers are free now
+                            nw0 = (qw.z >> 4) & 0x0f0f0f0fU; nw1 = (qw.w >> 4) & 0x0f0f0f0fU; nsc = s_hi;
+                            // The stage's middle: its token copies' turn. The tokens of stage s + 1 were copied two stages ago (younger: the rest
+                            // of that stage's operations and the next one's); behind the barrier every wave's have landed, and every wave
+                            // has read the last of stage s - 1, whose slot takes stage s + 3. (At a stage's border the barrier made both waves
+                            // of a SIMD wait for their first operands at once.)
+                            rg_wait<static_cast<int>(rg_stage_ops(NT, (p + 2U) & 3U, WHOLE) - NT + rg_stage_ops(NT, (p + 3U) & 3U, WHOLE))>();
+                            asm volatile("s_barrier" ::: "memory");
+                            copy_tokens(s + 3U, tok_stage[(p + 3U) & 3U]);
+                            if (p == 1) copy_sums((b >> 1) + 1U);
+                            if (!WHOLE) fetch_quants(s + 4U, qs[p]);             // the stage's quant registers are free now
+                            if (p == 0) fetch_header(b + 1U, hd_next);
+                            if (WHOLE && p == 0) {
+#pragma unroll
+                                for (uint32_t q4 = 0; q4 < 4U; ++q4) fetch_quants(s + 4U + q4, qn[q4]);
+                            }
                         } else {
-                            // first k-step of the next stage: its quants were fetched at the end of stage s - 3 (younger operations:
-                            // the whole of stages s - 2, s - 1 and s), its header - when it opens a super-block - in stage s - 3
+                            // first k-step of the next stage: its quants (the next super-block's header with them) were fetched in stage s - 3
+                            // (WHOLE: all of the next super-block's in stage 0); younger the three stages since
                             constexpr uint32_t pn = (p + 1U) & 3U;
-                            constexpr uint32_t younger = rg_stage_ops(NT, (p + 2U) & 3U) + rg_stage_ops(NT, (p + 3U) & 3U) + rg_stage_ops(NT, p);
-                            if (p == 3U) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(qs[pn]), "+v"(hd_next) : "n"(younger) : "memory");
+                            constexpr uint32_t younger = rg_stage_ops(NT, (p + 2U) & 3U, WHOLE) + rg_stage_ops(NT, (p + 3U) & 3U, WHOLE) + rg_stage_ops(NT, p, WHOLE);
+                            if (WHOLE) {
+                                if (p == 3U) {
+                                    asm volatile("s_waitcnt vmcnt(%5)" : "+v"(hd_next), "+v"(qn[0]), "+v"(qn[1]), "+v"(qn[2]), "+v"(qn[3]) : "n"(younger) : "memory");
+#pragma unroll
+                                    for (uint32_t q4 = 0; q4 < 4U; ++q4) qs[q4] = qn[q4];
+                                }
+                            } else if (p == 3U) asm volatile("s_waitcnt vmcnt(%2)" : "+v"(qs[pn]), "+v"(hd_next) : "n"(younger) : "memory");
                             else asm volatile("s_waitcnt vmcnt(%1)" : "+v"(qs[pn]) : "n"(younger) : "memory");
                             uint32_t n_lo, n_hi;
                             scales(p == 3U ? hd_next : hd_cur, pn, n_lo, n_hi);
-                            bfrag = expand(qs[pn].x & 0x0f0f0f0fU, qs[pn].y & 0x0f0f0f0fU, n_lo);
+                            nw0 = qs[pn].x & 0x0f0f0f0fU; nw1 = qs[pn].y & 0x0f0f0f0fU; nsc = n_lo;
                         }
                     }
                     if (p == 0 && m < LIVE) {                        // first MFMA of a super-block's product: it starts from zero
@@ -235,11 +286,18 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
                     } else {
                         part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[m % W], bcur, part[i], 0, 0, 0);
                     }
-                    if (m + W < N) request(m + W);
+                    if (m + W < N) request(m + W, tok_stage[p]);
+                    else request(m + W - N, tok_stage[(p + 1U) & 3U]);
+                    // this slot's share of the next k-step's four operand registers
+#pragma unroll
+                    for (uint32_t q = 4U * (m % PER) / PER; q < 4U * (m % PER + 1U) / PER; ++q)
+                        bnext[q] = expand_pair(q < 2U ? nw0 : nw1, q & 1U, nsc);
+                    if (p == 3U && m > N - LIVE) fold(i - 1U);       // (the tile before this one's last product is through)
                     // the scheduler otherwise sinks the request down to its use (registers are scarce) and the MFMA then waits
                     // for the whole LDS round trip: nothing moves across this point (1874 -> 1828 us gate / up, 1642 -> 1565 us down)
                     __builtin_amdgcn_sched_barrier(0);
                 }
+                bfrag = __builtin_bit_cast(half8, bnext);
                 if (p == 1U) {
                     // this lane's M operand: the eight sub-blocks of super-block 2 g + half of the group
                     if ((b & 1U) == half) {
@@ -267,12 +325,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
                     }
                 }
                 if (p == 3U) {
-                    // end of a super-block: running sum += d * P
-                    const float d = half_bits_to_float(hd_cur.x & 0xffffU);
-#pragma unroll
-                    for (uint32_t i = 0; i < LIVE; ++i)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(d, part[i][r], acc[i][r]);
+                    fold(LIVE - 1U);
                     if ((b & 1U) || b + 1U == blocks) {
                         // end of a group of 16 sub-blocks: running sum += S hi * M hi + S lo * M hi + S hi * M lo
                         const pf_lds* st = s_tile + ((b >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 16U * half;
@@ -288,11 +341,6 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
                     }
                     hd_cur = hd_next;
                 }
-                // the token copies of stage s + 1 were issued at the start of stage s - 2: younger operations = the rest of that
-                // stage and the whole of stages s - 1 and s
-                constexpr uint32_t younger_tokens = rg_stage_ops(NT, (p + 2U) & 3U) - NT + rg_stage_ops(NT, (p + 3U) & 3U) + rg_stage_ops(NT, p);
-                rg_wait<static_cast<int>(younger_tokens)>();
-                pf_barrier();
         };
         for (uint32_t b = 0; b < blocks; ++b) {
             stage(std::integral_constant<uint32_t, 0>{}, b);
@@ -362,6 +410,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
             }
     }
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(hd_cur), "+v"(hd_next), "+v"(qs[0]), "+v"(qs[1]), "+v"(qs[2]), "+v"(qs[3]) : : "memory");
+    pf_barrier();                                         // (every wave's copies have landed and its reads are through: the slots are free)
     };
     const uint32_t live_tiles = (count + 31U) / 32U;
     if constexpr (TILES == 4U) {
@@ -370,9 +419,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prefill_reg_kernel(PrefillArgs 
         else if (live_tiles == 2U) run_unit(std::integral_constant<uint32_t, 2>{});
         else run_unit(std::integral_constant<uint32_t, 1>{});
     } else {
-        static_assert(TILES == 2U, "live tiles of the narrow form");
-        if (live_tiles == 2U) run_unit(std::integral_constant<uint32_t, 2>{});
-        else run_unit(std::integral_constant<uint32_t, 1>{});
+        static_assert(TILES == 1U, "live tiles of the four-wave form");
+        run_unit(std::integral_constant<uint32_t, 1>{});
     }
     }   // units
 }

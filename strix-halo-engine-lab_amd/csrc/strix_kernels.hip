@@ -2304,8 +2304,8 @@ struct PrefillViews {
 // expert plan, sub-block sums of the input rows, gate / up + SwiGLU, down rows. check: the routes' check and the status words ride with the
 // sums (null: they are already written)
 int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v, uint32_t rows, hipStream_t st, const RouteCheck* check = nullptr) {
-    const uint32_t assignments = rows * wv.top_k, bound = plan_item_bound(wv.experts, assignments, kPfTile);
-    launch_plan(v.routes, wv.experts, assignments, kPfTile, bound, v.plan, st);
+    const uint32_t assignments = rows * wv.top_k, split = prefill_split(wv, assignments), bound = plan_item_bound(wv.experts, assignments, split);
+    launch_plan(v.routes, wv.experts, assignments, split, bound, v.plan, st);
     PrefillArgs a{};
     a.top_k = wv.top_k; a.exp_kind = wv.exp_kind; a.swiglu_limit = wv.swiglu_limit; a.x = static_cast<const uint8_t*>(v.input); a.x_stride = v.input_stride;
     uint8_t* ws = static_cast<uint8_t*>(v.h_f16);
