@@ -312,40 +312,39 @@ __global__ __launch_bounds__(1024) void plan_order_kernel(RoutesView routes, uin
     }
 }
 
-// Exclusive prefix sum of one value per thread over a 1024-thread workgroup (16 waves); `total` is the sum over all threads.
-// wave_totals: 16 shared words of the caller's, not reused before its next barrier.
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* wave_totals, uint32_t& total) {
-    const uint32_t lane = threadIdx.x & 63U, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (uint32_t d = 1; d < 64U; d <<= 1) {
-        const uint32_t below = __shfl_up(x, d);
-        if (lane >= d) x += below;
+// Inclusive prefix sum over a wavefront: row shifts inside the rows of 16, then the rows' totals by row broadcasts (DPP, no LDS).
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xF, 0xF, false));      // row_shr:1
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xF, 0xF, false));      // row_shr:2
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xF, 0xF, false));      // row_shr:4
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xF, 0xF, false));      // row_shr:8
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xA, 0xF, false));      // row_bcast:15 into rows 1 and 3
+    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xC, 0xF, false));      // row_bcast:31 into rows 2 and 3
+    return v;
+}
+// Lanes of the wavefront whose key (of `bits` bits) equals this lane's, among the lanes that `take` part: a ballot per bit.
+__device__ __forceinline__ uint64_t lanes_of_key(uint32_t key, uint32_t bits, bool take) {
+    uint64_t same = __ballot(take);
+    for (uint32_t b = 0; b < bits; ++b) {
+        const bool set = (key >> b) & 1U;
+        const uint64_t votes = __ballot(set);
+        same &= set ? votes : ~votes;
     }
-    if (lane == 63U) wave_totals[wave] = x;
-    __syncthreads();
-    uint32_t base = 0, sum = 0;
-    for (uint32_t w = 0; w < 16U; ++w) {
-        const uint32_t t = wave_totals[w];
-        base += w < wave ? t : 0U;
-        sum += t;
-    }
-    total = sum;
-    return base + x - v;
+    return same;
 }
 
 // The expert plan in one workgroup: thread e owns expert e (its count, three prefix sums for the offsets, the item numbers and the touched
 // list, then its own items). A batch of at most 1024 assignments (fill_order) is ordered here as well: wave w holds assignments
-// 64 w .. 64 w + 63, finds each one's position among its wave's assignments of the same expert by ballots (one round per expert named)
+// 64 w .. 64 w + 63, finds each one's position among its wave's assignments of the same expert by ballots (one per bit of the expert)
 // and leaves the wave's counts; a prefix over the waves and the expert's offset make it the position in the order. (A thread per expert
-// that walked every assignment took 12 us at 128 assignments; the order launch it saves at 257..1024 takes 4.7 us.)
+// that walked every assignment took 12 us at 128 assignments; the order launch it saves at 257..1024 takes 4.7 us.) Bound by latency: the
+// prefix sums by DPP with one hand-off through LDS for all three, 320 assignments over 128 experts 8.3 -> 4.9 us.
 constexpr uint32_t kPlanSmall = 1024;
 __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split,
                                                     uint32_t item_bound, uint32_t fill_order, uint32_t* plan) {
     __shared__ uint32_t count[kRouteMaxExperts];           // per expert: assignments, later (fill_order) its offset
     __shared__ uint16_t wave_counts[16][kRouteMaxExperts]; // fill_order: per wave and expert, later the prefix over the waves before
-    __shared__ uint32_t wave_totals[3][16];
-    __shared__ uint32_t wave_largest[16];
+    __shared__ u32x4 wave_totals[16];                      // per wave: assignments, items, touched experts, largest group
     const uint32_t tid = threadIdx.x, lane = tid & 63U, wave = tid >> 6, waves = (assignments + 63U) / 64U;
     count[tid] = 0;
     uint32_t mine = experts, rank = 0;                     // fill_order: this thread's assignment's expert, its position in the wave
@@ -355,13 +354,10 @@ __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t 
     }
     __syncthreads();
     if (fill_order) {
-        uint64_t left = __ballot(mine < experts);
-        while (left) {
-            const uint32_t e = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), __builtin_ctzll(left)));
-            const uint64_t same = __ballot(mine == e);
-            if (mine == e) rank = static_cast<uint32_t>(__popcll(same & ((1ULL << lane) - 1ULL)));
-            if (lane == 0) wave_counts[wave][e] = static_cast<uint16_t>(__popcll(same));
-            left &= ~same;
+        const uint64_t same = lanes_of_key(mine, 32U - static_cast<uint32_t>(__builtin_clz(experts)), mine < experts);
+        if (mine < experts) {
+            rank = static_cast<uint32_t>(__popcll(same & ((1ULL << lane) - 1ULL)));
+            if (rank == 0) wave_counts[wave][mine] = static_cast<uint16_t>(__popcll(same));
         }
     } else {
         for (uint32_t a = tid; a < assignments; a += 1024U) {
@@ -379,18 +375,24 @@ __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t 
         }
     }
     const uint32_t pieces = (c + split - 1U) / split;
-    uint32_t run, made, touched;
-    const uint32_t first = block_exclusive_scan(c, wave_totals[0], run);
-    const uint32_t item_from = block_exclusive_scan(pieces, wave_totals[1], made);
-    const uint32_t touched_from = block_exclusive_scan(c != 0 ? 1U : 0U, wave_totals[2], touched);
+    const uint32_t runs = wave_inclusive_scan(c), items_to = wave_inclusive_scan(pieces), touched_to = static_cast<uint32_t>(__popcll(__ballot(c != 0) & ((2ULL << lane) - 1ULL)));
     uint32_t largest = c;
 #pragma unroll
     for (int d = 32; d; d >>= 1) {
         const uint32_t other = __shfl_xor(largest, d);
         largest = other > largest ? other : largest;
     }
-    if (lane == 0) wave_largest[wave] = largest;
+    if (lane == 63U) wave_totals[wave] = u32x4{runs, items_to, touched_to, largest};
     __syncthreads();
+    u32x4 before = {0U, 0U, 0U, 0U}, all = {0U, 0U, 0U, 0U};
+#pragma unroll
+    for (uint32_t w = 0; w < 16U; ++w) {
+        const u32x4 t = wave_totals[w];
+        if (w < wave) { before.x += t.x; before.y += t.y; before.z += t.z; }
+        all.x += t.x; all.y += t.y; all.z += t.z; all.w = t.w > all.w ? t.w : all.w;
+    }
+    const uint32_t first = before.x + runs - c, item_from = before.y + items_to - pieces, touched_from = before.z + touched_to - (c != 0 ? 1U : 0U);
+    const uint32_t run = all.x, made = all.y, touched = all.z, most = all.w;
     uint32_t* offsets = plan + kPlanOffsetsAt;
     uint32_t* touched_ids = plan + plan_touched_at(experts);
     uint32_t* order = plan + plan_order_at(experts);
@@ -405,8 +407,6 @@ __global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t 
     }
     for (uint32_t u = made + tid; u < item_bound; u += 1024U) *reinterpret_cast<uint4*>(items + 4U * u) = make_uint4(0U, 0U, 0U, 0U);
     if (tid == 0) {
-        uint32_t most = 0;
-        for (uint32_t w = 0; w < 16U; ++w) most = wave_largest[w] > most ? wave_largest[w] : most;
         offsets[experts] = run;
         plan[0] = assignments; plan[1] = touched; plan[2] = most; plan[4] = made;
     }
@@ -994,44 +994,59 @@ __global__ __launch_bounds__(256) void down_quad_kernel(mi355_moe_weights w, Row
 // src/ds41_expert_tp.cpp:189-199 (product then add, slots in ascending expert id).
 // VEC = columns per thread (4: every row of rawdots / base / output starts on 16 bytes and hidden % 4 == 0). The slots'
 // values are all requested before the chain starts, so a thread has top_k loads in flight instead of one.
+// Bound by latency up to some hundred rows. So every wavefront looks the row up by itself - lane k the route and weight of slot k, its place
+// in the ascending order by comparison with the others' - and in slot order nothing stands in front of the values' loads: one way to memory
+// (two in ascending order), where one thread of the workgroup, a barrier and, for the order, an insertion sort over routes in memory took
+// up to four (16 rows x 6144, top-8 ascending: 8.4 -> 5.0 us; 333 rows x 2048, top-8 11.2 -> 6.3; 1000 rows 18.8 -> 13.0).
 template <int VEC>
 __global__ __launch_bounds__(256) void merge_kernel(mi355_moe_weights w, RowsK r, uint32_t form) {
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
-    __shared__ uint32_t slot_order[16];
-    __shared__ float slot_weight[16];
-    __shared__ uint32_t row_failed;
-    const uint32_t row = blockIdx.y, o = (blockIdx.x * 256U + threadIdx.x) * VEC;
-    if (threadIdx.x == 0) {
-        // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is this kernel's own), and
-        // neither does any row of a job whose down phase was skipped (its unweighted outputs are not this job's)
-        row_failed = (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE)) | (*r.job_status & MI355_STATUS_NONFINITE_PROJECTION);
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t j = i; j > 0 && r.routes_of(row)[slot_order[j]] < r.routes_of(row)[slot_order[j - 1]]; --j) {
-                    const uint32_t t = slot_order[j]; slot_order[j] = slot_order[j - 1]; slot_order[j - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
-    __syncthreads();
-    if (o >= w.hidden || row_failed) return;
+    const uint32_t row = blockIdx.y, o = (blockIdx.x * 256U + threadIdx.x) * VEC, lane = threadIdx.x & 63U, K = w.top_k;
+    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is this kernel's own), and
+    // neither does any row of a job whose down phase was skipped (its unweighted outputs are not this job's)
+    const uint32_t row_status = *r.status_of(row), job = *r.job_status;
+    const bool ascending = form == MI355_COMBINE_MULADD_ASCENDING_EXPERT;
+    const float weight = lane < K ? r.route_weights_of(row)[lane] : 0.0F;
+    const uint32_t at = o < w.hidden ? o : 0U;
+    const float* const values = reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(r.rawdots) + row * r.rawdots_rs) + at;
     vec_t e[16];
+    uint32_t slot[16];
+    if (!ascending) {
 #pragma unroll
-    for (uint32_t k = 0; k < 16U; ++k)
-        if (k < w.top_k) e[k] = *reinterpret_cast<const vec_t*>(r.rawdots_of(row * w.top_k + slot_order[k], w.hidden) + o);
-    vec_t y;
-    bool finite = true;
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) {
-        float acc = 0.0F;
+        for (uint32_t k = 0; k < 16U; ++k) slot[k] = k;
+    } else {
+        const uint32_t route = lane < K ? r.routes_of(row)[lane] : 0xffffffffU;
+        uint32_t place = 0;                               // stable: an equal expert in an earlier slot goes first
 #pragma unroll
         for (uint32_t k = 0; k < 16U; ++k) {
-            if (k >= w.top_k) continue;
-            const float v = e[k][c];
-            if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) acc = __builtin_fmaf(slot_weight[k], v, acc);
-            else acc = acc + slot_weight[k] * v;
+            const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(route), static_cast<int>(k)));
+            place += k < K && (other < route || (other == route && k < lane)) ? 1U : 0U;
         }
-        const float out = r.base ? acc + r.base_of(row)[o + c] : acc;
+#pragma unroll
+        for (uint32_t k = 0; k < 16U; ++k) slot[k] = k < K ? static_cast<uint32_t>(__builtin_ctzll(__ballot(lane < K && place == k))) : 0U;
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 16U; ++k)
+        if (k < K) e[k] = *reinterpret_cast<const vec_t*>(values + static_cast<size_t>(slot[k]) * w.hidden);
+    if (o >= w.hidden || (row_status & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE)) || (job & MI355_STATUS_NONFINITE_PROJECTION)) return;
+    vec_t y;
+    bool finite = true;
+    float acc[VEC];
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) acc[c] = 0.0F;
+#pragma unroll
+    for (uint32_t k = 0; k < 16U; ++k) {
+        if (k >= K) continue;
+        const float wt = f_of(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b_of(weight)), static_cast<int>(slot[k]))));
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) {
+            if (!ascending && k + r.shared_slots < K) acc[c] = __builtin_fmaf(wt, e[k][c], acc[c]);
+            else acc[c] = acc[c] + wt * e[k][c];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) {
+        const float out = r.base ? acc[c] + r.base_of(row)[o + c] : acc[c];
         finite = finite && finite_f(out);
         y[c] = out;
     }
@@ -2032,9 +2047,9 @@ int32_t enqueue_merge(const mi355_moe_weights* w, const mi355_moe_rows* r, uint3
     STRIX_REQUIRE(rows <= 65535U, "moe merge: at most 65535 rows per call");
     RowsK k = rows_k(*r, wv);
     k.shared_slots = shared_slots;
-    // four columns per thread once that still leaves every compute unit several workgroups (4096 rows x 4096: 194 -> 113 us;
-    // a decode batch is faster with one column per thread: 16 rows x 6144: 8.5 against 10.9 us)
-    const bool quads = static_cast<uint64_t>(rows) * ((wv.hidden + 1023U) / 1024U) >= 4ULL * compute_units() && wv.hidden % 4U == 0 && aligned(k.rawdots, 16) && k.rawdots_rs % 16U == 0 && aligned(k.output, 16) && k.output_stride % 4U == 0 &&
+    // four columns per thread once that still leaves every compute unit two workgroups (333 rows x 2048, 666 workgroups: 6.9 -> 6.3 us;
+    // a decode batch is faster with one column per thread: 16 rows x 6144: 5.0 against 6.1 us)
+    const bool quads = static_cast<uint64_t>(rows) * ((wv.hidden + 1023U) / 1024U) >= 2ULL * compute_units() && wv.hidden % 4U == 0 && aligned(k.rawdots, 16) && k.rawdots_rs % 16U == 0 && aligned(k.output, 16) && k.output_stride % 4U == 0 &&
                        (!k.base || (aligned(k.base, 16) && k.base_rs % 16U == 0));
     if (quads) merge_kernel<4><<<dim3((wv.hidden + 1023U) / 1024U, rows), 256, 0, hs(stream)>>>(wv, k, form);
     else merge_kernel<1><<<dim3((wv.hidden + 255U) / 256U, rows), 256, 0, hs(stream)>>>(wv, k, form);
