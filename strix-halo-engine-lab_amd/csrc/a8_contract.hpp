@@ -522,9 +522,9 @@ int32_t a8_down_rawdots(const mi355_a8_down_request* q, const mi355_a8_down_bind
     const uint32_t items = logical_rows * s.top_k;
     r.union_plan = union_plan;
     if (union_plan) {               // K-quant only: the items are the plan's entries
-        if (q->weight_type == MI355_TYPE_Q6_K) launch_down_q6k(w, r, dim3(s.hidden / kDownGroupsRows, items), items, 0U, 0U, st);
-        else if (logical_rows > 4U) launch_down_nb<8>(w, r, logical_rows, dim3(s.hidden / 64U, items), st);
-        else launch_down_nb<4>(w, r, logical_rows, dim3(s.hidden / 64U, items), st);
+        // (as the gate / up rows; the vector-ALU sweeps of four or eight before: 6 rows x top-16 over 64 experts of 1536 x 1536, Q6_K 89 -> 76 us
+        // the three calls, Q4_K 77 -> 68; 8 rows x top-8 over 30 experts of 4096 x 2048 144 -> 120, 111 -> 103)
+        launch_mma_down(w, r, logical_rows, 0, items, 4U, st);
     } else if (q->weight_type != MI355_TYPE_Q4_K) {
         const dim3 grid(s.hidden / kDownGroupsRows, items);
         if (q->weight_type == MI355_TYPE_Q8_0) down_groups_kernel<0><<<grid, 256, 0, st>>>(w, r, items, 0U, 0U);

@@ -26,7 +26,8 @@ uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments);
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at,
                              uint32_t order_at, hipStream_t st);
 
-// q4k_mma.hip: Q4_K experts on the int8 matrix cores. dense: the rows of a one-expert batch (0: planned items); width: the most rows an
+// q4k_mma.hip: experts on the int8 matrix cores (gate / up Q4_K or Q5_K; down Q4_K, Q6_K, or Q8_0 and Q5_1 rows of whole stages of 256 weights;
+// dense batches Q4_K). dense: the rows of a one-expert batch (0: planned items); width: the most rows an
 // item (or the dense batch) holds. The last leaves the raw gate and up values of a dense batch of at most 16 rows.
 void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st);
 void launch_mma_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st);

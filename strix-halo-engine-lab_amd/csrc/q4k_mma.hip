@@ -1,4 +1,4 @@
-// Q4_K experts on the int8 matrix cores (q4k_mma_moe.hpp): which instance serves a launch.
+// Experts on the int8 matrix cores (q4k_mma_moe.hpp): which instance serves a launch.
 #include "host_common.hpp"
 #include "launchers.hpp"
 #include "q4k_mma_moe.hpp"
@@ -22,44 +22,58 @@ inline MmaGrid mma_grid(const mi355_moe_weights& w, uint32_t rows, uint32_t dens
 }
 // the rows of a dense batch at a stride of their own (every dense buffer and strided view; not the executor's pointer tables)
 inline bool mma_direct(const A8Image& img, uint32_t dense) { return dense && img.per_row == 1U && !img.table; }
-template <int NAL>
+template <int FMT, int NAL>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items)));
     constexpr int DEPTH = NAL >= 8 ? 2 : 3;
-    if (mma_direct(r.in, dense)) q4k_mma_project_kernel<NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
-    else q4k_mma_project_kernel<NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    if (FMT == kMmaQ4K && mma_direct(r.in, dense)) q4k_mma_project_kernel<kMmaQ4K, NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    else q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
 // rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
-template <int NAL>
+template <int FMT, int NAL>
 inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     const uint32_t tiles = w.hidden / kMmaRows;
     const bool direct = mma_direct(r.h, dense);
-    if constexpr (NAL <= 8) {
+    if constexpr (FMT == kMmaQ4K) {
         const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, 1U);
         if (static_cast<uint64_t>(g.grid.x) * g.grid.y <= compute_units()) {
-            if (direct) q4k_mma_down_kernel<NAL, 2, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
-            else q4k_mma_down_kernel<NAL, 2, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            if (direct) q4k_mma_down_kernel<FMT, NAL, 2, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            else q4k_mma_down_kernel<FMT, NAL, 2, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
             return;
         }
     }
     const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, mma_run_tiles(w.ffn / 256U, NAL >= 8 ? 6U : 12U, static_cast<uint64_t>(tiles) * (dense ? 1U : items)));
-    constexpr int DEPTH = NAL >= 8 ? 2 : 3;
-    if (direct) q4k_mma_down_kernel<NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
-    else q4k_mma_down_kernel<NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    // (Q6_K: a fourth or sixth workgroup on a compute unit is worth more than a third slot: 24 rows of hidden 4096 / ffn 1536 / 64 experts
+    // 178.3 -> 176.5 us; Q8_0, 40 rows of hidden 2048 / ffn 768 / 128 experts, 124.4 us with three slots, 126.5 with two)
+    constexpr int DEPTH = NAL >= 8 || FMT == kMmaQ6K ? 2 : 3;
+    if (FMT == kMmaQ4K && direct) q4k_mma_down_kernel<kMmaQ4K, NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    else q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+}
+template <int FMT>
+inline void launch_mma_project_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
+    if (width <= 4U) launch_mma_project_nal<FMT, 2>(w, r, rows, dense, items, st);
+    else if (width <= 8U) launch_mma_project_nal<FMT, 4>(w, r, rows, dense, items, st);
+    else if (width <= 16U) launch_mma_project_nal<FMT, 8>(w, r, rows, dense, items, st);
+    else launch_mma_project_nal<FMT, 16>(w, r, rows, dense, items, st);
+}
+// (the down rows run best 16 rows to a sweep: 4096 rows over 256 experts, hidden 4096 / ffn 2048: 2.57 ms against 3.03 ms with 32)
+template <int FMT>
+inline void launch_mma_down_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
+    if (width <= 4U) launch_mma_down_nal<FMT, 2>(w, r, rows, dense, items, st);
+    else if (width <= 8U) launch_mma_down_nal<FMT, 4>(w, r, rows, dense, items, st);
+    else launch_mma_down_nal<FMT, 8>(w, r, rows, dense, items, st);
 }
 // width: the most rows an item (or the dense batch) holds
 void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
-    if (width <= 4U) launch_mma_project_nal<2>(w, r, rows, dense, items, st);
-    else if (width <= 8U) launch_mma_project_nal<4>(w, r, rows, dense, items, st);
-    else if (width <= 16U) launch_mma_project_nal<8>(w, r, rows, dense, items, st);
-    else launch_mma_project_nal<16>(w, r, rows, dense, items, st);
+    if (w.gate_type == MI355_TYPE_Q5_K) launch_mma_project_format<kMmaQ5K>(w, r, rows, dense, items, width, st);
+    else launch_mma_project_format<kMmaQ4K>(w, r, rows, dense, items, width, st);
 }
-// (the down rows run best 16 rows to a sweep: 4096 rows over 256 experts, hidden 4096 / ffn 2048: 2.57 ms against 3.03 ms with 32)
 void launch_mma_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
-    if (width <= 4U) launch_mma_down_nal<2>(w, r, rows, dense, items, st);
-    else if (width <= 8U) launch_mma_down_nal<4>(w, r, rows, dense, items, st);
-    else launch_mma_down_nal<8>(w, r, rows, dense, items, st);
+    if (w.down_type == MI355_TYPE_Q6_K) launch_mma_down_format<kMmaQ6K>(w, r, rows, dense, items, width, st);
+    else if (w.down_type == MI355_TYPE_Q8_0) launch_mma_down_format<kMmaQ80>(w, r, rows, dense, items, width, st);
+    else if (w.down_type == MI355_TYPE_Q5_1) launch_mma_down_format<kMmaQ51>(w, r, rows, dense, items, width, st);
+    else launch_mma_down_format<kMmaQ4K>(w, r, rows, dense, items, width, st);
 }
 void launch_mma_gate_up_rows(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, hipStream_t st) {
     const uint32_t tiles = w.ffn / kMmaRows;
@@ -67,8 +81,8 @@ void launch_mma_gate_up_rows(const mi355_moe_weights& w, const RowsK& r, uint32_
     const dim3 grid(tiles, 1, 2);
     const auto launch = [&](auto direct) {
         constexpr bool D = decltype(direct)::value;
-        if (rows <= 8U) q4k_mma_down_kernel<4, 3, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
-        else q4k_mma_down_kernel<8, 2, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
+        if (rows <= 8U) q4k_mma_down_kernel<kMmaQ4K, 4, 3, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
+        else q4k_mma_down_kernel<kMmaQ4K, 8, 2, 1, D, true><<<grid, 256, 0, st>>>(MmaArgs{w, r, l});
     };
     if (mma_direct(r.in, rows)) launch(std::true_type{});
     else launch(std::false_type{});

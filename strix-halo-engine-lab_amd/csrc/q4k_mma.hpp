@@ -1,4 +1,4 @@
-// Q4_K x A8 rows against 3..32 activation rows at a time: the exact group dots come from the int8 matrix cores, the
+// Q4_K x A8 rows (and the reference's other formats of expert rows, below) against 1..32 activation rows at a time: the exact group dots come from the int8 matrix cores, the
 // reference's fp32 chain stays on the vector ALU. The sweep below serves dense matrices and the routed
 // experts of larger batches (q4k_mma_moe.hpp: gate + up with the SwiGLU / A8 epilogue, and the down rows).
 //
@@ -19,8 +19,9 @@
 // two sub-blocks (delta 2p, delta 2p + 1, sum 2p, sum 2p + 1) in its four lanes and the multiplies take them by quad
 // broadcast (a DPP operand, no instruction of its own).
 //
-// Data path: a stage is one super-block of the 32 rows (4,608 bytes, rows back to back: a row is 144 = 128 + 16 bytes, so eight
-// neighbouring rows read eight different 16-byte bank groups), the 256 codes of every activation row (piece t of row a at
+// Data path: a stage is one super-block (256 weights) of the 32 rows in 16-byte pieces, an odd number of them from row to row, so that
+// sixteen neighbouring rows read sixteen different 16-byte bank groups (the even 14 and 12 of Q6_K and Q5_1: down rows of a layer of 40 rows,
+// hidden 2048 / ffn 768 / 128 experts, Q5_1 139 -> 127 us; three calls over a union of 6 x 16 Q6_K rows, 90 -> 78), the 256 codes of every activation row (piece t of row a at
 // position (t + a) % 16 of its 16 pieces, which spreads eight rows over the bank groups) and one table piece per row
 // (8 deltas, 8 sums). Everything arrives by global_load_lds_dwordx4 into a ring of DEPTH slots shared by the workgroup: a
 // wavefront waits for its own copies (counted s_waitcnt vmcnt), the workgroup barrier publishes all of them, and the slot
@@ -43,16 +44,24 @@ typedef __attribute__((address_space(3))) uint64_t lds_u64;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 constexpr uint32_t kMmaRows = 32;
+// Formats of the weight rows: bytes of 256 weights of a row and the 16-byte pieces that hold them (Q6_K: that hold them wherever in a piece
+// the 2-byte aligned block starts).
+enum MmaFormat { kMmaQ4K, kMmaQ5K, kMmaQ6K, kMmaQ80, kMmaQ51 };
+template <int FMT> constexpr uint32_t mma_block_bytes() { return FMT == kMmaQ4K ? 144U : FMT == kMmaQ5K ? 176U : FMT == kMmaQ6K ? 210U : FMT == kMmaQ80 ? 272U : 192U; }
+template <int FMT> constexpr uint32_t mma_pieces() { return (mma_block_bytes<FMT>() + 15U) / 16U; }
+// pieces from a row to the next one in a ring slot: an odd number, so that the same words of sixteen rows lie in different banks
+template <int FMT> constexpr uint32_t mma_pitch() { return mma_pieces<FMT>() | 1U; }
+template <int FMT> constexpr uint32_t mma_weight_copies() { return (mma_pitch<FMT>() + 1U) / 2U; }          // 1 KiB = 64 pieces, the last half a wave's
+template <int FMT> constexpr uint32_t mma_weight_bytes() { return 16U * mma_pitch<FMT>() * kMmaRows; }
 template <int NAL> constexpr uint32_t mma_acts() { return 2U * NAL; }                         // activation slots served (multiple of 4)
 template <int NAL> constexpr uint32_t mma_code_copies() { return mma_acts<NAL>() / 4U; }      // 1 KiB = 4 rows x 256 codes
 template <int NAL> constexpr uint32_t mma_table_copies() { return (mma_acts<NAL>() + 15U) / 16U; }   // 1 KiB = 16 rows x (8 deltas, 8 sums)
-// NM matrices share the activation rows of a sweep (gate and up): 4.5 KiB of weight pieces each (five copies, the last of half a wave)
-template <int NAL, int NM> constexpr uint32_t mma_copies() { return 5U * NM + mma_code_copies<NAL>() + mma_table_copies<NAL>(); }
-constexpr uint32_t kMmaWeightBytes = 144U * kMmaRows;
-template <int NAL, int NM> constexpr uint32_t mma_codes_at() { return kMmaWeightBytes * NM; }
-template <int NAL, int NM> constexpr uint32_t mma_table_at() { return mma_codes_at<NAL, NM>() + 256U * mma_acts<NAL>(); }
-template <int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<NAL, NM>() + 64U * mma_acts<NAL>(); }
-template <int NAL, int NM, int DEPTH, int TEAMS> constexpr uint32_t mma_ring_bytes() { return DEPTH * TEAMS * mma_slot_bytes<NAL, NM>(); }
+// NM matrices share the activation rows of a sweep (gate and up)
+template <int FMT, int NAL, int NM> constexpr uint32_t mma_copies() { return mma_weight_copies<FMT>() * NM + mma_code_copies<NAL>() + mma_table_copies<NAL>(); }
+template <int FMT, int NM> constexpr uint32_t mma_codes_at() { return mma_weight_bytes<FMT>() * NM; }
+template <int FMT, int NAL, int NM> constexpr uint32_t mma_table_at() { return mma_codes_at<FMT, NM>() + 256U * mma_acts<NAL>(); }
+template <int FMT, int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<FMT, NAL, NM>() + 64U * mma_acts<NAL>(); }
+template <int FMT, int NAL, int NM, int DEPTH, int TEAMS> constexpr uint32_t mma_ring_bytes() { return DEPTH * TEAMS * mma_slot_bytes<FMT, NAL, NM>(); }
 template <int NAL, int TEAMS> constexpr uint32_t mma_exchange_floats() { return TEAMS > 1 ? 2U * (TEAMS - 1U) * 4U * NAL * 64U : 1U; }
 template <int NAL, int NM> constexpr uint32_t mma_reduce_floats() { return 4U * NM * NAL * 64U; }
 
@@ -100,26 +109,31 @@ template <int NAL> __device__ __forceinline__ uint32_t mma_slot_act(uint32_t i) 
     return (2U * v + h) % mma_acts<NAL>();
 }
 
-// Per-lane byte offsets into a ring slot (constant over the sweep); matrix m's weights sit 4608 m further on.
+// Per-lane byte offsets into a ring slot (constant over the sweep); matrix m's weights sit mma_weight_bytes m further on.
 struct MmaLane {
-    uint32_t head, quants, even, odd, table;
+    uint32_t head, fifth, quants, even, odd, table;
     bool sum_lane;
     uint32_t shift, even_slot;         // halves form: of the lane's sub-block in the header words; all ones where the lane's slot is of half 0
-};
+    uint32_t start;                    // Q6_K: the lane's row's first byte in its piece, of the first super-block; even_slot: all ones where the
+};                                     // lane's half of K is its slot's
+
+// Bit `bit` of every byte of a fifth-bit word, as bit 4 (Q5_K)
+__device__ __forceinline__ u32x4 mma_fifth(const u32x4& qh, uint32_t bit) { return ((qh >> bit) & 0x01010101U) << 4; }
 
 // One landed super-block: for each matrix the wavefront's two group dots of its 32 rows against every activation slot, then the
 // lane's chain terms x[2P] + x[2P + 1] for its first nv activation rows. P is the wavefront's pair, a template argument so that
 // the scale / min unpacking has constant shifts.
-template <int NAL, int NM, int P>
+template <int FMT, int NAL, int NM, int P>
 __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLane& o, uint32_t nv, float (&term)[NM][NAL]) {
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) int32_t lds_i32;
     const u32x4 a_even = *(lds_u32x4*)(slot + o.even), a_odd = *(lds_u32x4*)(slot + o.odd);
-    u32x4 hd[NM], q[NM];
+    u32x4 hd[NM], q[NM], qh[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        hd[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.head);
-        q[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.quants);
+        hd[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.head);
+        q[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.quants);
+        if (FMT == kMmaQ5K) qh[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.fifth);
     }
     int32_t tab[NAL];
 #pragma unroll
@@ -130,7 +144,8 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
     }
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        const u32x4 lo = q[m] & 0x0f0f0f0fU, hi = (q[m] >> 4) & 0x0f0f0f0fU;
+        u32x4 lo = q[m] & 0x0f0f0f0fU, hi = (q[m] >> 4) & 0x0f0f0f0fU;
+        if (FMT == kMmaQ5K) { lo |= mma_fifth(qh[m], 2 * P); hi |= mma_fifth(qh[m], 2 * P + 1); }
         const i32x16 zero = {0};
         const i32x16 dot_even = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_even), __builtin_bit_cast(i32x4, lo), zero, 0, 0, 0);
         const i32x16 dot_odd = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_odd), __builtin_bit_cast(i32x4, hi), zero, 0, 0, 0);
@@ -163,19 +178,19 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
 // half's slots zeroed - accumulate into one result, whose register v holds activation row v's dot with sub-block 2p in the lanes of half 0
 // and with sub-block 2p + 1 in those of half 1. A lane then decodes one scale and one minimum instead of two, and the terms of two
 // activation rows meet through one exchange of the halves: x[2p] + x[2p + 1] of row 2v + h lands where the wide form leaves it.
-// (4 activation rows, gate and up: 140 -> 115 vector instructions a stage; dense 27648 x 5120, 4 rows 76.1 -> 75.0 us, Q8_0 down, 120 rows in
-// items of four 237 -> 234 us. With 8 activation rows, as many conversions and two products in a row, it is the slower one: 100 rows of
+// (4 activation rows, gate and up: 140 -> 115 vector instructions a stage; dense 27648 x 5120, 4 rows 76.1 -> 75.0 us. With 8 activation rows, as many conversions and two products in a row, it is the slower one: 100 rows of
 // hidden 2048 / ffn 768 / 128 experts 162.0 against 160.2 us, 90 rows of hidden 4096 / ffn 1536 / 64 experts 326 against 321.)
-template <int NAL, int NM, bool HIGH>
-__device__ __forceinline__ void mma_stage_terms_halves(const lds_u8* slot, const MmaLane& o, float (&term)[NM][NAL]) {
+template <int FMT, int NAL, int NM, bool HIGH>
+__device__ __forceinline__ void mma_stage_terms_halves(const lds_u8* slot, const MmaLane& o, uint32_t p, float (&term)[NM][NAL]) {
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) int32_t lds_i32;
     const u32x4 codes = *(lds_u32x4*)(slot + o.even);
-    u32x4 hd[NM], q[NM];
+    u32x4 hd[NM], q[NM], qh[NM];
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        hd[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.head);
-        q[m] = *(lds_u32x4*)(slot + kMmaWeightBytes * m + o.quants);
+        hd[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.head);
+        q[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.quants);
+        if (FMT == kMmaQ5K) qh[m] = *(lds_u32x4*)(slot + mma_weight_bytes<FMT>() * m + o.fifth);
     }
     float e[2 * NAL], f[2 * NAL];
 #pragma unroll
@@ -186,7 +201,8 @@ __device__ __forceinline__ void mma_stage_terms_halves(const lds_u8* slot, const
     const u32x4 a_even = codes & o.even_slot, a_odd = codes & ~o.even_slot;
 #pragma unroll
     for (int m = 0; m < NM; ++m) {
-        const u32x4 lo = q[m] & 0x0f0f0f0fU, hi = (q[m] >> 4) & 0x0f0f0f0fU;
+        u32x4 lo = q[m] & 0x0f0f0f0fU, hi = (q[m] >> 4) & 0x0f0f0f0fU;
+        if (FMT == kMmaQ5K) { lo |= mma_fifth(qh[m], 2U * p); hi |= mma_fifth(qh[m], 2U * p + 1U); }
         const i32x16 zero = {0};
         i32x16 dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_even), __builtin_bit_cast(i32x4, lo), zero, 0, 0, 0);
         dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a_odd), __builtin_bit_cast(i32x4, hi), dot, 0, 0, 0);
@@ -210,6 +226,116 @@ __device__ __forceinline__ void mma_stage_terms_halves(const lds_u8* slot, const
 }
 template <int NAL> constexpr bool mma_halves() { return NAL == 2; }
 
+// N words of LDS from a 2-byte aligned place
+template <int N> __device__ __forceinline__ void mma_words(const lds_u8* at, uint32_t (&out)[N]) {
+    typedef const __attribute__((address_space(3))) uint32_t lds_word;
+    const uint32_t address = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(at)), shift = address & 3U;
+    lds_word* const aligned = (lds_word*)(uintptr_t)(address & ~3U);
+    uint32_t raw[N + 1];
+#pragma unroll
+    for (int i = 0; i <= N; ++i) raw[i] = aligned[i];           // (the word behind an aligned run lies inside the slot: read, unused)
+#pragma unroll
+    for (int i = 0; i < N; ++i) out[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], shift);
+}
+
+// One landed stage of down rows in the other formats of the reference (256 weights of every row), added to the wavefront's accumulators.
+// Same products and result layout as above.
+//   Q8_0, Q5_1: wavefront p is chain p, which owns groups p and p + 4 of the stage, each added by itself (down_groups.hpp):
+//     first = d * float(dot); Q5_1: combined = first + m * float(code sum); chain += delta * combined.
+//   Q6_K: wavefront p is pair p (groups 2p, 2p + 1; q6k_quads.hpp): integer = s0 * dot(first 16) + s1 * dot(last 16),
+//     term = delta * (d * float(integer)), acc += term_2p + term_(2p+1). One product of K = 32 gives both dots: result register 2v + s of a
+//     lane belongs to activation row 2v + h and the group's half s, because slot i carries the codes of its half of K only (zeros in the
+//     other) - so 16 activation rows at most.
+// stage: of the row; where in its piece a Q6_K row's block starts (two bytes further every super-block: 210 = 13 * 16 + 2).
+template <int FMT, int NAL>
+__device__ __forceinline__ void mma_stage_other(const lds_u8* slot, const MmaLane& o, uint32_t p, uint32_t stage, float (&acc)[NAL]) {
+    typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+    typedef const __attribute__((address_space(3))) int32_t lds_i32;
+    typedef const __attribute__((address_space(3))) uint16_t lds_u16;
+    static_assert(NAL <= 8, "sixteen result registers");
+    u32x4 a0 = *(lds_u32x4*)(slot + o.even), a1 = *(lds_u32x4*)(slot + o.odd);
+    int32_t tab[NAL];
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) tab[v] = *(lds_i32*)(slot + o.table + 128U * v);
+    if (FMT == kMmaQ51 && o.sum_lane) {
+#pragma unroll
+        for (int v = 0; v < NAL; ++v) tab[v] = __builtin_bit_cast(int32_t, static_cast<float>(tab[v]));
+    }
+    uint32_t q0[4], q1[4];
+    float d0, d1 = 0.0F, m0 = 0.0F, m1 = 0.0F;
+    int s[2][2] = {{0, 0}, {0, 0}};
+    if constexpr (FMT == kMmaQ80) {
+        const lds_u8* const b0 = slot + o.quants;
+        mma_words<4>(b0 + o.fifth, q0);
+        mma_words<4>(b0 + 136U + o.fifth, q1);
+        d0 = half_bits_to_float(*(lds_u16*)b0);
+        d1 = half_bits_to_float(*(lds_u16*)(b0 + 136U));
+    } else if constexpr (FMT == kMmaQ51) {
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        typedef const __attribute__((address_space(3))) u32x2 lds_u32x2;
+        const lds_u8* const b0 = slot + o.quants;
+        uint32_t fifth[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const u32x2 head = *(lds_u32x2*)(b0 + 96 * k), n0 = *(lds_u32x2*)(b0 + 96 * k + 8), n1 = *(lds_u32x2*)(b0 + 96 * k + 16);
+            uint32_t (&q)[4] = k ? q1 : q0;
+            const uint32_t n[4] = {n0.x, n0.y, n1.x, n1.y};
+            fifth[k] = head.y >> (4U * o.shift);                     // o.shift: 4 in half 1 (weights 16 .. 31: high nibbles, bits 16 ..)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                q[i] = ((n[i] >> o.shift) & 0x0f0f0f0fU) | ((((fifth[k] >> (4 * i)) & 15U) * 0x00204081U & 0x01010101U) << 4);
+            (k ? d1 : d0) = half_bits_to_float(head.x & 0xffffU);
+            (k ? m1 : m0) = half_bits_to_float(head.x >> 16);
+        }
+    } else {
+        const lds_u8* const block = slot + o.head + ((o.start + 2U * stage) & 15U);
+        uint32_t qh[4], t[1];
+        mma_words<4>(block + o.quants, q0);
+        mma_words<4>(block + o.quants + 32U, q1);
+        mma_words<4>(block + o.fifth, qh);
+        mma_words<1>(block + 192U + 4U * p, t);
+        d0 = half_bits_to_float(*(lds_u16*)(block + 208U)) * 0.25F;
+        // four times the weight, ((nibble | pair << 4) - 32) << 2, is the six bits at the top of the byte with the highest one flipped; the
+        // factor leaves with d (exact: a power of two)
+        const uint32_t nibbles = p & 1U ? 2U : 30U, pairs = p & 1U ? 30U : 26U;             // rotations to the right
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t n0 = __builtin_amdgcn_alignbit(q0[i], q0[i], nibbles), n1 = __builtin_amdgcn_alignbit(q1[i], q1[i], nibbles);
+            const uint32_t h0 = __builtin_amdgcn_alignbit(qh[i], qh[i], pairs), h1 = __builtin_amdgcn_alignbit(qh[i], qh[i], pairs + 2U);
+            q0[i] = ((n0 & 0x3c3c3c3cU) | (h0 & 0xc0c0c0c0U)) ^ 0x80808080U;
+            q1[i] = ((n1 & 0x3c3c3c3cU) | (h1 & 0xc0c0c0c0U)) ^ 0x80808080U;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i >> 1][i & 1] = static_cast<int8_t>(t[0] >> (8 * i));
+        a0 = a0 & o.even_slot;
+        a1 = a1 & o.even_slot;
+    }
+    const u32x4 w0 = {q0[0], q0[1], q0[2], q0[3]}, w1 = {q1[0], q1[1], q1[2], q1[3]};
+    const i32x16 zero = {0};
+    const i32x16 dot0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a0), __builtin_bit_cast(i32x4, w0), zero, 0, 0, 0);
+    const i32x16 dot1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a1), __builtin_bit_cast(i32x4, w1), zero, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) {
+        const float e0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x00, 0xF, 0xF, true));
+        const float e1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x55, 0xF, 0xF, true));
+        if constexpr (FMT == kMmaQ6K) {
+            const int i0 = __mul24(s[0][0], dot0[2 * v]) + __mul24(s[0][1], dot0[2 * v + 1]);
+            const int i1 = __mul24(s[1][0], dot1[2 * v]) + __mul24(s[1][1], dot1[2 * v + 1]);
+            const float t0 = e0 * (d0 * static_cast<float>(i0)), t1 = e1 * (d0 * static_cast<float>(i1));
+            acc[v] = acc[v] + (t0 + t1);
+        } else {
+            float c0 = d0 * static_cast<float>(dot0[v]), c1 = d1 * static_cast<float>(dot1[v]);
+            if constexpr (FMT == kMmaQ51) {
+                const float f0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0xAA, 0xF, 0xF, true));
+                const float f1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0xFF, 0xF, 0xF, true));
+                c0 = c0 + (m0 * f0);
+                c1 = c1 + (m1 * f1);
+            }
+            acc[v] = acc[v] + (e0 * c0);
+            acc[v] = acc[v] + (e1 * c1);
+        }
+    }
+}
 // The activation rows of a run and where their results go, resolved once by one wavefront: addresses of the A8 image of row a (codes,
 // deltas, sums), OUT more addresses for the emitter, and the row's assignment.
 template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OUT) * mma_acts<NAL>(); }
@@ -228,16 +354,19 @@ template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OU
 // kept by team 0, which adds the terms of every super-block in ascending order: its own from registers, the other teams'
 // from an LDS exchange buffer, one stage group behind (the group's barrier publishes them).
 // Every wavefront of the workgroup calls this; ring, row table and `red` are free again when it returns.
-template <int NAL, int DEPTH, int TEAMS, int NM, class Rows, class Emit>
+template <int FMT, int NAL, int DEPTH, int TEAMS, int NM, class Rows, class Emit>
 __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* red, const uint8_t* const (&wrows)[NM], size_t row_stride, uint32_t stages,
                                         uint32_t tiles, uint32_t nacts, Rows rows, Emit emit) {
-    constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<NAL, NM>(), SLOT = mma_slot_bytes<NAL, NM>();
+    constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<FMT, NAL, NM>(), SLOT = mma_slot_bytes<FMT, NAL, NM>();
+    constexpr uint32_t CW = mma_weight_copies<FMT>(), PIECES = mma_pieces<FMT>(), PITCH = mma_pitch<FMT>(), BYTES = mma_block_bytes<FMT>();
     // Every wavefront issues PERW copies a stage, some of them for no lane (the rest of the last four; the ones that the first stage starts
     // early or late): no branches on the wavefront's number, one count to wait for.
-    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = 5U * NM;
+    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = CW * NM;
     constexpr uint32_t XTEAM = 4U * NAL * 64U;                                                  // floats one team exchanges per group
     static_assert(DEPTH >= 2 && DEPTH <= 4, "ring depth");
-    static_assert(TEAMS == 1 || (NM == 1 && NAL <= 8), "stage teams serve one matrix, every result register");
+    static_assert(TEAMS == 1 || (NM == 1 && NAL <= 8 && FMT == kMmaQ4K), "stage teams serve one matrix, every result register");
+    static_assert(NM == 1 || FMT == kMmaQ4K || FMT == kMmaQ5K, "gate and up rows");
+    static_assert(CW >= 4U && PIECES >= 8U, "copies 0 .. 3 are of whole waves");
     const uint32_t lane = threadIdx.x & 63U, j = lane & 31U, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = wave & 3U, team = wave >> 2;
     const uint32_t groups = (stages + TEAMS - 1U) / TEAMS;                                     // of a tile
@@ -245,33 +374,36 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     const uint32_t total = TEAMS == 1 ? groups * tiles : groups, my_total = TEAMS == 1 ? total : my_groups;
     const uint32_t nv = (nacts + 1U) / 2U;
 
-    // ---- this wavefront's copies of a stage, copy c = 4k + p: five per matrix (9 pieces of 16 bytes a row, rows back to back; the
-    // fifth moves the last half kilobyte), codes (16 pieces per row, piece t at position (t + a) % 16), table (per row [8 deltas][8 sums])
+    // ---- this wavefront's copies of a stage, copy c = 4k + p: CW per matrix (the pieces of 16 bytes of a row, rows PITCH apart; the
+    // last moves half a kilobyte), codes (16 pieces per row, piece t at position (t + a) % 16), table (per row [8 deltas][8 sums])
     const uint8_t* src[PERW];
-    uint32_t step[PERW], lands[PERW];
+    uint32_t step[PERW], lands[PERW], piece_at[PERW];
     uint64_t lanes[PERW];
 #pragma unroll
     for (uint32_t k = 0; k < PERW; ++k) {
         const uint32_t c = 4U * k + p;
         if (c < WEIGHTS) {
-            const uint32_t m = c / 5U, i = c - 5U * m, s = 64U * i + lane < kMmaRows * 9U ? 64U * i + lane : 0U, r = s / 9U, piece = s - 9U * r;
-            src[k] = wrows[m < NM ? m : 0] + static_cast<size_t>(r) * row_stride + 16U * piece + 144U * team;
-            step[k] = 144U * TEAMS;
-            lands[k] = kMmaWeightBytes * m + 1024U * i;
-            lanes[k] = i == 4U ? 0xffffffffULL : ~0ULL;
+            const uint32_t m = c / CW, i = c - CW * m, s = 64U * i + lane < kMmaRows * PITCH ? 64U * i + lane : 0U, r = s / PITCH;
+            const uint32_t piece = s - PITCH * r < PIECES ? s - PITCH * r : PIECES - 1U;
+            src[k] = wrows[m < NM ? m : 0] + static_cast<size_t>(r) * row_stride + BYTES * team;
+            if (FMT == kMmaQ6K) piece_at[k] = 16U * piece;           // (from the piece that the row's block starts in, found when it is copied)
+            else src[k] += 16U * piece;
+            step[k] = BYTES * TEAMS;
+            lands[k] = mma_weight_bytes<FMT>() * m + 1024U * i;
+            lanes[k] = i == CW - 1U ? 0xffffffffULL : ~0ULL;
         } else if (c < WEIGHTS + CC) {
             src[k] = nullptr;
             step[k] = 256U * TEAMS;
-            lands[k] = mma_codes_at<NAL, NM>() + 1024U * (c - WEIGHTS);
+            lands[k] = mma_codes_at<FMT, NM>() + 1024U * (c - WEIGHTS);
             lanes[k] = ~0ULL;
         } else {
             src[k] = nullptr;
             step[k] = 32U * TEAMS;
-            lands[k] = mma_table_at<NAL, NM>() + 1024U * (c - WEIGHTS - CC);
+            lands[k] = mma_table_at<FMT, NAL, NM>() + 1024U * (c - WEIGHTS - CC);
             lanes[k] = c >= TOTAL ? 0ULL : ACTS >= 16U ? ~0ULL : (1ULL << (4U * ACTS)) - 1ULL;
         }
     }
-    const size_t next_tile = kMmaRows * row_stride - 144U * static_cast<size_t>(stages);       // from a tile's end to the next one's start
+    const size_t next_tile = kMmaRows * row_stride - BYTES * static_cast<size_t>(stages);       // from a tile's end to the next one's start
     uint32_t issued = 0, issue_stage = 0;
     // copies of the next stage into a slot; PART 1: the weights (of the run's first stages, whose activation rows are not known yet), 2: the rest
     const auto start = [&](auto part_constant, lds_u8* slot) __attribute__((always_inline)) {
@@ -279,8 +411,10 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
             const bool mine = part == 0 || (4U * k + p < WEIGHTS) == (part == 1);
-            if (part == 0 && k == 0U) mma_copy16(src[k], slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
-            else mma_copy16_lanes(src[k], slot + lands[k], mine ? lanes[k] : 0ULL);
+            const uint8_t* from = src[k];
+            if (FMT == kMmaQ6K && 4U * k + p < WEIGHTS) from = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(from) & ~static_cast<uintptr_t>(15)) + piece_at[k];
+            if (part == 0 && k == 0U) mma_copy16(from, slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
+            else mma_copy16_lanes(from, slot + lands[k], mine ? lanes[k] : 0ULL);
             src[k] += mine ? step[k] : 0U;
         }
         if (TEAMS == 1 && ++issue_stage == stages) {
@@ -331,18 +465,38 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
 
     MmaLane o;
     {
-        const uint32_t ai = mma_slot_act<NAL>(j), c_base = mma_codes_at<NAL, NM>() + 256U * ai;
-        o.head = 144U * j;
-        o.quants = 144U * j + 16U + 32U * p + 16U * h;
-        o.even = c_base + 16U * ((4U * p + h + ai) & 15U);
-        o.odd = c_base + 16U * ((4U * p + 2U + h + ai) & 15U);
-        // quad lane 0, 1: delta of sub-block 2p, 2p + 1; quad lane 2, 3: their code sums
-        o.table = mma_table_at<NAL, NM>() + 64U * h + 4U * (2U * p + (lane & 1U) + 4U * (lane & 2U));
+        const uint32_t ai = mma_slot_act<NAL>(j), c_base = mma_codes_at<FMT, NM>() + 256U * ai;
+        o.head = 16U * PITCH * j;
+        if (FMT == kMmaQ4K || FMT == kMmaQ5K) {
+            o.fifth = 16U * PITCH * j + 16U + 16U * h;
+            o.quants = 16U * PITCH * j + (FMT == kMmaQ5K ? 48U : 16U) + 32U * p + 16U * h;
+        } else if (FMT == kMmaQ6K) {                              // from the block's first byte: nibbles, bit pairs
+            o.quants = 64U * (p >> 1) + 16U * h;
+            o.fifth = 128U + 32U * (p >> 1) + 16U * h;
+            o.start = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wrows[0]) + j * row_stride) & 15U;
+        } else {                                                  // chain p: block p of the stage, codes 16 h ..
+            o.quants = 16U * PITCH * j + (FMT == kMmaQ80 ? 34U : 24U) * p;
+            o.fifth = 2U + 16U * h;
+            o.shift = 4U * h;
+        }
+        // the lane's activation slot: groups 2p and 2p + 1, of chain p groups p and p + 4 (16-byte pieces 2 g + h of its row)
+        constexpr bool CHAINS = FMT == kMmaQ80 || FMT == kMmaQ51;
+        const uint32_t g0 = CHAINS ? p : 2U * p, g1 = CHAINS ? p + 4U : 2U * p + 1U;
+        o.even = c_base + 16U * ((2U * g0 + h + ai) & 15U);
+        o.odd = c_base + 16U * ((2U * g1 + h + ai) & 15U);
+        if (FMT == kMmaQ6K) {                                     // result register 2v + s: activation row 2v + h, half s of the group
+            const uint32_t reg = 4U * (j >> 3) + (j & 3U), act = ((reg & ~1U) + ((j >> 2) & 1U)) & (ACTS - 1U), base = mma_codes_at<FMT, NM>() + 256U * act;
+            o.even = base + 16U * ((2U * g0 + h + act) & 15U);
+            o.odd = base + 16U * ((2U * g1 + h + act) & 15U);
+            o.even_slot = (reg & 1U) == h ? ~0U : 0U;
+        }
+        // quad lane 0, 1: the deltas of g0, g1; quad lane 2, 3: their code sums
+        o.table = mma_table_at<FMT, NAL, NM>() + 64U * h + 4U * ((lane & 1U ? g1 : g0) + 4U * (lane & 2U));
         o.sum_lane = (lane & 2U) != 0;
-        if constexpr (mma_halves<NAL>()) {
+        if constexpr (mma_halves<NAL>() && (FMT == kMmaQ4K || FMT == kMmaQ5K)) {
             const uint32_t odd = (j >> 2) & 1U, act = (4U * (j >> 3) + (j & 3U)) & (ACTS - 1U);
-            o.even = mma_codes_at<NAL, NM>() + 256U * act + 16U * ((4U * p + 2U * odd + h + act) & 15U);
-            o.table = mma_table_at<NAL, NM>() + 4U * (2U * p + h);
+            o.even = mma_codes_at<FMT, NM>() + 256U * act + 16U * ((4U * p + 2U * odd + h + act) & 15U);
+            o.table = mma_table_at<FMT, NAL, NM>() + 4U * (2U * p + h);
             o.shift = 16U * (p & 1U) + 8U * h;
             o.even_slot = odd ? 0U : ~0U;
         }
@@ -420,16 +574,18 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         if (g < my_total) {
             const lds_u8* slot = ring + SLOT * (compute_slot * TEAMS + team);
             float term[NM][NAL];
-            if constexpr (mma_halves<NAL>()) {
-                if (p < 2U) mma_stage_terms_halves<NAL, NM, false>(slot, o, term);
-                else mma_stage_terms_halves<NAL, NM, true>(slot, o, term);
+            if constexpr (FMT != kMmaQ4K && FMT != kMmaQ5K) mma_stage_other<FMT, NAL>(slot, o, p, stage, acc[0]);
+            else if constexpr (mma_halves<NAL>()) {
+                if (p < 2U) mma_stage_terms_halves<FMT, NAL, NM, false>(slot, o, p, term);
+                else mma_stage_terms_halves<FMT, NAL, NM, true>(slot, o, p, term);
             } else switch (p) {
-            case 0: mma_stage_terms<NAL, NM, 0>(slot, o, nv, term); break;
-            case 1: mma_stage_terms<NAL, NM, 1>(slot, o, nv, term); break;
-            case 2: mma_stage_terms<NAL, NM, 2>(slot, o, nv, term); break;
-            default: mma_stage_terms<NAL, NM, 3>(slot, o, nv, term); break;
+            case 0: mma_stage_terms<FMT, NAL, NM, 0>(slot, o, nv, term); break;
+            case 1: mma_stage_terms<FMT, NAL, NM, 1>(slot, o, nv, term); break;
+            case 2: mma_stage_terms<FMT, NAL, NM, 2>(slot, o, nv, term); break;
+            default: mma_stage_terms<FMT, NAL, NM, 3>(slot, o, nv, term); break;
             }
-            if (TEAMS == 1) {
+            if (FMT != kMmaQ4K && FMT != kMmaQ5K) {
+            } else if (TEAMS == 1) {
 #pragma unroll
                 for (int m = 0; m < NM; ++m)
 #pragma unroll

@@ -69,10 +69,10 @@ template <class P> __device__ __forceinline__ uint64_t address(const P* p) { ret
 
 // Waves per SIMD: what the LDS of a workgroup allows (four of 36 KB, three of 44 or 46 KB, two of 73 KB), which for 16 rows the compiler misses
 // by a few registers when it is not told (200 rows of hidden 2048 / ffn 768 / 128 experts: 192.8 -> 172.3 us a layer, 219.6 before the run).
-template <int NAL, int DEPTH, bool DIRECT>
+template <int FMT, int NAL, int DEPTH, bool DIRECT>
 __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_project_kernel(MmaArgs k) {
     constexpr uint32_t ACTS = mma_acts<NAL>();
-    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<NAL, 2, DEPTH, 1>()];
+    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, 2, DEPTH, 1>()];
     __shared__ float red_mem[mma_reduce_floats<NAL, 2>()];
     __shared__ uint64_t at_mem[mma_row_words<NAL, 3>()];
     __shared__ uint32_t slot_mem[ACTS];
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
             at[5U * ACTS + a] = address(r.h_sums_of(i));
         };
         const MmaRowsOf<DIRECT, decltype(put)> rows{c0, k.r.in, k.l.dense_rows, at, slot, put};
-        mma_run<NAL, DEPTH, 1, 2>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, n, rows,
+        mma_run<FMT, NAL, DEPTH, 1, 2>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, n, rows,
                                   [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[2]) {
             const uint32_t j = lane & 31U, h = lane >> 5;
             const MmaArgs& args = mma_args();
@@ -142,10 +142,10 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
 // GATE_UP: the same sweep over gate (blockIdx.z = 0) or up (1) rows against the input image, raw values out to the gate / up
 // intermediates - the dense FFN's projection when that workspace exists (two launches' worth of narrow workgroups fill the
 // compute units better than the fused form's wide ones: 27648 x 5120, 8 rows: 54 + 5 us against 70 us).
-template <int NAL, int DEPTH, int TEAMS, bool DIRECT, bool GATE_UP = false>
+template <int FMT, int NAL, int DEPTH, int TEAMS, bool DIRECT, bool GATE_UP = false>
 __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
     constexpr uint32_t ACTS = mma_acts<NAL>();
-    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<NAL, 1, DEPTH, TEAMS>()];
+    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, 1, DEPTH, TEAMS>()];
     __shared__ float xbuf_mem[mma_exchange_floats<NAL, TEAMS>()];
     __shared__ float red_mem[mma_reduce_floats<NAL, 1>()];
     __shared__ uint64_t at_mem[mma_row_words<NAL, 1>()];
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
             at[3U * ACTS + a] = GATE_UP ? address(r.inter_of(blockIdx.z ? r.up_out : r.gate_out, i)) : address(r.rawdots_of(i, args.w.hidden));
         };
         const MmaRowsOf<DIRECT, decltype(put)> rows{c0, GATE_UP ? k.r.in : k.r.h, k.l.dense_rows, at, slot, put};
-        mma_run<NAL, DEPTH, TEAMS, 1>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride, (GATE_UP ? k.w.hidden : k.w.ffn) / 256U,
+        mma_run<FMT, NAL, DEPTH, TEAMS, 1>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride, (GATE_UP ? k.w.hidden : k.w.ffn) / 256U,
                                       tiles, n, rows, [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[1]) {
             const uint32_t a = 2U * v + (lane >> 5), at_out = (tile0 + tile) * kMmaRows + (lane & 31U);
             if (a >= n) return;

@@ -204,7 +204,6 @@ __device__ __forceinline__ WorkItem work_item(const mi355_moe_weights& w, const 
     return {e, index, e < w.experts ? index + 1U : index, index + 1U};      // an invalid route has no item (its row is flagged)
 }
 __device__ __forceinline__ uint32_t ordered(const RowsK& r, uint32_t order_at, uint32_t i) {
-    if (r.union_plan) return union_assignment(r.union_plan, i);
     return r.plan ? r.plan[order_at + i] : i;
 }
 

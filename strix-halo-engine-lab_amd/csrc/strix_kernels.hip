@@ -1668,7 +1668,7 @@ inline bool mma_dense(const mi355_moe_weights& w, const RowsK& r, uint32_t rows)
 // A decode batch whose expert's gate + up rows are several MB: one expert is swept once for the rows that chose it.
 inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows);
 inline bool large_expert(const mi355_moe_weights& w) { return 2ULL * w.ffn * (w.hidden / 256U) * kQ4kBlock >= (4ULL << 20); }
-// Routed experts with Q4_K gate / up rows, past the decode sizes or over large experts: the plan cuts an expert's rows into items of this
+// Routed experts past the decode sizes or of several MB: the plan cuts an expert's rows into items of this
 // many for the matrix-core sweeps (0: the vector-ALU sweeps serve the batch). The sweeps are bound by latency, so the narrow instances
 // (4 or 8 rows: 128 or 151 registers, four or three waves per SIMD) win while an expert holds few rows, and even one row per expert is
 // better off here than on the vector-ALU sweep. Layer times, hidden 2048 / ffn 768 / 128 experts top-8, items of 4 rows | of 16 in sweeps of 8 |
@@ -1676,17 +1676,20 @@ inline bool large_expert(const mi355_moe_weights& w) { return 2ULL * w.ffn * (w.
 // rows 118 | 126 | 167 (147), 60 rows 141 | 139 | 181 (171), 100 rows 177 | 163 | 189, 200 rows 266 | 220 | 218, 400 rows 445 | 340 | 337; hidden
 // 4096 / ffn 1536 / 64 experts: 24 rows 200 | 204 | 282 (260), 60 rows 300 | 267 | 288, 150 rows 550 | 439 | 414. A decode batch over large
 // experts keeps its items of two rows: one rank's half of hidden 6144 / ffn 2560 / 160 experts, 7, 10, 16 rows: 189, 231, 306 us against 199,
-// 251, 320. Down rows of another format run on their own sweeps of four rows, so items stay at four there (hidden 2048 / ffn 768 / 128
-// experts, Q6_K down, 30, 100, 300, 1000 rows: 117, 193, 394, 1101 us against 141, 234, 484, 1374; Q8_0 down 130, 217, 441, 1203 against 157, 259,
-// 532, 1474).
+// 251, 320; 10 rows of hidden 4096 / ffn 1536 / 64 experts, Q6_K | Q8_0 | Q5_K and Q5_1 rows: 271 | 271 | 258 -> 221 | 222 | 224 us.
+// The other formats' batches, on their vector-ALU sweeps (items of four) before: hidden 2048 / ffn 768 / 128 experts, Q6_K down, 40, 300, 1000 rows
+// 130, 395, 1105 -> 122, 258, 600 us; Q8_0 down 148, 440, 1203 -> 124, 245, 560; Q5_K gate / up and Q5_1 down 196, 774, 2310 -> 127, 264, 619.
 // Items of up to four 32-row sweeps: the later sweeps of a tile's weights hit the cache, and an expert with thousands of rows
 // still spreads over many workgroups.
 constexpr uint32_t kMmaItemRows = 128;
+inline bool q4k_both(const mi355_moe_weights& w) { return w.gate_type == MI355_TYPE_Q4_K && w.down_type == MI355_TYPE_Q4_K; }
+// down rows of whole stages of 256 weights (Q8_0 and Q5_1 rows may end on half a stage)
+inline bool mma_down_rows(const mi355_moe_weights& w) { return w.ffn % 256U == 0 && w.down_type != MI355_TYPE_Q5_K; }
 inline uint32_t mma_grouped_split(const mi355_moe_weights& w, uint32_t rows) {
-    if (w.gate_type != MI355_TYPE_Q4_K || w.experts == 1U) return 0U;
-    if (rows <= kFusedMaxRows) return w.down_type == MI355_TYPE_Q4_K && !quad_sweep(w, rows) && large_expert(w) ? 2U : 0U;
+    if ((w.gate_type != MI355_TYPE_Q4_K && w.gate_type != MI355_TYPE_Q5_K) || w.experts == 1U) return 0U;
+    if (rows <= kFusedMaxRows) return !quad_sweep(w, rows) && large_expert(w) ? 2U : 0U;
     const uint64_t assignments = static_cast<uint64_t>(rows) * w.top_k;
-    if (w.down_type != MI355_TYPE_Q4_K || assignments < 4ULL * w.experts) return 4U;
+    if (!mma_down_rows(w) || assignments < 4ULL * w.experts) return 4U;
     return assignments < 16ULL * w.experts ? 16U : kMmaItemRows;
 }
 // rows of one sweep over such an item
@@ -1715,8 +1718,12 @@ constexpr uint32_t kQuadMaxItems = 48;
 inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows) {
     return rows <= kFusedMaxRows && rows * w.top_k <= kQuadMaxItems && w.experts > 1U;
 }
-// grouped: the plan's items hold several assignments (the one-assignment sweeps do not apply)
+// grouped: the fused router's plan of a decode batch with always-on experts, whose items hold up to four assignments; the narrow matrix-core
+// sweeps serve it whatever its size (hidden 2048 / ffn 768 / 128 experts top-8 and one more, 5 rows, Q6_K | Q8_0 | Q4_K down: 88 | 93 | 86 -> 70 |
+// 71 | 65 us; 1 row 53 | 54 | 52 -> 50 | 50 | 49; Q5_K gate / up and Q5_1 down 83 -> 77, 1 row 50 -> 51).
 inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t umax, hipStream_t st, bool grouped = false) {
+    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && (grouped || split))
+        return launch_mma_project(w, r, rows, 0, umax, grouped ? 4U : mma_sweep_rows(w, rows, split), st);
     if (w.gate_type == MI355_TYPE_Q5_K) {
         // the deepest ring at which every workgroup of the launch is resident (4 waves x DEPTH x 4 KB each)
         const uint64_t groups = static_cast<uint64_t>(w.ffn / 32U) * umax;
@@ -1724,7 +1731,7 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
         else project_q5k_kernel<2><<<dim3(w.ffn / 32U, umax), 256, 0, st>>>(w, r, rows * w.top_k);
         return;
     }
-    if (!grouped && quad_sweep(w, rows)) {
+    if (quad_sweep(w, rows)) {
         const uint32_t items = rows * w.top_k;
         if (items <= 16U) project_quad_kernel<4><<<dim3(w.ffn / 32U, items), 256, 0, st>>>(w, r, items);
         else project_quad_kernel<2><<<dim3(w.ffn / 32U, items), 256, 0, st>>>(w, r, items);
@@ -1734,7 +1741,6 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
         if (rows > 4U && rows <= 16U && r.gate_out && r.up_out && dense_rows(r, w)) return launch_mma_gate_up(w, r, rows, st);
         return launch_mma_project(w, r, rows, rows, 0, rows, st);
     }
-    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) return launch_mma_project(w, r, rows, 0, umax, mma_sweep_rows(w, rows, split), st);
     if (dense_pairs_ok(w, rows) && dense_rows(r, w) && r.gate_out && r.up_out) return launch_project_dense(w, r, rows, st);
     const dim3 grid(w.ffn / 32U, umax);
     if (w.experts == 1U && rows > 4U) launch_project_nb<8>(w, r, rows, grid, st);
@@ -1742,6 +1748,12 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
 }
 // Returns true when the launch also published the output rows (a dense top-1 job with r.top1_form set: the two dense sweeps).
 inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t umax, hipStream_t st, bool grouped = false) {
+    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && mma_down_rows(w) && (grouped || split)) {
+        RowsK plain = r;
+        plain.top1_form = 0;
+        launch_mma_down(w, plain, rows, 0, umax, grouped ? 4U : mma_sweep_rows(w, rows, split), st);
+        return false;
+    }
     if (w.down_type != MI355_TYPE_Q4_K) {      // Q8_0 / Q5_1 (blocks of 32, four chains per row) and Q6_K (pairs per super-block)
         const uint32_t assignments = rows * w.top_k, items_at = plan_items_at(w.experts, assignments), order_at = plan_order_at(w.experts);
         const dim3 grid(w.hidden / kDownGroupsRows, umax);
@@ -1755,16 +1767,13 @@ inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t row
         else launch_down_q6k(w, r, grid, assignments, items_at, order_at, st);
         return false;
     }
-    if (!grouped && quad_sweep(w, rows)) {
+    if (quad_sweep(w, rows)) {
         const uint32_t items = rows * w.top_k;
         if (items <= 16U) down_quad_kernel<4><<<dim3(w.hidden / 64U, items), 256, 0, st>>>(w, r, items);
         else down_quad_kernel<2><<<dim3(w.hidden / 64U, items), 256, 0, st>>>(w, r, items);
         return false;
     }
     if (mma_dense(w, r, rows)) { launch_mma_down(w, r, rows, rows, 0, rows, st); return r.top1_form != 0; }
-    RowsK plain = r;
-    plain.top1_form = 0;
-    if (const uint32_t split = mma_grouped_split(w, rows); split && r.plan) { launch_mma_down(w, plain, rows, 0, umax, mma_sweep_rows(w, rows, split), st); return false; }
     if (dense_pairs_ok(w, rows) && dense_rows(r, w)) { launch_down_dense(w, r, rows, st); return r.top1_form != 0; }
     const dim3 grid(w.hidden / 64U, umax);
     if (w.experts == 1U && rows > 4U) launch_down_nb<8>(w, r, rows, grid, st);
@@ -1786,6 +1795,11 @@ inline uint32_t plan_split(const mi355_moe_weights& w, uint32_t rows) {
 }
 inline uint32_t item_bound(const mi355_moe_weights& w, uint32_t rows) {
     return plan_item_bound(w.experts, rows * w.top_k, plan_split(w, rows));
+}
+// Items by which a batch is admitted: of other formats than Q4_K those of four rows, however wide the batch's own are.
+inline uint32_t admitted_items(const mi355_moe_weights& w, uint32_t rows) {
+    const uint32_t split = plan_split(w, rows);
+    return plan_item_bound(w.experts, rows * w.top_k, w.experts == 1U || q4k_both(w) || split < 4U ? split : 4U);
 }
 
 // ======================================================================================================== admission
@@ -1823,7 +1837,7 @@ int32_t check_moe(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t 
     // rows are one grid dimension of the prologue and of the merge: every entry refuses a larger batch before its first launch
     STRIX_REQUIRE(rows <= 65535U, "moe: at most 65535 rows per call");
     // plan items are one grid dimension of the expert launches
-    STRIX_REQUIRE(cls != kIntegerClass || item_bound(*w, rows) <= 65535U, "moe: too many work items for one call (experts + rows * top_k / 4 must stay below 65536)");
+    STRIX_REQUIRE(cls != kIntegerClass || admitted_items(*w, rows) <= 65535U, "moe: too many work items for one call (experts + rows * top_k / 4 must stay below 65536)");
     wv = *w;
     if (wv.gate_row_stride == 0) wv.gate_row_stride = moe_row_bytes(w->gate_type, w->hidden);
     if (wv.gate_expert_stride == 0) wv.gate_expert_stride = wv.gate_row_stride * w->ffn;
