@@ -1,4 +1,4 @@
-// The matrix-core prefill of the routed experts: kernels of prefill_f16.hpp and prefill_reg.hpp, and the choice between them.
+// The matrix-core prefill of the routed experts: the kernels of prefill_reg.hpp and the choice between their forms.
 #include "host_common.hpp"
 #include "launchers.hpp"
 #include "prefill_reg.hpp"
@@ -47,20 +47,21 @@ __global__ __launch_bounds__(256) void prefill_prologue_kernel(const uint8_t* x,
 }
 
 namespace {
-// Which Q4_K batches the four-wave form of prefill_reg.hpp serves. It sweeps an expert's weights once per 32 rows, the wide form once per
+// Which batches the four-wave form of prefill_reg.hpp serves. It sweeps an expert's weights once per 32 rows, the wide form once per
 // 128; it has three times the workgroups in flight. Measured (wide, four waves), rows per expert on average and rounds of the wide form's
 // gate / up workgroups beside them: 8.5, 5.8 256, 199 us; 12.3, 13 185, 168; 15, 8.4 776, 707; 21, 3.5 195, 178; 22, 14 965, 1028;
 // 25, 9 867, 894; 37, 7.8 879, 961; 40, 3.3 435, 419; 46, 1.8 414, 380; 50, 4.2 270, 275; 56, 4.0 194, 178; 45, 18 1847, 2312.
+// Q8_0 rows are twice as wide, and the down rows are swept twice: 4, 3.2 182, 159; 12.5, 3.3 242, 230; 9.4, 3.2 414, 427; 15, 10 1220, 1364;
+// 21, 3.5 257, 285; 25, 3.6 538, 615; 37, 3.9 325, 369; 12.5, 0.3 79, 44; 50, 0.4 88, 48.
 bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
     const uint64_t e = wv.experts, a = assignments;
-    return a <= 16ULL * e || (a <= 56ULL * e && (128ULL * e + a) * wv.ffn <= 4ULL * compute_units() * 128U * 128U);
+    const bool q8 = wv.gate_type == MI355_TYPE_Q8_0 || wv.down_type == MI355_TYPE_Q8_0;
+    return a <= (q8 ? 13ULL : 16ULL) * e || (a <= 56ULL * e && (128ULL * e + a) * wv.ffn <= (q8 ? 1ULL : 4ULL) * compute_units() * 128U * 128U);
 }
-bool reg_gate(const mi355_moe_weights& wv) { return wv.gate_type == MI355_TYPE_Q4_K && wv.ffn % 128U == 0; }
-bool reg_down(const mi355_moe_weights& wv) { return wv.down_type == MI355_TYPE_Q4_K && wv.hidden % 256U == 0; }
 }  // namespace
 
 uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments) {
-    return reg_gate(wv) && reg_down(wv) && few_rows(wv, assignments) ? 32U : kPfTile;
+    return few_rows(wv, assignments) ? 32U : kPfTile;
 }
 
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, uint32_t items_at, uint32_t order_at, hipStream_t st) {
@@ -72,36 +73,25 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
     const auto grid_of = [&](uint32_t units, uint32_t each = 1U) { return units < each * resident ? units : each * resident; };
     const bool few = few_rows(wv, a.assignments);
     a.subs = prefill_split(wv, a.assignments) / 32U;
-    // gate / up + SwiGLU. Q4_K tensors: every wave expands its own rows in registers (prefill_reg.hpp); Q5_K / Q8_0: the loader /
-    // multiplier kernel (prefill_f16.hpp). Both leave h as two fp16 planes and its sub-block sums.
+    const auto launch = [&](auto mode, uint32_t type) {
+        constexpr int M = decltype(mode)::value;
+        const auto of = [&](auto format) {
+            constexpr int F = decltype(format)::value;
+            if (few) prefill_reg_kernel<M, 4, F><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
+            else prefill_reg_kernel<M, 8, F><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
+        };
+        if (type == MI355_TYPE_Q8_0) of(std::integral_constant<int, kRgQ80>{});
+        else if (type == MI355_TYPE_Q5_K) of(std::integral_constant<int, kRgQ5K>{});
+        else of(std::integral_constant<int, kRgQ4K>{});
+    };
+    // gate / up + SwiGLU: leaves h as two fp16 planes and its sub-block sums
     a.wa = wv.gate; a.wb = wv.up; a.expert_stride = wv.gate_expert_stride; a.row_stride = wv.gate_row_stride; a.k = wv.hidden; a.features = wv.ffn;
-    a.lo_pass = 0;
-    if (reg_gate(wv)) {
-        a.tiles = wv.ffn / (few ? 64U : 128U); a.units = item_slots * a.tiles;
-        if (few) prefill_reg_kernel<0, 4><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
-        else prefill_reg_kernel<0, 8><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
-    } else {
-        a.tiles = wv.ffn / 64U; a.units = item_slots * a.tiles;
-        if (wv.gate_type == MI355_TYPE_Q8_0) prefill_f16_kernel<0, 1><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        else if (wv.gate_type == MI355_TYPE_Q5_K) prefill_f16_kernel<0, 2><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        else prefill_f16_kernel<0, 0><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-    }
-    // down rows: h enters as hi + lo. The register-operand kernel multiplies both planes in one sweep of the weights; the loader /
-    // multiplier kernel runs a second pass over the lo plane that adds to the first pass's outputs.
+    a.tiles = wv.ffn / (few ? 64U : 128U); a.units = item_slots * a.tiles;
+    launch(std::integral_constant<int, 0>{}, wv.gate_type);
+    // down rows: h enters as hi + lo, both planes in one sweep of the weights
     a.wa = wv.down; a.wb = nullptr; a.expert_stride = wv.down_expert_stride; a.row_stride = wv.down_row_stride; a.k = wv.ffn; a.features = wv.hidden;
-    if (reg_down(wv)) {
-        a.tiles = wv.hidden / (few ? 128U : 256U); a.units = item_slots * a.tiles;
-        if (few) prefill_reg_kernel<1, 4><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
-        else prefill_reg_kernel<1, 8><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
-    } else {
-        a.tiles = wv.hidden / 128U; a.units = item_slots * a.tiles;
-        for (uint32_t pass = 0; pass < 2U; ++pass) {
-            a.lo_pass = pass;
-            if (wv.down_type == MI355_TYPE_Q8_0) prefill_f16_kernel<1, 1><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-            else if (wv.down_type == MI355_TYPE_Q5_K) prefill_f16_kernel<1, 2><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-            else prefill_f16_kernel<1, 0><<<grid_of(a.units), kPfThreads, 0, st>>>(a, items_at, order_at);
-        }
-    }
+    a.tiles = wv.hidden / (few ? 128U : 256U); a.units = item_slots * a.tiles;
+    launch(std::integral_constant<int, 1>{}, wv.down_type);
 }
 
 }  // namespace strix950

@@ -32,7 +32,6 @@ struct PrefillArgs {
     const uint8_t* x; uint64_t x_stride;          // MODE 0: fp16 token rows (bytes); MODE 1: unused
     _Float16* h;                                  // [assignments in plan order][ffn] fp16: written by MODE 0, read by MODE 1
     _Float16* h_lo;                               // the same shape: fp16(h - fp16(h)), so that hi + lo carries h to 22 bits
-    uint32_t lo_pass;                             // MODE 1 of prefill_f16_kernel: multiply the lo plane and ADD to the outputs (second pass)
     uint8_t* h_sums;                              // [assignments in plan order] sub-block sums of h: written by MODE 0, read by MODE 1
     const uint8_t* x_sums;                        // [rows] sub-block sums of the input rows (MODE 0)
     float* rawdots;                               // MODE 1: [assignment][hidden]

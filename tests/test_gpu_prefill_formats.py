@@ -1,0 +1,68 @@
+"""The fp16 prefill form on Q5_K and Q8_0 tensors: every number of token tiles and both workgroup forms against the exact-weight product."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def half(b):
+    return b.contiguous().view(torch.float16).to(torch.float64).squeeze(-1)
+
+
+def draw(gen, kind, rows, width):
+    """Random blocks (every code and factor occurs, small finite fp16 scales) and their values in double precision."""
+    per, size, scales = (32, 34, (1,)) if kind == "q8_0" else (256, 176, (1, 3))
+    b = torch.randint(0, 256, (rows, width // per, size), dtype=torch.uint8, device="cuda", generator=gen)
+    for at in scales:
+        b[..., at] = (b[..., at] & 0x03) | 0x0C
+    if kind == "q8_0":
+        return b.reshape(rows, -1), (half(b[..., 0:2])[..., None] * b[..., 2:].contiguous().view(torch.int8).to(torch.float64)).reshape(rows, width)
+    d, dmin, f = half(b[..., 0:2])[..., None], half(b[..., 2:4])[..., None], b[..., 4:16].to(torch.int64)
+    out = []
+    for j in range(8):                                     # (src/ggml_dequant.cpp: the K-quants' packed six-bit factors)
+        sc = f[..., j] & 63 if j < 4 else (f[..., j + 4] & 15) | ((f[..., j - 4] >> 6) << 4)
+        mn = f[..., j + 4] & 63 if j < 4 else (f[..., j + 4] >> 4) | ((f[..., j] >> 6) << 4)
+        nibbles = b[..., 48 + 32 * (j // 2):80 + 32 * (j // 2)].to(torch.int64)
+        q = (nibbles >> 4 if j & 1 else nibbles & 15) | (((b[..., 16:48].to(torch.int64) >> j) & 1) << 4)
+        out.append(d * sc[..., None] * q - dmin * mn[..., None])
+    return b.reshape(rows, -1), torch.stack(out, -2).reshape(rows, width)
+
+
+# rows per expert: one tile of 32 (both forms: few rows, and with three experts nothing else), two, three and four tiles, an item and a bit;
+# K of an odd number of super-blocks and of one
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(9, 256, 256, 3, 2), (40, 768, 512, 2, 1), (130, 512, 256, 1, 1), (190, 1280, 768, 2, 1), (70, 256, 1280, 1, 1),
+                                                           (2100, 512, 512, 32, 2), (2600, 256, 256, 32, 4)])
+@pytest.mark.parametrize("gate,down", [("q5_k", "q5_k"), ("q8_0", "q8_0"), ("q5_k", "q8_0"), ("q8_0", "q5_k")])
+def test_against_the_exact_product(strix, rows, hidden, ffn, experts, top_k, gate, down):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    (g, G), (u, U), (d, D) = draw(gen, gate, experts * ffn, hidden), draw(gen, gate, experts * ffn, hidden), draw(gen, down, experts * hidden, ffn)
+    kinds = dict(gate_type=getattr(strix, "TYPE_" + gate.upper()), down_type=getattr(strix, "TYPE_" + down.upper()))
+    layer = strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows, prefill_f16=True, **kinds)
+    x = (torch.randn((rows, hidden), device="cuda", generator=gen) * 0.25).to(torch.float16)
+    ids = torch.rand((rows, experts), device="cuda", generator=gen).topk(top_k, dim=1).indices.to(torch.int32)
+    layer.run_prefill_f16(x, ids, torch.rand((rows, top_k), device="cuda", generator=gen))
+    assert int(layer.status[:rows].sum()) == 0
+    raw = layer.rawdots.reshape(-1, hidden)[:rows * top_k].to(torch.float64)
+    flat, X = ids.reshape(-1).long(), x.to(torch.float64)
+    for e in range(experts):
+        at = (flat == e).nonzero().squeeze(1)
+        xe, Ge, Ue, De = X[at // top_k], G[e * ffn:(e + 1) * ffn], U[e * ffn:(e + 1) * ffn], D[e * hidden:(e + 1) * hidden]
+        a, b = xe @ Ge.T, xe @ Ue.T
+        s = 1 / (1 + torch.exp(-a))
+        h = a * s * b
+        # every product accumulates k / 16 matrix operations and the scaled partial sums of k / 32 blocks in fp32, each within 2^-24 of the sum of
+        # magnitudes: no more than (k / 8) 2^-24 of it; the activation's own operations and h's 22 bits add 2^-20 of h
+        step = 2.0 ** -24 / 8
+        ga, ua = xe.abs() @ Ge.abs().T * (hidden * step), xe.abs() @ Ue.abs().T * (hidden * step)
+        slope = (s + a * s * (1 - s)).abs()
+        dh = (b.abs() + ua) * slope.clamp(min=0.1) * ga * 1.1 + (a * s).abs() * ua + h.abs() * 2.0 ** -20
+        bound = dh @ De.abs().T + h.abs() @ De.abs().T * (ffn * step)
+        assert bool(((raw[at] - h @ De.T).abs() <= bound).all()), e
