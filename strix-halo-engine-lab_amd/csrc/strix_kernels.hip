@@ -1055,6 +1055,78 @@ __global__ __launch_bounds__(256) void merge_kernel(mi355_moe_weights w, RowsK r
 }
 
 constexpr uint32_t kDownMergeSlots = 8;        // top_k bound: 8 waves x 2 ring slots fill the LDS of a compute unit
+// The job word of a down + combine launch, asked for at its start. A batch planned from early routes (r.awords): the front launch left its
+// non-finite flags per assignment; every workgroup folds them to the same job word, the first workgroup of a row publishes its row's.
+struct DownJob { uint32_t job, word[2]; };
+__device__ __forceinline__ DownJob down_job_request(const RowsK& r, uint32_t assignments, uint32_t lane) {
+    DownJob d{0U, {0U, 0U}};
+    if (r.awords) {
+        if (lane < assignments) d.word[0] = r.awords[lane];
+        if (lane + 64U < assignments) d.word[1] = r.awords[lane + 64U];
+    } else d.job = *r.job_status;
+    return d;
+}
+__device__ __forceinline__ uint32_t down_job(const DownJob& d, const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t wave, uint32_t lane) {
+    if (!r.awords) return d.job;
+    const uint32_t job = (__ballot(d.word[0] >> 31) | __ballot(d.word[1] >> 31)) ? static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION) : 0U;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) r.plan[kPlanLinesAt + kLinesEpoch] += 1U;      // this call's epoch is spent
+    if (job && blockIdx.x == 0 && wave == 0) {
+        const uint32_t lo = row * w.top_k, hi = lo + w.top_k;
+        const bool mine = (lane >= lo && lane < hi && (d.word[0] >> 31)) || (lane + 64U >= lo && lane + 64U < hi && (d.word[1] >> 31));
+        const bool any = __ballot(mine) != 0;
+        if (lane == 0) {
+            if (any) atomicOr(r.status_of(row), r.nonfinite_bit);
+            atomicOr(r.job_status, static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION));
+        }
+    }
+    return job;
+}
+// What the fold of a row's slots needs beside their values, asked for at the start of the launch by the wavefront that folds (lane k:
+// weight and expert of slot k; the row's status as the launches before left it; the base of column o): behind the barrier it was up to
+// four ways to memory in a row, by one thread.
+struct SlotFold { float weight, base; uint32_t route, status; };
+__device__ __forceinline__ SlotFold slot_fold_request(const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t o, uint32_t form, uint32_t wave, uint32_t lane) {
+    SlotFold f{0.0F, 0.0F, 0xffffffffU, 0U};
+    if (wave != 0) return f;
+    f.status = *r.status_of(row);
+    if (lane < w.top_k) {
+        f.weight = r.route_weights_of(row)[lane];
+        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT) f.route = r.routes_of(row)[lane];
+    }
+    if (r.base) f.base = r.base_of(row)[o];
+    return f;
+}
+// The row's value of one column, as merge_kernel folds it (every lane of the wavefront takes part). Fail closed: a row flagged by an
+// earlier stage publishes nothing (the aggregate bit is the combine's own).
+template <class Value>
+__device__ __forceinline__ void slot_fold(const SlotFold& f, const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t o, uint32_t form, bool stores, uint32_t lane, Value value) {
+    if (f.status & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE)) return;
+    const uint32_t K = w.top_k;
+    const bool ascending = form == MI355_COMBINE_MULADD_ASCENDING_EXPERT;
+    uint32_t place = lane;                                   // of the lane's slot; stable: an equal expert in an earlier slot goes first
+    if (ascending) {
+        place = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kDownMergeSlots; ++k) {
+            const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(f.route), static_cast<int>(k)));
+            place += k < K && (other < f.route || (other == f.route && k < lane)) ? 1U : 0U;
+        }
+    }
+    float acc = 0.0F;
+#pragma unroll
+    for (uint32_t k = 0; k < kDownMergeSlots; ++k) {
+        if (k >= K) continue;
+        const uint32_t slot = ascending ? static_cast<uint32_t>(__builtin_ctzll(__ballot(lane < K && place == k))) : k;
+        const float wt = f_of(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b_of(f.weight)), static_cast<int>(slot)))), ev = value(slot);
+        if (!ascending && k + r.shared_slots < K) acc = __builtin_fmaf(wt, ev, acc);
+        else acc = acc + wt * ev;
+    }
+    if (!stores) return;
+    const float y = r.base ? acc + f.base : acc;
+    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
+    r.output[static_cast<size_t>(row) * r.output_stride + o] = y;
+}
+
 // Down rows and the ordered combine of a decode batch in one launch: a workgroup owns (row, 64 output columns) and has one
 // wave per slot of the row, wave k sweeping the down rows of the expert in slot k (the plan holds one item per assignment,
 // in assignment order); the waves leave their 64 values in LDS and wave 0 folds them exactly as merge_kernel does. Only
@@ -1066,34 +1138,13 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
     __shared__ __attribute__((aligned(16))) uint8_t ring_even[kDownMergeSlots][slot_bytes(1)];
     __shared__ __attribute__((aligned(16))) uint8_t ring_odd[kDownMergeSlots][slot_bytes(1)];
     __shared__ float slot_value[kDownMergeSlots][64];
-    __shared__ uint32_t slot_order[kDownMergeSlots];
-    __shared__ float slot_weight[kDownMergeSlots];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, row = blockIdx.y, o = blockIdx.x * 64U + lane;
-    uint32_t job;                                                              // (requested together with the item: one round trip, not two)
-    uint32_t word[2] = {0U, 0U};
-    if (r.awords) {
-        if (lane < assignments) word[0] = r.awords[lane];
-        if (lane + 64U < assignments) word[1] = r.awords[lane + 64U];
-    } else job = *r.job_status;
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item: one round trip, not two)
+    const SlotFold fold = slot_fold_request(w, r, row, o, form, wave, lane);
     const uint32_t a = row * w.top_k + wave;
     const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), a);
     const uint32_t e = __builtin_amdgcn_readfirstlane(item.e), begin = __builtin_amdgcn_readfirstlane(item.begin), end = __builtin_amdgcn_readfirstlane(item.end);
-    if (r.awords) {
-        // a batch planned from early routes: the front launch left its non-finite flags per assignment; every workgroup folds them
-        // to the same job word, the first workgroup of a row publishes its row's
-        job = (__ballot(word[0] >> 31) | __ballot(word[1] >> 31)) ? static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION) : 0U;
-        if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) r.plan[kPlanLinesAt + kLinesEpoch] += 1U;      // this call's epoch is spent
-        if (job && blockIdx.x == 0 && wave == 0) {
-            const uint32_t lo = row * w.top_k, hi = lo + w.top_k;
-            const bool mine = (lane >= lo && lane < hi && (word[0] >> 31)) || (lane + 64U >= lo && lane + 64U < hi && (word[1] >> 31));
-            const bool any = __ballot(mine) != 0;
-            if (lane == 0) {
-                if (any) atomicOr(r.status_of(row), r.nonfinite_bit);
-                atomicOr(r.job_status, static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION));
-            }
-        }
-    }
-    if (job & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
+    if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (begin != end) {                                                        // (an invalid route has no item: its row is flagged)
         const uint32_t first = item.first ? item.first - 1U : ordered(r, plan_order_at(w.experts), begin);
@@ -1112,32 +1163,14 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
         r.rawdots_of(src[0], w.hidden)[o] = value;
     }
     slot_value[wave][lane] = value;
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t j = i; j > 0 && r.routes_of(row)[slot_order[j]] < r.routes_of(row)[slot_order[j - 1]]; --j) {
-                    const uint32_t t = slot_order[j]; slot_order[j] = slot_order[j - 1]; slot_order[j - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
     __syncthreads();
-    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is the combine's own)
-    if (wave != 0 || (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE))) return;
-    float acc = 0.0F;
-    for (uint32_t k = 0; k < w.top_k; ++k) {
-        const float ev = slot_value[slot_order[k]][lane];
-        if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) acc = __builtin_fmaf(slot_weight[k], ev, acc);
-        else acc = acc + slot_weight[k] * ev;
-    }
-    const float y = r.base ? acc + r.base_of(row)[o] : acc;
-    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
-    r.output[static_cast<size_t>(row) * r.output_stride + o] = y;
+    if (wave == 0) slot_fold(fold, w, r, row, o, form, true, lane, [&](uint32_t slot) { return slot_value[slot][lane]; });
 }
 
 // down_merge_kernel for dense rows of at most four super-blocks (down_row_stride = B * 144): the 64 rows of a column block stream as B
 // contiguous stages of 1 KB pieces instead of B stages of 64 separate 144-byte blocks (a read-only launch of this shape moves the
 // same bytes in 11.8 us against 14.4 us), the block terms meet in LDS in block order and lane = row adds them in ascending order.
+// (Job word and fold written out: through the functions above, 1, 8, 16 rows of hidden 2048 / ffn 768 27.7, 45.9, 73.5 -> 28.2, 46.2, 73.9 us.)
 template <int B>
 __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     // (the two ring slots are separate LDS objects, as in down_merge_kernel)
@@ -1218,17 +1251,17 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_quad_kernel(m
     __shared__ __attribute__((aligned(16))) uint8_t mq2[DEPTH > 2 ? kDownMergeSlots : 1][DEPTH > 2 ? kQuadSlotBytes : 16];
     __shared__ __attribute__((aligned(16))) uint8_t mq3[DEPTH > 3 ? kDownMergeSlots : 1][DEPTH > 3 ? kQuadSlotBytes : 16];
     __shared__ float slot_value[kDownMergeSlots][kQuadRows];
-    __shared__ uint32_t slot_order[kDownMergeSlots];
-    __shared__ float slot_weight[kDownMergeSlots];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, rr = lane >> 2, row = blockIdx.y, o0 = blockIdx.x * kQuadRows;
     lds_u8* const ring[4] = {(lds_u8*)mq0[wave], (lds_u8*)mq1[wave], (lds_u8*)mq2[DEPTH > 2 ? wave : 0], (lds_u8*)mq3[DEPTH > 3 ? wave : 0]};
     lds_u8* slots[DEPTH];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) slots[i] = ring[i];
-    const uint32_t job = *r.job_status;                                        // (requested together with the item)
+    const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
+    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
     const uint32_t a = row * w.top_k + wave;
     const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), a);
-    if (job & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
+    if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
         const uint32_t src = __builtin_amdgcn_readfirstlane(item.first ? item.first - 1U : ordered(r, plan_order_at(w.experts), item.begin));
@@ -1241,28 +1274,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_quad_kernel(m
         if (p == 0) r.rawdots_of(src, w.hidden)[o0 + rr] = value;
     }
     if (p == 0) slot_value[wave][rr] = value;
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t j = i; j > 0 && r.routes_of(row)[slot_order[j]] < r.routes_of(row)[slot_order[j - 1]]; --j) {
-                    const uint32_t t = slot_order[j]; slot_order[j] = slot_order[j - 1]; slot_order[j - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
     __syncthreads();
-    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is the combine's own)
-    if (threadIdx.x >= kQuadRows || (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE))) return;
-    float acc = 0.0F;
-    for (uint32_t k = 0; k < w.top_k; ++k) {
-        const float ev = slot_value[slot_order[k]][lane];
-        if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) acc = __builtin_fmaf(slot_weight[k], ev, acc);
-        else acc = acc + slot_weight[k] * ev;
-    }
-    const uint32_t o = o0 + lane;
-    const float y = r.base ? acc + r.base_of(row)[o] : acc;
-    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
-    r.output[static_cast<size_t>(row) * r.output_stride + o] = y;
+    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q5_1 down rows of whole, 16-byte aligned super-blocks (the host executor's format,
@@ -1279,13 +1292,13 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
     static_assert(16U * ROWB == 1024U * WC, "the rows of a stage fill the weight copies");
     __shared__ __attribute__((aligned(16))) uint8_t ring_mem[DEPTH][kDownMergeSlots][SLOT];
     __shared__ float slot_value[kDownMergeSlots][16];
-    __shared__ uint32_t slot_order[kDownMergeSlots];
-    __shared__ float slot_weight[kDownMergeSlots];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o0 = blockIdx.x * 16U, o = o0 + rr;
-    const uint32_t job = *r.job_status;                                        // (requested together with the item)
+    const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
+    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
     const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
-    if (job & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
+    if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
         const uint32_t src = item.first ? item.first - 1U : ordered(r, plan_order_at(w.experts), item.begin);
@@ -1361,28 +1374,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
         if (j == 0) r.rawdots_of(src, w.hidden)[o] = value;
     }
     if (j == 0) slot_value[wave][rr] = value;
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t jj = i; jj > 0 && r.routes_of(row)[slot_order[jj]] < r.routes_of(row)[slot_order[jj - 1]]; --jj) {
-                    const uint32_t t = slot_order[jj]; slot_order[jj] = slot_order[jj - 1]; slot_order[jj - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
     __syncthreads();
-    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is the combine's own)
-    if (threadIdx.x >= 16U || (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE))) return;
-    float sum = 0.0F;
-    for (uint32_t k = 0; k < w.top_k; ++k) {
-        const float ev = slot_value[slot_order[k]][lane];
-        if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) sum = __builtin_fmaf(slot_weight[k], ev, sum);
-        else sum = sum + slot_weight[k] * ev;
-    }
-    const uint32_t oc = blockIdx.x * 16U + lane;
-    const float y = r.base ? sum + r.base_of(row)[oc] : sum;
-    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
-    r.output[static_cast<size_t>(row) * r.output_stride + oc] = y;
+    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q6_K down rows (src/moe_a8_down_contract.cpp:147-158): the workgroup of (row, 16 columns),
@@ -1390,13 +1383,13 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
 __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
     __shared__ float slot_value[kDownMergeSlots][16];
-    __shared__ uint32_t slot_order[kDownMergeSlots];
-    __shared__ float slot_weight[kDownMergeSlots];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, half = p >> 1, odd = p & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
-    const uint32_t job = *r.job_status;                                        // (requested together with the item)
+    const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
+    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
     const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
-    if (job & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
+    if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
         const uint32_t src = item.first ? item.first - 1U : ordered(r, plan_order_at(w.experts), item.begin);
@@ -1448,28 +1441,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi
         if (p == 0) r.rawdots_of(src, w.hidden)[o] = value;
     }
     if (p == 0) slot_value[wave][rr] = value;
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t jj = i; jj > 0 && r.routes_of(row)[slot_order[jj]] < r.routes_of(row)[slot_order[jj - 1]]; --jj) {
-                    const uint32_t t = slot_order[jj]; slot_order[jj] = slot_order[jj - 1]; slot_order[jj - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
     __syncthreads();
-    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is the combine's own)
-    if (threadIdx.x >= 16U || (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE))) return;
-    float sum = 0.0F;
-    for (uint32_t k = 0; k < w.top_k; ++k) {
-        const float ev = slot_value[slot_order[k]][lane];
-        if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) sum = __builtin_fmaf(slot_weight[k], ev, sum);
-        else sum = sum + slot_weight[k] * ev;
-    }
-    const uint32_t oc = blockIdx.x * 16U + lane;
-    const float y = r.base ? sum + r.base_of(row)[oc] : sum;
-    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
-    r.output[static_cast<size_t>(row) * r.output_stride + oc] = y;
+    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q8_0 down tensors (the host executor's format, src/cpu/core/routed_expert.cpp:110-126): the
@@ -1478,13 +1451,13 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi
 __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
     __shared__ float slot_value[kDownMergeSlots][16];
-    __shared__ uint32_t slot_order[kDownMergeSlots];
-    __shared__ float slot_weight[kDownMergeSlots];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, odd = j & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
-    const uint32_t job = *r.job_status;                                        // (requested together with the item)
+    const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
+    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
     const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
-    if (job & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
+    if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
         const uint32_t src = item.first ? item.first - 1U : ordered(r, plan_order_at(w.experts), item.begin);
@@ -1513,28 +1486,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q8_0_kernel(m
         if (j == 0) r.rawdots_of(src, w.hidden)[o] = value;
     }
     if (j == 0) slot_value[wave][rr] = value;
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_order[k] = k;
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT)
-            for (uint32_t i = 1; i < w.top_k; ++i)
-                for (uint32_t jj = i; jj > 0 && r.routes_of(row)[slot_order[jj]] < r.routes_of(row)[slot_order[jj - 1]]; --jj) {
-                    const uint32_t t = slot_order[jj]; slot_order[jj] = slot_order[jj - 1]; slot_order[jj - 1] = t;
-                }
-        for (uint32_t k = 0; k < w.top_k; ++k) slot_weight[k] = r.route_weights_of(row)[slot_order[k]];
-    }
     __syncthreads();
-    // fail closed: a row flagged by an earlier stage publishes nothing (the aggregate bit is the combine's own)
-    if (threadIdx.x >= 16U || (*r.status_of(row) & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE))) return;
-    float acc = 0.0F;
-    for (uint32_t k = 0; k < w.top_k; ++k) {
-        const float ev = slot_value[slot_order[k]][lane];
-        if (form == MI355_COMBINE_FMA_SLOT_ORDER && k + r.shared_slots < w.top_k) acc = __builtin_fmaf(slot_weight[k], ev, acc);
-        else acc = acc + slot_weight[k] * ev;
-    }
-    const uint32_t oc = blockIdx.x * 16U + lane;
-    const float y = r.base ? acc + r.base_of(row)[oc] : acc;
-    if (!finite_f(y)) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_AGGREGATE));
-    r.output[static_cast<size_t>(row) * r.output_stride + oc] = y;
+    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // SwiGLU + A8 re-quantisation of dense gate/up rows. Reference: src/cpu/core/routed_expert.cpp:147-170.
@@ -2154,6 +2107,21 @@ void launch_down_merge(const mi355_moe_weights& wv, const RowsK& k, uint32_t row
     else if (flat && B == 4U) down_merge_flat_kernel<4><<<grid, threads, 0, st>>>(wv, k, items, form);
     else down_merge_kernel<<<grid, threads, 0, st>>>(wv, k, items, form);
 }
+// The other formats' down rows + combine, 16 output columns a workgroup: which launches they take, and the launch.
+bool down_merge_format_takes(const mi355_moe_weights& wv, uint32_t rows) {
+    if (wv.top_k > kDownMergeSlots || wv.hidden % 16U != 0 || rows > 65535U) return false;
+    if (wv.down_type == MI355_TYPE_Q8_0) return wv.ffn % 128U == 0;
+    if (wv.down_type == MI355_TYPE_Q5_1) return wv.ffn % 256U == 0 && wv.down_row_stride % 16U == 0 && wv.down_expert_stride % 16U == 0;      // (what down_q51_ring_kernel's copies need)
+    return wv.down_type == MI355_TYPE_Q6_K;
+}
+bool launch_down_merge_format(const mi355_moe_weights& wv, const RowsK& k, uint32_t rows, uint32_t items, uint32_t form, hipStream_t st) {
+    if (!down_merge_format_takes(wv, rows)) return false;
+    const dim3 grid(wv.hidden / 16U, rows);
+    if (wv.down_type == MI355_TYPE_Q8_0) down_merge_q8_0_kernel<<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    else if (wv.down_type == MI355_TYPE_Q5_1) down_merge_q51_kernel<2><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    else down_merge_q6k_kernel<<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    return true;
+}
 
 int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, const float* logit_bias, float* scores, const LayerNorm& norm,
                       const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, uint32_t form, mi355_stream stream, uint32_t phase = kLayerWhole) {
@@ -2211,8 +2179,10 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     // From 8 assignments on (one row of top-8): measured at hidden 2048 / ffn 768 against the three launches of the smallest batches
     // (router, 16-row projection, 16-row down + combine): 1 row 28.7 / 31.3 us, 2 rows 31.6 / 35.4, 3 rows 33.4 / 37.8, 4 rows
     // 35.7 / 40.3, 5 rows 38.4 / 48.6, 6 rows 41.2 / 57.8.
+    // Down rows of another format, 1, 8, 16 rows against the router launch, the projection and the same down + combine launch: Q6_K 31.6, 67.5,
+    // 111.8 -> 26.2, 58.5, 95.2 us, Q8_0 31.0, 67.6, 111.7 -> 25.3, 58.6, 92.1, Q5_1 30.8, 61.0, 100.5 -> 24.9, 52.0, 83.8.
     if (!norm.on && p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
-        wv.down_type == MI355_TYPE_Q4_K && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
+        (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
         wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden) {
         a.awords = r->plan + kPlanAwordsAt;
         a.early_perturb = g_early_perturb.load(std::memory_order_relaxed);
@@ -2231,7 +2201,7 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
             STRIX_LAUNCHED("moe layer early routes + gate / up");
         }
         if (do_back) {
-            launch_down_merge(wv, k, rows, items, form, st);
+            if (!launch_down_merge_format(wv, k, rows, items, form, st)) launch_down_merge(wv, k, rows, items, form, st);
             STRIX_LAUNCHED("moe layer experts + combine");
         }
         return MI355_OK;
@@ -2269,19 +2239,7 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         STRIX_LAUNCHED("moe layer experts + combine");
         return MI355_OK;
     }
-    if (wv.down_type == MI355_TYPE_Q8_0 && wv.top_k <= kDownMergeSlots && wv.hidden % 16U == 0 && wv.ffn % 128U == 0 && rows <= 65535U) {
-        down_merge_q8_0_kernel<<<dim3(wv.hidden / 16U, rows), 64U * wv.top_k, 0, st>>>(wv, layer_rows(), items, form);
-        STRIX_LAUNCHED("moe layer experts + combine");
-        return MI355_OK;
-    }
-    if (wv.down_type == MI355_TYPE_Q5_1 && wv.top_k <= kDownMergeSlots && wv.hidden % 16U == 0 && rows <= 65535U && wv.ffn % 256U == 0 &&
-        wv.down_row_stride % 16U == 0 && wv.down_expert_stride % 16U == 0) {       // (what down_q51_ring_kernel's copies need)
-        down_merge_q51_kernel<2><<<dim3(wv.hidden / 16U, rows), 64U * wv.top_k, 0, st>>>(wv, layer_rows(), items, form);
-        STRIX_LAUNCHED("moe layer experts + combine");
-        return MI355_OK;
-    }
-    if (wv.down_type == MI355_TYPE_Q6_K && wv.top_k <= kDownMergeSlots && wv.hidden % 16U == 0 && rows <= 65535U) {
-        down_merge_q6k_kernel<<<dim3(wv.hidden / 16U, rows), 64U * wv.top_k, 0, st>>>(wv, layer_rows(), items, form);
+    if (launch_down_merge_format(wv, layer_rows(), rows, items, form, st)) {
         STRIX_LAUNCHED("moe layer experts + combine");
         return MI355_OK;
     }

@@ -1,0 +1,61 @@
+"""Decode layers planned from early routes with Q6_K, Q8_0 or Q5_1 down rows: the bits of the staged launches on the exact router's choice."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def blocks(gen, rows, width, per, size, scales):
+    w = torch.randint(0, 256, (rows, width // per, size), dtype=torch.uint8, device="cuda", generator=gen)
+    for at in scales:
+        w[..., at] = (w[..., at] & 0x03) | 0x0C
+    return w.reshape(rows, -1)
+
+
+# eight assignments (the fewest of this form) up to 128 (the most); rows of one and of several stages
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,amount", [(1, 2048, 768, 128, 8, 40), (16, 1024, 512, 32, 8, 40), (7, 512, 256, 24, 5, 300), (4, 768, 1280, 16, 2, 0)])
+@pytest.mark.parametrize("down", ["q6_k", "q8_0", "q5_1"])
+def test_early_routes_equal_staged_launches(strix, rows, hidden, ffn, experts, top_k, amount, down):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    g, u = (blocks(gen, experts * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, experts * hidden, ffn, *{"q6_k": (256, 210, (209,)), "q8_0": (32, 34, (1,)), "q5_1": (32, 24, (1, 3))}[down])
+    layer, staged = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows, down_type=getattr(strix, "TYPE_" + down.upper())) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+    base = torch.randn((rows, hidden), device="cuda", generator=gen)
+    ids, w = strix.route(x, router, top_k)[:2]
+
+    def run(displaced, form, b):
+        strix.lib().mi355_debug_early_route_perturb(displaced)
+        try:
+            y, got, weights, _ = layer.run_layer(x, router, base=b, combine=form)
+            torch.cuda.synchronize()
+        finally:
+            strix.lib().mi355_debug_early_route_perturb(0)
+        assert int(layer.status[:rows].sum()) == 0 and torch.equal(got, ids) and torch.equal(weights.view(torch.int32), w.view(torch.int32))
+        return y.clone()
+
+    for form in (strix.COMBINE_FMA_SLOT, strix.COMBINE_MULADD_ASC):
+        for b in (None, base):
+            want = staged.run(x, ids, w, base=b, combine=form)
+            for displaced in (0, amount):
+                assert torch.equal(run(displaced, form, b).view(torch.int32), want.view(torch.int32)), (form, displaced)
+    # a row whose projection overflows: the same status as the staged launches give, no row published, and the next call is whole again
+    good, x0 = run(0, strix.COMBINE_FMA_SLOT, None), x.clone()
+    wide = x.to(torch.float32)
+    wide[rows - 1] *= 1e37
+    layer.output.fill_(7.0)
+    y, got, weights, _ = layer.run_layer(wide, router)
+    staged.run(wide, got.clone(), weights.clone())
+    assert torch.equal(layer.status[:rows], staged.status[:rows]) and int(layer.status[rows - 1]) != 0
+    assert bool((layer.output[:rows] == 7.0).all())
+    x.copy_(x0)
+    assert torch.equal(run(amount, strix.COMBINE_FMA_SLOT, None).view(torch.int32), good.view(torch.int32))
