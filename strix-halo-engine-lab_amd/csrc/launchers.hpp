@@ -10,6 +10,8 @@ namespace strix950 {
 // route.hip: logits of a batch past the decode sizes into a.scores; softmax, selection and weights of every row of a.scores
 void launch_route_batch_logits(const RouteArgs& a, hipStream_t st);
 void launch_route_select(const RouteArgs& a, hipStream_t st);
+// RMSNorm of rows of any input kind into dense fp32 rows (weight may be null: a unit scale)
+void launch_norm_rows(const void* x, uint32_t kind, uint64_t x_stride, const float* weight, uint32_t hidden, float eps, float* normed, uint32_t rows, hipStream_t st);
 // A8 image, routes and status words of the rows of a staged batch. select: the router whose logits are in its scores (null: the routes
 // are given); q.status is not used.
 struct RouteCheck {

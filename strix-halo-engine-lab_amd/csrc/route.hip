@@ -72,4 +72,51 @@ void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, cons
 
 void launch_route_select(const RouteArgs& a, hipStream_t st) { route_select_kernel<<<a.rows, 64, 0, st>>>(a); }
 
+// RMSNorm of rows of any input kind into fp32 rows (the staged form of the fused norm): rmsnorm_f32_kernel's order.
+template <int KIND>
+__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const uint8_t* x, uint64_t x_stride, const float* w, uint32_t n, float eps, float* y) {
+    // row_norm_factor's chains and halvings, a thread per chain. Bound by latency: the first eight values of a chain and their weights are
+    // asked for at once and kept (one row of 2048 by one wavefront, element after element: 21 us).
+    constexpr uint32_t HELD = 8U;
+    __shared__ float partial[256];
+    const uint8_t* xr = x + blockIdx.x * x_stride;
+    const uint32_t l = threadIdx.x, L = n >= 512U ? 256U : 128U, end = l < L ? n : 0U;
+    float v[HELD], wv[HELD], a = 0.0F;
+#pragma unroll
+    for (uint32_t j = 0; j < HELD; ++j) {
+        const uint32_t i = l + L * j;
+        v[j] = i < end ? load_activation<KIND>(xr, i) : 0.0F;
+        wv[j] = w && i < end ? w[i] : 0.0F;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < HELD; ++j)
+        if (l + L * j < end) a = __builtin_fmaf(v[j], v[j], a);
+    for (uint32_t i = l + L * HELD; i < end; i += L) {
+        const float u = load_activation<KIND>(xr, i);
+        a = __builtin_fmaf(u, u, a);
+    }
+    partial[l] = a;
+    for (uint32_t h = L / 2U; h > 0; h >>= 1) {
+        __syncthreads();
+        if (l < h) partial[l] = partial[l] + partial[l + h];
+    }
+    __syncthreads();
+    const float r = 1.0F / __builtin_sqrtf(partial[0] / static_cast<float>(n) + eps);
+    float* yr = y + static_cast<size_t>(blockIdx.x) * n;
+#pragma unroll
+    for (uint32_t j = 0; j < HELD; ++j)
+        if (l + L * j < end) { const float u = v[j] * r; yr[l + L * j] = w ? u * wv[j] : u; }
+    for (uint32_t i = l + L * HELD; i < end; i += L) {
+        const float u = load_activation<KIND>(xr, i) * r;
+        yr[i] = w ? u * w[i] : u;
+    }
+}
+
+void launch_norm_rows(const void* x, uint32_t kind, uint64_t x_stride, const float* weight, uint32_t hidden, float eps, float* normed, uint32_t rows, hipStream_t st) {
+    const uint8_t* at = static_cast<const uint8_t*>(x);
+    if (kind == MI355_INPUT_F32) rmsnorm_rows_kernel<0><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+    else if (kind == MI355_INPUT_F16) rmsnorm_rows_kernel<1><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+    else rmsnorm_rows_kernel<2><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+}
+
 }  // namespace strix950

@@ -2074,19 +2074,6 @@ int32_t enqueue_staged(const mi355_moe_weights* w, const mi355_moe_rows* r, uint
     return enqueue_merge(w, r, rows, form, stream, shared_slots);
 }
 
-// RMSNorm of rows of any input kind into fp32 rows (the staged form of the fused norm): rmsnorm_f32_kernel's order.
-template <int KIND>
-__global__ __launch_bounds__(64) void rmsnorm_rows_kernel(const uint8_t* x, uint64_t x_stride, const float* w, uint32_t n, float eps, float* y) {
-    __shared__ float partial[256];
-    const uint8_t* xr = x + blockIdx.x * x_stride;
-    const float r = row_norm_factor<KIND>(partial, xr, n, eps);
-    float* yr = y + static_cast<size_t>(blockIdx.x) * n;
-    for (uint32_t i = threadIdx.x; i < n; i += 64U) {
-        const float v = load_activation<KIND>(xr, i) * r;
-        yr[i] = w ? v * w[i] : v;
-    }
-}
-
 struct LayerNorm { bool on; const float* weight; float eps; float* normed; };
 std::atomic<uint32_t> g_early_perturb{0};
 std::atomic<bool> g_down_merge_flat{true};
@@ -2139,13 +2126,11 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     STRIX_REQUIRE(!norm.on || (norm.normed && aligned(norm.normed, 16) && (!norm.weight || aligned(norm.weight, 16)) && norm.eps >= 0.0F),
                   "moe layer: the fused RMSNorm needs a 16-byte aligned fp32 [rows][hidden] view for the normalised rows, aligned weights, eps >= 0");
     hipStream_t st = hs(stream);
+    const auto norm_rows = [&] { launch_norm_rows(r->input, r->input_kind, r->input_stride, norm.weight, wv.hidden, norm.eps, norm.normed, rows, st); };
     if (rows > kFusedMaxRows || plan_split(wv, rows) != 1U) {      // large batches, and decode batches over large experts (shared sweeps): router, then the staged prologue / plan
         mi355_moe_rows staged = *r;
         if (norm.on && do_front) {
-            const uint8_t* x = static_cast<const uint8_t*>(r->input);
-            if (r->input_kind == MI355_INPUT_F32) rmsnorm_rows_kernel<0><<<rows, 64, 0, st>>>(x, r->input_stride, norm.weight, wv.hidden, norm.eps, norm.normed);
-            else if (r->input_kind == MI355_INPUT_F16) rmsnorm_rows_kernel<1><<<rows, 64, 0, st>>>(x, r->input_stride, norm.weight, wv.hidden, norm.eps, norm.normed);
-            else rmsnorm_rows_kernel<2><<<rows, 64, 0, st>>>(x, r->input_stride, norm.weight, wv.hidden, norm.eps, norm.normed);
+            norm_rows();
             STRIX_LAUNCHED("moe layer norm");
         }
         if (norm.on) { staged.input = norm.normed; staged.input_kind = MI355_INPUT_F32; staged.input_stride = 4ULL * wv.hidden; }
@@ -2179,11 +2164,17 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     // From 8 assignments on (one row of top-8): measured at hidden 2048 / ffn 768 against the three launches of the smallest batches
     // (router, 16-row projection, 16-row down + combine): 1 row 28.7 / 31.3 us, 2 rows 31.6 / 35.4, 3 rows 33.4 / 37.8, 4 rows
     // 35.7 / 40.3, 5 rows 38.4 / 48.6, 6 rows 41.2 / 57.8.
+    // With the RMSNorm, its rows in a launch of their own in front (the router launch that holds the norm before): Q4_K 36.5, 62.3, 102.9 ->
+    // 34.1, 53.9, 81.0 us, Q6_K 37.6, 74.1, 123.5 -> 32.9, 66.4, 102.5.
     // Down rows of another format, 1, 8, 16 rows against the router launch, the projection and the same down + combine launch: Q6_K 31.6, 67.5,
     // 111.8 -> 26.2, 58.5, 95.2 us, Q8_0 31.0, 67.6, 111.7 -> 25.3, 58.6, 92.1, Q5_1 30.8, 61.0, 100.5 -> 24.9, 52.0, 83.8.
-    if (!norm.on && p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
+    if (p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
         (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
         wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden) {
+        if (norm.on) {      // the normalised rows in a launch of their own; the front launch takes them as fp32 rows
+            if (do_front) norm_rows();
+            a.x = reinterpret_cast<const uint8_t*>(norm.normed); a.kind = MI355_INPUT_F32; a.x_stride = 4ULL * wv.hidden; a.norm_on = 0U;
+        }
         a.awords = r->plan + kPlanAwordsAt;
         a.early_perturb = g_early_perturb.load(std::memory_order_relaxed);
         // the early logits of row i (64-bit words) live in the row's (still unused) unweighted-output block: the exact logits own `scores`

@@ -59,3 +59,30 @@ def test_early_routes_equal_staged_launches(strix, rows, hidden, ffn, experts, t
     assert bool((layer.output[:rows] == 7.0).all())
     x.copy_(x0)
     assert torch.equal(run(amount, strix.COMBINE_FMA_SLOT, None).view(torch.int32), good.view(torch.int32))
+
+
+# fp32 rows, whose exact chain holds the row in registers (one step of 16 features each), and rows normalised in front of the launch
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(2, 256, 256, 16, 4), (16, 1280, 256, 24, 8), (9, 2048, 512, 48, 4)])
+@pytest.mark.parametrize("norm", [None, torch.float32, torch.bfloat16])
+def test_fp32_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_k, norm):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    g, u = (blocks(gen, experts * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, experts * hidden, ffn, 256, 210, (209,))
+    layer, staged = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows, down_type=strix.TYPE_Q6_K) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(norm or torch.float32)
+    scale = torch.rand((hidden,), device="cuda", generator=gen)
+    for displaced in (0, 60):
+        strix.lib().mi355_debug_early_route_perturb(displaced)
+        try:
+            y, ids, w, scores = layer.run_layer(x, router, norm=(scale, 1e-6) if norm else None)
+            torch.cuda.synchronize()
+        finally:
+            strix.lib().mi355_debug_early_route_perturb(0)
+        rows32 = strix.rmsnorm_f32(x.to(torch.float32), scale, 1e-6) if norm else x
+        if norm:
+            assert torch.equal(layer.normed[:rows].view(torch.int32), rows32.view(torch.int32))
+        want_ids, want_w, want_scores = strix.route(rows32, router, top_k)
+        assert torch.equal(ids, want_ids) and torch.equal(w.view(torch.int32), want_w.view(torch.int32))
+        assert torch.equal(scores.reshape(-1)[:rows * experts].view(torch.int32), want_scores.reshape(-1).view(torch.int32))
+        assert torch.equal(y.view(torch.int32), staged.run(rows32, want_ids, want_w).view(torch.int32)) and int(layer.status[:rows].sum()) == 0
