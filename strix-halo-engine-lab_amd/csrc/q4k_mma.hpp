@@ -79,7 +79,8 @@ __device__ __forceinline__ uint64_t mma_scalar(uint64_t v) {
     return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32)))) << 32 |
            static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v)));
 }
-// the same for the lanes of `lanes` only (every lane of the wavefront is active around it)
+// the same for the lanes of `lanes` only, at least one. Every lane of the wavefront is active around it: the kernels run whole wavefronts,
+// and no copy stands behind a condition on the lane. (A copy without a lane may not be counted as an operation in flight.)
 __device__ __forceinline__ void mma_copy16_lanes(const uint8_t* src, lds_u8* lds_at, uint64_t lanes) {
     const uint32_t at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds_at)));
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1"
@@ -359,9 +360,10 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
                                         uint32_t tiles, uint32_t nacts, Rows rows, Emit emit) {
     constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<FMT, NAL, NM>(), SLOT = mma_slot_bytes<FMT, NAL, NM>();
     constexpr uint32_t CW = mma_weight_copies<FMT>(), PIECES = mma_pieces<FMT>(), PITCH = mma_pitch<FMT>(), BYTES = mma_block_bytes<FMT>();
-    // Every wavefront issues PERW copies a stage, some of them for no lane (the rest of the last four; the ones that the first stage starts
-    // early or late): no branches on the wavefront's number, one count to wait for.
-    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = CW * NM;
+    // In the ring every wavefront issues PERW copies a stage - past the last one it copies the last one's first piece again, the same bytes to
+    // the same place - so there are no branches on the wavefront's number and one count to wait for. The run's first stages are issued in
+    // two parts of as many copies as a wavefront has there, and awaited whole.
+    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = CW * NM, WEIGHTS_LAST = WEIGHTS / 4U;        // (weight copies of wavefront 3)
     constexpr uint32_t XTEAM = 4U * NAL * 64U;                                                  // floats one team exchanges per group
     static_assert(DEPTH >= 2 && DEPTH <= 4, "ring depth");
     static_assert(TEAMS == 1 || (NM == 1 && NAL <= 8 && FMT == kMmaQ4K), "stage teams serve one matrix, every result register");
@@ -399,8 +401,8 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         } else {
             src[k] = nullptr;
             step[k] = 32U * TEAMS;
-            lands[k] = mma_table_at<FMT, NAL, NM>() + 1024U * (c - WEIGHTS - CC);
-            lanes[k] = c >= TOTAL ? 0ULL : ACTS >= 16U ? ~0ULL : (1ULL << (4U * ACTS)) - 1ULL;
+            lands[k] = mma_table_at<FMT, NAL, NM>() + 1024U * ((c < TOTAL ? c : TOTAL - 1U) - WEIGHTS - CC);
+            lanes[k] = c >= TOTAL ? 1ULL : ACTS >= 16U ? ~0ULL : (1ULL << (4U * ACTS)) - 1ULL;
         }
     }
     const size_t next_tile = kMmaRows * row_stride - BYTES * static_cast<size_t>(stages);       // from a tile's end to the next one's start
@@ -410,12 +412,12 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         constexpr int part = decltype(part_constant)::value;
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
-            const bool mine = part == 0 || (4U * k + p < WEIGHTS) == (part == 1);
+            if (part != 0 && (4U * k + p < WEIGHTS) != (part == 1)) continue;
             const uint8_t* from = src[k];
             if (FMT == kMmaQ6K && 4U * k + p < WEIGHTS) from = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(from) & ~static_cast<uintptr_t>(15)) + piece_at[k];
             if (part == 0 && k == 0U) mma_copy16(from, slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
-            else mma_copy16_lanes(from, slot + lands[k], mine ? lanes[k] : 0ULL);
-            src[k] += mine ? step[k] : 0U;
+            else mma_copy16_lanes(from, slot + lands[k], lanes[k]);
+            src[k] += step[k];
         }
         if (TEAMS == 1 && ++issue_stage == stages) {
             issue_stage = 0;
@@ -432,7 +434,10 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         for (uint32_t s = 0; s < first; ++s) start(std::integral_constant<int, 1>{}, slot_of(s));
     };
     const auto row_of_codes = [&](uint32_t k) { return (64U * (4U * k + p - WEIGHTS) + lane) >> 4; };                            // of the lane's 16 bytes
-    const auto row_of_table = [&](uint32_t k) { return (16U * (4U * k + p - WEIGHTS - CC) + (lane >> 2)) & (ACTS - 1U); };
+    const auto row_of_table = [&](uint32_t k) {
+        const uint32_t c = 4U * k + p < TOTAL ? 4U * k + p : TOTAL - 1U;
+        return (16U * (c - WEIGHTS - CC) + (lane >> 2)) & (ACTS - 1U);
+    };
     const auto set_rows = [&](auto codes_of, auto table_of) {
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
@@ -440,7 +445,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             if (c >= WEIGHTS && c < WEIGHTS + CC) {
                 const uint32_t a = row_of_codes(k);
                 src[k] = codes_of(a) + 16U * (((lane & 15U) - a) & 15U) + 256U * team;
-            } else if (c >= WEIGHTS + CC && c < TOTAL) {
+            } else if (c >= WEIGHTS + CC) {
                 const uint32_t q = lane & 3U;
                 src[k] = table_of(row_of_table(k), q < 2U) + 16U * (q & 1U) + 32U * team;
             }
@@ -454,8 +459,8 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             // (the words land in LDS like everything else: a register that a load in flight writes could be copied before it does)
             mma_copy4_lanes(rows.word(lane < nacts ? lane : 0U), rows.slot, (1ULL << ACTS) - 1ULL);
             start_weights();
-            if (DEPTH > 2 && first == DEPTH - 1U) mma_wait<PERW * (DEPTH - 1)>();
-            else mma_wait<PERW>();
+            if (DEPTH > 2 && first == DEPTH - 1U) mma_wait<WEIGHTS_LAST * (DEPTH - 1)>();
+            else mma_wait<WEIGHTS_LAST>();
             if (lane < ACTS) rows.put(lane, nacts, rows.slot[lane]);
         } else start_weights();
         mma_barrier();
@@ -556,10 +561,8 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         issue_slot = issue_slot + 1U == DEPTH ? 0U : issue_slot + 1U;
     };
     for (uint32_t g = 0; g < total; ++g) {
-        if (g < my_total) {
-            const uint32_t ahead = issued - 1U - g;              // this wavefront's stages started after its stage of group g
-            mma_wait_n<PERW>(ahead);
-        }
+        // this wavefront's stages started after its stage of group g (the first stages' copies are not PERW each: all of them before the first)
+        if (g < my_total) mma_wait_n<PERW>(g == 0U ? 0U : issued - 1U - g);
         mma_barrier();         // every copy of group g is in, the slots of group g - 1 are free, its exchanged terms are written
         // The values of the tile before leave in its successor's first stage. They are stores, which the counted waits count too: before
         // the stage's copies they delay those a little, behind them the next wait would wait for copies that it does not need -
