@@ -348,14 +348,17 @@ template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OU
 //   rows.word(a): address of a word that names activation row a (its place in the plan's order); rows.put(a, nacts, word): leaves the row's
 //   addresses in rows.at. Wavefront 3 asks for the words first, then every wavefront starts the weights of the first stages, so the
 //   look-up is in flight beside them. Rows::kDirect: the addresses need no look-up (rows.codes / rows.table), every wavefront works its
-//   own out and the row table serves the emitter only.
+//   own out and starts whole stages, so the first product waits for the first stage only; the row table serves the emitter, or (no kPut)
+//   nobody.
+//   RUNS: several tiles (else one: none of a run's bookkeeping; gate and up of a dense block, 27648 x 5120, 8 rows: 32.4 -> 31.9 us, and 33.4 with
+//   the weights of both first stages in front of the codes and the row table written in front of the first product).
 //
 // TEAMS > 1 (a matrix of few, long rows gives few workgroups, each with K / 256 dependent stages; one tile a run): TEAMS x 4 wavefronts;
 // team t takes super-blocks t, TEAMS + t, ... of the same 32 rows, so TEAMS stages are in the pipes at once. The chain order is
 // kept by team 0, which adds the terms of every super-block in ascending order: its own from registers, the other teams'
 // from an LDS exchange buffer, one stage group behind (the group's barrier publishes them).
 // Every wavefront of the workgroup calls this; ring, row table and `red` are free again when it returns.
-template <int FMT, int NAL, int DEPTH, int TEAMS, int NM, class Rows, class Emit>
+template <int FMT, int NAL, int DEPTH, int TEAMS, int NM, bool RUNS, class Rows, class Emit>
 __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* red, const uint8_t* const (&wrows)[NM], size_t row_stride, uint32_t stages,
                                         uint32_t tiles, uint32_t nacts, Rows rows, Emit emit) {
     constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<FMT, NAL, NM>(), SLOT = mma_slot_bytes<FMT, NAL, NM>();
@@ -373,7 +376,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = wave & 3U, team = wave >> 2;
     const uint32_t groups = (stages + TEAMS - 1U) / TEAMS;                                     // of a tile
     const uint32_t my_groups = team < stages - (groups - 1U) * TEAMS ? groups : groups - 1U;   // groups in which this team has a super-block
-    const uint32_t total = TEAMS == 1 ? groups * tiles : groups, my_total = TEAMS == 1 ? total : my_groups;
+    const uint32_t total = RUNS ? groups * tiles : groups, my_total = TEAMS == 1 ? total : my_groups;
     const uint32_t nv = (nacts + 1U) / 2U;
 
     // ---- this wavefront's copies of a stage, copy c = 4k + p: CW per matrix (the pieces of 16 bytes of a row, rows PITCH apart; the
@@ -419,7 +422,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             else mma_copy16_lanes(from, slot + lands[k], lanes[k]);
             src[k] += step[k];
         }
-        if (TEAMS == 1 && ++issue_stage == stages) {
+        if (RUNS && ++issue_stage == stages) {
             issue_stage = 0;
 #pragma unroll
             for (uint32_t k = 0; k < PERW; ++k) {
@@ -452,7 +455,6 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         }
     };
     if constexpr (Rows::kDirect) {
-        start_weights();
         set_rows([&](uint32_t a) { return rows.codes(a < nacts ? a : 0U); }, [&](uint32_t a, bool deltas) { return rows.table(a < nacts ? a : 0U, deltas); });
     } else {
         if (wave == 3U) {
@@ -553,22 +555,22 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
 
     // ---- the ring of stage groups
     issue_stage = 0;
-    for (; issued < first; ++issued) start(std::integral_constant<int, 2>{}, slot_of(issued));
-    if (Rows::kDirect && wave == 3U && lane < ACTS) rows.put(lane, nacts, 0U);       // (first read behind the first stage's barrier)
+    for (; issued < first; ++issued) start(std::integral_constant<int, Rows::kDirect ? 0 : 2>{}, slot_of(issued));
+    if (Rows::kDirect && Rows::kPut && wave == 3U && lane < ACTS) rows.put(lane, nacts, 0U);       // (first read behind the first stage's barrier)
     uint32_t issue_slot = DEPTH - 1U, compute_slot = 0, stage = 0, tile = 0;
     const auto issue = [&]() {
         if (issued < my_total) { start(std::integral_constant<int, 0>{}, slot_of(issue_slot)); ++issued; }
         issue_slot = issue_slot + 1U == DEPTH ? 0U : issue_slot + 1U;
     };
     for (uint32_t g = 0; g < total; ++g) {
-        // this wavefront's stages started after its stage of group g (the first stages' copies are not PERW each: all of them before the first)
-        if (g < my_total) mma_wait_n<PERW>(g == 0U ? 0U : issued - 1U - g);
+        // this wavefront's stages started after its stage of group g (first stages in two parts are not PERW copies each: all of them before the first)
+        if (g < my_total) mma_wait_n<PERW>(!Rows::kDirect && g == 0U ? 0U : issued - 1U - g);
         mma_barrier();         // every copy of group g is in, the slots of group g - 1 are free, its exchanged terms are written
         // The values of the tile before leave in its successor's first stage. They are stores, which the counted waits count too: before
         // the stage's copies they delay those a little, behind them the next wait would wait for copies that it does not need -
         // except in a ring of two slots, whose every wait is for everything.
         if (DEPTH == 2) issue();
-        if (TEAMS == 1 && stage == 0U && g != 0U) {
+        if (RUNS && stage == 0U && g != 0U) {
             emit_tile(tile - 1U);
             if (stages == 1U) mma_barrier();                     // (the next values are written in this stage)
         }
@@ -577,7 +579,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         if (g < my_total) {
             const lds_u8* slot = ring + SLOT * (compute_slot * TEAMS + team);
             float term[NM][NAL];
-            if constexpr (FMT != kMmaQ4K && FMT != kMmaQ5K) mma_stage_other<FMT, NAL>(slot, o, p, stage, acc[0]);
+            if constexpr (FMT != kMmaQ4K && FMT != kMmaQ5K) mma_stage_other<FMT, NAL>(slot, o, p, RUNS ? stage : g, acc[0]);
             else if constexpr (mma_halves<NAL>()) {
                 if (p < 2U) mma_stage_terms_halves<FMT, NAL, NM, false>(slot, o, p, term);
                 else mma_stage_terms_halves<FMT, NAL, NM, true>(slot, o, p, term);
@@ -606,16 +608,19 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             }
         }
         compute_slot = compute_slot + 1U == DEPTH ? 0U : compute_slot + 1U;
-        if (TEAMS == 1 && ++stage == stages) {
+        if (RUNS && ++stage == stages) {
             stage = 0;
             ++tile;
             leave();
             clear();
         }
     }
-    mma_barrier();             // the last values (TEAMS > 1: the last exchanged terms) are written; no copy is in flight
-    if (TEAMS > 1) {
-        if (team == 0U) { fold(groups - 1U); leave(); }
+    if (RUNS || TEAMS > 1) mma_barrier();      // the last values (TEAMS > 1: the last exchanged terms) are written; no copy is in flight
+    if (!RUNS) {
+        if (team == 0U) {
+            if (TEAMS > 1) fold(groups - 1U);
+            leave();
+        }
         mma_barrier();
         if (team == 0U) emit_tile(0U);
     } else emit_tile(tiles - 1U);

@@ -39,10 +39,10 @@ __device__ __forceinline__ MmaItem mma_item(const MmaArgs& k, uint32_t width) {
 // The rows c0 .. c0 + n of the plan's order (or of a dense batch), as mma_run asks for them; put_addresses(args, a, i) resolves every address
 // of row a, assignment i, once, so that nothing else of the kernel does. img: the A8 image the rows are read from. DIRECT: a dense batch
 // over one image per row at a stride, which needs no look-up - an instance of its own, because the strides and bases held for it cost
-// the planned batches 1.5 % (dense 27648 x 5120, 8 rows: 86.5 -> 84.6 us).
-template <bool DIRECT, class Put>
+// the planned batches 1.5 % (dense 27648 x 5120, 8 rows: 86.5 -> 84.6 us). PUT: the emitter reads the row table.
+template <bool DIRECT, bool PUT, class Put>
 struct MmaRowsOf {
-    static constexpr bool kDirect = DIRECT;
+    static constexpr bool kDirect = DIRECT, kPut = PUT;
     uint32_t c0;
     const A8Image& img;
     uint32_t dense;
@@ -96,8 +96,8 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
             at[4U * ACTS + a] = address(r.h_deltas_of(i));
             at[5U * ACTS + a] = address(r.h_sums_of(i));
         };
-        const MmaRowsOf<DIRECT, decltype(put)> rows{c0, k.r.in, k.l.dense_rows, at, slot, put};
-        mma_run<FMT, NAL, DEPTH, 1, 2>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, n, rows,
+        const MmaRowsOf<DIRECT, true, decltype(put)> rows{c0, k.r.in, k.l.dense_rows, at, slot, put};
+        mma_run<FMT, NAL, DEPTH, 1, 2, true>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, n, rows,
                                   [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[2]) {
             const uint32_t j = lane & 31U, h = lane >> 5;
             const MmaArgs& args = mma_args();
@@ -170,13 +170,16 @@ __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
             at[2U * ACTS + a] = address(img.sums_of(from));
             at[3U * ACTS + a] = GATE_UP ? address(r.inter_of(blockIdx.z ? r.up_out : r.gate_out, i)) : address(r.rawdots_of(i, args.w.hidden));
         };
-        const MmaRowsOf<DIRECT, decltype(put)> rows{c0, GATE_UP ? k.r.in : k.r.h, k.l.dense_rows, at, slot, put};
-        mma_run<FMT, NAL, DEPTH, TEAMS, 1>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride, (GATE_UP ? k.w.hidden : k.w.ffn) / 256U,
+        const MmaRowsOf<DIRECT, !DIRECT, decltype(put)> rows{c0, GATE_UP ? k.r.in : k.r.h, k.l.dense_rows, at, slot, put};
+        mma_run<FMT, NAL, DEPTH, TEAMS, 1, TEAMS == 1 && !GATE_UP>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride, (GATE_UP ? k.w.hidden : k.w.ffn) / 256U,
                                       tiles, n, rows, [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[1]) {
             const uint32_t a = 2U * v + (lane >> 5), at_out = (tile0 + tile) * kMmaRows + (lane & 31U);
             if (a >= n) return;
-            reinterpret_cast<float*>(at[3U * ACTS + a])[at_out] = value[0];
-            if (!GATE_UP && k.r.top1_form) mma_args().r.publish_top1(slot[a], at_out, value[0]);      // (top-1: assignment = row)
+            // (the rows of a dense batch: assignment = row, at a stride; the argument block read again at a workgroup's end is one way to memory more)
+            float* const out = !DIRECT ? reinterpret_cast<float*>(at[3U * ACTS + a])
+                               : GATE_UP ? k.r.inter_of(blockIdx.z ? k.r.up_out : k.r.gate_out, c0 + a) : k.r.rawdots_of(c0 + a, k.w.hidden);
+            out[at_out] = value[0];
+            if (!GATE_UP && k.r.top1_form) (DIRECT ? k.r : mma_args().r).publish_top1(DIRECT ? c0 + a : slot[a], at_out, value[0]);      // (top-1: assignment = row)
         });
     }
 }
