@@ -1055,19 +1055,28 @@ __global__ __launch_bounds__(256) void merge_kernel(mi355_moe_weights w, RowsK r
 }
 
 constexpr uint32_t kDownMergeSlots = 8;        // top_k bound: 8 waves x 2 ring slots fill the LDS of a compute unit
-// The job word of a down + combine launch, asked for at its start. A batch planned from early routes (r.awords): the front launch left its
-// non-finite flags per assignment; every workgroup folds them to the same job word, the first workgroup of a row publishes its row's.
-struct DownJob { uint32_t job, word[2]; };
+// What a down + combine launch looks up at its start, in this order and without a branch between the requests: its item, the job word and what
+// the fold needs. The sweep waits for the item; asked for behind the others, or behind branches whose arguments are fetched one block after
+// the other, it stood a way to memory further back. The launch, fold behind the barrier by one thread | requests in front of the item |
+// behind it: Q4_K, hidden 3072 / ffn 768 / 64 experts top-8, 1, 4 rows 5.8, 12.4 | 6.1, 13.1 | 6.1, 12.6 us, hidden 4096 / ffn 1280, top-4, 8
+// rows 26.2 | 24.7 | 23.9; hidden 2048 / ffn 768 / 128 experts top-8, 16 rows, Q6_K 40.4 | 40.8 | 39.4, Q8_0 38.2 | 36.8 | 36.7, Q5_1 30.2 | 31.0 | 29.4.
+//
+// the item of (row, slot): the fused router plans one per assignment, in assignment order
+__device__ __forceinline__ WorkItem slot_item(const mi355_moe_weights& w, const RowsK& r, uint32_t assignments, uint32_t a) {
+    const uint4 item = *reinterpret_cast<const uint4*>(r.plan + plan_items_at(w.experts, assignments) + 4U * a);
+    __builtin_amdgcn_sched_barrier(0);
+    return {item.x, item.y, item.z, item.w};
+}
+// The job word. A batch planned from early routes (r.awords): the front launch left its non-finite flags per assignment; every workgroup
+// folds them to the same job word, the first workgroup of a row publishes its row's.
+struct DownJob { uint32_t word[2]; };
 __device__ __forceinline__ DownJob down_job_request(const RowsK& r, uint32_t assignments, uint32_t lane) {
-    DownJob d{0U, {0U, 0U}};
-    if (r.awords) {
-        if (lane < assignments) d.word[0] = r.awords[lane];
-        if (lane + 64U < assignments) d.word[1] = r.awords[lane + 64U];
-    } else d.job = *r.job_status;
-    return d;
+    const uint32_t* const words = r.awords ? r.awords : r.job_status;
+    const uint32_t last = r.awords ? assignments - 1U : 0U;
+    return DownJob{{words[lane < last ? lane : last], words[lane + 64U < last ? lane + 64U : last]}};       // (past the last one: the last one again)
 }
 __device__ __forceinline__ uint32_t down_job(const DownJob& d, const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t wave, uint32_t lane) {
-    if (!r.awords) return d.job;
+    if (!r.awords) return __builtin_amdgcn_readfirstlane(d.word[0]);
     const uint32_t job = (__ballot(d.word[0] >> 31) | __ballot(d.word[1] >> 31)) ? static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION) : 0U;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) r.plan[kPlanLinesAt + kLinesEpoch] += 1U;      // this call's epoch is spent
     if (job && blockIdx.x == 0 && wave == 0) {
@@ -1081,19 +1090,17 @@ __device__ __forceinline__ uint32_t down_job(const DownJob& d, const mi355_moe_w
     }
     return job;
 }
-// What the fold of a row's slots needs beside their values, asked for at the start of the launch by the wavefront that folds (lane k:
-// weight and expert of slot k; the row's status as the launches before left it; the base of column o): behind the barrier it was up to
-// four ways to memory in a row, by one thread.
+// What the fold of a row's slots needs beside their values (lane k: weight and expert of slot k; the row's status as the launches before left
+// it, by a vector load; the base of column o - without one any word, which nothing reads).
 struct SlotFold { float weight, base; uint32_t route, status; };
-__device__ __forceinline__ SlotFold slot_fold_request(const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t o, uint32_t form, uint32_t wave, uint32_t lane) {
-    SlotFold f{0.0F, 0.0F, 0xffffffffU, 0U};
-    if (wave != 0) return f;
-    f.status = *r.status_of(row);
-    if (lane < w.top_k) {
-        f.weight = r.route_weights_of(row)[lane];
-        if (form == MI355_COMBINE_MULADD_ASCENDING_EXPERT) f.route = r.routes_of(row)[lane];
-    }
-    if (r.base) f.base = r.base_of(row)[o];
+__device__ __forceinline__ SlotFold slot_fold_request(const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t o, uint32_t lane) {
+    const uint32_t k = lane < w.top_k ? lane : 0U;
+    const float* const base = r.base ? r.base_of(row) + o : r.route_weights_of(row);
+    SlotFold f;
+    f.status = __hip_atomic_load(r.status_of(row), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    f.weight = r.route_weights_of(row)[k];
+    f.route = r.routes_of(row)[k];
+    f.base = *base;
     return f;
 }
 // The row's value of one column, as merge_kernel folds it (every lane of the wavefront takes part). Fail closed: a row flagged by an
@@ -1139,10 +1146,10 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
     __shared__ __attribute__((aligned(16))) uint8_t ring_odd[kDownMergeSlots][slot_bytes(1)];
     __shared__ float slot_value[kDownMergeSlots][64];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, row = blockIdx.y, o = blockIdx.x * 64U + lane;
-    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item: one round trip, not two)
-    const SlotFold fold = slot_fold_request(w, r, row, o, form, wave, lane);
     const uint32_t a = row * w.top_k + wave;
-    const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), a);
+    const WorkItem item = slot_item(w, r, assignments, a);
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item: one round trip, not two)
+    const SlotFold fold = slot_fold_request(w, r, row, o, lane);
     const uint32_t e = __builtin_amdgcn_readfirstlane(item.e), begin = __builtin_amdgcn_readfirstlane(item.begin), end = __builtin_amdgcn_readfirstlane(item.end);
     if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
@@ -1170,7 +1177,7 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
 // down_merge_kernel for dense rows of at most four super-blocks (down_row_stride = B * 144): the 64 rows of a column block stream as B
 // contiguous stages of 1 KB pieces instead of B stages of 64 separate 144-byte blocks (a read-only launch of this shape moves the
 // same bytes in 11.8 us against 14.4 us), the block terms meet in LDS in block order and lane = row adds them in ascending order.
-// (Job word and fold written out: through the functions above, 1, 8, 16 rows of hidden 2048 / ffn 768 27.7, 45.9, 73.5 -> 28.2, 46.2, 73.9 us.)
+// (Fold behind the barrier: asked for at the start, in front of the item, 1, 8, 16 rows of hidden 2048 / ffn 768 27.7, 45.9, 73.5 -> 28.2, 46.2, 73.9 us.)
 template <int B>
 __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     // (the two ring slots are separate LDS objects, as in down_merge_kernel)
@@ -1257,10 +1264,10 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_quad_kernel(m
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i) slots[i] = ring[i];
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
-    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
-    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
     const uint32_t a = row * w.top_k + wave;
-    const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), a);
+    const WorkItem item = slot_item(w, r, assignments, a);
+    const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
+    const SlotFold fold = slot_fold_request(w, r, row, oc, lane);
     if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
@@ -1295,9 +1302,9 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o0 = blockIdx.x * 16U, o = o0 + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const WorkItem item = slot_item(w, r, assignments, row * w.top_k + wave);
     const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
-    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
-    const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
+    const SlotFold fold = slot_fold_request(w, r, row, oc, lane);
     if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
@@ -1386,9 +1393,9 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, half = p >> 1, odd = p & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const WorkItem item = slot_item(w, r, assignments, row * w.top_k + wave);
     const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
-    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
-    const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
+    const SlotFold fold = slot_fold_request(w, r, row, oc, lane);
     if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
@@ -1454,9 +1461,9 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q8_0_kernel(m
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, odd = j & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
+    const WorkItem item = slot_item(w, r, assignments, row * w.top_k + wave);
     const DownJob job = down_job_request(r, assignments, lane);                // (requested together with the item)
-    const SlotFold fold = slot_fold_request(w, r, row, oc, form, wave, lane);
-    const WorkItem item = work_item(w, r, plan_items_at(w.experts, assignments), row * w.top_k + wave);
+    const SlotFold fold = slot_fold_request(w, r, row, oc, lane);
     if (down_job(job, w, r, row, wave, lane) & MI355_STATUS_NONFINITE_PROJECTION) return;                       // the whole job: no down rows, nothing published
     float value = 0.0F;
     if (item.begin != item.end) {                                              // (an invalid route has no item: its row is flagged)
