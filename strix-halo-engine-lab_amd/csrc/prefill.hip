@@ -51,12 +51,19 @@ namespace {
 // 128; it has three times the workgroups in flight. Measured (wide, four waves), rows per expert on average and rounds of the wide form's
 // gate / up workgroups beside them: 8.5, 5.8 256, 199 us; 12.3, 13 185, 168; 15, 8.4 776, 707; 21, 3.5 195, 178; 22, 14 965, 1028;
 // 25, 9 867, 894; 37, 7.8 879, 961; 40, 3.3 435, 419; 46, 1.8 414, 380; 50, 4.2 270, 275; 56, 4.0 194, 178; 45, 18 1847, 2312.
-// Q8_0 rows are twice as wide, and the down rows are swept twice: 4, 3.2 182, 159; 12.5, 3.3 242, 230; 9.4, 3.2 414, 427; 15, 10 1220, 1364;
-// 21, 3.5 257, 285; 25, 3.6 538, 615; 37, 3.9 325, 369; 12.5, 0.3 79, 44; 50, 0.4 88, 48.
+// Q8_0 rows are twice as wide, and the down rows are swept twice: up to 13 rows per expert, while rows times rounds are few, or the rows of an
+// expert, or the rows short, so that a workgroup's start is what it waits for. Measured the same way, hidden 2048 and more:
+// 4, 3.1 175, 148; 9.4, 3.2 467, 451; 9.4, 3.2 236, 225; 13, 3.3 247, 239; 6, 4.2 523, 449; 9.4, 4.3 536, 520; 13, 4.4 567, 645; 5, 5.2 316, 285;
+// 9, 5.4 340, 348; 12, 5.4 578, 656; 7, 6.3 363, 351; 9, 6.4 384, 397; 3.8, 7.7 910, 886; 6, 7.9 1055, 1107; 12.5, 8.2 1238, 1348; 2, 16 479, 420;
+// 4, 17 535, 509; 6, 17 566, 596; 9, 17 579, 694; hidden 1280, 13, 4.1 166, 128; hidden 1024, 13, 6.2 179, 148. Past 13 rows per expert: 21, 3.5 257, 285; 25, 3.6
+// 538, 615; 37, 3.9 325, 369; in one round 25, 0.9 123, 95; 37, 1.0 128, 120; 50, 0.7 134, 119.
 bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
-    const uint64_t e = wv.experts, a = assignments;
-    const bool q8 = wv.gate_type == MI355_TYPE_Q8_0 || wv.down_type == MI355_TYPE_Q8_0;
-    return a <= (q8 ? 13ULL : 16ULL) * e || (a <= 56ULL * e && (128ULL * e + a) * wv.ffn <= (q8 ? 1ULL : 4ULL) * compute_units() * 128U * 128U);
+    const uint64_t e = wv.experts, a = assignments, work = (128ULL * e + a) * wv.ffn, round = compute_units() * 128ULL * 128U;
+    if (wv.gate_type == MI355_TYPE_Q8_0 || wv.down_type == MI355_TYPE_Q8_0) {
+        const bool starts = a * work <= 51ULL * e * round || 2ULL * a <= 9ULL * e || wv.hidden <= 1280U;
+        return (a <= 13ULL * e && starts) || (a <= 56ULL * e && work <= round);
+    }
+    return a <= 16ULL * e || (a <= 56ULL * e && work <= 4ULL * round);
 }
 }  // namespace
 
