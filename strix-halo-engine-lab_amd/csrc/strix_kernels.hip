@@ -1648,6 +1648,11 @@ constexpr uint32_t kMmaItemRows = 128;
 inline bool q4k_both(const mi355_moe_weights& w) { return w.gate_type == MI355_TYPE_Q4_K && w.down_type == MI355_TYPE_Q4_K; }
 // down rows of whole stages of 256 weights (Q8_0 and Q5_1 rows may end on half a stage)
 inline bool mma_down_rows(const mi355_moe_weights& w) { return w.ffn % 256U == 0 && w.down_type != MI355_TYPE_Q5_K; }
+// factors and sums that the sweeps' copies of 16 bytes take (a dense bundle is admitted with any of four; the vector-ALU sweeps, which read them
+// word by word, serve items of any length)
+inline bool mma_image(const A8Image& img) {
+    return !img.table && aligned(img.deltas, 16) && aligned(img.sums, 16) && img.deltas_rs % 16U == 0 && img.sums_rs % 16U == 0;
+}
 inline uint32_t mma_grouped_split(const mi355_moe_weights& w, uint32_t rows) {
     if ((w.gate_type != MI355_TYPE_Q4_K && w.gate_type != MI355_TYPE_Q5_K) || w.experts == 1U) return 0U;
     if (rows <= kFusedMaxRows) return !quad_sweep(w, rows) && large_expert(w) ? 2U : 0U;
@@ -1685,7 +1690,7 @@ inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows) {
 // sweeps serve it whatever its size (hidden 2048 / ffn 768 / 128 experts top-8 and one more, 5 rows, Q6_K | Q8_0 | Q4_K down: 88 | 93 | 86 -> 70 |
 // 71 | 65 us; 1 row 53 | 54 | 52 -> 50 | 50 | 49; Q5_K gate / up and Q5_1 down 83 -> 77, 1 row 50 -> 51).
 inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t umax, hipStream_t st, bool grouped = false) {
-    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && (grouped || split))
+    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && mma_image(r.in) && (grouped || split))
         return launch_mma_project(w, r, rows, 0, umax, grouped ? 4U : mma_sweep_rows(w, rows, split), st);
     if (w.gate_type == MI355_TYPE_Q5_K) {
         // the deepest ring at which every workgroup of the launch is resident (4 waves x DEPTH x 4 KB each)
@@ -1694,7 +1699,7 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
         else project_q5k_kernel<2><<<dim3(w.ffn / 32U, umax), 256, 0, st>>>(w, r, rows * w.top_k);
         return;
     }
-    if (quad_sweep(w, rows)) {
+    if (!grouped && quad_sweep(w, rows)) {
         const uint32_t items = rows * w.top_k;
         if (items <= 16U) project_quad_kernel<4><<<dim3(w.ffn / 32U, items), 256, 0, st>>>(w, r, items);
         else project_quad_kernel<2><<<dim3(w.ffn / 32U, items), 256, 0, st>>>(w, r, items);
@@ -1711,7 +1716,7 @@ inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t 
 }
 // Returns true when the launch also published the output rows (a dense top-1 job with r.top1_form set: the two dense sweeps).
 inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t umax, hipStream_t st, bool grouped = false) {
-    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && mma_down_rows(w) && (grouped || split)) {
+    if (const uint32_t split = mma_grouped_split(w, rows); r.plan && mma_down_rows(w) && mma_image(r.h) && (grouped || split)) {
         RowsK plain = r;
         plain.top1_form = 0;
         launch_mma_down(w, plain, rows, 0, umax, grouped ? 4U : mma_sweep_rows(w, rows, split), st);
@@ -1721,7 +1726,7 @@ inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t row
         const uint32_t assignments = rows * w.top_k, items_at = plan_items_at(w.experts, assignments), order_at = plan_order_at(w.experts);
         const dim3 grid(w.hidden / kDownGroupsRows, umax);
         // Q5_1 rows of whole super-blocks at 16-byte aligned addresses stream through a copy ring (its depth by residency)
-        if (w.down_type == MI355_TYPE_Q5_1 && w.ffn % 256U == 0 && w.down_row_stride % 16U == 0 && w.down_expert_stride % 16U == 0) {
+        if (w.down_type == MI355_TYPE_Q5_1 && w.ffn % 256U == 0 && w.down_row_stride % 16U == 0 && w.down_expert_stride % 16U == 0 && mma_image(r.h)) {
             if (static_cast<uint64_t>(grid.x) * grid.y * 4U <= resident_waves(4U * group_slot_bytes())) down_q51_ring_kernel<4><<<grid, 256, 0, st>>>(w, r, assignments, items_at, order_at);
             else down_q51_ring_kernel<2><<<grid, 256, 0, st>>>(w, r, assignments, items_at, order_at);
         }
@@ -1730,7 +1735,7 @@ inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t row
         else launch_down_q6k(w, r, grid, assignments, items_at, order_at, st);
         return false;
     }
-    if (quad_sweep(w, rows)) {
+    if (!grouped && quad_sweep(w, rows)) {
         const uint32_t items = rows * w.top_k;
         if (items <= 16U) down_quad_kernel<4><<<dim3(w.hidden / 64U, items), 256, 0, st>>>(w, r, items);
         else down_quad_kernel<2><<<dim3(w.hidden / 64U, items), 256, 0, st>>>(w, r, items);

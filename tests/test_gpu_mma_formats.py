@@ -48,3 +48,33 @@ def test_batch_equals_pairs_of_rows(strix, rows, hidden, ffn, experts, top_k, ga
 def test_half_a_stage(strix, gate):
     """ffn 384: Q5_1 down rows keep their own sweep, the gate / up rows run here."""
     test_batch_equals_pairs_of_rows(strix, 80, 256, 384, 8, 2, gate, "q5_1")
+
+
+# a dense bundle may hold its factors and code sums at any word, which the sweeps' copies do not take: the same values from the sweeps that
+# read them word by word, over the batch's own plan (items of four, sixteen and more rows, and those of a layer with an always-on expert)
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(17, 256, 256, 64, 4), (60, 256, 512, 16, 4), (150, 512, 512, 8, 2), (14, 4096, 1024, 8, 4)])
+@pytest.mark.parametrize("gate,down", [("q4_k", "q4_k"), ("q4_k", "q6_k"), ("q5_k", "q8_0"), ("q5_k", "q5_1")])
+def test_factors_at_any_word(strix, rows, hidden, ffn, experts, top_k, gate, down):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    g, u, d = blocks(gen, gate, experts * ffn, hidden), blocks(gen, gate, experts * ffn, hidden), blocks(gen, down, experts * hidden, ffn)
+    kinds = dict(gate_type=getattr(strix, "TYPE_" + gate.upper()), down_type=getattr(strix, "TYPE_" + down.upper()))
+
+    def pair(n):
+        layer, moved = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, n, **kinds) for _ in range(2))
+        for name in ("deltas", "sums", "down_deltas", "down_sums"):
+            own = getattr(moved, name)
+            setattr(moved, name, torch.zeros(own.numel() + 1, dtype=own.dtype, device="cuda")[1:].reshape(own.shape))
+            assert getattr(moved, name).data_ptr() % 16 == 4
+        return layer, moved
+
+    x = torch.randn((rows, hidden), device="cuda", generator=gen)
+    ids = torch.rand((rows, experts), device="cuda", generator=gen).topk(top_k, dim=1).indices.to(torch.int32)
+    w = torch.rand((rows, top_k), device="cuda", generator=gen)
+    layer, moved = pair(rows)
+    want = layer.run(x, ids, w)
+    assert torch.equal(moved.run(x, ids, w).view(torch.int32), want.view(torch.int32))
+    assert int(layer.status.sum()) == 0 and int(moved.status.sum()) == 0
+    router = torch.randn((experts - 1, hidden), device="cuda", generator=gen) * 0.02
+    layer, moved = pair(5)
+    want = layer.run_layer(x[:5], router, shared_experts=1)[0]
+    assert torch.equal(moved.run_layer(x[:5], router, shared_experts=1)[0].view(torch.int32), want.view(torch.int32))
