@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from test_gpu_parity import early_choice
+
 pytestmark = pytest.mark.gpu
 
 
@@ -20,6 +22,10 @@ def blocks(gen, rows, width, per, size, scales):
     return w.reshape(rows, -1)
 
 
+# the word of the plan that the down launch of a layer with early routes, and no other, moves on by one
+EPOCH = 672 + 3 * 16 * 32 + 16
+
+
 # eight assignments (the fewest of this form) up to 128 (the most); rows of one and of several stages
 @pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,amount", [(1, 2048, 768, 128, 8, 40), (16, 1024, 512, 32, 8, 40), (7, 512, 256, 24, 5, 300), (4, 768, 1280, 16, 2, 0)])
 @pytest.mark.parametrize("down", ["q6_k", "q8_0", "q5_1"])
@@ -33,11 +39,16 @@ def test_early_routes_equal_staged_launches(strix, rows, hidden, ffn, experts, t
     base = torch.randn((rows, hidden), device="cuda", generator=gen)
     ids, w = strix.route(x, router, top_k)[:2]
 
+    if amount:                     # the displaced early choice is another one in some slots
+        assert int((torch.from_numpy(early_choice(x.cpu().numpy(), router.cpu().numpy(), top_k, amount).astype("int64")) != ids.cpu()).sum()) >= 2
+
     def run(displaced, form, b):
+        epoch = int(layer.plan[EPOCH])
         strix.lib().mi355_debug_early_route_perturb(displaced)
         try:
             y, got, weights, _ = layer.run_layer(x, router, base=b, combine=form)
             torch.cuda.synchronize()
+            assert int(layer.plan[EPOCH]) == epoch + 1
         finally:
             strix.lib().mi355_debug_early_route_perturb(0)
         assert int(layer.status[:rows].sum()) == 0 and torch.equal(got, ids) and torch.equal(weights.view(torch.int32), w.view(torch.int32))
@@ -73,16 +84,20 @@ def test_fp32_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_
     x = torch.randn((rows, hidden), device="cuda", generator=gen).to(norm or torch.float32)
     scale = torch.rand((hidden,), device="cuda", generator=gen)
     for displaced in (0, 60):
+        epoch = int(layer.plan[EPOCH])
         strix.lib().mi355_debug_early_route_perturb(displaced)
         try:
             y, ids, w, scores = layer.run_layer(x, router, norm=(scale, 1e-6) if norm else None)
             torch.cuda.synchronize()
+            assert int(layer.plan[EPOCH]) == epoch + 1
         finally:
             strix.lib().mi355_debug_early_route_perturb(0)
         rows32 = strix.rmsnorm_f32(x.to(torch.float32), scale, 1e-6) if norm else x
         if norm:
             assert torch.equal(layer.normed[:rows].view(torch.int32), rows32.view(torch.int32))
         want_ids, want_w, want_scores = strix.route(rows32, router, top_k)
+        if displaced:
+            assert int((torch.from_numpy(early_choice(rows32.cpu().numpy(), router.cpu().numpy(), top_k, displaced).astype("int64")) != want_ids.cpu()).sum()) >= 2
         assert torch.equal(ids, want_ids) and torch.equal(w.view(torch.int32), want_w.view(torch.int32))
         assert torch.equal(scores.reshape(-1)[:rows * experts].view(torch.int32), want_scores.reshape(-1).view(torch.int32))
         assert torch.equal(y.view(torch.int32), staged.run(rows32, want_ids, want_w).view(torch.int32)) and int(layer.status[:rows].sum()) == 0

@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from test_gpu_parity import PLAN_OFFSETS_AT
+
 pytestmark = pytest.mark.gpu
 
 
@@ -36,6 +38,30 @@ def draw(gen, kind, rows, width):
     return b.reshape(rows, -1), torch.stack(out, -2).reshape(rows, width)
 
 
+def check_down_product(layer, D, rows, hidden, ffn, experts, top_k, ids):
+    """The down rows alone, against double precision on the h that the launch itself read: two fp16 planes, hi and the rest of 22 bits.
+    A value takes ffn / 16 matrix operations per plane and a scaled sum per 32 weights, each rounded within 2^-24 of a partial sum, which is no larger
+    than the value by rms; the errors' signs are independent, so they add up as the square root of their number, and four times that leaves room
+    for the roundings inside an operation. A product without the rest of h, or with a part of it against other weights, is off by more
+    than three times the bound (1.2e-5 of the value at ffn 1280 with Q5_K rows throughout, 2e-4 elsewhere), which is checked here as well."""
+    pad4 = lambda v: (v + 3) & ~3
+    A = rows * top_k
+    plane = 2 * (A + 128) * ffn                                                   # bytes of a plane of [assignments in plan order][ffn]
+    hi, lo = (layer.h_f16[at:at + 2 * A * ffn].view(torch.float16).reshape(A, ffn).to(torch.float64) for at in (0, plane))
+    order_at = PLAN_OFFSETS_AT + pad4(experts + 1) + pad4(experts)
+    order = layer.plan[order_at:order_at + A].long()
+    expert = ids.reshape(-1).long()[order]
+    raw = layer.rawdots.reshape(-1, hidden)[:A].to(torch.float64)[order]
+    bound = 4 * 2.0 ** -24 * (2 * (ffn // 16) + ffn // 32) ** 0.5
+    off, off_hi, size = 0.0, 0.0, 0.0
+    for e in range(experts):
+        at, De = (expert == e).nonzero().squeeze(1), D[e * hidden:(e + 1) * hidden]
+        want = (hi[at] + lo[at]) @ De.T
+        off, off_hi, size = off + float((raw[at] - want).square().sum()), off_hi + float((lo[at] @ De.T).square().sum()), size + float(want.square().sum())
+    assert (off / size) ** 0.5 <= bound, ((off / size) ** 0.5, bound)
+    assert (off_hi / size) ** 0.5 >= 3 * bound, ((off_hi / size) ** 0.5, bound)
+
+
 # rows per expert: one tile of 32 (both forms: few rows, and with three experts nothing else), two, three and four tiles, an item and a bit;
 # K of an odd number of super-blocks and of one
 @pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(9, 256, 256, 3, 2), (40, 768, 512, 2, 1), (130, 512, 256, 1, 1), (190, 1280, 768, 2, 1), (70, 256, 1280, 1, 1),
@@ -50,6 +76,7 @@ def test_against_the_exact_product(strix, rows, hidden, ffn, experts, top_k, gat
     ids = torch.rand((rows, experts), device="cuda", generator=gen).topk(top_k, dim=1).indices.to(torch.int32)
     layer.run_prefill_f16(x, ids, torch.rand((rows, top_k), device="cuda", generator=gen))
     assert int(layer.status[:rows].sum()) == 0
+    check_down_product(layer, D, rows, hidden, ffn, experts, top_k, ids)
     raw = layer.rawdots.reshape(-1, hidden)[:rows * top_k].to(torch.float64)
     flat, X = ids.reshape(-1).long(), x.to(torch.float64)
     for e in range(experts):
