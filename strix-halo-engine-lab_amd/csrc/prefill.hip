@@ -79,12 +79,11 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
     const uint32_t resident = (cus > 8U ? cus : 256U) & ~7U;
     const auto grid_of = [&](uint32_t units, uint32_t each = 1U) { return units < each * resident ? units : each * resident; };
     const bool few = few_rows(wv, a.assignments);
-    a.subs = prefill_split(wv, a.assignments) / 32U;
     const auto launch = [&](auto mode, uint32_t type) {
         constexpr int M = decltype(mode)::value;
         const auto of = [&](auto format) {
             constexpr int F = decltype(format)::value;
-            if (few) prefill_reg_kernel<M, 4, F><<<grid_of(a.subs * a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
+            if (few) prefill_reg_kernel<M, 4, F><<<grid_of(a.units, 3U), 256, 0, st>>>(a, items_at, order_at);
             else prefill_reg_kernel<M, 8, F><<<grid_of(a.units), 512, 0, st>>>(a, items_at, order_at);
         };
         if (type == MI355_TYPE_Q8_0) of(std::integral_constant<int, kRgQ80>{});

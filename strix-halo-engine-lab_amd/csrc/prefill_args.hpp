@@ -37,7 +37,6 @@ struct PrefillArgs {
     float* rawdots;                               // MODE 1: [assignment][hidden]
     const uint32_t* plan; uint32_t experts, assignments;
     uint32_t* status; uint32_t* job_status;
-    uint32_t subs;                                // pieces of 32 rows an item may hold (the four-wave form)
     uint32_t tiles, items, units;                 // feature tiles per item, item bound of the launch, tiles * items rounded up to 8 items
     uint64_t status_rs, rawdots_rs;               // bytes between the rows of status / rawdots; rawdots_rs == 0: dense [assignment][features]
     uint32_t rawdots_bf16;                        // MODE 1: every unweighted output is stored once rounded to bfloat16 (as an fp32 value)

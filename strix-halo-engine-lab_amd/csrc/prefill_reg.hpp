@@ -31,7 +31,7 @@
 // What bounds it: with whole tiles of 128 rows a SIMD takes 38 ns a product (one such product after the other on random operands, out of
 // registers, takes it 20 ns at the clock that the chip's power leaves, with seven vector instructions beside each 26); with few rows
 // the weights' way to the registers. Q5_K and Q8_0 rows, through LDS by loader waves before (layer, top-8): hidden 2048 / ffn 768 / 128
-// experts, 100, 333, 1000, 4000 rows Q5_K 255, 353, 535, 1438 -> 134, 206, 341, 914 us, Q8_0 252, 335, 521, 1468 -> 184, 289, 377, 979;
+// experts, 100, 333, 1000, 4000 rows Q5_K 255, 353, 535, 1438 -> 134, 206, 341, 914 us, Q8_0 252, 335, 521, 1468 -> 184, 257, 348, 979;
 // 4096 rows of hidden 4096 / ffn 2048 / 64 experts 4720 -> 3409, 4994 -> 3830 (Q4_K 2857).
 #pragma once
 #include "device_math.hpp"
@@ -125,8 +125,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     constexpr uint32_t TOKENS = WAVES == 4U ? 32U : 128U;
     static_assert(TOKENS <= 16U * WAVES && TOKENS % (8U * WAVES) == 0, "one sums copy per wave, a token copy of 8 rows per wave and part");
     constexpr bool WHOLE = WAVES == 4U && FMT != kRgQ80;
-    // Q8_0: stages of weights in registers. The wide form has room for two beside its sums (with four, 38 and 110 registers spilled: 1000 rows of
-    // hidden 2048 / ffn 768 / 128 experts 342 -> 435 us).
+    // Q8_0: stages of weights in registers. The wide form has room for two beside its sums (32 registers of the gate / up rows are spilled at a
+    // unit's start and read at its end; with four stages 110, inside the K loop: 1000 rows of hidden 2048 / ffn 768 / 128 experts 342 -> 435 us).
     constexpr uint32_t RING8 = WAVES == 4U ? 4U : 2U;
     constexpr uint32_t BLOCK = FMT == kRgQ5K ? 176U : 144U, QUANTS_AT = FMT == kRgQ5K ? 48U : 16U;          // of a K-quant super-block
     // h enters as fp16 hi + lo. Q4_K: both planes in one sweep of the weights, two products per operand. Q5_K and Q8_0: K is swept twice, lo
@@ -154,18 +154,18 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     const size_t sum_row = pf_sum_row_bytes(a.k);
 
     // Wide: the tiles of an item run on one XCD, whose L2 then holds its token rows. Four waves: few rows per item, whose units differ in
-    // length more than their token rows cost: an item's tiles go round the XCDs (of the items that were made), and where the plan's
-    // items hold more rows than TOKENS (a.subs times as many) the first rows of every item come first.
+    // length more than their token rows cost: an item's tiles go round the XCDs (of the items that were made). An item holds at most
+    // TOKENS rows in either form (prefill_split).
     constexpr bool ROUND = WAVES == 4U;
-    const uint32_t units = ROUND ? a.plan[4] * a.tiles : a.units, subs = ROUND ? a.subs : 1U;
-    for (uint32_t at = blockIdx.x; at < subs * units; at += gridDim.x) {
-    const uint32_t sub = ROUND ? at / units : 0U, unit = at - sub * units, q = unit >> 3;
+    const uint32_t units = ROUND ? a.plan[4] * a.tiles : a.units;
+    for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+    const uint32_t q = unit >> 3;
     const uint32_t item_index = ROUND ? unit / a.tiles : (q / a.tiles) * 8U + (unit & 7U), tile = (ROUND ? unit : q) % a.tiles;
     if (item_index >= a.items) continue;
     const uint4 item = *reinterpret_cast<const uint4*>(a.plan + items_at + 4U * item_index);
-    const uint32_t e = item.x, begin = item.y + sub * TOKENS;
+    const uint32_t e = item.x, begin = item.y;
     if (begin >= item.z) continue;
-    const uint32_t count = item.z - begin < TOKENS ? item.z - begin : TOKENS;
+    const uint32_t count = item.z - begin;
 
     // ---- the lane's weight row
     uint32_t feature;                                  // MODE 0: gate (n31 < 16) / up feature; MODE 1: output column

@@ -26,8 +26,9 @@ template <int FMT, int NAL>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items)));
     constexpr int DEPTH = NAL >= 8 ? 2 : 3;
-    if (FMT == kMmaQ4K && mma_direct(r.in, dense)) q4k_mma_project_kernel<kMmaQ4K, NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
-    else q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    if constexpr (FMT == kMmaQ4K)
+        if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l}); return; }
+    q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
 // rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
@@ -47,8 +48,9 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
     // (Q6_K: a fourth or sixth workgroup on a compute unit is worth more than a third slot: 24 rows of hidden 4096 / ffn 1536 / 64 experts
     // 178.3 -> 176.5 us; Q8_0, 40 rows of hidden 2048 / ffn 768 / 128 experts, 124.4 us with three slots, 126.5 with two)
     constexpr int DEPTH = NAL >= 8 || FMT == kMmaQ6K ? 2 : 3;
-    if (FMT == kMmaQ4K && direct) q4k_mma_down_kernel<kMmaQ4K, NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
-    else q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+    if constexpr (FMT == kMmaQ4K)
+        if (direct) { q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l}); return; }
+    q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
 }
 template <int FMT>
 inline void launch_mma_project_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {

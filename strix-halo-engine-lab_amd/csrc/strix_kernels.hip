@@ -1633,7 +1633,7 @@ inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows);
 inline bool large_expert(const mi355_moe_weights& w) { return 2ULL * w.ffn * (w.hidden / 256U) * kQ4kBlock >= (4ULL << 20); }
 // Routed experts past the decode sizes or of several MB: the plan cuts an expert's rows into items of this
 // many for the matrix-core sweeps (0: the vector-ALU sweeps serve the batch). The sweeps are bound by latency, so the narrow instances
-// (4 or 8 rows: 128 or 151 registers, four or three waves per SIMD) win while an expert holds few rows, and even one row per expert is
+// (4 or 8 rows: 123 or 142 registers, four or three waves per SIMD) win while an expert holds few rows, and even one row per expert is
 // better off here than on the vector-ALU sweep. Layer times, hidden 2048 / ffn 768 / 128 experts top-8, items of 4 rows | of 16 in sweeps of 8 |
 // in sweeps of 16 (vector-ALU sweep, which served up to 4 rows per expert): 17 rows 88 | - | 130 us (109), 28 rows 101 | 114 | 152 (126), 40
 // rows 118 | 126 | 167 (147), 60 rows 141 | 139 | 181 (171), 100 rows 177 | 163 | 189, 200 rows 266 | 220 | 218, 400 rows 445 | 340 | 337; hidden
@@ -1688,7 +1688,8 @@ inline bool quad_sweep(const mi355_moe_weights& w, uint32_t rows) {
 }
 // grouped: the fused router's plan of a decode batch with always-on experts, whose items hold up to four assignments; the narrow matrix-core
 // sweeps serve it whatever its size (hidden 2048 / ffn 768 / 128 experts top-8 and one more, 5 rows, Q6_K | Q8_0 | Q4_K down: 88 | 93 | 86 -> 70 |
-// 71 | 65 us; 1 row 53 | 54 | 52 -> 50 | 50 | 49; Q5_K gate / up and Q5_1 down 83 -> 77, 1 row 50 -> 51).
+// 71 | 65 us; 1 row 53 | 54 | 52 -> 50 | 50 | 49; Q5_K gate / up and Q5_1 down without the norm 1, 2, 5, 16 rows 42.2, 54.0, 75.1, 132.7 -> 41.5,
+// 46.8, 64.2, 115.2).
 inline void launch_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t umax, hipStream_t st, bool grouped = false) {
     if (const uint32_t split = mma_grouped_split(w, rows); r.plan && mma_image(r.in) && (grouped || split))
         return launch_mma_project(w, r, rows, 0, umax, grouped ? 4U : mma_sweep_rows(w, rows, split), st);
@@ -1753,13 +1754,10 @@ inline bool launch_down(const mi355_moe_weights& w, const RowsK& r, uint32_t row
 // expert's weights comes from the last-level cache. A dense matrix: every row shares one sweep.
 inline uint32_t plan_split(const mi355_moe_weights& w, uint32_t rows) {
     if (w.experts == 1U) return 8;
-    if (const uint32_t split = mma_grouped_split(w, rows)) return split;     // items for the matrix-core sweep
-    if (rows > kFusedMaxRows) return 4U;
-    if (quad_sweep(w, rows)) return 1U;       // the 16-rows-per-wavefront sweep serves one assignment per item
-    // decode batches: one item per assignment while an expert's gate + up rows are a few MB (the second sweep of an expert
-    // that two rows chose is a cache hit and the short instruction streams finish sooner); larger experts that the matrix-core sweeps
-    // do not take are swept once for every two rows that chose them (hidden 6144, ffn 1280, 16 rows: 384 -> 351 us)
-    return large_expert(w) ? 2U : 1U;
+    // decode batches on the vector-ALU sweeps: one item per assignment (the second sweep of an expert that two rows chose is a cache hit
+    // while its gate + up rows are a few MB, and the short instruction streams finish sooner)
+    const uint32_t split = mma_grouped_split(w, rows);
+    return split ? split : 1U;
 }
 inline uint32_t item_bound(const mi355_moe_weights& w, uint32_t rows) {
     return plan_item_bound(w.experts, rows * w.top_k, plan_split(w, rows));
@@ -2217,7 +2215,7 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         STRIX_LAUNCHED("moe layer router");
     }
     // the fused router planned one item per routed assignment (and one per four rows of an always-on expert)
-    if (p->shared_experts) {       // items of several rows: the 64-row sweeps
+    if (p->shared_experts) {       // items of up to four rows: the narrow matrix-core sweeps
         if (do_front) {
             launch_project(wv, layer_rows(), rows, items, st, true);
             STRIX_LAUNCHED("moe layer gate / up");

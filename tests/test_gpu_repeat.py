@@ -83,7 +83,7 @@ def test_other_down_formats_repeat_their_bits(strix, down_type):
     assert repeat(lambda: layer.run_layer(x, wr), snap, 300) == 0
 
 
-# the matrix-core prefill (workgroup-shared rings between loader and multiplier waves, a barrier per step)
+# the matrix-core prefill (token rings shared by the workgroup's waves, a barrier per stage)
 @pytest.mark.parametrize("H,I,E,K,T", [(1024, 512, 12, 4, 300), (768, 1280, 5, 2, 150)])
 def test_prefill_f16_repeats_its_bits(strix, H, I, E, K, T):
     rng = np.random.default_rng(5000 + T)

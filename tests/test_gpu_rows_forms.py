@@ -316,8 +316,8 @@ def _bf16_round(a):
 
 
 @pytest.mark.parametrize("gate_type,down_type,H,I,E,K,T", [
-    (orc.Q4_K, orc.Q4_K, 1024, 512, 8, 2, 70),          # the register-operand kernels (one down pass)
-    (orc.Q8_0, orc.Q8_0, 512, 256, 4, 2, 33),           # the loader / multiplier kernels (two down passes: the rounding belongs to the second)
+    (orc.Q4_K, orc.Q4_K, 1024, 512, 8, 2, 70),          # both halves of h in one sweep of K
+    (orc.Q8_0, orc.Q8_0, 512, 256, 4, 2, 33),           # K swept twice in one launch, the low half of h first (the rounding comes after both)
     (orc.Q4_K, orc.Q4_K, 2048, 768, 16, 4, 9)])
 def test_prefill_rows_f16_strided_views(strix, gate_type, down_type, H, I, E, K, T):
     """mi355_moe_enqueue_prefill_rows_f16 (known_rows::PrefillRows / enqueue_prefill with the fp16 form,
