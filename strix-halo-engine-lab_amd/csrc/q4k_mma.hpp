@@ -348,8 +348,8 @@ template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OU
 //   rows.word(a): address of a word that names activation row a (its place in the plan's order); rows.put(a, nacts, word): leaves the row's
 //   addresses in rows.at. Wavefront 3 asks for the words first, then every wavefront starts the weights of the first stages, so the
 //   look-up is in flight beside them. Rows::kDirect: the addresses need no look-up (rows.codes / rows.table), every wavefront works its
-//   own out and starts whole stages, so the first product waits for the first stage only; the row table serves the emitter, or (no kPut)
-//   nobody.
+//   own out and starts whole stages (but for four rows), so the first product waits for the first stage only; the row table serves the
+//   emitter, or (no kPut) nobody.
 //   RUNS: several tiles (else one: none of a run's bookkeeping; gate and up of a dense block, 27648 x 5120, 8 rows: 32.4 -> 31.9 us, and 33.4 with
 //   the weights of both first stages in front of the codes and the row table written in front of the first product).
 //
@@ -408,6 +408,9 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             lanes[k] = c >= TOTAL ? 1ULL : ACTS >= 16U ? ~0ULL : (1ULL << (4U * ACTS)) - 1ULL;
         }
     }
+    // The first stages in one part each, or the weights of both first (27648 x 5120, 4 rows 63.0 | 62.7 us, 8 rows 69.0 | 71.1; 14848 x 5120, 44 rows
+    // 141.4 | 143.5: with more rows a stage's codes are as many bytes as its weights).
+    constexpr bool WHOLE = Rows::kDirect && (!Rows::kPut || NAL > 2);
     const size_t next_tile = kMmaRows * row_stride - BYTES * static_cast<size_t>(stages);       // from a tile's end to the next one's start
     uint32_t issued = 0, issue_stage = 0;
     // copies of the next stage into a slot; PART 1: the weights (of the run's first stages, whose activation rows are not known yet), 2: the rest
@@ -455,6 +458,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         }
     };
     if constexpr (Rows::kDirect) {
+        if (!WHOLE) start_weights();
         set_rows([&](uint32_t a) { return rows.codes(a < nacts ? a : 0U); }, [&](uint32_t a, bool deltas) { return rows.table(a < nacts ? a : 0U, deltas); });
     } else {
         if (wave == 3U) {
@@ -555,7 +559,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
 
     // ---- the ring of stage groups
     issue_stage = 0;
-    for (; issued < first; ++issued) start(std::integral_constant<int, Rows::kDirect ? 0 : 2>{}, slot_of(issued));
+    for (; issued < first; ++issued) start(std::integral_constant<int, WHOLE ? 0 : 2>{}, slot_of(issued));
     if (Rows::kDirect && Rows::kPut && wave == 3U && lane < ACTS) rows.put(lane, nacts, 0U);       // (first read behind the first stage's barrier)
     uint32_t issue_slot = DEPTH - 1U, compute_slot = 0, stage = 0, tile = 0;
     const auto issue = [&]() {
@@ -564,7 +568,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     };
     for (uint32_t g = 0; g < total; ++g) {
         // this wavefront's stages started after its stage of group g (first stages in two parts are not PERW copies each: all of them before the first)
-        if (g < my_total) mma_wait_n<PERW>(!Rows::kDirect && g == 0U ? 0U : issued - 1U - g);
+        if (g < my_total) mma_wait_n<PERW>(!WHOLE && g == 0U ? 0U : issued - 1U - g);
         mma_barrier();         // every copy of group g is in, the slots of group g - 1 are free, its exchanged terms are written
         // The values of the tile before leave in its successor's first stage. They are stores, which the counted waits count too: before
         // the stage's copies they delay those a little, behind them the next wait would wait for copies that it does not need -
