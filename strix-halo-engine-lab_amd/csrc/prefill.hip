@@ -94,7 +94,7 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
     a.wa = wv.gate; a.wb = wv.up; a.expert_stride = wv.gate_expert_stride; a.row_stride = wv.gate_row_stride; a.k = wv.hidden; a.features = wv.ffn;
     a.tiles = wv.ffn / (few ? 64U : 128U); a.units = item_slots * a.tiles;
     launch(std::integral_constant<int, 0>{}, wv.gate_type);
-    // down rows: h enters as hi + lo, both planes in one sweep of the weights
+    // down rows: h enters as hi + lo, both planes in one sweep of the weights (Q4_K) or in two of one launch
     a.wa = wv.down; a.wb = nullptr; a.expert_stride = wv.down_expert_stride; a.row_stride = wv.down_row_stride; a.k = wv.ffn; a.features = wv.hidden;
     a.tiles = wv.hidden / (few ? 128U : 256U); a.units = item_slots * a.tiles;
     launch(std::integral_constant<int, 1>{}, wv.down_type);
