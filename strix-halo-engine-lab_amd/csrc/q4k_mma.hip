@@ -25,18 +25,20 @@ inline bool mma_direct(const A8Image& img, uint32_t dense) { return dense && img
 template <int FMT, int NAL>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items)));
-    constexpr int DEPTH = NAL >= 8 ? 2 : 3;
+    constexpr int DEPTH = NAL >= 8 ? 2 : 3, THREADS = 64 * mma_waves<2, mma_wide<FMT, NAL>()>();
     if constexpr (FMT == kMmaQ4K)
-        if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l}); return; }
-    q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+        if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
+    q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
 // rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
 template <int FMT, int NAL>
 inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const uint32_t tiles = w.hidden / kMmaRows;
+    constexpr bool WIDE = mma_wide<FMT, NAL>();
+    constexpr int THREADS = WIDE ? 512 : 256;
+    const uint32_t tiles = w.hidden / (WIDE ? 2U * kMmaRows : kMmaRows);           // (the wide form: two at a time)
     const bool direct = mma_direct(r.h, dense);
-    if constexpr (FMT == kMmaQ4K) {
+    if constexpr (FMT == kMmaQ4K && !WIDE) {
         const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, 1U);
         if (static_cast<uint64_t>(g.grid.x) * g.grid.y <= compute_units()) {
             if (direct) q4k_mma_down_kernel<FMT, NAL, 2, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
@@ -49,8 +51,8 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
     // 178.3 -> 176.5 us; Q8_0, 40 rows of hidden 2048 / ffn 768 / 128 experts, 124.4 us with three slots, 126.5 with two)
     constexpr int DEPTH = NAL >= 8 || FMT == kMmaQ6K ? 2 : 3;
     if constexpr (FMT == kMmaQ4K)
-        if (direct) { q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, true><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l}); return; }
-    q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, 256, 0, st>>>(MmaArgs{w, r, g.l});
+        if (direct) { q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, true><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
+    q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
 template <int FMT>
 inline void launch_mma_project_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
@@ -59,12 +61,19 @@ inline void launch_mma_project_format(const mi355_moe_weights& w, const RowsK& r
     else if (width <= 16U) launch_mma_project_nal<FMT, 8>(w, r, rows, dense, items, st);
     else launch_mma_project_nal<FMT, 16>(w, r, rows, dense, items, st);
 }
-// (the down rows run best 16 rows to a sweep: 4096 rows over 256 experts, hidden 4096 / ffn 2048: 2.57 ms against 3.03 ms with 32)
+// (rows of another format: sixteen activation rows to a sweep at most, whose two halves of a group take the result registers of 32)
 template <int FMT>
 inline void launch_mma_down_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
     if (width <= 4U) launch_mma_down_nal<FMT, 2>(w, r, rows, dense, items, st);
     else if (width <= 8U) launch_mma_down_nal<FMT, 4>(w, r, rows, dense, items, st);
-    else launch_mma_down_nal<FMT, 8>(w, r, rows, dense, items, st);
+    else {
+        // The wide form from a workgroup per compute unit on: dense 8192 x 4096, 64 rows (256 workgroups) 25.8 -> 23.7 us; with fewer its stages, of
+        // twice the rows, follow one another in fewer places (5120 x 27648, 32 | 64 rows, 80 | 160 workgroups 81 | 109 us against 115 | 116).
+        const uint64_t groups = static_cast<uint64_t>(w.hidden / (2U * kMmaRows)) * (dense ? (dense + 31U) / 32U : items);
+        if constexpr (mma_wide<FMT, 16>())
+            if (width > 16U && groups >= compute_units()) return launch_mma_down_nal<FMT, 16>(w, r, rows, dense, items, st);
+        launch_mma_down_nal<FMT, 8>(w, r, rows, dense, items, st);
+    }
 }
 // width: the most rows an item (or the dense batch) holds
 void launch_mma_project(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {

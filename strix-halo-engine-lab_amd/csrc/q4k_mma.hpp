@@ -60,9 +60,13 @@ template <int NAL> constexpr uint32_t mma_table_copies() { return (mma_acts<NAL>
 template <int FMT, int NAL, int NM> constexpr uint32_t mma_copies() { return mma_weight_copies<FMT>() * NM + mma_code_copies<NAL>() + mma_table_copies<NAL>(); }
 template <int FMT, int NM> constexpr uint32_t mma_codes_at() { return mma_weight_bytes<FMT>() * NM; }
 template <int FMT, int NAL, int NM> constexpr uint32_t mma_table_at() { return mma_codes_at<FMT, NM>() + 256U * mma_acts<NAL>(); }
-template <int FMT, int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<FMT, NAL, NM>() + 64U * mma_acts<NAL>(); }
+template <int FMT, int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<FMT, NAL, NM>() + (mma_acts<NAL>() < 16U ? 64U * mma_acts<NAL>() : 1024U * mma_table_copies<NAL>()); }
 template <int FMT, int NAL, int NM, int DEPTH, int TEAMS> constexpr uint32_t mma_ring_bytes() { return DEPTH * TEAMS * mma_slot_bytes<FMT, NAL, NM>(); }
 template <int NAL, int TEAMS> constexpr uint32_t mma_exchange_floats() { return TEAMS > 1 ? 2U * (TEAMS - 1U) * 4U * NAL * 64U : 1U; }
+// The wide form (mma_stage_wide) serves the sweeps of 32 activation rows.
+template <int FMT, int NAL> constexpr bool mma_wide() { return NAL == 16 && (FMT == kMmaQ4K || FMT == kMmaQ5K); }
+// Wavefronts that sweep a tile together: four (one a pair accumulator), in the wide form four for each matrix.
+template <int NM, bool WIDE> constexpr uint32_t mma_waves() { return WIDE ? 4U * NM : 4U; }
 template <int NAL, int NM> constexpr uint32_t mma_reduce_floats() { return 4U * NM * NAL * 64U; }
 
 // Workgroup barrier that orders LDS traffic only (__syncthreads() would also wait for every copy in flight, i.e. drain the
@@ -116,7 +120,8 @@ struct MmaLane {
     bool sum_lane;
     uint32_t shift, even_slot;         // halves form: of the lane's sub-block in the header words; all ones where the lane's slot is of half 0
     uint32_t start;                    // Q6_K: the lane's row's first byte in its piece, of the first super-block; even_slot: all ones where the
-};                                     // lane's half of K is its slot's
+                                       // lane's half of K is its slot's. Wide form: its slot's code sum of its half of the pair; even_slot: half 0
+};
 
 // Bit `bit` of every byte of a fifth-bit word, as bit 4 (Q5_K)
 __device__ __forceinline__ u32x4 mma_fifth(const u32x4& qh, uint32_t bit) { return ((qh >> bit) & 0x01010101U) << 4; }
@@ -125,7 +130,7 @@ __device__ __forceinline__ u32x4 mma_fifth(const u32x4& qh, uint32_t bit) { retu
 // lane's chain terms x[2P] + x[2P + 1] for its first nv activation rows. P is the wavefront's pair, a template argument so that
 // the scale / min unpacking has constant shifts.
 template <int FMT, int NAL, int NM, int P>
-__device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLane& o, uint32_t nv, float (&term)[NM][NAL]) {
+__device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLane& o, float (&term)[NM][NAL]) {
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) int32_t lds_i32;
     const u32x4 a_even = *(lds_u32x4*)(slot + o.even), a_odd = *(lds_u32x4*)(slot + o.odd);
@@ -158,9 +163,6 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
         const float D1 = d * static_cast<float>(s1), M1 = dm * static_cast<float>(m1);
 #pragma unroll
         for (int v = 0; v < NAL; ++v) {
-            // the widest sweep skips the result registers past a short chunk, four at a time (straight-line code either way: a
-            // loop exit here would turn the register arrays into indexed accesses)
-            if (NAL > 8 && static_cast<uint32_t>(v & ~3) >= nv) continue;
             const float e0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x00, 0xF, 0xF, true));
             const float e1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x55, 0xF, 0xF, true));
             const float f0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0xAA, 0xF, 0xF, true));
@@ -171,6 +173,64 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
             term[m][v] = x0 + x1;
         }
     }
+}
+
+// The same in the wide form, one matrix a wavefront. v of a sub-block is an outer product (a minimum per weight row, a code sum per activation
+// row), so a v_mfma_f32_32x32x2_f32 leaves it in the dots' layout: k = 0 carries sub-block 2p and k = 1 sub-block 2p + 1, each product
+// with the other one's operands zero (a * b rounded once, + 0). A sub-block's terms take the place of its dots before the other's products
+// are made, and the deltas come as broadcast reads, asked for in front of the products they wait with: 64 registers of results and deltas
+// beside the accumulators, so that four wavefronts share a SIMD where two did (gate and up on one wavefront each took 240).
+// Bound by the chain and by what a stage waits for (operands, products, the barrier), in about equal parts. Measured, before -> now: 1000 rows of
+// hidden 2048 / ffn 768 / 128 experts gate / up 327 -> 297 us, down rows (16 activation rows a sweep before) 167 -> 146; dense 27648 x 5120,
+// 32 rows gate / up 105 -> 95 us. Not faster: one wavefront for both matrices with u as one fma on biased dots, at two wavefronts a SIMD (a
+// third fewer vector instructions, 301 us), the same without a barrier from rings of the wavefronts' own (305), a workgroup per chunk (307).
+template <int FMT, int NAL>
+__device__ __forceinline__ void mma_stage_wide(const lds_u8* slot, const MmaLane& o, uint32_t p, float (&acc)[NAL]) {
+    typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+    typedef const __attribute__((address_space(3))) int32_t lds_i32;
+    typedef float f32x16_t __attribute__((ext_vector_type(16)));
+    const u32x4 hd = *(lds_u32x4*)(slot + o.head), q = *(lds_u32x4*)(slot + o.quants), a_even = *(lds_u32x4*)(slot + o.even);
+    const int32_t sum = *(lds_i32*)(slot + o.start);
+    u32x4 fifth = {0U, 0U, 0U, 0U};
+    if (FMT == kMmaQ5K) fifth = *(lds_u32x4*)(slot + o.fifth);
+    __builtin_amdgcn_sched_barrier(0);
+    // (q4k_factors with the wavefront's shifts: six bits, or four and the two above another word's six)
+    const bool high = p >= 2U;
+    const uint32_t shift = 16U * (p & 1U), low_bits = high ? 4U : 6U, top_bits = high ? 2U : 0U;
+    const uint32_t scales = high ? hd.w : hd.y, mins = high ? hd.w >> 4 : hd.z;
+    const auto factor = [&](uint32_t word, uint32_t top, uint32_t at) {
+        return static_cast<float>(__builtin_amdgcn_ubfe(word, at, low_bits) | (__builtin_amdgcn_ubfe(top, at + 6U, top_bits) << 4));
+    };
+    const float d = half_bits_to_float(hd.x & 0xffffU), dm = half_bits_to_float(hd.x >> 16);
+    const float D0 = d * factor(scales, hd.y, shift), D1 = d * factor(scales, hd.y, shift + 8U);
+    const float M = dm * factor(mins, hd.z, o.shift), f = static_cast<float>(sum);          // of the lane's half of the pair
+    const auto products = [&](uint32_t odd, u32x4 n, const u32x4& a, i32x16& dot, f32x16_t& least) __attribute__((always_inline)) {
+        if (FMT == kMmaQ5K) n |= mma_fifth(fifth, 2U * p + odd);
+        const i32x16 zero = {0};
+        const f32x16_t none = {0.0F};
+        const uint32_t in = odd ? ~o.even_slot : o.even_slot;
+        dot = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, n), zero, 0, 0, 0);
+        least = __builtin_amdgcn_mfma_f32_32x32x2f32(f_of(b_of(f) & in), f_of(b_of(M) & in), none, 0, 0, 0);
+    };
+    i32x16 dot;
+    f32x16_t least;
+    products(0, q & 0x0f0f0f0fU, a_even, dot, least);
+    __builtin_amdgcn_sched_barrier(0);
+    const u32x4 a_odd = *(lds_u32x4*)(slot + o.odd);
+    float e[NAL], x0[NAL];
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) e[v] = *(const lds_f32*)(slot + o.table + 128U * v);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) x0[v] = e[v] * (D0 * static_cast<float>(dot[v]) - least[v]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) e[v] = *(const lds_f32*)(slot + o.table + 128U * v + 4U);
+    products(1, (q >> 4) & 0x0f0f0f0fU, a_odd, dot, least);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int v = 0; v < NAL; ++v) acc[v] = acc[v] + (x0[v] + e[v] * (D1 * static_cast<float>(dot[v]) - least[v]));
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // The same for few activation rows (NAL == 2), where the scales, the nibbles and the layout's own moves outweigh the chain: each half of
@@ -350,6 +410,7 @@ template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OU
 //   look-up is in flight beside them. Rows::kDirect: the addresses need no look-up (rows.codes / rows.table), every wavefront works its
 //   own out and starts whole stages (but for four rows), so the first product waits for the first stage only; the row table serves the
 //   emitter, or (no kPut) nobody.
+//   WIDE: mma_stage_wide's form, four wavefronts for each of the NM matrices. tile_rows: rows from a tile to the next.
 //   RUNS: several tiles (else one: none of a run's bookkeeping; gate and up of a dense block, 27648 x 5120, 8 rows: 32.4 -> 31.9 us, and 33.4 with
 //   the weights of both first stages in front of the codes and the row table written in front of the first product).
 //
@@ -358,22 +419,24 @@ template <int NAL, int OUT> constexpr uint32_t mma_row_words() { return (3U + OU
 // kept by team 0, which adds the terms of every super-block in ascending order: its own from registers, the other teams'
 // from an LDS exchange buffer, one stage group behind (the group's barrier publishes them).
 // Every wavefront of the workgroup calls this; ring, row table and `red` are free again when it returns.
-template <int FMT, int NAL, int DEPTH, int TEAMS, int NM, bool RUNS, class Rows, class Emit>
+template <int FMT, int NAL, int DEPTH, int TEAMS, int NM, bool RUNS, bool WIDE, class Rows, class Emit>
 __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* red, const uint8_t* const (&wrows)[NM], size_t row_stride, uint32_t stages,
-                                        uint32_t tiles, uint32_t nacts, Rows rows, Emit emit) {
+                                        uint32_t tiles, uint32_t tile_rows, uint32_t nacts, Rows rows, Emit emit) {
     constexpr uint32_t ACTS = mma_acts<NAL>(), CC = mma_code_copies<NAL>(), TOTAL = mma_copies<FMT, NAL, NM>(), SLOT = mma_slot_bytes<FMT, NAL, NM>();
     constexpr uint32_t CW = mma_weight_copies<FMT>(), PIECES = mma_pieces<FMT>(), PITCH = mma_pitch<FMT>(), BYTES = mma_block_bytes<FMT>();
     // In the ring every wavefront issues PERW copies a stage - past the last one it copies the last one's first piece again, the same bytes to
     // the same place - so there are no branches on the wavefront's number and one count to wait for. The run's first stages are issued in
     // two parts of as many copies as a wavefront has there, and awaited whole.
-    constexpr uint32_t PERW = (TOTAL + 3U) / 4U, WEIGHTS = CW * NM, WEIGHTS_LAST = WEIGHTS / 4U;        // (weight copies of wavefront 3)
+    constexpr uint32_t W = mma_waves<NM, WIDE>(), MATS = 4U * NM / W;                             // wavefronts of a team; matrices of a wavefront
+    constexpr uint32_t PERW = (TOTAL + W - 1U) / W, WEIGHTS = CW * NM, WEIGHTS_LAST = (WEIGHTS - 3U + W - 1U) / W;        // (weight copies of wavefront 3)
     constexpr uint32_t XTEAM = 4U * NAL * 64U;                                                  // floats one team exchanges per group
     static_assert(DEPTH >= 2 && DEPTH <= 4, "ring depth");
     static_assert(TEAMS == 1 || (NM == 1 && NAL <= 8 && FMT == kMmaQ4K), "stage teams serve one matrix, every result register");
+    static_assert(!WIDE || (TEAMS == 1 && (FMT == kMmaQ4K || FMT == kMmaQ5K)), "wide form");
     static_assert(NM == 1 || FMT == kMmaQ4K || FMT == kMmaQ5K, "gate and up rows");
     static_assert(CW >= 4U && PIECES >= 8U, "copies 0 .. 3 are of whole waves");
     const uint32_t lane = threadIdx.x & 63U, j = lane & 31U, h = lane >> 5;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), p = wave & 3U, team = wave >> 2;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wave % W, p = w & 3U, matrix = w >> 2, team = wave / W;
     const uint32_t groups = (stages + TEAMS - 1U) / TEAMS;                                     // of a tile
     const uint32_t my_groups = team < stages - (groups - 1U) * TEAMS ? groups : groups - 1U;   // groups in which this team has a super-block
     const uint32_t total = RUNS ? groups * tiles : groups, my_total = TEAMS == 1 ? total : my_groups;
@@ -386,7 +449,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     uint64_t lanes[PERW];
 #pragma unroll
     for (uint32_t k = 0; k < PERW; ++k) {
-        const uint32_t c = 4U * k + p;
+        const uint32_t c = W * k + w;
         if (c < WEIGHTS) {
             const uint32_t m = c / CW, i = c - CW * m, s = 64U * i + lane < kMmaRows * PITCH ? 64U * i + lane : 0U, r = s / PITCH;
             const uint32_t piece = s - PITCH * r < PIECES ? s - PITCH * r : PIECES - 1U;
@@ -411,17 +474,17 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     // The first stages in one part each, or the weights of both first (27648 x 5120, 4 rows 63.0 | 62.7 us, 8 rows 69.0 | 71.1; 14848 x 5120, 44 rows
     // 141.4 | 143.5: with more rows a stage's codes are as many bytes as its weights).
     constexpr bool WHOLE = Rows::kDirect && (!Rows::kPut || NAL > 2);
-    const size_t next_tile = kMmaRows * row_stride - BYTES * static_cast<size_t>(stages);       // from a tile's end to the next one's start
+    const size_t next_tile = tile_rows * row_stride - BYTES * static_cast<size_t>(stages);       // from a tile's end to the next one's start
     uint32_t issued = 0, issue_stage = 0;
     // copies of the next stage into a slot; PART 1: the weights (of the run's first stages, whose activation rows are not known yet), 2: the rest
     const auto start = [&](auto part_constant, lds_u8* slot) __attribute__((always_inline)) {
         constexpr int part = decltype(part_constant)::value;
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
-            if (part != 0 && (4U * k + p < WEIGHTS) != (part == 1)) continue;
+            if (part != 0 && (W * k + w < WEIGHTS) != (part == 1)) continue;
             const uint8_t* from = src[k];
-            if (FMT == kMmaQ6K && 4U * k + p < WEIGHTS) from = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(from) & ~static_cast<uintptr_t>(15)) + piece_at[k];
-            if (part == 0 && k == 0U) mma_copy16(from, slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
+            if (FMT == kMmaQ6K && W * k + w < WEIGHTS) from = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(from) & ~static_cast<uintptr_t>(15)) + piece_at[k];
+            if (W == 4U && part == 0 && k == 0U) mma_copy16(from, slot + lands[k]);            // (copies 0 .. 3: weights of a whole wave)
             else mma_copy16_lanes(from, slot + lands[k], lanes[k]);
             src[k] += step[k];
         }
@@ -429,7 +492,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
             issue_stage = 0;
 #pragma unroll
             for (uint32_t k = 0; k < PERW; ++k) {
-                const bool weights = 4U * k + p < WEIGHTS;
+                const bool weights = W * k + w < WEIGHTS;
                 if (part == 0 || weights == (part == 1)) src[k] += weights ? next_tile : 0U - static_cast<size_t>(step[k]) * stages;
             }
         }
@@ -439,15 +502,15 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     const auto start_weights = [&]() {
         for (uint32_t s = 0; s < first; ++s) start(std::integral_constant<int, 1>{}, slot_of(s));
     };
-    const auto row_of_codes = [&](uint32_t k) { return (64U * (4U * k + p - WEIGHTS) + lane) >> 4; };                            // of the lane's 16 bytes
+    const auto row_of_codes = [&](uint32_t k) { return (64U * (W * k + w - WEIGHTS) + lane) >> 4; };                            // of the lane's 16 bytes
     const auto row_of_table = [&](uint32_t k) {
-        const uint32_t c = 4U * k + p < TOTAL ? 4U * k + p : TOTAL - 1U;
-        return (16U * (c - WEIGHTS - CC) + (lane >> 2)) & (ACTS - 1U);
+        const uint32_t c = W * k + w < TOTAL ? W * k + w : TOTAL - 1U;
+        return (16U * (c - WEIGHTS - CC) + (lane >> 2)) % ACTS;
     };
     const auto set_rows = [&](auto codes_of, auto table_of) {
 #pragma unroll
         for (uint32_t k = 0; k < PERW; ++k) {
-            const uint32_t c = 4U * k + p;
+            const uint32_t c = W * k + w;
             if (c >= WEIGHTS && c < WEIGHTS + CC) {
                 const uint32_t a = row_of_codes(k);
                 src[k] = codes_of(a) + 16U * (((lane & 15U) - a) & 15U) + 256U * team;
@@ -471,7 +534,7 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         } else start_weights();
         mma_barrier();
         set_rows([&](uint32_t a) { return reinterpret_cast<const uint8_t*>(rows.at[a]); },
-                 [&](uint32_t a, bool deltas) { return reinterpret_cast<const uint8_t*>(rows.at[(deltas ? ACTS : 2U * ACTS) + a]); });
+                 [&](uint32_t a, bool deltas) { return reinterpret_cast<const uint8_t*>(rows.at[(deltas ? Rows::kActs : 2U * Rows::kActs) + a]); });
     }
 
     MmaLane o;
@@ -504,7 +567,16 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         // quad lane 0, 1: the deltas of g0, g1; quad lane 2, 3: their code sums
         o.table = mma_table_at<FMT, NAL, NM>() + 64U * h + 4U * ((lane & 1U ? g1 : g0) + 4U * (lane & 2U));
         o.sum_lane = (lane & 2U) != 0;
-        if constexpr (mma_halves<NAL>() && (FMT == kMmaQ4K || FMT == kMmaQ5K)) {
+        if constexpr (WIDE) {
+            o.head += mma_weight_bytes<FMT>() * matrix;
+            o.fifth += mma_weight_bytes<FMT>() * matrix;
+            o.quants += mma_weight_bytes<FMT>() * matrix;
+            o.table = mma_table_at<FMT, NAL, NM>() + 64U * h + 8U * p;                          // the deltas of activation row 2v + h
+            o.start = mma_table_at<FMT, NAL, NM>() + 64U * ai + 32U + 4U * (2U * p + h);        // the code sum of the lane's slot and half of the pair
+            o.shift = 16U * (p & 1U) + 8U * h;
+            o.even_slot = h ? 0U : ~0U;
+        }
+        if constexpr (!WIDE && mma_halves<NAL>() && (FMT == kMmaQ4K || FMT == kMmaQ5K)) {
             const uint32_t odd = (j >> 2) & 1U, act = (4U * (j >> 3) + (j & 3U)) & (ACTS - 1U);
             o.even = mma_codes_at<FMT, NM>() + 256U * act + 16U * ((4U * p + 2U * odd + h + act) & 15U);
             o.table = mma_table_at<FMT, NAL, NM>() + 4U * (2U * p + h);
@@ -513,12 +585,12 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         }
     }
 
-    float acc[NM][NAL], own[NAL];
+    float acc[MATS][NAL], own[NAL];
 #pragma unroll
     for (int v = 0; v < NAL; ++v) own[v] = 0.0F;
     const auto clear = [&]() {
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
+        for (uint32_t m = 0; m < MATS; ++m)
 #pragma unroll
             for (int v = 0; v < NAL; ++v) acc[m][v] = 0.0F;
     };
@@ -538,14 +610,14 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
     };
     const auto leave = [&]() {
 #pragma unroll
-        for (int m = 0; m < NM; ++m)
+        for (uint32_t m = 0; m < MATS; ++m)
 #pragma unroll
-            for (int v = 0; v < NAL; ++v) red[((m * 4U + p) * NAL + v) * 64U + lane] = acc[m][v];
+            for (int v = 0; v < NAL; ++v) red[((m * 4U + w) * NAL + v) * 64U + lane] = acc[m][v];
     };
     const auto emit_tile = [&](uint32_t tile) {
         uint32_t lane = threadIdx.x & 63U;
         asm volatile("" : "+v"(lane));         // (what follows from it is worked out here, once a tile, not held in registers over the sweep)
-        for (uint32_t v = p; v < nv; v += 4U) {
+        for (uint32_t v = w; v < nv; v += W) {
             float value[NM];
 #pragma unroll
             for (uint32_t m = 0; m < NM; ++m) {
@@ -582,26 +654,24 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
         if (TEAMS > 1 && team == 0U && g > 0U) fold(g - 1U);
         if (g < my_total) {
             const lds_u8* slot = ring + SLOT * (compute_slot * TEAMS + team);
-            float term[NM][NAL];
-            if constexpr (FMT != kMmaQ4K && FMT != kMmaQ5K) mma_stage_other<FMT, NAL>(slot, o, p, RUNS ? stage : g, acc[0]);
+            float term[MATS][NAL];
+            if constexpr (WIDE) mma_stage_wide<FMT, NAL>(slot, o, p, acc[0]);
+            else if constexpr (FMT != kMmaQ4K && FMT != kMmaQ5K) mma_stage_other<FMT, NAL>(slot, o, p, RUNS ? stage : g, acc[0]);
             else if constexpr (mma_halves<NAL>()) {
                 if (p < 2U) mma_stage_terms_halves<FMT, NAL, NM, false>(slot, o, p, term);
                 else mma_stage_terms_halves<FMT, NAL, NM, true>(slot, o, p, term);
             } else switch (p) {
-            case 0: mma_stage_terms<FMT, NAL, NM, 0>(slot, o, nv, term); break;
-            case 1: mma_stage_terms<FMT, NAL, NM, 1>(slot, o, nv, term); break;
-            case 2: mma_stage_terms<FMT, NAL, NM, 2>(slot, o, nv, term); break;
-            default: mma_stage_terms<FMT, NAL, NM, 3>(slot, o, nv, term); break;
+            case 0: mma_stage_terms<FMT, NAL, NM, 0>(slot, o, term); break;
+            case 1: mma_stage_terms<FMT, NAL, NM, 1>(slot, o, term); break;
+            case 2: mma_stage_terms<FMT, NAL, NM, 2>(slot, o, term); break;
+            default: mma_stage_terms<FMT, NAL, NM, 3>(slot, o, term); break;
             }
-            if (FMT != kMmaQ4K && FMT != kMmaQ5K) {
+            if ((FMT != kMmaQ4K && FMT != kMmaQ5K) || WIDE) {
             } else if (TEAMS == 1) {
 #pragma unroll
-                for (int m = 0; m < NM; ++m)
+                for (uint32_t m = 0; m < MATS; ++m)
 #pragma unroll
-                    for (int v = 0; v < NAL; ++v) {
-                        if (NAL > 8 && static_cast<uint32_t>(v & ~3) >= nv) continue;
-                        acc[m][v] = acc[m][v] + term[m][v];
-                    }
+                    for (int v = 0; v < NAL; ++v) acc[m][v] = acc[m][v] + term[m][v];
             } else if (team == 0U) {
 #pragma unroll
                 for (int v = 0; v < NAL; ++v) own[v] = term[0][v];

@@ -40,9 +40,10 @@ __device__ __forceinline__ MmaItem mma_item(const MmaArgs& k, uint32_t width) {
 // of row a, assignment i, once, so that nothing else of the kernel does. img: the A8 image the rows are read from. DIRECT: a dense batch
 // over one image per row at a stride, which needs no look-up - an instance of its own, because the strides and bases held for it cost
 // the planned batches 1.5 % (dense 27648 x 5120, 8 rows: 86.5 -> 84.6 us). PUT: the emitter reads the row table.
-template <bool DIRECT, bool PUT, class Put>
+template <uint32_t ACTS, bool DIRECT, bool PUT, class Put>
 struct MmaRowsOf {
     static constexpr bool kDirect = DIRECT, kPut = PUT;
+    static constexpr uint32_t kActs = ACTS;             // rows that the row table has room for
     uint32_t c0;
     const A8Image& img;
     uint32_t dense;
@@ -67,10 +68,20 @@ struct MmaRowsOf {
 };
 template <class P> __device__ __forceinline__ uint64_t address(const P* p) { return reinterpret_cast<uint64_t>(p); }
 
-// Waves per SIMD: what the LDS of a workgroup allows (four of 36 KB, three of 44 or 46 KB, two of 73 KB), which for 16 rows the compiler misses
+// The sweep of a chunk of n rows, run(NAL): of the wide form (NAL == 16) with no chain for the result registers past a short chunk.
+template <int NAL, class Run> __device__ __forceinline__ void mma_chunk(uint32_t n, Run run) {
+    if constexpr (NAL == 16) {
+        if (n > 24U) run(std::integral_constant<int, 16>{});
+        else if (n > 16U) run(std::integral_constant<int, 12>{});
+        else if (n > 8U) run(std::integral_constant<int, 8>{});
+        else run(std::integral_constant<int, 4>{});
+    } else run(std::integral_constant<int, NAL>{});
+}
+
+// Waves per SIMD: what the LDS of a workgroup allows (four of 36 KB, three of 44 or 46 KB, two of eight wavefronts and 73 KB), which for 16 rows the compiler misses
 // by a few registers when it is not told (200 rows of hidden 2048 / ffn 768 / 128 experts: 192.8 -> 172.3 us a layer, 219.6 before the run).
 template <int FMT, int NAL, int DEPTH, bool DIRECT>
-__global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_project_kernel(MmaArgs k) {
+__global__ __launch_bounds__(NAL == 16 ? 512 : 256, NAL == 2 || NAL == 16 ? 4 : 3) void q4k_mma_project_kernel(MmaArgs k) {
     constexpr uint32_t ACTS = mma_acts<NAL>();
     __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, 2, DEPTH, 1>()];
     __shared__ float red_mem[mma_reduce_floats<NAL, 2>()];
@@ -96,9 +107,8 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
             at[4U * ACTS + a] = address(r.h_deltas_of(i));
             at[5U * ACTS + a] = address(r.h_sums_of(i));
         };
-        const MmaRowsOf<DIRECT, true, decltype(put)> rows{c0, k.r.in, k.l.dense_rows, at, slot, put};
-        mma_run<FMT, NAL, DEPTH, 1, 2, true>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, n, rows,
-                                  [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[2]) {
+        const MmaRowsOf<ACTS, DIRECT, true, decltype(put)> rows{c0, k.r.in, k.l.dense_rows, at, slot, put};
+        const auto emit = [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[2]) {
             const uint32_t j = lane & 31U, h = lane >> 5;
             const MmaArgs& args = mma_args();
             const RowsK& r = args.r;
@@ -135,7 +145,11 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
                 reinterpret_cast<float*>(at[4U * ACTS + a])[grp] = dl;
                 reinterpret_cast<int32_t*>(at[5U * ACTS + a])[grp] = sum;
             }
-        });
+        };
+        const auto run = [&](auto nal) __attribute__((always_inline)) {
+            mma_run<FMT, decltype(nal)::value, DEPTH, 1, 2, true, mma_wide<FMT, NAL>()>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, kMmaRows, n, rows, emit);
+        };
+        mma_chunk<NAL>(n, run);
     }
 }
 
@@ -143,11 +157,12 @@ __global__ __launch_bounds__(256, NAL == 2 ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_
 // intermediates - the dense FFN's projection when that workspace exists (two launches' worth of narrow workgroups fill the
 // compute units better than the fused form's wide ones: 27648 x 5120, 8 rows: 54 + 5 us against 70 us).
 template <int FMT, int NAL, int DEPTH, int TEAMS, bool DIRECT, bool GATE_UP = false>
-__global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
-    constexpr uint32_t ACTS = mma_acts<NAL>();
-    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, 1, DEPTH, TEAMS>()];
+__global__ __launch_bounds__(NAL == 16 ? 512 : 256 * TEAMS, NAL == 16 ? 4 : 1) void q4k_mma_down_kernel(MmaArgs k) {
+    // the wide form: over two tiles at a time, as if they were of two matrices
+    constexpr uint32_t ACTS = mma_acts<NAL>(), NM = mma_wide<FMT, NAL>() ? 2U : 1U, TILE = NM * kMmaRows;
+    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, NM, DEPTH, TEAMS>()];
     __shared__ float xbuf_mem[mma_exchange_floats<NAL, TEAMS>()];
-    __shared__ float red_mem[mma_reduce_floats<NAL, 1>()];
+    __shared__ float red_mem[mma_reduce_floats<NAL, NM>()];
     __shared__ uint64_t at_mem[mma_row_words<NAL, 1>()];
     __shared__ uint32_t slot_mem[ACTS];
     lds_u64* const at = (lds_u64*)at_mem;
@@ -158,7 +173,9 @@ __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
     const MmaItem item = mma_item(k, ACTS);
     if (item.begin == item.end) return;
     const uint32_t tile0 = blockIdx.x * k.l.run, tiles = k.l.tiles - tile0 < k.l.run ? k.l.tiles - tile0 : k.l.run;
-    const uint8_t* const wrows[1] = {matrix + static_cast<size_t>(item.e) * expert_stride + static_cast<size_t>(tile0 * kMmaRows) * row_stride};
+    const uint8_t* wrows[NM];
+#pragma unroll
+    for (uint32_t m = 0; m < NM; ++m) wrows[m] = matrix + static_cast<size_t>(item.e) * expert_stride + static_cast<size_t>(tile0 * TILE + m * kMmaRows) * row_stride;
     for (uint32_t c0 = item.begin; c0 < item.end; c0 += ACTS) {
         const uint32_t n = item.end - c0 < ACTS ? item.end - c0 : ACTS;
         const auto put = [&](const MmaArgs& args, uint32_t a, uint32_t i) {
@@ -170,17 +187,25 @@ __global__ __launch_bounds__(256 * TEAMS) void q4k_mma_down_kernel(MmaArgs k) {
             at[2U * ACTS + a] = address(img.sums_of(from));
             at[3U * ACTS + a] = GATE_UP ? address(r.inter_of(blockIdx.z ? r.up_out : r.gate_out, i)) : address(r.rawdots_of(i, args.w.hidden));
         };
-        const MmaRowsOf<DIRECT, !DIRECT, decltype(put)> rows{c0, GATE_UP ? k.r.in : k.r.h, k.l.dense_rows, at, slot, put};
-        mma_run<FMT, NAL, DEPTH, TEAMS, 1, TEAMS == 1 && !GATE_UP>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride, (GATE_UP ? k.w.hidden : k.w.ffn) / 256U,
-                                      tiles, n, rows, [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[1]) {
-            const uint32_t a = 2U * v + (lane >> 5), at_out = (tile0 + tile) * kMmaRows + (lane & 31U);
+        const MmaRowsOf<ACTS, DIRECT, !DIRECT, decltype(put)> rows{c0, GATE_UP ? k.r.in : k.r.h, k.l.dense_rows, at, slot, put};
+        const auto emit = [&](uint32_t tile, uint32_t v, uint32_t lane, const float (&value)[NM]) {
+            const uint32_t a = 2U * v + (lane >> 5), at_out = (tile0 + tile) * TILE + (lane & 31U);
             if (a >= n) return;
             // (the rows of a dense batch: assignment = row, at a stride; the argument block read again at a workgroup's end is one way to memory more)
             float* const out = !DIRECT ? reinterpret_cast<float*>(at[3U * ACTS + a])
                                : GATE_UP ? k.r.inter_of(blockIdx.z ? k.r.up_out : k.r.gate_out, c0 + a) : k.r.rawdots_of(c0 + a, k.w.hidden);
-            out[at_out] = value[0];
-            if (!GATE_UP && k.r.top1_form) (DIRECT ? k.r : mma_args().r).publish_top1(DIRECT ? c0 + a : slot[a], at_out, value[0]);      // (top-1: assignment = row)
-        });
+#pragma unroll
+            for (uint32_t m = 0; m < NM; ++m) {
+                out[at_out + m * kMmaRows] = value[m];
+                if (!GATE_UP && k.r.top1_form)      // (top-1: assignment = row)
+                    (DIRECT ? k.r : mma_args().r).publish_top1(DIRECT ? c0 + a : slot[a], at_out + m * kMmaRows, value[m]);
+            }
+        };
+        const auto run = [&](auto nal) __attribute__((always_inline)) {
+            mma_run<FMT, decltype(nal)::value, DEPTH, TEAMS, NM, TEAMS == 1 && !GATE_UP, mma_wide<FMT, NAL>()>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride,
+                                                                                                  (GATE_UP ? k.w.hidden : k.w.ffn) / 256U, tiles, TILE, n, rows, emit);
+        };
+        mma_chunk<NAL>(n, run);
     }
 }
 
