@@ -9,7 +9,7 @@
 // eight rows read different banks. Lane (i, q) then reads feature 4 t + q of row i and of expert i for step t of
 // the chain with one 32-bit LDS read each (16-byte reads and a transpose between the lanes cost 16 half-rate vector operations per
 // eight steps, which the fp32 matrix instruction does not overlap with: 22 us a launch). Bound by the chain, 13.4 ns per 4 features.
-// Measured at hidden 2048, 128 experts: 40 and 1000 rows 100 -> 17 us; 4096 rows, hidden 4096, 256 experts: 221 -> 110 us (lane-wise fma
+// Measured at hidden 2048, 128 experts: 40 and 1000 rows 100 -> 15 and 17 us; 4096 rows, hidden 4096, 256 experts: 221 -> 110 us (lane-wise fma
 // chains on tiles of 64 rows x 64 experts before, of which a batch of 40 rows gave two workgroups).
 #pragma once
 #include "route_wave.hpp"
@@ -26,16 +26,16 @@ __device__ __forceinline__ void route_copy16(const void* src, uint32_t lds_at) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_at), "v"(src) : "memory", "m0");
 }
 
-template <int KIND, int DEPTH>
-__global__ __launch_bounds__(256) void route_mma_kernel(RouteArgs a) {
+template <int KIND, int DEPTH, uint32_t WAVES>
+__global__ __launch_bounds__(64 * WAVES) void route_mma_kernel(RouteArgs a) {
     constexpr uint32_t COPIES = route_block_copies<KIND>(), SLOT = 1024U * COPIES;
-    __shared__ __attribute__((aligned(16))) uint8_t ring[4 * route_ring_bytes<KIND, DEPTH>()];
+    __shared__ __attribute__((aligned(16))) uint8_t ring[WAVES * route_ring_bytes<KIND, DEPTH>()];
     typedef __attribute__((address_space(3))) uint8_t lds_byte;
     typedef const __attribute__((address_space(3))) uint32_t lds_u32;
     typedef const __attribute__((address_space(3))) uint16_t lds_u16;
     typedef const __attribute__((address_space(3))) float lds_f32;
     const uint32_t lane = threadIdx.x & 63U, i = lane & 15U, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t r0 = blockIdx.y * 16U, e0 = (blockIdx.x * 4U + wave) * 16U;
+    const uint32_t r0 = blockIdx.y * 16U, e0 = (blockIdx.x * WAVES + wave) * 16U;
     if (e0 >= a.p.experts) return;
     const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte*)ring)) + wave * route_ring_bytes<KIND, DEPTH>());
     // copier role: lane l of a copy of eight 128-byte rows (fp16 / bf16 activations: sixteen 64-byte rows)
@@ -111,17 +111,24 @@ __global__ __launch_bounds__(256) void route_mma_kernel(RouteArgs a) {
     }
 }
 
-// A ring of eight blocks where one workgroup per compute unit holds the launch, of four (two or three workgroups share a unit) beyond.
+// While a wave's workgroup finds room beside two others (fp32 rows: beside one), a ring of sixteen blocks (48 KB, 64 KB): a block is chained in
+// 107 ns, so eight are 0.9 us ahead, less than a cold fetch takes (hidden 2048, 128 experts, 40 | 333 rows 16.7 | 15.9 -> 14.7 | 14.4 us; hidden 6144,
+// 160 experts, 17 rows 39.3 -> 36.5; 1008 waves of hidden 2048 17.3 | 30.0). Else four waves a workgroup: a ring of eight where one workgroup per
+// compute unit holds the launch, of four (two or three workgroups share a unit) beyond.
 inline void launch_route_mma(const RouteArgs& a, uint32_t compute_units, hipStream_t st) {
-    const dim3 grid((a.p.experts + 63U) / 64U, (a.rows + 15U) / 16U);
-    const auto launch = [&](auto depth) {
+    const uint32_t rows = (a.rows + 15U) / 16U, experts = (a.p.experts + 15U) / 16U;
+    const uint64_t waves = static_cast<uint64_t>(rows) * experts, units = compute_units;
+    const auto launch = [&](auto depth, auto per) {
         constexpr int DEPTH = decltype(depth)::value;
-        if (a.kind == MI355_INPUT_F32) route_mma_kernel<0, DEPTH><<<grid, 256, 0, st>>>(a);
-        else if (a.kind == MI355_INPUT_F16) route_mma_kernel<1, DEPTH><<<grid, 256, 0, st>>>(a);
-        else route_mma_kernel<2, DEPTH><<<grid, 256, 0, st>>>(a);
+        constexpr uint32_t WAVES = decltype(per)::value;
+        const dim3 grid((experts + WAVES - 1U) / WAVES, rows);
+        if (a.kind == MI355_INPUT_F32) route_mma_kernel<0, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
+        else if (a.kind == MI355_INPUT_F16) route_mma_kernel<1, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
+        else route_mma_kernel<2, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
     };
-    if (static_cast<uint64_t>(grid.x) * grid.y > compute_units) launch(std::integral_constant<int, 4>{});
-    else launch(std::integral_constant<int, 8>{});
+    if (waves <= (a.kind == MI355_INPUT_F32 ? 2U : 3U) * units) launch(std::integral_constant<int, 16>{}, std::integral_constant<uint32_t, 1U>{});
+    else if (static_cast<uint64_t>((experts + 3U) / 4U) * rows <= units) launch(std::integral_constant<int, 8>{}, std::integral_constant<uint32_t, 4U>{});
+    else launch(std::integral_constant<int, 4>{}, std::integral_constant<uint32_t, 4U>{});
 }
 
 }  // namespace strix950

@@ -59,3 +59,16 @@ def test_rows_of_any_values(strix, dtype):
         parts = [strix.route(x[r:r + 8].contiguous(), router, top_k, bias=bias) for r in range(0, rows, 8)]
         for got, want in zip(batch, zip(*parts)):
             assert torch.equal(got.view(torch.int32), torch.cat(want).view(torch.int32))
+
+
+# around the lines between the rings: sixteen blocks of a workgroup of one wave (as many blocks, one less and one more; 512 and 528, 768 and 784
+# waves), eight and four of a workgroup of four waves; a row's value does not depend on the batch, so decode batches state it
+@pytest.mark.parametrize("rows,experts,hidden", [(40, 20, 480), (40, 20, 512), (40, 20, 544), (512, 256, 128), (513, 250, 288), (768, 256, 160), (769, 256, 544), (4097, 64, 96)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_rings_of_a_batch(strix, rows, experts, hidden, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    x, w = torch.randn((rows, hidden), device="cuda", generator=gen).to(dtype), torch.randn((experts, hidden), device="cuda", generator=gen) * 0.05
+    batch = strix.route(x, w, 4)
+    for r in (0, rows // 2, rows - 16):
+        for got, want in zip(batch, strix.route(x[r:r + 16].contiguous(), w, 4)):
+            assert torch.equal(got[r:r + 16].view(torch.int32), want.view(torch.int32)), r
