@@ -27,23 +27,17 @@ void launch_route_batch_logits(const RouteArgs& a, hipStream_t st) {
     else route_logits_kernel<2><<<blocks, 64, 0, st>>>(a);
 }
 
-// The row-wise start of a staged batch in one launch: the A8 image of the row, its routes (SELECT: from the logits in a.scores), the check
-// of the routes and the row's status word. One workgroup per row; the last wave takes the routes while the others quantise.
-// Bound by latency (a launch of this size costs about 4.5 us whatever it does): one launch in the place of three (select, clear and
-// validate, A8 image) or two.
-// (With the selection at most eight waves: its registers for 1024 experts would not fit sixteen.)
-constexpr uint32_t kPrologueThreads[2] = {1024, 512};
-template <int KIND, bool SELECT>
-__global__ __launch_bounds__(kPrologueThreads[SELECT]) void prologue_rows_kernel(A8RowArgs q, RouteArgs a, RouteCheck c) {
-    __shared__ __attribute__((aligned(16))) float sel_p[SELECT ? kRouteMaxExperts : 4U];
-    const uint32_t row = blockIdx.x, lane = threadIdx.x & 63U, image_threads = blockDim.x - 64U;
+// The start of a staged batch in one launch: the expert plan (a workgroup per expert), and a workgroup per row for the A8 image of the row, the
+// check of its routes (by a wave of their own) and its status word. Bound by latency (a launch of this size costs about 4.5 us whatever it does).
+template <int KIND>
+__global__ __launch_bounds__(1024) void prologue_rows_kernel(A8RowArgs q, RouteCheck c, uint32_t image_threads, PlanArgs plan) {
+    __shared__ PlanLds lds;
+    if (blockIdx.x < plan.experts) return plan_block(lds, plan, blockIdx.x);
+    if (threadIdx.x >= image_threads + 64U) return;
+    const uint32_t row = blockIdx.x - plan.experts, lane = threadIdx.x & 63U;
     int bad_value = 0, bad_route = 0;
     if (threadIdx.x < image_threads) bad_value = a8_row<KIND>(q, row, image_threads);
     else {
-        if constexpr (SELECT) {
-            route_select_row<false>(sel_p, a, row);
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");      // (the ids and weights other lanes of this wave have stored)
-        }
         for (uint32_t k = lane; k < c.top_k; k += 64U) {
             if (c.routes[static_cast<size_t>(row) * c.top_k + k] >= c.experts) bad_route = 1;
             if (c.route_weights && !finite_f(c.route_weights[static_cast<size_t>(row) * c.top_k + k])) bad_route = 1;
@@ -57,17 +51,12 @@ __global__ __launch_bounds__(kPrologueThreads[SELECT]) void prologue_rows_kernel
     }
 }
 
-void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, const RouteArgs* select, const RouteCheck& c, hipStream_t st) {
-    const uint32_t image = a8_row_threads(q.width) + 64U, most = kPrologueThreads[select != nullptr], threads = image < most ? image : most;
-    const auto launch = [&](auto chosen) {
-        constexpr bool SELECT = decltype(chosen)::value;
-        const RouteArgs a = SELECT ? *select : RouteArgs{};
-        if (kind == MI355_INPUT_F32) prologue_rows_kernel<0, SELECT><<<rows, threads, 0, st>>>(q, a, c);
-        else if (kind == MI355_INPUT_F16) prologue_rows_kernel<1, SELECT><<<rows, threads, 0, st>>>(q, a, c);
-        else prologue_rows_kernel<2, SELECT><<<rows, threads, 0, st>>>(q, a, c);
-    };
-    if (select) launch(std::true_type{});
-    else launch(std::false_type{});
+void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, const RouteCheck& c, const PlanArgs& plan, hipStream_t st) {
+    const uint32_t image = a8_row_threads(q.width) + 64U, used = image < 1024U ? image : 1024U;
+    const uint32_t threads = plan.experts && used < 512U ? 512U : used, grid = plan.experts + rows;
+    if (kind == MI355_INPUT_F32) prologue_rows_kernel<0><<<grid, threads, 0, st>>>(q, c, used - 64U, plan);
+    else if (kind == MI355_INPUT_F16) prologue_rows_kernel<1><<<grid, threads, 0, st>>>(q, c, used - 64U, plan);
+    else prologue_rows_kernel<2><<<grid, threads, 0, st>>>(q, c, used - 64U, plan);
 }
 
 void launch_route_select(const RouteArgs& a, hipStream_t st) { route_select_kernel<<<a.rows, 64, 0, st>>>(a); }

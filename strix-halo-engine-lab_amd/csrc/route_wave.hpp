@@ -428,16 +428,7 @@ __device__ __forceinline__ uint64_t key_max_wave(uint64_t key) {        // the w
 }
 // Returns, in lane k < top_k + shared_experts, the expert of slot k.
 // shared_out: ids and weights are also read by other workgroups of the same launch (device-scope stores).
-// ALONE: the wave is its workgroup; otherwise other waves of the workgroup run beside it and only this wave is ordered.
-template <bool ALONE>
-__device__ __forceinline__ void select_sync() {
-    if constexpr (ALONE) __syncthreads();
-    else {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-template <uint32_t PER, bool ALONE>
+template <uint32_t PER>
 __device__ __forceinline__ uint32_t route_select_row_per(float* p_lds, const RouteArgs& a, uint32_t row, bool shared_out) {
     const uint32_t lane = threadIdx.x & 63U, E = a.p.experts, K = a.p.top_k, P = K + a.p.shared_experts;
     float* z = a.scores + static_cast<size_t>(row) * E;
@@ -455,7 +446,7 @@ __device__ __forceinline__ uint32_t route_select_row_per(float* p_lds, const Rou
         const uint32_t e = lane + 64U * i;
         if (e < E) p_lds[e] = exp_of(a.p.exp_kind, v[i] - m);
     }
-    select_sync<ALONE>();
+    __syncthreads();
     // denominator: ascending expert order from 0, computed by every lane (LDS broadcast reads, 16 values fetched ahead)
     float total = 0.0F;
     {
@@ -513,16 +504,15 @@ __device__ __forceinline__ uint32_t route_select_row_per(float* p_lds, const Rou
         a.ids[static_cast<size_t>(row) * P + lane] = my_id;
         a.weights[static_cast<size_t>(row) * P + lane] = a.p.shared_slot_weights ? a.p.shared_slot_weights[static_cast<size_t>(row) * a.p.shared_experts + (lane - K)] : 1.0F;
     }
-    select_sync<ALONE>();
+    __syncthreads();
     return my_id;
 }
-template <bool ALONE = true>
 __device__ __forceinline__ uint32_t route_select_row(float* p_lds, const RouteArgs& a, uint32_t row, bool shared_out = false) {
     const uint32_t E = a.p.experts;
-    if (E <= 128U) return route_select_row_per<2, ALONE>(p_lds, a, row, shared_out);
-    if (E <= 256U) return route_select_row_per<4, ALONE>(p_lds, a, row, shared_out);
-    if (E <= 512U) return route_select_row_per<8, ALONE>(p_lds, a, row, shared_out);
-    return route_select_row_per<16, ALONE>(p_lds, a, row, shared_out);
+    if (E <= 128U) return route_select_row_per<2>(p_lds, a, row, shared_out);
+    if (E <= 256U) return route_select_row_per<4>(p_lds, a, row, shared_out);
+    if (E <= 512U) return route_select_row_per<8>(p_lds, a, row, shared_out);
+    return route_select_row_per<16>(p_lds, a, row, shared_out);
 }
 
 }  // namespace strix950

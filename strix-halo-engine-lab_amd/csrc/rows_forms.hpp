@@ -256,7 +256,7 @@ int32_t mi355_moe_strided_enqueue_csr(const mi355_moe_weights* w, const mi355_mo
     mi355_moe_weights wv; RowsK k;
     if (const int32_t rc = check_strided(w, v, rows, wv, k, false)) return rc;
     hipStream_t st = hs(stream);
-    launch_plan(RoutesView{k.routes, k.routes_rs, wv.top_k}, wv.experts, rows * wv.top_k, plan_split(wv, rows), item_bound(wv, rows), v->plan, st);
+    launch_plan(PlanArgs{RoutesView{k.routes, k.routes_rs, wv.top_k}, wv.experts, rows * wv.top_k, plan_split(wv, rows), item_bound(wv, rows), v->plan}, st);
     strided_job_status_kernel<<<1, 1024, 0, st>>>(v->status, rows, v->job_status);
     STRIX_LAUNCHED("moe strided plan");
     return MI355_OK;

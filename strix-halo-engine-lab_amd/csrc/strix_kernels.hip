@@ -12,6 +12,7 @@
 #include "device_math.hpp"
 #include "host_common.hpp"
 #include "launchers.hpp"
+#include "plan_block.hpp"
 #include "plan_layout.hpp"
 #include "q4k_rows.hpp"
 #include "q4k_blocks.hpp"
@@ -272,151 +273,10 @@ __global__ __launch_bounds__(64) __attribute__((aligned(65536))) void route_deco
 // ======================================================================================================== expert plan
 // (layout of the plan words: see the router section above)
 
-// The routes of a batch as the plan kernels read them: assignment a = row a / top_k, slot a % top_k, rows `rs` bytes apart.
-struct RoutesView {
-    const uint32_t* base;
-    uint64_t rs;
-    uint32_t top_k;
-    __device__ __forceinline__ uint32_t at(uint32_t a) const {
-        if (rs == 4ULL * top_k) return base[a];
-        const uint32_t row = a / top_k;
-        return reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(base) + row * rs)[a - row * top_k];
-    }
-};
-inline RoutesView dense_routes(const uint32_t* routes, uint32_t top_k) { return RoutesView{routes, 4ULL * top_k, top_k}; }
-
-// Stable order of a large batch: one 16-wave workgroup per expert. Every wave owns a contiguous sixteenth of the assignments:
-// it first counts its own assignments of the expert (ballot + population count, 64 at a time), the counts of the waves before
-// it give its first position, and a second walk places them in index order (the offsets are already in the plan).
-__global__ __launch_bounds__(1024) void plan_order_kernel(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t* plan) {
-    __shared__ uint32_t wave_count[16];
-    const uint32_t e = blockIdx.x, lane = threadIdx.x & 63U, wave = threadIdx.x >> 6;
-    const uint32_t first = plan[kPlanOffsetsAt + e], end = plan[kPlanOffsetsAt + e + 1];
-    if (first == end) return;                                   // uniform over the workgroup
-    const uint32_t per = ((assignments + 15U) / 16U + 63U) & ~63U;
-    const uint32_t lo = wave * per < assignments ? wave * per : assignments, hi = lo + per < assignments ? lo + per : assignments;
-    uint32_t mine_total = 0;
-    for (uint32_t a0 = lo; a0 < hi; a0 += 64U) {
-        const uint32_t a = a0 + lane;
-        mine_total += static_cast<uint32_t>(__popcll(__ballot(a < hi && routes.at(a) == e)));
-    }
-    if (lane == 0) wave_count[wave] = mine_total;
-    __syncthreads();
-    uint32_t at = first;
-    for (uint32_t w = 0; w < wave; ++w) at += wave_count[w];
-    const uint32_t stop = at + mine_total;
-    uint32_t* order = plan + plan_order_at(experts);
-    for (uint32_t a0 = lo; a0 < hi && at < stop; a0 += 64U) {
-        const uint32_t a = a0 + lane;
-        const bool mine = a < hi && routes.at(a) == e;
-        const uint64_t votes = __ballot(mine);
-        if (mine) order[at + __popcll(votes & ((1ULL << lane) - 1ULL))] = a;
-        at += static_cast<uint32_t>(__popcll(votes));
-    }
-}
-
-// Inclusive prefix sum over a wavefront: row shifts inside the rows of 16, then the rows' totals by row broadcasts (DPP, no LDS).
-__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x111, 0xF, 0xF, false));      // row_shr:1
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x112, 0xF, 0xF, false));      // row_shr:2
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x114, 0xF, 0xF, false));      // row_shr:4
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x118, 0xF, 0xF, false));      // row_shr:8
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x142, 0xA, 0xF, false));      // row_bcast:15 into rows 1 and 3
-    v += static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x143, 0xC, 0xF, false));      // row_bcast:31 into rows 2 and 3
-    return v;
-}
-// Lanes of the wavefront whose key (of `bits` bits) equals this lane's, among the lanes that `take` part: a ballot per bit.
-__device__ __forceinline__ uint64_t lanes_of_key(uint32_t key, uint32_t bits, bool take) {
-    uint64_t same = __ballot(take);
-    for (uint32_t b = 0; b < bits; ++b) {
-        const bool set = (key >> b) & 1U;
-        const uint64_t votes = __ballot(set);
-        same &= set ? votes : ~votes;
-    }
-    return same;
-}
-
-// The expert plan in one workgroup: thread e owns expert e (its count, three prefix sums for the offsets, the item numbers and the touched
-// list, then its own items). A batch of at most 1024 assignments (fill_order) is ordered here as well: wave w holds assignments
-// 64 w .. 64 w + 63, finds each one's position among its wave's assignments of the same expert by ballots (one per bit of the expert)
-// and leaves the wave's counts; a prefix over the waves and the expert's offset make it the position in the order. (A thread per expert
-// that walked every assignment took 12 us at 128 assignments; the order launch it saves at 257..1024 takes 4.7 us.) Bound by latency: the
-// prefix sums by DPP with one hand-off through LDS for all three, 320 assignments over 128 experts 8.3 -> 4.9 us.
-constexpr uint32_t kPlanSmall = 1024;
-__global__ __launch_bounds__(1024) void plan_kernel(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split,
-                                                    uint32_t item_bound, uint32_t fill_order, uint32_t* plan) {
-    __shared__ uint32_t count[kRouteMaxExperts];           // per expert: assignments, later (fill_order) its offset
-    __shared__ uint16_t wave_counts[16][kRouteMaxExperts]; // fill_order: per wave and expert, later the prefix over the waves before
-    __shared__ u32x4 wave_totals[16];                      // per wave: assignments, items, touched experts, largest group
-    const uint32_t tid = threadIdx.x, lane = tid & 63U, wave = tid >> 6, waves = (assignments + 63U) / 64U;
-    count[tid] = 0;
-    uint32_t mine = experts, rank = 0;                     // fill_order: this thread's assignment's expert, its position in the wave
-    if (fill_order) {
-        for (uint32_t w = 0; w < waves; ++w) wave_counts[w][tid] = 0;
-        if (tid < assignments) mine = routes.at(tid);
-    }
-    __syncthreads();
-    if (fill_order) {
-        const uint64_t same = lanes_of_key(mine, 32U - static_cast<uint32_t>(__builtin_clz(experts)), mine < experts);
-        if (mine < experts) {
-            rank = static_cast<uint32_t>(__popcll(same & ((1ULL << lane) - 1ULL)));
-            if (rank == 0) wave_counts[wave][mine] = static_cast<uint16_t>(__popcll(same));
-        }
-    } else {
-        for (uint32_t a = tid; a < assignments; a += 1024U) {
-            const uint32_t e = routes.at(a);
-            if (e < experts) atomicAdd(&count[e], 1U);
-        }
-    }
-    __syncthreads();
-    uint32_t c = tid < experts ? count[tid] : 0U;
-    if (fill_order && tid < experts) {
-        for (uint32_t w = 0; w < waves; ++w) {
-            const uint32_t here = wave_counts[w][tid];
-            wave_counts[w][tid] = static_cast<uint16_t>(c);
-            c += here;
-        }
-    }
-    const uint32_t pieces = (c + split - 1U) / split;
-    const uint32_t runs = wave_inclusive_scan(c), items_to = wave_inclusive_scan(pieces), touched_to = static_cast<uint32_t>(__popcll(__ballot(c != 0) & ((2ULL << lane) - 1ULL)));
-    uint32_t largest = c;
-#pragma unroll
-    for (int d = 32; d; d >>= 1) {
-        const uint32_t other = __shfl_xor(largest, d);
-        largest = other > largest ? other : largest;
-    }
-    if (lane == 63U) wave_totals[wave] = u32x4{runs, items_to, touched_to, largest};
-    __syncthreads();
-    u32x4 before = {0U, 0U, 0U, 0U}, all = {0U, 0U, 0U, 0U};
-#pragma unroll
-    for (uint32_t w = 0; w < 16U; ++w) {
-        const u32x4 t = wave_totals[w];
-        if (w < wave) { before.x += t.x; before.y += t.y; before.z += t.z; }
-        all.x += t.x; all.y += t.y; all.z += t.z; all.w = t.w > all.w ? t.w : all.w;
-    }
-    const uint32_t first = before.x + runs - c, item_from = before.y + items_to - pieces, touched_from = before.z + touched_to - (c != 0 ? 1U : 0U);
-    const uint32_t run = all.x, made = all.y, touched = all.z, most = all.w;
-    uint32_t* offsets = plan + kPlanOffsetsAt;
-    uint32_t* touched_ids = plan + plan_touched_at(experts);
-    uint32_t* order = plan + plan_order_at(experts);
-    uint32_t* items = plan + plan_items_at(experts, assignments);
-    if (tid < experts) {
-        offsets[tid] = first;
-        if (c != 0) {
-            touched_ids[touched_from] = tid;
-            for (uint32_t b = 0, k = item_from; b < c; b += split, ++k)
-                *reinterpret_cast<uint4*>(items + 4U * k) = make_uint4(tid, first + b, first + (b + split < c ? b + split : c), 0U);
-        }
-    }
-    for (uint32_t u = made + tid; u < item_bound; u += 1024U) *reinterpret_cast<uint4*>(items + 4U * u) = make_uint4(0U, 0U, 0U, 0U);
-    if (tid == 0) {
-        offsets[experts] = run;
-        plan[0] = assignments; plan[1] = touched; plan[2] = most; plan[4] = made;
-    }
-    if (!fill_order) return;                               // large batches: plan_order_kernel follows
-    count[tid] = first;
-    __syncthreads();
-    if (mine < experts) order[count[mine] + wave_counts[wave][mine] + rank] = tid;
+// A plan in a launch of its own.
+__global__ __launch_bounds__(1024) void plan_kernel(PlanArgs p) {
+    __shared__ PlanLds lds;
+    plan_block(lds, p, blockIdx.x);
 }
 
 // ======================================================================================================== Q4_K x A8 rows
@@ -1671,12 +1531,9 @@ inline void launch_mma_gate_up(const mi355_moe_weights& w, const RowsK& r, uint3
                                                                                 r.down_sums, r.h_out, r.status, r.job_status);
 }
 
-inline void launch_plan(RoutesView routes, uint32_t experts, uint32_t assignments, uint32_t split, uint32_t bound, uint32_t* plan,
-                        hipStream_t st) {
-    // past an assignment per thread of plan_kernel, a workgroup per expert orders its assignments in a launch of its own
-    const bool large = assignments > kPlanSmall;
-    plan_kernel<<<1, 1024, 0, st>>>(routes, experts, assignments, split, bound, large ? 0U : 1U, plan);
-    if (large) plan_order_kernel<<<experts, 1024, 0, st>>>(routes, experts, assignments, plan);
+inline void launch_plan(const PlanArgs& p, hipStream_t st) {
+    const uint32_t waves = (p.assignments + 63U) / 64U;
+    plan_kernel<<<p.experts, 64U * (waves < 16U ? waves : 16U), 0, st>>>(p);
 }
 // Decode batches of at most this many assignments (six tokens at top-8) run the 16-rows-per-wavefront sweep (q4k_quads.hpp),
 // with a 4-slot ring up to 16 assignments and a 2-slot ring above (every workgroup of the launch stays resident); measured
@@ -1975,12 +1832,16 @@ namespace {
 RouteCheck route_check(const mi355_moe_weights& wv, const mi355_moe_rows& r) {
     return RouteCheck{r.routes, r.route_weights, wv.experts, wv.top_k, r.status, r.job_status};
 }
-int32_t enqueue_prologue_rows(const mi355_moe_weights& wv, const mi355_moe_rows& r, uint32_t rows, const RouteArgs* select, hipStream_t st) {
+PlanArgs batch_plan(const mi355_moe_weights& wv, const mi355_moe_rows& r, uint32_t rows) {
+    return PlanArgs{dense_routes(r.routes, wv.top_k), wv.experts, rows * wv.top_k, plan_split(wv, rows), item_bound(wv, rows), r.plan};
+}
+// plan: the batch's plan as well
+int32_t enqueue_prologue_rows(const mi355_moe_weights& wv, const mi355_moe_rows& r, uint32_t rows, bool plan, hipStream_t st) {
     STRIX_REQUIRE(r.codes && r.deltas, "A8: null pointer");
     STRIX_REQUIRE(rows <= 65535U, "A8: at most 65535 rows per call");
     const bool vec = aligned(r.input, 16) && r.input_stride % 16U == 0 && aligned(r.codes, 8);
     launch_prologue_rows(A8RowArgs{static_cast<const uint8_t*>(r.input), r.input_stride, wv.hidden, r.codes, r.deltas, r.sums, nullptr, kA8StatusNone, vec, 0U},
-                         r.input_kind, rows, select, route_check(wv, r), st);
+                         r.input_kind, rows, route_check(wv, r), plan ? batch_plan(wv, r, rows) : PlanArgs{}, st);
     STRIX_LAUNCHED("moe prologue");
     return MI355_OK;
 }
@@ -1990,13 +1851,13 @@ int32_t mi355_moe_enqueue_prologue(const mi355_moe_weights* w, const mi355_moe_r
     mi355_moe_weights wv;
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;
     STRIX_REQUIRE(r->input && r->input_kind <= MI355_INPUT_BF16, "moe prologue: input view invalid");
-    return enqueue_prologue_rows(wv, *r, rows, nullptr, hs(stream));
+    return enqueue_prologue_rows(wv, *r, rows, false, hs(stream));
 }
 
 int32_t mi355_moe_enqueue_csr(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, mi355_stream stream) {
     mi355_moe_weights wv;
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;
-    launch_plan(dense_routes(r->routes, wv.top_k), wv.experts, rows * wv.top_k, plan_split(wv, rows), item_bound(wv, rows), r->plan, hs(stream));
+    launch_plan(batch_plan(wv, *r, rows), hs(stream));
     STRIX_LAUNCHED("moe plan");
     return MI355_OK;
 }
@@ -2048,10 +1909,8 @@ int32_t mi355_moe_enqueue(const mi355_moe_weights* w, const mi355_moe_rows* r, u
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;   // the whole bundle is validated before the first enqueue
     STRIX_REQUIRE(form <= MI355_COMBINE_MULADD_ASCENDING_EXPERT, "moe: unknown combine form");
     STRIX_REQUIRE(r->input && r->input_kind <= MI355_INPUT_BF16, "moe: input view invalid");
-    if (const int32_t rc = mi355_moe_enqueue_prologue(w, r, rows, stream)) return rc;
     // a dense matrix on the pair-per-lane sweep reads no expert plan
-    if (!(dense_pairs_ok(wv, rows) && r->gate_out && r->up_out))
-        if (const int32_t rc = mi355_moe_enqueue_csr(w, r, rows, stream)) return rc;
+    if (const int32_t rc = enqueue_prologue_rows(wv, *r, rows, !(dense_pairs_ok(wv, rows) && r->gate_out && r->up_out), hs(stream))) return rc;
     if (const int32_t rc = mi355_moe_enqueue_project(w, r, rows, stream)) return rc;
     // a dense top-1 job: the down launch publishes each row's output with its one unweighted value (no merge launch)
     RowsK k = rows_k(*r, wv);
@@ -2067,15 +1926,13 @@ int32_t mi355_moe_enqueue(const mi355_moe_weights* w, const mi355_moe_rows* r, u
 namespace {
 // mi355_moe_enqueue by halves: front = prologue, plan, gate / up; back = down rows, combine.
 int32_t enqueue_staged(const mi355_moe_weights* w, const mi355_moe_rows* r, uint32_t rows, uint32_t form, mi355_stream stream, bool do_front, bool do_back,
-                       uint32_t shared_slots = 0, const RouteArgs* select = nullptr) {
+                       uint32_t shared_slots = 0) {
     mi355_moe_weights wv;
     if (const int32_t rc = check_moe(w, r, rows, wv)) return rc;
     STRIX_REQUIRE(form <= MI355_COMBINE_MULADD_ASCENDING_EXPERT, "moe: unknown combine form");
     if (do_front) {
         STRIX_REQUIRE(r->input && r->input_kind <= MI355_INPUT_BF16, "moe: input view invalid");
-        if (const int32_t rc = enqueue_prologue_rows(wv, *r, rows, select, hs(stream))) return rc;
-        if (!(dense_pairs_ok(wv, rows) && r->gate_out && r->up_out))
-            if (const int32_t rc = mi355_moe_enqueue_csr(w, r, rows, stream)) return rc;
+        if (const int32_t rc = enqueue_prologue_rows(wv, *r, rows, !(dense_pairs_ok(wv, rows) && r->gate_out && r->up_out), hs(stream))) return rc;
         if (const int32_t rc = mi355_moe_enqueue_project(w, r, rows, stream)) return rc;
     }
     if (!do_back) return MI355_OK;
@@ -2150,16 +2007,13 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         RouteArgs a{};
         a.p = *p; a.x = static_cast<const uint8_t*>(staged.input); a.kind = staged.input_kind; a.x_stride = staged.input_stride; a.rows = rows; a.hidden = wv.hidden;
         a.wr = router_weight; a.bias = logit_bias; a.ids = ids; a.weights = weights; a.scores = scores;
-        // the selection rides in the prologue's launch while that is one round of workgroups: its registers let a compute unit hold one
-        // (40 rows: 157.8 -> 154.4 us a layer; 1000 rows, four rounds: 631 -> 636 us, hence the line)
-        const bool fused_select = rows <= compute_units();
         if (do_front) {
             if (const int32_t rc = check_route(p, staged.input, staged.input_kind, wv.hidden, staged.input_stride, router_weight, ids, weights, scores)) return rc;
             launch_route_logits(a, st);
-            if (!fused_select) launch_route_select(a, st);
+            launch_route_select(a, st);
             STRIX_LAUNCHED("moe layer router");
         }
-        return enqueue_staged(w, &staged, rows, form, stream, do_front, do_back, p->shared_experts, fused_select ? &a : nullptr);
+        return enqueue_staged(w, &staged, rows, form, stream, do_front, do_back, p->shared_experts);
     }
     RouteArgs a{};
     a.p = *p; a.x = static_cast<const uint8_t*>(r->input); a.kind = r->input_kind; a.x_stride = r->input_stride; a.rows = rows; a.hidden = wv.hidden;
@@ -2296,7 +2150,7 @@ struct PrefillViews {
 // sums (null: they are already written)
 int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v, uint32_t rows, hipStream_t st, const RouteCheck* check = nullptr) {
     const uint32_t assignments = rows * wv.top_k, split = prefill_split(wv, assignments), bound = plan_item_bound(wv.experts, assignments, split);
-    launch_plan(v.routes, wv.experts, assignments, split, bound, v.plan, st);
+    const PlanArgs plan{v.routes, wv.experts, assignments, split, bound, v.plan};
     PrefillArgs a{};
     a.top_k = wv.top_k; a.exp_kind = wv.exp_kind; a.swiglu_limit = wv.swiglu_limit; a.x = static_cast<const uint8_t*>(v.input); a.x_stride = v.input_stride;
     uint8_t* ws = static_cast<uint8_t*>(v.h_f16);
@@ -2306,7 +2160,7 @@ int32_t enqueue_prefill_core(const mi355_moe_weights& wv, const PrefillViews& v,
     a.x_sums = x_sums;
     a.rawdots = v.rawdots; a.rawdots_rs = v.rawdots_rs; a.rawdots_bf16 = v.rawdots_bf16; a.plan = v.plan; a.experts = wv.experts; a.assignments = assignments;
     a.status = v.status; a.status_rs = v.status_rs; a.job_status = v.job_status; a.items = bound;
-    launch_prefill_products(wv, a, rows, x_sums, check, plan_items_at(wv.experts, assignments), plan_order_at(wv.experts), st);
+    launch_prefill_products(wv, a, rows, x_sums, check, plan, plan_items_at(wv.experts, assignments), plan_order_at(wv.experts), st);
     STRIX_LAUNCHED("moe prefill f16");
     return MI355_OK;
 }

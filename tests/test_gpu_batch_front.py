@@ -47,6 +47,33 @@ def test_plan_order(strix, rows, top_k, experts, skew):
     assert np.array_equal(covered, np.arange(A)) and all(offsets[e] <= b < z <= offsets[e + 1] for e, b, z, _ in items)
 
 
+# the plan that is made beside the rows of a batch, in the launch that quantises them or sums them for the prefill: around a turn of 64 assignments a
+# wavefront, the eight turns it asks for together and more; experts that nothing chose, ids of no expert
+@pytest.mark.parametrize("rows,top_k,experts", [(3, 1, 2), (17, 4, 1024), (65, 4, 5), (513, 8, 300), (600, 16, 40), (4200, 3, 3)])
+@pytest.mark.parametrize("prefill", [False, True])
+def test_plan_beside_the_rows(strix, rows, top_k, experts, prefill):
+    rng = np.random.default_rng(rows + experts)
+    ids = np.minimum(rng.integers(0, experts, (rows, top_k)), rng.integers(0, experts, (rows, top_k)))
+    ids[rows // 2, 0] = experts + 3
+    H = I = 256
+    w = torch.zeros((experts * 256, 144), dtype=torch.uint8, device="cuda")
+    layer = strix.MoeLayer(H, I, experts, top_k, w, w, w, rows, prefill_f16=prefill)
+    x, routes, ones = torch.zeros((rows, H), device="cuda", dtype=torch.float16), torch.from_numpy(ids.astype(np.int32)).cuda(), torch.ones((rows, top_k), device="cuda")
+    (layer.run_prefill_f16 if prefill else layer.run)(x, routes, ones)
+    plan = layer.plan.cpu().numpy()
+    flat, A = ids.reshape(-1), rows * top_k
+    counts = np.bincount(flat[flat < experts], minlength=experts)
+    offsets, order_at = np.concatenate([[0], np.cumsum(counts)]), PLAN_OFFSETS_AT + pad4(experts + 1) + pad4(experts)
+    assert plan[0] == A and plan[1] == np.count_nonzero(counts) and plan[2] == counts.max()
+    assert np.array_equal(plan[PLAN_OFFSETS_AT:PLAN_OFFSETS_AT + experts + 1], offsets)
+    assert np.array_equal(plan[PLAN_OFFSETS_AT + pad4(experts + 1):][:plan[1]], np.nonzero(counts)[0])
+    order = np.argsort(np.where(flat < experts, flat, experts), kind="stable")[:A - 1]
+    assert np.array_equal(plan[order_at:order_at + A - 1], order)
+    items = plan[order_at + pad4(A):][:4 * plan[4]].reshape(-1, 4)
+    assert np.array_equal(np.concatenate([np.arange(b, e) for _, b, e, _ in items]), np.arange(A - 1)) and all(offsets[e] <= b < z <= offsets[e + 1] for e, b, z, _ in items)
+    assert [bool(s & strix.STATUS_INVALID_ROUTE) for s in layer.status[:rows].cpu().tolist()] == [r == rows // 2 for r in range(rows)]
+
+
 # widths around the image's 448 threads of eight values; experts around the selection's register steps; a row with an infinity
 # (its weights are not finite either: both status bits), rows past and within the decode sizes (large experts: shared sweeps)
 @pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(17, 256, 256, 5, 2), (40, 3584, 256, 130, 8), (33, 3840, 256, 16, 4), (18, 8192, 256, 20, 16), (16, 6144, 1280, 24, 8)])
