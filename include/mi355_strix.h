@@ -296,13 +296,12 @@ void mi355_debug_down_merge_flat(uint32_t on);
 int32_t mi355_shared_gate(const void* x, uint32_t input_kind, uint32_t rows, uint32_t hidden, uint64_t x_stride_bytes,
                           const float* scalar_weight, uint32_t exp_kind, float* gate, uint64_t gate_stride, mi355_stream);
 
-/* The layer with the RMSNorm of its input inside the first launch (the reference normalises the residual stream in front of
+/* The layer with the RMSNorm of its input in front (the reference normalises the residual stream in front of
  * the MoE, src/ops/norm/norm.hpp:40-58, and runs the shared expert beside the routed ones, src/hip_shared_expert_launcher.hip):
  * rows->input holds the raw rows; the router, the A8 image and the experts see y = (x * r) * norm_weight,
  * r = 1 / sqrt(mean(x^2) + norm_eps), bit for bit mi355_rmsnorm_f32 (lane-strided fma chains, LDS halving) followed by
  * mi355_moe_enqueue_layer on y; norm_weight may be NULL (unit scale). normed: fp32 [rows][hidden], receives y (the input of
- * anything else that reads the normalised rows). For rows <= 16 every workgroup of the router / prologue launch derives its
- * row's r itself, so no launch is added; larger batches run one norm launch first.
+ * anything else that reads the normalised rows). One norm launch runs first.
  * A shared expert stored as expert `experts` of the same tensors is the policy's shared_experts = 1: every row then carries
  * one more slot with weight 1, its gate / up / down rows are swept once per four rows, and the ordered combine adds it last. */
 int32_t mi355_moe_enqueue_layer_normed(const mi355_route_policy* policy, const float* router_weight, const float* logit_bias,

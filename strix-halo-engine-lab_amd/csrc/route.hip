@@ -61,21 +61,22 @@ void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, cons
 
 void launch_route_select(const RouteArgs& a, hipStream_t st) { route_select_kernel<<<a.rows, 64, 0, st>>>(a); }
 
-// RMSNorm of rows of any input kind into fp32 rows (the staged form of the fused norm): rmsnorm_f32_kernel's order.
-template <int KIND>
+// RMSNorm of rows of any input kind into fp32 rows (the staged form of the fused norm), bit for bit rmsnorm_f32_kernel: lane l of L = 256
+// (n >= 512) or 128 chains fma(x, x, a) over x[l], x[l + L], ...; the L partial sums are halved, l with l + 128, l + 64, ..., l + 1.
+// A thread per chain. Bound by latency: the HELD first values of a chain and their weights are asked for at once and kept (one by one past
+// the first eight, 1 row of 2048 fp16 values, 8 of 3072, 1 of 4096, 3 of 6144: 5.5, 8.5, 11, 16 us, now 2.2, 2.7, 4.7, 4.0), and every wave
+// halves the sums by itself, in registers (1 barrier for 9).
+template <int KIND, uint32_t HELD>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const uint8_t* x, uint64_t x_stride, const float* w, uint32_t n, float eps, float* y) {
-    // row_norm_factor's chains and halvings, a thread per chain. Bound by latency: the first eight values of a chain and their weights are
-    // asked for at once and kept (one row of 2048 by one wavefront, element after element: 21 us).
-    constexpr uint32_t HELD = 8U;
     __shared__ float partial[256];
     const uint8_t* xr = x + blockIdx.x * x_stride;
-    const uint32_t l = threadIdx.x, L = n >= 512U ? 256U : 128U, end = l < L ? n : 0U;
+    const uint32_t l = threadIdx.x, lane = l & 63U, L = n >= 512U ? 256U : 128U, end = l < L ? n : 0U;
     float v[HELD], wv[HELD], a = 0.0F;
 #pragma unroll
     for (uint32_t j = 0; j < HELD; ++j) {
-        const uint32_t i = l + L * j;
-        v[j] = i < end ? load_activation<KIND>(xr, i) : 0.0F;
-        wv[j] = w && i < end ? w[i] : 0.0F;
+        const uint32_t i = min(l + L * j, n - 1U);  // (no branch a value: the conversion in it would wait for its load)
+        v[j] = load_activation<KIND>(xr, i);
+        wv[j] = w ? w[i] : 0.0F;
     }
 #pragma unroll
     for (uint32_t j = 0; j < HELD; ++j)
@@ -85,12 +86,11 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const uint8_t* x, uin
         a = __builtin_fmaf(u, u, a);
     }
     partial[l] = a;
-    for (uint32_t h = L / 2U; h > 0; h >>= 1) {
-        __syncthreads();
-        if (l < h) partial[l] = partial[l] + partial[l + h];
-    }
     __syncthreads();
-    const float r = 1.0F / __builtin_sqrtf(partial[0] / static_cast<float>(n) + eps);
+    float sum = L == 256U ? (partial[lane] + partial[lane + 128U]) + (partial[lane + 64U] + partial[lane + 192U]) : partial[lane] + partial[lane + 64U];
+    sum = sum + __shfl_xor(sum, 32);
+    sum = sum + xor16_f(sum); sum = sum + xor8_f(sum); sum = sum + xor4_f(sum); sum = sum + xor2_f(sum); sum = sum + xor1_f(sum);
+    const float r = 1.0F / __builtin_sqrtf(sum / static_cast<float>(n) + eps);
     float* yr = y + static_cast<size_t>(blockIdx.x) * n;
 #pragma unroll
     for (uint32_t j = 0; j < HELD; ++j)
@@ -103,9 +103,15 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const uint8_t* x, uin
 
 void launch_norm_rows(const void* x, uint32_t kind, uint64_t x_stride, const float* weight, uint32_t hidden, float eps, float* normed, uint32_t rows, hipStream_t st) {
     const uint8_t* at = static_cast<const uint8_t*>(x);
-    if (kind == MI355_INPUT_F32) rmsnorm_rows_kernel<0><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
-    else if (kind == MI355_INPUT_F16) rmsnorm_rows_kernel<1><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
-    else rmsnorm_rows_kernel<2><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+    const auto launch = [&](auto held) {
+        constexpr uint32_t HELD = decltype(held)::value;
+        if (kind == MI355_INPUT_F32) rmsnorm_rows_kernel<0, HELD><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+        else if (kind == MI355_INPUT_F16) rmsnorm_rows_kernel<1, HELD><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+        else rmsnorm_rows_kernel<2, HELD><<<rows, 256, 0, st>>>(at, x_stride, weight, hidden, eps, normed);
+    };
+    if (hidden <= 2048U) launch(std::integral_constant<uint32_t, 8>{});
+    else if (hidden <= 4096U) launch(std::integral_constant<uint32_t, 16>{});
+    else launch(std::integral_constant<uint32_t, 32>{});
 }
 
 }  // namespace strix950

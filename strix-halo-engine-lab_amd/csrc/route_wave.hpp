@@ -30,37 +30,11 @@ struct RouteArgs {
     // fused decode extras (all null / zero for the plain router)
     int8_t* codes; float* deltas; int32_t* sums; uint32_t* status; uint32_t* job_status; uint32_t* plan;
     uint32_t route_blocks, quant_blocks;
-    // RMSNorm of the input rows inside the launch (norm_on): the router and the A8 image see y = (x * r) * norm_w, r = 1 / sqrt(mean(x^2) + eps)
-    // in the declared order of src/cpu/core/reference.cpp:86-103; normed (optional) receives y as fp32 [rows][hidden]
-    uint32_t norm_on; const float* norm_w; float norm_eps; float* normed;
     // early-routes form (route_early.hpp): one word per assignment - the count of finished projection waves in the low half, a
     // non-finite projection in bit 31 -, and a test knob that displaces the early logits so that the repair path runs
     uint32_t* awords; uint32_t early_perturb;
     float* early_logits; uint32_t early_stride;      // where the early logits of row i go: early_logits + i * early_stride (floats)
 };
-
-// r of one row by a 64-thread workgroup, bit for bit rmsnorm_f32_kernel: lane l of L = 256 (n >= 512) or 128 chains
-// fma(x, x, a) over x[l], x[l + L], ...; the L partial sums are halved in LDS; thread t stands for lanes t, t + 64, ...
-template <int KIND>
-__device__ __forceinline__ float row_norm_factor(float* partial /* 256 floats of LDS */, const uint8_t* xrow, uint32_t n, float eps) {
-    const uint32_t t = threadIdx.x & 63U, L = n >= 512U ? 256U : 128U;
-    for (uint32_t l = t; l < L; l += 64U) {
-        float a = 0.0F;
-        for (uint32_t i = l; i < n; i += L) {
-            const float v = load_activation<KIND>(xrow, i);
-            a = __builtin_fmaf(v, v, a);
-        }
-        partial[l] = a;
-    }
-    for (uint32_t h = L / 2U; h > 0; h >>= 1) {
-        __syncthreads();
-        for (uint32_t l = t; l < h; l += 64U) partial[l] = partial[l] + partial[l + h];
-    }
-    __syncthreads();
-    const float r = 1.0F / __builtin_sqrtf(partial[0] / static_cast<float>(n) + eps);
-    __syncthreads();
-    return r;
-}
 
 // ---------------------------------------------------------------------------------------------------- logit chains
 // Logits of 8 experts x 8 rows -> scores[row][expert] (used as the logit workspace). hidden % 32 == 0.
@@ -179,31 +153,20 @@ __device__ __forceinline__ void route_logits_block(RouteLds& lds, const RouteArg
 constexpr uint32_t kChainChunk = 512;                 // features per ring slot
 constexpr uint32_t kChainPitch = kChainChunk + 4;     // floats; +16 bytes keeps the 8 weight rows on different banks
 constexpr uint32_t kChainExperts = 8;
-template <bool NORM>
-struct __attribute__((aligned(16))) ChainSlotT {
+struct __attribute__((aligned(16))) ChainSlot {
     float w[kChainExperts][kChainPitch];
     float x[kChainChunk];                             // the row's features as fp32
     uint32_t raw[kChainChunk / 2];                    // fp16 / bf16 input as copied (unused for fp32 input)
-    float nw[NORM ? kChainChunk : 4];                 // the norm weights of the chunk (fused RMSNorm only)
 };
-// Four slots of the plain form are 78,336 bytes: two one-wave workgroups fit a compute unit's 160 KB (with the norm weights: one).
-template <int KIND, bool NORM = false> constexpr uint32_t chain_copies() { return 2U * kChainExperts + (KIND == 0 ? 2U : 1U) + (NORM ? 2U : 0U); }
+// Four slots of the plain form are 78,336 bytes: two one-wave workgroups fit a compute unit's 160 KB.
+template <int KIND> constexpr uint32_t chain_copies() { return 2U * kChainExperts + (KIND == 0 ? 2U : 1U); }
 
 // Start the copy of features [k0, k0 + 512) of 8 router-weight rows and of the activation row. Every chunk issues the
 // same number of copy instructions (the waits count them): lanes past the end of the row re-fetch its last piece into
 // slot positions that are never read.
-template <int KIND, bool NORM = false>
-__device__ __forceinline__ void chain_start(ChainSlotT<NORM>& slot, const RouteArgs& a, uint32_t row, uint32_t e0, uint32_t k0) {
+template <int KIND>
+__device__ __forceinline__ void chain_start(ChainSlot& slot, const RouteArgs& a, uint32_t row, uint32_t e0, uint32_t k0) {
     const uint32_t lane = threadIdx.x & 63U;
-    if constexpr (NORM) {       // (a null norm weight is a unit scale: the router weights stand in and are not used)
-        const float* nsrc = a.norm_w ? a.norm_w : a.wr;
-#pragma unroll
-        for (uint32_t j = 0; j < 2U; ++j) {
-            const uint32_t k = k0 + 256U * j + 4U * lane, kk = k + 4U <= a.hidden ? k : a.hidden - 4U;
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(nsrc + kk),
-                                             (__attribute__((address_space(3))) void*)(&slot.nw[256U * j]), 16, 0, 0);
-        }
-    }
 #pragma unroll
     for (uint32_t i = 0; i < kChainExperts; ++i) {
         const uint32_t e = e0 + i < a.p.experts ? e0 + i : a.p.experts - 1U;
@@ -234,21 +197,8 @@ __device__ __forceinline__ void chain_start(ChainSlotT<NORM>& slot, const RouteA
 // wavefront complete in order, so the writes only have to be issued before the reads - no barrier. __syncthreads() here
 // would also wait for every copy in flight, i.e. drain the three chunks the ring keeps ahead of the chain.
 __device__ __forceinline__ void chain_publish() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-template <int KIND, bool NORM = false>
-__device__ __forceinline__ void chain_widen(ChainSlotT<NORM>& slot, float factor = 1.0F, bool scaled = false) {
-    if constexpr (KIND == 0 && NORM) {
-        // fp32 rows arrive as they are: scale them in place, y = (x * r) * w
-        const uint32_t lane = threadIdx.x & 63U;
-#pragma unroll
-        for (uint32_t j = 0; j < 2U; ++j) {
-            f32x4 v = *reinterpret_cast<const f32x4*>(&slot.x[256U * j + 4U * lane]);
-            const f32x4 w = *reinterpret_cast<const f32x4*>(&slot.nw[256U * j + 4U * lane]);
-            v.x = v.x * factor; v.y = v.y * factor; v.z = v.z * factor; v.w = v.w * factor;
-            if (scaled) { v.x = v.x * w.x; v.y = v.y * w.y; v.z = v.z * w.z; v.w = v.w * w.w; }
-            *reinterpret_cast<f32x4*>(&slot.x[256U * j + 4U * lane]) = v;
-        }
-        chain_publish();
-    }
+template <int KIND>
+__device__ __forceinline__ void chain_widen(ChainSlot& slot) {
     if constexpr (KIND != 0) {
         const uint32_t lane = threadIdx.x & 63U;
         const u32x4 r = *reinterpret_cast<const u32x4*>(&slot.raw[4U * lane]);
@@ -258,13 +208,6 @@ __device__ __forceinline__ void chain_widen(ChainSlotT<NORM>& slot, float factor
         for (int q = 0; q < 4; ++q) {
             if constexpr (KIND == 1) { f[2 * q] = half_bits_to_float(h[q] & 0xffffU); f[2 * q + 1] = half_bits_to_float(h[q] >> 16); }
             else { f[2 * q] = f_of(h[q] << 16); f[2 * q + 1] = f_of(h[q] & 0xffff0000U); }
-        }
-        if constexpr (NORM) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                f[q] = f[q] * factor;
-                if (scaled) f[q] = f[q] * slot.nw[8U * lane + q];
-            }
         }
         *reinterpret_cast<f32x4*>(&slot.x[8U * lane]) = f32x4{f[0], f[1], f[2], f[3]};
         *reinterpret_cast<f32x4*>(&slot.x[8U * lane + 4U]) = f32x4{f[4], f[5], f[6], f[7]};
@@ -277,8 +220,7 @@ __device__ __forceinline__ void chain_widen(ChainSlotT<NORM>& slot, float factor
 // no instruction of its own). Measured on MI355X a wave pays ~5 cycles per dependent fma and ~9 per ds_read_b128, with no
 // overlap between them; operands are requested up to 48 features before they are chained.
 struct ChainStep { f32x4 w[4]; float x; };
-template <bool NORM>
-__device__ __forceinline__ void chain_load(ChainStep& s, const ChainSlotT<NORM>& slot, uint32_t el, uint32_t k) {
+__device__ __forceinline__ void chain_load(ChainStep& s, const ChainSlot& slot, uint32_t el, uint32_t k) {
     const float* wrow = slot.w[el] + k;
 #pragma unroll
     for (uint32_t i = 0; i < 4U; ++i) s.w[i] = *reinterpret_cast<const f32x4*>(wrow + 4U * i);
@@ -315,11 +257,10 @@ template <int N>
 __device__ __forceinline__ void chain_wait() { __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8)); }      // (and every LDS read returned: the next copy reuses a slot this wave has read)
 
 // Logits of experts [e0, e0 + 8) for one row -> scores[row][expert] (+ bias), stored for readers in other workgroups of
-// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects. NORM: the row's norm factor is computed here, in the fourth
-// slot, while the first three chunks are on their way.
-template <int KIND, bool NORM = false>
-__device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slots)[4], const RouteArgs& a, uint32_t row, uint32_t e0) {
-    constexpr uint32_t NI = chain_copies<KIND, NORM>();
+// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects.
+template <int KIND>
+__device__ __forceinline__ void route_chain_block(ChainSlot* const (&slots)[4], const RouteArgs& a, uint32_t row, uint32_t e0) {
+    constexpr uint32_t NI = chain_copies<KIND>();
     const uint32_t lane = threadIdx.x & 63U, chunks = (a.hidden + kChainChunk - 1U) / kChainChunk;
     const bool butterfly = a.p.logits_order == MI355_LOGITS_LANE32_BUTTERFLY;
     const uint32_t el = lane & 7U;                      // chain form: the lane's expert
@@ -327,12 +268,7 @@ __device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slot
     float acc = 0.0F, part[4] = {0.0F, 0.0F, 0.0F, 0.0F};
 #pragma unroll
     for (uint32_t s = 0; s < 3U; ++s)
-        if (s < chunks) chain_start<KIND, NORM>(*slots[s], a, row, e0, s * kChainChunk);
-    float r = 1.0F;
-    if constexpr (NORM) {
-        r = row_norm_factor<KIND>(reinterpret_cast<float*>(slots[3]), a.x + row * a.x_stride, a.hidden, a.norm_eps);
-        chain_publish();      // the scratch reads are complete before the ring reaches the fourth slot
-    }
+        if (s < chunks) chain_start<KIND>(*slots[s], a, row, e0, s * kChainChunk);
     for (uint32_t c0 = 0; c0 < chunks; c0 += 4U) {
 #pragma unroll
         for (uint32_t s = 0; s < 4U; ++s) {
@@ -343,13 +279,13 @@ __device__ __forceinline__ void route_chain_block(ChainSlotT<NORM>* const (&slot
                 if (ahead == 0) chain_wait<0>();
                 else if (ahead == 1) chain_wait<NI>();
                 else chain_wait<2 * NI>();
-                if (c + 3U < chunks) chain_start<KIND, NORM>(*slots[(s + 3U) % 4U], a, row, e0, (c + 3U) * kChainChunk);
-                ChainSlotT<NORM>& slot = *slots[s];
-                chain_widen<KIND, NORM>(slot, r, a.norm_w != nullptr);
+                if (c + 3U < chunks) chain_start<KIND>(*slots[(s + 3U) % 4U], a, row, e0, (c + 3U) * kChainChunk);
+                ChainSlot& slot = *slots[s];
+                chain_widen<KIND>(slot);
                 const uint32_t kc = a.hidden - c * kChainChunk < kChainChunk ? a.hidden - c * kChainChunk : kChainChunk;
                 if (!butterfly) {
-                    // full chunk: straight-line code, operands fetched three steps of 16 features ahead (against one step: layers without the
-                    // norm 0.2..0.4 us faster, e.g. hidden 3072, 8 rows 75.1 -> 74.9; with it the same, 89.7; logits alone 0.1 us slower of 30)
+                    // full chunk: straight-line code, operands fetched three steps of 16 features ahead (against one step: layers 0.2..0.4
+                    // us faster, e.g. hidden 3072, 8 rows 75.1 -> 74.9; logits alone 0.1 us slower of 30)
                     constexpr uint32_t AHEAD = 3U;
                     if (kc == kChainChunk) {
                         ChainStep S[AHEAD + 1U];
