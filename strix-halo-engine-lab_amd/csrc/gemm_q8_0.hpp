@@ -14,6 +14,8 @@
 // buffers while the other is multiplied; rows are pitched by 16 bytes so that eight neighbouring rows read different banks.
 // What bounds it now, at 4096 x 4096 and 64 x 64 tiles: a stage takes 0.8 us of products (two waves per SIMD, 192 full-rate vector
 // operations and six matrix operations each) and 0.55 us of copies that are not hidden; every workgroup pays about 5 us of start and end.
+// With every copy from the first cache 1000 rows of 8192 x 16384 take 743 us instead of 887; the vector operations alone are 460. A chain whose products and
+// operands were asked for a tile ahead (the factors as one v_mfma_f32_32x32x2_f32 a tile, twice the matrix time) waited less and issued no more: 967 us.
 // Copying global -> LDS without registers, four stages ahead (raw 34-byte blocks, shifted by the readers) measured 64 us at 500 rows
 // against 56: the readers' 32-bit LDS reads cost more than the copies they hide.
 // Measured, 4096 x 4096: 500 rows 323 -> 56 us, 1000 rows 640 -> 112 us, 32 rows 31 -> 13 us against the row sweep (gemv_q8_0_a8_kernel).
@@ -40,6 +42,11 @@ template <int KS, int NA, bool DW>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a8_view v, uint32_t o_tiles, uint32_t a_tiles) {
     constexpr uint32_t OT = gemm_out_rows<KS>(), AT = 32U * NA, G = gemm_groups<KS>(), P = gemm_pitch<KS>(), R = 32U / KS;
     constexpr uint32_t LEVELS = R == 8U ? 3U : 2U, ABLK = AT * G / kGemmThreads > 0U ? AT * G / kGemmThreads : 1U;
+    // The next stage's copies go to LDS in front of a stage's products, a stage after they were asked for, or behind them, half as long after. Tiles of
+    // 32 weight rows copy twice the bytes a product, so the wait counts there: before -> now, 100 rows of 8192 x 1024 39.1 -> 36.0 us, 300 rows of
+    // 4096 x 2048 41.7 -> 39.3, 50 rows of 4096 x 4096 23.3 -> 21.7, 32 rows 17.0 -> 16.7. Tiles of 64 lose: 4096 x 4096, 500 rows 62.2 -> 62.5,
+    // 8192 x 16384, 1000 rows 887 -> 893.
+    constexpr bool EARLY = KS == 8;
     static_assert(OT * G == kGemmThreads, "one weight block per thread and stage");
     __shared__ __attribute__((aligned(16))) uint8_t wbuf[2][OT * P];
     __shared__ __attribute__((aligned(16))) uint8_t abuf[2][AT * P];
@@ -155,11 +162,13 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
 
     fetch(0);
     stage(0);
+    if (EARLY) fetch(1);                                        // (R stages at least)
     __syncthreads();
     uint32_t in_pass = 0, pass = 0;
     for (uint32_t s = 0; s < stages; ++s) {
         const uint32_t buf = s & 1U;
-        if (s + 1U < stages) fetch(s + 1U);
+        if (EARLY && s + 1U < stages) stage(buf ^ 1U);
+        if (s + (EARLY ? 2U : 1U) < stages) fetch(s + (EARLY ? 2U : 1U));
         const bool second = 2U * in_pass + 1U < chunks;         // the stage's second chunk exists
         const mm_f32x32 none = {0};
         if constexpr (NA == 2) {                                // one factor product per group: its two blocks are the two activation tiles
@@ -199,7 +208,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
                 }
             }
         }
-        if (s + 1U < stages) stage(buf ^ 1U);
+        if (!EARLY && s + 1U < stages) stage(buf ^ 1U);
         __syncthreads();
     }
 
