@@ -100,6 +100,10 @@ __host__ __device__ constexpr uint32_t rg_stage_ops(int fmt, uint32_t nt, uint32
 __device__ __forceinline__ void copy16_to_lds_at(const uint8_t* src, uint32_t lds_at) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_at), "v"(src) : "memory", "m0");
 }
+// four bytes per lane (lane l lands at lds_at + 4 l)
+__device__ __forceinline__ void copy4_to_lds_at(const uint32_t* src, uint32_t lds_at) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds_at), "v"(src) : "memory", "m0");
+}
 
 struct Rg8 { u32x4 a, b; uint32_t e; };                   // Q8_0: a stage's words of a lane
 struct RgFactor { uint32_t sc; half2v mul, add; };
@@ -144,6 +148,18 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     pf_lds* const tok_stage[4] = {(pf_lds*)tok0, (pf_lds*)tok1, (pf_lds*)tok2, (pf_lds*)tok3};
     pf_lds* const s_tile = (pf_lds*)s_tile_mem;
 
+    // LIST: the workgroup's units, up to 64 at a time, are listed in LDS (expert, first row in plan order, rows, feature tile), and the assignments of a
+    // unit's rows are there before it starts. Asked for one after the other in front of a unit's first copy, item and assignments are two trips to
+    // memory that nothing hides, and the stores at its end wait for a third: 1000 rows of hidden 2048 / ffn 768 / 128 experts 296 -> 266 us, 4096 rows
+    // of hidden 4096 / ffn 2048 / 256 experts 3968 -> 3804. The four-wave form has one to three units a workgroup and two more of them beside
+    // it: the list costs it more than it saves (64 rows 95.9 -> 97.9 us), and so did copies that run on from a unit into the next (97.4; 333
+    // rows 162.2 -> 158.8, Q8_0 rows 169.5 -> 173.6).
+    constexpr bool LIST = WAVES == 8U;
+    __shared__ __attribute__((aligned(16))) uint4 unit_mem[LIST ? 64U : 1U];
+    __shared__ uint32_t unit_count;
+    __shared__ uint32_t order_mem[2][LIST ? TOKENS : 1U];
+    static_assert(!LIST || TOKENS % 64U == 0, "copies of whole waves");
+
     if (MODE == 1 && (*a.job_status & MI355_STATUS_NONFINITE_PROJECTION)) return;
     const uint32_t* order = a.plan + order_at;
     const uint32_t lane = threadIdx.x & 63U, wave = threadIdx.x >> 6, n31 = lane & 31U, half = lane >> 5;
@@ -158,14 +174,41 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     // TOKENS rows in either form (prefill_split).
     constexpr bool ROUND = WAVES == 4U;
     const uint32_t units = ROUND ? a.plan[4] * a.tiles : a.units;
-    for (uint32_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
-    const uint32_t q = unit >> 3;
-    const uint32_t item_index = ROUND ? unit / a.tiles : (q / a.tiles) * 8U + (unit & 7U), tile = (ROUND ? unit : q) % a.tiles;
-    if (item_index >= a.items) continue;
-    const uint4 item = *reinterpret_cast<const uint4*>(a.plan + items_at + 4U * item_index);
-    const uint32_t e = item.x, begin = item.y;
-    if (begin >= item.z) continue;
-    const uint32_t count = item.z - begin;
+    const auto item_of = [&](uint32_t unit) {           // (a unit that does not exist: no rows)
+        const uint32_t q = unit >> 3;
+        const uint32_t item_index = ROUND ? unit / a.tiles : (q / a.tiles) * 8U + (unit & 7U), at = (ROUND ? unit : q) % a.tiles;
+        uint4 item = {0U, 0U, 0U, 0U};
+        if (unit < units && item_index < a.items) item = *reinterpret_cast<const uint4*>(a.plan + items_at + 4U * item_index);
+        return uint4{item.x, item.y, item.y < item.z ? item.z - item.y : 0U, at};
+    };
+    const auto copy_assignments = [&](uint32_t u) {     // of listed unit u (past its rows: the last one's again)
+        if (wave_s >= TOKENS / 64U) return;
+        const uint4 item = unit_mem[u];
+        copy4_to_lds_at(order + item.y + (threadIdx.x < item.z ? threadIdx.x : item.z - 1U),
+                        static_cast<uint32_t>(reinterpret_cast<uintptr_t>((pf_lds*)order_mem[u & 1U])) + 256U * wave_s);
+    };
+    for (uint32_t base = blockIdx.x; base < units; base += (LIST ? 64U : 1U) * gridDim.x) {
+    uint32_t listed = 1;
+    if constexpr (LIST) {
+        if (threadIdx.x < 64U) {
+            const uint4 item = item_of(base + lane * gridDim.x);
+            const uint64_t lives = __ballot(item.z != 0U);
+            if (item.z) unit_mem[__popcll(lives & ((1ULL << lane) - 1ULL))] = item;
+            if (lane == 0U) unit_count = __popcll(lives);
+        }
+        pf_barrier();
+        listed = __builtin_amdgcn_readfirstlane(unit_count);
+        if (listed) copy_assignments(0);
+        rg_wait<0>();
+        pf_barrier();                                   // (and unit_count is free again)
+    }
+    for (uint32_t u = 0; u < listed; ++u) {
+    const uint4 item = LIST ? unit_mem[u] : item_of(base);
+    const uint32_t e = __builtin_amdgcn_readfirstlane(item.x), begin = __builtin_amdgcn_readfirstlane(item.y);
+    const uint32_t count = __builtin_amdgcn_readfirstlane(item.z), tile = __builtin_amdgcn_readfirstlane(item.w);
+    if (!LIST && count == 0U) continue;
+    const uint32_t* const assignment = LIST ? order_mem[u & 1U] : order + begin;
+    if (LIST && u + 1U < listed) copy_assignments(u + 1U);              // (older than every counted copy; awaited at the unit's end)
 
     // ---- the lane's weight row
     uint32_t feature;                                  // MODE 0: gate (n31 < 16) / up feature; MODE 1: output column
@@ -181,7 +224,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     for (uint32_t i = 0; i < PARTS; ++i) {
         const uint32_t row = PART_ROWS * i + 8U * wave + (lane >> 3), tok = row < count ? row : count - 1U;
         const uint32_t piece = (lane & 7U) ^ ((row >> 1) & 7U);
-        if (MODE == 0) tsrc[0][i] = a.x + static_cast<size_t>(order[begin + tok] / a.top_k) * a.x_stride + 16U * piece;
+        if (MODE == 0) tsrc[0][i] = a.x + static_cast<size_t>(assignment[tok] / a.top_k) * a.x_stride + 16U * piece;
         else {
             // (h rows past the item's are other items' rows or the padding rows of the workspace: read, multiplied and never stored)
             const size_t from = static_cast<size_t>(begin + row) * a.k;
@@ -193,7 +236,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     const uint8_t* ssrc;
     {
         const uint32_t row = (threadIdx.x >> 2) & (TOKENS - 1U), part = threadIdx.x & 3U, tok = row < count ? row : count - 1U;
-        const uint8_t* base = MODE == 0 ? a.x_sums + static_cast<size_t>(order[begin + tok] / a.top_k) * sum_row
+        const uint8_t* base = MODE == 0 ? a.x_sums + static_cast<size_t>(assignment[tok] / a.top_k) * sum_row
                                         : a.h_sums + static_cast<size_t>(begin + tok) * sum_row;
         ssrc = base + 16U * (part & 1U) + (part >> 1) * (sum_row / 2U);
     }
@@ -560,7 +603,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                     a.h[at] = h_hi;
                     a.h_lo[at] = h_lo;
                     if (!(finite_f(g) && finite_f(u) && finite_f(static_cast<float>(h_hi)))) {     // h beyond fp16 counts as non-finite
-                        atomicOr(pf_status_of(a, order[begin + t]), static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION));
+                        atomicOr(pf_status_of(a, assignment[t]), static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION));
                         atomicOr(a.job_status, static_cast<uint32_t>(MI355_STATUS_NONFINITE_PROJECTION));
                     }
                 }
@@ -582,7 +625,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
 #pragma unroll
             for (uint32_t r = 0; r < 16U; ++r) {
                 const uint32_t t = 32U * i + 8U * (r / 4U) + 4U * half + (r & 3U);
-                if (t < count) pf_rawdots_of(a, order[begin + t])[f_out] = a.rawdots_bf16 ? pf_round_bf16(acc[i][r]) : acc[i][r];
+                if (t < count) pf_rawdots_of(a, assignment[t])[f_out] = a.rawdots_bf16 ? pf_round_bf16(acc[i][r]) : acc[i][r];
             }
     }
     if constexpr (FMT == kRgQ80) {
@@ -603,7 +646,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         static_assert(TILES == 1U, "live tiles of the four-wave form");
         run_unit(std::integral_constant<uint32_t, 1>{});
     }
-    }   // units
+    }   // listed units
+    }
 }
 
 }  // namespace strix950

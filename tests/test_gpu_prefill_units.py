@@ -1,0 +1,56 @@
+"""Workgroups of the wide fp16 prefill form over several units: lists with gaps, lists that are filled again, the last unit of each."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def strix():
+    from __graft_entry__ import load_package
+    pkg = load_package()
+    pkg.require_gpu()
+    return pkg
+
+
+def tensors(strix, gen, kind, experts, hidden, ffn):
+    draw = lambda rows, width: strix.quantize_weight_rows(kind, torch.randn((rows, width), device="cuda", generator=gen) * 0.05)
+    return draw(experts * ffn, hidden), draw(experts * ffn, hidden), draw(experts * hidden, ffn)
+
+
+# experts of no, of 57 (the fewest rows that one expert alone gives the wide form), of a whole item and of an item and one more row
+@pytest.mark.parametrize("kind", ["q4_k", "q8_0"])
+@pytest.mark.parametrize("hidden,ffn,counts", [(512, 2304, [0, 57, 128, 129, 0, 300, 64, 200, 0, 385, 90, 257, 511]), (2048, 1280, [0, 0, 700, 58])])
+def test_units_of_uneven_experts(strix, kind, hidden, ffn, counts):
+    """Every row's output is what its expert alone gives it: the sums of a row do not depend on the batch, so the bits are the same."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    kind = {"q4_k": strix.TYPE_Q4_K, "q8_0": strix.TYPE_Q8_0}[kind]
+    experts, rows = len(counts), sum(counts)
+    gate, up, down = tensors(strix, gen, kind, experts, hidden, ffn)
+    ids = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(rows, generator=torch.Generator().manual_seed(6))].to("cuda", torch.int32).reshape(rows, 1)
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).half()
+    weights = torch.rand((rows, 1), device="cuda", generator=gen)
+    layer = strix.MoeLayer(hidden, ffn, experts, 1, gate, up, down, rows, prefill_f16=True, gate_type=kind, down_type=kind)
+    out = layer.run_prefill_f16(x, ids, weights).clone()
+    for e, n in enumerate(counts):
+        if n == 0:
+            continue
+        at = (ids.reshape(-1) == e).nonzero().squeeze(1)
+        one = strix.MoeLayer(hidden, ffn, 1, 1, gate[e * ffn:(e + 1) * ffn], up[e * ffn:(e + 1) * ffn], down[e * hidden:(e + 1) * hidden], n,
+                             prefill_f16=True, gate_type=kind, down_type=kind)
+        alone = one.run_prefill_f16(x[at].contiguous(), torch.zeros((n, 1), dtype=torch.int32, device="cuda"), weights[at].contiguous())
+        assert torch.equal(out[at], alone), (e, n)
+    assert int(layer.status.max()) == 0
+
+
+def test_lists_are_filled_again(strix):
+    """More than 64 units a workgroup on 256 compute units (136 item slots of 132 tiles): bit for bit the rows in pieces."""
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    hidden, ffn, rows, piece = 256, 16896, 16500, 5500
+    gate, up, down = tensors(strix, gen, strix.TYPE_Q4_K, 1, hidden, ffn)
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).half()
+    ids, one = torch.zeros((rows, 1), dtype=torch.int32, device="cuda"), torch.ones((rows, 1), device="cuda")
+    whole = strix.MoeLayer(hidden, ffn, 1, 1, gate, up, down, rows, prefill_f16=True).run_prefill_f16(x, ids, one)
+    parts = strix.MoeLayer(hidden, ffn, 1, 1, gate, up, down, piece, prefill_f16=True)
+    for at in range(0, rows, piece):
+        assert torch.equal(whole[at:at + piece], parts.run_prefill_f16(x[at:at + piece], ids[:piece], one[:piece])), at
