@@ -31,7 +31,8 @@ inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, u
     q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
-// rows x 27648, 8 rows: 59 -> 33 us; ring depths 2..4 within 2 us of each other in both forms).
+// rows x 27648, 8 rows: 59 -> 33 us). Three slots a team where they hold up to eight rows: dense 27648 x 5120, 4 | 8 rows, two, three, four slots 74.4, 72.1,
+// 73.6 | 86.1, 83.4, 83.9 us; sixteen rows are the same with two (102.3).
 template <int FMT, int NAL>
 inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     constexpr bool WIDE = mma_wide<FMT, NAL>();
@@ -41,8 +42,9 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
     if constexpr (FMT == kMmaQ4K && !WIDE) {
         const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, 1U);
         if (static_cast<uint64_t>(g.grid.x) * g.grid.y <= compute_units()) {
-            if (direct) q4k_mma_down_kernel<FMT, NAL, 2, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
-            else q4k_mma_down_kernel<FMT, NAL, 2, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            constexpr int DEEP = NAL <= 4 ? 3 : 2;
+            if (direct) q4k_mma_down_kernel<FMT, NAL, DEEP, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            else q4k_mma_down_kernel<FMT, NAL, DEEP, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
             return;
         }
     }
