@@ -54,3 +54,15 @@ def test_lists_are_filled_again(strix):
     parts = strix.MoeLayer(hidden, ffn, 1, 1, gate, up, down, piece, prefill_f16=True)
     for at in range(0, rows, piece):
         assert torch.equal(whole[at:at + piece], parts.run_prefill_f16(x[at:at + piece], ids[:piece], one[:piece])), at
+
+
+def test_many_experts_in_another_order(strix):
+    """600 experts of few rows each, several items' tiles a workgroup: a batch and the same rows in another order."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    hidden, ffn, rows, experts, top_k = 256, 256, 1400, 600, 8
+    layer = strix.MoeLayer(hidden, ffn, experts, top_k, *tensors(strix, gen, strix.TYPE_Q4_K, experts, hidden, ffn), rows, prefill_f16=True)
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).half()
+    ids = (torch.rand((rows, experts), device="cuda", generator=gen) + torch.linspace(0, 1, experts, device="cuda")).topk(top_k).indices.int()
+    weights = torch.rand((rows, top_k), device="cuda", generator=gen)
+    out = layer.run_prefill_f16(x, ids, weights).clone()
+    assert torch.equal(layer.run_prefill_f16(x.flip(0), ids.flip(0), weights.flip(0)).flip(0), out)
