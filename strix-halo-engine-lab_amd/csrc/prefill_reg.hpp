@@ -261,6 +261,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         const uint8_t* at = wrow + static_cast<size_t>(sc >> 2) * BLOCK + QUANTS_AT + 32U * (sc & 3U) + 16U * half;
         asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qs) : "v"(at) : "memory");
     };
+    const auto fetch_whole = [&](uint32_t b, u32x4 (&q)[4]) {           // the quants of a super-block
+        const uint8_t* at = wrow + static_cast<size_t>(block_of(b)) * BLOCK + 16U * half;
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[0]) : "v"(at), "n"(QUANTS_AT) : "memory");
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[1]) : "v"(at), "n"(QUANTS_AT + 32U) : "memory");
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[2]) : "v"(at), "n"(QUANTS_AT + 64U) : "memory");
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[3]) : "v"(at), "n"(QUANTS_AT + 96U) : "memory");
+    };
 
     // Q8_0: a stage is two blocks (fp16 d, 32 codes; 34 bytes), 68 bytes from a 4-byte boundary. The lane's 16 codes of the first lie two
     // bytes past a word (four words and the next), those of the second on one. Its words hold d of the first block (half 0: in front of the
@@ -365,8 +372,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         asm volatile("s_waitcnt vmcnt(%3)" : "+v"(q8[0].a), "+v"(q8[0].b), "+v"(q8[0].e) : "n"(RING8 == 4U ? 2U * NT + 9U : NT + 3U) : "memory");
     } else if constexpr (WHOLE) {
         fetch_header(0, hd_cur, f_cur);
-#pragma unroll
-        for (uint32_t j = 0; j < 4U; ++j) fetch_quants(j, qs[j]);
+        fetch_whole(0, qs);
         copy_tokens(0, tok_stage[0]); copy_sums(0);
         copy_tokens(1, tok_stage[1]);
         copy_tokens(2, tok_stage[2]);
@@ -459,10 +465,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                                 if (!WHOLE) fetch_quants(s + 4U, qs[p]);
                                 if (p == 0) fetch_header(b + 1U, hd_next, f_next);
                             }
-                            if (WHOLE && p == 0) {
-#pragma unroll
-                                for (uint32_t q4 = 0; q4 < 4U; ++q4) fetch_quants(s + 4U + q4, qn[q4]);
-                            }
+                            if (WHOLE && p == 0) fetch_whole(b + 1U, qn);
                         } else {
                             // first k-step of the next stage: its quants (the next super-block's header with them) were fetched in stage s - 3
                             // (WHOLE: all of the next super-block's in stage 0); younger the three stages since
