@@ -129,6 +129,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     constexpr uint32_t TOKENS = WAVES == 4U ? 32U : 128U;
     static_assert(TOKENS <= 16U * WAVES && TOKENS % (8U * WAVES) == 0, "one sums copy per wave, a token copy of 8 rows per wave and part");
     constexpr bool WHOLE = WAVES == 4U && FMT != kRgQ80;
+    // SCALED: the operand of a Q4_K weight is 2^-14 sc q, as the packed product of a subnormal (the nibble where it lies in its byte: 2^-24 q or 2^-20 q)
+    // and 2^10 sc or 2^6 sc: exact, no shift for the high nibbles, and no 1024 to take out of the sum again.
+    constexpr bool SCALED = FMT == kRgQ4K;
     // Q8_0: stages of weights in registers. The wide form has room for two beside its sums (32 registers of the gate / up rows are spilled at a
     // unit's start and read at its end; with four stages 110, inside the K loop: 1000 rows of hidden 2048 / ffn 768 / 128 experts 342 -> 435 us).
     constexpr uint32_t RING8 = WAVES == 4U ? 4U : 2U;
@@ -298,6 +301,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     };
     // two weights: bytes 0, 1 or (odd) 2, 3 of a word
     const auto expand_pair = [&](uint32_t w, uint32_t odd, const RgFactor& f) -> uint32_t {
+        if (SCALED) return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U)) * f.mul);
         if (FMT == kRgQ4K) return __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U) * f.sc + magic;
         const half2v t = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(magic, w, odd ? 0x05030502U : 0x05010500U));
         if (FMT == kRgQ5K) return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, f.mul, f.add));
@@ -309,6 +313,25 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     // a word of four nibbles (Q5_K: with their fifth bits, bit `bit` of each byte of f)
     const auto low = [&](uint32_t w, uint32_t f, uint32_t bit) -> uint32_t {
         return (w & 0x0f0f0f0fU) | (FMT == kRgQ5K ? ((f >> bit) & 0x01010101U) << 4 : 0U);
+    };
+    const auto high = [&](uint32_t w, uint32_t f, uint32_t bit) -> uint32_t { return SCALED ? w & 0xf0f0f0f0U : low(w >> 4, f, bit); };
+    // four bytes of the packed six-bit factors as fp16 integers, bytes 0 and 1 or (odd) 2 and 3 in a register
+    const auto six_bits = [&](uint32_t m, uint32_t odd) -> half2v {
+        const half2v offset = {static_cast<_Float16>(-1024.0F), static_cast<_Float16>(-1024.0F)};
+        return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(magic, m, odd ? 0x05030502U : 0x05010500U)) + offset;
+    };
+    // SCALED: 2^10 sc of sub-block 2 p and 2^6 sc of 2 p + 1
+    half2v scaled[4];
+    const auto set_scaled = [&](const u32x4& hd) {
+        const uint32_t first = hd.y & 0x3f3f3f3fU, last = (hd.w & 0x0f0f0f0fU) | ((hd.y >> 2) & 0x30303030U);
+        const half2v units = {static_cast<_Float16>(1024.0F), static_cast<_Float16>(64.0F)};
+#pragma unroll
+        for (uint32_t q = 0; q < 4U; ++q) scaled[q] = six_bits(q < 2U ? first : last, q & 1U) * units;
+    };
+    const auto scaled_factor = [&](uint32_t p, uint32_t odd) -> RgFactor {
+        RgFactor f{};
+        f.mul = odd ? half2v{scaled[p].y, scaled[p].y} : half2v{scaled[p].x, scaled[p].x};
+        return f;
     };
     // Q8_0: words 2 k, 2 k + 1 of the lane's codes of the stage's first block, as unsigned bytes code + 128
     const auto first_codes = [&](const Rg8& r, uint32_t k, uint32_t& w0, uint32_t& w1) {
@@ -358,7 +381,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         for (uint32_t r = 0; r < RING8; ++r) q8[r] = Rg8{{0U, 0U, 0U, 0U}, {0U, 0U, 0U, 0U}, 0U};
     }
     float d_last = 0.0F;                                               // Q8_0: d of the last block of the stage before
-    u32x4 mreg_hi = {0U, 0U, 0U, 0U}, mreg_lo = {0U, 0U, 0U, 0U};      // B operand of the S x M product: Q4_K -(1024 d + dmin m_j), Q5_K -(dmin m_j), j = 8 half .. + 8
     if constexpr (FMT == kRgQ80) {
         fetch_blocks(0, q8[0]);
         copy_tokens(0, tok_stage[0]);
@@ -396,7 +418,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     } else {
         uint32_t s_lo, s_hi;
         scales(hd_cur, 0, s_lo, s_hi);
-        bfrag = expand(low(qs[0].x, f_cur.x, 0U), low(qs[0].y, f_cur.y, 0U), factor_of(s_lo));
+        if (SCALED) set_scaled(hd_cur);
+        bfrag = expand(low(qs[0].x, f_cur.x, 0U), low(qs[0].y, f_cur.y, 0U), SCALED ? scaled_factor(0U, 0U) : factor_of(s_lo));
     }
     // A stage's MFMAs as a flat sequence of slots m = (k-step j, plane, token tile i); the A operand of slot m + W is requested right after
     // the MFMA of slot m into the registers that MFMA has just read (a window of W operands, which runs on over the stages' borders).
@@ -415,10 +438,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                 const uint32_t s = 4U * b + p, bb = SWEEPS == 2U && b >= blocks ? b - blocks : b;            // (bb: of the rows)
                 uint32_t s_lo = 0, s_hi = 0;
                 if (FMT != kRgQ80) scales(hd_cur, p, s_lo, s_hi);
-                const RgFactor f_lo = factor_of(s_lo), f_hi = factor_of(s_hi);
+                const RgFactor f_lo = SCALED ? scaled_factor(p, 0U) : factor_of(s_lo), f_hi = SCALED ? scaled_factor(p, 1U) : factor_of(s_hi);
                 const u32x4 qw = qs[p];
                 const Rg8 r8 = q8[p % RING8];
-                const float d_now = half_bits_to_float(hd_cur.x & 0xffffU);
+                const float d_now = half_bits_to_float(hd_cur.x & 0xffffU) * (SCALED ? 16384.0F : 1.0F);
                 float d_first = 0.0F, d_second = 0.0F;                                   // Q8_0: of the stage's two blocks
                 if (FMT == kRgQ80) {
                     const uint32_t mine = half ? r8.e >> 16 : r8.a.x & 0xffffU;
@@ -445,10 +468,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                             else { nw0 = low(qw.z, f_cur.z, 2U * p); nw1 = low(qw.w, f_cur.w, 2U * p); nf = f_lo; }
                         } else if (j == 1) {
                             if (FMT == kRgQ80) { nw0 = r8.b.x ^ 0x80808080U; nw1 = r8.b.y ^ 0x80808080U; }
-                            else { nw0 = low(qw.x >> 4, f_cur.x, 2U * p + 1U); nw1 = low(qw.y >> 4, f_cur.y, 2U * p + 1U); nf = f_hi; }
+                            else { nw0 = high(qw.x, f_cur.x, 2U * p + 1U); nw1 = high(qw.y, f_cur.y, 2U * p + 1U); nf = f_hi; }
                         } else if (j == 2) {
                             if (FMT == kRgQ80) { nw0 = r8.b.z ^ 0x80808080U; nw1 = r8.b.w ^ 0x80808080U; }
-                            else { nw0 = low(qw.z >> 4, f_cur.z, 2U * p + 1U); nw1 = low(qw.w >> 4, f_cur.w, 2U * p + 1U); nf = f_hi; }
+                            else { nw0 = high(qw.z, f_cur.z, 2U * p + 1U); nw1 = high(qw.w, f_cur.w, 2U * p + 1U); nf = f_hi; }
                             // The stage's middle: its token copies' turn. The tokens of stage s + 1 were copied two stages ago (younger: the rest
                             // of that stage's operations and the next one's); behind the barrier every wave's have landed, and every wave
                             // has read the last of stage s - 1, whose slot takes stage s + 3. (At a stage's border the barrier made both waves
@@ -486,8 +509,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                                 else asm volatile("s_waitcnt vmcnt(%1)" : "+v"(qs[pn]) : "n"(younger) : "memory");
                                 uint32_t n_lo, n_hi;
                                 scales(p == 3U ? hd_next : hd_cur, pn, n_lo, n_hi);
+                                if (SCALED && p == 3U) set_scaled(hd_next);
                                 const u32x4 fb = p == 3U ? f_next : f_cur;
-                                nw0 = low(qs[pn].x, fb.x, 2U * pn); nw1 = low(qs[pn].y, fb.y, 2U * pn); nf = factor_of(n_lo);
+                                nw0 = low(qs[pn].x, fb.x, 2U * pn); nw1 = low(qs[pn].y, fb.y, 2U * pn); nf = SCALED ? scaled_factor(pn, 0U) : factor_of(n_lo);
                             }
                         }
                     }
@@ -513,67 +537,24 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                 }
                 bfrag = __builtin_bit_cast(half8, bnext);
                 d_last = d_second;
-                if (FMT != kRgQ80 && !WHOLE && p == 1U) {
-                    // this lane's M operand: the eight sub-blocks of super-block 2 g + half of the group
-                    if ((bb & 1U) == half) {
-                        const float d = half_bits_to_float(hd_cur.x & 0xffffU), dm = half_bits_to_float(hd_cur.x >> 16);
-                        const float d1024 = FMT == kRgQ5K ? 0.0F : 1024.0F * d;          // (Q5_K operands carry no offset)
-                        uint32_t mh[4], ml[4];
-#pragma unroll
-                        for (int jj = 0; jj < 8; jj += 2) {
-                            float v[2];
-#pragma unroll
-                            for (int t = 0; t < 2; ++t) {
-                                const uint32_t sh = 8U * ((jj + t) & 3U);
-                                const uint32_t mn = (jj + t) < 4 ? ((hd_cur.z >> sh) & 63U) : (((hd_cur.w >> (sh + 4U)) & 15U) | (((hd_cur.z >> (sh + 6U)) & 3U) << 4));
-                                v[t] = -(d1024 + dm * static_cast<float>(mn));
-                            }
-                            const half2v hh = __builtin_convertvector(float2v{v[0], v[1]}, half2v);
-                            mh[jj / 2] = __builtin_bit_cast(uint32_t, hh);
-                            ml[jj / 2] = pack_half2(v[0] - static_cast<float>(hh.x), v[1] - static_cast<float>(hh.y));
-                        }
-                        mreg_hi = u32x4{mh[0], mh[1], mh[2], mh[3]};
-                        mreg_lo = u32x4{ml[0], ml[1], ml[2], ml[3]};
-                    } else if ((bb & 1U) == 0 && bb + 1U == blocks) {  // odd count: the last group's second super-block does not exist
-                        mreg_hi = u32x4{0U, 0U, 0U, 0U};
-                        mreg_lo = u32x4{0U, 0U, 0U, 0U};
-                    }
-                }
                 if (FMT != kRgQ80 && p == 3U) {
-                    // The minimums of the four-wave form, super-block by super-block: S hi and S lo (K = 8 + 8) against the exact fp16 integers m_j, scaled by
-                    // -dmin in fp32, and against -1024 into the product itself. Two products where the wide form has one and a half, and 16 more vector
-                    // operations a tile, but none of the 75 a super-block that split M into hi + lo, which one tile does not pay for: 64 | 333 rows of
-                    // hidden 2048 / ffn 768 / 128 experts 96.4 | 163.3 -> 94.1 | 158.1 us, Q5_K 192.0 -> 186.2; the error against 64 bits falls by
-                    // a tenth (Q5_K: a fifth).
-                    if (WHOLE && (SWEEPS == 1U || b >= blocks)) {          // (the sums are of hi + lo: once)
-                        const half8 sums = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(s_tile + ((bb >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 32U * half + 16U * (bb & 1U));
-                        const uint32_t m_lo = hd_cur.z & 0x3f3f3f3fU, m_hi = ((hd_cur.w >> 4) & 0x0f0f0f0fU) | ((hd_cur.z >> 2) & 0x30303030U);
-                        const half2v offset = {static_cast<_Float16>(-1024.0F), static_cast<_Float16>(-1024.0F)};
+                    fold(LIVE - 1U, d_now);
+                    // the super-block's minimums: S hi and S lo (K = 8 + 8; the sums are of hi + lo, once) against the integers m_j, times -dmin
+                    if (SWEEPS == 1U || b >= blocks) {
+                        const pf_lds* st = s_tile + ((bb >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 32U * half + 16U * (bb & 1U);
+                        const uint32_t first = hd_cur.z & 0x3f3f3f3fU, last = ((hd_cur.w >> 4) & 0x0f0f0f0fU) | ((hd_cur.z >> 2) & 0x30303030U);
                         u32x4 mins;
 #pragma unroll
-                        for (uint32_t q = 0; q < 4U; ++q)
-                            mins[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, __builtin_amdgcn_perm(magic, q < 2U ? m_lo : m_hi, q & 1U ? 0x05030502U : 0x05010500U)) + offset);
-                        const uint32_t two = __builtin_bit_cast(uint32_t, offset);
+                        for (uint32_t q = 0; q < 4U; ++q) mins[q] = __builtin_bit_cast(uint32_t, six_bits(q < 2U ? first : last, q & 1U));
                         const floatx16 zero = {0.0F};
-                        if (FMT == kRgQ4K) part[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, __builtin_bit_cast(half8, u32x4{two, two, two, two}), part[0], 0, 0, 0);
-                        const floatx16 least = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, __builtin_bit_cast(half8, mins), zero, 0, 0, 0);
+#pragma unroll
+                        for (uint32_t i = 0; i < LIVE; ++i)
+                            part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const __attribute__((address_space(3))) half8*>(st + i * 32U * 64U), __builtin_bit_cast(half8, mins), zero, 0, 0, 0);
                         const float minus_dmin = -half_bits_to_float(hd_cur.x >> 16);
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[0][r] = __builtin_fmaf(minus_dmin, least[r], acc[0][r]);
-                    }
-                    fold(LIVE - 1U, d_now);
-                    if (!WHOLE && (SWEEPS == 1U || b >= blocks) && ((bb & 1U) || bb + 1U == blocks)) {          // (the sums are of hi + lo: once)
-                        // end of a group of 16 sub-blocks: running sum += S hi * M hi + S lo * M hi + S hi * M lo
-                        const pf_lds* st = s_tile + ((bb >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 16U * half;
-                        const half8 mh = __builtin_bit_cast(half8, mreg_hi), ml = __builtin_bit_cast(half8, mreg_lo);
+                        for (uint32_t i = 0; i < LIVE; ++i)
 #pragma unroll
-                        for (uint32_t i = 0; i < LIVE; ++i) {
-                            const half8 sh = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(st + i * 32U * 64U);
-                            const half8 sl = *reinterpret_cast<const __attribute__((address_space(3))) half8*>(st + i * 32U * 64U + 32U);
-                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, mh, acc[i], 0, 0, 0);
-                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sl, mh, acc[i], 0, 0, 0);
-                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sh, ml, acc[i], 0, 0, 0);
-                        }
+                            for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(minus_dmin, part[i][r], acc[i][r]);
                     }
                     hd_cur = hd_next;
                     f_cur = f_next;
