@@ -5,15 +5,17 @@
 // integer-dot class's bits: no weight is rounded.
 //
 // Arithmetic, Q4_K. w = d_b (sc_j q) - dmin_b m_j (src/ggml_dequant.cpp:119-130). The MFMA operand of a weight is the fp16 number
-// 1024 + sc_j q, made by ONE integer multiply-add per two weights: (q1 << 16 | q0) * sc + 0x64006400 (sc q <= 945 < 1024
-// stays inside the mantissa of 0x6400 = 1024.0). With S_bj[t] = sum of x_k[t] over sub-block j of super-block b,
-//   out[t][f] = sum_b d_b[f] P_b[t][f] + sum_(b,j) S_bj[t] M_bj[f],
-//   P_b = sum_(k in b) (1024 + sc_j q_k) x_k[t]  (fp16 MFMA, fp32 accumulation),   M_bj[f] = -(1024 d_b + dmin_b m_j).
-// d_b is applied in fp32 once per super-block; the second sum is a K / 32-long product with S and M each carried as fp16
-// hi + lo (three MFMAs per 16 sub-blocks). In the down product the activation h is carried as fp16 hi + lo as well,
-// so that the only roundings of the whole expert are fp32 accumulations.
+// 2^-14 sc_j q, made by ONE packed multiplication per two weights (SCALED below; sc q <= 945: exact). With S_bj[t] = sum of x_k[t]
+// over sub-block j of super-block b,
+//   out[t][f] = sum_b (2^14 d_b[f] P_b[t][f] - dmin_b[f] L_b[t][f]),
+//   P_b = sum_(k in b) 2^-14 sc_j q_k x_k[t],   L_b = sum_(j in b) m_j S_bj[t]   (fp16 MFMAs, fp32 accumulation),
+// S as fp16 hi + lo in one product (K = 8 + 8) against the exact integers m_j. In the down product the activation h is carried as
+// fp16 hi + lo as well, so that the only roundings of the whole expert are fp32 accumulations. Before, the operand was 1024 + sc q and
+// 1024 d + dmin m a second operand split into hi + lo: 64 | 333 rows of hidden 2048 / ffn 768 / 128 experts 96.4 | 163.3 us, now 90.8 | 151.0 (with
+// a super-block's quants from one address), 300 rows of hidden 5120 / ffn 1536 / 160 experts 874 -> 811, Q5_K, 333 rows 192 -> 178;
+// with four token tiles 1000 rows 266 -> 260. Error against 64 bits 1.9e-6 -> 5.5e-7, Q5_K 7.4e-8 -> 6.2e-8.
 // Q5_K: the same blocks with 32 fifth-bit bytes after the factors (bit j of byte k for element k of sub-block j). sc q <= 1953 is an exact
-// fp16 integer but past the offset's mantissa: fma(1024 + q, sc, -1024 sc), packed; M_bj = -(dmin_b m_j).
+// fp16 integer: fma(1024 + q, sc, -1024 sc), packed; no 2^14.
 // Q8_0: one d per 32 codes and no minimum (src/ggml_dequant.cpp:84-87): the codes are exact fp16 integers, (1152 + code) - 1152, P is of a block.
 //
 // Work decomposition. A plan item holds at most 128 rows of one expert. A 512-thread workgroup owns (item, 256 weight rows):
@@ -259,17 +261,16 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
             asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(fifth) : "v"(bits) : "memory");
         }
     };
-    const auto fetch_quants = [&](uint32_t s, u32x4& qs) {
-        const uint32_t sc = stage_of(s);
-        const uint8_t* at = wrow + static_cast<size_t>(sc >> 2) * BLOCK + QUANTS_AT + 32U * (sc & 3U) + 16U * half;
-        asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qs) : "v"(at) : "memory");
-    };
-    const auto fetch_whole = [&](uint32_t b, u32x4 (&q)[4]) {           // the quants of a super-block
+    // the quants of stage 4 b + p (an offset from the super-block's one address, which costs less than an address a stage)
+    const auto fetch_quants = [&](uint32_t b, auto p, u32x4& qs) {
         const uint8_t* at = wrow + static_cast<size_t>(block_of(b)) * BLOCK + 16U * half;
-        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[0]) : "v"(at), "n"(QUANTS_AT) : "memory");
-        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[1]) : "v"(at), "n"(QUANTS_AT + 32U) : "memory");
-        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[2]) : "v"(at), "n"(QUANTS_AT + 64U) : "memory");
-        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(q[3]) : "v"(at), "n"(QUANTS_AT + 96U) : "memory");
+        asm volatile("global_load_dwordx4 %0, %1, off offset:%2" : "=v"(qs) : "v"(at), "n"(QUANTS_AT + 32U * decltype(p)::value) : "memory");
+    };
+    const auto fetch_whole = [&](uint32_t b, u32x4 (&q)[4]) {           // of a super-block
+        fetch_quants(b, std::integral_constant<uint32_t, 0>{}, q[0]);
+        fetch_quants(b, std::integral_constant<uint32_t, 1>{}, q[1]);
+        fetch_quants(b, std::integral_constant<uint32_t, 2>{}, q[2]);
+        fetch_quants(b, std::integral_constant<uint32_t, 3>{}, q[3]);
     };
 
     // Q8_0: a stage is two blocks (fp16 d, 32 codes; 34 bytes), 68 bytes from a 4-byte boundary. The lane's 16 codes of the first lie two
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     };
 
     // ---- expansion: 8 nibbles (low or high) of two quant words -> the B operand of one k-step: four registers of two fp16
-    // numbers 1024 + sc q each
+    // numbers each
     uint32_t magic;
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
     // Q5_K: sc q is up to 1953, past the offset's mantissa: fma(1024 + q, sc, -1024 sc) = sc q, exact. Q8_0: 1152 + code, minus 1152.
@@ -302,7 +303,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     // two weights: bytes 0, 1 or (odd) 2, 3 of a word
     const auto expand_pair = [&](uint32_t w, uint32_t odd, const RgFactor& f) -> uint32_t {
         if (SCALED) return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U)) * f.mul);
-        if (FMT == kRgQ4K) return __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U) * f.sc + magic;
         const half2v t = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(magic, w, odd ? 0x05030502U : 0x05010500U));
         if (FMT == kRgQ5K) return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(t, f.mul, f.add));
         return __builtin_bit_cast(uint32_t, t + half2v{minus, minus});
@@ -401,10 +401,10 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         // younger than the token copies and sums of stage 0: two stages of NT
         rg_wait_for<2U * NT, FMT == kRgQ5K>(f_cur, hd_cur, qs[0], qs[1], qs[2], qs[3]);
     } else {
-        fetch_header(0, hd_cur, f_cur); fetch_quants(0, qs[0]);
-        copy_tokens(0, tok_stage[0]); copy_sums(0); fetch_quants(1, qs[1]);
-        copy_tokens(1, tok_stage[1]); fetch_quants(2, qs[2]);
-        copy_tokens(2, tok_stage[2]); fetch_quants(3, qs[3]);
+        fetch_header(0, hd_cur, f_cur); fetch_quants(0, std::integral_constant<uint32_t, 0>{}, qs[0]);
+        copy_tokens(0, tok_stage[0]); copy_sums(0); fetch_quants(0, std::integral_constant<uint32_t, 1>{}, qs[1]);
+        copy_tokens(1, tok_stage[1]); fetch_quants(0, std::integral_constant<uint32_t, 2>{}, qs[2]);
+        copy_tokens(2, tok_stage[2]); fetch_quants(0, std::integral_constant<uint32_t, 3>{}, qs[3]);
         // younger than the token copies of stage 0: sums + quants, then two stages of NT + 1
         rg_wait_for<2U * NT + 4U, FMT == kRgQ5K>(f_cur, hd_cur, qs[0]);
     }
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                             }      // the stage's quant registers are free now
                             else {
                                 if (p == 1) copy_sums(SWEEPS == 2U && b + 1U == blocks ? 0U : (bb >> 1) + 1U);
-                                if (!WHOLE) fetch_quants(s + 4U, qs[p]);
+                                if (!WHOLE) fetch_quants(b + 1U, p_constant, qs[p]);
                                 if (p == 0) fetch_header(b + 1U, hd_next, f_next);
                             }
                             if (WHOLE && p == 0) fetch_whole(b + 1U, qn);
@@ -538,23 +538,38 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                 bfrag = __builtin_bit_cast(half8, bnext);
                 d_last = d_second;
                 if (FMT != kRgQ80 && p == 3U) {
-                    fold(LIVE - 1U, d_now);
                     // the super-block's minimums: S hi and S lo (K = 8 + 8; the sums are of hi + lo, once) against the integers m_j, times -dmin
-                    if (SWEEPS == 1U || b >= blocks) {
-                        const pf_lds* st = s_tile + ((bb >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 32U * half + 16U * (bb & 1U);
+                    const bool least = SWEEPS == 1U || b >= blocks;
+                    const pf_lds* st = s_tile + ((bb >> 1) & 1U) * (TOKENS * 64U) + n31 * 64U + 32U * half + 16U * (bb & 1U);
+                    const float minus_dmin = -half_bits_to_float(hd_cur.x >> 16);
+                    u32x4 mins = {0U, 0U, 0U, 0U};
+                    if (least) {
                         const uint32_t first = hd_cur.z & 0x3f3f3f3fU, last = ((hd_cur.w >> 4) & 0x0f0f0f0fU) | ((hd_cur.z >> 2) & 0x30303030U);
-                        u32x4 mins;
 #pragma unroll
                         for (uint32_t q = 0; q < 4U; ++q) mins[q] = __builtin_bit_cast(uint32_t, six_bits(q < 2U ? first : last, q & 1U));
+                    }
+                    const auto minimums = [&](uint32_t i) __attribute__((always_inline)) {
                         const floatx16 zero = {0.0F};
+                        return __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const __attribute__((address_space(3))) half8*>(st + i * 32U * 64U), __builtin_bit_cast(half8, mins), zero, 0, 0, 0);
+                    };
+                    const auto take = [&](uint32_t i, const floatx16& product) __attribute__((always_inline)) {
 #pragma unroll
-                        for (uint32_t i = 0; i < LIVE; ++i)
-                            part[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const __attribute__((address_space(3))) half8*>(st + i * 32U * 64U), __builtin_bit_cast(half8, mins), zero, 0, 0, 0);
-                        const float minus_dmin = -half_bits_to_float(hd_cur.x >> 16);
+                        for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(minus_dmin, product[r], acc[i][r]);
+                    };
+                    if constexpr (LIVE == 1U) {                      // (registers for both products)
+                        if (least) {
+                            const floatx16 product = minimums(0);
+                            fold(0, d_now);
+                            take(0, product);
+                        } else fold(0, d_now);
+                    } else {
+                        fold(LIVE - 1U, d_now);
+                        if (least) {
 #pragma unroll
-                        for (uint32_t i = 0; i < LIVE; ++i)
+                            for (uint32_t i = 0; i < LIVE; ++i) part[i] = minimums(i);
 #pragma unroll
-                            for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(minus_dmin, part[i][r], acc[i][r]);
+                            for (uint32_t i = 0; i < LIVE; ++i) take(i, part[i]);
+                        }
                     }
                     hd_cur = hd_next;
                     f_cur = f_next;
