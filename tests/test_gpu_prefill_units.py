@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from test_gpu_prefill_formats import draw
+
 pytestmark = pytest.mark.gpu
 
 
@@ -14,21 +16,25 @@ def strix():
 
 
 def tensors(strix, gen, kind, experts, hidden, ffn):
-    draw = lambda rows, width: strix.quantize_weight_rows(kind, torch.randn((rows, width), device="cuda", generator=gen) * 0.05)
-    return draw(experts * ffn, hidden), draw(experts * ffn, hidden), draw(experts * hidden, ffn)
+    def rows_of(rows, width):
+        if kind == strix.TYPE_Q5_K:
+            return draw(gen, "q5_k", rows, width)[0]
+        return strix.quantize_weight_rows(kind, torch.randn((rows, width), device="cuda", generator=gen) * 0.05)
+    return rows_of(experts * ffn, hidden), rows_of(experts * ffn, hidden), rows_of(experts * hidden, ffn)
 
 
-# experts of no, of 57 (the fewest rows that one expert alone gives the wide form), of a whole item and of an item and one more row
-@pytest.mark.parametrize("kind", ["q4_k", "q8_0"])
-@pytest.mark.parametrize("hidden,ffn,counts", [(512, 2304, [0, 57, 128, 129, 0, 300, 64, 200, 0, 385, 90, 257, 511]), (2048, 1280, [0, 0, 700, 58])])
+# experts of no, of one to four token tiles, of a whole item and of an item and one more row
+@pytest.mark.parametrize("kind", ["q4_k", "q5_k", "q8_0"])
+@pytest.mark.parametrize("hidden,ffn,counts", [(512, 2304, [0, 57, 128, 129, 0, 300, 64, 200, 0, 385, 90, 257, 511]), (2048, 1280, [0, 0, 2000, 58])])
 def test_units_of_uneven_experts(strix, kind, hidden, ffn, counts):
-    """Every row's output is what its expert alone gives it: the sums of a row do not depend on the batch, so the bits are the same."""
+    """Every row's output is what its expert alone gives it: the sums of a row do not depend on the batch nor on the form (the batch takes the wide
+    one; an expert alone is few units, which the four-wave form takes), so the bits are the same."""
     gen = torch.Generator(device="cuda").manual_seed(5)
-    kind = {"q4_k": strix.TYPE_Q4_K, "q8_0": strix.TYPE_Q8_0}[kind]
+    kind = {"q4_k": strix.TYPE_Q4_K, "q5_k": strix.TYPE_Q5_K, "q8_0": strix.TYPE_Q8_0}[kind]
     experts, rows = len(counts), sum(counts)
     gate, up, down = tensors(strix, gen, kind, experts, hidden, ffn)
     ids = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(rows, generator=torch.Generator().manual_seed(6))].to("cuda", torch.int32).reshape(rows, 1)
-    x = torch.randn((rows, hidden), device="cuda", generator=gen).half()
+    x = (torch.randn((rows, hidden), device="cuda", generator=gen) * (0.05 if kind == strix.TYPE_Q5_K else 1.0)).half()
     weights = torch.rand((rows, 1), device="cuda", generator=gen)
     layer = strix.MoeLayer(hidden, ffn, experts, 1, gate, up, down, rows, prefill_f16=True, gate_type=kind, down_type=kind)
     out = layer.run_prefill_f16(x, ids, weights).clone()
