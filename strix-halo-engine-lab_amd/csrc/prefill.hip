@@ -60,6 +60,9 @@ namespace {
 // 9, 5.4 340, 348; 12, 5.4 578, 656; 7, 6.3 363, 351; 9, 6.4 384, 397; 3.8, 7.7 910, 886; 6, 7.9 1055, 1107; 12.5, 8.2 1238, 1348; 2, 16 479, 420;
 // 4, 17 535, 509; 6, 17 566, 596; 9, 17 579, 694; hidden 1280, 13, 4.1 166, 128; hidden 1024, 13, 6.2 179, 148. Past 13 rows per expert: 21, 3.5 257, 285; 25, 3.6
 // 538, 615; 37, 3.9 325, 369; in one round 25, 0.9 123, 95; 37, 1.0 128, 120; 50, 0.7 134, 119.
+// Measured again for 50 to 80 rows per expert (rows, rounds, wide, four waves): Q4_K 62, 1.1 152, 129; 70, 1.5 142, 127; 70, 0.5 198, 162; 75, 1.6 258, 226; 77, 2.0 301, 260;
+// 78, 1.5 124, 134; 94, 2.6 205, 213; 150, 2.2 309, 355; Q5_K 62, 1.1 170, 159; 70, 1.5 156, 152; 75, 1.6 299, 294; Q8_0 62, 0.7 114, 95; 70, 0.5 268, 245; 75, 0.9 192, 213;
+// 75, 1.0 150, 166.
 // However many rows an expert has, while the four-wave form's units (of 32 rows) find room at once, three workgroups a compute unit, which the wide
 // form's leave mostly idle. Units, then the same two times, one expert: Q4_K hidden 2048 / ffn 768, 56 86.5, 50.9; 154 86.6, 52.4; 448 91.3, 67.0; 4096 /
 // 2048, 240 146, 79.9; Q8_0 56 109, 55.7; 448 116, 84.6; 240 201, 98.4; Q5_K 448 99.9, 74.7; 240 168, 93.4; of 16 and 32 experts Q4_K 728 95.3, 81.3; 728 70.7, 57.3;
@@ -71,9 +74,9 @@ bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
     const uint64_t e = wv.experts, a = assignments, work = (128ULL * e + a) * wv.ffn, round = compute_units() * 128ULL * 128U;
     if (wv.gate_type == MI355_TYPE_Q8_0 || wv.down_type == MI355_TYPE_Q8_0) {
         const bool starts = a * work <= 51ULL * e * round || 2ULL * a <= 9ULL * e || wv.hidden <= 1280U;
-        return (a <= 13ULL * e && starts) || (a <= 56ULL * e && work <= round);
+        return (a <= 13ULL * e && starts) || (a <= 70ULL * e && work <= round);
     }
-    return a <= 16ULL * e || (a <= 56ULL * e && work <= 4ULL * round);
+    return a <= 16ULL * e || (a <= 56ULL * e && work <= 4ULL * round) || (a <= 75ULL * e && work <= 2ULL * round);
 }
 }  // namespace
 
