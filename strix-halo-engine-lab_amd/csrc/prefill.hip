@@ -65,7 +65,7 @@ namespace {
 // 75, 1.0 150, 166.
 // However many rows an expert has, while the four-wave form's units (of 32 rows) find room at once, three workgroups a compute unit, which the wide
 // form's leave mostly idle. Units, then the same two times, one expert: Q4_K hidden 2048 / ffn 768, 56 86.5, 50.9; 154 86.6, 52.4; 448 91.3, 67.0; 4096 /
-// 2048, 240 146, 79.9; Q8_0 56 109, 55.7; 448 116, 84.6; 240 201, 98.4; Q5_K 448 99.9, 74.7; 240 168, 93.4; of 16 and 32 experts Q4_K 728 95.3, 81.3; 728 70.7, 57.3;
+// 2048, 224 146, 79.9; Q8_0 56 109, 55.7; 448 116, 84.6; 224 201, 98.4; Q5_K 448 99.9, 74.7; 224 168, 93.4; of 16 and 32 experts Q4_K 728 95.3, 81.3; 728 70.7, 57.3;
 // Q5_K 728 102, 92.0; Q8_0 728 84.8, 72.4. Past that: Q4_K 928 73.4, 64.9; 1024 156, 155; 1106 112, 109; 1344 106, 110; Q8_0 928 86.2, 85.8; 1024 212, 257; 1106 133,
 // 147; Q5_K 1024 177, 196; 1106 119, 122.
 bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
