@@ -30,11 +30,39 @@ struct RouteArgs {
     // fused decode extras (all null / zero for the plain router)
     int8_t* codes; float* deltas; int32_t* sums; uint32_t* status; uint32_t* job_status; uint32_t* plan;
     uint32_t route_blocks, quant_blocks;
+    // RMSNorm of the rows inside the fused launch (normed not null; hidden <= kChainNormHidden): the router and the A8 image see y = (x * r) * norm_w,
+    // r = 1 / sqrt(mean(x^2) + eps); normed receives y as fp32 [rows][hidden]; norm_w may be null
+    const float* norm_w; float norm_eps; float* normed;
     // early-routes form (route_early.hpp): one word per assignment - the count of finished projection waves in the low half, a
     // non-finite projection in bit 31 -, and a test knob that displaces the early logits so that the repair path runs
     uint32_t* awords; uint32_t early_perturb;
     float* early_logits; uint32_t early_stride;      // where the early logits of row i go: early_logits + i * early_stride (floats)
 };
+
+// ---------------------------------------------------------------------------------------------------- RMSNorm by one wavefront
+// The norm factor of a row of n features (a multiple of 256 up to kChainNormHidden), bit for bit rmsnorm_f32_kernel: lane t holds the chains t, t + 64, ... of
+// L = 256 (n >= 512) or 128, features t + 64 m, all asked for at once; the L sums are halved as there.
+constexpr uint32_t kChainNormHidden = 1536, kNormHeld = kChainNormHidden / 64U;
+template <int KIND>
+__device__ __forceinline__ void norm_ask(float (&v)[kNormHeld], const uint8_t* xrow, uint32_t n) {
+#pragma unroll
+    for (uint32_t m = 0; m < kNormHeld; ++m) v[m] = load_activation<KIND>(xrow, (64U * m < n ? 64U * m : n - 64U) + (threadIdx.x & 63U));
+}
+__device__ __forceinline__ float norm_factor(const float (&v)[kNormHeld], uint32_t n, float eps) {
+    float p[4];
+#pragma unroll
+    for (uint32_t c = 0; c < 4U; ++c) p[c] = __builtin_fmaf(v[c], v[c], 0.0F);
+    float sum;
+    if (n >= 512U) {
+#pragma unroll
+        for (uint32_t m = 4; m < kNormHeld; ++m)
+            if (64U * m < n) p[m & 3U] = __builtin_fmaf(v[m], v[m], p[m & 3U]);
+        sum = (p[0] + p[2]) + (p[1] + p[3]);
+    } else sum = __builtin_fmaf(v[2], v[2], p[0]) + __builtin_fmaf(v[3], v[3], p[1]);
+    sum = sum + __shfl_xor(sum, 32);
+    sum = sum + xor16_f(sum); sum = sum + xor8_f(sum); sum = sum + xor4_f(sum); sum = sum + xor2_f(sum); sum = sum + xor1_f(sum);
+    return 1.0F / __builtin_sqrtf(sum / static_cast<float>(n) + eps);
+}
 
 // ---------------------------------------------------------------------------------------------------- logit chains
 // Logits of 8 experts x 8 rows -> scores[row][expert] (used as the logit workspace). hidden % 32 == 0.
@@ -197,17 +225,27 @@ __device__ __forceinline__ void chain_start(ChainSlot& slot, const RouteArgs& a,
 // wavefront complete in order, so the writes only have to be issued before the reads - no barrier. __syncthreads() here
 // would also wait for every copy in flight, i.e. drain the three chunks the ring keeps ahead of the chain.
 __device__ __forceinline__ void chain_publish() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-template <int KIND>
-__device__ __forceinline__ void chain_widen(ChainSlot& slot) {
-    if constexpr (KIND != 0) {
+// NORM (fp32 rows as well): y = (x * factor) * w, w the lane's eight norm weights of the chunk.
+template <int KIND, bool NORM>
+__device__ __forceinline__ void chain_widen(ChainSlot& slot, float factor, const float (&w)[8]) {
+    if constexpr (KIND != 0 || NORM) {
         const uint32_t lane = threadIdx.x & 63U;
-        const u32x4 r = *reinterpret_cast<const u32x4*>(&slot.raw[4U * lane]);
-        const uint32_t h[4] = {r.x, r.y, r.z, r.w};
         float f[8];
+        if constexpr (KIND == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if constexpr (KIND == 1) { f[2 * q] = half_bits_to_float(h[q] & 0xffffU); f[2 * q + 1] = half_bits_to_float(h[q] >> 16); }
-            else { f[2 * q] = f_of(h[q] << 16); f[2 * q + 1] = f_of(h[q] & 0xffff0000U); }
+            for (uint32_t q = 0; q < 8U; ++q) f[q] = slot.x[8U * lane + q];
+        } else {
+            const u32x4 r = *reinterpret_cast<const u32x4*>(&slot.raw[4U * lane]);
+            const uint32_t h[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (KIND == 1) { f[2 * q] = half_bits_to_float(h[q] & 0xffffU); f[2 * q + 1] = half_bits_to_float(h[q] >> 16); }
+                else { f[2 * q] = f_of(h[q] << 16); f[2 * q + 1] = f_of(h[q] & 0xffff0000U); }
+            }
+        }
+        if constexpr (NORM) {
+#pragma unroll
+            for (uint32_t q = 0; q < 8U; ++q) f[q] = (f[q] * factor) * w[q];
         }
         *reinterpret_cast<f32x4*>(&slot.x[8U * lane]) = f32x4{f[0], f[1], f[2], f[3]};
         *reinterpret_cast<f32x4*>(&slot.x[8U * lane + 4U]) = f32x4{f[4], f[5], f[6], f[7]};
@@ -257,8 +295,9 @@ template <int N>
 __device__ __forceinline__ void chain_wait() { __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (0 << 8)); }      // (and every LDS read returned: the next copy reuses a slot this wave has read)
 
 // Logits of experts [e0, e0 + 8) for one row -> scores[row][expert] (+ bias), stored for readers in other workgroups of
-// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects.
-template <int KIND>
+// the same launch. hidden % 32 == 0. slots: 4 separate LDS objects. NORM: of the row's RMSNorm (hidden <= kChainNormHidden), whose factor is worked out while the
+// chunks, three at most, are on their way.
+template <int KIND, bool NORM>
 __device__ __forceinline__ void route_chain_block(ChainSlot* const (&slots)[4], const RouteArgs& a, uint32_t row, uint32_t e0) {
     constexpr uint32_t NI = chain_copies<KIND>();
     const uint32_t lane = threadIdx.x & 63U, chunks = (a.hidden + kChainChunk - 1U) / kChainChunk;
@@ -266,9 +305,22 @@ __device__ __forceinline__ void route_chain_block(ChainSlot* const (&slots)[4], 
     const uint32_t el = lane & 7U;                      // chain form: the lane's expert
     const uint32_t bh = lane >> 5, bl = lane & 31U;     // butterfly form: experts bh, bh + 2, bh + 4, bh + 6; partial sum bl
     float acc = 0.0F, part[4] = {0.0F, 0.0F, 0.0F, 0.0F};
+    static_assert(kChainNormHidden <= 3U * kChainChunk, "norm weights of three chunks");
+    float norm_weights[4][8] = {}, held[kNormHeld], factor = 1.0F;
+    if constexpr (NORM) {
+        norm_ask<KIND>(held, a.x + row * a.x_stride, a.hidden);
+#pragma unroll
+        for (uint32_t s = 0; s < 3U; ++s) {
+            const uint32_t k = kChainChunk * s + 8U * lane, from = k < a.hidden ? k : a.hidden - 8U;
+#pragma unroll
+            for (uint32_t q = 0; q < 8U; ++q) norm_weights[s][q] = a.norm_w ? a.norm_w[from + q] : 1.0F;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (uint32_t s = 0; s < 3U; ++s)
         if (s < chunks) chain_start<KIND>(*slots[s], a, row, e0, s * kChainChunk);
+    if constexpr (NORM) factor = norm_factor(held, a.hidden, a.norm_eps);
     for (uint32_t c0 = 0; c0 < chunks; c0 += 4U) {
 #pragma unroll
         for (uint32_t s = 0; s < 4U; ++s) {
@@ -281,7 +333,7 @@ __device__ __forceinline__ void route_chain_block(ChainSlot* const (&slots)[4], 
                 else chain_wait<2 * NI>();
                 if (c + 3U < chunks) chain_start<KIND>(*slots[(s + 3U) % 4U], a, row, e0, (c + 3U) * kChainChunk);
                 ChainSlot& slot = *slots[s];
-                chain_widen<KIND>(slot);
+                chain_widen<KIND, NORM>(slot, factor, norm_weights[s]);
                 const uint32_t kc = a.hidden - c * kChainChunk < kChainChunk ? a.hidden - c * kChainChunk : kChainChunk;
                 if (!butterfly) {
                     // full chunk: straight-line code, operands fetched three steps of 16 features ahead (against one step: layers 0.2..0.4

@@ -145,17 +145,29 @@ __global__ __launch_bounds__(256) void rmsnorm_f32_kernel(const float* x, const 
 // block; the last of a row's blocks publishes the row's status word.
 // Row r counts its finished blocks in ticket[r * stride] and collects its flags in flags[r * stride]. LINES: the words are reached
 // by device-scope atomics only and the count is a plain arrival (route_early.hpp); otherwise the count is an acquire-release ticket.
-template <int KIND, bool LINES = false>
+// NORM: the image of the row's RMSNorm, which is left in a.normed too (a block's eight groups are of one row: hidden % 256 == 0).
+template <int KIND, bool NORM, bool LINES = false>
 __device__ __forceinline__ void a8_prologue_block(const RouteArgs& a, uint32_t qb, uint32_t* ticket, uint32_t* flags, uint32_t stride,
                                                   uint32_t* row_tag = nullptr, uint32_t epoch = 0) {
     const uint32_t lane = threadIdx.x;
     {
         const uint32_t groups = a.hidden / 32U, total = a.rows * groups, g0 = qb * 8U;
+        float factor = 1.0F;
+        if constexpr (NORM) {
+            float held[kNormHeld];
+            norm_ask<KIND>(held, a.x + (g0 / groups) * a.x_stride, a.hidden);
+            factor = norm_factor(held, a.hidden, a.norm_eps);
+        }
         for (uint32_t i = 0; i < 8U; i += 2U) {
             const uint32_t g = g0 + i + (lane >> 5), j = lane & 31U;
             if (g < total) {
                 const uint32_t r = g / groups, gi = g % groups;
-                const float v = load_activation<KIND>(a.x + r * a.x_stride, gi * 32U + j);
+                float v = load_activation<KIND>(a.x + r * a.x_stride, gi * 32U + j);
+                if constexpr (NORM) {
+                    v = v * factor;
+                    if (a.norm_w) v = v * a.norm_w[gi * 32U + j];
+                    a.normed[static_cast<size_t>(r) * a.hidden + gi * 32U + j] = v;
+                }
                 const float amax = max32(__builtin_fabsf(v));
                 const bool tiny = amax > 0.0F && amax < 0x1p-119F;
                 const float delta = (amax == 0.0F || tiny) ? 1.0F : amax / 127.0F;
@@ -203,7 +215,7 @@ __device__ __forceinline__ void a8_prologue_block(const RouteArgs& a, uint32_t q
 // The place of the code is fixed: the 82 KB of an instance are more than the instruction cache holds, and by where they started - that is, by the
 // size of the kernels in front - the same instructions took 18.8 or 20.3 us (8 fp16 rows of hidden 3072, 64 experts; 16 rows 20.3 or 21.7). At a
 // multiple of 64 KB | 4 KB, 1, 2, 4, 8, 16 rows: 18.3, 18.9, 17.8, 19.3, 21.6 | 18.8, 19.2, 18.4, 19.2, 20.6.
-template <int KIND>
+template <int KIND, bool NORM = false>
 __global__ __launch_bounds__(64) __attribute__((aligned(65536))) void route_decode_kernel(RouteArgs a) {
     __shared__ ChainSlot slot0;
     __shared__ ChainSlot slot1;
@@ -220,7 +232,7 @@ __global__ __launch_bounds__(64) __attribute__((aligned(65536))) void route_deco
     uint32_t* tickets = a.plan ? a.plan + kPlanTicketsAt : nullptr;
     if (bid < a.route_blocks) {
         const uint32_t row = bid / neb;
-        route_chain_block<KIND>(slots, a, row, (bid % neb) * 8U);
+        route_chain_block<KIND, NORM>(slots, a, row, (bid % neb) * 8U);
         if (!a.plan) return;
         // hand-off between workgroups: the wave's logit stores happen before the barrier, the barrier before lane 0's
         // ticket increment, which releases them at device scope; the workgroup that takes the row's last ticket acquires with
@@ -259,7 +271,7 @@ __global__ __launch_bounds__(64) __attribute__((aligned(65536))) void route_deco
             }
         }
     } else {
-        a8_prologue_block<KIND>(a, bid - a.route_blocks, tickets + 16U, tickets + 128U, 1U);
+        a8_prologue_block<KIND, NORM>(a, bid - a.route_blocks, tickets + 16U, tickets + 128U, 1U);
     }
 }
 
@@ -594,7 +606,7 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
     }
     bid -= nb.early;
     if (bid < nb.prologue) {
-        a8_prologue_block<KIND, true>(a, bid, lines + kLinesPrologue, lines + kLinesPrologue + 1U, kLineWords, lines + kLinesRowTags, epoch);
+        a8_prologue_block<KIND, false, true>(a, bid, lines + kLinesPrologue, lines + kLinesPrologue + 1U, kLineWords, lines + kLinesRowTags, epoch);
         return;
     }
     bid -= nb.prologue;
@@ -1788,9 +1800,14 @@ void launch_route_logits(RouteArgs& a, hipStream_t st) {
     if (a.rows <= kFusedMaxRows) {
         a.route_blocks = neb * a.rows;
         const uint32_t blocks = a.route_blocks + a.quant_blocks;
-        if (a.kind == MI355_INPUT_F32) route_decode_kernel<0><<<blocks, 64, 0, st>>>(a);
-        else if (a.kind == MI355_INPUT_F16) route_decode_kernel<1><<<blocks, 64, 0, st>>>(a);
-        else route_decode_kernel<2><<<blocks, 64, 0, st>>>(a);
+        const auto launch = [&](auto norm) {
+            constexpr bool NORM = decltype(norm)::value;
+            if (a.kind == MI355_INPUT_F32) route_decode_kernel<0, NORM><<<blocks, 64, 0, st>>>(a);
+            else if (a.kind == MI355_INPUT_F16) route_decode_kernel<1, NORM><<<blocks, 64, 0, st>>>(a);
+            else route_decode_kernel<2, NORM><<<blocks, 64, 0, st>>>(a);
+        };
+        if (a.normed) launch(std::true_type{});
+        else launch(std::false_type{});
     } else launch_route_batch_logits(a, st);
 }
 }  // namespace
@@ -2009,13 +2026,6 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     a.wr = router_weight; a.bias = logit_bias; a.ids = ids; a.weights = weights; a.scores = scores;
     a.codes = r->codes; a.deltas = r->deltas; a.sums = r->sums; a.status = r->status; a.job_status = r->job_status; a.plan = r->plan;
     a.quant_blocks = (rows * (wv.hidden / 32U) + 7U) / 8U;
-    if (norm.on) {
-        // The normalised rows in a launch of their own; the router takes them as fp32 rows. (In the router's launch every workgroup worked its
-        // row's factor out again, in front of its chain. Layers of 1 row x 4096, 3 x 6144, 8 x 3072, 16 x 4096 fp32 rows: 59.5, 85.4, 74.5,
-        // 139.4 us, now 46.6, 62.1, 67.3, 96.8; 5 rows of 2048 with an always-on expert 64.2 -> 61.0.)
-        if (do_front) norm_rows();
-        a.x = reinterpret_cast<const uint8_t*>(norm.normed); a.kind = MI355_INPUT_F32; a.x_stride = 4ULL * wv.hidden;
-    }
     const uint32_t items = rows * wv.top_k;
     // Early routes (route_early.hpp): the expert choice from lane-parallel logits in a short first launch, the exact router beside
     // the projection, down rows + combine on the verified work items. Taken where the 64-row projection sweep and the down +
@@ -2028,9 +2038,17 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     // 35.7 / 40.3, 5 rows 38.4 / 48.6, 6 rows 41.2 / 57.8.
     // Down rows of another format, 1, 8, 16 rows against the router launch, the projection and the same down + combine launch: Q6_K 31.6, 67.5,
     // 111.8 -> 26.2, 58.5, 95.2 us, Q8_0 31.0, 67.6, 111.7 -> 25.3, 58.6, 92.1, Q5_1 30.8, 61.0, 100.5 -> 24.9, 52.0, 83.8.
-    if (p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
-        (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
-        wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden) {
+    const bool early = p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
+                       (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
+                       wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden;
+    if (norm.on && (early || wv.hidden > kChainNormHidden)) {
+        // The normalised rows in a launch of their own; the router takes them as fp32 rows. (In the router's launch every workgroup works its
+        // row's factor out again, in front of its chain. Layers of 1 row x 4096, 3 x 6144, 8 x 3072, 16 x 4096 fp32 rows: 59.5, 85.4, 74.5,
+        // 139.4 us, so 46.6, 62.1, 67.3, 96.8; 5 rows of 2048 with an always-on expert 64.2 -> 61.0.)
+        if (do_front) norm_rows();
+        a.x = reinterpret_cast<const uint8_t*>(norm.normed); a.kind = MI355_INPUT_F32; a.x_stride = 4ULL * wv.hidden;
+    } else if (norm.on) { a.norm_w = norm.weight; a.norm_eps = norm.eps; a.normed = norm.normed; }
+    if (early) {
         a.awords = r->plan + kPlanAwordsAt;
         a.early_perturb = g_early_perturb.load(std::memory_order_relaxed);
         // the early logits of row i (64-bit words) live in the row's (still unused) unweighted-output block: the exact logits own `scores`

@@ -2,6 +2,8 @@
 (mi355_moe_enqueue_layer_normed; the reference normalises in front of the MoE, src/ops/norm/norm.hpp:40-58, declared order
 src/cpu/core/reference.cpp:86-103) and the shared expert as an always-on expert of the same launches (policy.shared_experts).
 Bit for bit the oracle composition rmsnorm -> route -> A8 -> experts -> ordered combine."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -56,6 +58,62 @@ def test_rmsnorm_inside_the_layer_entry(strix, kind, H, I, E, K, T, scaled):
     # the standalone kernel gives the same rows
     if kind == "f32":
         assert np.array_equal(bits(strix.rmsnorm_f32(x_t.cuda(), dev(nw) if scaled else None, eps).cpu().numpy()), bits(want_n))
+
+
+# The norm inside the router's launch (hidden up to 1536, no early routes) and in a launch of its own: both sides of that line, each count of values that
+# the norm launch holds (2048, 4096, 8192 and rows with a rest), with an always-on expert, without a norm weight, and a staged batch.
+@pytest.mark.parametrize("kind,H,E,K,S,T,scaled", [
+    ("f32", 256, 8, 2, 1, 16, True), ("f16", 512, 8, 2, 0, 3, False), ("bf16", 768, 12, 3, 1, 2, True), ("f16", 1280, 8, 2, 0, 2, True), ("bf16", 1536, 8, 2, 1, 16, True),
+    ("f32", 1536, 8, 2, 0, 3, True), ("f16", 1792, 8, 2, 0, 3, True), ("f16", 2304, 8, 2, 1, 3, True), ("bf16", 4096, 6, 2, 0, 16, True), ("f32", 4352, 6, 2, 0, 2, False),
+    ("f16", 6144, 6, 2, 1, 8, True), ("bf16", 8192, 6, 2, 0, 1, True), ("f16", 8448, 4, 2, 1, 4, True), ("f32", 8448, 4, 1, 0, 2, False), ("bf16", 8448, 4, 2, 0, 20, True)])
+def test_norm_of_every_width(strix, kind, H, E, K, S, T, scaled):
+    I, eps = 256, 1e-5
+    rng = np.random.default_rng(H + T + S)
+    gate, up, down = layer_tensors(rng, H, I, E + S, orc.Q4_K, orc.Q4_K)
+    x_t = torch.from_numpy((rng.standard_normal((T, H)) * 3.0).astype(np.float32)).to(DT[kind])
+    nw = (1.0 + 0.2 * rng.standard_normal(H)).astype(np.float32) if scaled else None
+    wr = (rng.standard_normal((E, H)) * 0.02).astype(np.float32)
+    layer = strix.MoeLayer(H, I, E + S, K + S, dev(gate), dev(up), dev(down), T)
+    y, ids, wts, _ = layer.run_layer(x_t.cuda(), dev(wr), norm=(dev(nw) if scaled else None, eps), shared_experts=S)
+    want_n = orc.rmsnorm_f32(x_t.to(torch.float32).numpy(), nw, eps)
+    assert np.array_equal(bits(layer.normed[:T].cpu().numpy()), bits(want_n))
+    ids_r, w_r, _, _ = orc.route(want_n, wr, K)
+    ids_ref = np.concatenate([ids_r, np.tile(np.arange(E, E + S, dtype=np.uint32), (T, 1))], axis=1)
+    w_ref = np.concatenate([w_r, np.ones((T, S), np.float32)], axis=1)
+    assert np.array_equal(ids.cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(bits(wts.cpu().numpy()), bits(w_ref))
+    c, d, s, _ = orc.quantize_a8(want_n)
+    assert np.array_equal(layer.codes[:T].cpu().numpy(), c) and np.array_equal(bits(layer.deltas[:T].cpu().numpy()), bits(d))
+    ref = orc.routed_experts(H, I, K + S, gate, up, down, orc.Q4_K, c, d, s, ids_ref)
+    assert np.array_equal(bits(y.cpu().numpy()), bits(orc.combine(0, w_ref, ids_ref, ref.rawdots)))
+    assert np.all(layer.status[:T].cpu().numpy() == 0)
+
+
+def launches(program):
+    """The nodes that a captured program holds."""
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        program()
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=side):
+        program()
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    count = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+@pytest.mark.parametrize("H,S,T,more", [(256, 0, 1, 0), (1024, 0, 3, 0), (1024, 1, 16, 0), (1536, 1, 1, 0), (1792, 0, 1, 1), (2048, 1, 16, 1)])
+def test_launches_of_the_norm(strix, H, S, T, more):
+    """Short rows without early routes are normalised inside the router's launch: a launch more took such a layer 2.5 to 3 us longer."""
+    I, E, K = 256, 8, 2
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    layer = strix.MoeLayer(H, I, E + S, K + S, draw((E + S) * I, H), draw((E + S) * I, H), draw((E + S) * H, I), T)
+    x, router = torch.randn((T, H), device="cuda", generator=gen).half(), torch.randn((E, H), device="cuda", generator=gen) * 0.02
+    weight = torch.ones(H, device="cuda")
+    plain = launches(lambda: layer.run_layer(x, router, shared_experts=S))
+    assert launches(lambda: layer.run_layer(x, router, shared_experts=S, norm=(weight, 1e-6))) == plain + more
 
 
 @pytest.mark.parametrize("gate_type,down_type,H,I,E,K,S,T", [
