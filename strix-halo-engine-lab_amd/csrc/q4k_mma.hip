@@ -31,8 +31,10 @@ inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, u
     q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
-// rows x 27648, 8 rows: 59 -> 33 us). Three slots a team where they hold up to eight rows: dense 27648 x 5120, 4 | 8 rows, two, three, four slots 74.4, 72.1,
-// 73.6 | 86.1, 83.4, 83.9 us; sixteen rows are the same with two (102.3).
+// rows x 27648, 8 rows: 59 -> 33 us). Three slots a team where they hold up to eight rows and the matrix is long enough for the third to pay for its
+// start: dense blocks over weights of more than 1 GB in turn, hidden | ffn, two, three slots, 4 and 8 rows: 4096 | 4096 27.7, 27.9 and 27.0, 27.5 us; 2048 |
+// 8192 26.6, 26.5 and 27.8, 27.9; 6144 | 6144 35.2, 35.3 and 36.3, 36.3; 2048 | 16384 35.8, 34.9 and 40.5, 40.0; 8192 | 8192 43.3, 42.6 and 44.6, 44.1; 4096 |
+// 14336 40.7, 40.0 and 47.8, 47.1; 5120 | 27648 73.7, 71.4 and 83.9, 80.9 (four slots 73.6 and 83.9). Sixteen rows are the same with two (102.3).
 template <int FMT, int NAL>
 inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     constexpr bool WIDE = mma_wide<FMT, NAL>();
@@ -42,9 +44,13 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
     if constexpr (FMT == kMmaQ4K && !WIDE) {
         const MmaGrid g = mma_grid(w, rows, dense, items, tiles, 2U * NAL, 1U);
         if (static_cast<uint64_t>(g.grid.x) * g.grid.y <= compute_units()) {
-            constexpr int DEEP = NAL <= 4 ? 3 : 2;
-            if (direct) q4k_mma_down_kernel<FMT, NAL, DEEP, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
-            else q4k_mma_down_kernel<FMT, NAL, DEEP, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            const auto launch = [&](auto slots) {
+                constexpr int DEEP = decltype(slots)::value;
+                if (direct) q4k_mma_down_kernel<FMT, NAL, DEEP, 4, true><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+                else q4k_mma_down_kernel<FMT, NAL, DEEP, 4, false><<<g.grid, 1024, 0, st>>>(MmaArgs{w, r, g.l});
+            };
+            if (NAL <= 4 && static_cast<uint64_t>(tiles) * (w.ffn / 256U) >= 4096U) launch(std::integral_constant<int, NAL <= 4 ? 3 : 2>{});
+            else launch(std::integral_constant<int, 2>{});
             return;
         }
     }

@@ -62,3 +62,20 @@ def test_dense_rows_equal_one_by_one(strix, rows, hidden, ffn):
     out = layer.run(x, ids, one)
     for r in range(rows):
         assert torch.equal(out[r:r + 1].view(torch.int32), alone.run(x[r:r + 1], ids[:1], one[:1]).view(torch.int32)), r
+
+
+# long down rows of a dense block in stage teams: both numbers of ring slots (2048 | 16384 is the least matrix of three), stages that the teams do not
+# share evenly, fewer stages than teams; against batches of one row, which the vector-ALU sweeps serve
+@pytest.mark.parametrize("hidden,ffn", [(256, 512), (512, 8448), (2048, 16384), (2048, 16640), (1024, 33024)])
+@pytest.mark.parametrize("rows", [3, 4, 5, 8])
+def test_stage_teams_equal_one_by_one(strix, hidden, ffn, rows):
+    gen = torch.Generator(device="cuda").manual_seed(hidden + ffn + rows)
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    tensors = draw(ffn, hidden), draw(ffn, hidden), draw(hidden, ffn)
+    layer, one = (strix.MoeLayer(hidden, ffn, 1, 1, *tensors, n, intermediates=True) for n in (rows, 1))
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+    ids, weights = torch.zeros((rows, 1), dtype=torch.int32, device="cuda"), torch.ones((rows, 1), device="cuda")
+    out = layer.run(x, ids, weights).clone()
+    assert int(layer.status[:rows].sum()) == 0
+    for r in range(rows):
+        assert torch.equal(out[r:r + 1].view(torch.int32), one.run(x[r:r + 1], ids[r:r + 1], weights[r:r + 1]).view(torch.int32)), r
