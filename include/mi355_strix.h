@@ -286,6 +286,9 @@ void mi355_debug_early_route_perturb(uint32_t amount);
  * most four super-blocks as contiguous stages; on = 0 sends them through the 144-byte-block stages that every other shape uses, so that
  * the two forms can be compared (same bits). Process-wide; the default is on. */
 void mi355_debug_down_merge_flat(uint32_t on);
+/* Test and measurement aid (no counterpart in the reference): the workgroup form of the fp16 prefill. 0 (the default): by the rule on the
+ * batch's size; 1: four wavefronts, items of at most 32 rows; 2: the wide form, items of at most 128. The two give the same bits. Process-wide. */
+void mi355_debug_prefill_form(uint32_t form);
 
 /* The scalar gate of an always-on shared expert (tensor ffn_gate_inp_shexp, fp32 [hidden]): gate[row * gate_stride] =
  * 1 / (1 + exp(-dot(x[row], scalar_weight))), the reference's shared_gate_dot (src/hip_shared_expert_launcher.hip:624-645): 256

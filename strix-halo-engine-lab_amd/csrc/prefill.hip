@@ -3,6 +3,8 @@
 #include "launchers.hpp"
 #include "prefill_reg.hpp"
 
+#include <atomic>
+
 namespace strix950 {
 
 // What a batch needs besides its plan before the products, one workgroup per row: the row's sub-block sums (a thread per sub-block of 32,
@@ -80,8 +82,11 @@ bool few_rows(const mi355_moe_weights& wv, uint32_t assignments) {
 }
 }  // namespace
 
+std::atomic<uint32_t> g_prefill_form{0};
+
 uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments) {
-    return few_rows(wv, assignments) ? 32U : kPfTile;
+    const uint32_t form = g_prefill_form.load(std::memory_order_relaxed);
+    return (form ? form == 1U : few_rows(wv, assignments)) ? kPfFewRows : kPfTile;
 }
 
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, const PlanArgs& plan, uint32_t items_at, uint32_t order_at, hipStream_t st) {
@@ -91,7 +96,7 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
     const uint32_t cus = compute_units();
     const uint32_t resident = (cus > 8U ? cus : 256U) & ~7U;
     const auto grid_of = [&](uint32_t units, uint32_t each = 1U) { return units < each * resident ? units : each * resident; };
-    const bool few = few_rows(wv, a.assignments);
+    const bool few = plan.split == kPfFewRows;          // (the form that the plan's items are made for)
     const auto launch = [&](auto mode, uint32_t type) {
         constexpr int M = decltype(mode)::value;
         const auto of = [&](auto format) {
@@ -114,3 +119,5 @@ void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_
 }
 
 }  // namespace strix950
+
+extern "C" void mi355_debug_prefill_form(uint32_t form) { strix950::g_prefill_form.store(form, std::memory_order_relaxed); }

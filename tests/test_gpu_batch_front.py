@@ -101,12 +101,11 @@ def test_layer_equals_router_then_experts(strix, rows, hidden, ffn, experts, top
     assert all(s & strix.STATUS_INVALID_ROUTE for s in layer.status[:rows].cpu().tolist())
 
 
-# narrow prefill (few rows per expert on average) with items of one row, around 64 and 128 rows, and the wide form for comparison
+# the four-wave prefill with experts of one row, around 32, 64 and 128 rows, against the wide form on each expert alone
 @pytest.mark.parametrize("counts,hidden,ffn", [((1, 64, 0, 65, 31, 0, 32, 0, 0, 0, 0, 0), 256, 768), ((128, 0, 0, 0, 33, 1, 0, 0, 0, 0, 0, 0), 512, 256),
                                                ((129, 63, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0), 1280, 768)])
-def test_narrow_prefill_equals_wide(strix, counts, hidden, ffn):
+def test_narrow_prefill_equals_wide(strix, prefill_forms, counts, hidden, ffn):
     E = len(counts)
-    assert sum(counts) <= 24 * E                                           # the narrow form's rule
     gen = torch.Generator(device="cuda").manual_seed(hidden)
     draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
     gate, up, down = draw(E * ffn, hidden), draw(E * ffn, hidden), draw(E * hidden, ffn)
@@ -115,12 +114,17 @@ def test_narrow_prefill_equals_wide(strix, counts, hidden, ffn):
     T = len(ids)
     x = torch.randn((T, hidden), device="cuda", generator=gen).to(torch.float16)
     ones = torch.ones((T, 1), device="cuda")
-    narrow = strix.MoeLayer(hidden, ffn, E, 1, gate, up, down, T, prefill_f16=True).run_prefill_f16(x, ids, ones)
-    for e in {int(i) for i in ids.flatten()}:                              # expert by expert as one-expert layers: the wide form past 24 rows
+    prefill_forms.use("four_waves")
+    layer = strix.MoeLayer(hidden, ffn, E, 1, gate, up, down, T, prefill_f16=True)
+    narrow = layer.run_prefill_f16(x, ids, ones)
+    prefill_forms.check(layer)
+    prefill_forms.use("wide")
+    for e in {int(i) for i in ids.flatten()}:                              # expert by expert as one-expert layers
         rows = (ids[:, 0] == e).nonzero()[:, 0]
         pick = lambda t, n: t[e * n:(e + 1) * n].contiguous()
         alone = strix.MoeLayer(hidden, ffn, 1, 1, pick(gate, ffn), pick(up, ffn), pick(down, hidden), len(rows), prefill_f16=True)
         got = alone.run_prefill_f16(x[rows].contiguous(), torch.zeros_like(ids[rows]), ones[rows])
+        prefill_forms.check(alone)
         assert torch.equal(got, narrow[rows])                              # the same products and sums in the same order
 
 

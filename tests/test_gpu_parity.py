@@ -1067,7 +1067,7 @@ def random_q8_0(rng, shape_rows, width):
     (1024, 768, 6, 2, 200, orc.Q5_K, orc.Q5_K, True),
     (768, 512, 3, 2, 150, orc.Q4_K, orc.Q5_K, True),
     (512, 1024, 1, 1, 140, orc.Q5_K, orc.Q8_0, True)])
-def test_prefill_f16_mfma_q8_0_tensors(strix, H, I, E, K, T, gate_type, down_type, random_bytes):
+def test_prefill_f16_mfma_q8_0_tensors(strix, prefill_form, H, I, E, K, T, gate_type, down_type, random_bytes):
     """The matrix-core prefill form with Q8_0 / Q5_K / mixed expert tensors (the always-on shared expert is experts = top_k = 1
     with weight 1) against the exact-weight product, tolerance 2e-3 as for Q4_K: max abs error over the output rms, and
     elementwise on every output above a hundredth of the rms, for the unweighted down outputs and the combined output."""
@@ -1090,6 +1090,7 @@ def test_prefill_f16_mfma_q8_0_tensors(strix, H, I, E, K, T, gate_type, down_typ
         ids_ref, w_ref, _, _ = orc.route(x.astype(np.float32), wr, K)
     layer = strix.MoeLayer(H, I, E, K, dev(gate), dev(up), dev(down), T, prefill_f16=True, gate_type=gate_type, down_type=down_type)
     y = layer.run_prefill_f16(dev(x), dev(ids_ref.astype(np.int32)), dev(w_ref)).cpu().numpy()
+    prefill_form.check(layer)
     want, raw_ref = exact_weight_layer(x, ids_ref, w_ref, gate, up, down, H, I, K, gate_type=gate_type, down_type=down_type)
     for got, ref in ((layer.rawdots[:T].cpu().numpy(), raw_ref), (y, want)):
         ref64 = ref.astype(np.float64)
@@ -1107,10 +1108,10 @@ def test_prefill_f16_mfma_q8_0_tensors(strix, H, I, E, K, T, gate_type, down_typ
             layer.run(dev(x[:1]), dev(ids_ref[:1].astype(np.int32)), dev(w_ref[:1]))
 
 
-def test_prefill_f16_h_beyond_fp16_fails_closed(strix):
+def test_prefill_f16_h_beyond_fp16_fails_closed(strix, prefill_form):
     """The prefill form keeps h in fp16: a row whose h leaves the fp16 range is flagged as a non-finite projection, the job's
     down phase is skipped, the merge publishes no row, and a clean call on the same buffers afterwards is unaffected."""
-    H, I, E, K, T = 512, 256, 4, 2, 40
+    H, I, E, K, T = 512, 256, 4, 2, 90
     rng = np.random.default_rng(77)
     gate, up, down = make_layer(rng, H, I, E)
     x = rng.standard_normal((T, H)).astype(np.float16)
@@ -1118,6 +1119,7 @@ def test_prefill_f16_h_beyond_fp16_fails_closed(strix):
     ids, w, _, _ = orc.route(x.astype(np.float32), wr, K)
     layer = strix.MoeLayer(H, I, E, K, dev(gate), dev(up), dev(down), T, prefill_f16=True)
     want = layer.run_prefill_f16(dev(x), dev(ids.astype(np.int32)), dev(w)).clone()
+    prefill_form.check(layer)
     assert int(layer.status.sum()) == 0
     loud = x.copy()
     loud[3] *= 4096.0                                       # gate and up of row 3 grow 4096-fold: h far beyond 65504
@@ -1136,7 +1138,7 @@ def test_prefill_f16_h_beyond_fp16_fails_closed(strix):
                                        # many experts chosen by few rows each (plan items of 1 to 32 rows: token tiles with no
                                        # live row beside one that has some), 3 / 5 / 8 super-blocks per row
                                        (768, 1280, 16, 4, 60), (512, 256, 40, 8, 33), (256, 256, 24, 2, 9), (2048, 768, 64, 8, 100)])
-def test_prefill_f16_mfma_matches_exact_weight_product(strix, H, I, E, K, T):
+def test_prefill_f16_mfma_matches_exact_weight_product(strix, prefill_form, H, I, E, K, T):
     """The fp16 MFMA prefill form against the exact-weight product: tolerance 2e-3 (fp16 activations), both as max abs
     error over the output rms and elementwise on the outputs of at least rms size; the gate / up / down tiles are checked
     through the unweighted down outputs as well as the combined output. One dense projection is also tied to the oracle's BASE-class
@@ -1148,6 +1150,7 @@ def test_prefill_f16_mfma_matches_exact_weight_product(strix, H, I, E, K, T):
     ids_ref, w_ref, _, _ = orc.route(x.astype(np.float32), wr, K)
     layer = strix.MoeLayer(H, I, E, K, dev(gate), dev(up), dev(down), T, prefill_f16=True)
     y = layer.run_prefill_f16(dev(x), dev(ids_ref.astype(np.int32)), dev(w_ref)).cpu().numpy()
+    prefill_form.check(layer)
     want, raw_ref = exact_weight_layer(x, ids_ref, w_ref, gate, up, down, H, I, K)
     for got, ref in ((layer.rawdots[:T].cpu().numpy(), raw_ref), (y, want)):
         ref64 = ref.astype(np.float64)

@@ -85,7 +85,7 @@ def test_other_down_formats_repeat_their_bits(strix, down_type):
 
 # the matrix-core prefill (token rings shared by the workgroup's waves, a barrier per stage)
 @pytest.mark.parametrize("H,I,E,K,T", [(1024, 512, 12, 4, 300), (768, 1280, 5, 2, 150)])
-def test_prefill_f16_repeats_its_bits(strix, H, I, E, K, T):
+def test_prefill_f16_repeats_its_bits(strix, prefill_form, H, I, E, K, T):
     rng = np.random.default_rng(5000 + T)
     gate, up, down = make_layer(rng, H, I, E)
     wr = dev((rng.standard_normal((E, H)) * 0.02).astype(np.float32))
@@ -97,4 +97,5 @@ def test_prefill_f16_repeats_its_bits(strix, H, I, E, K, T):
     def run():
         out["y"] = layer.run_prefill_f16(x, ids, wts)
     assert repeat(run, lambda: (out["y"], layer.rawdots[:T]), 100) == 0
+    prefill_form.check(layer)
     assert int(layer.status[:T].sum()) == 0

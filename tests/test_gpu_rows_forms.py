@@ -319,7 +319,7 @@ def _bf16_round(a):
     (orc.Q4_K, orc.Q4_K, 1024, 512, 8, 2, 70),          # both halves of h in one sweep of K
     (orc.Q8_0, orc.Q8_0, 512, 256, 4, 2, 33),           # K swept twice in one launch, the low half of h first (the rounding comes after both)
     (orc.Q4_K, orc.Q4_K, 2048, 768, 16, 4, 9)])
-def test_prefill_rows_f16_strided_views(strix, gate_type, down_type, H, I, E, K, T):
+def test_prefill_rows_f16_strided_views(strix, prefill_form, gate_type, down_type, H, I, E, K, T):
     """mi355_moe_enqueue_prefill_rows_f16 (known_rows::PrefillRows / enqueue_prefill with the fp16 form,
     include/strix/hip_moe_q4k_a8_known_rows.hpp:75-111): every view strided inside one record per row. The unweighted outputs are
     bit for bit those of the dense entry point (the same kernels behind another view), with rawdots_bf16 their bfloat16 rounding;
@@ -336,6 +336,7 @@ def test_prefill_rows_f16_strided_views(strix, gate_type, down_type, H, I, E, K,
     wts = rng.random((T, K)).astype(np.float32)
     layer = strix.MoeLayer(H, I, E, K, dev(gate), dev(up), dev(down), T, prefill_f16=True, gate_type=gate_type, down_type=down_type)
     dense_raw = layer.run_prefill_f16(dev(x), dev(ids), dev(wts), combine=strix.COMBINE_NONE).cpu().numpy().copy()
+    prefill_form.check(layer)
     assert int(layer.status.sum()) == 0
     dense_out = layer.run_prefill_f16(dev(x), dev(ids), dev(wts)).cpu().numpy().copy()
 
