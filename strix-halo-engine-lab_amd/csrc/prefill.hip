@@ -7,36 +7,26 @@
 
 namespace strix950 {
 
-// What a batch needs besides its plan before the products, one workgroup per row: the row's sub-block sums (a thread per sub-block of 32,
-// fp32 sum in index order), zeros in the padding slots of the sums of h of the row's assignments (ffn / 32 not a multiple of 16; every
-// assignment has a row of sums, whichever order the plan gives them), and - with a check - the routes' check and the status words.
+// What a batch needs before the products: the expert plan (a workgroup per expert), and a workgroup per row for the row's sub-block sums (a thread per
+// sub-block of 32, fp32 sum in index order) and - with a check - the routes' check and the status words.
 // Bound by latency: one launch in the place of three (333 rows: about 4.5 us each).
-__global__ __launch_bounds__(512) void prefill_prologue_kernel(const uint8_t* x, uint64_t x_stride, uint32_t k, uint8_t* x_sums, uint8_t* h_sums, uint32_t ffn,
-                                                              uint32_t top_k, RouteCheck check, PlanArgs plan) {
+__global__ __launch_bounds__(512) void prefill_prologue_kernel(const uint8_t* x, uint64_t x_stride, uint32_t k, uint8_t* x_sums, uint32_t top_k, RouteCheck check, PlanArgs plan) {
     __shared__ PlanLds lds;
     if (blockIdx.x < plan.experts) return plan_block(lds, plan, blockIdx.x);
     if (threadIdx.x >= 256U) return;
-    const uint32_t row = blockIdx.x - plan.experts, slots = pf_sum_slots(k), h_slots = pf_sum_slots(ffn), h_used = ffn / 32U, pad = h_slots - h_used;
+    const uint32_t row = blockIdx.x - plan.experts;
     _Float16* hi = reinterpret_cast<_Float16*>(x_sums + static_cast<size_t>(row) * pf_sum_row_bytes(k));
-    _Float16* lo = hi + slots;
-    for (uint32_t s = threadIdx.x; s < slots; s += 256U) {
+    _Float16* lo = hi + pf_sum_slots(k);
+    for (uint32_t s = threadIdx.x; s < k / 32U; s += 256U) {
         float sum = 0.0F;
-        if (s < k / 32U) {
-            const half8* p = reinterpret_cast<const half8*>(x + static_cast<size_t>(row) * x_stride + 64U * s);
+        const half8* p = reinterpret_cast<const half8*>(x + static_cast<size_t>(row) * x_stride + 64U * s);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const half8 v = p[i];
+        for (int i = 0; i < 4; ++i) {
+            const half8 v = p[i];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) sum += static_cast<float>(v[j]);
-            }
+            for (int j = 0; j < 8; ++j) sum += static_cast<float>(v[j]);
         }
         split_half(sum, hi[s], lo[s]);
-    }
-    for (uint32_t i = threadIdx.x; i < pad * top_k; i += 256U) {
-        const uint32_t slot = i / pad, s = h_used + i - slot * pad;
-        _Float16* out = reinterpret_cast<_Float16*>(h_sums + (static_cast<size_t>(row) * top_k + slot) * pf_sum_row_bytes(ffn));
-        out[s] = static_cast<_Float16>(0.0F);
-        out[h_slots + s] = static_cast<_Float16>(0.0F);
     }
     if (!check.status || threadIdx.x < 192U) return;
     uint32_t bad = 0;
@@ -90,7 +80,7 @@ uint32_t prefill_split(const mi355_moe_weights& wv, uint32_t assignments) {
 }
 
 void launch_prefill_products(const mi355_moe_weights& wv, PrefillArgs a, uint32_t rows, uint8_t* x_sums, const RouteCheck* check, const PlanArgs& plan, uint32_t items_at, uint32_t order_at, hipStream_t st) {
-    prefill_prologue_kernel<<<plan.experts + rows, 512, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums, a.h_sums, wv.ffn, wv.top_k, check ? *check : RouteCheck{}, plan);
+    prefill_prologue_kernel<<<plan.experts + rows, 512, 0, st>>>(a.x, a.x_stride, wv.hidden, x_sums, wv.top_k, check ? *check : RouteCheck{}, plan);
     const uint32_t item_slots = (a.items + 7U) / 8U * 8U;
     // persistent workgroups, as many as are resident: one per compute unit (LDS allows no second one) or `each` of the four-wave form
     const uint32_t cus = compute_units();

@@ -11,7 +11,7 @@ namespace strix950 {
 
 constexpr uint32_t kPfTile = 128;                 // weight rows and tokens per workgroup tile; the most rows of a plan item
 constexpr uint32_t kPfFewRows = 32;               // the most rows of an item of the four-wave form
-// sub-block sums of a row: two fp16 planes (hi, lo) of `pf_sum_slots(k)` halves each, the slots past k / 32 zero
+// sub-block sums of a row: two fp16 planes (hi, lo) of `pf_sum_slots(k)` halves each (copied 16 at a time; the slots past k / 32 hold nothing and are never multiplied)
 __host__ __device__ constexpr uint32_t pf_sum_slots(uint32_t k) { return (k / 32U + 15U) & ~15U; }
 __host__ __device__ constexpr size_t pf_sum_row_bytes(uint32_t k) { return 4U * static_cast<size_t>(pf_sum_slots(k)); }
 // bytes of the fp16 workspace: h [assignments][ffn], sums of h [assignments], sums of the input rows [rows]

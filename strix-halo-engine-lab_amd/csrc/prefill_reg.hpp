@@ -108,7 +108,7 @@ __device__ __forceinline__ void copy4_to_lds_at(const uint32_t* src, uint32_t ld
 }
 
 struct Rg8 { u32x4 a, b; uint32_t e; };                   // Q8_0: a stage's words of a lane
-struct RgFactor { uint32_t sc; half2v mul, add; };
+struct RgFactor { half2v mul, add; };
 
 // Waits until at most N younger operations are out, for the registers that follow (FIRST: the first of them as well)
 template <uint32_t N, bool FIRST> __device__ __forceinline__ void rg_wait_for(u32x4& f, u32x4& a, u32x4& b) {
@@ -290,16 +290,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     asm volatile("v_mov_b32 %0, 0x64006400" : "=v"(magic));
     // Q5_K: sc q is up to 1953, past the offset's mantissa: fma(1024 + q, sc, -1024 sc) = sc q, exact. Q8_0: 1152 + code, minus 1152.
     const _Float16 minus = static_cast<_Float16>(-1152.0F);
-    const auto factor_of = [&](uint32_t sc) -> RgFactor {
-        RgFactor f{};
-        f.sc = sc;
-        if (FMT == kRgQ5K) {
-            const _Float16 c = static_cast<_Float16>(static_cast<float>(sc)), n = c * static_cast<_Float16>(-1024.0F);
-            f.mul = half2v{c, c};
-            f.add = half2v{n, n};
-        }
-        return f;
-    };
     // two weights: bytes 0, 1 or (odd) 2, 3 of a word
     const auto expand_pair = [&](uint32_t w, uint32_t odd, const RgFactor& f) -> uint32_t {
         if (SCALED) return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0U, w, odd ? 0x0c030c02U : 0x0c010c00U)) * f.mul);
@@ -328,22 +318,23 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
 #pragma unroll
         for (uint32_t q = 0; q < 4U; ++q) scaled[q] = six_bits(q < 2U ? first : last, q & 1U) * units;
     };
-    const auto scaled_factor = [&](uint32_t p, uint32_t odd) -> RgFactor {
+    // of sub-block 2 p or (odd) 2 p + 1; SCALED: of the header that set_scaled was given (Q5_K: src/cpu/core/routed_expert.cpp:65-71)
+    const auto factor_of = [&](const u32x4& hd, uint32_t p, uint32_t odd) -> RgFactor {
         RgFactor f{};
-        f.mul = odd ? half2v{scaled[p].y, scaled[p].y} : half2v{scaled[p].x, scaled[p].x};
+        if (SCALED) f.mul = odd ? half2v{scaled[p].y, scaled[p].y} : half2v{scaled[p].x, scaled[p].x};
+        else if (FMT == kRgQ5K) {
+            const uint32_t at = 16U * (p & 1U) + 8U * odd, first = (hd.y >> at) & 255U, last = (hd.w >> at) & 255U;
+            const uint32_t sc = p < 2U ? (first & 63U) : ((last & 15U) | ((first >> 6) << 4));
+            const _Float16 c = static_cast<_Float16>(static_cast<float>(sc)), n = c * static_cast<_Float16>(-1024.0F);
+            f.mul = half2v{c, c};
+            f.add = half2v{n, n};
+        }
         return f;
     };
     // Q8_0: words 2 k, 2 k + 1 of the lane's codes of the stage's first block, as unsigned bytes code + 128
     const auto first_codes = [&](const Rg8& r, uint32_t k, uint32_t& w0, uint32_t& w1) {
         w0 = __builtin_amdgcn_alignbyte(k ? r.a.w : r.a.y, k ? r.a.z : r.a.x, 2U) ^ 0x80808080U;
         w1 = __builtin_amdgcn_alignbyte(k ? r.e : r.a.z, k ? r.a.w : r.a.y, 2U) ^ 0x80808080U;
-    };
-    // sc of sub-blocks 2 p and 2 p + 1 (src/cpu/core/routed_expert.cpp:65-71)
-    const auto scales = [&](const u32x4& hd, uint32_t p, uint32_t& s_lo, uint32_t& s_hi) {
-        const uint32_t sh0 = 16U * (p & 1U), sh1 = sh0 + 8U;
-        const uint32_t fa0 = (hd.y >> sh0) & 255U, fc0 = (hd.w >> sh0) & 255U, fa1 = (hd.y >> sh1) & 255U, fc1 = (hd.w >> sh1) & 255U;
-        s_lo = p < 2U ? (fa0 & 63U) : ((fc0 & 15U) | ((fa0 >> 6) << 4));
-        s_hi = p < 2U ? (fa1 & 63U) : ((fc1 & 15U) | ((fa1 >> 6) << 4));
     };
 
     // Everything from the first fetch to the last store is instantiated per number of token tiles that hold a row of the item
@@ -416,10 +407,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         first_codes(q8[0], 0U, w0, w1);
         bfrag = expand(w0, w1, RgFactor{});
     } else {
-        uint32_t s_lo, s_hi;
-        scales(hd_cur, 0, s_lo, s_hi);
         if (SCALED) set_scaled(hd_cur);
-        bfrag = expand(low(qs[0].x, f_cur.x, 0U), low(qs[0].y, f_cur.y, 0U), SCALED ? scaled_factor(0U, 0U) : factor_of(s_lo));
+        bfrag = expand(low(qs[0].x, f_cur.x, 0U), low(qs[0].y, f_cur.y, 0U), factor_of(hd_cur, 0U, 0U));
     }
     // A stage's MFMAs as a flat sequence of slots m = (k-step j, plane, token tile i); the A operand of slot m + W is requested right after
     // the MFMA of slot m into the registers that MFMA has just read (a window of W operands, which runs on over the stages' borders).
@@ -436,9 +425,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
         const auto stage = [&](auto p_constant, uint32_t b) __attribute__((always_inline)) {
                 constexpr uint32_t p = decltype(p_constant)::value;
                 const uint32_t s = 4U * b + p, bb = SWEEPS == 2U && b >= blocks ? b - blocks : b;            // (bb: of the rows)
-                uint32_t s_lo = 0, s_hi = 0;
-                if (FMT != kRgQ80) scales(hd_cur, p, s_lo, s_hi);
-                const RgFactor f_lo = SCALED ? scaled_factor(p, 0U) : factor_of(s_lo), f_hi = SCALED ? scaled_factor(p, 1U) : factor_of(s_hi);
+                const RgFactor f_lo = factor_of(hd_cur, p, 0U), f_hi = factor_of(hd_cur, p, 1U);
                 const u32x4 qw = qs[p];
                 const Rg8 r8 = q8[p % RING8];
                 const float d_now = half_bits_to_float(hd_cur.x & 0xffffU) * (SCALED ? 16384.0F : 1.0F);
@@ -507,11 +494,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
                                     }
                                 } else if (p == 3U) rg_wait_for<younger, FMT == kRgQ5K>(f_next, hd_next, qs[pn]);
                                 else asm volatile("s_waitcnt vmcnt(%1)" : "+v"(qs[pn]) : "n"(younger) : "memory");
-                                uint32_t n_lo, n_hi;
-                                scales(p == 3U ? hd_next : hd_cur, pn, n_lo, n_hi);
                                 if (SCALED && p == 3U) set_scaled(hd_next);
                                 const u32x4 fb = p == 3U ? f_next : f_cur;
-                                nw0 = low(qs[pn].x, fb.x, 2U * pn); nw1 = low(qs[pn].y, fb.y, 2U * pn); nf = SCALED ? scaled_factor(pn, 0U) : factor_of(n_lo);
+                                nw0 = low(qs[pn].x, fb.x, 2U * pn); nw1 = low(qs[pn].y, fb.y, 2U * pn); nf = factor_of(p == 3U ? hd_next : hd_cur, pn, 0U);
                             }
                         }
                     }

@@ -79,3 +79,21 @@ def test_many_experts_in_another_order(strix, prefill_form):
     out = layer.run_prefill_f16(x, ids, weights).clone()
     prefill_form.check(layer)
     assert torch.equal(layer.run_prefill_f16(x.flip(0), ids.flip(0), weights.flip(0)).flip(0), out)
+
+
+@pytest.mark.parametrize("kind", ["q4_k", "q5_k"])
+def test_workspace_of_nan(strix, prefill_form, kind):
+    """Sums past a row's sub-blocks (hidden 1280 and ffn 768 leave eight slots of a group of sixteen) and rows of h past an item's are read and never part of a
+    value: a workspace full of NaN gives the bits of a clean one."""
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    hidden, ffn, rows, experts, top_k = 1280, 768, 150, 4, 2
+    kind = {"q4_k": strix.TYPE_Q4_K, "q5_k": strix.TYPE_Q5_K}[kind]
+    layer = strix.MoeLayer(hidden, ffn, experts, top_k, *tensors(strix, gen, kind, experts, hidden, ffn), rows, prefill_f16=True, gate_type=kind, down_type=kind)
+    x = (torch.randn((rows, hidden), device="cuda", generator=gen) * 0.05).half()
+    ids = torch.rand((rows, experts), device="cuda", generator=gen).topk(top_k).indices.int()
+    weights = torch.rand((rows, top_k), device="cuda", generator=gen)
+    layer.h_f16.zero_()
+    want = layer.run_prefill_f16(x, ids, weights).clone()
+    layer.h_f16.fill_(0xFF)
+    assert torch.equal(layer.run_prefill_f16(x, ids, weights), want) and int(layer.status[:rows].sum()) == 0
+    prefill_form.check(layer)
