@@ -22,13 +22,16 @@ inline MmaGrid mma_grid(const mi355_moe_weights& w, uint32_t rows, uint32_t dens
 }
 // the rows of a dense batch at a stride of their own (every dense buffer and strided view; not the executor's pointer tables)
 inline bool mma_direct(const A8Image& img, uint32_t dense) { return dense && img.per_row == 1U && !img.table; }
-template <int FMT, int NAL>
+inline uint32_t mma_project_run(const mi355_moe_weights& w, uint32_t dense, uint32_t items) {
+    return mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items));
+}
+template <int FMT, int NAL, bool WIDE = false>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
-    const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_run_tiles(w.hidden / 256U, 8U, static_cast<uint64_t>(w.ffn / 32U) * (dense ? 1U : items)));
-    constexpr int DEPTH = NAL >= 8 ? 2 : 3, THREADS = 64 * mma_waves<2, mma_wide<FMT, NAL>()>();
+    const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_project_run(w, dense, items));
+    constexpr int DEPTH = NAL >= 8 ? 2 : 3, THREADS = 64 * mma_waves<2, WIDE>();
     if constexpr (FMT == kMmaQ4K)
-        if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
-    q4k_mma_project_kernel<FMT, NAL, DEPTH, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
+        if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true, WIDE><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
+    q4k_mma_project_kernel<FMT, NAL, DEPTH, false, WIDE><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
 // A launch with no more workgroups than compute units (few, long rows) runs four stages of a tile at a time (measured at 5120
 // rows x 27648, 8 rows: 59 -> 33 us). Three slots a team where they hold up to eight rows and the matrix is long enough for the third to pay for its
@@ -62,11 +65,31 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
         if (direct) { q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, true><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
     q4k_mma_down_kernel<FMT, NAL, DEPTH, 1, false><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
+// Gate / up rows past 16 activation rows: the wide form, or gate and up on one wavefront, which starts and ends a workgroup sooner (four wavefronts meet
+// where eight do, and no register is spilled). So the line goes by the stages that a workgroup runs over, by rows an expert where they are few, and lies higher
+// for Q5_K, whose wide form spills more. One wavefront against wide (time ratio; above one: wide is faster), rows an expert 18, 24, 32, 45, 64, 96:
+//   Q4_K  160 experts of ffn 512    4 stages .89 .92 .97 1.01 1.03 1.11   6 .97 .99 1.03 1.04 1.07 1.10   8 1.00 1.02 1.06 1.08 1.07 1.12
+//         80 experts of ffn 1536    4, runs of two tiles, 1.05 1.06 1.07 1.12 1.10 1.12   6 .96 .98 1.01 1.05 1.07 1.08   10 1.05 1.01 1.07 1.10 1.10 1.13
+//         32 experts of ffn 1024    4 .96 .91 .95 1.02 1.05 1.06   6 .97 .99 1.03 1.05 1.07 1.06   8 .95 .97 1.05 1.05 1.06 1.11   16 1.10 1.09 1.14 1.12 1.14 1.16
+//   Q5_K  160 experts of ffn 512    4 .83 .86 .90 .92 .97 1.06   6 .89 .93 .97 .96 .97 .98   8 .91 .95 .97 .99 .98 1.00   10 .96 .96 1.02 .99 1.03 1.05
+//         80 experts of ffn 1536    4, runs of two tiles, .99 .97 1.00 .99 1.03 1.05   6 .90 .91 .94 .98 .96 .98   8 .91 .95 .93 .98 .98 1.03
+//         32 experts of ffn 1024    4 .89 .89 .90 .97 .99 1.01   6 .93 .91 .97 1.02 1.03 1.07   8 .99 .96 1.04 1.06 1.09 1.11   12 1.06 1.08 1.15 1.14 1.13 1.14
+// (95 experts top-6 of 1536 x 1536, Q5_K, 31 rows an expert: 231 us, wide 243; 128 experts of 2048 x 768, Q4_K, 62 rows: 327, wide 297.) Dense, ffn 8192, 32, 36,
+// 48, 64 rows: 4 stages 1.11 .99 .96 1.00, 6 1.12 .97 .98 1.12, 8 1.13 1.01 1.05 1.11.
+template <int FMT>
+inline bool mma_project_wide(const mi355_moe_weights& w, uint32_t rows, uint32_t dense, uint32_t run) {
+    const uint32_t stages = w.hidden / 256U;
+    if (dense) return dense <= 32U || dense > 48U || stages >= 8U;
+    const uint64_t steps = static_cast<uint64_t>(stages) * run, rows_of_all = static_cast<uint64_t>(rows) * w.top_k;
+    if (FMT == kMmaQ5K) return stages >= 12U || steps * rows_of_all >= 400ULL * w.experts;
+    return steps >= 8U || steps * rows_of_all >= 180ULL * w.experts;
+}
 template <int FMT>
 inline void launch_mma_project_format(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, uint32_t width, hipStream_t st) {
     if (width <= 4U) launch_mma_project_nal<FMT, 2>(w, r, rows, dense, items, st);
     else if (width <= 8U) launch_mma_project_nal<FMT, 4>(w, r, rows, dense, items, st);
     else if (width <= 16U) launch_mma_project_nal<FMT, 8>(w, r, rows, dense, items, st);
+    else if (mma_project_wide<FMT>(w, rows, dense, mma_project_run(w, dense, items))) launch_mma_project_nal<FMT, 16, true>(w, r, rows, dense, items, st);
     else launch_mma_project_nal<FMT, 16>(w, r, rows, dense, items, st);
 }
 // (rows of another format: sixteen activation rows to a sweep at most, whose two halves of a group take the result registers of 32)

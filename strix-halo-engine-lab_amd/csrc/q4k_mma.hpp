@@ -63,7 +63,7 @@ template <int FMT, int NAL, int NM> constexpr uint32_t mma_table_at() { return m
 template <int FMT, int NAL, int NM> constexpr uint32_t mma_slot_bytes() { return mma_table_at<FMT, NAL, NM>() + (mma_acts<NAL>() < 16U ? 64U * mma_acts<NAL>() : 1024U * mma_table_copies<NAL>()); }
 template <int FMT, int NAL, int NM, int DEPTH, int TEAMS> constexpr uint32_t mma_ring_bytes() { return DEPTH * TEAMS * mma_slot_bytes<FMT, NAL, NM>(); }
 template <int NAL, int TEAMS> constexpr uint32_t mma_exchange_floats() { return TEAMS > 1 ? 2U * (TEAMS - 1U) * 4U * NAL * 64U : 1U; }
-// The wide form (mma_stage_wide) serves the sweeps of 32 activation rows.
+// The wide form (mma_stage_wide) serves sweeps of 32 activation rows: of Q4_K down rows, and of gate / up rows where it is the faster one (mma_project_wide).
 template <int FMT, int NAL> constexpr bool mma_wide() { return NAL == 16 && (FMT == kMmaQ4K || FMT == kMmaQ5K); }
 // Wavefronts that sweep a tile together: four (one a pair accumulator), in the wide form four for each matrix.
 template <int NM, bool WIDE> constexpr uint32_t mma_waves() { return WIDE ? 4U * NM : 4U; }
@@ -130,7 +130,7 @@ __device__ __forceinline__ u32x4 mma_fifth(const u32x4& qh, uint32_t bit) { retu
 // lane's chain terms x[2P] + x[2P + 1] for its first nv activation rows. P is the wavefront's pair, a template argument so that
 // the scale / min unpacking has constant shifts.
 template <int FMT, int NAL, int NM, int P>
-__device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLane& o, float (&term)[NM][NAL]) {
+__device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLane& o, uint32_t nv, float (&term)[NM][NAL]) {
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) int32_t lds_i32;
     const u32x4 a_even = *(lds_u32x4*)(slot + o.even), a_odd = *(lds_u32x4*)(slot + o.odd);
@@ -163,6 +163,9 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
         const float D1 = d * static_cast<float>(s1), M1 = dm * static_cast<float>(m1);
 #pragma unroll
         for (int v = 0; v < NAL; ++v) {
+            // the widest sweep skips the result registers past a short chunk, four at a time (straight-line code either way: a
+            // loop exit here would turn the register arrays into indexed accesses)
+            if (NAL > 8 && static_cast<uint32_t>(v & ~3) >= nv) continue;
             const float e0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x00, 0xF, 0xF, true));
             const float e1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0x55, 0xF, 0xF, true));
             const float f0 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(tab[v], 0xAA, 0xF, 0xF, true));
@@ -179,7 +182,8 @@ __device__ __forceinline__ void mma_stage_terms(const lds_u8* slot, const MmaLan
 // row), so a v_mfma_f32_32x32x2_f32 leaves it in the dots' layout: k = 0 carries sub-block 2p and k = 1 sub-block 2p + 1, each product
 // with the other one's operands zero (a * b rounded once, + 0). A sub-block's terms take the place of its dots before the other's products
 // are made, and the deltas come as broadcast reads, asked for in front of the products they wait with: 64 registers of results and deltas
-// beside the accumulators, so that four wavefronts share a SIMD where two did (gate and up on one wavefront each took 240).
+// beside the accumulators, so that four wavefronts share a SIMD where two did (gate and up on one wavefront took 240). That is the bound of 128 registers a
+// wavefront: the kernels spill 23 to 29 of gate / up and 4 to 7 of the down rows, written and read outside the stage loop, once a chunk or tile.
 // Bound by the chain and by what a stage waits for (operands, products, the barrier), in about equal parts. Measured, before -> now: 1000 rows of
 // hidden 2048 / ffn 768 / 128 experts gate / up 327 -> 297 us, down rows (16 activation rows a sweep before) 167 -> 146; dense 27648 x 5120,
 // 32 rows gate / up 105 -> 95 us. Not faster: one wavefront for both matrices with u as one fma on biased dots, at two wavefronts a SIMD (a
@@ -661,17 +665,20 @@ __device__ __forceinline__ void mma_run(lds_u8* ring, lds_f32* xbuf, lds_f32* re
                 if (p < 2U) mma_stage_terms_halves<FMT, NAL, NM, false>(slot, o, p, term);
                 else mma_stage_terms_halves<FMT, NAL, NM, true>(slot, o, p, term);
             } else switch (p) {
-            case 0: mma_stage_terms<FMT, NAL, NM, 0>(slot, o, term); break;
-            case 1: mma_stage_terms<FMT, NAL, NM, 1>(slot, o, term); break;
-            case 2: mma_stage_terms<FMT, NAL, NM, 2>(slot, o, term); break;
-            default: mma_stage_terms<FMT, NAL, NM, 3>(slot, o, term); break;
+            case 0: mma_stage_terms<FMT, NAL, NM, 0>(slot, o, nv, term); break;
+            case 1: mma_stage_terms<FMT, NAL, NM, 1>(slot, o, nv, term); break;
+            case 2: mma_stage_terms<FMT, NAL, NM, 2>(slot, o, nv, term); break;
+            default: mma_stage_terms<FMT, NAL, NM, 3>(slot, o, nv, term); break;
             }
             if ((FMT != kMmaQ4K && FMT != kMmaQ5K) || WIDE) {
             } else if (TEAMS == 1) {
 #pragma unroll
                 for (uint32_t m = 0; m < MATS; ++m)
 #pragma unroll
-                    for (int v = 0; v < NAL; ++v) acc[m][v] = acc[m][v] + term[m][v];
+                    for (int v = 0; v < NAL; ++v) {
+                        if (NAL > 8 && static_cast<uint32_t>(v & ~3) >= nv) continue;
+                        acc[m][v] = acc[m][v] + term[m][v];
+                    }
             } else if (team == 0U) {
 #pragma unroll
                 for (int v = 0; v < NAL; ++v) own[v] = term[0][v];

@@ -68,9 +68,9 @@ struct MmaRowsOf {
 };
 template <class P> __device__ __forceinline__ uint64_t address(const P* p) { return reinterpret_cast<uint64_t>(p); }
 
-// The sweep of a chunk of n rows, run(NAL): of the wide form (NAL == 16) with no chain for the result registers past a short chunk.
-template <int NAL, class Run> __device__ __forceinline__ void mma_chunk(uint32_t n, Run run) {
-    if constexpr (NAL == 16) {
+// The sweep of a chunk of n rows, run(NAL): of the wide form with no chain for the result registers past a short chunk.
+template <int NAL, bool WIDE, class Run> __device__ __forceinline__ void mma_chunk(uint32_t n, Run run) {
+    if constexpr (WIDE) {
         if (n > 24U) run(std::integral_constant<int, 16>{});
         else if (n > 16U) run(std::integral_constant<int, 12>{});
         else if (n > 8U) run(std::integral_constant<int, 8>{});
@@ -80,8 +80,8 @@ template <int NAL, class Run> __device__ __forceinline__ void mma_chunk(uint32_t
 
 // Waves per SIMD: what the LDS of a workgroup allows (four of 36 KB, three of 44 or 46 KB, two of eight wavefronts and 73 KB), which for 16 rows the compiler misses
 // by a few registers when it is not told (200 rows of hidden 2048 / ffn 768 / 128 experts: 192.8 -> 172.3 us a layer, 219.6 before the run).
-template <int FMT, int NAL, int DEPTH, bool DIRECT>
-__global__ __launch_bounds__(NAL == 16 ? 512 : 256, NAL == 2 || NAL == 16 ? 4 : 3) void q4k_mma_project_kernel(MmaArgs k) {
+template <int FMT, int NAL, int DEPTH, bool DIRECT, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 512 : 256, NAL == 2 || WIDE ? 4 : NAL <= 8 ? 3 : 2) void q4k_mma_project_kernel(MmaArgs k) {
     constexpr uint32_t ACTS = mma_acts<NAL>();
     __shared__ __attribute__((aligned(16))) uint8_t ring_mem[mma_ring_bytes<FMT, NAL, 2, DEPTH, 1>()];
     __shared__ float red_mem[mma_reduce_floats<NAL, 2>()];
@@ -147,9 +147,9 @@ __global__ __launch_bounds__(NAL == 16 ? 512 : 256, NAL == 2 || NAL == 16 ? 4 : 
             }
         };
         const auto run = [&](auto nal) __attribute__((always_inline)) {
-            mma_run<FMT, decltype(nal)::value, DEPTH, 1, 2, true, mma_wide<FMT, NAL>()>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, kMmaRows, n, rows, emit);
+            mma_run<FMT, decltype(nal)::value, DEPTH, 1, 2, true, WIDE>((lds_u8*)ring_mem, nullptr, (lds_f32*)red_mem, wrows, k.w.gate_row_stride, k.w.hidden / 256U, tiles, kMmaRows, n, rows, emit);
         };
-        mma_chunk<NAL>(n, run);
+        mma_chunk<NAL, WIDE>(n, run);
     }
 }
 
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NAL == 16 ? 512 : 256 * TEAMS, NAL == 16 ? 4 : 1) v
             mma_run<FMT, decltype(nal)::value, DEPTH, TEAMS, NM, TEAMS == 1 && !GATE_UP, mma_wide<FMT, NAL>()>((lds_u8*)ring_mem, (lds_f32*)xbuf_mem, (lds_f32*)red_mem, wrows, row_stride,
                                                                                                   (GATE_UP ? k.w.hidden : k.w.ffn) / 256U, tiles, TILE, n, rows, emit);
         };
-        mma_chunk<NAL>(n, run);
+        mma_chunk<NAL, mma_wide<FMT, NAL>()>(n, run);
     }
 }
 

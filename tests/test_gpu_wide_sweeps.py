@@ -1,5 +1,5 @@
-"""The 32-row matrix-core sweeps (two tiles of weight rows, eight wavefronts): chunks around the lines between their result registers (8, 16, 24
-and 32 rows), both K-quant gate formats, scales and minimums that are not finite."""
+"""The 32-row matrix-core sweeps (gate and up on one wavefront, or wide: two tiles of weight rows, eight wavefronts): chunks around the lines between their
+result registers (8, 16, 24 and 32 rows), both K-quant gate formats, scales and minimums that are not finite."""
 import pytest
 import torch
 
@@ -24,12 +24,17 @@ def blocks(strix, gen, kind, rows, width):
 
 
 # rows of the experts (one choice a row); hidden and ffn of one super-block, of two and more, of a run of tiles; against batches of two rows,
-# which other sweeps serve. The sums have one order, so the bits are the same.
-@pytest.mark.parametrize("counts,hidden,ffn", [((1, 8, 9, 16, 17, 24, 25, 32, 33), 256, 256), ((128, 65, 40, 0, 41, 0), 512, 768), ((129, 31, 1, 64), 2304, 256)])
+# which other sweeps serve. The sums have one order, so the bits are the same. wide: the form of the gate / up rows by stages times rows an expert (the down
+# rows are wide at hidden 3072).
+@pytest.mark.parametrize("counts,hidden,ffn,wide", [
+    ((1, 8, 9, 16, 17, 24, 25, 32, 33), 256, 256, False), ((128, 65, 40, 0, 41, 0), 512, 768, False), ((38, 27, 1, 14), 1792, 256, False),
+    ((450, 360, 401, 395), 256, 256, True), ((200, 240, 193, 177), 512, 512, True), ((129, 31, 1, 64), 2304, 256, True), ((1, 8, 9, 16, 17, 24, 25, 32, 33), 3072, 256, True)])
 @pytest.mark.parametrize("gate", ["q4_k", "q5_k"])
 @pytest.mark.parametrize("special", [None, 0x7C00, 0xFC00])
-def test_chunks_equal_pairs_of_rows(strix, counts, hidden, ffn, gate, special):
+def test_chunks_equal_pairs_of_rows(strix, counts, hidden, ffn, wide, gate, special):
     E, T = len(counts), sum(counts)
+    stages = hidden // 256
+    assert wide == (stages >= 12 or stages * T >= 400 * E if gate == "q5_k" else stages >= 8 or stages * T >= 180 * E)      # (workgroups of one tile)
     assert T >= 16 * E                                                     # the rule of items longer than 16 rows
     gen = torch.Generator(device="cuda").manual_seed(hidden + ffn)
     gt = strix.TYPE_Q4_K if gate == "q4_k" else strix.TYPE_Q5_K
@@ -51,8 +56,9 @@ def test_chunks_equal_pairs_of_rows(strix, counts, hidden, ffn, gate, special):
         assert bool(same.all()), r
 
 
-# a dense block: rows of one chunk and of three, few workgroups of down rows (which stay on sixteen rows a sweep) and one per compute unit
-@pytest.mark.parametrize("rows,hidden,ffn", [(17, 512, 1024), (25, 256, 512), (70, 8192, 512)])
+# a dense block: rows of one chunk and of three, few workgroups of down rows (which stay on sixteen rows a sweep) and one per compute unit; 33 and 48 rows of
+# few stages: gate and up on one wavefront
+@pytest.mark.parametrize("rows,hidden,ffn", [(17, 512, 1024), (25, 256, 512), (33, 1792, 512), (48, 256, 1024), (70, 8192, 512)])
 def test_dense_rows_equal_one_by_one(strix, rows, hidden, ffn):
     gen = torch.Generator(device="cuda").manual_seed(rows)
     g, u, d = (blocks(strix, gen, "q4_k", n, m) for n, m in ((ffn, hidden), (ffn, hidden), (hidden, ffn)))
