@@ -592,8 +592,8 @@ class MoeLayer:
         """Router + experts + combine through mi355_moe_enqueue_layer. Returns (output, ids, weights, scores).
         shared_experts: the last `shared_experts` experts of the tensors are always on (the router picks among the others);
         shared_slot_weights [rows][shared_experts]: their weights in the place of 1 (the sigmoid gate of shared_gate()).
-        norm: (weight or None, eps) - the RMSNorm of x runs inside the first launch (mi355_moe_enqueue_layer_normed); the
-        normalised rows are left in self.normed."""
+        norm: (weight or None, eps) - the RMSNorm of x runs in front (mi355_moe_enqueue_layer_normed: a launch of its own, or inside the
+        router's for few short rows); the normalised rows are left in self.normed."""
         rows = x.shape[0]
         if router_weight.shape[0] != self.experts - shared_experts or router_weight.shape[1] != self.hidden:
             raise StrixError(E_INVALID_ARGUMENT, "the router weight must be [experts - shared_experts][hidden]")

@@ -43,8 +43,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
     constexpr uint32_t OT = gemm_out_rows<KS>(), AT = 32U * NA, G = gemm_groups<KS>(), P = gemm_pitch<KS>(), R = 32U / KS;
     constexpr uint32_t LEVELS = R == 8U ? 3U : 2U, ABLK = AT * G / kGemmThreads > 0U ? AT * G / kGemmThreads : 1U;
     // The next stage's copies go to LDS in front of a stage's products, a stage after they were asked for, or behind them, half as long after. Tiles of
-    // 32 weight rows copy twice the bytes a product, so the wait counts there: before -> now, 100 rows of 8192 x 1024 39.1 -> 36.0 us, 300 rows of
-    // 4096 x 2048 41.7 -> 39.3, 50 rows of 4096 x 4096 23.3 -> 21.7, 32 rows 17.0 -> 16.7. Tiles of 64 lose: 4096 x 4096, 500 rows 62.2 -> 62.5,
+    // 32 weight rows copy twice the bytes a product, so the wait counts there: before -> now, 100 rows of 8192 x 1024 39.1 -> 36.6 us, 300 rows of
+    // 4096 x 2048 41.5 -> 40.1, 50 rows of 4096 x 4096 23.2 -> 22.1, 32 rows 17.0 -> 16.7. Tiles of 64 lose: 4096 x 4096, 500 rows 62.2 -> 62.5,
     // 8192 x 16384, 1000 rows 887 -> 893.
     constexpr bool EARLY = KS == 8;
     static_assert(OT * G == kGemmThreads, "one weight block per thread and stage");

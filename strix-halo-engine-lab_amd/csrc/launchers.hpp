@@ -19,7 +19,7 @@ struct RouteCheck {
     uint32_t experts, top_k;
     uint32_t *status, *job_status;
 };
-// plan (unless its words are null): the expert plan of the rows' routes as well.
+// plan (unless it has no experts): the expert plan of the rows' routes as well.
 void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, const RouteCheck& c, const PlanArgs& plan, hipStream_t st);
 
 // prefill.hip: the most rows of a plan item for the products of a batch

@@ -26,7 +26,7 @@ struct RoutesView {
 };
 inline RoutesView dense_routes(const uint32_t* routes, uint32_t top_k) { return RoutesView{routes, 4ULL * top_k, top_k}; }
 
-struct PlanArgs { RoutesView routes; uint32_t experts, assignments, split, item_bound; uint32_t* plan; };      // (plan null: no plan)
+struct PlanArgs { RoutesView routes; uint32_t experts, assignments, split, item_bound; uint32_t* plan; };      // (no experts: no plan, nothing else is read)
 
 // Inclusive prefix sum over a wavefront: row shifts inside the rows of 16, then the rows' totals by row broadcasts (DPP, no LDS).
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {

@@ -134,8 +134,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
     // SCALED: the operand of a Q4_K weight is 2^-14 sc q, as the packed product of a subnormal (the nibble where it lies in its byte: 2^-24 q or 2^-20 q)
     // and 2^10 sc or 2^6 sc: exact, no shift for the high nibbles, and no 1024 to take out of the sum again.
     constexpr bool SCALED = FMT == kRgQ4K;
-    // Q8_0: stages of weights in registers. The wide form has room for two beside its sums (32 registers of the gate / up rows are spilled at a
-    // unit's start and read at its end; with four stages 110, inside the K loop: 1000 rows of hidden 2048 / ffn 768 / 128 experts 342 -> 435 us).
+    // Q8_0: stages of weights in registers. The wide form has room for two beside its sums (14 registers of the gate / up rows and 9 of the
+    // down rows are spilled at a unit's start and read at its end, as 7 and 5 of Q4_K and Q5_K are; with four stages 110, inside the K loop: 1000 rows of hidden
+    // 2048 / ffn 768 / 128 experts 342 -> 435 us).
     constexpr uint32_t RING8 = WAVES == 4U ? 4U : 2U;
     constexpr uint32_t BLOCK = FMT == kRgQ5K ? 176U : 144U, QUANTS_AT = FMT == kRgQ5K ? 48U : 16U;          // of a K-quant super-block
     // h enters as fp16 hi + lo. Q4_K: both planes in one sweep of the weights, two products per operand. Q5_K and Q8_0: K is swept twice, lo
@@ -155,8 +156,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4U ? 3 : 2) void prefill_reg_k
 
     // LIST: the workgroup's units, up to 64 at a time, are listed in LDS (expert, first row in plan order, rows, feature tile), and the assignments of a
     // unit's rows are there before it starts. Asked for one after the other in front of a unit's first copy, item and assignments are two trips to
-    // memory that nothing hides, and the stores at its end wait for a third: 1000 rows of hidden 2048 / ffn 768 / 128 experts 296 -> 266 us, 4096 rows
-    // of hidden 4096 / ffn 2048 / 256 experts 3968 -> 3804. The four-wave form has one to three units a workgroup and two more of them beside
+    // memory that nothing hides, and the stores at its end wait for a third: 1000 rows of hidden 2048 / ffn 768 / 128 experts 291 -> 268 us, 4096 rows
+    // of hidden 4096 / ffn 2048 / 256 experts 3932 -> 3806. The four-wave form has one to three units a workgroup and two more of them beside
     // it: the list costs it more than it saves (64 rows 95.9 -> 97.9 us), and so did copies that run on from a unit into the next (97.4; 333
     // rows 162.2 -> 158.8, Q8_0 rows 169.5 -> 173.6).
     constexpr bool LIST = WAVES == 8U;

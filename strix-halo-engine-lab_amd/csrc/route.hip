@@ -61,7 +61,7 @@ void launch_prologue_rows(const A8RowArgs& q, uint32_t kind, uint32_t rows, cons
 
 void launch_route_select(const RouteArgs& a, hipStream_t st) { route_select_kernel<<<a.rows, 64, 0, st>>>(a); }
 
-// RMSNorm of rows of any input kind into fp32 rows (the staged form of the fused norm), bit for bit rmsnorm_f32_kernel: lane l of L = 256
+// RMSNorm of rows of any input kind into fp32 rows (in front of a layer that does not norm its rows in the router's launch), bit for bit rmsnorm_f32_kernel: lane l of L = 256
 // (n >= 512) or 128 chains fma(x, x, a) over x[l], x[l + L], ...; the L partial sums are halved, l with l + 128, l + 64, ..., l + 1.
 // A thread per chain. Bound by latency: the HELD first values of a chain and their weights are asked for at once and kept (one by one past
 // the first eight, 1 row of 2048 fp16 values, 8 of 3072, 1 of 4096, 3 of 6144: 5.5, 8.5, 11, 16 us, now 2.2, 2.7, 4.7, 4.0), and every wave

@@ -2000,7 +2000,7 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     STRIX_REQUIRE(p->experts + p->shared_experts == wv.experts && p->top_k + p->shared_experts == wv.top_k,
                   "moe layer: router policy (experts, top_k, always-on experts) and expert tensors disagree on experts / top_k");
     STRIX_REQUIRE(!norm.on || (norm.normed && aligned(norm.normed, 16) && (!norm.weight || aligned(norm.weight, 16)) && norm.eps >= 0.0F),
-                  "moe layer: the fused RMSNorm needs a 16-byte aligned fp32 [rows][hidden] view for the normalised rows, aligned weights, eps >= 0");
+                  "moe layer: the RMSNorm needs a 16-byte aligned fp32 [rows][hidden] view for the normalised rows, aligned weights, eps >= 0");
     hipStream_t st = hs(stream);
     const auto norm_rows = [&] { launch_norm_rows(r->input, r->input_kind, r->input_stride, norm.weight, wv.hidden, norm.eps, norm.normed, rows, st); };
     if (rows > kFusedMaxRows || plan_split(wv, rows) != 1U) {      // large batches, and decode batches over large experts (shared sweeps): router, then the staged prologue / plan
@@ -2043,8 +2043,8 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
                        wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden;
     if (norm.on && (early || wv.hidden > kChainNormHidden)) {
         // The normalised rows in a launch of their own; the router takes them as fp32 rows. (In the router's launch every workgroup works its
-        // row's factor out again, in front of its chain. Layers of 1 row x 4096, 3 x 6144, 8 x 3072, 16 x 4096 fp32 rows: 59.5, 85.4, 74.5,
-        // 139.4 us, so 46.6, 62.1, 67.3, 96.8; 5 rows of 2048 with an always-on expert 64.2 -> 61.0.)
+        // row's factor out again, in front of its chain. Layers of 1 row x 4096, 3 x 6144, 8 x 3072, 16 x 4096 fp32 rows: 60.5, 86.5, 74.5,
+        // 139.4 us, with this launch 46.6, 62.1, 67.3, 96.8; 5 rows of 2048 with an always-on expert 64.2 -> 61.0.)
         if (do_front) norm_rows();
         a.x = reinterpret_cast<const uint8_t*>(norm.normed); a.kind = MI355_INPUT_F32; a.x_stride = 4ULL * wv.hidden;
     } else if (norm.on) { a.norm_w = norm.weight; a.norm_eps = norm.eps; a.normed = norm.normed; }
