@@ -284,6 +284,79 @@ __global__ __launch_bounds__(1024) void plan_kernel(PlanArgs p) {
     plan_block(lds, p, blockIdx.x);
 }
 
+// Lanes of the wavefront whose key (of `bits` bits) equals this lane's, among the lanes that `take` part: a ballot per bit.
+__device__ __forceinline__ uint64_t lanes_of_key(uint32_t key, uint32_t bits, bool take) {
+    uint64_t same = __ballot(take);
+    for (uint32_t b = 0; b < bits; ++b) {
+        const bool set = (key >> b) & 1U;
+        const uint64_t votes = __ballot(set);
+        same &= set ? votes : ~votes;
+    }
+    return same;
+}
+
+// The same for at most kPlanSmall assignments, by one workgroup: thread e owns expert e, thread a assignment a. Wave w finds each of its 64 assignments'
+// position among its own of the same expert by ballots and leaves the wave's counts; a prefix over the waves and the expert's offset make it the
+// position in the order. Bound by latency; alone in its launch it is through before a workgroup per expert has started. A workgroup per expert -> one, 64 |
+// 1024 assignments over 128 experts 3.8 | 5.8 -> 3.5 | 4.2 us, over 512 4.6 | 7.8 -> 3.6 | 4.6, over 1024 5.4 | 13.1 -> 4.0 | 5.3; 4096 the other way, 16.2 and 6.0 us.
+// (Beside the workgroups of the rows it is the longest one: plan_block.hpp.)
+constexpr uint32_t kPlanSmall = 1024;
+__global__ __launch_bounds__(1024) void plan_small_kernel(PlanArgs p) {
+    __shared__ uint32_t offset[kRouteMaxExperts];
+    __shared__ uint16_t wave_counts[16][kRouteMaxExperts];         // per wave and expert, later the prefix over the waves before
+    __shared__ u32x4 wave_totals[16];                              // per wave: assignments, items, touched experts, largest group
+    const uint32_t tid = threadIdx.x, lane = tid & 63U, wave = tid >> 6, waves = (p.assignments + 63U) / 64U, experts = p.experts;
+    for (uint32_t w = 0; w < waves; ++w) wave_counts[w][tid] = 0;
+    const uint32_t mine = tid < p.assignments ? p.routes.at(tid) : experts;
+    __syncthreads();
+    const uint64_t same = lanes_of_key(mine, 32U - static_cast<uint32_t>(__builtin_clz(experts)), mine < experts);
+    const uint32_t rank = static_cast<uint32_t>(__popcll(same & ((1ULL << lane) - 1ULL)));
+    if (mine < experts && rank == 0) wave_counts[wave][mine] = static_cast<uint16_t>(__popcll(same));
+    __syncthreads();
+    uint32_t c = 0;
+    if (tid < experts)
+        for (uint32_t w = 0; w < waves; ++w) {
+            const uint32_t here = wave_counts[w][tid];
+            wave_counts[w][tid] = static_cast<uint16_t>(c);
+            c += here;
+        }
+    const uint32_t pieces = (c + p.split - 1U) / p.split;
+    const uint32_t runs = wave_inclusive_scan(c), items_to = wave_inclusive_scan(pieces), touched_to = static_cast<uint32_t>(__popcll(__ballot(c != 0) & ((2ULL << lane) - 1ULL)));
+    uint32_t largest = c;
+#pragma unroll
+    for (int d = 32; d; d >>= 1) {
+        const uint32_t other = __shfl_xor(largest, d);
+        largest = other > largest ? other : largest;
+    }
+    if (lane == 63U) wave_totals[wave] = u32x4{runs, items_to, touched_to, largest};
+    __syncthreads();
+    u32x4 before = {0U, 0U, 0U, 0U}, all = {0U, 0U, 0U, 0U};
+#pragma unroll
+    for (uint32_t w = 0; w < 16U; ++w) {
+        const u32x4 t = wave_totals[w];
+        if (w < wave) { before.x += t.x; before.y += t.y; before.z += t.z; }
+        all.x += t.x; all.y += t.y; all.z += t.z; all.w = t.w > all.w ? t.w : all.w;
+    }
+    const uint32_t first = before.x + runs - c;
+    uint32_t* const items = p.plan + plan_items_at(experts, p.assignments);
+    if (tid < experts) {
+        p.plan[kPlanOffsetsAt + tid] = first;
+        if (c != 0) {
+            p.plan[plan_touched_at(experts) + before.z + touched_to - 1U] = tid;
+            for (uint32_t b = 0, k = before.y + items_to - pieces; b < c; b += p.split, ++k)
+                *reinterpret_cast<uint4*>(items + 4U * k) = make_uint4(tid, first + b, first + (b + p.split < c ? b + p.split : c), 0U);
+        }
+    }
+    for (uint32_t u = all.y + tid; u < p.item_bound; u += 1024U) *reinterpret_cast<uint4*>(items + 4U * u) = make_uint4(0U, 0U, 0U, 0U);
+    if (tid == 0) {
+        p.plan[kPlanOffsetsAt + experts] = all.x;
+        p.plan[0] = p.assignments; p.plan[1] = all.z; p.plan[2] = all.w; p.plan[4] = all.y;
+    }
+    offset[tid] = first;
+    __syncthreads();
+    if (mine < experts) p.plan[plan_order_at(experts) + offset[mine] + wave_counts[wave][mine] + rank] = tid;
+}
+
 // ======================================================================================================== Q4_K x A8 rows
 // gate + up + SwiGLU + A8 re-quantisation: one wavefront per (touched expert, 32-output group). Lanes 0..31 hold the
 // gate rows of the group, lanes 32..63 the up rows; one cross-half exchange pairs them, then both halves evaluate the
@@ -1537,8 +1610,8 @@ inline void launch_mma_gate_up(const mi355_moe_weights& w, const RowsK& r, uint3
 }
 
 inline void launch_plan(const PlanArgs& p, hipStream_t st) {
-    const uint32_t waves = (p.assignments + 63U) / 64U;
-    plan_kernel<<<p.experts, 64U * (waves < 16U ? waves : 16U), 0, st>>>(p);
+    if (p.assignments <= kPlanSmall) plan_small_kernel<<<1, 1024, 0, st>>>(p);
+    else plan_kernel<<<p.experts, 1024, 0, st>>>(p);
 }
 // Decode batches of at most this many assignments (six tokens at top-8) run the 16-rows-per-wavefront sweep (q4k_quads.hpp),
 // with a 4-slot ring up to 16 assignments and a 2-slot ring above (every workgroup of the launch stays resident); measured

@@ -1,4 +1,4 @@
-"""The start of a staged batch: the plan's order around its single-launch limit, and the launch that selects, checks and quantises a row."""
+"""The start of a staged batch: the plan's order around the limit of its one workgroup, and the launch that selects, checks and quantises a row."""
 import numpy as np
 import pytest
 import torch
@@ -22,13 +22,17 @@ def pad4(n):
     return (n + 3) // 4 * 4
 
 
-# assignments around a wave's 64, around 1024 (an assignment per thread of the plan's workgroup) and past it; one expert that takes
-# everything, more experts than assignments
-@pytest.mark.parametrize("rows,top_k,experts,skew", [(1, 1, 2, 0), (63, 1, 5, 0), (64, 1, 1024, 0), (65, 1, 3, 2), (32, 8, 128, 0), (257, 1, 16, 1), (341, 3, 40, 0),
-                                                     (64, 16, 300, 2), (1025, 1, 64, 1), (205, 5, 7, 0)])
+# assignments around a wave's 64, around 1024 (an assignment per thread of the plan's one workgroup) and past it (a workgroup per expert); one expert that
+# takes everything (skew 2), more experts than assignments, ids of no expert (skew 3)
+@pytest.mark.parametrize("rows,top_k,experts,skew", [(1, 1, 2, 0), (1, 1, 1, 0), (63, 1, 5, 0), (64, 1, 1024, 0), (65, 1, 3, 2), (32, 8, 128, 0), (257, 1, 16, 1), (341, 3, 40, 0),
+                                                     (64, 16, 300, 2), (64, 16, 1024, 0), (1025, 1, 64, 1), (205, 5, 7, 0), (2049, 1, 1, 0), (100, 16, 1024, 0),
+                                                     (40, 8, 31, 3), (128, 8, 1023, 3), (200, 8, 64, 3)])
 def test_plan_order(strix, rows, top_k, experts, skew):
     rng = np.random.default_rng(rows * top_k + experts)
     ids = np.minimum(rng.integers(0, experts, (rows, top_k)), rng.integers(0, experts, (rows, top_k)) // (1 if skew == 0 else 4)) if skew < 2 else np.full((rows, top_k), experts - 1)
+    if skew == 3:
+        ids = rng.integers(0, experts, (rows, top_k))
+        ids.reshape(-1)[::7] = experts + rng.integers(0, 2000, ids.reshape(-1)[::7].shape)
     H = I = 256
     row = H // 256 * 144
     w = torch.zeros((experts * 256, row), dtype=torch.uint8, device="cuda")
@@ -38,13 +42,16 @@ def test_plan_order(strix, rows, top_k, experts, skew):
     layer.stage("csr", x, routes, torch.ones((rows, top_k), device="cuda"))
     plan = layer.plan.cpu().numpy()
     flat, A = ids.reshape(-1), rows * top_k
+    live = np.flatnonzero(flat < experts)
     order_at = PLAN_OFFSETS_AT + pad4(experts + 1) + pad4(experts)
-    offsets = np.concatenate([[0], np.cumsum(np.bincount(flat, minlength=experts))])
+    offsets = np.concatenate([[0], np.cumsum(np.bincount(flat[live], minlength=experts))])
     assert np.array_equal(plan[PLAN_OFFSETS_AT:PLAN_OFFSETS_AT + experts + 1], offsets)
-    assert np.array_equal(plan[order_at:order_at + A], np.argsort(flat, kind="stable"))
+    assert plan[0] == A and plan[1] == len(set(flat[live])) and plan[2] == np.diff(offsets).max()
+    assert np.array_equal(plan[PLAN_OFFSETS_AT + pad4(experts + 1):][:plan[1]], np.unique(flat[live]))
+    assert np.array_equal(plan[order_at:order_at + len(live)], live[np.argsort(flat[live], kind="stable")])
     items = plan[order_at + pad4(A):][:4 * plan[4]].reshape(-1, 4)
     covered = np.concatenate([np.arange(b, e) for _, b, e, _ in items])
-    assert np.array_equal(covered, np.arange(A)) and all(offsets[e] <= b < z <= offsets[e + 1] for e, b, z, _ in items)
+    assert np.array_equal(covered, np.arange(len(live))) and all(offsets[e] <= b < z <= offsets[e + 1] for e, b, z, _ in items)
 
 
 # the plan that is made beside the rows of a batch, in the launch that quantises them or sums them for the prefill: around a turn of 64 assignments a
