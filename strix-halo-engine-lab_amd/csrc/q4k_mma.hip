@@ -29,7 +29,7 @@ template <int FMT, int NAL, bool WIDE = false>
 inline void launch_mma_project_nal(const mi355_moe_weights& w, const RowsK& r, uint32_t rows, uint32_t dense, uint32_t items, hipStream_t st) {
     const MmaGrid g = mma_grid(w, rows, dense, items, w.ffn / 32U, 2U * NAL, mma_project_run(w, dense, items));
     constexpr int DEPTH = NAL >= 8 ? 2 : 3, THREADS = 64 * mma_waves<2, WIDE>();
-    if constexpr (FMT == kMmaQ4K)
+    if constexpr (FMT == kMmaQ4K && (WIDE || NAL < 16))
         if (mma_direct(r.in, dense)) { q4k_mma_project_kernel<FMT, NAL, DEPTH, true, WIDE><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l}); return; }
     q4k_mma_project_kernel<FMT, NAL, DEPTH, false, WIDE><<<g.grid, THREADS, 0, st>>>(MmaArgs{w, r, g.l});
 }
@@ -74,12 +74,12 @@ inline void launch_mma_down_nal(const mi355_moe_weights& w, const RowsK& r, uint
 //   Q5_K  160 experts of ffn 512    4 .83 .86 .90 .92 .97 1.06   6 .89 .93 .97 .96 .97 .98   8 .91 .95 .97 .99 .98 1.00   10 .96 .96 1.02 .99 1.03 1.05
 //         80 experts of ffn 1536    4, runs of two tiles, .99 .97 1.00 .99 1.03 1.05   6 .90 .91 .94 .98 .96 .98   8 .91 .95 .93 .98 .98 1.03
 //         32 experts of ffn 1024    4 .89 .89 .90 .97 .99 1.01   6 .93 .91 .97 1.02 1.03 1.07   8 .99 .96 1.04 1.06 1.09 1.11   12 1.06 1.08 1.15 1.14 1.13 1.14
-// (95 experts top-6 of 1536 x 1536, Q5_K, 31 rows an expert: 231 us, wide 243; 128 experts of 2048 x 768, Q4_K, 62 rows: 327, wide 297.) Dense, ffn 8192, 32, 36,
-// 48, 64 rows: 4 stages 1.11 .99 .96 1.00, 6 1.12 .97 .98 1.12, 8 1.13 1.01 1.05 1.11.
+// (95 experts top-6 of 1536 x 1536, Q5_K, 31 rows an expert: 231 us, wide 243; 128 experts of 2048 x 768, Q4_K, 62 rows: 327, wide 297.) Dense blocks are wide: 34
+// and 48 rows, ffn 4096 1.11 1.10 (4 stages), 1.14 1.14 (7); 8192 .99 .98, 1.01 .99; 16384 .98 1.02, 1.04 1.08; 28672 1.00 1.04, 1.05 1.08.
 template <int FMT>
 inline bool mma_project_wide(const mi355_moe_weights& w, uint32_t rows, uint32_t dense, uint32_t run) {
     const uint32_t stages = w.hidden / 256U;
-    if (dense) return dense <= 32U || dense > 48U || stages >= 8U;
+    if (dense) return true;
     const uint64_t steps = static_cast<uint64_t>(stages) * run, rows_of_all = static_cast<uint64_t>(rows) * w.top_k;
     if (FMT == kMmaQ5K) return stages >= 12U || steps * rows_of_all >= 400ULL * w.experts;
     return steps >= 8U || steps * rows_of_all >= 180ULL * w.experts;

@@ -56,8 +56,7 @@ def test_chunks_equal_pairs_of_rows(strix, counts, hidden, ffn, wide, gate, spec
         assert bool(same.all()), r
 
 
-# a dense block: rows of one chunk and of three, few workgroups of down rows (which stay on sixteen rows a sweep) and one per compute unit; 33 and 48 rows of
-# few stages: gate and up on one wavefront
+# a dense block: rows of one chunk and of three, few workgroups of down rows (which stay on sixteen rows a sweep) and one per compute unit
 @pytest.mark.parametrize("rows,hidden,ffn", [(17, 512, 1024), (25, 256, 512), (33, 1792, 512), (48, 256, 1024), (70, 8192, 512)])
 def test_dense_rows_equal_one_by_one(strix, rows, hidden, ffn):
     gen = torch.Generator(device="cuda").manual_seed(rows)
