@@ -304,7 +304,7 @@ int32_t mi355_shared_gate(const void* x, uint32_t input_kind, uint32_t rows, uin
  * rows->input holds the raw rows; the router, the A8 image and the experts see y = (x * r) * norm_weight,
  * r = 1 / sqrt(mean(x^2) + norm_eps), bit for bit mi355_rmsnorm_f32 (lane-strided fma chains, LDS halving) followed by
  * mi355_moe_enqueue_layer on y; norm_weight may be NULL (unit scale). normed: fp32 [rows][hidden], receives y (the input of
- * anything else that reads the normalised rows). One norm launch runs first, or the router's launch norms the rows (up to 16 rows of at most 1536 features).
+ * anything else that reads the normalised rows). One norm launch runs first, or the router's launch norms the rows (up to 16 rows of at most 1536 features). normed may be the fp32 input itself.
  * A shared expert stored as expert `experts` of the same tensors is the policy's shared_experts = 1: every row then carries
  * one more slot with weight 1, its gate / up / down rows are swept once per four rows, and the ordered combine adds it last. */
 int32_t mi355_moe_enqueue_layer_normed(const mi355_route_policy* policy, const float* router_weight, const float* logit_bias,

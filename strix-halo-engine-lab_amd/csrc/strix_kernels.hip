@@ -2114,7 +2114,11 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     const bool early = p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
                        (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
                        wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden;
-    if (norm.on && (early || wv.hidden > kChainNormHidden)) {
+    // (rows that are normalised in place: the router's workgroups would read what others of their launch have written)
+    const uint64_t raw = reinterpret_cast<uint64_t>(r->input), raw_end = raw + (rows - 1U) * r->input_stride + (r->input_kind == MI355_INPUT_F32 ? 4ULL : 2ULL) * wv.hidden;
+    const uint64_t out = reinterpret_cast<uint64_t>(norm.normed), out_end = out + 4ULL * rows * wv.hidden;
+    const bool in_place = raw < out_end && out < raw_end;
+    if (norm.on && (early || wv.hidden > kChainNormHidden || in_place)) {
         // The normalised rows in a launch of their own; the router takes them as fp32 rows. (In the router's launch every workgroup works its
         // row's factor out again, in front of its chain. Layers of 1 row x 4096, 3 x 6144, 8 x 3072, 16 x 4096 fp32 rows: 60.5, 86.5, 74.5,
         // 139.4 us, with this launch 46.6, 62.1, 67.3, 96.8; 5 rows of 2048 with an always-on expert 64.2 -> 61.0.)

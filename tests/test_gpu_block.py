@@ -88,6 +88,21 @@ def test_norm_of_every_width(strix, kind, H, E, K, S, T, scaled):
     assert np.all(layer.status[:T].cpu().numpy() == 0)
 
 
+@pytest.mark.parametrize("H,T,S", [(512, 16, 1), (1536, 3, 0), (2048, 16, 1), (1024, 40, 0)])
+def test_rows_normalised_in_place(strix, H, T, S):
+    """fp32 rows whose normalised form takes their own place: the bits of a buffer of its own."""
+    I, E, K = 256, 32, 2
+    gen = torch.Generator(device="cuda").manual_seed(H + T)
+    draw = lambda n, m: strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((n, m), device="cuda", generator=gen) * 0.02)
+    layer = strix.MoeLayer(H, I, E + S, K + S, draw((E + S) * I, H), draw((E + S) * I, H), draw((E + S) * H, I), T)
+    x, router = torch.randn((T, H), device="cuda", generator=gen), torch.randn((E, H), device="cuda", generator=gen) * 0.02
+    weight = 1.0 + 0.1 * torch.randn(H, device="cuda", generator=gen)
+    want = [t.clone() for t in layer.run_layer(x, router, shared_experts=S, norm=(weight, 1e-6))] + [layer.normed.clone()]
+    layer.normed = x
+    got = list(layer.run_layer(x, router, shared_experts=S, norm=(weight, 1e-6))) + [x]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def launches(program):
     """The nodes that a captured program holds."""
     side = torch.cuda.Stream()
