@@ -193,18 +193,17 @@ __device__ __forceinline__ uint32_t early_select_row(const RouteArgs& a, uint32_
 }
 
 // ---------------------------------------------------------------------------------------------------- the exact chain as a side block
-// The reference's chain inside the layer launch: a one-wave block that owns two experts of one row. Its two router-weight rows
-// are requested whole at the block's start (one 10,240-byte LDS object each, the launch's two ring slots), so once they have
-// landed the chain no longer touches memory - the other waves of the launch saturate it. Lane 0 / 1 run the chains of the two
-// experts, the weight operand by 128-bit LDS reads 16 features ahead.
-//   fp16 / bf16 rows: the row rides along as 16-bit values in the 2 KB behind each weight row (features 0..1023 behind the
-//     first, the rest behind the second); per 16 features one 16-bit LDS read leaves feature k + t in lane t of every row of 16
-//     lanes, widened once, and the fma takes it by a DPP row broadcast (chain_run of route_wave.hpp).
-//   fp32 rows do not fit beside the weights: they sit in registers, feature 16 i + t in register i of lane t of every row of 16 lanes, for
-//     the same fma (one feature at a time through v_readlane before, which took four times as long a step: 1 row of hidden 2048 / ffn 768
-//     / 128 experts 37.2 -> 28.5 us, 8 rows 49.1 -> 46.9).
-// Needs hidden <= 2048, hidden % 64 == 0.
-constexpr uint32_t kSideExperts = 2, kSideMaxHidden = 2048, kSideSlotBytes = 10240, kSideRowBytes = 8192;
+// The reference's chain inside the layer launch: a one-wave block that owns two experts of one row. The two router-weight rows and the
+// row itself come in chunks through the launch's two ring slots: chunks of 1024 features of fp16 / bf16 rows in two places (8 KB of weights and 2 KB of the
+// row each), of 512 features of fp32 rows in three (4 KB and 2 KB). As many chunks as there are places are requested at the block's start - no row of
+// hidden 2048 and 16 bits a value needs more -, and a place is filled anew when its chunk is through: the other waves of the launch saturate the memory, so
+// what is awaited has to be asked for microseconds before. Lane 0 / 1 run the chains of the two experts, the weight operand by 128-bit LDS reads 48 features
+// ahead; per 16 features one LDS read leaves feature k + t in lane t of every row of 16 lanes, widened once, and the fma takes it by a DPP row
+// broadcast (chain_run of route_wave.hpp). (fp32 rows in registers before, all 128 of hidden 2048.)
+// Needs hidden % 64 == 0.
+constexpr uint32_t kSideExperts = 2, kSideSlotBytes = 10240;
+template <int KIND> constexpr uint32_t side_chunk() { return KIND == 0 ? 512U : 1024U; }
+template <int KIND> constexpr uint32_t side_places() { return KIND == 0 ? 3U : 2U; }
 
 __device__ __forceinline__ void side_copy16(const void* src, uint32_t lds_at) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_at), "v"(src) : "memory", "m0");
@@ -212,103 +211,82 @@ __device__ __forceinline__ void side_copy16(const void* src, uint32_t lds_at) {
 
 template <int KIND>
 __device__ __forceinline__ void side_chain_block(lds_u8* ring0, lds_u8* ring1, const RouteArgs& a, uint32_t row, uint32_t e0) {
-    const uint32_t lane = threadIdx.x & 63U, row_bytes = a.hidden * 4U;
+    constexpr uint32_t CHUNK = side_chunk<KIND>(), PLACES = side_places<KIND>(), SIZE = KIND == 0 ? 4U : 2U, WBYTES = 4U * CHUNK, XBYTES = SIZE * CHUNK;
+    static_assert(XBYTES == 2048U && (PLACES == 2U ? 2U * WBYTES + XBYTES <= kSideSlotBytes : 4U * WBYTES + XBYTES <= kSideSlotBytes), "two ring slots hold the places");
+    const uint32_t lane = threadIdx.x & 63U, chunks = (a.hidden + CHUNK - 1U) / CHUNK;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    lds_u8* const ring[kSideExperts] = {ring0, ring1};
+    // place p: weights of both experts, the row's values. Of the third one the weights lie behind the first, the values behind the second
+    const auto weights_of = [&](uint32_t p) { return p == 1U ? ring1 : p == 0U ? ring0 : ring0 + 2U * WBYTES + XBYTES; };
+    const auto values_of = [&](uint32_t p) { return p == 0U ? ring0 + 2U * WBYTES : p == 1U ? ring1 + 2U * WBYTES : ring1 + 2U * WBYTES + XBYTES; };
+    const uint8_t* const xrow = a.x + row * a.x_stride;
+    const float* wrow[kSideExperts];
 #pragma unroll
-    for (uint32_t i = 0; i < kSideExperts; ++i) {
-        const uint32_t e = e0 + i < a.p.experts ? e0 + i : a.p.experts - 1U;
-        const uint8_t* src = reinterpret_cast<const uint8_t*>(a.wr + static_cast<size_t>(e) * a.hidden) + 16U * lane;
-        const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring[i]));
-        for (uint32_t off = 0; off < row_bytes; off += 1024U)
-            if (off + 16U * lane < row_bytes) side_copy16(src + off, at + off);
-    }
-    const uint8_t* xrow = a.x + row * a.x_stride;
+    for (uint32_t i = 0; i < kSideExperts; ++i) wrow[i] = a.wr + static_cast<size_t>(e0 + i < a.p.experts ? e0 + i : a.p.experts - 1U) * a.hidden;
+    // Every chunk is the same number of copies (the waits count them): pieces past the row's end fetch its last one again, into places that are never read.
+    constexpr uint32_t WC = WBYTES / 1024U, XC = XBYTES / 1024U, COPIES = kSideExperts * WC + XC;
+    const auto start = [&](uint32_t c, uint32_t p) {
+        const uint32_t k0 = c * CHUNK, w_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(weights_of(p))), x_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(values_of(p)));
+#pragma unroll
+        for (uint32_t j = 0; j < WC; ++j) {
+            const uint32_t k = k0 + 256U * j + 4U * lane, from = k < a.hidden ? k : a.hidden - 4U;
+#pragma unroll
+            for (uint32_t i = 0; i < kSideExperts; ++i) side_copy16(wrow[i] + from, w_at + WBYTES * i + 1024U * j);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < XC; ++j) {
+            const uint32_t k = k0 + 1024U / SIZE * j + 16U / SIZE * lane, from = k < a.hidden ? k : a.hidden - 16U / SIZE;
+            side_copy16(xrow + static_cast<size_t>(SIZE) * from, x_at + 1024U * j);
+        }
+    };
+    const auto widen = [&](uint32_t v) {
+        if constexpr (KIND == 0) return f_of(v);
+        else if constexpr (KIND == 1) return half_bits_to_float(v);
+        else return f_of(v << 16);
+    };
+#pragma unroll
+    for (uint32_t p = 0; p < PLACES; ++p)
+        if (p < chunks) start(p, p);
     float acc = 0.0F;
-    const float* wrow = reinterpret_cast<const float*>((lane & 1U) ? (uint8_t*)ring1 : (uint8_t*)ring0);
-    if constexpr (KIND == 0) {
-        // lane t of every row of 16 lanes: features t, 16 + t, 32 + t, ... (the launch's LDS lets two waves on a SIMD: 256 registers are there)
-        constexpr uint32_t STEPS = kSideMaxHidden / 16U;
-        float x[STEPS];
-#pragma unroll
-        for (uint32_t i = 0; i < STEPS; ++i) x[i] = *reinterpret_cast<const float*>(xrow + 64U * (16U * i < a.hidden ? i : 0U) + 4U * (lane & 15U));
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        ChainStep S[4];
-        const auto load = [&](ChainStep& step, uint32_t k) {
-            const uint32_t kk = k < a.hidden ? k : a.hidden - 16U;      // (past the end: a valid place, never used)
-#pragma unroll
-            for (uint32_t i = 0; i < 4U; ++i) step.w[i] = *reinterpret_cast<const f32x4*>(wrow + kk + 4U * i);
-        };
-#pragma unroll
-        for (uint32_t i = 0; i < 3U; ++i) load(S[i], 16U * i);
-#pragma unroll
-        for (uint32_t i = 0; i < STEPS; i += 4U) {
-            if (16U * i >= a.hidden) break;                             // hidden % 64 == 0 on this path
-#pragma unroll
-            for (uint32_t j = 0; j < 4U; ++j) {
-                load(S[(j + 3U) & 3U], 16U * (i + j + 3U));
-                S[j].x = x[i + j];
-                __builtin_amdgcn_sched_barrier(0);
-                acc = chain_run(S[j], acc);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-    } else {
-        // the row as it is (2 bytes per feature) behind the weight rows: 1024 features = 2 KB = two copies of 64 x 16 bytes each
-#pragma unroll
-        for (uint32_t i = 0; i < kSideExperts; ++i) {
-            const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring[i])) + kSideRowBytes;
-#pragma unroll
-            for (uint32_t j = 0; j < 2U; ++j) {
-                const uint32_t k = 1024U * i + 512U * j + 8U * lane;
-                if (k < a.hidden) side_copy16(xrow + 2U * k, at + 1024U * j);
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        const uint32_t t = lane & 15U;
-        // the 16-bit value of feature k + t as read; it is widened only when its 16 steps are about to run, so the read's latency
-        // hides behind the steps in front of it
-        auto raw_of = [&](uint32_t k) {
-            return static_cast<uint32_t>(*reinterpret_cast<const uint16_t*>((k < 1024U ? (uint8_t*)ring0 : (uint8_t*)ring1) + kSideRowBytes + 2U * ((k & 1023U) + t)));
-        };
-        auto widen = [&](uint32_t h) {
-            if constexpr (KIND == 1) return half_bits_to_float(h);
-            else return f_of(h << 16);
-        };
-        // Operands are fetched 48 features ahead of the chain (four buffers): with one step of 16 ahead every step waited for its
+    for (uint32_t c = 0, p = 0; c < chunks; ++c, p = p + 1U == PLACES ? 0U : p + 1U) {
+        const uint32_t younger = chunks - 1U - c < PLACES - 1U ? chunks - 1U - c : PLACES - 1U;         // chunks asked for behind this one
+        if (younger == 0U) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (younger == 1U) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2U * COPIES) : "memory");
+        const lds_u8* const w = weights_of(p) + (lane & 1U ? WBYTES : 0U);
+        const lds_u8* const x = values_of(p) + SIZE * (lane & 15U);
+        const uint32_t n = a.hidden - c * CHUNK < CHUNK ? a.hidden - c * CHUNK : CHUNK;
+        // operands are fetched 48 features ahead of the chain (four buffers): with one step of 16 ahead every step waited for its
         // LDS reads (128 waits of ~200 cycles: the loop took 12.6 us inside the layer launch against ~5 us for the 2048 fmas).
-        ChainStep S0, S1, S2, S3;
-        uint32_t r0, r1, r2, r3;
-        auto load = [&](ChainStep& s, uint32_t& raw, uint32_t k) {
-            const uint32_t kk = k < a.hidden ? k : a.hidden - 16U;      // (past the end: a valid place, never used)
+        ChainStep S[4];
+        uint32_t raw[4];         // the value of feature k + t as read; widened only when its 16 steps are about to run
+        const auto load = [&](uint32_t s, uint32_t k) {
+            typedef const __attribute__((address_space(3))) f32x4 lds_f32x4;
+            typedef const __attribute__((address_space(3))) uint32_t lds_u32c;
+            typedef const __attribute__((address_space(3))) uint16_t lds_u16c;
+            const uint32_t kk = k < n ? k : n - 16U;            // (past the end: a valid place, never used)
 #pragma unroll
-            for (uint32_t i = 0; i < 4U; ++i) s.w[i] = *reinterpret_cast<const f32x4*>(wrow + kk + 4U * i);
-            raw = raw_of(kk);
+            for (uint32_t i = 0; i < 4U; ++i) S[s].w[i] = *(lds_f32x4*)(w + 4U * kk + 16U * i);
+            if constexpr (KIND == 0) raw[s] = *(lds_u32c*)(x + SIZE * kk);
+            else raw[s] = *(lds_u16c*)(x + SIZE * kk);
         };
-        load(S0, r0, 0U); load(S1, r1, 16U); load(S2, r2, 32U);
-        for (uint32_t k = 0; k < a.hidden; k += 64U) {      // hidden % 64 == 0 on this path
-            load(S3, r3, k + 48U);
-            __builtin_amdgcn_sched_barrier(0);
-            S0.x = widen(r0);
-            acc = chain_run(S0, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            load(S0, r0, k + 64U);
-            __builtin_amdgcn_sched_barrier(0);
-            S1.x = widen(r1);
-            acc = chain_run(S1, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            load(S1, r1, k + 80U);
-            __builtin_amdgcn_sched_barrier(0);
-            S2.x = widen(r2);
-            acc = chain_run(S2, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            load(S2, r2, k + 96U);
-            __builtin_amdgcn_sched_barrier(0);
-            S3.x = widen(r3);
-            acc = chain_run(S3, acc);
-            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t s = 0; s < 3U; ++s) load(s, 16U * s);
+        for (uint32_t k = 0; k < n; k += 64U) {                 // hidden % 64 == 0 on this path
+#pragma unroll
+            for (uint32_t s = 0; s < 4U; ++s) {
+                load((s + 3U) & 3U, k + 16U * (s + 3U));
+                __builtin_amdgcn_sched_barrier(0);
+                S[s].x = widen(raw[s]);
+                acc = chain_run(S[s], acc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (c + PLACES < chunks) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (every read of the place has returned)
+            start(c + PLACES, p);
         }
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const uint32_t e = e0 + lane;
     if (lane < kSideExperts && e < a.p.experts)
         __hip_atomic_store(a.scores + static_cast<size_t>(row) * a.p.experts + e, a.bias ? acc + a.bias[e] : acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

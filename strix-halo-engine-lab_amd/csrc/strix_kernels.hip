@@ -514,16 +514,21 @@ __global__ __launch_bounds__(64, DEPTH > 3 ? 1 : 2) void project_wave_kernel(mi3
 // Two ring slots of 10,240 bytes: eight workgroups share a compute unit.
 constexpr uint32_t kFrontSpinLimit = 1U << 22;
 struct FrontBlocks { uint32_t early, prologue, side; };
+constexpr uint32_t kFrontRunWaves = 1024;      // sweeps from which on rows of more than eight super-blocks stream as contiguous stages
 
-// gate + up + SwiGLU + A8 of assignment `at` on expert e, outputs 32 grp .. 32 grp + 31: rows in dense GGUF order stream as
-// contiguous stages (q4k_blocks.hpp), others as one super-block of each row per stage.
-__device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r, uint32_t e, uint32_t grp, uint32_t at) {
+// gate + up + SwiGLU + A8 of assignment `at` on expert e, outputs 32 grp .. 32 grp + 31: rows in dense GGUF order whose super-blocks fill a stage's 64 lanes
+// (hidden 512, 1024, 2048 and, where the launch's sweeps are enough to be bound by memory, 4096 and more) stream as contiguous stages (q4k_blocks.hpp), others as one
+// super-block of each row per stage: a contiguous stage of 48 blocks works as long as one of 64, and its chain runs over the lanes in as many steps
+// as a row has blocks. Layers, contiguous -> block by block: hidden 1280, 1, 4, 12 rows 30.2, 33.3, 53.7 -> 26.4, 29.6, 44.9 us; 1536 30.5, 34.2 -> 27.2, 31.1; 1792
+// 34.6, 41.9 -> 31.8, 39.7; 2304, 1 row 38.3 -> 30.4; 6144, 1 row (640 sweeps) 97.5 -> 79.3; 4096, 1, 2, 4 rows (384, 512, 1536 sweeps) 53.9, 54.4, 76.9 -> 48.5, 49.8, 81.0.
+__device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r, uint32_t e, uint32_t grp, uint32_t at, uint32_t assignments) {
     const size_t base = static_cast<size_t>(e) * w.gate_expert_stride + static_cast<size_t>(grp * 32U) * w.gate_row_stride;
     const uint8_t* gate = w.gate + base;
     const uint8_t* up = w.up + base;
     const uint32_t B = w.hidden / 256U;
-    if (w.gate_row_stride == static_cast<uint64_t>(B) * kQ4kBlock && block_lanes_ok(B, 32U)) {
-        const BlockLanes g = block_lanes(B, 32U);
+    const BlockLanes g = block_lanes(B, 32U);
+    const bool runs = g.used == 64U && (B <= 8U || assignments * (w.ffn / 32U) > kFrontRunWaves);
+    if (runs && w.gate_row_stride == static_cast<uint64_t>(B) * kQ4kBlock && block_lanes_ok(B, 32U)) {
         const uint32_t half = 32U / g.R;                  // stages of the gate rows, then as many of the up rows
         float value[1];
         const auto stage_base = [&](uint32_t s) { return s < half ? gate + static_cast<size_t>(s) * g.stage_bytes : up + static_cast<size_t>(s - half) * g.stage_bytes; };
@@ -547,9 +552,9 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
     uint32_t* lines = a.plan + kPlanLinesAt;
     if (!arrive_last(&lines[kLinesSide + row * kLineWords], neb)) return;
     const uint32_t expert = route_select_row(reinterpret_cast<float*>((uint8_t*)slots[0]), a, row);
-    const uint32_t K = a.p.top_k, groups = w.ffn / 32U;
-    if (lane < K) {
-        const uint32_t at = row * K + lane;
+    const uint32_t K = a.p.top_k, P = w.top_k, groups = w.ffn / 32U;          // P: with the always-on slots, which no choice concerns
+    if (lane < P) {
+        const uint32_t at = row * P + lane;
         *reinterpret_cast<uint4*>(a.plan + plan_items_at(w.experts, assignments) + 4U * at) = make_uint4(expert, at, at + 1U, at + 1U);
         a.plan[plan_order_at(w.experts) + at] = at;
     }
@@ -559,7 +564,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
     uint32_t image = 0;
     bool there = false;
     for (uint32_t spins = 0; spins < kFrontSpinLimit && !there; ++spins) {
-        if (lane < K) tag = __hip_atomic_load(&etags[row * K + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane < K) tag = __hip_atomic_load(&etags[row * P + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         image = __hip_atomic_load(&lines[kLinesRowTags + row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         there = __ballot(lane < K && static_cast<uint32_t>(tag >> 32) != epoch) == 0 && image == epoch;
         if (!there) __builtin_amdgcn_s_sleep(16);
@@ -574,7 +579,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
     // such a slot needs exists already, under the slot that held its expert, and is copied. Only an expert the early choice did not
     // hold at all is swept again. (With the optional fp32 intermediates bound every differing slot is swept again.)
     const uint32_t image_words = w.ffn / 4U + 2U * groups;         // codes, deltas, sums of one assignment, in 32-bit words
-    if (differ && !r.gate_out && !r.up_out && !r.h_out && K * image_words * 4U <= kSideSlotBytes) {
+    if (differ && !r.gate_out && !r.up_out && !r.h_out) {
         uint32_t src = 0xffU;
         for (uint32_t j = 0; j < K; ++j) {
             const uint32_t held = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint32_t>(tag)), static_cast<int>(j)));
@@ -585,7 +590,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             // every speculative wave of the row has to be through: a slot is read as a source or overwritten as a destination
             bool through = false;
             for (uint32_t spins = 0; spins < kFrontSpinLimit && !through; ++spins) {
-                const uint32_t seen = lane < K ? __hip_atomic_load(&r.awords[row * K + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffffU : groups;
+                const uint32_t seen = lane < K ? __hip_atomic_load(&r.awords[row * P + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffffU : groups;
                 through = __ballot(seen < groups) == 0;
                 if (!through) __builtin_amdgcn_s_sleep(32);
             }
@@ -601,22 +606,35 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             };
             uint32_t* stage = reinterpret_cast<uint32_t*>((uint8_t*)slots[0]);
             uint32_t flags = 0;                                   // bit k: the source of slot k carried the non-finite flag
-            for (uint64_t left = copy; left;) {                   // all sources first: a source may itself be a destination
-                const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(left))) - 1U;
-                left &= left - 1ULL;
-                const uint32_t from = row * K + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(src), static_cast<int>(k)));
-                for (uint32_t i = lane; i < image_words; i += 64U) stage[k * image_words + i] = __hip_atomic_load(image_word(from, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                flags |= (__hip_atomic_load(&r.awords[from], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 31) << k;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             for (uint64_t left = copy; left;) {
                 const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(left))) - 1U;
                 left &= left - 1ULL;
-                const uint32_t to = row * K + k;
-                for (uint32_t i = lane; i < image_words; i += 64U) __hip_atomic_store(image_word(to, i), stage[k * image_words + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (lane == 0) __hip_atomic_store(&r.awords[to], groups | (((flags >> k) & 1U) << 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t from = row * P + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(src), static_cast<int>(k)));
+                flags |= (__hip_atomic_load(&r.awords[from], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 31) << k;
+            }
+            // as many words of every image at a time as the ring slot holds; of those all sources first: a source may itself be a destination
+            const uint32_t piece = kSideSlotBytes / 4U / K;
+            for (uint32_t w0 = 0; w0 < image_words; w0 += piece) {
+                const uint32_t n = image_words - w0 < piece ? image_words - w0 : piece;
+                for (uint64_t left = copy; left;) {
+                    const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(left))) - 1U;
+                    left &= left - 1ULL;
+                    const uint32_t from = row * P + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(src), static_cast<int>(k)));
+                    for (uint32_t i = lane; i < n; i += 64U) stage[k * piece + i] = __hip_atomic_load(image_word(from, w0 + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                for (uint64_t left = copy; left;) {
+                    const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(left))) - 1U;
+                    left &= left - 1ULL;
+                    for (uint32_t i = lane; i < n; i += 64U) __hip_atomic_store(image_word(row * P + k, w0 + i), stage[k * piece + i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            for (uint64_t left = copy; left;) {
+                const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(left))) - 1U;
+                left &= left - 1ULL;
+                if (lane == 0) __hip_atomic_store(&r.awords[row * P + k], groups | (((flags >> k) & 1U) << 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");      // the staged images are out of LDS before a sweep reuses the slot
             differ &= ~copy;
@@ -625,7 +643,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
     while (differ) {
         const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(differ))) - 1U;
         differ &= differ - 1ULL;
-        const uint32_t at = row * K + k, e = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(expert), static_cast<int>(k)));
+        const uint32_t at = row * P + k, e = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(expert), static_cast<int>(k)));
         uint32_t seen = 0;
         for (uint32_t spins = 0; spins < kFrontSpinLimit; ++spins) {
             seen = __hip_atomic_load(&r.awords[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xffffU;
@@ -638,7 +656,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             continue;
         }
         if (lane == 0) __hip_atomic_store(&r.awords[at], groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (uint32_t grp = 0; grp < groups; ++grp) front_project(slots, w, r, e, grp, at);
+        for (uint32_t grp = 0; grp < groups; ++grp) front_project(slots, w, r, e, grp, at, assignments);
     }
 }
 
@@ -651,7 +669,7 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
     lds_u8* const slots[2] = {(lds_u8*)ring0, (lds_u8*)ring1};
     lds_u8* const (&sl)[2] = slots;
     uint32_t bid = blockIdx.x;
-    const uint32_t lane = threadIdx.x, K = a.p.top_k;
+    const uint32_t lane = threadIdx.x, K = a.p.top_k, P = w.top_k;      // P: with the always-on slots (experts behind the routed ones)
     uint32_t* lines = a.plan + kPlanLinesAt;
     const uint32_t epoch = lines[kLinesEpoch] + 1U;                 // (stored back by the down launch of this call)
     unsigned long long* etags = reinterpret_cast<unsigned long long*>(a.plan + kPlanEtagsAt);
@@ -660,7 +678,7 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
         // the row's first early block also selects: it clears the row's assignment words before anything else (acknowledged long before
         // its tags go out), brings its own four logits, then reads the row's logits until every one carries this call's epoch
         const bool selects = bid % neb == 0;
-        if (selects && lane < K) __hip_atomic_store(&r.awords[row * K + lane], 0U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (selects && lane < P) __hip_atomic_store(&r.awords[row * P + lane], 0U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         early_logits_block<KIND>(a, row, (bid % neb) * kEarlyExperts, epoch);
         if (bid == 0 && lane == 0) {
             *a.job_status = 0;
@@ -668,13 +686,13 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
         }
         if (!selects) return;
         bool ok;
-        const uint32_t expert = early_select_row(a, row, epoch, ok);
+        const uint32_t chosen = early_select_row(a, row, epoch, ok), expert = lane < K ? chosen : a.p.experts + (lane - K);
         if (!ok) {
             if (lane == 0) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_INVALID_ROUTE));
             return;
         }
         stores_acknowledged();
-        if (lane < K) __hip_atomic_store(&etags[row * K + lane], (static_cast<unsigned long long>(epoch) << 32) | expert, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane < P) __hip_atomic_store(&etags[row * P + lane], (static_cast<unsigned long long>(epoch) << 32) | expert, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
     bid -= nb.early;
@@ -690,7 +708,7 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
     bid -= nb.side;
     // Projection block: assignment `at`, 32-output group `grp`. (Sharing one sweep among the rows that chose an expert was
     // measured slower: the sweeps that serve several rows finish last, and the others do not speed up.)
-    const uint32_t groups = w.ffn / 32U, at = bid / groups, grp = bid - at * groups, row = at / K;
+    const uint32_t groups = w.ffn / 32U, at = bid / groups, grp = bid - at * groups, row = at / P;
     unsigned long long tag = 0;
     uint32_t image = 0;
     bool there = false;
@@ -717,7 +735,7 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
         else if (quarter == 2U) __builtin_amdgcn_s_setprio(2);
         else if (quarter == 3U) __builtin_amdgcn_s_setprio(3);
     }
-    front_project(sl, w, r, e, grp, at);
+    front_project(sl, w, r, e, grp, at, assignments);
     stores_acknowledged();
     if (lane == 0) __hip_atomic_fetch_add(&r.awords[at], 1U, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -996,6 +1014,7 @@ __global__ __launch_bounds__(256) void merge_kernel(mi355_moe_weights w, RowsK r
 }
 
 constexpr uint32_t kDownMergeSlots = 8;        // top_k bound: 8 waves x 2 ring slots fill the LDS of a compute unit
+constexpr uint32_t kDownMergeMost = 16;        // of the forms of 16 columns, whose slots are smaller or none (instances of 8, 9 - top-8 and an always-on expert - and 16)
 // What a down + combine launch looks up at its start, in this order and without a branch between the requests: its item, the job word and what
 // the fold needs. The sweep waits for the item; asked for behind the others, or behind branches whose arguments are fetched one block after
 // the other, it stood a way to memory further back. The launch, fold behind the barrier by one thread | requests in front of the item |
@@ -1046,7 +1065,7 @@ __device__ __forceinline__ SlotFold slot_fold_request(const mi355_moe_weights& w
 }
 // The row's value of one column, as merge_kernel folds it (every lane of the wavefront takes part). Fail closed: a row flagged by an
 // earlier stage publishes nothing (the aggregate bit is the combine's own).
-template <class Value>
+template <uint32_t SLOTS, class Value>
 __device__ __forceinline__ void slot_fold(const SlotFold& f, const mi355_moe_weights& w, const RowsK& r, uint32_t row, uint32_t o, uint32_t form, bool stores, uint32_t lane, Value value) {
     if (f.status & ~static_cast<uint32_t>(MI355_STATUS_AGGREGATE)) return;
     const uint32_t K = w.top_k;
@@ -1055,14 +1074,14 @@ __device__ __forceinline__ void slot_fold(const SlotFold& f, const mi355_moe_wei
     if (ascending) {
         place = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < kDownMergeSlots; ++k) {
+        for (uint32_t k = 0; k < SLOTS; ++k) {
             const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(f.route), static_cast<int>(k)));
             place += k < K && (other < f.route || (other == f.route && k < lane)) ? 1U : 0U;
         }
     }
     float acc = 0.0F;
 #pragma unroll
-    for (uint32_t k = 0; k < kDownMergeSlots; ++k) {
+    for (uint32_t k = 0; k < SLOTS; ++k) {
         if (k >= K) continue;
         const uint32_t slot = ascending ? static_cast<uint32_t>(__builtin_ctzll(__ballot(lane < K && place == k))) : k;
         const float wt = f_of(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(b_of(f.weight)), static_cast<int>(slot)))), ev = value(slot);
@@ -1112,7 +1131,7 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
     }
     slot_value[wave][lane] = value;
     __syncthreads();
-    if (wave == 0) slot_fold(fold, w, r, row, o, form, true, lane, [&](uint32_t slot) { return slot_value[slot][lane]; });
+    if (wave == 0) slot_fold<kDownMergeSlots>(fold, w, r, row, o, form, true, lane, [&](uint32_t slot) { return slot_value[slot][lane]; });
 }
 
 // down_merge_kernel for dense rows of at most four super-blocks (down_row_stride = B * 144): the 64 rows of a column block stream as B
@@ -1192,13 +1211,13 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(m
 // The same for the smallest decode batches, in the 16-rows-per-wavefront layout of down_quad_kernel: a workgroup owns (row, 16
 // output columns), wave k sweeps the 16 down rows of the expert in slot k (lane = (row, pair)), the slots' values meet in LDS
 // and the first sixteen lanes of wave 0 fold them as merge_kernel does. One launch instead of two for one to six rows.
-template <int DEPTH>
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_quad_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
-    __shared__ __attribute__((aligned(16))) uint8_t mq0[kDownMergeSlots][kQuadSlotBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t mq1[kDownMergeSlots][kQuadSlotBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t mq2[DEPTH > 2 ? kDownMergeSlots : 1][DEPTH > 2 ? kQuadSlotBytes : 16];
-    __shared__ __attribute__((aligned(16))) uint8_t mq3[DEPTH > 3 ? kDownMergeSlots : 1][DEPTH > 3 ? kQuadSlotBytes : 16];
-    __shared__ float slot_value[kDownMergeSlots][kQuadRows];
+template <int DEPTH, uint32_t SLOTS>
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_quad_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+    __shared__ __attribute__((aligned(16))) uint8_t mq0[SLOTS][kQuadSlotBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t mq1[SLOTS][kQuadSlotBytes];
+    __shared__ __attribute__((aligned(16))) uint8_t mq2[DEPTH > 2 ? SLOTS : 1][DEPTH > 2 ? kQuadSlotBytes : 16];
+    __shared__ __attribute__((aligned(16))) uint8_t mq3[DEPTH > 3 ? SLOTS : 1][DEPTH > 3 ? kQuadSlotBytes : 16];
+    __shared__ float slot_value[SLOTS][kQuadRows];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, rr = lane >> 2, row = blockIdx.y, o0 = blockIdx.x * kQuadRows;
     lds_u8* const ring[4] = {(lds_u8*)mq0[wave], (lds_u8*)mq1[wave], (lds_u8*)mq2[DEPTH > 2 ? wave : 0], (lds_u8*)mq3[DEPTH > 3 ? wave : 0]};
     lds_u8* slots[DEPTH];
@@ -1223,14 +1242,14 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_quad_kernel(m
     }
     if (p == 0) slot_value[wave][rr] = value;
     __syncthreads();
-    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
+    if (wave == 0) slot_fold<SLOTS>(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q5_1 down rows of whole, 16-byte aligned super-blocks (the host executor's format,
 // src/cpu/core/routed_expert.cpp:110-126): the workgroup of (row, 16 columns), wave k = the expert in slot k, each wave with
 // the copy ring, the lane layout and the chain order of down_q51_ring_kernel for its one assignment.
-template <int DEPTH>
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+template <int DEPTH, uint32_t SLOTS>
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) float lds_f32c;
     typedef const __attribute__((address_space(3))) int32_t lds_i32c;
@@ -1238,8 +1257,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
     // a slot: the 16 rows' 8 groups (3 KB), the one assignment's 256 codes and its [8 deltas][8 sums]
     constexpr uint32_t ROWB = kGroupStage * kBlock, CODES_AT = 1024U * WC, TABLE_AT = CODES_AT + 256U, SLOT = TABLE_AT + 64U;
     static_assert(16U * ROWB == 1024U * WC, "the rows of a stage fill the weight copies");
-    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[DEPTH][kDownMergeSlots][SLOT];
-    __shared__ float slot_value[kDownMergeSlots][16];
+    __shared__ __attribute__((aligned(16))) uint8_t ring_mem[DEPTH][SLOTS][SLOT];
+    __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o0 = blockIdx.x * 16U, o = o0 + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
@@ -1323,14 +1342,15 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q51_kernel(mi
     }
     if (j == 0) slot_value[wave][rr] = value;
     __syncthreads();
-    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
+    if (wave == 0) slot_fold<SLOTS>(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q6_K down rows (src/moe_a8_down_contract.cpp:147-158): the workgroup of (row, 16 columns),
 // wave k = the expert in slot k, lane = (row, pair) with the direct loads and the order of down_q6k_kernel.
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+template <uint32_t SLOTS>
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
-    __shared__ float slot_value[kDownMergeSlots][16];
+    __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, half = p >> 1, odd = p & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
@@ -1390,15 +1410,16 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q6k_kernel(mi
     }
     if (p == 0) slot_value[wave][rr] = value;
     __syncthreads();
-    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
+    if (wave == 0) slot_fold<SLOTS>(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // Down rows + combine in one launch for Q8_0 down tensors (the host executor's format, src/cpu/core/routed_expert.cpp:110-126): the
 // workgroup of (row, 16 columns) again, wave k = the expert in slot k, lane = (row, chain) with the direct block loads and the
 // chain order of down_groups_kernel<0>; one item per assignment (the fused decode router's plan).
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+template <uint32_t SLOTS>
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
-    __shared__ float slot_value[kDownMergeSlots][16];
+    __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, odd = j & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
     const uint32_t oc = blockIdx.x * 16U + (lane & 15U);                       // the folding lane's column
@@ -1435,7 +1456,7 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_q8_0_kernel(m
     }
     if (j == 0) slot_value[wave][rr] = value;
     __syncthreads();
-    if (wave == 0) slot_fold(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
+    if (wave == 0) slot_fold<SLOTS>(fold, w, r, row, oc, form, lane < 16U, lane, [&](uint32_t slot) { return slot_value[slot][lane & 15U]; });
 }
 
 // SwiGLU + A8 re-quantisation of dense gate/up rows. Reference: src/cpu/core/routed_expert.cpp:147-170.
@@ -2043,20 +2064,38 @@ void launch_down_merge(const mi355_moe_weights& wv, const RowsK& k, uint32_t row
     else if (flat && B == 4U) down_merge_flat_kernel<4><<<grid, threads, 0, st>>>(wv, k, items, form);
     else down_merge_kernel<<<grid, threads, 0, st>>>(wv, k, items, form);
 }
+// launch(SLOTS): of the instance for that many slots
+template <class Launch> void down_merge_slots(uint32_t slots, Launch launch) {
+    if (slots <= kDownMergeSlots) launch(std::integral_constant<uint32_t, kDownMergeSlots>{});
+    else if (slots == kDownMergeSlots + 1U) launch(std::integral_constant<uint32_t, kDownMergeSlots + 1U>{});
+    else launch(std::integral_constant<uint32_t, kDownMergeMost>{});
+}
 // The other formats' down rows + combine, 16 output columns a workgroup: which launches they take, and the launch.
-bool down_merge_format_takes(const mi355_moe_weights& wv, uint32_t rows) {
-    if (wv.top_k > kDownMergeSlots || wv.hidden % 16U != 0 || rows > 65535U) return false;
+bool down_merge_format_takes(const mi355_moe_weights& wv, const A8Image& h, uint32_t rows) {
+    if (wv.top_k > kDownMergeMost || wv.hidden % 16U != 0 || rows > 65535U) return false;
     if (wv.down_type == MI355_TYPE_Q8_0) return wv.ffn % 128U == 0;
-    if (wv.down_type == MI355_TYPE_Q5_1) return wv.ffn % 256U == 0 && wv.down_row_stride % 16U == 0 && wv.down_expert_stride % 16U == 0;      // (what down_q51_ring_kernel's copies need)
+    if (wv.down_type == MI355_TYPE_Q5_1) return wv.ffn % 256U == 0 && wv.down_row_stride % 16U == 0 && wv.down_expert_stride % 16U == 0 && mma_image(h);      // (what down_q51_ring_kernel's copies need)
     return wv.down_type == MI355_TYPE_Q6_K;
 }
 bool launch_down_merge_format(const mi355_moe_weights& wv, const RowsK& k, uint32_t rows, uint32_t items, uint32_t form, hipStream_t st) {
-    if (!down_merge_format_takes(wv, rows)) return false;
+    if (!down_merge_format_takes(wv, k.h, rows)) return false;
     const dim3 grid(wv.hidden / 16U, rows);
-    if (wv.down_type == MI355_TYPE_Q8_0) down_merge_q8_0_kernel<<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
-    else if (wv.down_type == MI355_TYPE_Q5_1) down_merge_q51_kernel<2><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
-    else down_merge_q6k_kernel<<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    down_merge_slots(wv.top_k, [&](auto slots) {
+        constexpr uint32_t SLOTS = decltype(slots)::value;
+        if (wv.down_type == MI355_TYPE_Q8_0) down_merge_q8_0_kernel<SLOTS><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+        else if (wv.down_type == MI355_TYPE_Q5_1) down_merge_q51_kernel<2, SLOTS><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+        else down_merge_q6k_kernel<SLOTS><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    });
     return true;
+}
+// Q4_K down rows, 16 columns a workgroup (rings of four slots for one or two rows, where eight of them fit)
+void launch_down_merge_quad(const mi355_moe_weights& wv, const RowsK& k, uint32_t rows, uint32_t items, uint32_t form, hipStream_t st) {
+    const dim3 grid(wv.hidden / kQuadRows, rows);
+    down_merge_slots(wv.top_k, [&](auto slots) {
+        constexpr uint32_t SLOTS = decltype(slots)::value;
+        if (SLOTS == kDownMergeSlots && rows <= 2U) down_merge_quad_kernel<SLOTS == kDownMergeSlots ? 4 : 2, SLOTS><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+        else down_merge_quad_kernel<2, SLOTS><<<grid, 64U * wv.top_k, 0, st>>>(wv, k, items, form);
+    });
 }
 
 int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, const float* logit_bias, float* scores, const LayerNorm& norm,
@@ -2103,17 +2142,26 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     // Early routes (route_early.hpp): the expert choice from lane-parallel logits in a short first launch, the exact router beside
     // the projection, down rows + combine on the verified work items. Taken where the 64-row projection sweep and the down +
     // combine launch serve the batch.
-    // Up to two rounds of the down + combine launch's workgroups (each fills a compute unit's LDS): at hidden 2048 / ffn 768, 9..16
-    // rows take 61.5 / 63.2 / 71.4 / 78.0 us (9, 10, 12, 16 rows) against 66.8 / 75.4 / 88.4 / 100 us on the router launch, the
-    // 64-row projection and the staged down rows + combine.
     // From 8 assignments on (one row of top-8): measured at hidden 2048 / ffn 768 against the three launches of the smallest batches
     // (router, 16-row projection, 16-row down + combine): 1 row 28.7 / 31.3 us, 2 rows 31.6 / 35.4, 3 rows 33.4 / 37.8, 4 rows
     // 35.7 / 40.3, 5 rows 38.4 / 48.6, 6 rows 41.2 / 57.8.
     // Down rows of another format, 1, 8, 16 rows against the router launch, the projection and the same down + combine launch: Q6_K 31.6, 67.5,
     // 111.8 -> 26.2, 58.5, 95.2 us, Q8_0 31.0, 67.6, 111.7 -> 25.3, 58.6, 92.1, Q5_1 30.8, 61.0, 100.5 -> 24.9, 52.0, 83.8.
-    const bool early = p->shared_experts == 0 && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
-                       (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeSlots && items <= kEarlyMaxAssignments &&
-                       wv.hidden <= kSideMaxHidden && wv.hidden % 64U == 0 && (wv.hidden / 64U) * rows <= 2U * compute_units() && 2U * wv.experts <= wv.top_k * wv.hidden;
+    // Any width, however many rounds the down + combine launch's workgroups take (each of 64 columns fills a compute unit's LDS). Router launch, projection,
+    // down rows -> early routes, rows of hidden / ffn / experts, top-8: 1 of 2304 / 768 / 64 32.9 -> 30.4 us, 1 of 4096 / 1536 / 64 51.4 -> 48.5, 1 of 6144 / 2560 / 160
+    // 107.2 -> 79.3, 4 of 4096 / 1536 / 64 101.5 -> 77.3, 8 of 4096 / 768 / 128 93.9 -> 75.9, 16 of them 156.5 -> 127.2, 16 of 5120 / 512 / 128 143.6 -> 123.4; fp32 rows, 5 of 6144 / 768 / 64
+    // 103.2 -> 79.9; Q8_0 down rows, 16 of 4096 / 768 / 128 192.4 -> 164.4; top-16 and top-10, 1, 4 rows of 2048 / 768 / 128 36.8, 49.8 -> 29.7, 39.5. Batches of more than
+    // kQuadMaxItems assignments over large experts share their sweeps instead (above): 16 rows of one rank's half of 6144 / 2560 / 160 291.6, with early routes 352.1.
+    // Always-on experts: a row's slot more, whose weights every row sweeps by itself where the plan of the router launch has four rows share a sweep. 1, 2, 5, 8, 14
+    // rows of 2048 / 768 / 128 40.4, 43.7, 59.1, 72.4, 94.7 -> 31.8, 32.3, 48.3, 61.7, 88.0 us, Q6_K down rows 41.8, 45.9, 62.4, 79.2, 106.5 -> 32.5, 34.2, 55.4, 71.7, 104.1, 4 rows of
+    // 4096 / 1536 / 64 111.4 -> 91.8. The line at 64 MB of them: 43 MB 91.0 -> 82.3 us, 73 MB 132.1 -> 138.5, 80 MB 180.3 -> 182.3, but 70 MB 64.7 -> 59.7. Rows of up to kChainNormHidden
+    // features stay with the router launch, which norms them for nothing, and whose chain is short.
+    const RowsK k = [&] { RowsK view = layer_rows(); view.awords = r->plan + kPlanAwordsAt; return view; }();
+    const uint64_t expert_bytes = 2ULL * wv.ffn * moe_row_bytes(wv.gate_type, wv.hidden) + static_cast<uint64_t>(wv.hidden) * moe_row_bytes(wv.down_type, wv.ffn);
+    const bool always_on = p->shared_experts == 0 || (wv.hidden > kChainNormHidden && p->shared_experts * rows * expert_bytes <= (64ULL << 20));
+    const bool early = always_on && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
+                       (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, k.h, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeMost &&
+                       items <= kEarlyMaxAssignments && wv.hidden % 64U == 0 && 2U * wv.experts <= wv.top_k * wv.hidden;
     // (rows that are normalised in place: the router's workgroups would read what others of their launch have written)
     const uint64_t raw = reinterpret_cast<uint64_t>(r->input), raw_end = raw + (rows - 1U) * r->input_stride + (r->input_kind == MI355_INPUT_F32 ? 4ULL : 2ULL) * wv.hidden;
     const uint64_t out = reinterpret_cast<uint64_t>(norm.normed), out_end = out + 4ULL * rows * wv.hidden;
@@ -2130,8 +2178,6 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         a.early_perturb = g_early_perturb.load(std::memory_order_relaxed);
         // the early logits of row i (64-bit words) live in the row's (still unused) unweighted-output block: the exact logits own `scores`
         a.early_logits = r->rawdots; a.early_stride = wv.top_k * wv.hidden;
-        RowsK k = layer_rows();
-        k.awords = a.awords;
         RowsK front = k;
         front.plan = nullptr;              // (the front launch names its assignments itself: the work items are written inside it)
         const FrontBlocks nb{rows * ((p->experts + kEarlyExperts - 1U) / kEarlyExperts), a.quant_blocks, rows * ((p->experts + kSideExperts - 1U) / kSideExperts)};
@@ -2143,7 +2189,9 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
             STRIX_LAUNCHED("moe layer early routes + gate / up");
         }
         if (do_back) {
-            if (!launch_down_merge_format(wv, k, rows, items, form, st)) launch_down_merge(wv, k, rows, items, form, st);
+            if (launch_down_merge_format(wv, k, rows, items, form, st)) {
+            } else if (wv.top_k <= kDownMergeSlots) launch_down_merge(wv, k, rows, items, form, st);
+            else launch_down_merge_quad(wv, k, rows, items, form, st);
             STRIX_LAUNCHED("moe layer experts + combine");
         }
         return MI355_OK;
@@ -2175,9 +2223,7 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         return MI355_OK;
     }
     if (quad_sweep(wv, rows) && wv.down_type == MI355_TYPE_Q4_K && wv.top_k <= kDownMergeSlots && wv.hidden % kQuadRows == 0 && rows <= 65535U) {
-        const dim3 grid(wv.hidden / kQuadRows, rows);
-        if (rows <= 2U) down_merge_quad_kernel<4><<<grid, 64U * wv.top_k, 0, st>>>(wv, layer_rows(), items, form);
-        else down_merge_quad_kernel<2><<<grid, 64U * wv.top_k, 0, st>>>(wv, layer_rows(), items, form);
+        launch_down_merge_quad(wv, layer_rows(), rows, items, form, st);
         STRIX_LAUNCHED("moe layer experts + combine");
         return MI355_OK;
     }

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import orc
 from test_gpu_parity import early_choice
 
 pytestmark = pytest.mark.gpu
@@ -101,3 +102,64 @@ def test_fp32_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_
         assert torch.equal(ids, want_ids) and torch.equal(w.view(torch.int32), want_w.view(torch.int32))
         assert torch.equal(scores.reshape(-1)[:rows * experts].view(torch.int32), want_scores.reshape(-1).view(torch.int32))
         assert torch.equal(y.view(torch.int32), staged.run(rows32, want_ids, want_w).view(torch.int32)) and int(layer.status[:rows].sum()) == 0
+
+
+# rows of more chunks than the side chain's ring has places, the last one partial; more rows than two rounds of the down + combine launch; sweeps of whole and of
+# partial stages; images of h that a repair copies in one piece and in several
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(1, 2304, 256, 16, 8), (3, 3328, 256, 24, 4), (16, 4096, 256, 16, 8), (5, 4096, 2304, 10, 8), (2, 8192, 256, 24, 16)])
+@pytest.mark.parametrize("dtype,down", [(torch.float16, "q4_k"), (torch.bfloat16, "q8_0"), (torch.float32, "q4_k")])
+def test_long_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_k, dtype, down):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    g, u = (blocks(gen, experts * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, experts * hidden, ffn, *{"q4_k": (256, 144, (1, 3)), "q8_0": (32, 34, (1,))}[down])
+    layer, staged = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows, down_type=getattr(strix, "TYPE_" + down.upper())) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(dtype)
+    ids, w, scores = (t.clone() for t in strix.route(x, router, top_k))
+    want = staged.run(x, ids, w)
+    assert int((torch.from_numpy(early_choice(x.float().cpu().numpy(), router.cpu().numpy(), top_k, 150).astype("int64")) != ids.cpu()).sum()) >= 2
+    for displaced in (0, 150, 0):
+        epoch = int(layer.plan[EPOCH])
+        strix.lib().mi355_debug_early_route_perturb(displaced)
+        try:
+            y, got, weights, s = layer.run_layer(x, router)
+            torch.cuda.synchronize()
+        finally:
+            strix.lib().mi355_debug_early_route_perturb(0)
+        assert int(layer.plan[EPOCH]) == epoch + 1 and int(layer.status[:rows].sum()) == 0
+        assert torch.equal(got, ids) and torch.equal(weights.view(torch.int32), w.view(torch.int32))
+        assert torch.equal(s.reshape(-1)[:rows * experts].view(torch.int32), scores.reshape(-1).view(torch.int32))
+        assert torch.equal(y.view(torch.int32), want.view(torch.int32)), displaced
+
+
+# always-on slots: nine (an instance of their own), ten and more, up to eight; with and without a gate; as many assignments as the form takes
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,shared", [(1, 2048, 256, 24, 8, 1), (14, 1792, 256, 32, 8, 1), (5, 2048, 768, 16, 6, 2), (8, 2304, 256, 24, 14, 2), (6, 1792, 512, 16, 8, 2)])
+@pytest.mark.parametrize("down", ["q4_k", "q6_k", "q8_0", "q5_1"])
+@pytest.mark.parametrize("gated", [False, True])
+def test_always_on_slots_equal_the_router_launch(strix, rows, hidden, ffn, experts, top_k, shared, down, gated):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden + top_k)
+    E, K = experts + shared, top_k + shared
+    g, u = (blocks(gen, E * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, E * hidden, ffn, *{"q4_k": (256, 144, (1, 3)), "q6_k": (256, 210, (209,)), "q8_0": (32, 34, (1,)), "q5_1": (32, 24, (1, 3))}[down])
+    layer, staged = (strix.MoeLayer(hidden, ffn, E, K, g, u, d, rows, down_type=getattr(strix, "TYPE_" + down.upper())) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+    gates = torch.rand((rows, shared), device="cuda", generator=gen) if gated else None
+    ids, w = (t.clone() for t in strix.route(x, router, top_k)[:2])
+    all_ids = torch.cat([ids, torch.arange(experts, E, device="cuda", dtype=torch.int32).expand(rows, shared)], dim=1).contiguous()
+    all_w = torch.cat([w, gates if gated else torch.ones((rows, shared), device="cuda")], dim=1).contiguous()
+    staged.run(x, all_ids, all_w)
+    for form in (strix.COMBINE_FMA_SLOT, strix.COMBINE_MULADD_ASC):
+        want = orc.combine_shared(form, all_w.cpu().numpy(), all_ids.cpu().numpy(), staged.rawdots[:rows].cpu().numpy().reshape(rows, K, hidden), shared)
+        for displaced in (0, 200):
+            epoch = int(layer.plan[EPOCH])
+            strix.lib().mi355_debug_early_route_perturb(displaced)
+            try:
+                y, got, weights, _ = layer.run_layer(x, router, combine=form, shared_experts=shared, shared_slot_weights=gates)
+                torch.cuda.synchronize()
+            finally:
+                strix.lib().mi355_debug_early_route_perturb(0)
+            assert int(layer.plan[EPOCH]) == epoch + 1 and int(layer.status[:rows].sum()) == 0
+            assert torch.equal(got, all_ids) and torch.equal(weights.view(torch.int32), all_w.view(torch.int32))
+            assert torch.equal(layer.rawdots[:rows].view(torch.int32), staged.rawdots[:rows].view(torch.int32))
+            assert torch.equal(y.view(torch.int32), torch.from_numpy(want).cuda().view(torch.int32)), (form, displaced)
