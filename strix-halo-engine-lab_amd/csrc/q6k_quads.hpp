@@ -6,8 +6,7 @@
 // (term_2p + term_(2p+1)) to pair accumulator p, and the row's value is (acc0 + acc1) + (acc2 + acc3).
 //
 // Layout as in q4k_quads.hpp / down_groups.hpp: 16 output rows per wavefront, lane = (row, pair p), up to four assignments
-// per weight pass. Both groups of a pair share `half`, so a lane reads 64 bytes of nibbles, 32 bytes of bit pairs and four
-// scale bytes per block. Blocks are only 2-byte aligned (210 bytes): every multi-byte read is made of aligned words.
+// per weight pass. Blocks are only 2-byte aligned (210 bytes): every multi-byte read is made of aligned words.
 #pragma once
 #include "device_math.hpp"
 #include "q4k_rows.hpp"
@@ -16,23 +15,67 @@ namespace strix950 {
 
 constexpr uint32_t kQ6kBlock = 210;
 
-// N words starting at a 2-byte aligned address, from N + 1 aligned words
+// N words starting at a 2-byte aligned address, from N + 1 aligned words: the caller's N words are followed by two more bytes that may be read. (128-bit loads
+// from the 2-byte aligned address itself are slower: layers of 8, 16 rows of 2048 / 768 / 128 59.7, 98.4 us. The words are reached from the pointer, not from its value
+// as a number, so that they are global loads and not flat ones, which wait for the LDS as well.)
 template <int N>
 __device__ __forceinline__ void load_words_2aligned(const uint8_t* at, uint32_t (&out)[N]) {
-    const uintptr_t address = reinterpret_cast<uintptr_t>(at);
-    const uint32_t* aligned = reinterpret_cast<const uint32_t*>(address & ~static_cast<uintptr_t>(3));
-    const uint32_t shift = static_cast<uint32_t>(address) & 3U;
+    const uint32_t shift = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(at)) & 3U;
+    const uint32_t* aligned = reinterpret_cast<const uint32_t*>(at - shift);
     uint32_t raw[N + 1];
 #pragma unroll
-    for (int i = 0; i < N; ++i) raw[i] = aligned[i];
-    raw[N] = shift ? aligned[N] : 0U;                         // an aligned start needs no straddling word: not read
+    for (int i = 0; i <= N; ++i) raw[i] = aligned[i];
 #pragma unroll
     for (int i = 0; i < N; ++i) out[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], shift);
 }
 
+// A block by direct loads. Both pairs of a half of the block are made of the same bytes, so lane (row, half, t) reads weights 16 t .. 16 t + 15 of all
+// four groups of its half - 16 + 16 bytes of nibbles and 16 of bit pairs, once -, and the lanes t = 0, 1 exchange the parts of the group integers: each
+// ends with the two groups of pair p = 2 half + t. The loads are what bounds these kernels (their number, at 2-byte aligned places): with each
+// lane reading its pair's 64 + 32 bytes every byte was read twice.
+// q: four times the weight (((nibble | pair << 4) - 32) << 2 is the six bits at the top of the byte with the highest one flipped); d: a quarter of the factor (exact).
+struct Q6kPart { uint32_t q[4][4]; int s[4]; float d; };
+__device__ __forceinline__ void q6k_part(Q6kPart& w, const uint8_t* block, uint32_t half, uint32_t t) {
+    typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+    uint32_t a[4], b[4], h[4];
+    load_words_2aligned<4>(block + 64U * half + 16U * t, a);
+    load_words_2aligned<4>(block + 64U * half + 32U + 16U * t, b);
+    load_words_2aligned<4>(block + 128U + 32U * half + 16U * t, h);
+    const u32x2_a2 scales = *reinterpret_cast<const u32x2_a2*>(block + 192U + 8U * half);
+    w.d = half_bits_to_float(*reinterpret_cast<const uint16_t*>(block + 208U)) * 0.25F;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        w.q[0][i] = (((a[i] << 2) & 0x3c3c3c3cU) | ((h[i] << 6) & 0xc0c0c0c0U)) ^ 0x80808080U;
+        w.q[1][i] = (((b[i] << 2) & 0x3c3c3c3cU) | ((h[i] << 4) & 0xc0c0c0c0U)) ^ 0x80808080U;
+        w.q[2][i] = (((a[i] >> 2) & 0x3c3c3c3cU) | ((h[i] << 2) & 0xc0c0c0c0U)) ^ 0x80808080U;
+        w.q[3][i] = (((b[i] >> 2) & 0x3c3c3c3cU) | (h[i] & 0xc0c0c0c0U)) ^ 0x80808080U;
+    }
+    w.s[0] = __builtin_amdgcn_sbfe(scales.x, 8U * t, 8U);
+    w.s[1] = __builtin_amdgcn_sbfe(scales.x, 16U + 8U * t, 8U);
+    w.s[2] = __builtin_amdgcn_sbfe(scales.y, 8U * t, 8U);
+    w.s[3] = __builtin_amdgcn_sbfe(scales.y, 16U + 8U * t, 8U);
+}
+// term_2p + term_(2p+1) of the lane's pair p for the activation row whose codes and deltas of the super-block are given
+__device__ __forceinline__ float q6k_part_term(const Q6kPart& w, const int8_t* codes, const float* deltas, uint32_t half, uint32_t t) {
+    typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
+    typedef float f32x2_g __attribute__((ext_vector_type(2)));
+    const __attribute__((address_space(1))) u32x4_g* from = (const __attribute__((address_space(1))) u32x4_g*)(codes + 128U * half + 16U * t);
+    const f32x2_g delta = *(const __attribute__((address_space(1))) f32x2_g*)(deltas + 4U * half + 2U * t);
+    int part[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4U; ++k) {
+        const u32x4_g c = from[2U * k];
+        int dot = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dot = __builtin_amdgcn_sdot4(static_cast<int>(w.q[k][i]), static_cast<int>(c[i]), dot, false);
+        part[k] = __mul24(w.s[k], dot);
+    }
+    const int first = (t ? part[2] : part[0]) + xor1_i(t ? part[0] : part[2]), second = (t ? part[3] : part[1]) + xor1_i(t ? part[1] : part[3]);
+    return delta.x * (w.d * static_cast<float>(first)) + delta.y * (w.d * static_cast<float>(second));
+}
+
 __global__ __launch_bounds__(256) void down_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments,
                                                        uint32_t items_at, uint32_t order_at) {
-    typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
     constexpr uint32_t NA = 4;
     const WorkItem item = work_item(w, r, items_at, blockIdx.y);
     const uint32_t e = item.e, begin = item.begin, end = item.end;
@@ -40,7 +83,7 @@ __global__ __launch_bounds__(256) void down_q6k_kernel(mi355_moe_weights w, Rows
     if (*r.job_status & MI355_STATUS_NONFINITE_PROJECTION) return;
     const uint32_t lane = threadIdx.x & 63U, wave = threadIdx.x >> 6, p = lane & 3U, half = p >> 1, odd = p & 1U;
     const uint32_t o = blockIdx.x * 64U + 16U * wave + (lane >> 2);
-    const uint32_t groups = w.ffn / 32U, blocks = w.ffn / 256U;
+    const uint32_t blocks = w.ffn / 256U;
     const uint8_t* wrow = w.down + static_cast<size_t>(e) * w.down_expert_stride + static_cast<size_t>(o) * w.down_row_stride;
     for (uint32_t c0 = begin; c0 < end; c0 += NA) {
         const uint32_t na = end - c0 < NA ? end - c0 : NA;
@@ -55,50 +98,13 @@ __global__ __launch_bounds__(256) void down_q6k_kernel(mi355_moe_weights w, Rows
             h_codes[a] = r.h.codes_of(src[a]);
             h_deltas[a] = r.h.deltas_of(src[a]);
         }
-#pragma unroll 2
+#pragma unroll 1
         for (uint32_t b = 0; b < blocks; ++b) {
-            const uint8_t* blk = wrow + static_cast<size_t>(b) * kQ6kBlock;
-            uint32_t ql[16], qh[8];
-            load_words_2aligned<16>(blk + 64U * half, ql);
-            load_words_2aligned<8>(blk + 128U + 32U * half, qh);
-            const uint16_t* tail = reinterpret_cast<const uint16_t*>(blk + 192U);
-            const uint32_t sc01 = tail[2U * p], sc23 = tail[2U * p + 1U];          // scales 4p, 4p + 1 | 4p + 2, 4p + 3
-            const float d = half_bits_to_float(tail[8]);
-            // signed weights of groups 2p (k = 0) and 2p + 1 (k = 1), four per word
-            uint32_t q[2][8];
+            Q6kPart part;
+            q6k_part(part, wrow + static_cast<size_t>(b) * kQ6kBlock, half, odd);
 #pragma unroll
-            for (uint32_t k = 0; k < 2U; ++k)
-#pragma unroll
-                for (uint32_t i = 0; i < 8U; ++i) {
-                    const uint32_t nibbles = (ql[8U * k + i] >> (4U * odd)) & 0x0f0f0f0fU;
-                    const uint32_t pairs = (qh[i] >> (4U * odd + 2U * k)) & 0x03030303U;
-                    const uint32_t six = nibbles | (pairs << 4);                   // 0 .. 63 per byte
-                    q[k][i] = ((six | 0x80808080U) - 0x20202020U) ^ 0x80808080U;   // minus 32 per byte, no borrow between bytes
-                }
-            const int s[2][2] = {{static_cast<int8_t>(sc01 & 255U), static_cast<int8_t>(sc01 >> 8)},
-                                 {static_cast<int8_t>(sc23 & 255U), static_cast<int8_t>(sc23 >> 8)}};
-#pragma unroll
-            for (uint32_t a = 0; a < NA; ++a) {
-                if (a < na) {                                     // uniform over the workgroup
-                    const u32x4_g* codes = reinterpret_cast<const u32x4_g*>(h_codes[a] + 256U * b + 64U * p);
-                    const float2 delta = *reinterpret_cast<const float2*>(h_deltas[a] + 8U * b + 2U * p);
-                    float term[2];
-#pragma unroll
-                    for (uint32_t k = 0; k < 2U; ++k) {
-                        const u32x4_g c_lo = codes[2U * k], c_hi = codes[2U * k + 1U];
-                        const uint32_t cw[8] = {c_lo.x, c_lo.y, c_lo.z, c_lo.w, c_hi.x, c_hi.y, c_hi.z, c_hi.w};
-                        int first = 0, last = 0;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            first = __builtin_amdgcn_sdot4(static_cast<int>(q[k][i]), static_cast<int>(cw[i]), first, false);
-                            last = __builtin_amdgcn_sdot4(static_cast<int>(q[k][4 + i]), static_cast<int>(cw[4 + i]), last, false);
-                        }
-                        const int integer = s[k][0] * first + s[k][1] * last;
-                        term[k] = (k == 0 ? delta.x : delta.y) * (d * static_cast<float>(integer));
-                    }
-                    acc[a] = acc[a] + (term[0] + term[1]);
-                }
-            }
+            for (uint32_t a = 0; a < NA; ++a)
+                if (a < na) acc[a] = acc[a] + q6k_part_term(part, h_codes[a] + 256U * b, h_deltas[a] + 8U * b, half, odd);         // (uniform over the workgroup)
         }
 #pragma unroll
         for (uint32_t a = 0; a < NA; ++a) {

@@ -1346,10 +1346,12 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_we
 }
 
 // Down rows + combine in one launch for Q6_K down rows (src/moe_a8_down_contract.cpp:147-158): the workgroup of (row, 16 columns),
-// wave k = the expert in slot k, lane = (row, pair) with the direct loads and the order of down_q6k_kernel.
+// wave k = the expert in slot k, lane = (row, pair) with the direct loads and the order of down_q6k_kernel. Bound by its loads (q6k_part); three blocks' worth of them
+// asked for together (a bound on the registers, for a workgroup more on a compute unit, costs more than it gives: 8, 16 rows 55.8, 88.6 us). Layers of hidden 2048 /
+// ffn 768 / 128 experts top-8, 1, 8, 16 rows 25.7, 57.8, 92.1 -> 25.1, 54.3, 85.9 us; 5 of them with the norm and an always-on expert 57.3 -> 53.6; 4 rows of 4096 /
+// 1536 / 64 103.4 -> 94.2; 6 rows of 3072 / 2304 / 32 top-4 100.6 -> 87.8.
 template <uint32_t SLOTS>
 __global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
-    typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
     __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, half = p >> 1, odd = p & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
@@ -1366,42 +1368,11 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_we
         const int8_t* h_codes = r.h.codes_of(src);
         const float* h_deltas = r.h.deltas_of(src);
         float acc = 0.0F;
-#pragma unroll 2
+#pragma unroll 3
         for (uint32_t b = 0; b < blocks; ++b) {
-            const uint8_t* blk = wrow + static_cast<size_t>(b) * kQ6kBlock;
-            uint32_t ql[16], qh[8];
-            load_words_2aligned<16>(blk + 64U * half, ql);
-            load_words_2aligned<8>(blk + 128U + 32U * half, qh);
-            const uint16_t* tail = reinterpret_cast<const uint16_t*>(blk + 192U);
-            const uint32_t sc01 = tail[2U * p], sc23 = tail[2U * p + 1U];          // scales 4p, 4p + 1 | 4p + 2, 4p + 3
-            const float d = half_bits_to_float(tail[8]);
-            const int s[2][2] = {{static_cast<int8_t>(sc01 & 255U), static_cast<int8_t>(sc01 >> 8)},
-                                 {static_cast<int8_t>(sc23 & 255U), static_cast<int8_t>(sc23 >> 8)}};
-            const u32x4_g* codes = reinterpret_cast<const u32x4_g*>(h_codes + 256U * b + 64U * p);
-            const float2 delta = *reinterpret_cast<const float2*>(h_deltas + 8U * b + 2U * p);
-            float term[2];
-#pragma unroll
-            for (uint32_t k = 0; k < 2U; ++k) {
-                uint32_t q[8];
-#pragma unroll
-                for (uint32_t i = 0; i < 8U; ++i) {
-                    const uint32_t nibbles = (ql[8U * k + i] >> (4U * odd)) & 0x0f0f0f0fU;
-                    const uint32_t pairs = (qh[i] >> (4U * odd + 2U * k)) & 0x03030303U;
-                    const uint32_t six = nibbles | (pairs << 4);                   // 0 .. 63 per byte
-                    q[i] = ((six | 0x80808080U) - 0x20202020U) ^ 0x80808080U;      // minus 32 per byte, no borrow between bytes
-                }
-                const u32x4_g c_lo = codes[2U * k], c_hi = codes[2U * k + 1U];
-                const uint32_t cw[8] = {c_lo.x, c_lo.y, c_lo.z, c_lo.w, c_hi.x, c_hi.y, c_hi.z, c_hi.w};
-                int first = 0, last = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    first = __builtin_amdgcn_sdot4(static_cast<int>(q[i]), static_cast<int>(cw[i]), first, false);
-                    last = __builtin_amdgcn_sdot4(static_cast<int>(q[4 + i]), static_cast<int>(cw[4 + i]), last, false);
-                }
-                const int integer = s[k][0] * first + s[k][1] * last;
-                term[k] = (k == 0 ? delta.x : delta.y) * (d * static_cast<float>(integer));
-            }
-            acc = acc + (term[0] + term[1]);
+            Q6kPart part;
+            q6k_part(part, wrow + static_cast<size_t>(b) * kQ6kBlock, half, odd);
+            acc = acc + q6k_part_term(part, h_codes + 256U * b, h_deltas + 8U * b, half, odd);
         }
         value = acc;
         value = value + xor1_f(value);          // acc0 + acc1 | acc2 + acc3
@@ -1416,9 +1387,13 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_we
 // Down rows + combine in one launch for Q8_0 down tensors (the host executor's format, src/cpu/core/routed_expert.cpp:110-126): the
 // workgroup of (row, 16 columns) again, wave k = the expert in slot k, lane = (row, chain) with the direct block loads and the
 // chain order of down_groups_kernel<0>; one item per assignment (the fused decode router's plan).
+// (The image of h by global loads - from a pointer that may come out of a table they were flat ones, which wait for the LDS as well -, three groups of a chain's asked
+// for together, two in the wider workgroups: 8, 16 rows of 2048 / 768 / 128 57.5, 90.1 -> 56.3, 88.7 us, 4 of 4096 / 1536 / 64 98.9 -> 96.6.)
 template <uint32_t SLOTS>
 __global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
+    typedef const __attribute__((address_space(1))) u32x4_g global_u32x4;
+    typedef const __attribute__((address_space(1))) float global_f32;
     __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, odd = j & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
@@ -1435,19 +1410,19 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_w
         const int8_t* h_codes = r.h.codes_of(src);
         const float* h_deltas = r.h.deltas_of(src);
         float chain = 0.0F;
-#pragma unroll 2
+#pragma unroll (SLOTS > kDownMergeSlots ? 2 : 3)
         for (uint32_t c = 0; c < per_chain; ++c) {
             const uint32_t g = 4U * c + j;
             float d, m;
             uint32_t q[8];
             load_group_block<0>(wrow + static_cast<size_t>(c) * (4U * 34U), odd, d, m, q);
-            const u32x4_g* codes = reinterpret_cast<const u32x4_g*>(h_codes + 32U * g);
+            const global_u32x4* codes = (const global_u32x4*)(h_codes + 32U * g);
             const u32x4_g c_lo = codes[0], c_hi = codes[1];
             const uint32_t cw[8] = {c_lo.x, c_lo.y, c_lo.z, c_lo.w, c_hi.x, c_hi.y, c_hi.z, c_hi.w};
             int dot = 0;
 #pragma unroll
             for (int i = 0; i < 8; ++i) dot = __builtin_amdgcn_sdot4(static_cast<int>(q[i]), static_cast<int>(cw[i]), dot, false);
-            chain = chain + (h_deltas[g] * (d * static_cast<float>(dot)));
+            chain = chain + ((((const global_f32*)h_deltas)[g]) * (d * static_cast<float>(dot)));
         }
         value = chain;
         value = value + xor1_f(value);          // chain0 + chain1 | chain2 + chain3
