@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) void down_groups_kernel(mi355_moe_weights w, R
 #pragma unroll
             for (uint32_t a = 0; a < kDownGroupsAssignments; ++a) {
                 if (a < na) {                                     // uniform over the workgroup
-                    const u32x4_g* codes = reinterpret_cast<const u32x4_g*>(h_codes[a] + 32U * g);
+                    const auto* codes = in_global<u32x4_g>(h_codes[a] + 32U * g);
                     const u32x4_g c_lo = codes[0], c_hi = codes[1];
                     const uint32_t cw[8] = {c_lo.x, c_lo.y, c_lo.z, c_lo.w, c_hi.x, c_hi.y, c_hi.z, c_hi.w};
                     int dot = 0;
@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256) void down_groups_kernel(mi355_moe_weights w, R
                     for (int i = 0; i < 8; ++i) dot = __builtin_amdgcn_sdot4(static_cast<int>(q[i]), static_cast<int>(cw[i]), dot, false);
                     const float first = d * static_cast<float>(dot);
                     float combined = first;
-                    if (FMT == 1) combined = first + (m * static_cast<float>(h_sums[a][g]));
-                    chain[a] = chain[a] + (h_deltas[a][g] * combined);
+                    if (FMT == 1) combined = first + (m * static_cast<float>(in_global<int32_t>(h_sums[a])[g]));
+                    chain[a] = chain[a] + (in_global<float>(h_deltas[a])[g] * combined);
                 }
             }
         }

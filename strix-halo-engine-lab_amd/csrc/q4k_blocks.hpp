@@ -36,6 +36,24 @@ __device__ __forceinline__ float wave_shr1(float v) {       // lane l receives l
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xF, 0xF, true));
 }
 
+// Codes of an activation row in LDS for lanes that read different blocks of it: 16-byte piece t of block b lies at position t ^ b of the block's sixteen (b below
+// LOW, a power of two up to 16), so that eight neighbouring lanes read different banks. Piece t of the lane's block: from `at[t % LOW]`, 16 LOW (t / LOW) bytes on.
+template <uint32_t LOW> struct SpreadCodes {
+    uint32_t at[LOW];
+    __device__ __forceinline__ SpreadCodes(const lds_u8* image, uint32_t b) {
+        const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(image)) + 256U * b, turn = 16U * b;
+#pragma unroll
+        for (uint32_t t = 0; t < LOW; ++t) at[t] = base + ((16U * t) ^ turn);
+    }
+    __device__ __forceinline__ void read(u32x4 (&code)[16]) const {
+        typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+#pragma unroll
+        for (uint32_t t = 0; t < 16U; ++t) code[t] = *(lds_u32x4*)(uintptr_t)(at[t % LOW] + 16U * LOW * (t / LOW));
+    }
+};
+// byte of the row's codes that belongs at byte 16 place of their image
+__device__ __forceinline__ uint32_t spread_source(uint32_t place) { return 16U * (place ^ ((place >> 4) & 15U)); }
+
 // stage_base(s): first byte of stage s (16-byte aligned). Returns, in lane i < stages * R, the value of row i (rows in stage
 // order) against image row `image_row` of img; other lanes: 0. slots: DEPTH separate LDS objects of >= 9,216 bytes with
 // nothing in flight; on exit every copy has landed and been consumed.
@@ -68,13 +86,13 @@ __device__ __forceinline__ float sweep_block_lanes(lds_u8* const (&slots)[DEPTH]
     u32x4 code[16];
     float delta[8], fsum[8];
     {
-        const u32x4* cs = reinterpret_cast<const u32x4*>(img.codes_of(image_row) + 256U * b);
+        const auto* cs = in_global<u32x4>(img.codes_of(image_row) + 256U * b);
 #pragma unroll
         for (int i = 0; i < 16; ++i) code[i] = cs[i];
-        const f32x4* ds = reinterpret_cast<const f32x4*>(img.deltas_of(image_row) + 8U * b);
+        const auto* ds = in_global<f32x4>(img.deltas_of(image_row) + 8U * b);
         const f32x4 d0 = ds[0], d1 = ds[1];
         typedef int i32x4 __attribute__((ext_vector_type(4)));
-        const i32x4* ss = reinterpret_cast<const i32x4*>(img.sums_of(image_row) + 8U * b);
+        const auto* ss = in_global<i32x4>(img.sums_of(image_row) + 8U * b);
         const i32x4 s0 = ss[0], s1 = ss[1];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -82,6 +100,7 @@ __device__ __forceinline__ float sweep_block_lanes(lds_u8* const (&slots)[DEPTH]
             fsum[j] = static_cast<float>(s0[j]); fsum[4 + j] = static_cast<float>(s1[j]);
         }
     }
+    if (DEPTH == 2) block_lane_wait<0>();            // (what the first stage waits for; said here, no later stage waits for the activation loads again)
     float value = 0.0F;
     for (uint32_t s0 = 0; s0 < stages; s0 += DEPTH) {
 #pragma unroll
@@ -157,7 +176,7 @@ __device__ __forceinline__ float sweep_block_lanes(lds_u8* const (&slots)[DEPTH]
 // instructions and 16 LDS accesses per sweep in the place of 114 per stage). STAGES * 1 KB must fit a slot.
 template <int STAGES, class StageBase>
 __device__ __forceinline__ float sweep_block_lanes_terms(lds_u8* const (&slots)[2], StageBase stage_base, const BlockLanes g, const A8Image& img, uint32_t image_row) {
-    static_assert(STAGES >= 2 && STAGES <= 9, "terms of every stage side by side in one slot");
+    static_assert(STAGES == 4 || STAGES == 8, "rows of as many blocks as there are stages; terms of every stage side by side in one slot");
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) f32x4 lds_f32x4;
     typedef __attribute__((address_space(3))) f32x4 lds_f32x4_w;
@@ -170,24 +189,30 @@ __device__ __forceinline__ float sweep_block_lanes_terms(lds_u8* const (&slots)[
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(base + 1024U * i),
                                              (__attribute__((address_space(3))) void*)(slot + 1024U * i), 16, 0, 0);
     };
-    start(0U, slots[0]);
-    // the lane's share of the activation row: block b's 256 codes, 8 deltas, 8 sums
-    u32x4 code[16];
-    float delta[8], fsum[8];
+    // the lane's share of the activation row: block b's 256 codes, 8 deltas, 8 sums. The codes come through the second slot, whose first stage is asked for when
+    // they are in registers: by direct loads eight lanes of which ask for the same bytes they are twice as many accesses as the first stage.
+    // (Plain copy instructions, waited for by count: the reads wait for them and not for the stage behind them.)
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    const auto* ds = in_global<f32x4>(img.deltas_of(image_row) + 8U * b);
+    const auto* ss = in_global<i32x4>(img.sums_of(image_row) + 8U * b);
+    const f32x4 d0 = ds[0], d1 = ds[1];
+    const i32x4 s0 = ss[0], s1 = ss[1];
     {
-        const u32x4* cs = reinterpret_cast<const u32x4*>(img.codes_of(image_row) + 256U * b);
+        const uint8_t* codes = reinterpret_cast<const uint8_t*>(img.codes_of(image_row));
+        const uint32_t lds_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(slots[1])));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) code[i] = cs[i];
-        const f32x4* ds = reinterpret_cast<const f32x4*>(img.deltas_of(image_row) + 8U * b);
-        const f32x4 d0 = ds[0], d1 = ds[1];
-        typedef int i32x4 __attribute__((ext_vector_type(4)));
-        const i32x4* ss = reinterpret_cast<const i32x4*>(img.sums_of(image_row) + 8U * b);
-        const i32x4 s0 = ss[0], s1 = ss[1];
+        for (uint32_t c = 0; c < STAGES / 4U; ++c)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_at + 1024U * c), "v"(codes + spread_source(64U * c + lane)) : "memory", "m0");
+    }
+    start(0U, slots[0]);
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kBlockLaneCopies) : "memory");
+    u32x4 code[16];
+    SpreadCodes<STAGES>(slots[1], b).read(code);
+    float delta[8], fsum[8];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            delta[j] = d0[j]; delta[4 + j] = d1[j];
-            fsum[j] = static_cast<float>(s0[j]); fsum[4 + j] = static_cast<float>(s1[j]);
-        }
+    for (int j = 0; j < 4; ++j) {
+        delta[j] = d0[j]; delta[4 + j] = d1[j];
+        fsum[j] = static_cast<float>(s0[j]); fsum[4 + j] = static_cast<float>(s1[j]);
     }
     float t[STAGES][4];
 #pragma unroll
@@ -283,7 +308,7 @@ __device__ __forceinline__ float sweep_flat_rows(lds_u8* const (&slots)[DEPTH], 
 #pragma unroll
         for (uint32_t i = 0; i < kActCopies; ++i) {
             const uint32_t piece = i * 64U + lane;
-            const uint8_t* src = piece < 16U * B ? codes + 16U * piece : piece < 18U * B ? deltas + 16U * (piece - 16U * B) : sums + 16U * (piece - 18U * B);
+            const uint8_t* src = piece < 16U * B ? codes + spread_source(piece) : piece < 18U * B ? deltas + 16U * (piece - 16U * B) : sums + 16U * (piece - 18U * B);
             if (piece < kActPieces)                                // (the lanes past the image copy nothing)
                 __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)(act + 1024U * i), 16, 0, 0);
         }
@@ -302,9 +327,7 @@ __device__ __forceinline__ float sweep_flat_rows(lds_u8* const (&slots)[DEPTH], 
         const uint32_t b = (64U * static_cast<uint32_t>(s) + lane) % static_cast<uint32_t>(B);
         u32x4 code[16];
         float delta[8], fsum[8];
-        lds_u32x4* cs = (lds_u32x4*)(act + 256U * b);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) code[i] = cs[i];
+        SpreadCodes<(B < 3 ? 2U : B < 5 ? 4U : 16U)>(act, b).read(code);
         lds_f32x4* ds = (lds_f32x4*)(act + 256U * B + 32U * b);
         const f32x4 d0 = ds[0], d1 = ds[1];
         lds_i32x4* ss = (lds_i32x4*)(act + 288U * B + 32U * b);

@@ -127,9 +127,18 @@ __device__ __forceinline__ void quad_block_compute_q5k(const lds_u8* slot, uint3
 template <int DEPTH, bool Q5K = false>
 __device__ __forceinline__ float sweep_quads(lds_u8* const (&slots)[DEPTH], QuadSourceT<Q5K ? 11U : 9U> source, uint32_t blocks, const A8Image& img, uint32_t row) {
     const uint32_t lane = threadIdx.x & 63U, groups = img.width / 32U;
-    const float* deltas = img.deltas_of(row);
-    const int32_t* sums = img.sums_of(row);
+    const auto* deltas = in_global<float>(img.deltas_of(row));
+    const auto* sums = in_global<int32_t>(img.sums_of(row));
     float acc = 0.0F, vd = 0.0F, vf = 0.0F;
+    int32_t vs = 0;
+    // the per-lane group deltas / sums: groups 8 b .. 8 b + 63; the first ones are asked for in front of the first stages (behind them, the
+    // first stage's wait would be for all of them). Not of Q5_K rows, whose kernel would pass 128 registers (16 rows of 2048 / 768 / 128 103.1 -> 106.1 us)
+    const auto refill = [&](uint32_t b) {
+        const uint32_t g = b * 8U + lane;
+        vd = g < groups ? deltas[g] : 0.0F;
+        vs = g < groups ? sums[g] : 0;
+    };
+    if (!Q5K) refill(0U);
 #pragma unroll
     for (int s = 0; s < DEPTH - 1; ++s)
         if (static_cast<uint32_t>(s) < blocks) source.start(slots[s]);
@@ -138,14 +147,11 @@ __device__ __forceinline__ float sweep_quads(lds_u8* const (&slots)[DEPTH], Quad
         for (int s = 0; s < DEPTH; ++s) {
             const uint32_t b = b0 + s;
             if (b < blocks) {
-                if ((b & 7U) == 0) {           // refill the per-lane group deltas / sums: groups 8 b .. 8 b + 63
-                    const uint32_t g = b * 8U + lane;
-                    vd = g < groups ? deltas[g] : 0.0F;
-                    vf = g < groups ? static_cast<float>(sums[g]) : 0.0F;
-                }
+                if ((Q5K || b != 0U) && (b & 7U) == 0) refill(b);
                 const uint32_t last = b + DEPTH - 1U < blocks ? b + DEPTH - 1U : blocks;
                 wait_stages_ahead<kQuadCopies>(last - 1U - b);
                 if (b + DEPTH - 1U < blocks) source.start(slots[(s + DEPTH - 1) % DEPTH]);
+                if ((b & 7U) == 0) vf = static_cast<float>(vs);
                 if (Q5K) quad_block_compute_q5k(slots[s], b, vd, vf, acc);
                 else quad_block_compute(slots[s], b, vd, vf, acc);
             }

@@ -146,6 +146,15 @@ struct RowsK : mi355_moe_rows {
     __device__ __forceinline__ float* h_deltas_of(uint32_t i) const { return const_cast<float*>(h.deltas_of(i)); }
     __device__ __forceinline__ int32_t* h_sums_of(uint32_t i) const { return const_cast<int32_t*>(h.sums_of(i)); }
 };
+// The views of a whole-layer launch, which are dense ones always (no table of addresses, no job list, one image a row): said to the compiler, which otherwise
+// joins the paths of every look-up behind a wait for all that is in flight, a stage's copies among it, and reads through flat addresses.
+__device__ __forceinline__ RowsK dense_views(RowsK r) {
+    r.in.table = r.h.table = nullptr;
+    r.in.per_row = r.h.per_row = 1U;
+    r.assignments = nullptr;
+    r.union_plan = nullptr;
+    return r;
+}
 // One work item of an expert launch: assignments [begin, end) of the plan order belong to expert e. Without a plan
 // (plan == nullptr) item i is assignment i alone, its expert read from the routes (or from the job's list): the single-row
 // forms of the reference entry points (include/strix/hip_moe_q4k_a8_probe.hpp:12, include/strix/hip_moe_a8_down.hpp:11-30) and
@@ -280,6 +289,10 @@ __device__ __forceinline__ void q4k_factors(const u32x4& hd, uint32_t& sc, uint3
     }
 }
 
+// An address of an A8 image as one of global memory. It may come out of a table, so the compiler cannot tell, and a flat load counts as an LDS access
+// as well: a wave that awaits it drains its copy ring and its LDS reads.
+template <class T> __device__ __forceinline__ const __attribute__((address_space(1))) T* in_global(const void* p) { return (const __attribute__((address_space(1))) T*)p; }
+
 // Uniform view of the NA activation rows of one sweep (row bases, wave-uniform).
 template <int NA>
 struct ActRows {
@@ -387,8 +400,8 @@ __device__ __forceinline__ void sweep_rows(lds_u8* const (&slots)[DEPTH], StageS
                     const uint32_t g = b * 8U + lane;
 #pragma unroll
                     for (int a = 0; a < NA; ++a) {
-                        vd[a] = g < act.groups ? act.deltas[a][g] : 0.0F;
-                        vf[a] = g < act.groups ? static_cast<float>(act.sums[a][g]) : 0.0F;
+                        vd[a] = g < act.groups ? in_global<float>(act.deltas[a])[g] : 0.0F;
+                        vf[a] = g < act.groups ? static_cast<float>(in_global<int32_t>(act.sums[a])[g]) : 0.0F;
                     }
                 }
                 // started so far: stages 0 .. min(blocks, b + DEPTH - 1) - 1; stage b must have landed

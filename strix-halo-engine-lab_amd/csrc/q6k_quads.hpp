@@ -59,8 +59,8 @@ __device__ __forceinline__ void q6k_part(Q6kPart& w, const uint8_t* block, uint3
 __device__ __forceinline__ float q6k_part_term(const Q6kPart& w, const int8_t* codes, const float* deltas, uint32_t half, uint32_t t) {
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
     typedef float f32x2_g __attribute__((ext_vector_type(2)));
-    const __attribute__((address_space(1))) u32x4_g* from = (const __attribute__((address_space(1))) u32x4_g*)(codes + 128U * half + 16U * t);
-    const f32x2_g delta = *(const __attribute__((address_space(1))) f32x2_g*)(deltas + 4U * half + 2U * t);
+    const auto* from = in_global<u32x4_g>(codes + 128U * half + 16U * t);
+    const f32x2_g delta = *in_global<f32x2_g>(deltas + 4U * half + 2U * t);
     int part[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4U; ++k) {
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void down_q6k_kernel(mi355_moe_weights w, Rows
             h_codes[a] = r.h.codes_of(src[a]);
             h_deltas[a] = r.h.deltas_of(src[a]);
         }
-#pragma unroll 1
+#pragma unroll 2
         for (uint32_t b = 0; b < blocks; ++b) {
             Q6kPart part;
             q6k_part(part, wrow + static_cast<size_t>(b) * kQ6kBlock, half, odd);

@@ -521,6 +521,8 @@ constexpr uint32_t kFrontRunWaves = 1024;      // sweeps from which on rows of m
 // super-block of each row per stage: a contiguous stage of 48 blocks works as long as one of 64, and its chain runs over the lanes in as many steps
 // as a row has blocks. Layers, contiguous -> block by block: hidden 1280, 1, 4, 12 rows 30.2, 33.3, 53.7 -> 26.4, 29.6, 44.9 us; 1536 30.5, 34.2 -> 27.2, 31.1; 1792
 // 34.6, 41.9 -> 31.8, 39.7; 2304, 1 row 38.3 -> 30.4; 6144, 1 row (640 sweeps) 97.5 -> 79.3; 4096, 1, 2, 4 rows (384, 512, 1536 sweeps) 53.9, 54.4, 76.9 -> 48.5, 49.8, 81.0.
+// REPAIR (an assignment that a side block sweeps again, a rare one, by a single wave): block by block whatever the shape, which keeps the registers of the launch's main path.
+template <bool REPAIR = false>
 __device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r, uint32_t e, uint32_t grp, uint32_t at, uint32_t assignments) {
     const size_t base = static_cast<size_t>(e) * w.gate_expert_stride + static_cast<size_t>(grp * 32U) * w.gate_row_stride;
     const uint8_t* gate = w.gate + base;
@@ -528,7 +530,7 @@ __device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const m
     const uint32_t B = w.hidden / 256U;
     const BlockLanes g = block_lanes(B, 32U);
     const bool runs = g.used == 64U && (B <= 8U || assignments * (w.ffn / 32U) > kFrontRunWaves);
-    if (runs && w.gate_row_stride == static_cast<uint64_t>(B) * kQ4kBlock && block_lanes_ok(B, 32U)) {
+    if (!REPAIR && runs && w.gate_row_stride == static_cast<uint64_t>(B) * kQ4kBlock && block_lanes_ok(B, 32U)) {
         const uint32_t half = 32U / g.R;                  // stages of the gate rows, then as many of the up rows
         float value[1];
         const auto stage_base = [&](uint32_t s) { return s < half ? gate + static_cast<size_t>(s) * g.stage_bytes : up + static_cast<size_t>(s - half) * g.stage_bytes; };
@@ -656,12 +658,13 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             continue;
         }
         if (lane == 0) __hip_atomic_store(&r.awords[at], groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (uint32_t grp = 0; grp < groups; ++grp) front_project(slots, w, r, e, grp, at, assignments);
+        for (uint32_t grp = 0; grp < groups; ++grp) front_project<true>(slots, w, r, e, grp, at, assignments);
     }
 }
 
 template <int KIND>
-__global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, RouteArgs a, FrontBlocks nb) {
+__global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, RouteArgs a, FrontBlocks nb) {
+    const RowsK r = dense_views(views);
     // exactly 20,480 bytes of LDS: eight workgroups fill a compute unit's 160 KB (one more byte and only seven fit)
     __shared__ __attribute__((aligned(16))) uint8_t ring0[kSideSlotBytes];
     __shared__ __attribute__((aligned(16))) uint8_t ring1[kSideSlotBytes];
@@ -1099,7 +1102,8 @@ __device__ __forceinline__ void slot_fold(const SlotFold& f, const mi355_moe_wei
 // in assignment order); the waves leave their 64 values in LDS and wave 0 folds them exactly as merge_kernel does. Only
 // waves of one workgroup exchange data, so nothing depends on the visibility of another workgroup's stores.
 // Reference: src/cpu/core/routed_expert.cpp:429-447, src/moe_a8_down_contract.cpp:146, include/strix/moe/combine.hpp:36-59.
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     // the two ring slots are separate LDS objects: the compiler then knows that a copy into one never touches the other and lets
     // the reads of the landed slot go ahead while the next stage's copy is in flight (as slots of one array it waited for both)
     __shared__ __attribute__((aligned(16))) uint8_t ring_even[kDownMergeSlots][slot_bytes(1)];
@@ -1139,7 +1143,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_kernel(mi355_
 // same bytes in 11.8 us against 14.4 us), the block terms meet in LDS in block order and lane = row adds them in ascending order.
 // (Fold behind the barrier: asked for at the start, in front of the item, 1, 8, 16 rows of hidden 2048 / ffn 768 27.7, 45.9, 73.5 -> 28.2, 46.2, 73.9 us.)
 template <int B>
-__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     // (the two ring slots are separate LDS objects, as in down_merge_kernel)
     __shared__ __attribute__((aligned(16))) uint8_t ring_even[kDownMergeSlots][kFlatStageBytes];
     __shared__ __attribute__((aligned(16))) uint8_t ring_odd[kDownMergeSlots][kFlatStageBytes];
@@ -1212,7 +1217,8 @@ __global__ __launch_bounds__(64 * kDownMergeSlots) void down_merge_flat_kernel(m
 // output columns), wave k sweeps the 16 down rows of the expert in slot k (lane = (row, pair)), the slots' values meet in LDS
 // and the first sixteen lanes of wave 0 fold them as merge_kernel does. One launch instead of two for one to six rows.
 template <int DEPTH, uint32_t SLOTS>
-__global__ __launch_bounds__(64 * SLOTS) void down_merge_quad_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_quad_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     __shared__ __attribute__((aligned(16))) uint8_t mq0[SLOTS][kQuadSlotBytes];
     __shared__ __attribute__((aligned(16))) uint8_t mq1[SLOTS][kQuadSlotBytes];
     __shared__ __attribute__((aligned(16))) uint8_t mq2[DEPTH > 2 ? SLOTS : 1][DEPTH > 2 ? kQuadSlotBytes : 16];
@@ -1249,7 +1255,8 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_quad_kernel(mi355_moe_w
 // src/cpu/core/routed_expert.cpp:110-126): the workgroup of (row, 16 columns), wave k = the expert in slot k, each wave with
 // the copy ring, the lane layout and the chain order of down_q51_ring_kernel for its one assignment.
 template <int DEPTH, uint32_t SLOTS>
-__global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
     typedef const __attribute__((address_space(3))) float lds_f32c;
     typedef const __attribute__((address_space(3))) int32_t lds_i32c;
@@ -1351,7 +1358,8 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_we
 // ffn 768 / 128 experts top-8, 1, 8, 16 rows 25.7, 57.8, 92.1 -> 25.1, 54.3, 85.9 us; 5 of them with the norm and an always-on expert 57.3 -> 53.6; 4 rows of 4096 /
 // 1536 / 64 103.4 -> 94.2; 6 rows of 3072 / 2304 / 32 top-4 100.6 -> 87.8.
 template <uint32_t SLOTS>
-__global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, p = lane & 3U, half = p >> 1, odd = p & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
@@ -1390,10 +1398,9 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_we
 // (The image of h by global loads - from a pointer that may come out of a table they were flat ones, which wait for the LDS as well -, three groups of a chain's asked
 // for together, two in the wider workgroups: 8, 16 rows of 2048 / 768 / 128 57.5, 90.1 -> 56.3, 88.7 us, 4 of 4096 / 1536 / 64 98.9 -> 96.6.)
 template <uint32_t SLOTS>
-__global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK r, uint32_t assignments, uint32_t form) {
+__global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
+    const RowsK r = dense_views(views);
     typedef uint32_t u32x4_g __attribute__((ext_vector_type(4)));
-    typedef const __attribute__((address_space(1))) u32x4_g global_u32x4;
-    typedef const __attribute__((address_space(1))) float global_f32;
     __shared__ float slot_value[SLOTS][16];
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63U, j = lane & 3U, odd = j & 1U, rr = lane >> 2, row = blockIdx.y;
     const uint32_t o = blockIdx.x * 16U + rr;
@@ -1416,13 +1423,13 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q8_0_kernel(mi355_moe_w
             float d, m;
             uint32_t q[8];
             load_group_block<0>(wrow + static_cast<size_t>(c) * (4U * 34U), odd, d, m, q);
-            const global_u32x4* codes = (const global_u32x4*)(h_codes + 32U * g);
+            const auto* codes = in_global<u32x4_g>(h_codes + 32U * g);
             const u32x4_g c_lo = codes[0], c_hi = codes[1];
             const uint32_t cw[8] = {c_lo.x, c_lo.y, c_lo.z, c_lo.w, c_hi.x, c_hi.y, c_hi.z, c_hi.w};
             int dot = 0;
 #pragma unroll
             for (int i = 0; i < 8; ++i) dot = __builtin_amdgcn_sdot4(static_cast<int>(q[i]), static_cast<int>(cw[i]), dot, false);
-            chain = chain + ((((const global_f32*)h_deltas)[g]) * (d * static_cast<float>(dot)));
+            chain = chain + (in_global<float>(h_deltas)[g] * (d * static_cast<float>(dot)));
         }
         value = chain;
         value = value + xor1_f(value);          // chain0 + chain1 | chain2 + chain3
