@@ -9,8 +9,10 @@
 // eight rows read different banks. Lane (i, q) then reads feature 4 t + q of row i and of expert i for step t of
 // the chain with one 32-bit LDS read each (16-byte reads and a transpose between the lanes cost 16 half-rate vector operations per
 // eight steps, which the fp32 matrix instruction does not overlap with: 22 us a launch). Bound by the chain, 13.4 ns per 4 features.
-// Measured at hidden 2048, 128 experts: 40 and 1000 rows 100 -> 15 and 17 us; 4096 rows, hidden 4096, 256 experts: 221 -> 110 us (lane-wise fma
-// chains on tiles of 64 rows x 64 experts before, of which a batch of 40 rows gave two workgroups).
+// Measured with the selection behind it, LDS reads in front of a block's products and address arithmetic between them -> reads between the
+// products, vector operations in front: hidden 2048, 128 experts, 40 | 333 | 1000 rows 19.0 | 19.3 | 20.3 -> 17.1 | 17.4 | 18.3 us; 17 rows of hidden 6144, 160 experts
+// 42.3 -> 36.9; 100 of 4096, 64 experts 29.8 -> 26.0; 4096 rows of 4096, 256 experts 110 -> 98. (Lane-wise fma chains on tiles of 64 rows x 64
+// experts, of which a batch of 40 rows gives two workgroups, take 100 us for the first.)
 #pragma once
 #include "route_wave.hpp"
 
@@ -24,6 +26,11 @@ template <int KIND, int DEPTH> constexpr uint32_t route_ring_bytes() { return 10
 // 16 bytes per lane, global -> LDS (lane l lands at lds_at + 16 l), as a plain instruction: arrival is awaited by count
 __device__ __forceinline__ void route_copy16(const void* src, uint32_t lds_at) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_at), "v"(src) : "memory", "m0");
+}
+
+// the same from a base of the wave and a byte offset per lane
+__device__ __forceinline__ void route_copy16_at(uint64_t base, uint32_t offset, uint32_t lds_at) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_at), "v"(offset), "s"(base) : "memory", "m0");
 }
 
 template <int KIND, int DEPTH, uint32_t WAVES>
@@ -40,20 +47,32 @@ __global__ __launch_bounds__(64 * WAVES) void route_mma_kernel(RouteArgs a) {
     const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte*)ring)) + wave * route_ring_bytes<KIND, DEPTH>());
     // copier role: lane l of a copy of eight 128-byte rows (fp16 / bf16 activations: sixteen 64-byte rows)
     const auto row_of = [&](uint32_t r) { return a.x + (r0 + r < a.rows ? r0 + r : a.rows - 1U) * a.x_stride; };
-    const auto expert_of = [&](uint32_t e) { return a.wr + static_cast<size_t>(e0 + e < a.p.experts ? e0 + e : a.p.experts - 1U) * a.hidden; };
-    const uint8_t* src[COPIES];
-    const uint32_t piece8 = (lane & 7U) ^ (lane >> 3);
-    src[0] = reinterpret_cast<const uint8_t*>(expert_of(lane >> 3)) + 16U * piece8;
-    src[1] = reinterpret_cast<const uint8_t*>(expert_of(8U + (lane >> 3))) + 16U * piece8;
+    const uint32_t piece8 = (lane & 7U) ^ (lane >> 3), last = a.p.experts - 1U - e0;
+    // experts: the wave's first one, and bytes from there (sixteen rows of at most 64 KB)
+    const uint64_t w_base = reinterpret_cast<uint64_t>(a.wr + static_cast<size_t>(e0) * a.hidden);
+    const uint32_t w_off[2] = {((lane >> 3) < last ? lane >> 3 : last) * 4U * a.hidden + 16U * piece8, (8U + (lane >> 3) < last ? 8U + (lane >> 3) : last) * 4U * a.hidden + 16U * piece8};
+    const uint8_t* x_src[COPIES - 2U];
     if constexpr (KIND == 0) {
-        src[2] = row_of(lane >> 3) + 16U * piece8;
-        src[3] = row_of(8U + (lane >> 3)) + 16U * piece8;
-    } else src[2] = row_of(lane >> 2) + 16U * ((lane & 3U) ^ ((lane >> 3) & 3U));
+        x_src[0] = row_of(lane >> 3) + 16U * piece8;
+        x_src[1] = row_of(8U + (lane >> 3)) + 16U * piece8;
+    } else x_src[0] = row_of(lane >> 2) + 16U * ((lane & 3U) ^ ((lane >> 3) & 3U));
     const uint32_t blocks = a.hidden / 32U;
-    const auto issue = [&](uint32_t at) {               // (past the end: the last block again, never read; the counts stay the same)
-        const uint32_t k = 32U * (at < blocks ? at : blocks - 1U), slot = __builtin_amdgcn_readfirstlane(base + (at % DEPTH) * SLOT);
+    // copies of block `at` (past the end: the last block again, never read; the counts stay the same)
+    const auto issue_weights = [&](uint32_t at) __attribute__((always_inline)) {
+        const uint32_t k = at < blocks ? at : blocks - 1U, slot = __builtin_amdgcn_readfirstlane(base + (at % DEPTH) * SLOT);
 #pragma unroll
-        for (uint32_t c = 0; c < COPIES; ++c) route_copy16(src[c] + (c < 2U || KIND == 0 ? 4U : 2U) * k, slot + 1024U * c);
+        for (uint32_t c = 0; c < 2U; ++c) route_copy16_at(w_base + 128ULL * k, w_off[c], slot + 1024U * c);
+    };
+    const uint8_t* x_next[COPIES - 2U];
+    const auto place_rows = [&](uint32_t at) __attribute__((always_inline)) {
+        const uint32_t k = at < blocks ? at : blocks - 1U;
+#pragma unroll
+        for (uint32_t c = 0; c < COPIES - 2U; ++c) x_next[c] = x_src[c] + (KIND == 0 ? 128U : 64U) * k;
+    };
+    const auto issue_rows = [&](uint32_t at) __attribute__((always_inline)) {
+        const uint32_t slot = __builtin_amdgcn_readfirstlane(base + (at % DEPTH) * SLOT);
+#pragma unroll
+        for (uint32_t c = 0; c < COPIES - 2U; ++c) route_copy16(x_next[c], slot + 2048U + 1024U * c);
     };
     // step t of half h: LDS bytes of the lane's expert and row value inside a slot
     uint32_t w_at[8], x_at[8];
@@ -64,33 +83,47 @@ __global__ __launch_bounds__(64 * WAVES) void route_mma_kernel(RouteArgs a) {
         else x_at[t] = base + 2048U + 64U * i + 16U * ((t >> 1) ^ ((i >> 1) & 3U)) + 2U * ((4U * t + q) & 7U);
     }
     struct Block { float w[8]; uint32_t x[8]; };
-    const auto read = [&](Block& b, uint32_t slot) {
+    const auto read = [&](Block& b, uint32_t slot, uint32_t from, uint32_t to) __attribute__((always_inline)) {
 #pragma unroll
-        for (uint32_t t = 0; t < 8U; ++t) {
+        for (uint32_t t = from; t < to; ++t) {
             b.w[t] = *(lds_f32*)(uintptr_t)(w_at[t] + slot * SLOT);
             if constexpr (KIND == 0) b.x[t] = *(lds_u32*)(uintptr_t)(x_at[t] + slot * SLOT);
             else b.x[t] = *(lds_u16*)(uintptr_t)(x_at[t] + slot * SLOT);
         }
     };
     f32x4 acc = {0.0F, 0.0F, 0.0F, 0.0F};
-    const auto chain = [&](const Block& b) {
 #pragma unroll
-        for (uint32_t t = 0; t < 8U; ++t) {
-            const float x = KIND == 0 ? f_of(b.x[t]) : KIND == 1 ? half_bits_to_float(b.x[t]) : f_of(b.x[t] << 16);
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x, b.w[t], acc, 0, 0, 0);
-        }
-    };
-#pragma unroll
-    for (uint32_t s = 0; s < DEPTH; ++s) issue(s);
+    for (uint32_t s = 0; s < DEPTH; ++s) { issue_weights(s); place_rows(s); issue_rows(s); }
     Block now, next;
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES * (DEPTH - 1U)) : "memory");
-    read(now, 0);
-    const auto step = [&](uint32_t at, uint32_t s, Block& here, Block& ahead) {
+    read(now, 0, 0U, 8U);
+    // The vector ALU stands still while an fp32 product runs, and each change from one to the other costs 17 cycles (chain alone 32 cycles a product;
+    // with one vector operation in every gap 49, with four 72; with eight conversions in front of eight products 38): a block's vector
+    // operations come first, in one run. LDS reads, copies and scalar operations go on beside a product (two reads in every gap 34,
+    // sixteen in front of eight products 53), so they stand in the gaps.
+    const auto step = [&](uint32_t at, uint32_t s, const Block& here, Block& ahead) __attribute__((always_inline)) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // this block is in registers: its slot is free
-        issue(at + DEPTH);
-        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES * (DEPTH - 1U)) : "memory");
-        read(ahead, (s + 1U) % DEPTH);
-        chain(here);
+        float x[8];
+#pragma unroll
+        for (uint32_t t = 0; t < 8U; ++t) {
+            x[t] = KIND == 0 ? f_of(here.x[t]) : KIND == 1 ? half_bits_to_float(here.x[t]) : f_of(here.x[t] << 16);
+            asm volatile("" : "+v"(x[t]));
+        }
+        place_rows(at + DEPTH);
+#pragma unroll
+        for (uint32_t c = 0; c < COPIES - 2U; ++c) asm volatile("" : "+v"(x_next[c]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t t = 0; t < 8U; ++t) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t], here.w[t], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t == 0U) issue_weights(at + DEPTH);
+            else if (t == 1U) {
+                issue_rows(at + DEPTH);
+                asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES * (DEPTH - 1U)) : "memory");
+            } else if (t < 6U) read(ahead, (s + 1U) % DEPTH, 2U * t - 4U, 2U * t - 2U);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
     for (uint32_t at = 0; at < blocks; at += DEPTH) {               // (slot s of a turn holds block at + s: the offsets are constants)
 #pragma unroll
@@ -112,8 +145,8 @@ __global__ __launch_bounds__(64 * WAVES) void route_mma_kernel(RouteArgs a) {
 }
 
 // While a wave's workgroup finds room beside two others (fp32 rows: beside one), a ring of sixteen blocks (48 KB, 64 KB): a block is chained in
-// 107 ns, so eight are 0.9 us ahead, less than a cold fetch takes (hidden 2048, 128 experts, 40 | 333 rows 16.7 | 15.9 -> 14.7 | 14.4 us; hidden 6144,
-// 160 experts, 17 rows 39.3 -> 36.5; 1008 waves of hidden 2048 17.3 | 30.0). Else four waves a workgroup: a ring of eight where one workgroup per
+// 125 ns, so eight are 1 us ahead, less than a cold fetch takes (hidden 2048, 128 experts, 40 | 333 rows 16.7 | 15.9 -> 14.7 | 14.4 us; hidden 6144,
+// 160 experts, 17 rows 39.3 -> 36.5; 1008 waves of hidden 2048 17.3 | 30.0, with a block in 140 ns). Else four waves a workgroup: a ring of eight where one workgroup per
 // compute unit holds the launch, of four (two or three workgroups share a unit) beyond.
 inline void launch_route_mma(const RouteArgs& a, uint32_t compute_units, hipStream_t st) {
     const uint32_t rows = (a.rows + 15U) / 16U, experts = (a.p.experts + 15U) / 16U;
