@@ -144,7 +144,124 @@ __global__ __launch_bounds__(64 * WAVES) void route_mma_kernel(RouteArgs a) {
     }
 }
 
-// While a wave's workgroup finds room beside two others (fp32 rows: beside one), a ring of sixteen blocks (48 KB, 64 KB): a block is chained in
+// The same with a second wave that brings the operands: it starts the copies, awaits them, widens fp16 / bf16 rows to fp32 in LDS, four blocks ahead, and meets the
+// chaining wave once for those. That one has no vector operation between its products: 35.4 cycles each, where it does everything
+// itself 46 (meeting once a block the second wave is the slower one of the two with rows to widen: 43). Logits and selection, one wave -> two: 40 fp16 | fp32 rows of
+// hidden 2048, 128 experts 17.0 | 17.9 -> 14.5 | 14.3 us, 333 rows 17.3 -> 14.8; 17 rows of 6144, 160 experts 36.8 -> 29.2; 100 of 4096, 64 experts 26.1 -> 21.0.
+template <int KIND, int DEPTH>
+__global__ __launch_bounds__(128) void route_mma_pair_kernel(RouteArgs a) {
+    constexpr uint32_t COPIES = route_block_copies<KIND>(), SLOT = 1024U * COPIES, TURN = 4U, WIDENED = 2U * TURN;       // blocks from meeting to meeting, blocks of widened rows
+    static_assert(DEPTH % WIDENED == 0, "a block's places follow from its place in the ring");
+    __shared__ __attribute__((aligned(16))) uint8_t ring[route_ring_bytes<KIND, DEPTH>() + (KIND == 0 ? 0U : 2048U * WIDENED)];
+    typedef __attribute__((address_space(3))) uint8_t lds_byte;
+    typedef const __attribute__((address_space(3))) float lds_f32;
+    typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+    typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+    const uint32_t lane = threadIdx.x & 63U, i = lane & 15U, q = lane >> 4;
+    const uint32_t r0 = blockIdx.y * 16U, e0 = blockIdx.x * 16U, blocks = a.hidden / 32U;
+    const uint32_t base = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_byte*)ring)));
+    const uint32_t widened = base + route_ring_bytes<KIND, DEPTH>();
+    const auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) != 0U) {
+        const auto row_of = [&](uint32_t r) { return a.x + (r0 + r < a.rows ? r0 + r : a.rows - 1U) * a.x_stride; };
+        const auto expert_of = [&](uint32_t e) { return reinterpret_cast<const uint8_t*>(a.wr + static_cast<size_t>(e0 + e < a.p.experts ? e0 + e : a.p.experts - 1U) * a.hidden); };
+        const uint32_t piece8 = (lane & 7U) ^ (lane >> 3), row = lane >> 2, piece = lane & 3U;
+        const uint8_t* src[COPIES];
+        src[0] = expert_of(lane >> 3) + 16U * piece8;
+        src[1] = expert_of(8U + (lane >> 3)) + 16U * piece8;
+        if constexpr (KIND == 0) {
+            src[2] = row_of(lane >> 3) + 16U * piece8;
+            src[3] = row_of(8U + (lane >> 3)) + 16U * piece8;
+        } else src[2] = row_of(row) + 16U * piece;
+        const auto issue = [&](uint32_t at) {           // (past the end: the last block again, never read; the counts stay the same)
+            const uint32_t k = at < blocks ? at : blocks - 1U, slot = __builtin_amdgcn_readfirstlane(base + (at % DEPTH) * SLOT);
+#pragma unroll
+            for (uint32_t c = 0; c < COPIES; ++c) route_copy16(src[c] + (c < 2U || KIND == 0 ? 128U : 64U) * k, slot + 1024U * c);
+        };
+        const auto widen = [&](uint32_t at) {           // blocks at .. at + TURN - 1
+            if constexpr (KIND != 0) {
+                u32x4 raw[TURN];
+#pragma unroll
+                for (uint32_t b = 0; b < TURN; ++b) raw[b] = *(lds_u32x4*)(uintptr_t)(base + ((at + b) % DEPTH) * SLOT + 2048U + 16U * lane);
+#pragma unroll
+                for (uint32_t b = 0; b < TURN; ++b) {
+                    f32x4 f[2];
+#pragma unroll
+                    for (uint32_t n = 0; n < 4U; ++n) {
+                        f[n >> 1][2U * (n & 1U)] = KIND == 1 ? half_bits_to_float(raw[b][n] & 0xffffU) : f_of(raw[b][n] << 16);
+                        f[n >> 1][2U * (n & 1U) + 1U] = KIND == 1 ? half_bits_to_float(raw[b][n] >> 16) : f_of(raw[b][n] & 0xffff0000U);
+                    }
+                    const uint32_t to = widened + 2048U * ((at + b) % WIDENED) + 128U * row;
+#pragma unroll
+                    for (uint32_t n = 0; n < 2U; ++n) *(lds_f32x4*)(uintptr_t)(to + 16U * ((2U * piece + n) ^ (row & 7U))) = f[n];
+                }
+            }
+        };
+        for (uint32_t s = 0; s < DEPTH; ++s) issue(s);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES * (DEPTH - TURN)) : "memory");
+        widen(0);
+        meet();
+        for (uint32_t at = 0; at + TURN <= blocks; at += TURN) {
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"(COPIES * (DEPTH - 2U * TURN)) : "memory");
+            widen(at + TURN);
+            meet();                                     // blocks at .. at + 3 are in the chaining wave's registers or behind them, the next four in LDS
+#pragma unroll
+            for (uint32_t b = 0; b < TURN; ++b) issue(at + DEPTH + b);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // no copy may land after the workgroup has given its LDS back
+        return;
+    }
+    // step t: LDS bytes of the lane's expert and row value (feature 4 t + q) inside a slot
+    uint32_t w_at[8], x_at[8];
+#pragma unroll
+    for (uint32_t t = 0; t < 8U; ++t) {
+        const uint32_t in = 128U * i + 16U * (t ^ (i & 7U)) + 4U * q;
+        w_at[t] = base + in;
+        x_at[t] = (KIND == 0 ? base + 2048U : widened) + in;
+    }
+    struct Block { float w[8], x[8]; };
+    const auto read = [&](Block& b, uint32_t s, uint32_t from, uint32_t to) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t t = from; t < to; ++t) {
+            b.w[t] = *(lds_f32*)(uintptr_t)(w_at[t] + s * SLOT);
+            b.x[t] = *(lds_f32*)(uintptr_t)(x_at[t] + (KIND == 0 ? s * SLOT : (s % WIDENED) * 2048U));
+        }
+    };
+    f32x4 acc = {0.0F, 0.0F, 0.0F, 0.0F};
+    Block now, next;
+    const auto step = [&](uint32_t s, const Block& here, Block& ahead) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t t = 0; t < 8U; ++t) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(here.x[t], here.w[t], acc, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t == 0U && s % TURN == TURN - 1U) meet();
+            if (t > 0U && t < 5U) read(ahead, (s + 1U) % DEPTH, 2U * t - 2U, 2U * t);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    meet();
+    read(now, 0, 0U, 8U);
+    for (uint32_t at = 0; at < blocks; at += DEPTH) {               // (slot s of a turn holds block at + s: the offsets are constants)
+#pragma unroll
+        for (uint32_t s = 0; s < DEPTH; s += 2U) {
+            if (at + s < blocks) step(s, now, next);
+            if (at + s + 1U < blocks) step(s + 1U, next, now);
+        }
+    }
+    const uint32_t e = e0 + i;
+    if (e >= a.p.experts) return;
+    const float bias = a.bias ? a.bias[e] : 0.0F;
+#pragma unroll
+    for (uint32_t t = 0; t < 4U; ++t) {
+        const uint32_t r = r0 + 4U * q + t;
+        if (r < a.rows) a.scores[static_cast<size_t>(r) * a.p.experts + e] = a.bias ? acc[t] + bias : acc[t];
+    }
+}
+
+// Two waves a tile while their workgroup finds room beside another (1000 rows of hidden 2048, 128 experts, 504 tiles: one wave 17.7, two 17.4 us; 1500 rows 18.8 | 30).
+// Past that, while a wave's workgroup finds room beside two others, a ring of sixteen blocks (48 KB; of fp32 rows 64 KB, which leaves no room for a third): a block is chained in
 // 125 ns, so eight are 1 us ahead, less than a cold fetch takes (hidden 2048, 128 experts, 40 | 333 rows 16.7 | 15.9 -> 14.7 | 14.4 us; hidden 6144,
 // 160 experts, 17 rows 39.3 -> 36.5; 1008 waves of hidden 2048 17.3 | 30.0, with a block in 140 ns). Else four waves a workgroup: a ring of eight where one workgroup per
 // compute unit holds the launch, of four (two or three workgroups share a unit) beyond.
@@ -155,11 +272,17 @@ inline void launch_route_mma(const RouteArgs& a, uint32_t compute_units, hipStre
         constexpr int DEPTH = decltype(depth)::value;
         constexpr uint32_t WAVES = decltype(per)::value;
         const dim3 grid((experts + WAVES - 1U) / WAVES, rows);
-        if (a.kind == MI355_INPUT_F32) route_mma_kernel<0, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
-        else if (a.kind == MI355_INPUT_F16) route_mma_kernel<1, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
+        if (a.kind == MI355_INPUT_F32) {
+            if constexpr (DEPTH < 16) route_mma_kernel<0, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
+        } else if (a.kind == MI355_INPUT_F16) route_mma_kernel<1, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
         else route_mma_kernel<2, DEPTH, WAVES><<<grid, 64U * WAVES, 0, st>>>(a);
     };
-    if (waves <= (a.kind == MI355_INPUT_F32 ? 2U : 3U) * units) launch(std::integral_constant<int, 16>{}, std::integral_constant<uint32_t, 1U>{});
+    if (waves <= 2U * units) {
+        const dim3 grid(experts, rows);
+        if (a.kind == MI355_INPUT_F32) route_mma_pair_kernel<0, 16><<<grid, 128, 0, st>>>(a);
+        else if (a.kind == MI355_INPUT_F16) route_mma_pair_kernel<1, 16><<<grid, 128, 0, st>>>(a);
+        else route_mma_pair_kernel<2, 16><<<grid, 128, 0, st>>>(a);
+    } else if (a.kind != MI355_INPUT_F32 && waves <= 3U * units) launch(std::integral_constant<int, 16>{}, std::integral_constant<uint32_t, 1U>{});
     else if (static_cast<uint64_t>((experts + 3U) / 4U) * rows <= units) launch(std::integral_constant<int, 8>{}, std::integral_constant<uint32_t, 4U>{});
     else launch(std::integral_constant<int, 4>{}, std::integral_constant<uint32_t, 4U>{});
 }

@@ -72,3 +72,20 @@ def test_rings_of_a_batch(strix, rows, experts, hidden, dtype):
     for r in (0, rows // 2, rows - 16):
         for got, want in zip(batch, strix.route(x[r:r + 16].contiguous(), w, 4)):
             assert torch.equal(got[r:r + 16].view(torch.int32), want.view(torch.int32)), r
+
+
+# decode rows past 2048 features, whose logits alone run on the matrix cores too, in two waves a tile: blocks around the meetings of the waves (every
+# four blocks) and the ring's end (sixteen)
+@pytest.mark.parametrize("rows,experts,hidden,top_k", [(1, 16, 2080, 2), (7, 33, 2112, 4), (16, 130, 2144, 8), (15, 20, 2176, 4), (9, 64, 2560, 8), (16, 17, 6144, 8), (3, 5, 16384, 2)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_wide_decode_rows(strix, rows, experts, hidden, top_k, dtype):
+    gen = torch.Generator().manual_seed(rows + experts + hidden)
+    x = torch.randn((rows, hidden), generator=gen).to(dtype)
+    w = torch.randn((experts, hidden), generator=gen) * 0.05
+    x[0, ::3] *= 2.0 ** -20
+    w[0] *= 2.0 ** -120
+    bias = torch.randn(experts, generator=gen) if experts % 2 else None
+    ids, weights, scores = strix.route(x.cuda(), w.cuda(), top_k, bias=None if bias is None else bias.cuda())
+    ids_ref, w_ref, s_ref, _ = orc.route(x.float().numpy(), w.numpy(), top_k, bias=None if bias is None else bias.numpy())
+    assert np.array_equal(bits(scores.cpu().numpy()), bits(s_ref))
+    assert np.array_equal(ids.cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(bits(weights.cpu().numpy()), bits(w_ref))
