@@ -10,15 +10,15 @@
 // twice an add); the factors scale * delta of two such tiles are one v_mfma_f32_32x32x1_2b_f32 (products rounded once, +0 added); then
 // a multiply and an add. Bound by those three vector operations and the two matrix operations they wait for.
 // Memory: per stage the KS groups of one lane class in two chunks of 32 groups, for every row of the tile: a thread copies one weight
-// block (nine dwords around its 34 bytes, shifted into place) and one or two activation groups through registers into one of two LDS
+// block (nine dwords around its 34 bytes, shifted into place; 777 rows of 3104 x 5000, rows aligned to 2 bytes, 133 us by 16-bit loads, 118) and one or two activation groups through registers into one of two LDS
 // buffers while the other is multiplied; rows are pitched by 16 bytes so that eight neighbouring rows read different banks.
 // What bounds it now, at 4096 x 4096 and 64 x 64 tiles: a stage takes 0.8 us of products (two waves per SIMD, 192 full-rate vector
-// operations and six matrix operations each) and 0.55 us of copies that are not hidden; every workgroup pays about 5 us of start and end.
-// With every copy from the first cache 1000 rows of 8192 x 16384 take 743 us instead of 887; the vector operations alone are 460. A chain whose products and
+// operations and six matrix operations each) and 0.4 us of copies that are not hidden; every workgroup pays about 5 us of start and end.
+// With every copy from the first cache 1000 rows of 8192 x 16384 take 743 us, where all waves wrote their copies at once 874, now 775; the vector operations alone are 460. A chain whose products and
 // operands were asked for a tile ahead (the factors as one v_mfma_f32_32x32x2_f32 a tile, twice the matrix time) waited less and issued no more: 967 us.
 // Copying global -> LDS without registers, four stages ahead (raw 34-byte blocks, shifted by the readers) measured 64 us at 500 rows
 // against 56: the readers' 32-bit LDS reads cost more than the copies they hide.
-// Measured, 4096 x 4096: 500 rows 323 -> 56 us, 1000 rows 640 -> 112 us, 32 rows 31 -> 13 us against the row sweep (gemv_q8_0_a8_kernel).
+// Measured, 4096 x 4096: 500 rows 323 -> 50 us, 1000 rows 640 -> 98 us, 32 rows 31 -> 12 us against the row sweep (gemv_q8_0_a8_kernel).
 #pragma once
 #include "device_math.hpp"
 #include "host_common.hpp"
@@ -38,15 +38,10 @@ template <int KS> constexpr uint32_t gemm_out_rows() { return 32U * (8U / KS); }
 // the value of the stage-pass p of R in lane order: p with its log2(R) bits reversed
 template <int R> __device__ __forceinline__ uint32_t gemm_lane_of_pass(uint32_t p) { return __builtin_bitreverse32(p) >> (R == 8 ? 29 : 30); }
 
-template <int KS, int NA, bool DW>
+template <int KS, int NA>
 __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a8_view v, uint32_t o_tiles, uint32_t a_tiles) {
     constexpr uint32_t OT = gemm_out_rows<KS>(), AT = 32U * NA, G = gemm_groups<KS>(), P = gemm_pitch<KS>(), R = 32U / KS;
     constexpr uint32_t LEVELS = R == 8U ? 3U : 2U, ABLK = AT * G / kGemmThreads > 0U ? AT * G / kGemmThreads : 1U;
-    // The next stage's copies go to LDS in front of a stage's products, a stage after they were asked for, or behind them, half as long after. Tiles of
-    // 32 weight rows copy twice the bytes a product, so the wait counts there: before -> now, 100 rows of 8192 x 1024 39.1 -> 36.6 us, 300 rows of
-    // 4096 x 2048 41.5 -> 40.1, 50 rows of 4096 x 4096 23.2 -> 22.1, 32 rows 17.0 -> 16.7. Tiles of 64 lose: 4096 x 4096, 500 rows 62.2 -> 62.5,
-    // 8192 x 16384, 1000 rows 887 -> 893.
-    constexpr bool EARLY = KS == 8;
     static_assert(OT * G == kGemmThreads, "one weight block per thread and stage");
     __shared__ __attribute__((aligned(16))) uint8_t wbuf[2][OT * P];
     __shared__ __attribute__((aligned(16))) uint8_t abuf[2][AT * P];
@@ -57,6 +52,11 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
     if (ot >= o_tiles) return;
     const uint32_t t = threadIdx.x, lane = t & 63U, j = lane & 31U, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6), kw = wave % KS, og = wave / KS;
+    // The next stage's copies go to LDS in front of a stage's products, a stage after they were asked for, in the first four waves, and behind them, half as long
+    // after, in the other four: a SIMD has one wave of each, so that one writes its copies while the other multiplies. All waves behind (tiles of 64 weight
+    // rows) or in front (32) -> now: 4096 x 4096, 500 rows 55 -> 50 us, 1000 rows 110 -> 98, 50 rows 18.4 -> 16.6; 100 rows of 8192 x 1024 30.9 -> 27.9; 300 rows of 4096 x
+    // 2048 34.3 -> 31.2.
+    const bool early = wave < 4U;
     const uint32_t groups = v.in / 32U, chunks = (groups + 31U) / 32U, per_pass = (chunks + 1U) / 2U, stages = R * per_pass;
 
     // ---- loader role
@@ -89,19 +89,14 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
         // (nothing here touches a loaded value: the loads are in flight while the previous stage is multiplied)
         scale_next = b[0];
         live = g < groups;
-        if constexpr (DW) {
-            const uint32_t c0 = gg * kQ80Block + 2U;
-            code_shift = c0 & 3U;                    // first code byte: 0 or 2 past a dword boundary
-            const uint32_t* dw = reinterpret_cast<const uint32_t*>(wsrc) + (c0 >> 2);
-            const mm_u32x4_a4 lo = *reinterpret_cast<const mm_u32x4_a4*>(dw), hi = *reinterpret_cast<const mm_u32x4_a4*>(dw + 4);
+        // the nine aligned dwords around the 32 codes (of an aligned block, and of what ends the tensor, none that holds no byte of the block)
+        // (found from the pointer: an address made of an integer would be loaded through the flat path, which the LDS waits wait for as well)
+        code_shift = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(b + 1)) & 3U;     // first code byte: 0 or 2 past a dword boundary
+        const uint32_t* dw = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(b + 1) - code_shift);
+        const mm_u32x4_a4 lo = *reinterpret_cast<const mm_u32x4_a4*>(dw), hi = *reinterpret_cast<const mm_u32x4_a4*>(dw + 4);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { wd[i] = lo[i]; wd[4 + i] = hi[i]; }
-            wd[8] = dw[code_shift ? 8 : 7];          // (an aligned block ends with its eighth dword)
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) wd[i] = static_cast<uint32_t>(b[1 + 2 * i]) | (static_cast<uint32_t>(b[2 + 2 * i]) << 16);
-            wd[8] = 0;
-        }
+        for (int i = 0; i < 4; ++i) { wd[i] = lo[i]; wd[4 + i] = hi[i]; }
+        wd[8] = dw[code_shift ? 8 : 7];
         if (loads_acts) {
 #pragma unroll
             for (uint32_t b2 = 0; b2 < ABLK; ++b2) {
@@ -115,8 +110,8 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
         u32x4 w0, w1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            w0[i] = DW ? __builtin_amdgcn_alignbyte(wd[i + 1], wd[i], code_shift) : wd[i];
-            w1[i] = DW ? __builtin_amdgcn_alignbyte(wd[i + 5], wd[i + 4], code_shift) : wd[i + 4];
+            w0[i] = __builtin_amdgcn_alignbyte(wd[i + 1], wd[i], code_shift);
+            w1[i] = __builtin_amdgcn_alignbyte(wd[i + 5], wd[i + 4], code_shift);
         }
         u32x4* wdst = reinterpret_cast<u32x4*>(&wbuf[buf][wrow * P + 32U * wg]);
         wdst[0] = w0; wdst[1] = w1;
@@ -162,13 +157,13 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
 
     fetch(0);
     stage(0);
-    if (EARLY) fetch(1);                                        // (R stages at least)
+    if (early) fetch(1);                                        // (R stages at least)
     __syncthreads();
     uint32_t in_pass = 0, pass = 0;
     for (uint32_t s = 0; s < stages; ++s) {
         const uint32_t buf = s & 1U;
-        if (EARLY && s + 1U < stages) stage(buf ^ 1U);
-        if (s + (EARLY ? 2U : 1U) < stages) fetch(s + (EARLY ? 2U : 1U));
+        if (early && s + 1U < stages) stage(buf ^ 1U);
+        if (s + (early ? 2U : 1U) < stages) fetch(s + (early ? 2U : 1U));
         const bool second = 2U * in_pass + 1U < chunks;         // the stage's second chunk exists
         const mm_f32x32 none = {0};
         if constexpr (NA == 2) {                                // one factor product per group: its two blocks are the two activation tiles
@@ -208,7 +203,7 @@ __global__ __launch_bounds__(kGemmThreads, 2) void gemm_q8_0_a8_kernel(mi355_q8a
                 }
             }
         }
-        if (!EARLY && s + 1U < stages) stage(buf ^ 1U);
+        if (!early && s + 1U < stages) stage(buf ^ 1U);
         __syncthreads();
     }
 
@@ -253,12 +248,11 @@ static_assert(gemm_takes<4, 2>(32U, 32768U, 1048512U) && !gemm_takes<4, 2>(32U, 
 
 // false: the row sweep serves the product
 template <int KS, int NA>
-inline bool launch_gemm_q8_0(const mi355_q8a8_view& v, bool dw, hipStream_t st) {
+inline bool launch_gemm_q8_0(const mi355_q8a8_view& v, hipStream_t st) {
     if (!gemm_takes<KS, NA>(v.in, v.count, v.rows)) return false;
     const uint32_t o_tiles = (v.count + gemm_out_rows<KS>() - 1U) / gemm_out_rows<KS>(), a_tiles = (v.rows + 32U * NA - 1U) / (32U * NA);
     const uint32_t blocks = static_cast<uint32_t>(gemm_blocks<KS, NA>(v.count, v.rows));
-    if (dw) gemm_q8_0_a8_kernel<KS, NA, true><<<blocks, kGemmThreads, 0, st>>>(v, o_tiles, a_tiles);
-    else gemm_q8_0_a8_kernel<KS, NA, false><<<blocks, kGemmThreads, 0, st>>>(v, o_tiles, a_tiles);
+    gemm_q8_0_a8_kernel<KS, NA><<<blocks, kGemmThreads, 0, st>>>(v, o_tiles, a_tiles);
     return true;
 }
 

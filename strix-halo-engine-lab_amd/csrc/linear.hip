@@ -11,8 +11,10 @@ namespace strix950 {
 // One aligned group of 32 lanes per output row: lane l owns the reference's accumulator lane l (groups g = l, l + 32,
 // ... ascending), then the tree32 butterfly. Up to RB activation rows share one sweep of the weight row.
 // Reference: src/cpu/core/reference.cpp:57-84, src/core/integer_math.hpp:11-13,43-47.
-// DW: the weight rows are 4-byte aligned. A block (34 bytes: fp16 scale, 32 codes) is then fetched as nine aligned dwords
-// (two 128-bit loads and one 32-bit load) around its codes and shifted into place, instead of seventeen 16-bit loads.
+// A block (34 bytes: fp16 scale, 32 codes) is fetched as nine aligned dwords (two 128-bit loads and one 32-bit load) around its codes, wherever the
+// 2-byte aligned row starts, and shifted into place; no dword is read that holds no byte of it. (Rows of 4128 and 1056 features by seventeen 16-bit loads a
+// block: 8 rows x 8192 outputs 25.8 us, now 23.2, 4 x 4096 9.1, 8.7.) DW: the rows are 4-byte aligned, so the place follows from the block's number (1 row of
+// 4096 x 4096 4.5 us, from the address 4.8).
 // CHAIN (RB = 1): the row contract of the reference's dense A8 profile (src/hip_q8_rows_gemv.hpp:1155-1170; host statement
 // tests/dense_a8_small_reference_tests.cpp:93-104): acc = +0, then for the blocks in ascending order acc = fma(float(d_w) * delta,
 // float(dot), acc), and a NaN result is stored as 0x7fc00000. The lanes evaluate their blocks as before and leave every block's
@@ -36,18 +38,13 @@ __global__ __launch_bounds__(256) void gemv_q8_0_a8_kernel(mi355_q8a8_view v) {
         const unsigned short* b = reinterpret_cast<const unsigned short*>(wrow + static_cast<size_t>(g) * kQ80Block);
         const float scale = half_bits_to_float(b[0]);
         int w[8];
-        if constexpr (DW) {
-            const uint32_t c0 = g * kQ80Block + 2U, shift = c0 & 3U;          // first code byte: 0 or 2 past a dword boundary
-            const uint32_t* dw = reinterpret_cast<const uint32_t*>(wrow) + (c0 >> 2);
-            const u32x4_a4 lo4 = *reinterpret_cast<const u32x4_a4*>(dw), hi4 = *reinterpret_cast<const u32x4_a4*>(dw + 4);
-            const uint32_t last = dw[shift ? 8 : 7];                          // (an aligned block ends with its eighth dword)
-            const uint32_t d[9] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w, last};
+        const uint32_t c0 = g * kQ80Block + 2U, shift = (DW ? c0 : static_cast<uint32_t>(reinterpret_cast<uintptr_t>(b + 1))) & 3U;   // first code byte: 0 or 2 past a dword boundary
+        const uint32_t* dw = DW ? reinterpret_cast<const uint32_t*>(wrow) + (c0 >> 2) : reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint8_t*>(b + 1) - shift);
+        const u32x4_a4 lo4 = *reinterpret_cast<const u32x4_a4*>(dw), hi4 = *reinterpret_cast<const u32x4_a4*>(dw + 4);
+        const uint32_t last = dw[shift ? 8 : 7];                          // (an aligned block ends with its eighth dword)
+        const uint32_t d[9] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w, last};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(__builtin_amdgcn_alignbyte(d[i + 1], d[i], shift));
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(static_cast<uint32_t>(b[1 + 2 * i]) | (static_cast<uint32_t>(b[2 + 2 * i]) << 16));
-        }
+        for (int i = 0; i < 8; ++i) w[i] = static_cast<int>(__builtin_amdgcn_alignbyte(d[i + 1], d[i], shift));
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             if (static_cast<uint32_t>(r) < nr) {
@@ -175,8 +172,8 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
         // where they do not; 32 activation rows for a batch that fits them. (4096 x 4096: 12 rows 13.1 us on the row sweep and 12.8 on the
         // matrix cores, 16384 x 8192: 78 and 46 us; 8 rows 8.8 and 12.7 us.) What the tiles do not take stays on the row sweep.
         const uint64_t wide = static_cast<uint64_t>((v->count + 63U) / 64U) * ((v->rows + 63U) / 64U);
-        const bool taken = v->rows <= 32U ? launch_gemm_q8_0<8, 1>(*v, dw, st)
-                           : wide < compute_units() ? launch_gemm_q8_0<8, 2>(*v, dw, st) : launch_gemm_q8_0<4, 2>(*v, dw, st);
+        const bool taken = v->rows <= 32U ? launch_gemm_q8_0<8, 1>(*v, st)
+                           : wide < compute_units() ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
         if (!taken) launch(std::integral_constant<int, 16>{});
     }
     STRIX_LAUNCHED("gemv_q8_0_a8");
