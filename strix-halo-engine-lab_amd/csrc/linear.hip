@@ -163,17 +163,26 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
         else gemv_q8_0_a8_kernel<RB, false><<<g, 256, 0, st>>>(*v);
     };
     STRIX_REQUIRE((v->rows + 15U) / 16U <= 65535U, "Q8_0 product: too many rows for one launch");
-    if (v->rows == 1U) launch(std::integral_constant<int, 1>{});
-    else if (v->rows == 2U) launch(std::integral_constant<int, 2>{});
-    else if (v->rows <= 4U) launch(std::integral_constant<int, 4>{});
-    else if (v->rows <= 8U) launch(std::integral_constant<int, 8>{});
+    // A sweep of few outputs leaves the chip idle, and its time is a workgroup's: rows share one only as far as the launch then still has three workgroups a compute
+    // unit (of eight outputs each), four rows up to six while the weights are few, for nine rows and more up to five. us, rows a workgroup 1, 2, 4, 8 and tiles:
+    //   8192 x 512: 8 rows (512 workgroups of one row) 5.5, 6.9, 9.3, 14.2, 18.9; 16 rows (512 of two) 8.7, 7.6, 9.2, 14.1, 19.0; 64 rows (1024 of four) 28.5, 19.8, 15.7, -, 27.9
+    //   2048 x 2048: 3 rows (768 of one) 3.3, 3.6, 3.9; 4 rows (512 of two) 3.8, 3.6, 4.3; 8 rows (512 of four) 5.4, 4.5, 4.5, 5.8, 7.9; 16 rows (1024) -, 6.6, 5.8, 6.0, 8.1;
+    //   32 rows (2048) -, 11.1, 9.1, 8.5, 8.2; 6144 x 4096: 8 rows (1024) -, 18.1, 15.3, 19.5, 17.4, 12 rows (1536) -, -, 19.8, 21.4, 17.5; 2048 x 10240: 8 rows (2560) -, -, 13.7, 11.6, 15.3
+    // Five to eight rows of many weights are on the matrix cores, whose time hardly depends on the rows, sweep | tiles: 5, 8 rows of 4096 x 7168 13.3, 16.5 | 13.5, 13.6; of 4128 x 8192
+    // 18.2, 23.5 | 17.5; of 8192 x 8192 26.3, 33.1 | 23.6; of 8192 x 16384 56, 75 | 45; of 2048 x 12288 11.1, 13.7 | 15.6; five rows where the tiles leave an
+    // eighth of the compute units idle, 8192 x 5120, 21.2 | 21.9.
+    const uint64_t units = compute_units(), weights = static_cast<uint64_t>(v->in) * v->count;
+    const auto groups = [&](uint32_t rb) { return static_cast<uint64_t>(grid) * ((v->rows + rb - 1U) / rb); };
+    if (v->rows == 1U || groups(1U) <= 3U * units) launch(std::integral_constant<int, 1>{});
+    else if (v->rows == 2U || groups(2U) <= 3U * units) launch(std::integral_constant<int, 2>{});
+    else if (v->rows <= 4U || (weights < (1ULL << 25) && groups(4U) <= (v->rows <= 8U ? 6U : 5U) * units)) launch(std::integral_constant<int, 4>{});
+    else if (v->rows <= 8U && (weights < (7ULL << 22) || (v->rows == 5U && 7U * units > v->count / 4U))) launch(std::integral_constant<int, 8>{});
     else {
         // Tiles of 64 weight rows x 64 activation rows where they fill the compute units, 32 weight rows (K split over twice the waves)
-        // where they do not; 32 activation rows for a batch that fits them. (4096 x 4096: 12 rows 13.1 us on the row sweep and 12.8 on the
-        // matrix cores, 16384 x 8192: 78 and 46 us; 8 rows 8.8 and 12.7 us.) What the tiles do not take stays on the row sweep.
+        // where they do not; 32 activation rows for a batch that fits them. What the tiles do not take stays on the row sweep.
         const uint64_t wide = static_cast<uint64_t>((v->count + 63U) / 64U) * ((v->rows + 63U) / 64U);
         const bool taken = v->rows <= 32U ? launch_gemm_q8_0<8, 1>(*v, st)
-                           : wide < compute_units() ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
+                           : wide < units ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
         if (!taken) launch(std::integral_constant<int, 16>{});
     }
     STRIX_LAUNCHED("gemv_q8_0_a8");

@@ -115,3 +115,42 @@ def test_products_of_any_factors(strix):
         assert torch.equal(got.isnan(), want[:n].isnan())
         clean = ~got.isnan()
         assert torch.equal(got[clean].view(torch.int32), want[:n][clean].view(torch.int32))
+
+
+# around the lines between one, two, four and eight rows to a workgroup of the row sweep and the tiles: 768 workgroups of one and of two rows, 1536 and 1280 of
+# four, 2^25 weights (five rows); tiles with remainders of rows, outputs and groups, of full-range codes and factors over many binades
+@pytest.mark.parametrize("rows,width,count", [(3, 64, 2048), (3, 64, 2056), (8, 1056, 768), (8, 96, 776), (6, 64, 2049), (8, 64, 6144), (8, 64, 6145), (16, 1056, 769),
+                                              (9, 1056, 3408), (9, 1056, 3416), (17, 32, 2177), (32, 992, 1301), (33, 2432, 1163), (70, 1536, 700), (257, 1056, 193),
+                                              (5, 4096, 8191), (5, 4128, 8193), (7, 4096, 7168), (500, 2080, 1111)])
+def test_lines_of_the_products(strix, rows, width, count):
+    rng = np.random.default_rng(rows + count)
+    w = rng.integers(0, 256, (count, width // 32, 34), dtype=np.uint8)
+    w[..., 1] = rng.integers(0, 0x78, w[..., 1].shape)
+    codes = rng.integers(-127, 128, (rows, width)).astype(np.int8)
+    deltas = np.exp2(rng.uniform(-120, 10, (rows, width // 32))).astype(np.float32)
+    want, _ = orc.gemv_q8_0_a8(w.reshape(count, -1), codes, deltas, width, count, threads=8)
+    shifted = torch.zeros(w.size + 2, dtype=torch.uint8, device="cuda")
+    shifted[2:] = dev(w).reshape(-1)
+    for weights in (dev(w.reshape(count, -1)), shifted[2:]):
+        got = strix.gemv_q8_0_a8(weights, dev(codes), dev(deltas), width, count).cpu().numpy()
+        assert np.array_equal(bits(got), bits(want))
+
+
+def test_tiles_of_any_factors(strix):
+    """Infinite, NaN, zero and negative factors on the tiles against the row sweep (which NaN survives where two meet is open)."""
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    rows, width, count = 300, 1056, 1100
+    w = strix.quantize_weight_rows(strix.TYPE_Q8_0, torch.randn((count, width), device="cuda", generator=gen) * 0.02).reshape(count, -1, 34)
+    for o, half in enumerate((0x7C00, 0xFC00, 0x7E00, 0x0000, 0x8000), start=1):
+        w[o, o, 0], w[o, o, 1] = half & 255, half >> 8
+    codes = torch.randint(-127, 128, (rows, width), dtype=torch.int8, device="cuda", generator=gen)
+    deltas = torch.rand((rows, width // 32), device="cuda", generator=gen)
+    deltas[1, 3], deltas[2, 5], deltas[3, 6], deltas[4, 7], deltas[5], deltas[6], deltas[7] = float("inf"), float("nan"), -float("inf"), 0.0, 3e38, -1.0, -0.0
+    codes[8, :32], deltas[8, 0] = 0, float("inf")
+    product = lambda r0, r1: strix.gemv_q8_0_a8(w.reshape(count, -1), codes[r0:r1], deltas[r0:r1], width, count)
+    want = torch.cat([product(r, min(r + 8, rows)) for r in range(0, rows, 8)])
+    for n in (40, 65, 300):
+        got = product(0, n)
+        assert torch.equal(got.isnan(), want[:n].isnan())
+        clean = ~got.isnan()
+        assert torch.equal(got[clean].view(torch.int32), want[:n][clean].view(torch.int32))
