@@ -178,11 +178,13 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
     else if (v->rows <= 4U || (weights < (1ULL << 25) && groups(4U) <= (v->rows <= 8U ? 6U : 5U) * units)) launch(std::integral_constant<int, 4>{});
     else if (v->rows <= 8U && (weights < (7ULL << 22) || (v->rows == 5U && 7U * units > v->count / 4U))) launch(std::integral_constant<int, 8>{});
     else {
-        // Tiles of 64 weight rows x 64 activation rows where they fill the compute units, 32 weight rows (K split over twice the waves)
-        // where they do not; 32 activation rows for a batch that fits them. What the tiles do not take stays on the row sweep.
-        const uint64_t wide = static_cast<uint64_t>((v->count + 63U) / 64U) * ((v->rows + 63U) / 64U);
-        const bool taken = v->rows <= 32U ? launch_gemm_q8_0<8, 1>(*v, st)
-                           : wide < units ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
+        // Tiles of 32 weight x 32 activation rows, then 32 x 64 (K split over twice the waves of the last), while one round of the compute units holds
+        // them: one takes 12, 17.5, 27 us at 4096 features whatever the rest of the chip does, so a second round of a small one is longer than
+        // one of the next. us, 32 x 32 | 32 x 64 | 64 x 64: 4096 x 4096, 64 rows 12.5 | 16.6, 100 rows - | 17.7, 160 rows - | 31.8 | 26; 2048 x 2048, 300 rows - | 19.1 | 15; 8192 x
+        // 1024, 100 rows 19.4 | 27.9. What the tiles do not take stays on the row sweep.
+        const uint64_t stripes = (static_cast<uint64_t>(v->count) + 31U) / 32U;
+        const bool taken = v->rows <= 32U || stripes * ((v->rows + 31U) / 32U) <= units ? launch_gemm_q8_0<8, 1>(*v, st)
+                           : stripes * ((v->rows + 63U) / 64U) <= units ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
         if (!taken) launch(std::integral_constant<int, 16>{});
     }
     STRIX_LAUNCHED("gemv_q8_0_a8");

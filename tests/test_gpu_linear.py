@@ -118,10 +118,11 @@ def test_products_of_any_factors(strix):
 
 
 # around the lines between one, two, four and eight rows to a workgroup of the row sweep and the tiles: 768 workgroups of one and of two rows, 1536 and 1280 of
-# four, 2^25 weights (five rows); tiles with remainders of rows, outputs and groups, of full-range codes and factors over many binades
+# four, 2^25 weights (five rows), 256 tiles of 32 x 32 and of 32 x 64; tiles with remainders of rows, outputs and groups, of full-range codes and factors over many binades
 @pytest.mark.parametrize("rows,width,count", [(3, 64, 2048), (3, 64, 2056), (8, 1056, 768), (8, 96, 776), (6, 64, 2049), (8, 64, 6144), (8, 64, 6145), (16, 1056, 769),
                                               (9, 1056, 3408), (9, 1056, 3416), (17, 32, 2177), (32, 992, 1301), (33, 2432, 1163), (70, 1536, 700), (257, 1056, 193),
-                                              (5, 4096, 8191), (5, 4128, 8193), (7, 4096, 7168), (500, 2080, 1111)])
+                                              (5, 4096, 8191), (5, 4128, 8193), (7, 4096, 7168), (500, 2080, 1111), (33, 992, 4096), (33, 992, 4129), (100, 96, 2081),
+                                              (300, 1056, 833), (200, 96, 2050)])
 def test_lines_of_the_products(strix, rows, width, count):
     rng = np.random.default_rng(rows + count)
     w = rng.integers(0, 256, (count, width // 32, 34), dtype=np.uint8)
