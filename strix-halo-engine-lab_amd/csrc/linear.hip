@@ -171,7 +171,7 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
     // Five to eight rows of many weights are on the matrix cores, whose time hardly depends on the rows, sweep | tiles: 5, 8 rows of 4096 x 7168 13.3, 16.5 | 13.5, 13.6; of 4128 x 8192
     // 18.2, 23.5 | 17.5; of 8192 x 8192 26.3, 33.1 | 23.6; of 8192 x 16384 56, 75 | 45; of 2048 x 12288 11.1, 13.7 | 15.6; five rows where the tiles leave an
     // eighth of the compute units idle, 8192 x 5120, 21.2 | 21.9.
-    const uint64_t units = compute_units(), weights = static_cast<uint64_t>(v->in) * v->count;
+    const uint64_t units = v->rows == 1U ? 0U : compute_units(), weights = static_cast<uint64_t>(v->in) * v->count;
     const auto groups = [&](uint32_t rb) { return static_cast<uint64_t>(grid) * ((v->rows + rb - 1U) / rb); };
     if (v->rows == 1U || groups(1U) <= 3U * units) launch(std::integral_constant<int, 1>{});
     else if (v->rows == 2U || groups(2U) <= 3U * units) launch(std::integral_constant<int, 2>{});
