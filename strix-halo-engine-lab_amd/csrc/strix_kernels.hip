@@ -501,7 +501,7 @@ __global__ __launch_bounds__(64, DEPTH > 3 ? 1 : 2) void project_wave_kernel(mi3
 //     compares its ids with the early ones: where they differ it waits until the assignment's speculative waves have all
 //     finished (their count in the assignment's word), clears the word's non-finite flag and recomputes the assignment's h image
 //     on the exact expert;
-//   projection blocks (assignment, 32-output group): wait for the assignment's tag and the row's tag, then one sweep of the
+//   projection blocks (assignment, 32-output group): wait for the assignment's tag and the tags of all rows, then one sweep of the
 //     tagged expert's gate / up rows; each counts itself into its assignment's word when its part of the h image is acknowledged.
 // Blocks are dispatched in index order, so what a waiting block waits for has been dispatched before it (the repair waits for
 // projection blocks, which themselves wait only for blocks in front of them); every wait is bounded, and a wait that runs out (it
@@ -546,6 +546,16 @@ __device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const m
     project_chunk<1, 2>(slots, source, w, r, grp, 0U, at);
 }
 
+// The A8 images of every row of the launch are stored. Of every row, not of the one that a sweep reads: deltas and sums of neighbouring rows (hidden / 8 bytes
+// each), and code rows of a caller's image that is aligned to 16 bytes only, share cache lines, and the sweep's plain loads bring whole lines into its die's
+// L2, where a later sweep of the neighbour would find what it held before. (All lanes; a row's tag per lane, all of them in one line.)
+__device__ __forceinline__ bool images_there(const uint32_t* lines, uint32_t rows, uint32_t epoch) {
+    const uint32_t lane = threadIdx.x & 63U;
+    uint32_t tag = epoch;
+    if (lane < rows) tag = __hip_atomic_load(&lines[kLinesRowTags + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __ballot(tag != epoch) == 0;
+}
+
 template <int KIND>
 __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r,
                                                   const RouteArgs& a, uint32_t sb, uint32_t assignments, uint32_t epoch) {
@@ -560,15 +570,14 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
         *reinterpret_cast<uint4*>(a.plan + plan_items_at(w.experts, assignments) + 4U * at) = make_uint4(expert, at, at + 1U, at + 1U);
         a.plan[plan_order_at(w.experts) + at] = at;
     }
-    // the early choice of this row and the A8 image of its input (the repair reads it)
+    // the early choice of this row and the A8 images of the input (the repair reads its row's)
     const unsigned long long* etags = reinterpret_cast<const unsigned long long*>(a.plan + kPlanEtagsAt);
     unsigned long long tag = 0;
-    uint32_t image = 0;
     bool there = false;
     for (uint32_t spins = 0; spins < kFrontSpinLimit && !there; ++spins) {
         if (lane < K) tag = __hip_atomic_load(&etags[row * P + lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        image = __hip_atomic_load(&lines[kLinesRowTags + row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        there = __ballot(lane < K && static_cast<uint32_t>(tag >> 32) != epoch) == 0 && image == epoch;
+        const bool images = images_there(lines, a.rows, epoch);
+        there = __ballot(lane < K && static_cast<uint32_t>(tag >> 32) != epoch) == 0 && images;
         if (!there) __builtin_amdgcn_s_sleep(16);
     }
     asm volatile("" ::: "memory");
@@ -713,12 +722,11 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
     // measured slower: the sweeps that serve several rows finish last, and the others do not speed up.)
     const uint32_t groups = w.ffn / 32U, at = bid / groups, grp = bid - at * groups, row = at / P;
     unsigned long long tag = 0;
-    uint32_t image = 0;
     bool there = false;
     for (uint32_t spins = 0; spins < kFrontSpinLimit && !there; ++spins) {
         tag = __hip_atomic_load(&etags[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        image = __hip_atomic_load(&lines[kLinesRowTags + row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        there = static_cast<uint32_t>(tag >> 32) == epoch && image == epoch;
+        const bool images = images_there(lines, a.rows, epoch);
+        there = static_cast<uint32_t>(tag >> 32) == epoch && images;
         // a block that finds nothing at its first look started with the launch: the tags are microseconds away (one long sleep,
         // about 3 us); a block dispatched later, into a freed slot, finds them at once
         if (!there) { if (spins == 0) __builtin_amdgcn_s_sleep(127); else __builtin_amdgcn_s_sleep(8); }

@@ -163,3 +163,26 @@ def test_always_on_slots_equal_the_router_launch(strix, rows, hidden, ffn, exper
             assert torch.equal(got, all_ids) and torch.equal(weights.view(torch.int32), all_w.view(torch.int32))
             assert torch.equal(layer.rawdots[:rows].view(torch.int32), staged.rawdots[:rows].view(torch.int32))
             assert torch.equal(y.view(torch.int32), torch.from_numpy(want).cuda().view(torch.int32)), (form, displaced)
+
+
+# rows whose deltas and sums (hidden / 8 bytes each) share cache lines with their neighbours' in the image that the launch writes and reads; other rows in every
+# call, so that what a line held before is wrong
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(16, 256, 512, 16, 8), (16, 1280, 768, 32, 8), (13, 1792, 512, 32, 8), (16, 2304, 512, 32, 8), (11, 3328, 768, 24, 8)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_rows_that_share_lines_of_the_image(strix, rows, hidden, ffn, experts, top_k, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    g, u = (blocks(gen, experts * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, experts * hidden, ffn, 256, 144, (1, 3))
+    layer, staged = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    inputs = [(torch.randn((rows, hidden), device="cuda", generator=gen) * 2.0 ** (4 * i - 8)).to(dtype) for i in range(5)]
+    epoch = int(layer.plan[EPOCH])
+    outs = []
+    for x in inputs:
+        y, ids, w, _ = layer.run_layer(x, router)
+        outs.append((y.clone(), ids.clone(), w.clone(), layer.status[:rows].clone()))
+    assert int(layer.plan[EPOCH]) == epoch + len(inputs)
+    for x, (y, ids, w, status) in zip(inputs, outs):
+        want_ids, want_w = strix.route(x, router, top_k)[:2]
+        assert torch.equal(ids, want_ids) and torch.equal(w.view(torch.int32), want_w.view(torch.int32)) and int(status.sum()) == 0
+        assert torch.equal(y.view(torch.int32), staged.run(x, want_ids, want_w).view(torch.int32))
