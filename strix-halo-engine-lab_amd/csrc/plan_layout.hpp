@@ -20,15 +20,15 @@ constexpr uint32_t kPlanTicketsAt = 16, kPlanTicketWords = 256;
 // Behind the ticket words, also at a fixed place, the words of a decode batch planned from early routes (route_early.hpp):
 //   one word per assignment (finished projection waves in the low half, bit 31 = non-finite projection);
 //   one 64-bit tag per assignment {epoch, early expert};
-//   three 128-byte lines per row (arrival counts of the early blocks, of the A8 prologue blocks - with the row's flag word beside
-//     it - and of the exact router's side blocks) and a line with one tag per row (epoch of the call whose A8 image of that row is
+//   three 128-byte lines per row (the 64-bit word {epoch, slots} that the row's side block leaves for its helpers, arrival counts of the A8
+//     prologue blocks - with the row's flag word beside it - and of the exact router's side blocks) and a line with one tag per row (epoch of the call whose A8 image of that row is
 //     complete) and the epoch word.
 // Counts are zero when the plan is allocated and every launch leaves them zero. The epoch of a call is the epoch word + 1; the
 // call's down launch stores it back, so tags of earlier calls never look current and nothing has to be reset.
 constexpr uint32_t kLineWords = 32, kEarlyMaxAssignments = 128, kEarlyMinAssignments = 8, kEarlyMaxRows = 16;
 constexpr uint32_t kPlanAwordsAt = kPlanTicketsAt + kPlanTicketWords, kPlanEtagsAt = kPlanAwordsAt + kEarlyMaxAssignments;
 constexpr uint32_t kPlanLinesAt = (kPlanEtagsAt + 2U * kEarlyMaxAssignments + kLineWords - 1U) / kLineWords * kLineWords;      // (lines of a 128-byte aligned plan)
-constexpr uint32_t kLinesEarly = 0, kLinesPrologue = kEarlyMaxRows * kLineWords, kLinesSide = 2U * kEarlyMaxRows * kLineWords;
+constexpr uint32_t kLinesVerdict = 0, kLinesPrologue = kEarlyMaxRows * kLineWords, kLinesSide = 2U * kEarlyMaxRows * kLineWords;
 constexpr uint32_t kLinesRowTags = 3U * kEarlyMaxRows * kLineWords, kLinesEpoch = kLinesRowTags + kEarlyMaxRows;
 constexpr uint32_t kPlanOffsetsAt = kPlanLinesAt + kLinesRowTags + kLineWords;
 static_assert(kPlanEtagsAt % 2U == 0 && kPlanOffsetsAt % 4U == 0, "tags on 8 bytes, the plan arrays on 16");

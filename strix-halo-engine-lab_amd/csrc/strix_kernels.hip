@@ -503,9 +503,11 @@ __global__ __launch_bounds__(64, DEPTH > 3 ? 1 : 2) void project_wave_kernel(mi3
 //     on the exact expert;
 //   projection blocks (assignment, 32-output group): wait for the assignment's tag and the tags of all rows, then one sweep of the
 //     tagged expert's gate / up rows; each counts itself into its assignment's word when its part of the h image is acknowledged.
+//   helper blocks of a row (experts of many bytes only): wait for the side block's word {epoch, slots}, and sweep every helpers-th group
+//     of the slots named there, whose tags name the exact experts by then, in the side block's place.
 // Blocks are dispatched in index order, so what a waiting block waits for has been dispatched before it (the repair waits for
-// projection blocks, which themselves wait only for blocks in front of them); every wait is bounded, and a wait that runs out (it
-// cannot, short of a lost launch) flags the row as an invalid route: nothing of it is published. Everything that crosses
+// projection blocks, which themselves wait only for blocks in front of them; nothing waits for a helper); every wait is bounded, and a wait that
+// runs out (it cannot, short of a lost launch) flags the row as an invalid route: nothing of it is published. Everything that crosses
 // workgroups inside the launch - logits, tags, counts, the A8 images of x and of h, the optional fp32 intermediates - moves by
 // device-scope stores and loads (an assignment that is repaired is written twice, by waves of different XCDs, and the later
 // write has to win at the memory side).
@@ -513,7 +515,14 @@ __global__ __launch_bounds__(64, DEPTH > 3 ? 1 : 2) void project_wave_kernel(mi3
 // L2 channel that holds it, and every weight stream crossing that channel with it.
 // Two ring slots of 10,240 bytes: eight workgroups share a compute unit.
 constexpr uint32_t kFrontSpinLimit = 1U << 22;
-struct FrontBlocks { uint32_t early, prologue, side; };
+struct FrontBlocks { uint32_t early, prologue, side, helpers; };       // helpers: per row
+// An assignment whose expert the early choice did not hold (two logits at the edge of the choice within rounding: rare) is swept again, by the side block's one wave while an
+// expert's gate and up rows are few, else by helper blocks, kFrontHelpers of them over the rows: one wave takes 0.1 ms a MB. Layers with one such assignment in
+// a row, one wave | helpers, us: 1 row of 2048 / 2048 (4.7 MB) 583 | 66, 1, 4 rows of 4096 / 1536 (7 MB) 793, 822 | 76, 129, 1, 6 rows of 6144 / 2560 (18 MB) 1896, 2076 | 156, 464; of
+// 2048 / 768 (1.8 MB) 237. Helpers that wait for nothing, none | 64: 1 row of 2048 / 768 25.0 | 25.6, of 4096 / 512 (2.4 MB) 31.3 | 32.3, of 2048 / 2048 39.3 | 39.5, 1, 4 rows of 4096 / 1536
+// 47.3, 75.6 | 47.3, 75.8, 1 row of 6144 / 2560 77.1 | 77.0.
+constexpr uint64_t kFrontLoneBytes = 4ULL << 20;
+constexpr uint32_t kFrontHelpers = 64;
 constexpr uint32_t kFrontRunWaves = 1024;      // sweeps from which on rows of more than eight super-blocks stream as contiguous stages
 
 // gate + up + SwiGLU + A8 of assignment `at` on expert e, outputs 32 grp .. 32 grp + 31: rows in dense GGUF order whose super-blocks fill a stage's 64 lanes
@@ -556,13 +565,19 @@ __device__ __forceinline__ bool images_there(const uint32_t* lines, uint32_t row
     return __ballot(tag != epoch) == 0;
 }
 
-template <int KIND>
+// the word of a row in which its side block tells the row's helpers {epoch, the slots to sweep again}
+__device__ __forceinline__ unsigned long long* verdict_of(uint32_t* lines, uint32_t row) { return reinterpret_cast<unsigned long long*>(lines + kLinesVerdict + row * kLineWords); }
+
+template <int KIND, bool HELPED>
 __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r,
                                                   const RouteArgs& a, uint32_t sb, uint32_t assignments, uint32_t epoch) {
     const uint32_t lane = threadIdx.x & 63U, neb = (a.p.experts + kSideExperts - 1U) / kSideExperts, row = sb / neb;
     side_chain_block<KIND>(slots[0], slots[1], a, row, (sb % neb) * kSideExperts);
     uint32_t* lines = a.plan + kPlanLinesAt;
     if (!arrive_last(&lines[kLinesSide + row * kLineWords], neb)) return;
+    const auto tell_helpers = [&](uint32_t again) {
+        if (HELPED && lane == 0) __hip_atomic_store(verdict_of(lines, row), (static_cast<unsigned long long>(epoch) << 32) | again, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     const uint32_t expert = route_select_row(reinterpret_cast<float*>((uint8_t*)slots[0]), a, row);
     const uint32_t K = a.p.top_k, P = w.top_k, groups = w.ffn / 32U;          // P: with the always-on slots, which no choice concerns
     if (lane < P) {
@@ -571,7 +586,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
         a.plan[plan_order_at(w.experts) + at] = at;
     }
     // the early choice of this row and the A8 images of the input (the repair reads its row's)
-    const unsigned long long* etags = reinterpret_cast<const unsigned long long*>(a.plan + kPlanEtagsAt);
+    unsigned long long* etags = reinterpret_cast<unsigned long long*>(a.plan + kPlanEtagsAt);
     unsigned long long tag = 0;
     bool there = false;
     for (uint32_t spins = 0; spins < kFrontSpinLimit && !there; ++spins) {
@@ -583,6 +598,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
     asm volatile("" ::: "memory");
     if (!there) {
         if (lane == 0) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_INVALID_ROUTE));
+        tell_helpers(0U);
         return;
     }
     uint64_t differ = __ballot(lane < K && static_cast<uint32_t>(tag) != expert);
@@ -608,6 +624,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             asm volatile("" ::: "memory");
             if (!through) {
                 if (lane == 0) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_INVALID_ROUTE));
+                tell_helpers(0U);
                 return;
             }
             const auto image_word = [&](uint32_t at, uint32_t i) -> uint32_t* {
@@ -651,6 +668,7 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             differ &= ~copy;
         }
     }
+    uint32_t again = 0;
     while (differ) {
         const uint32_t k = static_cast<uint32_t>(__ffsll(static_cast<long long>(differ))) - 1U;
         differ &= differ - 1ULL;
@@ -667,11 +685,42 @@ __device__ __forceinline__ void side_router_block(lds_u8* const (&slots)[2], con
             continue;
         }
         if (lane == 0) __hip_atomic_store(&r.awords[at], groups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (uint32_t grp = 0; grp < groups; ++grp) front_project<true>(slots, w, r, e, grp, at, assignments);
+        if constexpr (HELPED) {
+            if (lane == 0) __hip_atomic_store(&etags[at], (static_cast<unsigned long long>(epoch) << 32) | e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            again |= 1U << k;
+        } else {
+            for (uint32_t grp = 0; grp < groups; ++grp) front_project<true>(slots, w, r, e, grp, at, assignments);
+        }
+    }
+    if (again) stores_acknowledged();
+    tell_helpers(again);
+}
+
+// One of a row's helpers: waits for the side block's word and sweeps its share of the slots named there, every helpers-th of their groups.
+__device__ __forceinline__ void front_helper_block(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r, uint32_t* plan, uint32_t row, uint32_t helper,
+                                                   uint32_t helpers, uint32_t assignments, uint32_t epoch) {
+    unsigned long long word = 0;
+    for (uint32_t spins = 0; spins < kFrontSpinLimit && static_cast<uint32_t>(word >> 32) != epoch; ++spins) {
+        if (spins == 0) __builtin_amdgcn_s_sleep(127); else __builtin_amdgcn_s_sleep(2);
+        word = __hip_atomic_load(verdict_of(plan + kPlanLinesAt, row), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("" ::: "memory");
+    if (static_cast<uint32_t>(word >> 32) != epoch) {
+        if ((threadIdx.x & 63U) == 0) atomicOr(r.status_of(row), static_cast<uint32_t>(MI355_STATUS_INVALID_ROUTE));
+        return;
+    }
+    const unsigned long long* etags = reinterpret_cast<const unsigned long long*>(plan + kPlanEtagsAt);
+    const uint32_t groups = w.ffn / 32U;
+    uint32_t grp = helper;
+    for (uint32_t left = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(word)); left; left &= left - 1U) {
+        const uint32_t at = row * w.top_k + static_cast<uint32_t>(__builtin_ctz(left));
+        const uint32_t e = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(__hip_atomic_load(&etags[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+        for (; grp < groups; grp += helpers) front_project<true>(slots, w, r, e, grp, at, assignments);
+        grp -= groups;
     }
 }
 
-template <int KIND>
+template <int KIND, bool HELPED>
 __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, RouteArgs a, FrontBlocks nb) {
     const RowsK r = dense_views(views);
     // exactly 20,480 bytes of LDS: eight workgroups fill a compute unit's 160 KB (one more byte and only seven fit)
@@ -714,10 +763,15 @@ __global__ __launch_bounds__(64, 2) void layer_front_kernel(mi355_moe_weights w,
     }
     bid -= nb.prologue;
     if (bid < nb.side) {
-        side_router_block<KIND>(sl, w, r, a, bid, assignments, epoch);
+        side_router_block<KIND, HELPED>(sl, w, r, a, bid, assignments, epoch);
         return;
     }
     bid -= nb.side;
+    if (HELPED && bid >= assignments * (w.ffn / 32U)) {
+        bid -= assignments * (w.ffn / 32U);
+        front_helper_block(sl, w, r, a.plan, bid / nb.helpers, bid % nb.helpers, nb.helpers, assignments, epoch);
+        return;
+    }
     // Projection block: assignment `at`, 32-output group `grp`. (Sharing one sweep among the rows that chose an expert was
     // measured slower: the sweeps that serve several rows finish last, and the others do not speed up.)
     const uint32_t groups = w.ffn / 32U, at = bid / groups, grp = bid - at * groups, row = at / P;
@@ -2173,12 +2227,20 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
         a.early_logits = r->rawdots; a.early_stride = wv.top_k * wv.hidden;
         RowsK front = k;
         front.plan = nullptr;              // (the front launch names its assignments itself: the work items are written inside it)
-        const FrontBlocks nb{rows * ((p->experts + kEarlyExperts - 1U) / kEarlyExperts), a.quant_blocks, rows * ((p->experts + kSideExperts - 1U) / kSideExperts)};
-        const uint32_t blocks = nb.early + nb.prologue + nb.side + items * (wv.ffn / 32U);
+        const uint32_t groups = wv.ffn / 32U;
+        const bool large = 2ULL * wv.ffn * moe_row_bytes(wv.gate_type, wv.hidden) > kFrontLoneBytes;
+        const uint32_t helpers = !large ? 0U : groups < kFrontHelpers / rows ? groups : kFrontHelpers / rows;
+        const FrontBlocks nb{rows * ((p->experts + kEarlyExperts - 1U) / kEarlyExperts), a.quant_blocks, rows * ((p->experts + kSideExperts - 1U) / kSideExperts), helpers};
+        const uint32_t blocks = nb.early + nb.prologue + nb.side + items * groups + rows * helpers;
         if (do_front) {
-            if (a.kind == MI355_INPUT_F32) layer_front_kernel<0><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
-            else if (a.kind == MI355_INPUT_F16) layer_front_kernel<1><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
-            else layer_front_kernel<2><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
+            const auto launch = [&](auto helped) {
+                constexpr bool HELPED = decltype(helped)::value;
+                if (a.kind == MI355_INPUT_F32) layer_front_kernel<0, HELPED><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
+                else if (a.kind == MI355_INPUT_F16) layer_front_kernel<1, HELPED><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
+                else layer_front_kernel<2, HELPED><<<blocks, 64, 0, st>>>(wv, front, items, a, nb);
+            };
+            if (helpers) launch(std::true_type{});
+            else launch(std::false_type{});
             STRIX_LAUNCHED("moe layer early routes + gate / up");
         }
         if (do_back) {

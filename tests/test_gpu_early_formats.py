@@ -186,3 +186,65 @@ def test_rows_that_share_lines_of_the_image(strix, rows, hidden, ffn, experts, t
         want_ids, want_w = strix.route(x, router, top_k)[:2]
         assert torch.equal(ids, want_ids) and torch.equal(w.view(torch.int32), want_w.view(torch.int32)) and int(status.sum()) == 0
         assert torch.equal(y.view(torch.int32), staged.run(x, want_ids, want_w).view(torch.int32))
+
+
+def wide_layer(strix, rows, hidden, ffn, experts, top_k, intermediates=False):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden + ffn)
+    g, u = (blocks(gen, experts * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, experts * hidden, ffn, 256, 144, (1, 3))
+    layer, staged = (strix.MoeLayer(hidden, ffn, experts, top_k, g, u, d, rows, intermediates=intermediates) for _ in range(2))
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    return layer, staged, router, torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+
+
+# experts of more than 4 MB of gate and up rows, whose assignments are swept again by helper blocks: more and fewer helpers a row than groups of 32 outputs, none, one
+# and several slots of a row, an assignment that overflows on the exact expert and one that does on the early one
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(1, 2048, 2048, 16, 8), (16, 2304, 1792, 16, 8), (5, 4096, 1536, 24, 6), (3, 6144, 768, 16, 16)])
+@pytest.mark.parametrize("intermediates", [False, True])
+def test_repairs_by_helpers(strix, rows, hidden, ffn, experts, top_k, intermediates):
+    layer, staged, router, x = wide_layer(strix, rows, hidden, ffn, experts, top_k, intermediates)
+    for scale in (1.0, 2.0 ** 14):
+        rows32 = x.float() * scale
+        ids, w = (t.clone() for t in strix.route(rows32, router, top_k)[:2])
+        layer.output.fill_(7.0)
+        staged.output.fill_(7.0)
+        want = staged.run(rows32, ids, w).clone()
+        for displaced in (0, 20, 100, 300, 0):
+            strix.lib().mi355_debug_early_route_perturb(displaced)
+            try:
+                y, got, _, _ = layer.run_layer(rows32, router)
+                torch.cuda.synchronize()
+            finally:
+                strix.lib().mi355_debug_early_route_perturb(0)
+            assert torch.equal(got, ids) and torch.equal(layer.status[:rows], staged.status[:rows])
+            assert torch.equal(y.view(torch.int32), want.view(torch.int32)), (scale, displaced)
+            assert torch.equal(layer.down_codes[:rows * top_k], staged.down_codes[:rows * top_k])
+
+
+def test_a_repair_of_a_large_expert_is_shared(strix):
+    """One wave sweeps 18 MB in 1.8 ms, which would be twenty times the layer."""
+    layer, _, router, x = wide_layer(strix, 1, 6144, 2560, 32, 8)
+    ids = strix.route(x, router, 8)[0].cpu()
+
+    def missed(displaced):
+        early = early_choice(x.float().cpu().numpy(), router.cpu().numpy(), 8, displaced)[0].tolist()
+        return len(set(ids[0].tolist()) - set(early))
+
+    def micros(displaced):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        taken = []
+        strix.lib().mi355_debug_early_route_perturb(displaced)
+        try:
+            for _ in range(12):
+                begin.record()
+                layer.run_layer(x, router)
+                end.record()
+                torch.cuda.synchronize()
+                taken.append(begin.elapsed_time(end) * 1e3)
+        finally:
+            strix.lib().mi355_debug_early_route_perturb(0)
+        return min(taken)
+
+    displaced = next(d for d in range(1, 400) if missed(d) == 1)
+    plain, repaired = micros(0), micros(displaced)
+    assert repaired < 5 * plain, (plain, repaired)
