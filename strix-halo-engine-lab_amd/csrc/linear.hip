@@ -164,19 +164,31 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
     };
     STRIX_REQUIRE((v->rows + 15U) / 16U <= 65535U, "Q8_0 product: too many rows for one launch");
     // A sweep of few outputs leaves the chip idle, and its time is a workgroup's: rows share one only as far as the launch then still has three workgroups a compute
-    // unit (of eight outputs each), four rows up to six while the weights are few, for nine rows and more up to five. us, rows a workgroup 1, 2, 4, 8 and tiles:
+    // unit (of eight outputs each), four rows up to five (six of rows of 4096 features and more; past eight rows, and past five workgroups, while the weights are few). us, rows a workgroup 1, 2, 4, 8 and tiles:
     //   8192 x 512: 8 rows (512 workgroups of one row) 5.5, 6.9, 9.3, 14.2, 18.9; 16 rows (512 of two) 8.7, 7.6, 9.2, 14.1, 19.0; 64 rows (1024 of four) 28.5, 19.8, 15.7, -, 27.9
     //   2048 x 2048: 3 rows (768 of one) 3.3, 3.6, 3.9; 4 rows (512 of two) 3.8, 3.6, 4.3; 8 rows (512 of four) 5.4, 4.5, 4.5, 5.8, 7.9; 16 rows (1024) -, 6.6, 5.8, 6.0, 8.1;
-    //   32 rows (2048) -, 11.1, 9.1, 8.5, 8.2; 6144 x 4096: 8 rows (1024) -, 18.1, 15.3, 19.5, 17.4, 12 rows (1536) -, -, 19.8, 21.4, 17.5; 2048 x 10240: 8 rows (2560) -, -, 13.7, 11.6, 15.3
-    // Five to eight rows of many weights are on the matrix cores, whose time hardly depends on the rows, sweep | tiles: 5, 8 rows of 4096 x 7168 13.3, 16.5 | 13.5, 13.6; of 4128 x 8192
-    // 18.2, 23.5 | 17.5; of 8192 x 8192 26.3, 33.1 | 23.6; of 8192 x 16384 56, 75 | 45; of 2048 x 12288 11.1, 13.7 | 15.6; five rows where the tiles leave an
-    // eighth of the compute units idle, 8192 x 5120, 21.2 | 21.9.
-    const uint64_t units = v->rows == 1U ? 0U : compute_units(), weights = static_cast<uint64_t>(v->in) * v->count;
+    //   32 rows (2048) -, 11.1, 9.1, 8.5, 8.2; 6144 x 4096: 8 rows (1024) -, 18.1, 15.3, 19.5, 17.4, 12 rows (1536) -, -, 19.8, 21.4, 17.5; 2048 x 10240: 8 rows (2560) -, -, 13.7, 11.6, 15.3;
+    //   5, 8 rows, four | eight: 8192 x 4096 (1024) 18.5, 19.7 | 20.7, 28.1 (tiles 21.9), 8192 x 5120 (1280) 20.6, 22.5 | 21.9, 29.1 (22.3), 2112 x 6019 (1506) 9.1, 10.9 | 8.3, 10.2,
+    //   3072 x 6144 (1536) 9.1, 11.3 | 8.9, 11.0, 4096 x 6144 11.1, 13.8 | 11.2, 14.1, 5120 x 6144 14.2, 17.5 | 14.8, 18.8 (16.0)
+    // Five to eight rows of many weights are on the matrix cores, whose time hardly depends on the rows but is that of whole rounds of tiles, one to a compute unit: in one round
+    // always, in more as far as the last one is full, the more rows the less so, and of rows below 4096 features, whose tiles are mostly start and
+    // end, only full ones. 5, 8 rows, sweep of eight | tiles (rounds begun, of which filled): 4096 x 8192 15.0, 18.3 | 14.3 (1, 1); 7168 x 7168 22.6, 28.4 | 22.7
+    // (1, 0.88); 6144 x 6144 18.3, 24.0 | 18.2 (1, 0.75); 2048 x 16384 16.7, 20.7 | 16.5 (2, 2); 4096 x 14336 22.2, 27.4 | 25.2 (2, 1.75); 8192 x 12288 35.8, 44.8 | 42.6 (2, 1.5);
+    // 8192 x 10240 31.6, 38.8 | 42.0 (2, 1.25); 3072 x 12288 16.8, 20.0 | 23.4 (2, 1.5); 2048 x 28672 23.0, 28.1 | 29.4 (4, 3.5); 1024 x 28672 13.8, 16.6 | 26.3 (4, 3.5).
+    const uint64_t known = v->rows == 1U ? 0U : compute_units(), units = known ? known : 1U, weights = static_cast<uint64_t>(v->in) * v->count;
     const auto groups = [&](uint32_t rb) { return static_cast<uint64_t>(grid) * ((v->rows + rb - 1U) / rb); };
+    const auto rounds = [&](uint64_t blocks) { return (blocks + units - 1U) / units; };
+    const auto few_rows_tiled = [&] {        // of five to eight rows
+        const uint64_t tiles = gemm_blocks<8, 1>(v->count, v->rows), places = rounds(tiles) * units;
+        if (weights < (7ULL << 22)) return false;
+        if (places == units) return true;
+        return v->in < 4096U ? v->in >= 2048U && 16U * tiles >= 15U * places : 10U * (places - tiles) <= (v->rows - 5U) * places;
+    };
     if (v->rows == 1U || groups(1U) <= 3U * units) launch(std::integral_constant<int, 1>{});
     else if (v->rows == 2U || groups(2U) <= 3U * units) launch(std::integral_constant<int, 2>{});
-    else if (v->rows <= 4U || (weights < (1ULL << 25) && groups(4U) <= (v->rows <= 8U ? 6U : 5U) * units)) launch(std::integral_constant<int, 4>{});
-    else if (v->rows <= 8U && (weights < (7ULL << 22) || (v->rows == 5U && 7U * units > v->count / 4U))) launch(std::integral_constant<int, 8>{});
+    else if (v->rows <= 4U || (groups(4U) <= 5U * units && (v->rows <= 8U || weights < (1ULL << 25))) ||
+             (v->rows <= 8U && groups(4U) <= 6U * units && v->in >= 4096U && weights < (1ULL << 25))) launch(std::integral_constant<int, 4>{});
+    else if (v->rows <= 8U && !few_rows_tiled()) launch(std::integral_constant<int, 8>{});
     else {
         // Tiles of 32 weight x 32 activation rows, then 32 x 64 (K split over twice the waves of the last), while one round of the compute units holds
         // them: one takes 12, 17.5, 27 us at 4096 features whatever the rest of the chip does, so a second round of a small one is longer than

@@ -118,11 +118,12 @@ def test_products_of_any_factors(strix):
 
 
 # around the lines between one, two, four and eight rows to a workgroup of the row sweep and the tiles: 768 workgroups of one and of two rows, 1536 and 1280 of
-# four, 2^25 weights (five rows), 256 tiles of 32 x 32 and of 32 x 64; tiles with remainders of rows, outputs and groups, of full-range codes and factors over many binades
+# four, 2^25 weights (five to eight rows: one round of tiles three quarters full, full and partial rounds), 256 tiles of 32 x 32 and of 32 x 64; tiles with remainders of rows, outputs and groups, of full-range codes and factors over many binades
 @pytest.mark.parametrize("rows,width,count", [(3, 64, 2048), (3, 64, 2056), (8, 1056, 768), (8, 96, 776), (6, 64, 2049), (8, 64, 6144), (8, 64, 6145), (16, 1056, 769),
                                               (9, 1056, 3408), (9, 1056, 3416), (17, 32, 2177), (32, 992, 1301), (33, 2432, 1163), (70, 1536, 700), (257, 1056, 193),
                                               (5, 4096, 8191), (5, 4128, 8193), (7, 4096, 7168), (500, 2080, 1111), (33, 992, 4096), (33, 992, 4129), (100, 96, 2081),
-                                              (300, 1056, 833), (200, 96, 2050)])
+                                              (300, 1056, 833), (200, 96, 2050), (5, 1024, 28673), (8, 2048, 14337), (6, 2048, 16383), (8, 4096, 12321), (7, 8192, 4095), (8, 6144, 6113),
+                                              (5, 6144, 6145)])
 def test_lines_of_the_products(strix, rows, width, count):
     rng = np.random.default_rng(rows + count)
     w = rng.integers(0, 256, (count, width // 32, 34), dtype=np.uint8)
@@ -155,3 +156,29 @@ def test_tiles_of_any_factors(strix):
         assert torch.equal(got.isnan(), want[:n].isnan())
         clean = ~got.isnan()
         assert torch.equal(got[clean].view(torch.int32), want[:n][clean].view(torch.int32))
+
+
+# the fifth row of a batch over weights that end in the middle of a round of tiles
+@pytest.mark.parametrize("width,count,rows,more,most", [(1024, 28672, 4, 5, 1.35), (3072, 12288, 4, 5, 1.35)])
+def test_a_little_more_costs_little(strix, width, count, rows, more, most):
+    """No step from one round of the compute units to two, nearly twice the time, where another form takes less."""
+    counts = count if isinstance(count, tuple) else (count, count)
+    w = [strix.quantize_weight_rows(strix.TYPE_Q8_0, torch.randn((counts[1], width), device="cuda") * 0.02) for _ in range(8)]
+
+    def micros(rows, count):
+        codes, deltas, _, _ = strix.quantize_a8(torch.randn((rows, width), device="cuda"))
+        y = torch.empty((rows, count), device="cuda")
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        taken = []
+        for _ in range(7):
+            torch.cuda.synchronize()
+            begin.record()
+            for i in range(64):
+                strix.gemv_q8_0_a8(w[i % 8], codes, deltas, width, count, y)
+            end.record()
+            torch.cuda.synchronize()
+            taken.append(begin.elapsed_time(end) * 1e3 / 64)
+        return min(taken)
+
+    before, after = micros(rows, counts[0]), micros(more, counts[1])
+    assert after < most * before, (before, after)
