@@ -190,13 +190,16 @@ int32_t mi355_gemv_q8_0_a8(const mi355_q8a8_view* v, mi355_stream stream) {
              (v->rows <= 8U && groups(4U) <= 6U * units && v->in >= 4096U && weights < (1ULL << 25))) launch(std::integral_constant<int, 4>{});
     else if (v->rows <= 8U && !few_rows_tiled()) launch(std::integral_constant<int, 8>{});
     else {
-        // Tiles of 32 weight x 32 activation rows, then 32 x 64 (K split over twice the waves of the last), while one round of the compute units holds
-        // them: one takes 12, 17.5, 27 us at 4096 features whatever the rest of the chip does, so a second round of a small one is longer than
-        // one of the next. us, 32 x 32 | 32 x 64 | 64 x 64: 4096 x 4096, 64 rows 12.5 | 16.6, 100 rows - | 17.7, 160 rows - | 31.8 | 26; 2048 x 2048, 300 rows - | 19.1 | 15; 8192 x
-        // 1024, 100 rows 19.4 | 27.9. What the tiles do not take stays on the row sweep.
-        const uint64_t stripes = (static_cast<uint64_t>(v->count) + 31U) / 32U;
-        const bool taken = v->rows <= 32U || stripes * ((v->rows + 31U) / 32U) <= units ? launch_gemm_q8_0<8, 1>(*v, st)
-                           : stripes * ((v->rows + 63U) / 64U) <= units ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
+        // Tiles of 32 weight x 32 activation rows, 32 x 64 (K split over twice the waves of the last) or 64 x 64, whichever rounds take the shortest: a round is
+        // 3.0 + 3.9 n, 3.3 + 6.2 n, 3.5 + 10.2 n us long for n runs of 64 groups a row, and a stripe of tiles stays on one of eight dies (gemm_blocks counts what that leaves empty).
+        // us, 32 x 32 | 32 x 64 | 64 x 64 (rounds): 1024, 4096, 8192 features, 96 rows x 4096 13.7, 22.7, 38.6 | 9.3, 17.6, 31.1 | 12.4, 26.2, 46.6 (2, 1, 1); 427 x 2195 26.2, 43.0, 73.6 |
+        // 17.2, 31.8, 55.6 | 23.0, 48.8, 89.1 (4, 2, 2); 128 x 6144 20.3, 33.8, 57.3 | 16.8, 32.2, 57.7 | 12.8, 27.3, 50.8 (3, 2, 1); 800 x 1280 26.0, 42.9, 74.6 | 23.4, 44.8, 80.3 | 22.9, 48.7,
+        // 89.6 (4, 3, 2). What the tiles do not take stays on the row sweep.
+        const uint64_t n = (v->in / 32U + 63U) / 64U;
+        const uint64_t narrow = rounds(gemm_blocks<8, 1>(v->count, v->rows)) * (30U + 39U * n), tall = rounds(gemm_blocks<8, 2>(v->count, v->rows)) * (33U + 62U * n),
+                       wide = rounds(gemm_blocks<4, 2>(v->count, v->rows)) * (35U + 102U * n);
+        const bool taken = v->rows <= 32U || (narrow <= tall && narrow <= wide) ? launch_gemm_q8_0<8, 1>(*v, st)
+                           : tall <= wide ? launch_gemm_q8_0<8, 2>(*v, st) : launch_gemm_q8_0<4, 2>(*v, st);
         if (!taken) launch(std::integral_constant<int, 16>{});
     }
     STRIX_LAUNCHED("gemv_q8_0_a8");

@@ -123,7 +123,7 @@ def test_products_of_any_factors(strix):
                                               (9, 1056, 3408), (9, 1056, 3416), (17, 32, 2177), (32, 992, 1301), (33, 2432, 1163), (70, 1536, 700), (257, 1056, 193),
                                               (5, 4096, 8191), (5, 4128, 8193), (7, 4096, 7168), (500, 2080, 1111), (33, 992, 4096), (33, 992, 4129), (100, 96, 2081),
                                               (300, 1056, 833), (200, 96, 2050), (5, 1024, 28673), (8, 2048, 14337), (6, 2048, 16383), (8, 4096, 12321), (7, 8192, 4095), (8, 6144, 6113),
-                                              (5, 6144, 6145)])
+                                              (5, 6144, 6145), (427, 992, 2195), (800, 96, 1280)])
 def test_lines_of_the_products(strix, rows, width, count):
     rng = np.random.default_rng(rows + count)
     w = rng.integers(0, 256, (count, width // 32, 34), dtype=np.uint8)
@@ -158,8 +158,8 @@ def test_tiles_of_any_factors(strix):
         assert torch.equal(got[clean].view(torch.int32), want[:n][clean].view(torch.int32))
 
 
-# the fifth row of a batch over weights that end in the middle of a round of tiles
-@pytest.mark.parametrize("width,count,rows,more,most", [(1024, 28672, 4, 5, 1.35), (3072, 12288, 4, 5, 1.35)])
+# the fifth row of a batch over weights that end in the middle of a round of tiles; outputs whose stripes of tiles leave places of a die empty
+@pytest.mark.parametrize("width,count,rows,more,most", [(1024, 28672, 4, 5, 1.35), (3072, 12288, 4, 5, 1.35), (2048, (2048, 2195), 427, 427, 1.5)])
 def test_a_little_more_costs_little(strix, width, count, rows, more, most):
     """No step from one round of the compute units to two, nearly twice the time, where another form takes less."""
     counts = count if isinstance(count, tuple) else (count, count)
