@@ -523,13 +523,16 @@ struct FrontBlocks { uint32_t early, prologue, side, helpers; };       // helper
 // 47.3, 75.6 | 47.3, 75.8, 1 row of 6144 / 2560 77.1 | 77.0.
 constexpr uint64_t kFrontLoneBytes = 4ULL << 20;
 constexpr uint32_t kFrontHelpers = 64;
-constexpr uint32_t kFrontRunWaves = 1024;      // sweeps from which on rows of more than eight super-blocks stream as contiguous stages
+constexpr uint32_t kFrontRunWaves = 86;        // sweeps per super-block of a row past which rows of more than eight of them stream as contiguous stages
 
 // gate + up + SwiGLU + A8 of assignment `at` on expert e, outputs 32 grp .. 32 grp + 31: rows in dense GGUF order whose super-blocks fill a stage's 64 lanes
-// (hidden 512, 1024, 2048 and, where the launch's sweeps are enough to be bound by memory, 4096 and more) stream as contiguous stages (q4k_blocks.hpp), others as one
+// (hidden 512, 1024, 2048 and, where the launch's sweeps are enough to be bound by memory, 4096 and 8192) stream as contiguous stages (q4k_blocks.hpp), others as one
 // super-block of each row per stage: a contiguous stage of 48 blocks works as long as one of 64, and its chain runs over the lanes in as many steps
 // as a row has blocks. Layers, contiguous -> block by block: hidden 1280, 1, 4, 12 rows 30.2, 33.3, 53.7 -> 26.4, 29.6, 44.9 us; 1536 30.5, 34.2 -> 27.2, 31.1; 1792
-// 34.6, 41.9 -> 31.8, 39.7; 2304, 1 row 38.3 -> 30.4; 6144, 1 row (640 sweeps) 97.5 -> 79.3; 4096, 1, 2, 4 rows (384, 512, 1536 sweeps) 53.9, 54.4, 76.9 -> 48.5, 49.8, 81.0.
+// 34.6, 41.9 -> 31.8, 39.7; 2304, 1 row 38.3 -> 30.4; 6144, 1 row 97.5 -> 79.3. How many sweeps are enough, contiguous | block by block, rows of hidden / ffn (sweeps):
+//   4096: 2 of 1024 (512) 50.8 | 45.7; 3 of 1536 (1152) 68.8 | 66.1; 10 of 512 (1280) 64.8 | 60.3; 5 of 1024 (1280) 75.0 | 73.6; 7 of 768 (1344) 66.2 | 65.8; 11 of 512 (1408) 66.6 |
+//   68.4; 6 of 1024 (1536) 78.1 | 80.1; 4 of 1536 (1536) 74.7 | 78.2; 5 of 2560, top-4 (1600) 84.7 | 93.7. 8192: 1 of 2048 (512) 97.3 | 77.0; 6 of 1024 (1536) 144.7 | 140.0; 4 of
+//   2048 (2048) 195.2 | 174.8; 5 of 2048 (2560) 230.4 | 223.7; 6 of 2048 (3072) 242.4 | 244.8.
 // REPAIR (an assignment that a side block sweeps again, a rare one, by a single wave): block by block whatever the shape, which keeps the registers of the launch's main path.
 template <bool REPAIR = false>
 __device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const mi355_moe_weights& w, const RowsK& r, uint32_t e, uint32_t grp, uint32_t at, uint32_t assignments) {
@@ -538,7 +541,7 @@ __device__ __forceinline__ void front_project(lds_u8* const (&slots)[2], const m
     const uint8_t* up = w.up + base;
     const uint32_t B = w.hidden / 256U;
     const BlockLanes g = block_lanes(B, 32U);
-    const bool runs = g.used == 64U && (B <= 8U || assignments * (w.ffn / 32U) > kFrontRunWaves);
+    const bool runs = g.used == 64U && (B <= 8U || assignments * (w.ffn / 32U) > kFrontRunWaves * B);
     if (!REPAIR && runs && w.gate_row_stride == static_cast<uint64_t>(B) * kQ4kBlock && block_lanes_ok(B, 32U)) {
         const uint32_t half = 32U / g.R;                  // stages of the gate rows, then as many of the up rows
         float value[1];

@@ -106,7 +106,8 @@ def test_fp32_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_
 
 # rows of more chunks than the side chain's ring has places, the last one partial; more rows than two rounds of the down + combine launch; sweeps of whole and of
 # partial stages; images of h that a repair copies in one piece and in several
-@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(1, 2304, 256, 16, 8), (3, 3328, 256, 24, 4), (16, 4096, 256, 16, 8), (5, 4096, 2304, 10, 8), (2, 8192, 256, 24, 16)])
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k", [(1, 2304, 256, 16, 8), (3, 3328, 256, 24, 4), (16, 4096, 256, 16, 8), (5, 4096, 2304, 10, 8), (2, 8192, 256, 24, 16),
+                                                           (10, 4096, 512, 16, 8), (11, 4096, 512, 16, 8), (6, 8192, 2048, 10, 8)])
 @pytest.mark.parametrize("dtype,down", [(torch.float16, "q4_k"), (torch.bfloat16, "q8_0"), (torch.float32, "q4_k")])
 def test_long_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_k, dtype, down):
     gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
