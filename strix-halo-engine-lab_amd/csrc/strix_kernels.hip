@@ -2204,11 +2204,18 @@ int32_t enqueue_layer(const mi355_route_policy* p, const float* router_weight, c
     // kQuadMaxItems assignments over large experts share their sweeps instead (above): 16 rows of one rank's half of 6144 / 2560 / 160 291.6, with early routes 352.1.
     // Always-on experts: a row's slot more, whose weights every row sweeps by itself where the plan of the router launch has four rows share a sweep. 1, 2, 5, 8, 14
     // rows of 2048 / 768 / 128 40.4, 43.7, 59.1, 72.4, 94.7 -> 31.8, 32.3, 48.3, 61.7, 88.0 us, Q6_K down rows 41.8, 45.9, 62.4, 79.2, 106.5 -> 32.5, 34.2, 55.4, 71.7, 104.1, 4 rows of
-    // 4096 / 1536 / 64 111.4 -> 91.8. The line at 64 MB of them: 43 MB 91.0 -> 82.3 us, 73 MB 132.1 -> 138.5, 80 MB 180.3 -> 182.3, but 70 MB 64.7 -> 59.7. Rows of up to kChainNormHidden
-    // features stay with the router launch, which norms them for nothing, and whose chain is short.
+    // 4096 / 1536 / 64 111.4 -> 91.8. What the shared sweeps save grows with the bytes of these weights over the rows, what the early routes save with the chain: the line lies at 32 KiB a
+    // feature, up to 3072 features at no more than 64 MiB. Router launch | early routes (MiB of them), us: 2048 / 2560 top-4, 7, 9 rows (59, 76) 81.7 | 75.7, 93.5 | 97.6; 1792 / 2048
+    // top-4, 9, 10 (53, 59) 78.7 | 77.7, 82.1 | 92.4; 3072 / 2048 top-4, 6, 7, 8 (61, 71, 81) 89.5 | 87.4, 96.3 | 101.2, 103.3 | 105.1; 3840 / 2048 top-4, 7, 9 (89, 114) 117.0 | 113.6,
+    // 135.3 | 135.9; 5120 / 2048 top-4, 6, 8 (101, 135) 135.0 | 114.6, 157.4 | 153.6; 6144 / 2560, 3 rows top-8 (76) 176.8 | 172.4, 8 top-2 (202) 139.3 | 130.1. Rows of up to
+    // kChainNormHidden features, whose chain is short and which the router launch norms for nothing, only of experts no wider than they are long and five slots: 8 rows of 1280 / 2048
+    // top-4 63.0 | 65.5, 7 of 1024 / 2560 top-2 42.6 | 45.8, 8 of 1536 / 1536 top-4 56.4 | 51.6, 1, 4, 14 of 1024 / 512 / 128 37.6, 37.4, 55.3 | 31.2, 31.1, 42.1, with the norm 38.6, 38.2, 58.1 |
+    // 33.8, 33.2, 44.4, 14 of 1280 / 1024 / 64 with the norm, Q6_K, Q8_0 down rows 93.9, 92.0 | 88.2, 89.3, 6 of 1280 / 768 top-4 with it 41.0 | 35.1. (Three slots with it gain no more
+    // than runs of one program differ, 16 rows of 1024 / 512 37.0 | 35.1, without it 37.9 | 30.9.)
     const RowsK k = [&] { RowsK view = layer_rows(); view.awords = r->plan + kPlanAwordsAt; return view; }();
     const uint64_t expert_bytes = 2ULL * wv.ffn * moe_row_bytes(wv.gate_type, wv.hidden) + static_cast<uint64_t>(wv.hidden) * moe_row_bytes(wv.down_type, wv.ffn);
-    const bool always_on = p->shared_experts == 0 || (wv.hidden > kChainNormHidden && p->shared_experts * rows * expert_bytes <= (64ULL << 20));
+    const uint64_t most = wv.hidden > 2048U && wv.hidden <= 3072U ? 64ULL << 20 : static_cast<uint64_t>(wv.hidden) << 15;
+    const bool always_on = p->shared_experts == 0 || ((wv.hidden > kChainNormHidden || (wv.ffn <= wv.hidden && wv.top_k >= 5U)) && p->shared_experts * rows * expert_bytes <= most);
     const bool early = always_on && p->logits_order == MI355_LOGITS_FMA_ASCENDING && wv.gate_type == MI355_TYPE_Q4_K &&
                        (wv.down_type == MI355_TYPE_Q4_K || down_merge_format_takes(wv, k.h, rows)) && items >= kEarlyMinAssignments && wv.experts > 1U && wv.top_k <= kDownMergeMost &&
                        items <= kEarlyMaxAssignments && wv.hidden % 64U == 0 && 2U * wv.experts <= wv.top_k * wv.hidden;

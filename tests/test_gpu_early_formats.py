@@ -134,7 +134,8 @@ def test_long_rows_equal_staged_launches(strix, rows, hidden, ffn, experts, top_
 
 
 # always-on slots: nine (an instance of their own), ten and more, up to eight; with and without a gate; as many assignments as the form takes
-@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,shared", [(1, 2048, 256, 24, 8, 1), (14, 1792, 256, 32, 8, 1), (5, 2048, 768, 16, 6, 2), (8, 2304, 256, 24, 14, 2), (6, 1792, 512, 16, 8, 2)])
+@pytest.mark.parametrize("rows,hidden,ffn,experts,top_k,shared", [(1, 2048, 256, 24, 8, 1), (14, 1792, 256, 32, 8, 1), (5, 2048, 768, 16, 6, 2), (8, 2304, 256, 24, 14, 2), (6, 1792, 512, 16, 8, 2),
+                                                                  (2, 256, 256, 16, 4, 1), (14, 1280, 1024, 16, 8, 1), (4, 1536, 1536, 12, 4, 2)])
 @pytest.mark.parametrize("down", ["q4_k", "q6_k", "q8_0", "q5_1"])
 @pytest.mark.parametrize("gated", [False, True])
 def test_always_on_slots_equal_the_router_launch(strix, rows, hidden, ffn, experts, top_k, shared, down, gated):
@@ -164,6 +165,30 @@ def test_always_on_slots_equal_the_router_launch(strix, rows, hidden, ffn, exper
             assert torch.equal(got, all_ids) and torch.equal(weights.view(torch.int32), all_w.view(torch.int32))
             assert torch.equal(layer.rawdots[:rows].view(torch.int32), staged.rawdots[:rows].view(torch.int32))
             assert torch.equal(y.view(torch.int32), torch.from_numpy(want).cuda().view(torch.int32)), (form, displaced)
+
+
+# the lines up to which always-on experts take early routes: of their bytes (9 | 10 rows of 1792 / 2048, 4 | 5 of 3072 / 2304), the experts' width and the slots of
+# rows of up to 1536 features; a row's bits are the same on both sides
+@pytest.mark.parametrize("hidden,ffn,top_k,early,late", [(1792, 2048, 4, 9, 10), (3072, 2304, 4, 5, 6), (1280, 1280, 4, 5, None), (1280, 1536, 4, None, 5), (1024, 256, 3, None, 16)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_lines_of_always_on_experts(strix, hidden, ffn, top_k, early, late, norm):
+    gen = torch.Generator(device="cuda").manual_seed(hidden + ffn)
+    experts, rows = 16, max(early or 0, late or 0)
+    g, u = (blocks(gen, (experts + 1) * ffn, hidden, 256, 144, (1, 3)) for _ in range(2))
+    d = blocks(gen, (experts + 1) * hidden, ffn, 256, 144, (1, 3))
+    layer = strix.MoeLayer(hidden, ffn, experts + 1, top_k + 1, g, u, d, rows)
+    router = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    x = torch.randn((rows, hidden), device="cuda", generator=gen).to(torch.float16)
+    scale = torch.rand((hidden,), device="cuda", generator=gen)
+    singles = [layer.run_layer(x[i:i + 1], router, shared_experts=1, norm=(scale, 1e-6) if norm else None)[0].clone() for i in range(rows)]
+    for n, moved in ((early, 1), (late, 0)):
+        if not n:
+            continue
+        epoch = int(layer.plan[EPOCH])
+        y = layer.run_layer(x[:n], router, shared_experts=1, norm=(scale, 1e-6) if norm else None)[0]
+        torch.cuda.synchronize()
+        assert int(layer.plan[EPOCH]) == epoch + moved and int(layer.status[:n].sum()) == 0
+        assert torch.equal(y.view(torch.int32), torch.cat(singles[:n]).view(torch.int32))
 
 
 # rows whose deltas and sums (hidden / 8 bytes each) share cache lines with their neighbours' in the image that the launch writes and reads; other rows in every
