@@ -89,3 +89,29 @@ def test_wide_decode_rows(strix, rows, experts, hidden, top_k, dtype):
     ids_ref, w_ref, s_ref, _ = orc.route(x.float().numpy(), w.numpy(), top_k, bias=None if bias is None else bias.numpy())
     assert np.array_equal(bits(scores.cpu().numpy()), bits(s_ref))
     assert np.array_equal(ids.cpu().numpy().astype(np.uint32), ids_ref) and np.array_equal(bits(weights.cpu().numpy()), bits(w_ref))
+
+
+# infinities, NaN, zeros of both signs and values that overflow in decode rows of that width: the bits of the chains that the vector ALU runs beside a layer's sweeps
+@pytest.mark.parametrize("rows,hidden", [(13, 2304), (16, 4096)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_wide_decode_rows_of_any_values(strix, rows, hidden, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(rows + hidden)
+    experts, top_k, ffn, inf, nan = 32, 8, 256, float("inf"), float("nan")
+    x = torch.randn((rows, hidden), device="cuda", generator=gen)
+    x[1, 5], x[2, 2071], x[3, 9], x[4, 3], x[4, 2100], x[5], x[6], x[7], x[8] = inf, -inf, nan, inf, -inf, inf, nan, 0.0, -0.0
+    x[9] *= 3e38
+    x[10] *= 1e-42
+    x = x.to(dtype)
+    gate, up = (strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((experts * ffn, hidden), device="cuda", generator=gen)) for _ in range(2))
+    down = strix.quantize_weight_rows(strix.TYPE_Q4_K, torch.randn((experts * hidden, ffn), device="cuda", generator=gen))
+    layer = strix.MoeLayer(hidden, ffn, experts, top_k, gate, up, down, rows)
+    w = torch.randn((experts, hidden), device="cuda", generator=gen) * 0.02
+    bad = w.clone()
+    bad[3, 2], bad[4, 2200], bad[5, 5] = inf, nan, -inf
+    for router in (w, bad):
+        scores = strix.route(x, router, top_k)[2]
+        beside = layer.run_layer(x, router)[3]
+        assert torch.equal(scores.reshape(-1).view(torch.int32), beside.reshape(-1)[:rows * experts].view(torch.int32))
+        want = orc.route(x.float().cpu().numpy(), router.cpu().numpy(), top_k)[2]
+        got = scores.cpu().numpy().reshape(want.shape)
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~np.isnan(want)], want[~np.isnan(want)])
