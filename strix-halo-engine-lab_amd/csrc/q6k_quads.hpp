@@ -15,7 +15,8 @@ namespace strix950 {
 
 constexpr uint32_t kQ6kBlock = 210;
 
-// N words starting at a 2-byte aligned address, from N + 1 aligned words: the caller's N words are followed by two more bytes that may be read. (128-bit loads
+// N words starting at a 2-byte aligned address, from N + 1 aligned words: the caller's N words are followed by four more bytes that may be read (all four of them
+// are where the address is a multiple of four, else two). (128-bit loads
 // from the 2-byte aligned address itself are slower: layers of 8, 16 rows of 2048 / 768 / 128 59.7, 98.4 us. The words are reached from the pointer, not from its value
 // as a number, so that they are global loads and not flat ones, which wait for the LDS as well.)
 template <int N>

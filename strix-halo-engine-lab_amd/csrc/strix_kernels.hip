@@ -1420,7 +1420,7 @@ __global__ __launch_bounds__(64 * SLOTS) void down_merge_q51_kernel(mi355_moe_we
 // Down rows + combine in one launch for Q6_K down rows (src/moe_a8_down_contract.cpp:147-158): the workgroup of (row, 16 columns),
 // wave k = the expert in slot k, lane = (row, pair) with the direct loads and the order of down_q6k_kernel. Bound by its loads (q6k_part); three blocks' worth of them
 // asked for together (a bound on the registers, for a workgroup more on a compute unit, costs more than it gives: 8, 16 rows 55.8, 88.6 us). Layers of hidden 2048 /
-// ffn 768 / 128 experts top-8, 1, 8, 16 rows 25.7, 57.8, 92.1 -> 25.1, 54.3, 85.9 us; 5 of them with the norm and an always-on expert 57.3 -> 53.6; 4 rows of 4096 /
+// ffn 768 / 128 experts top-8, 1, 8, 16 rows 25.7, 57.8, 92.1 -> 25.1, 54.3, 85.9 us; 5 of them with the norm and an always-on expert 57.3 -> 52.0; 4 rows of 4096 /
 // 1536 / 64 103.4 -> 94.2; 6 rows of 3072 / 2304 / 32 top-4 100.6 -> 87.8.
 template <uint32_t SLOTS>
 __global__ __launch_bounds__(64 * SLOTS) void down_merge_q6k_kernel(mi355_moe_weights w, RowsK views, uint32_t assignments, uint32_t form) {
@@ -2114,7 +2114,9 @@ void launch_down_merge(const mi355_moe_weights& wv, const RowsK& k, uint32_t row
     else if (flat && B == 4U) down_merge_flat_kernel<4><<<grid, threads, 0, st>>>(wv, k, items, form);
     else down_merge_kernel<<<grid, threads, 0, st>>>(wv, k, items, form);
 }
-// launch(SLOTS): of the instance for that many slots
+// launch(SLOTS): of the instance for that many slots. Nine, top-8 and an always-on expert, have one of their own: more workgroups a compute unit than with sixteen slots' LDS, more registers than
+// waves of 1024 threads may have. Layers of 2048 / 768 / 128 with it, instance of sixteen | nine, 1, 5, 12 rows, us: Q4_K 31.9, 46.3, 76.0 | 31.4, 44.4, 71.7; Q6_K 30.1, 49.0, 84.8 | 29.9,
+// 47.0, 81.1; Q8_0 29.9, 49.0, 83.7 | 30.0, 48.6, 82.6; Q5_1 30.1, 50.3, 84.6 | 29.8, 48.2, 79.6.
 template <class Launch> void down_merge_slots(uint32_t slots, Launch launch) {
     if (slots <= kDownMergeSlots) launch(std::integral_constant<uint32_t, kDownMergeSlots>{});
     else if (slots == kDownMergeSlots + 1U) launch(std::integral_constant<uint32_t, kDownMergeSlots + 1U>{});
